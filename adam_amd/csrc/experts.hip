@@ -257,35 +257,38 @@ __device__ __forceinline__ bool pick_tile(const uint32_t* __restrict__ cnt, uint
 template <class T>
 __device__ __forceinline__ void put_activation(const XSpec& s, T* opnd, uint32_t arow, uint32_t n0, f4_t gt, f4_t up) {
   const uint32_t c = (n0 >> 5) * 16u + (n0 & 15u), F = (s.ff + 15u) & ~15u;
-  T* d = opnd + s.act_opnd + (uint64_t)arow * s.ff_stride + c;
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  t4 y;
 #pragma unroll
-  for (int i = 0; i < 4; i++) if (c + i < F) d[i] = (T)(silu_f(gt[i]) * up[i]);
+  for (int i = 0; i < 4; i++) y[i] = (T)(silu_f(gt[i]) * up[i]);
+  if (c < F) *(t4*)(opnd + s.act_opnd + (uint64_t)arow * s.ff_stride + c) = y;       // (F: whole runs of 16; rows start on 8 elements)
 }
 __device__ __forceinline__ void put_part(const XSpec& s, float* parts, uint32_t entry, uint32_t n0, f4_t v) {
   float* d = parts + (uint64_t)entry * s.width + n0;
+  if ((s.width & 3u) == 0u) { if (n0 < s.width) *(f4_t*)d = v; return; }
 #pragma unroll
   for (int i = 0; i < 4; i++) if (n0 + i < s.width) d[i] = v[i];
 }
 
-template <int BM, int BN, bool IN>
-__global__ void __launch_bounds__(256)
+template <int BM, int BN, int WM, int WN, int ST, bool IN>
+__global__ void __launch_bounds__(64 * WM * WN)
 k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
                 const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n) {
-  __shared__ __attribute__((aligned(16))) bf16_t la[2 * BN * 64], lb[2 * BM * 64];
-  constexpr int NTN = BN / 32, NTM = BM / 32;
+  __shared__ __attribute__((aligned(16))) bf16_t la[ST * BN * 64], lb[ST * BM * 64];
+  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16;
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t c = lane & 15u, kg = lane >> 4, kp = IN ? s.k_stride : s.ff_stride, n = IN ? 2u * ((s.ff + 15u) & ~15u) : s.width;
   Tile t;
   if (!pick_tile(cnt, s.experts, BM, tiles_n, t)) return;
-  const uint32_t m0 = t.m * BM, n0 = t.n * BN, wn = (wave & 1u) * (BN / 2), wm = (wave >> 1) * (BM / 2);
+  const uint32_t m0 = t.m * BM, n0 = t.n * BN, wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
   const bf16_t* We = W + (IN ? s.gate_up + (uint64_t)t.e * s.gate_up_step : s.down + (uint64_t)t.e * s.down_step);
   const uint32_t* le = list + (uint64_t)t.e * rows;
   f4_t acc[NTN][NTM];
-  tile_product<BM, BN>(acc, TileRows<BN>(wave, lane, [&](uint32_t r) { return We + (uint64_t)min(n0 + r, n - 1u) * kp; }),
-                       TileRows<BM>(wave, lane, [&](uint32_t r) {
-                         const uint32_t i = min(m0 + r, t.count - 1u);
-                         return opnd + (IN ? s.opnd + (uint64_t)(le[i] / s.top) * kp : s.act_opnd + (uint64_t)(t.first + i) * kp);
-                       }), kp, la, lb, wave, lane);
+  tile_product<BM, BN, WM, WN, ST>(acc, TileRows<BN, WM * WN>(wave, lane, [&](uint32_t r) { return We + (uint64_t)min(n0 + r, n - 1u) * kp; }),
+                                   TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) {
+                                     const uint32_t i = min(m0 + r, t.count - 1u);
+                                     return opnd + (IN ? s.opnd + (uint64_t)(le[i] / s.top) * kp : s.act_opnd + (uint64_t)(t.first + i) * kp);
+                                   }), kp, la, lb, wave, lane);
 #pragma unroll
   for (int j = 0; j < NTM; j++) {
     const uint32_t i = m0 + wm + 16u * j + c;
@@ -368,9 +371,9 @@ static void experts_product(Map* mo, Map* mw, const XSpec& s, float* parts, cons
   if (mo->dtype == DTYPE_F32)
     k_experts_f32<IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (float*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
   else if (entries >= (uint64_t)s.experts * 96u)
-    k_experts_tiled<128, 128, IN><<<grid(128, cdiv(n, 128)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 128));
+    k_experts_tiled<128, 256, 2, 4, 3, IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256));
   else
-    k_experts_tiled<64, 64, IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
+    k_experts_tiled<64, 64, 2, 2, 4, IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
   count_launch();
 }
 

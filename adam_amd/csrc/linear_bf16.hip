@@ -5,7 +5,7 @@
 //                through registers, float32 multiply-adds; store, add to the residual, gate / up pairs combined, or
 //                store + best row of the workgroup (arg-max)
 //   2..32 rows   k_linear_skinny: bf16 matrix instructions straight from memory, K split over the waves of a workgroup
-//   more rows    k_linear_tiled<BM, BN>: bf16 matrix instructions over LDS tiles filled by direct-to-LDS loads
+//   more rows    k_linear_tiled<BM, BN, ...>: bf16 matrix instructions over a ring of LDS tiles filled by direct-to-LDS loads
 //   float32 operand map: k_linear_f32, the float32 matrix instruction over the widened weights
 // Rows of more than one token pass through the operand map (bf16 or float32, rows k_stride apart, zero beyond k):
 // k_operand_rows writes f(x) there, unless the producer already did.
@@ -294,28 +294,34 @@ k_best_row(const float* __restrict__ act, uint64_t src, uint32_t stride, uint32_
 }
 
 // ---- results of the matrix-instruction kernels --------------------------------------------------------------------
-// Lane l of a 16 x 16 result holds matrix rows (outputs) 4 (l / 16) + 0..3 of token l % 16.
+// Lane l of a 16 x 16 result holds matrix rows (outputs) 4 (l / 16) + 0..3 of token l % 16: one 16-byte (bfloat16:
+// 8-byte) access where the rows' places allow it, four narrow ones at a ragged end.
 __device__ __forceinline__ void put_out(const LinSpec& s, float* act, uint32_t row, uint32_t n0, f4_t v) {
   float* d = act + s.out + (uint64_t)row * s.out_stride + n0;
-  if (s.biased) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) if (n0 + i < s.n) v[i] += act[s.bias + n0 + i];
+  if (((s.out | s.out_stride) & 3u) == 0u && (!s.biased || (s.bias & 3u) == 0u) && n0 + 4u <= s.n) {
+    if (s.biased) v += *(const f4_t*)(act + s.bias + n0);
+    if (s.epi == 1u) v += *(const f4_t*)d;
+    *(f4_t*)d = v;
+    return;
   }
-  if (s.epi == 1u) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) if (n0 + i < s.n) d[i] += v[i];
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; i++) if (n0 + i < s.n) d[i] = v[i];
+  for (int i = 0; i < 4; i++) if (n0 + i < s.n) {
+    const float y = s.biased ? v[i] + act[s.bias + n0 + i] : v[i];
+    d[i] = s.epi == 1u ? d[i] + y : y;
   }
 }
 // gate rows n0 .. n0 + 3 and their up rows -> the activation's operand rows
 template <class T>
 __device__ __forceinline__ void put_pair(const LinSpec& s, T* opnd, uint32_t row, uint32_t n0, f4_t gt, f4_t up) {
   const uint32_t c = (n0 >> 5) * 16u + (n0 & 15u);
+  typedef T t4 __attribute__((ext_vector_type(4)));
   T* d = opnd + s.out_opnd + (uint64_t)row * s.out_opnd_stride + c;
+  t4 y;
 #pragma unroll
-  for (int i = 0; i < 4; i++) if (n0 + i < s.n) d[i] = (T)(silu_f(gt[i]) * up[i]);
+  for (int i = 0; i < 4; i++) y[i] = (T)(silu_f(gt[i]) * up[i]);
+  if (((s.out_opnd | s.out_opnd_stride) & 3u) == 0u && n0 + 4u <= s.n) { *(t4*)d = y; return; }
+#pragma unroll
+  for (int i = 0; i < 4; i++) if (n0 + i < s.n) d[i] = y[i];
 }
 // two neighbouring runs of 16 rows of an epi 2 product, from row n0 on: a pair, or two runs of the tail
 template <class T>
@@ -385,12 +391,12 @@ k_linear_skinny(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, floa
 }
 
 // ---- tiles --------------------------------------------------------------------------------------------------------
-template <int BM, int BN>
-__global__ void __launch_bounds__(256)
+template <int BM, int BN, int WM, int WN, int ST>
+__global__ void __launch_bounds__(64 * WM * WN)
 k_linear_tiled(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, bf16_t* opnd, const LinSpec s, uint32_t rows,
                uint32_t tiles_m, uint32_t tiles_n) {
-  __shared__ __attribute__((aligned(16))) bf16_t la[2 * BN * 64], lb[2 * BM * 64];
-  constexpr int NTN = BN / 32, NTM = BM / 32;
+  __shared__ __attribute__((aligned(16))) bf16_t la[ST * BN * 64], lb[ST * BM * 64];
+  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16;
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t c = lane & 15u, kg = lane >> 4, kp = s.k_stride;
   // workgroups land on the eight dies in turn: give every die a run of neighbouring tiles
@@ -398,10 +404,11 @@ k_linear_tiled(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float
   const uint32_t id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if (id >= total || (blockIdx.x >> 3) >= per) return;
   const uint32_t m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
-  const uint32_t wn = (wave & 1u) * (BN / 2), wm = (wave >> 1) * (BM / 2);
+  const uint32_t wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
   f4_t acc[NTN][NTM];
-  tile_product<BM, BN>(acc, TileRows<BN>(wave, lane, [&](uint32_t r) { return W + (uint64_t)min(n0 + r, s.n - 1u) * kp; }),
-                       TileRows<BM>(wave, lane, [&](uint32_t r) { return X + (uint64_t)min(m0 + r, rows - 1u) * kp; }), kp, la, lb, wave, lane);
+  tile_product<BM, BN, WM, WN, ST>(
+      acc, TileRows<BN, WM * WN>(wave, lane, [&](uint32_t r) { return W + (uint64_t)min(n0 + r, s.n - 1u) * kp; }),
+      TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) { return X + (uint64_t)min(m0 + r, rows - 1u) * kp; }), kp, la, lb, wave, lane);
 #pragma unroll
   for (int j = 0; j < NTM; j++) {
     const uint32_t row = m0 + wm + 16u * j + c;
@@ -515,13 +522,26 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   if (rows <= 16) k_linear_skinny<1><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows);
   else if (rows <= 32) k_linear_skinny<2><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows);
   else {
-    const uint32_t big = cdiv(rows, 128) * cdiv(s.n, 128);
-    if (big >= (uint32_t)g.n_cu * 3 / 4) {
-      k_linear_tiled<128, 128><<<cdiv(big, 8) * 8, 256, 0, g.stream>>>(W, X, act, op, s, rows, cdiv(rows, 128), cdiv(s.n, 128));
-    } else {
-      const uint32_t small = cdiv(rows, 64) * cdiv(s.n, 64);
-      k_linear_tiled<64, 64><<<cdiv(small, 8) * 8, 256, 0, g.stream>>>(W, X, act, op, s, rows, cdiv(rows, 64), cdiv(s.n, 64));
+    // The tile that gets through the rows soonest: rounds over the CUs times what a step of 64 columns takes there
+    // (1/100 us, measured with all CUs at work on 2048 x 28672 x 4096, 600 x 12672 x 4096, 300 x 10304 x 2048 and
+    // 300 x 4096 x 4096; with at most one workgroup a CU, with two where two fit).
+    const auto cost = [&](uint32_t bm, uint32_t bn, uint32_t one, uint32_t two) {
+      const uint64_t tiles = (uint64_t)cdiv(rows, bm) * cdiv(s.n, bn), cu = (uint64_t)g.n_cu, fit = two ? 2 * cu : cu, left = tiles % fit;
+      return tiles / fit * (two ? two : one) + (left == 0 ? 0 : left <= cu ? one : two);
+    };
+    const uint64_t c[6] = {cost(256, 256, 170, 0), cost(256, 128, 105, 0), cost(128, 256, 105, 0), cost(128, 128, 63, 0), cost(64, 128, 50, 80),
+                           cost(64, 64, 40, 55)};
+#define LT(BM, BN, WM, WN, ST) do { const uint32_t t = cdiv(rows, BM) * cdiv(s.n, BN); \
+      k_linear_tiled<BM, BN, WM, WN, ST><<<cdiv(t, 8) * 8, 64 * WM * WN, 0, g.stream>>>(W, X, act, op, s, rows, cdiv(rows, BM), cdiv(s.n, BN)); } while (0)
+    switch (std::min_element(c, c + 6) - c) {
+      case 0: LT(256, 256, 2, 4, 2); break;
+      case 1: LT(256, 128, 4, 2, 3); break;
+      case 2: LT(128, 256, 2, 4, 3); break;
+      case 3: LT(128, 128, 2, 4, 4); break;
+      case 4: LT(64, 128, 2, 2, 3); break;
+      default: LT(64, 64, 2, 2, 4); break;
     }
+#undef LT
   }
   count_launch();
   return check_launch();

@@ -31,67 +31,102 @@ __device__ __forceinline__ float wsum64(float v) {
 }
 
 // ---- tiles of the many-row products ---------------------------------------------------------------------------------
-// BM tokens x BN matrix rows, 64 columns of K a step, four waves as 2 x 2.  Tiles go straight to LDS (16 bytes a lane,
-// eight rows of 128 bytes an instruction); chunk j of a row sits at slot j ^ (row & 7), which spreads the 16-byte reads
-// of 16 rows over the banks.  Two buffers: the next step's loads run under this step's products.  Where a lane's rows
-// start is settled once, so they may lie anywhere.
-template <int R> struct TileRows {
-  const bf16_t* p[R / 32];
+// 16 bytes a lane from memory straight to LDS, lane l's to byte `lds` + 16 l.  Written out because the compiler, which
+// cannot tell the buffers of a ring apart, waits for every such load in flight before it reads LDS (two buffers then hide
+// nothing: 2048 x 28672 x 4096 took 600 us).  No register is loaded, so there is none to wait for: `ring_wait` stands
+// ahead of the reads of the bytes.  M0 is set by every such load and used by nothing else in these kernels.
+__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_byte(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p; }
+// all but the last N loads of this wave have arrived and its reads of LDS are done; then every wave's
+template <int N>
+__device__ __forceinline__ void ring_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+// R rows of 64 columns (128 bytes, a cache line) a step, loaded by NW waves, eight rows an instruction; chunk j (16 bytes)
+// of a row sits at slot j ^ (row & 7), which spreads the 16-byte reads of neighbouring rows over the banks (no conflict
+// counted; runs of 32 columns, whose rows are half a line, loaded 15 % slower).  Where a lane's rows start is settled once,
+// so they may lie anywhere.
+template <int R, int NW> struct TileRows {
+  static constexpr int N = R / (8 * NW);                     // loads a step and lane
+  static_assert(N * 8 * NW == R, "whole loads");
+  const bf16_t* p[N];
   template <class Row>
   __device__ __forceinline__ TileRows(uint32_t wave, uint32_t lane, Row row) {
 #pragma unroll
-    for (int i = 0; i < R / 32; i++) {
-      const uint32_t r = (uint32_t)i * 32u + wave * 8u + (lane >> 3);
+    for (int i = 0; i < N; i++) {
+      const uint32_t r = ((uint32_t)i * NW + wave) * 8u + (lane >> 3);
       p[i] = row(r) + (((lane & 7u) ^ (r & 7u)) << 3);
     }
   }
-  __device__ __forceinline__ void load(uint32_t k, bf16_t* lds, uint32_t wave) const {
-#pragma unroll
-    for (int i = 0; i < R / 32; i++)
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p[i] + k),
-                                       (__attribute__((address_space(3))) void*)(lds + ((uint32_t)i * 32u + wave * 8u) * 64u), 16, 0, 0);
+  __device__ __forceinline__ void load(int i, uint32_t k, uint32_t lds, uint32_t wave) const {
+    load_to_lds(p[i] + k, lds + ((uint32_t)i * NW + wave) * 1024u);
   }
 };
-// acc[i][j]: matrix rows wn + 16 i, tokens wm + 16 j of the tile; la: 2 BN 64, lb: 2 BM 64 elements
-template <int BM, int BN>
-__device__ __forceinline__ void tile_product(f4_t (&acc)[BN / 32][BM / 32], const TileRows<BN>& w, const TileRows<BM>& x, uint32_t kp,
-                                             bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane) {
-  constexpr int NTN = BN / 32, NTM = BM / 32;
-  const uint32_t c = lane & 15u, kg = lane >> 4, wn = (wave & 1u) * (BN / 2), wm = (wave >> 1) * (BM / 2);
+// BM tokens x BN matrix rows by WM x WN waves; acc[i][j]: matrix rows wn + 16 i, tokens wm + 16 j of a wave's part; la: ST
+// BN 64, lb: ST BM 64 elements.  A ring of ST buffers of 64 columns: a step's loads are asked for ST - 1 steps ahead.  A
+// step is two halves of 32 columns; a half's operands are read from LDS under the products of the half before, on both
+// sides of the step's one barrier.  What bounds it (256 x 256, two buffers): of the 1.75 us a step takes on all CUs the
+// products need 1.0, the loads alone 0.7 (23 TB/s out of the L2s), reads of LDS run beside both; loads and reads in a run
+// ahead of the products instead of among them: 1.95 us.
+template <int BM, int BN, int WM, int WN, int ST>
+__device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM / 16], const TileRows<BN, WM * WN>& w, const TileRows<BM, WM * WN>& x,
+                                             uint32_t kp, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane) {
+  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16, LOADS = TileRows<BN, WM * WN>::N + TileRows<BM, WM * WN>::N;
+  const uint32_t c = lane & 15u, kg = lane >> 4, wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
+  const uint32_t ba = lds_byte(la), bb = lds_byte(lb);
 #pragma unroll
   for (int i = 0; i < NTN; i++)
 #pragma unroll
     for (int j = 0; j < NTM; j++) acc[i][j] = (f4_t){0, 0, 0, 0};
-  w.load(0, la, wave);
-  x.load(0, lb, wave);
+  const auto load = [&](int i, uint32_t k, uint32_t into) {       // (steps past the end re-read the last: the count in flight stays)
+    const uint32_t kc = min(k, kp - 64u);
+    if (i < TileRows<BN, WM * WN>::N) w.load(i, kc, ba + into * (BN * 128u), wave);
+    else x.load(i - TileRows<BN, WM * WN>::N, kc, bb + into * (BM * 128u), wave);
+  };
+  bf8_t a[2][NTN], b[2][NTM];
+  const auto read = [&](int i, uint32_t buf, int h) {
+    const uint32_t at = ((4u * h + kg) ^ (c & 7u)) << 3;
+    if (i < NTM) b[h][i] = *(const bf8_t*)(lb + buf * (BM * 64) + (wm + 16u * i + c) * 64u + at);
+    else a[h][i - NTM] = *(const bf8_t*)(la + buf * (BN * 64) + (wn + 16u * (i - NTM) + c) * 64u + at);
+  };
+  // four products, then a few of the next half's reads and (LD) one of the loads, and so on: the matrix pipe is never
+  // behind a run of either
+  constexpr int NP = NTN * NTM / 4, READS = NP > 1 ? (NTN + NTM + NP - 2) / (NP - 1) : NTN + NTM, LOADS_EACH = (LOADS + NP - 1) / NP;
+  const auto half = [&](int h, uint32_t from, uint32_t k, uint32_t into) {
+#pragma unroll
+    for (int q = 0; q < NP; q++) {
+#pragma unroll
+      for (int i = 0; i < READS; i++) if (q * READS + i < NTN + NTM) read(q * READS + i, from, 1 - h);
+      if (h == 1) {
+#pragma unroll
+        for (int i = 0; i < LOADS_EACH; i++) if (q * LOADS_EACH + i < LOADS) load(q * LOADS_EACH + i, k, into);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int i = (4 * q + u) / NTM, j = (4 * q + u) % NTM;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[h][i], b[h][j], acc[i][j], 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < ST; t++)
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) load(i, (uint32_t)t * 64u, t);
+  ring_wait<LOADS * (ST - 1)>();
+#pragma unroll
+  for (int i = 0; i < NTN + NTM; i++) read(i, 0, 0);
   uint32_t buf = 0;
-  for (uint32_t k = 0; k < kp; k += 64u, buf ^= 1u) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();                       // this step's tiles have arrived, the other buffer is no longer read
-    if (k + 64u < kp) {
-      w.load(k + 64u, la + (buf ^ 1u) * (BN * 64), wave);
-      x.load(k + 64u, lb + (buf ^ 1u) * (BM * 64), wave);
-    }
-    const bf16_t *ta = la + buf * (BN * 64), *tb = lb + buf * (BM * 64);
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      bf8_t a[NTN], b[NTM];
-#pragma unroll
-      for (int i = 0; i < NTN; i++) {
-        const uint32_t r = wn + 16u * i + c;
-        a[i] = *(const bf8_t*)(ta + r * 64u + (((4u * h + kg) ^ (r & 7u)) << 3));
-      }
-#pragma unroll
-      for (int j = 0; j < NTM; j++) {
-        const uint32_t r = wm + 16u * j + c;
-        b[j] = *(const bf8_t*)(tb + r * 64u + (((4u * h + kg) ^ (r & 7u)) << 3));
-      }
-#pragma unroll
-      for (int i = 0; i < NTN; i++)
-#pragma unroll
-        for (int j = 0; j < NTM; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
+  for (uint32_t k = 0; k < kp; k += 64u) {
+    const uint32_t next = buf + 1 == ST ? 0 : buf + 1;
+    half(0, buf, 0, 0);
+    ring_wait<LOADS * (ST - 2)>();                 // the next step's tiles have arrived, this step's are no longer read
+    half(1, next, k + ST * 64u, buf);
+    buf = next;
   }
+  ring_wait<0>();                                  // nothing is on its way to LDS when the workgroup ends
 }
 // The same in float32: 64 tokens x 64 matrix rows, 32 columns a step, on the float32 matrix instruction.  Within a run of
 // 16 columns, instruction i takes column 4 g + i from lane group g on both sides, so a lane's operands are one 16-byte

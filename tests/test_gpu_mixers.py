@@ -14,7 +14,7 @@ from adam_amd.engine import GenerationConfig
 from adam_amd.mixer_engine import MixerEngine
 from adam_amd.models import load_engine, vomotar_config
 from adam_amd.safetensors_file import f32_to_bf16
-from gpu_util import note
+from gpu_util import f32map, note, read, rel_l2, up
 from mixer_cases import CONFIGS, config, delta, floats, par, rel, weights, write_model
 from mixer_pair import CA, OP, ST, WS, WT, Pair
 from oracle import mixers_np as M
@@ -64,6 +64,34 @@ def test_linear(hip, dtype, rows, n, k, groups, epi):
         s2 = A.LinearSpec(w=0, n=out_w, k=out_w, k_stride=w2, opnd=oo, ready=1, out=out, out_stride=out_w + 3)
         p.call("linear_dev", WS, OP, WT, p.up(s2.words()), 0, rows)
     p.same(WS, out, rows * (out_w + 3) - 3, tol, "out")
+
+
+@pytest.mark.parametrize("rows,n,k,biased,add", [
+    (2000, 8170, 64, 0, 0), (2048, 4096, 128, 1, 1), (1999, 4090, 192, 1, 0), (600, 12600, 64, 0, 1), (300, 10300, 128, 1, 0),
+    (300, 6001, 320, 0, 0), (40, 300, 256, 1, 1), (33, 64, 64, 0, 0), (100, 131, 1024, 0, 1)])
+def test_linear_tiles(hip, rows, n, k, biased, add):
+    """Every tile of the many-row product (256 x 256 down to 64 x 64 on 256 CUs), rings shorter and longer than K, ragged ends."""
+    note(f"linear tiles rows {rows} n {n} k {k}")
+    rng = np.random.default_rng(n)
+    st = n + (0 if n % 4 == 0 else 3)
+    W = f32_to_bf16(rng.standard_normal((n, k)).astype(np.float32))
+    x = f32_to_bf16(rng.standard_normal((rows, k)).astype(np.float32))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, x.size)
+    hip.scatter_contiguous(OP, 0, x.reshape(-1))
+    old = rng.standard_normal((rows + 1) * st).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    f32map(hip, WS, old.size + n, np.concatenate([old, bias]))
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=k, opnd=0, ready=1, out=0, out_stride=st, epi=add, bias=old.size, biased=biased)
+    hip.linear_dev(WS, OP, WT, up(hip, spec.words()), 0, rows)
+    got = read(hip, WS, 0, old.size).reshape(rows + 1, st)
+    f64 = lambda b: (b.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    old = old.reshape(rows + 1, st)
+    want = f64(x) @ f64(W).T + (bias if biased else 0.0) + (old[:rows, :n] if add else 0.0)
+    # exact products, float32 sums of at most 1026 terms: 1026 * 2^-24 relative to the terms' root sum of squares at most
+    assert rel_l2(got[:rows, :n], want) < 6.2e-5
+    assert np.array_equal(got[:rows, n:], old[:rows, n:]) and np.array_equal(got[rows], old[rows])       # nothing beyond
 
 
 @pytest.mark.parametrize("rows", [1, 3])
