@@ -22,6 +22,7 @@
 // each, so that small matrices still spread over the whole chip; their partial tiles are summed through LDS in
 // a fixed order.
 #include "gemv_common.h"
+#include "lds_ring.h"
 #include <algorithm>
 
 namespace adamah {
@@ -327,6 +328,176 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
       if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;   // the add behind it
     }
   }
+}
+
+// ---- more than 64 activation rows ------------------------------------------------------------------------------------
+// Eight waves of 64 weight rows each, side by side, over 32 MA activation rows: a wave has 2 x MA results of 32 x 32.  A step
+// is 64 columns (two blocks); its packed weights (16 KB), their scales (2 KB) and both planes of the activations (8 KB per 32
+// rows) go straight to LDS, a ring of three stages and more.  512 x 28672 x 4096: 319 -> 246 us = 489 TFLOP/s (matrix pipe
+// 58 % busy on the CUs that have a workgroup).  What bounds it is the vector work beside the matrix instructions (a
+// multiply-add per result and block, the unpacking): they share a wave's issue, so what counts is that no instruction of
+// either kind waits for another.  LDS reads without bank conflicts: 266 -> 246 us.
+// v_mfma_f32_32x32x16_f16: lane l supplies row l % 32, k = 8 (l / 32) .. + 7 of either operand and receives rows
+// 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32 -- here the columns are weight rows, so a block's scale is one number per
+// lane.  An instruction covers half a block; two permutes bring a block's words to the half of the wave that owns them.
+typedef float f16q_t __attribute__((ext_vector_type(16)));
+#define RING_W 16384u
+#define RING_S 2048u
+#define MFMA32_F16(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8q_t, a), __builtin_bit_cast(h8q_t, b), c, 0, 0, 0)
+
+template <int MA>
+__global__ void __launch_bounds__(512)
+k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ xh, const u4q_t* __restrict__ xl,
+               uint32_t K, uint32_t N, uint32_t M, uint32_t gbase, uint32_t c_val, uint32_t by_val, uint32_t pairs_per, float* out,
+               float* __restrict__ part, const uint32_t* __restrict__ lc, const float* __restrict__ scale, GemmSegs segs) {
+  constexpr uint32_t BM = 32u * MA, BN = 512u, RING_STAGE = RING_W + RING_S + MA * 8192u;
+  constexpr int LOADS = 3 + MA, RING_ST = MA == 1 ? 6 : MA == 2 ? 4 : 3;      // loads of a wave and stage: 2 of weights, 1 of scales, MA of activations
+  __shared__ __attribute__((aligned(16))) uint8_t ring[RING_ST * RING_STAGE];
+  const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t r32 = lane & 31u, h = lane >> 5;
+  const uint32_t n0 = blockIdx.x * BN, m0 = blockIdx.y * BM, kz = blockIdx.z;
+  const uint32_t nblk = K >> 5, pairs = K >> 6, p_lo = kz * pairs_per, p_hi = min(pairs, p_lo + pairs_per);
+  const uint32_t steps = p_hi - p_lo;
+
+  // piece j of an activation row lies at j ^ slot(row): no two rows that are read together meet in a bank
+  const auto slot = [](uint32_t row) { return (row & 7u) ^ ((row >> 4) & 1u); };
+  // a load is a base for the wave and an offset for the lane
+  uint32_t wo[2], so, xo[MA];
+#pragma unroll
+  for (uint32_t u = 0; u < 2; u++)                           // 32 rows of 32 bytes an instruction; LDS: [row][32]
+    wo[u] = (min(n0 + (wave * 2u + u) * 32u + (lane >> 1), N - 1u) * nblk + (lane & 1u)) << 4;
+  so = min(n0 + wave * 64u + lane, N - 1u) * nblk * 2u;      // 64 rows of 4 bytes; LDS: [row][4]
+#pragma unroll
+  for (uint32_t u = 0; u < MA; u++) {                        // 8 rows of 128 bytes; LDS: [plane][row][8 pieces, swizzled]
+    const uint32_t row = ((wave * MA + u) * 8u) % BM + (lane >> 3);
+    xo[u] = (min(m0 + row, M - 1u) * (K >> 3) + ((lane & 7u) ^ slot(row))) << 4;
+  }
+  const uint32_t base = lds_byte(ring);
+  // load i of this wave for step s of this share; steps past its end re-read its last one (the count in flight stays)
+  const auto load = [&](int i, uint32_t s, uint32_t into) {
+    const uint32_t at = base + into * RING_STAGE;
+    const uint64_t pair = min(p_lo + s, p_hi - 1u);
+    if (i < 2) load_to_lds(W + (((uint64_t)gbase + pair * 2u) << 4), wo[i], at + (wave * 2u + i) * 1024u);
+    else if (i == 2) load4_to_lds(d16 + gbase + pair * 2u, so, at + RING_W + wave * 256u);
+    else {
+      const uint32_t j = wave * MA + (i - 3);
+      load_to_lds((j >= 4u * MA ? xl : xh) + pair * 8u, xo[i - 3], at + RING_W + RING_S + j * 1024u);
+    }
+  };
+
+  f16q_t acc[2][MA], blk[2], zero;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    zero[i] = 0.f; blk[1][i] = 0.f;
+#pragma unroll
+    for (int w = 0; w < 2; w++)
+#pragma unroll
+      for (int t = 0; t < MA; t++) acc[w][t][i] = 0.f;
+  }
+  DEQK_INIT(dk);
+  u4q_t q[2], raw[2], wf[2][2][2], fr[2][2];              // wf [block][tile][half], fr [plane][half]
+  h2q_t ds[2];
+  float d[2][2], dn[2][2], dlast = 0.f;                      // [tile][block]
+  const uint32_t wrow = (wave * 64u + r32) * 32u + h * 16u, srow = RING_W + (wave * 64u + r32) * 4u;
+  const uint32_t xrow = RING_W + RING_S + r32 * 128u;
+  const auto read_w = [&](const uint8_t* st, int w) {
+    raw[w] = *(const u4q_t*)(st + wrow + w * 1024u);
+    ds[w] = *(const h2q_t*)(st + srow + w * 128u);
+  };
+  const auto take_w = [&](int w) {
+    const u2s_t a = __builtin_amdgcn_permlane32_swap(raw[w].x, raw[w].y, false, false), b = __builtin_amdgcn_permlane32_swap(raw[w].z, raw[w].w, false, false);
+    q[w] = (u4q_t){a.x, b.x, a.y, b.y};                      // block 0's halves, block 1's halves
+    dn[w][0] = (float)ds[w].x; dn[w][1] = (float)ds[w].y;
+  };
+  const auto unpack = [&](int b, int w, int e) { wf[b][w][e] = deq_word(b ? (e ? q[w].w : q[w].z) : (e ? q[w].y : q[w].x), dk); };
+  const auto read_x = [&](const uint8_t* st, int b, int t, int plane, int e) {
+    fr[plane][e] = *(const u4q_t*)(st + xrow + plane * (MA * 4096u) + t * 4096u + (((4u * b + 2u * e + h) ^ slot(r32)) << 4));
+  };
+#pragma unroll
+  for (int s = 0; s < RING_ST - 1; s++)
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) load(i, s, s);
+  ring_wait<LOADS * (RING_ST - 2)>();
+#pragma unroll
+  for (int w = 0; w < 2; w++) {
+    read_w(ring, w);
+    take_w(w);
+    unpack(0, w, 0); unpack(0, w, 1);
+    d[w][0] = dn[w][0]; d[w][1] = dn[w][1];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) read_x(ring, 0, 0, i >> 1, i & 1);
+  uint32_t buf = 0, next = 1, into = RING_ST - 1;
+  for (uint32_t s = 0; s < steps; s++) {
+    const uint8_t *st = ring + buf * RING_STAGE, *sn = ring + next * RING_STAGE;
+    constexpr int NT = 2 * MA;                               // tiles of a block
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      if (b) ring_wait<LOADS * (RING_ST - 3)>();             // the next stage is here, the one before is no longer read
+#pragma unroll
+      for (int x = 0; x < NT; x++) {
+        const int t = x >> 1, w = x & 1;
+        // four instructions of this tile (32 clocks of the matrix pipe each) and between them the scaling of the last
+        // tile's result, which is there once two of them have gone out (behind the first it held up the second: 266 us
+        // for 512 x 28672 x 4096), and what the next tiles, block and stages need
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+          blk[w] = MFMA32_F16(fr[m >> 1][m & 1], wf[b][w][m & 1], m ? blk[w] : zero);
+          const int pw = 1 - w, pt = w ? t : (x ? t - 1 : MA - 1);
+          const float ps = w ? d[0][b] : (x ? d[1][b] : (b ? d[1][0] : dlast));
+#pragma unroll
+          for (int i = m ? 5 * m - 5 : 0; i < (m == 3 ? 16 : 5 * m); i++) acc[pw][pt][i] = fmaf(blk[pw][i], ps, acc[pw][pt][i]);
+          if (w == 1) {                                      // its last use: the same operand of the next 32 rows
+            if (t + 1 < MA) read_x(st, b, t + 1, m >> 1, m & 1);
+            else if (b == 0) read_x(st, 1, 0, m >> 1, m & 1);
+            else read_x(sn, 0, 0, m >> 1, m & 1);
+          }
+          if (b == 1 && x == 0 && m < 2) read_w(sn, m);
+          if (b == 1 && x == 1 && m >= 2) take_w(m - 2);
+          if (b == 0 && m == 0) for (int u = x * 4 / NT; u < (x + 1) * 4 / NT; u++) unpack(1, u >> 1, u & 1);
+          if (b == 1 && MA > 1 && x >= 2 && m == 0) for (int u = (x - 2) * 4 / (NT - 2); u < (x - 1) * 4 / (NT - 2); u++) unpack(0, u >> 1, u & 1);
+          if (b == 1) for (int u = (4 * x + m) * LOADS / (4 * NT); u < (4 * x + m + 1) * LOADS / (4 * NT); u++) load(u, s + RING_ST - 1u, into);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (MA == 1 && b == 1 && x == 1) {
+#pragma unroll
+          for (int u = 0; u < 4; u++) unpack(0, u >> 1, u & 1);
+        }
+      }
+    }
+    dlast = d[1][1];
+#pragma unroll
+    for (int w = 0; w < 2; w++) { d[w][0] = dn[w][0]; d[w][1] = dn[w][1]; }
+    into = buf; buf = next; next = next + 1u == RING_ST ? 0u : next + 1u;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; i++) acc[1][MA - 1][i] = fmaf(blk[1][i], dlast, acc[1][MA - 1][i]);
+  ring_wait<0>();
+  const uint64_t c_off = (by_val & 2u) || part || segs.count ? (uint64_t)c_val : (uint64_t)lc[0];
+#pragma unroll
+  for (int t = 0; t < MA; t++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const uint32_t row = m0 + t * 32u + 8u * (i >> 2) + 4u * h + (i & 3u);
+      if (row >= M) continue;
+      const float inv = part ? 1.f : scale[2 * (uint64_t)row + 1];
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        const uint32_t n = n0 + wave * 64u + w * 32u + r32;
+        if (n >= N) continue;
+        if (part) { part[((uint64_t)kz * M + row) * N + n] = acc[w][t][i]; continue; }
+        const float y = acc[w][t][i] * inv;
+        if (segs.count) {
+          uint32_t sgi = 0;
+#pragma unroll
+          for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
+          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y;
+        } else {
+          out[c_off + (uint64_t)row * N + n] = y;
+          if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;
+        }
+      }
+    }
 }
 
 // Few activation rows (M <= 32): the weights are read once and nothing is reused, so the work is
@@ -954,16 +1125,46 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // Preconditions (checked by the caller against the host copies of the handles): Q4 map whose blocks
 // in range are in the block16 layout, K a multiple of 128, weight bases block aligned, all operands
 // in range.
-// Shares of K a one-op Q4 matmul of M rows is cut into (1: one launch): 2 .. 4 where the widest tile (256 weight rows
-// x 128 rows) would give fewer than three quarters of the CUs a workgroup and the shares fill them, each share at
-// least 1024 elements long.
-uint32_t gemm_q4_k_shares(uint32_t M, uint32_t K, uint32_t N) {
-  if (M < 128 || tuning("ADAMAH_GEMM_SPLITK", 1) == 0) return 1;
-  const uint64_t w256 = (uint64_t)cdiv(N, 256) * cdiv(M, 128);
-  if (w256 * 4 >= 3ull * (uint64_t)g.n_cu) return 1;
-  uint32_t sp = (uint32_t)std::min<uint64_t>(4, (uint64_t)g.n_cu / std::max<uint64_t>(1, w256));
-  while (sp > 1 && K / sp < 1024u) sp--;
-  return sp > 1 && w256 * sp * 4 >= 3ull * (uint64_t)g.n_cu ? sp : 1u;
+// How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: MA > 0
+// k_gemm_q4_ring<MA>, 0 the tiled kernel; over how many shares of K.  Estimates in us, fitted to M = 33 .. 512 over 28672 x
+// 4096, 6144 x 4096, 4096 x 4096, 4096 x 14336, 13824 x 1152 and 1152 x 6912 (within 20 %; between near equals either is
+// fine): a ring step takes 1.5 (MA = 2) or 2.3 us (MA = 4) alone and 2.1 or 3.4 with all CUs at work, a 128-column step of
+// the 64 x 64 tile 1.3 .. 2.3, of the 64 x 256 tile 3; shares cost a launch and the passes over the partial sums.
+// Measured either way (us): 48 x 4096 x 14336 137 -> 33 over 16 shares, 100 x 4096 x 4096 43 -> 32, 48 x 13824 x 1152 16
+// (21 over two shares).
+struct GemmPlan { int ma; uint32_t shares; };
+static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
+  const uint64_t cu = (uint64_t)g.n_cu, steps = cdiv(K, 128), pairs = K / 64;
+  const auto cdiv64 = [](uint64_t x, uint64_t y) { return (x + y - 1) / y; };
+  const uint64_t small = cdiv64(N, 64) * cdiv64(M, 64);
+  const double passes = (double)M * (double)N * 4.0 / 4.5e6;              // one pass over a result
+  double best = (double)steps * (small <= cu / 2 ? 1.3 : small <= cu ? 1.75 : 2.3) * std::max(1.0, (double)small / (3.0 * (double)cu));
+  if (small * 64 * 64 >= 96 * 128 * cu) best = 1e30;                      // (a large product: the ring's)
+  GemmPlan p = {0, 1};
+  if (tuning("ADAMAH_GEMM_SPLITK", 1) == 0) return p;
+  if (M <= 64) {
+    const uint64_t w = cdiv64(N, 256);
+    uint64_t sp = std::min<uint64_t>(16, std::max<uint64_t>(1, 2 * cu / w));
+    while (sp > 1 && K / sp < 512u) sp--;
+    if (sp > 1 && 3.0 * (double)cdiv64(steps, sp) + 9.0 < (double)steps * (small <= cu / 2 ? 1.3 : small <= cu ? 1.75 : 2.2)) p.shares = (uint32_t)sp;
+    return p;
+  }
+  if (b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) return p;
+  for (int ma = 2; ma <= 4; ma += 2) {
+    const uint64_t tiles = cdiv64(N, 512) * cdiv64(M, 32 * (uint64_t)ma);
+    for (uint64_t sp = 1; sp <= 16 && sp * 4 <= pairs && (sp == 1 || tiles * sp <= cu); sp++) {
+      const uint64_t wgs = tiles * sp;
+      const double full = std::min(1.0, (double)wgs / (double)cu), t = ma == 2 ? 1.5 + 0.6 * full : 2.3 + 1.1 * full;
+      const double us = (double)cdiv64(wgs, cu) * ((double)cdiv64(pairs, sp) * t + 10.0) + (sp > 1 ? 4.0 + (2.0 * (double)sp + 1.0) * passes : 0.0);
+      if (us < best) { best = us; p = {ma, (uint32_t)sp}; }
+    }
+  }
+  return p;
+}
+// Whether the matmul's launches also store an add that consumes its result (more than 32 rows, one op)
+bool gemm_q4_adds(uint32_t M, uint32_t K, uint32_t N, int64_t b) {
+  const GemmPlan p = gemm_plan(M, K, N, b);
+  return p.ma > 0 || p.shares > 1;
 }
 
 int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const uint32_t* lb, const uint32_t* lc,
@@ -973,7 +1174,7 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   const uint32_t b_val = b_host >= 0 ? (uint32_t)b_host : 0u, c_val = c_host >= 0 ? (uint32_t)c_host : 0u;
   const uint32_t by_val = n_ops == 1 ? ((b_host >= 0 ? 1u : 0u) | (c_host >= 0 ? 2u : 0u)) : 0u;
   if (((q8 || out) && M > 32) || ((out || segs) && n_ops != 1) || (out && segs) || (segs && segs->glu && M > 32) ||
-      (segs && segs->add && M > 32 && (n_ops != 1 || q8 || gemm_q4_k_shares(M, K, N) < 2)))
+      (segs && segs->add && M > 32 && (n_ops != 1 || q8 || !gemm_q4_adds(M, K, N, b_host))))
     return ADAMAH_ERR_INVALID;
   GemmSegs sg = {};
   if (segs) sg = *segs;
@@ -1049,6 +1250,35 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     keep();
     return check_launch();
   }
+  GemmPlan plan = n_ops == 1 && !q8 && !out ? gemm_plan(M, K, N, b_host) : GemmPlan{0, 1};
+  const auto add_up = [&](uint32_t shares) {
+    const uint64_t quads = ((uint64_t)M * N + 3) / 4;
+    k_gemm_splitk_sum<<<cdiv(quads, 256), 256, 0, g.stream>>>(g_part_buf, shares, M, N, act, c_val, by_val, lc, g_scale_buf, sg);
+    count_launch();
+  };
+  if (plan.shares > 1 && !ensure_part_buf((size_t)plan.shares * M * N)) {
+    if (sg.add) return ADAMAH_ERR_MEMORY;        // (the tiled kernel in one launch stores no add)
+    plan = {0, 1};
+  }
+  if (plan.ma) {
+    const uint32_t pairs = K >> 6, per = cdiv(pairs, plan.shares), shares = cdiv(pairs, per);
+    const dim3 grid(cdiv(N, 512), cdiv(M, 32 * plan.ma), shares);
+#define GR(T) k_gemm_q4_ring<T><<<grid, 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, (uint32_t)(b_host >> 5), c_val, by_val, per, act, shares > 1 ? g_part_buf : nullptr, lc, g_scale_buf, sg)
+    if (plan.ma == 2) GR(2); else GR(4);
+#undef GR
+    count_launch();
+    if (shares > 1) add_up(shares);
+    keep();
+    return check_launch();
+  }
+  if (plan.shares > 1) {                         // 33 .. 64 rows: 256 weight rows a workgroup over shares of K
+    const uint32_t kper = cdiv(cdiv(K >> 5, plan.shares), 4u) * 4u, shares = cdiv(K >> 5, kper);
+    k_gemm_q4_f16_tiled<4, 2, 8><<<dim3(cdiv(N, 256), cdiv(M, 64), shares), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, shares, kper, g_part_buf);
+    count_launch();
+    add_up(shares);
+    keep();
+    return check_launch();
+  }
   // Tile per workgroup: 16 NW R weight rows x 16 MT activation rows (NW waves with R tiles of 16 weight rows each).
   // Every workgroup stages its activation tile (two fp16 planes: 64 KB per step of 128 weights at MT = 8) from L2,
   // while its weights are 4.5 bits each, so the bytes a workgroup moves per flop fall with the number of weight
@@ -1065,27 +1295,9 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   NW = (uint32_t)knob("ADAMAH_GEMM_NW", (int)NW) >= 8 ? 8 : 4;
   R = R >= 4 && mt == 4 ? 4 : R >= 2 ? 2 : 1;
   if (mt == 4 && NW == 8 && R == 1) R = 2;
-  // A narrow matrix under many rows (N = 4096 / 6144 at M = 512) gives the widest tile (256 weight rows x 128 rows)
-  // too few workgroups for the chip, and the smaller tiles that do fill it re-stage more activations per flop: there
-  // the widest tile is launched over 2 .. 4 shares of K, raw sums into scratch, and a second launch adds the shares.
-  uint32_t ksplit = 1, kper = K >> 5;
-  {
-    const uint32_t sp = n_ops == 1 && !q8 && !out ? gemm_q4_k_shares(M, K, N) : 1u;
-    if (sp > 1 && ensure_part_buf((size_t)sp * M * N)) {
-      ksplit = sp; mt = 8; R = 2; NW = 8;
-      kper = cdiv(cdiv(K >> 5, ksplit), 4u) * 4u;
-      ksplit = cdiv(K >> 5, kper);
-    } else if (sg.add && M > 32) return ADAMAH_ERR_MEMORY;   // (only the split launch stores the add of many rows)
-  }
-  dim3 grid(cdiv(N, 16 * NW * R), cdiv(M, 16 * mt), ksplit > 1 ? ksplit : n_ops);
-#define GT(T, RR, W) k_gemm_q4_f16_tiled<T, RR, W><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, ksplit, kper, g_part_buf)
-  if (ksplit > 1) {
-    GT(8, 2, 8);
-    count_launch();
-    const uint64_t quads = ((uint64_t)M * N + 3) / 4;
-    k_gemm_splitk_sum<<<cdiv(quads, 256), 256, 0, g.stream>>>(g_part_buf, ksplit, M, N, act, c_val, by_val, lc, g_scale_buf, sg);
-  }
-  else if (mt == 4 && NW == 8) { if (R == 4) GT(4, 4, 8); else GT(4, 2, 8); }
+  dim3 grid(cdiv(N, 16 * NW * R), cdiv(M, 16 * mt), n_ops);
+#define GT(T, RR, W) k_gemm_q4_f16_tiled<T, RR, W><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, 1, K >> 5, nullptr)
+  if (mt == 4 && NW == 8) { if (R == 4) GT(4, 4, 8); else GT(4, 2, 8); }
   else if (mt == 4) { if (R == 4) GT(4, 4, 4); else if (R == 2) GT(4, 2, 4); else GT(4, 1, 4); }
   else if (NW == 8) { if (R == 2) GT(8, 2, 8); else GT(8, 1, 8); }
   else { if (R == 2) GT(8, 2, 4); else GT(8, 1, 4); }

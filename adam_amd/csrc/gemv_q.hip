@@ -574,7 +574,7 @@ int op_matmul_t_xq(uint32_t dtype, uint32_t map_act, uint32_t map_wt, uint32_t h
     if (ok) {
       flush_pending();
       return launch_gemm_q4_mfma(ma, mw, la, lb, lc, M, K, N, n_ops, dtype == DTYPE_Q8, nullptr,
-                                 n_ops == 1 ? (int64_t)ah[0] : -1, n_ops == 1 ? (int64_t)ch[0] : -1);
+                                 n_ops == 1 ? (int64_t)ah[0] : -1, n_ops == 1 ? (int64_t)ch[0] : -1, nullptr, n_ops == 1 ? (int64_t)bh[0] : -1);
     }
   }
 generic:

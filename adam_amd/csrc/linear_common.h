@@ -1,6 +1,6 @@
 // Products with bfloat16 weight maps: the operand structs shared by the launchers and the ops built on them.
 #pragma once
-#include "common.h"
+#include "lds_ring.h"
 #include "../../include/adamah_hip.h"
 
 namespace adamah {
@@ -31,18 +31,6 @@ __device__ __forceinline__ float wsum64(float v) {
 }
 
 // ---- tiles of the many-row products ---------------------------------------------------------------------------------
-// 16 bytes a lane from memory straight to LDS, lane l's to byte `lds` + 16 l.  Written out because the compiler, which
-// cannot tell the buffers of a ring apart, waits for every such load in flight before it reads LDS (two buffers then hide
-// nothing: 2048 x 28672 x 4096 took 600 us).  No register is loaded, so there is none to wait for: `ring_wait` stands
-// ahead of the reads of the bytes.  M0 is set by every such load and used by nothing else in these kernels.
-__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
-}
-__device__ __forceinline__ uint32_t lds_byte(const void* p) { return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p; }
-// all but the last N loads of this wave have arrived and its reads of LDS are done; then every wave's
-template <int N>
-__device__ __forceinline__ void ring_wait() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
-
 // R rows of 64 columns (128 bytes, a cache line) a step, loaded by NW waves, eight rows an instruction; chunk j (16 bytes)
 // of a row sits at slot j ^ (row & 7), which spreads the 16-byte reads of neighbouring rows over the banks (no conflict
 // counted; runs of 32 columns, whose rows are half a line, loaded 15 % slower).  Where a lane's rows start is settled once,

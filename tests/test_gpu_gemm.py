@@ -452,3 +452,23 @@ def test_narrow_matrix_under_many_rows_split_over_k(hip, monkeypatch, M, N, K, N
         assert rel_l2(got1[m], want[m]) < TOL_Q4 and rel_l2(got0[m], want[m]) < TOL_Q4, m
     assert rel_l2(got1, got0) < 1e-5
     assert l1 == l0 + 1, (l1, l0)        # the launch that adds the shares
+
+
+@pytest.mark.parametrize("M,N,K,base", [(1000, 3201, 128, 0), (777, 4100, 256, 64), (2049, 1537, 384, 32), (65, 4100, 4096, 0), (97, 1152, 6912, 128),
+                                        (341, 13824, 1152, 0), (33, 4100, 4096, 32), (64, 1153, 6912, 0), (130, 515, 14336, 0)])
+def test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base):
+    """The tiles of the many-row matmul and its shares of K at ragged ends: rows and weight rows past the last tile, shares of
+    unequal length, fewer steps of K than the ring has stages, weights that begin at an odd block."""
+    note(f"gemm q4 ring M={M} N={N} K={K} base={base}")
+    rng = np.random.default_rng(M + N)
+    qt = quant.quantize_q4_0(rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05))
+    x = rng.standard_normal((M, K), dtype=np.float32) * np.exp(rng.standard_normal((M, 1))).astype(np.float32)
+    load_qtensor(hip, 1, qt, offset=base, total=base + qt.size)
+    f32map(hip, 0, M * K + M * N + N, x.reshape(-1))
+    hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [base]), up(hip, [M * K]), M, K, N, 1)
+    got = read(hip, 0, M * K, M * N + N)
+    want = x.astype(np.float64) @ qt.dequant().astype(np.float64).T
+    for m in range(0, M, max(1, M // 64)):
+        assert rel_l2(got[m * N:(m + 1) * N], want[m]) < TOL_Q4, m
+    assert rel_l2(got[(M - 1) * N:M * N], want[M - 1]) < TOL_Q4 and rel_l2(got[:M * N], want.reshape(-1)) < TOL_Q4
+    assert not got[M * N:].any()                   # nothing beyond the last row
