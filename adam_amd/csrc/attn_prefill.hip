@@ -299,7 +299,8 @@ template <int D, bool CAP, int WPH>
 __global__ void __launch_bounds__(256 * WPH)
 k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt, const uint4* __restrict__ vt,
                     const AttpBases bs, const AttpVt gv, uint32_t H, uint32_t n_quads, uint32_t n_ttiles, uint32_t m,
-                    uint32_t seq0, uint32_t q_stride, uint32_t o_stride, float scale, float cap, uint32_t vt_tiles) {
+                    uint32_t seq0, uint32_t q_stride, uint32_t o_stride, float scale, float cap, uint32_t vt_tiles,
+                    uint32_t splits, float* __restrict__ part) {
   constexpr int KS = D / 32;           // 32-dim steps of the score product
   constexpr int NB = D / 16;           // 16-dim blocks of the output
   const uint32_t lane = threadIdx.x & 63u;
@@ -313,12 +314,16 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
   const bool live = head_raw < H;
   if (WPH == 1 && !live) return;       // (no barrier in the one-wave form)
   const uint32_t head = min(head_raw, H - 1u);
-  const uint32_t t0 = (n_ttiles - 1u - blockIdx.x / n_quads) * 16u;
+  // splits > 1 (few heads, few tokens: most CUs would have no workgroup): a workgroup takes one of `splits` runs of the
+  // tile's keys and leaves its running state in part, for k_attn_prefill_join
+  const uint32_t job = blockIdx.x / n_quads, split = job % splits;
+  const uint32_t t0 = (n_ttiles - 1u - job / splits) * 16u;
   const uint32_t rows = min(16u, m - t0);
   const uint32_t nkeys = seq0 + t0 + rows - 1u;          // cache rows the tile's last query sees
   const uint32_t n_tiles = (nkeys + 31u) >> 5;
-  const uint32_t t_split = WPH == 2 ? (n_tiles + 1u) >> 1 : n_tiles;
-  const uint32_t T_lo = !live ? 0u : half ? t_split : 0u, T_hi = !live ? 0u : half ? n_tiles : t_split;
+  const uint32_t per = (n_tiles + splits - 1u) / splits, T0 = min(split * per, n_tiles), T1 = min(T0 + per, n_tiles);
+  const uint32_t t_split = WPH == 2 ? T0 + ((T1 - T0 + 1u) >> 1) : T1;
+  const uint32_t T_lo = !live ? 0u : half ? t_split : T0, T_hi = !live ? 0u : half ? T1 : t_split;
   const uint4* kbase = kt + (uint64_t)gv.grp[head] * vt_tiles * (2u * KS * 64u) + lane;
   const uint4* vbase = vt + (uint64_t)gv.grp[head] * vt_tiles * (NB * 64u) + g * 16u + n;
 
@@ -476,6 +481,7 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
     const float mm = fmaxf(m_run, m1);
     const float f0 = __builtin_amdgcn_exp2f(m_run - mm), f1 = __builtin_amdgcn_exp2f(m1 - mm);
     l_run = l_run * f0 + l1 * f1;
+    m_run = mm;
     float g0[4], g1[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) { g0[r] = __shfl(f0, (int)(4u * g + r), 64); g1[r] = __shfl(f1, (int)(4u * g + r), 64); }
@@ -487,6 +493,19 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
 
   float l_tot = l_run + __shfl_xor(l_run, 16, 64);
   l_tot += __shfl_xor(l_tot, 32, 64);
+  if (splits > 1u) {
+    const uint64_t row0 = ((uint64_t)split * H + head) * m + t0;      // [run of keys][head][token]
+    float* const pa = part + 2ull * splits * H * m;                   // (maximum, sum) of all rows, then their values
+    if (g == 0 && n < rows) { part[2 * (row0 + n)] = m_run; part[2 * (row0 + n) + 1] = l_tot; }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      if (4u * g + r >= rows) continue;
+      float* dst = pa + (row0 + 4u * g + r) * D + n;
+#pragma unroll
+      for (int b = 0; b < NB; b++) dst[16 * b] = acc[b][r];
+    }
+    return;
+  }
   const float inv_l = 1.0f / l_tot;
   float il[4];
 #pragma unroll
@@ -499,6 +518,34 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
 #pragma unroll
     for (int b = 0; b < NB; b++) dst[16 * b] = acc[b][r] * il[r];
   }
+}
+
+// The runs of keys of a split launch, brought to their common maximum and added up in order (a run that a query sees
+// nothing of has the maximum -1e30: its factor is exactly 0).  Four values per thread, a row of the grid per token.
+__global__ void __launch_bounds__(256)
+k_attn_prefill_join(const float* __restrict__ part, float* out, const AttpBases bs, uint32_t H, uint32_t D, uint32_t m, uint32_t splits,
+                    uint32_t o_stride) {
+  const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * 4u, t = blockIdx.y;
+  if (i >= H * D) return;
+  const uint32_t head = i / D, d = i % D;
+  const float* const pa = part + 2ull * splits * H * m;
+  float M = ATTP_NEG;
+  for (uint32_t s = 0; s < splits; s++) M = fmaxf(M, part[2 * (((uint64_t)s * H + head) * m + t)]);
+  float L = 0.f;
+  f4p_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (uint32_t s = 0; s < splits; s++) {
+    const uint64_t row = ((uint64_t)s * H + head) * m + t;
+    const float f = __builtin_amdgcn_exp2f(part[2 * row] - M);
+    const f4p_t v = *(const f4p_t*)(pa + row * D + d);
+    L = fmaf(part[2 * row + 1], f, L);
+#pragma unroll
+    for (int k = 0; k < 4; k++) o[k] = fmaf(v[k], f, o[k]);
+  }
+  float* dst = out + (uint64_t)bs.o[head] + (uint64_t)t * o_stride + d;
+  const float il = 1.0f / L;
+#pragma unroll
+  for (int k = 0; k < 4; k++) dst[k] = o[k] * il;
 }
 
 // transposed V tiles of the chunk launches: grown on demand, released at shutdown
@@ -576,11 +623,15 @@ size_t launch_attn_chunk(const std::vector<PendOp>& q, size_t i, int* rc) {
   for (uint32_t h = 0; h < H; h++) { bs.q[h] = q0[h]; bs.sc[h] = sc[h]; bs.o[h] = o0[h]; bs.kb[h] = kb[h]; bs.vb[h] = vb[h]; }
   float* d = (float*)mp->buf;
   // Both products on the matrix cores (a wave per head and 16-token tile) when that gives at least half the CUs a
-  // workgroup; a chunk with few heads or few tokens (Gemma-3-1B: 4 heads, 32 workgroups for 512 tokens) spreads wider on
-  // the kernel above, whose workgroups are one head each and split the cache between their waves.
-  // ADAMAH_ATTN_PREFILL_MFMA: 0 never, 1 by that rule (default), 2 always.
+  // workgroup; with few heads or few tokens, over runs of keys that give them one, where there are keys enough to pay for
+  // the launches that arrange the keys and join the runs (about 15 us; the kernel above walks 64 or, at a head size of 256,
+  // 32 keys in 2.8 and 5.6 us): 24 tokens of 32 heads of 128 over 4000 keys 175 -> 27 us, 17 tokens of 4 heads of 256 over
+  // 529 keys 93 -> 25 us.
+  // ADAMAH_ATTN_PREFILL_MFMA: 0 never, 1 by that rule (default), 2 always (in one run).
   const int mfma_mode = tuning("ADAMAH_ATTN_PREFILL_MFMA", 1);
-  if (mfma_mode == 2 || (mfma_mode == 1 && cdiv(H, 4u) * cdiv(m, 16u) * 2u >= (uint32_t)g.n_cu)) {
+  const uint32_t quads_tiles = cdiv(H, 4u) * cdiv(m, 16u);
+  const bool few = quads_tiles * 2u < (uint32_t)g.n_cu;
+  if (mfma_mode == 2 || (mfma_mode == 1 && (!few || seq_last >= (D == 64 ? 640u : D == 128 ? 384u : 96u)))) {
     // the visible V rows of every KV head transposed into tiles first
     AttpVt gv; AttpVtSrc src;
     uint32_t n_grp = 0;
@@ -592,7 +643,8 @@ size_t launch_attn_chunk(const std::vector<PendOp>& q, size_t i, int* rc) {
     }
     const uint32_t tiles = cdiv(seq_last, 32u);
     const size_t plane = (size_t)n_grp * tiles * 32u * D * sizeof(__half);   // V tiles, then K tiles
-    const size_t need = 2 * plane;
+    const uint32_t splits = few && mfma_mode == 1 ? std::max(1u, std::min((uint32_t)g.n_cu / quads_tiles, tiles / 2u)) : 1u;
+    const size_t need = 2 * plane + (splits > 1 ? (size_t)splits * H * m * (D + 2) * sizeof(float) : 0);
     bool ok = true;
     if (need > g_vt_bytes) {
       hipStreamSynchronize(g.stream);
@@ -606,14 +658,15 @@ size_t launch_attn_chunk(const std::vector<PendOp>& q, size_t i, int* rc) {
     if (ok) {
       const uint32_t n_quads = cdiv(H, 4u), n_tt = cdiv(m, 16u);
       uint4* const g_kt = (uint4*)((char*)g_vt + plane);
+      float* const part = (float*)((char*)g_vt + 2 * plane);
       // two waves per head where the launch has at most one workgroup per CU (ADAMAH_ATTN_PREFILL_WPH: 1 / 2 force)
       const int wph_mode = tuning("ADAMAH_ATTN_PREFILL_WPH", 0);
-      const int wph = wph_mode == 1 || wph_mode == 2 ? wph_mode : (n_quads * n_tt <= (uint32_t)g.n_cu ? 2 : 1);
-#define APM_ARGS d, d, g_kt, g_vt, bs, gv, H, n_quads, n_tt, m, s0.n, qs, os, a0.eps, a0.f2, tiles
+      const int wph = wph_mode == 1 || wph_mode == 2 ? wph_mode : (n_quads * n_tt * splits <= (uint32_t)g.n_cu ? 2 : 1);
+#define APM_ARGS d, d, g_kt, g_vt, bs, gv, H, n_quads, n_tt, m, s0.n, qs, os, a0.eps, a0.f2, tiles, splits, part
 #define APM(DD)                                                                                                   \
   do {                                                                                                            \
     k_kv_tile_arrange<DD><<<dim3(tiles, n_grp), 256, 0, g.stream>>>(mp->kv16, mp->kv_start, src, seq_last, tiles, g_vt, g_kt); \
-    const dim3 gr_(n_quads * n_tt);                                                                               \
+    const dim3 gr_(n_quads * n_tt * splits);                                                                               \
     if (wph == 2 && DD <= 128) {   /* (D = 256 needs more registers than two waves per SIMD have) */              \
       constexpr int D2_ = DD <= 128 ? DD : 128;                                                                   \
       if (a0.f2 > 0.0f) k_attn_prefill_mfma<D2_, true, 2><<<gr_, 512, 0, g.stream>>>(APM_ARGS);                  \
@@ -626,7 +679,8 @@ size_t launch_attn_chunk(const std::vector<PendOp>& q, size_t i, int* rc) {
       if (D == 64) APM(64); else if (D == 128) APM(128); else APM(256);
 #undef APM
 #undef APM_ARGS
-      count_launch(2);
+      if (splits > 1) k_attn_prefill_join<<<dim3(cdiv(H * D, 1024u), m), 256, 0, g.stream>>>(part, d, bs, H, D, m, splits, os);
+      count_launch(splits > 1 ? 3 : 2);
       *rc = check_launch();
       return 2 * (size_t)m;
     }

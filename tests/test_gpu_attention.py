@@ -184,6 +184,33 @@ def test_prefill_chunk_is_one_causal_launch(hip, chunk_impl, m, seq0, Hq, Hkv, d
     assert rel_l2(scores, ref_scores) < 1e-5
 
 
+@pytest.mark.parametrize("m,seq0,Hq,Hkv,d,softcap,gap", [
+    (24, 4001, 32, 8, 128, 0.0, 0), (17, 513, 4, 1, 256, 50.0, 0), (33, 700, 6, 3, 64, 30.0, 8), (40, 1200, 3, 1, 128, 0.0, 0),
+    (2, 383, 1, 1, 128, 0.0, 1), (16, 97, 4, 4, 256, 0.0, 0), (100, 650, 5, 1, 64, 0.0, 0), (3, 9000, 2, 1, 128, 0.0, 0)])
+def test_prefill_chunk_over_runs_of_keys(hip, m, seq0, Hq, Hkv, d, softcap, gap):
+    """Few heads and tokens behind many keys: runs of keys on workgroups of their own, joined by a third launch.  Against
+    float64 over the same fp16 keys and values; the products take queries and weights as exact two-term sums, so what is
+    left are float32 sums and exponentials (a few 2^-22 of scores of a few units): 4e-6."""
+    rng = np.random.default_rng(m * 1000 + seq0)
+    cap_len = seq0 + m + 7
+    q = rng.standard_normal((m, Hq, d)).astype(np.float32)
+    K, V = (rng.standard_normal((Hkv, cap_len, d)).astype(np.float32) for _ in range(2))
+    scale = float(1.0 / np.sqrt(d))
+    note(f"attention chunk over runs m={m} seq0={seq0} {Hq}q/{Hkv}kv d={d}")
+    out, scores, launches = chunk_case(hip, q, K, V, seq0, cap_len, scale, softcap, gap)
+    assert launches == 3
+    K16, V16 = (x.astype(np.float16).astype(np.float64) for x in (K, V))
+    for t in range(m):
+        for h in range(Hq):
+            raw = K16[h // (Hq // Hkv), :seq0 + t] @ q[t, h].astype(np.float64)
+            s = raw * scale
+            s = softcap * np.tanh(s / softcap) if softcap else s
+            p = np.exp(s - s.max())
+            assert rel_l2(out[t, h], p / p.sum() @ V16[h // (Hq // Hkv), :seq0 + t]) < 4e-6, (t, h)
+            if t == m - 1:
+                assert rel_l2(scores[h], raw) < 1e-5
+
+
 def test_causal_rows_entry_point_equals_the_pairs_issued_one_by_one(hip, chunk_impl):
     """adamah_attn_causal_rows_dev (an extension: m pairs in one native call) leaves the words the 2 m calls
     leave, in as many launches; the oracle's form of it agrees within the attention bar; bad arguments fail."""
