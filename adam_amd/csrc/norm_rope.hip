@@ -492,6 +492,11 @@ int adamah_qk_norm_rope_rows_dev(uint32_t map_act, uint32_t map_wt, const uint32
                                  uint32_t pos0, float freq_base) {
   if (m == 0) return ADAMAH_OK;
   if (!q_src_handles || !k_src_handles || !dst_handles) return ADAMAH_ERR_INVALID;
+  int rc = ADAMAH_OK;
+  Map* ma = get_f32_map(map_act);
+  if (ma && map_act == map_wt && launch_qk_rows(ma, q_src_handles, locs_q_wt, k_src_handles, locs_k_wt, dst_handles, m, q_rows, q_dim, k_rows,
+                                                k_dim, pos0, freq_base, &rc))
+    return rc;
   for (uint32_t t = 0; t < m; t++) {
     const int r = map_qk_norm_rope_x_dev(map_act, map_wt, q_src_handles[t], locs_q_wt, k_src_handles[t], locs_k_wt,
                                          dst_handles[t], q_rows, q_dim, k_rows, k_dim, pos0 + t, freq_base);

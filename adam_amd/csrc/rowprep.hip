@@ -35,10 +35,8 @@ __device__ __forceinline__ void store_row_elem(float* act, __half* kv16, uint64_
 }
 
 // One 256-thread workgroup per task, as the stand-alone kernels have per row.
-__global__ void __launch_bounds__(256)
-k_row_tasks(float* act, const RowTasks ts, __half* kv16, uint64_t kv_start, uint64_t kv_count) {
+__device__ __forceinline__ void run_row_task(float* act, const RowTask& t, __half* kv16, uint64_t kv_start, uint64_t kv_count) {
   __shared__ float sh[4];
-  const RowTask t = ts.t[blockIdx.x];
   const uint32_t tid = threadIdx.x, dim = t.dim, half = dim >> 1;
   float inv = 1.f;
   if (t.flags & 1u) {
@@ -70,6 +68,63 @@ k_row_tasks(float* act, const RowTasks ts, __half* kv16, uint64_t kv_start, uint
       store_row_elem(act, kv16, kv_start, kv_count, t.dst, t.cache, i, y);
     }
   }
+}
+__global__ void __launch_bounds__(256)
+k_row_tasks(float* act, const RowTasks ts, __half* kv16, uint64_t kv_start, uint64_t kv_count) {
+  run_row_task(act, ts.t[blockIdx.x], kv16, kv_start, kv_count);
+}
+
+// Norm and rotation of all heads of m consecutive tokens, a workgroup per row and token: the rows of a token lie q_step /
+// k_step / dst_step elements behind those of the token before.  (As row tasks, 60 to a launch, 512 tokens of 5 heads took
+// 43 launches of 4 us and the host longer than that to issue them; 10 us as one.)
+#define QKROWS_MAX 64u
+struct QkRows { uint32_t src[QKROWS_MAX], w[QKROWS_MAX], q_rows, q_dim, k_dim, q_step, k_step, dst, dst_step, pos0; float base; };
+__global__ void __launch_bounds__(256)
+k_qk_norm_rope_rows(float* act, const QkRows r) {
+  const uint32_t row = blockIdx.x, t = blockIdx.y;
+  const bool q = row < r.q_rows;
+  run_row_task(act, {r.src[row] + t * (q ? r.q_step : r.k_step), r.dst + t * r.dst_step + (q ? row * r.q_dim : r.q_rows * r.q_dim + (row - r.q_rows) * r.k_dim),
+                     ROWT_NONE, r.w[row], q ? r.q_dim : r.k_dim, r.pos0 + t, 3u, r.base}, nullptr, 0, 0);
+}
+
+// The m (Q rows, K rows, destination) lists as one launch: false where a list is not known on the host or steps by another
+// stride from some token to the next, where a token's result would land on what another one reads or writes, or where the
+// rows fit a run of row tasks (which the copies behind them join).
+bool launch_qk_rows(Map* m, const uint32_t* hq, uint32_t hqw, const uint32_t* hk, uint32_t hkw, const uint32_t* hd, uint32_t n_tok,
+                    uint32_t q_rows, uint32_t q_dim, uint32_t k_rows, uint32_t k_dim, uint32_t pos0, float base, int* rc) {
+  const uint64_t n = (uint64_t)q_rows + k_rows, width = (uint64_t)q_rows * q_dim + (uint64_t)k_rows * k_dim;
+  if (n_tok < 2 || n == 0 || n > QKROWS_MAX || n * n_tok <= ROWT_MAX || ((q_dim | k_dim) & 1u) || (q_rows && !q_dim) || (k_rows && !k_dim)) return false;
+  const uint32_t *wq = q_rows ? res_host(hqw, q_rows) : nullptr, *wk = k_rows ? res_host(hkw, k_rows) : nullptr;
+  if ((q_rows && !wq) || (k_rows && !wk)) return false;
+  QkRows r = {};
+  r.q_rows = q_rows; r.q_dim = q_dim; r.k_dim = k_dim; r.pos0 = pos0; r.base = base;
+  for (uint32_t t = 0; t < n_tok; t++) {
+    const uint32_t *q = q_rows ? res_host(hq[t], q_rows) : nullptr, *k = k_rows ? res_host(hk[t], k_rows) : nullptr, *d = res_host(hd[t], 1);
+    if (!d || (q_rows && !q) || (k_rows && !k)) return false;
+    if (t == 0) {
+      for (uint32_t i = 0; i < q_rows; i++) { r.src[i] = q[i]; r.w[i] = wq[i]; }
+      for (uint32_t i = 0; i < k_rows; i++) { r.src[q_rows + i] = k[i]; r.w[q_rows + i] = wk[i]; }
+      r.dst = d[0];
+    }
+    if (t == 1) {
+      if (d[0] < r.dst || (q_rows && q[0] < r.src[0]) || (k_rows && k[0] < r.src[q_rows])) return false;
+      r.dst_step = d[0] - r.dst; r.q_step = q_rows ? q[0] - r.src[0] : 0u; r.k_step = k_rows ? k[0] - r.src[q_rows] : 0u;
+    }
+    if ((uint64_t)d[0] != r.dst + (uint64_t)t * r.dst_step) return false;
+    for (uint32_t i = 0; i < q_rows; i++) if ((uint64_t)q[i] != r.src[i] + (uint64_t)t * r.q_step) return false;
+    for (uint32_t i = 0; i < k_rows; i++) if ((uint64_t)k[i] != r.src[q_rows + i] + (uint64_t)t * r.k_step) return false;
+  }
+  const uint64_t last = n_tok - 1, d0 = r.dst, d1 = d0 + last * r.dst_step + width;
+  if (r.dst_step < width || d1 > m->n_elems) return false;
+  for (uint32_t i = 0; i < n; i++) {
+    const uint64_t dim = i < q_rows ? q_dim : k_dim, s0 = r.src[i], s1 = s0 + last * (i < q_rows ? r.q_step : r.k_step) + dim, w0 = r.w[i], w1 = w0 + dim;
+    if (s1 > m->n_elems || w1 > m->n_elems || (s0 < d1 && d0 < s1) || (w0 < d1 && d0 < w1)) return false;
+  }
+  flush_pending();
+  k_qk_norm_rope_rows<<<dim3((uint32_t)n, n_tok), 256, 0, g.stream>>>((float*)m->buf, r);
+  count_launch();
+  *rc = check_launch();
+  return true;
 }
 
 static bool overlap(uint32_t a, uint32_t na, uint32_t b, uint32_t nb) {

@@ -142,6 +142,42 @@ def test_qk_norm_rope_rows_entry_point_equals_per_token_calls(hip):
         hip.qk_norm_rope_rows_dev(0, 0, [987654], 1, [987655], 1, [987656], Hq, D, Hk, D, pos0, 1e6)
 
 
+@pytest.mark.parametrize("m,Hq,Hk,D,case", [
+    (13, 4, 1, 256, "apart"), (64, 1, 0, 2, "apart"), (65, 1, 0, 2, "apart"), (2, 30, 20, 6, "apart"), (2, 40, 30, 6, "apart"),
+    (40, 3, 2, 64, "in place"), (40, 3, 2, 64, "one astray"), (33, 2, 2, 34, "backwards")])
+def test_qk_norm_rope_of_many_rows(hip, m, Hq, Hk, D, case):
+    """One launch for all tokens where the rows step evenly and clear of each other; where they do not (results over the
+    sources, a row elsewhere, results laid down in reverse) and where they fit one list of row tasks, token by token.  The
+    same words either way."""
+    n = Hq + Hk
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal(m * n * D + D).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, 2 * D).astype(np.float32)
+    w0, dst0 = x.size, x.size + 2 * D
+
+    def go(one_call):
+        f32map(hip, 0, dst0 + (m + 1) * n * D, np.concatenate([x, w]))
+        src = lambda t: t * n * D + (D if case == "one astray" and t == m // 2 else 0)
+        dst = lambda t: src(t) if case == "in place" else dst0 + (m - 1 - t if case == "backwards" else t) * n * D
+        qs = [up(hip, src(t) + np.arange(Hq) * D) for t in range(m)]
+        ks = [up(hip, src(t) + (Hq + np.arange(max(Hk, 1))) * D) for t in range(m)]
+        ds = [up(hip, [dst(t)]) for t in range(m)]
+        qw, kw = up(hip, [w0] * Hq), up(hip, [w0 + D] * max(Hk, 1))
+        hip.batch_begin()
+        if one_call:
+            hip.qk_norm_rope_rows_dev(0, 0, qs, qw, ks, kw, ds, Hq, D, Hk, D, 7, 1e4)
+        else:
+            for t in range(m):
+                hip.map_qk_norm_rope_x_dev(0, 0, qs[t], qw, ks[t], kw, ds[t], Hq, D, Hk, D, 7 + t, 1e4)
+        hip.batch_end()
+        return read(hip, 0, 0, dst0 + (m + 1) * n * D), hip.get_last_barrier_count()
+
+    note(f"qk_norm_rope of many rows m={m} {Hq}+{Hk}x{D} {case}")
+    (a, la), (b, _) = go(True), go(False)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert la == 1 or case != "apart" or n > 64
+
+
 def test_kv_append_rounds_to_fp16_and_mirrors(hip):
     Hkv, d, cap = 2, 64, 8
     rng = np.random.default_rng(6)
