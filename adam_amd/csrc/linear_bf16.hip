@@ -75,10 +75,11 @@ __device__ __forceinline__ void group_inverse(const LinSpec& s, float* inv, floa
   }
 }
 // f(x) of one row by a workgroup of NT threads; put(i, value) for i in [0, k_stride).  first: this workgroup also stores
-// what the spec wants kept.  inv: LDS, LIN_MAX_GROUPS floats, part: LDS, 2 NT / 64 floats.
-template <int NT, class Put>
-__device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32_t row, bool first, float* inv, float* part, Put put) {
-  const uint32_t tid = threadIdx.x;
+// what the spec wants kept.  put4(c, values): elements 4 c .. 4 c + 3.  inv: LDS, LIN_MAX_GROUPS floats, part: LDS, NT / 16
+// floats.
+template <int NT, class Put, class Put4>
+__device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32_t row, bool first, float* inv, float* part, Put put, Put4 put4) {
+  const uint32_t tid = threadIdx.x, gl = s.groups ? s.k / s.groups >> 2 : 64u;          // lanes (of four elements) a group has
   const float* x = act + s.src + (uint64_t)row * s.src_stride;
   float* keep = act + s.keep + (uint64_t)row * s.keep_stride;
   const bool kept = first && s.kept;
@@ -122,6 +123,80 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
       if (i < s.k) done(i, xv[j], nv[j]);
     }
     for (uint32_t i = tid + (uint32_t)R * NT; i < s.k; i += NT) done(i, sum_at(i), s.wt_len ? wt[i] : 0.f);
+  } else if (s.k <= 16u * NT && ((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) == 0u &&
+             (!s.gate_act || ((s.gate | s.gate_stride) & 3u) == 0u) && (!s.wt_len || ((s.wt | s.wt_len) & 3u) == 0u) &&
+             (!s.groups || ((s.k / s.groups & 3u) == 0u && ((gl & 63u) == 0u || (gl < 64u && (gl & (gl - 1u)) == 0u))))) {
+    // The row makes one trip: up to four times four elements a thread, everything asked for at once (twelve rows of 4096,
+    // one float a load and each pass waiting for the one before: 15.8 us; so: 5.0).  A group is a power of two of
+    // neighbouring lanes, or whole waves' worth, whose sums meet in LDS.
+    constexpr int R = 4, NW = NT / 64;
+    const uint32_t n4 = s.k >> 2, wave = tid >> 6;
+    const float* gt = act + s.gate + (uint64_t)row * s.gate_stride;
+    f4_t xv[R], gv[R], wv[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const uint32_t c = tid + (uint32_t)j * NT;
+      if (c >= n4) break;
+      xv[j] = *(const f4_t*)(x + 4u * c);
+      if (s.gate_act) gv[j] = *(const f4_t*)(gt + 4u * c);
+      if (s.wt_len) wv[j] = *(const f4_t*)(wt + (s.wt_len == s.k ? 4u * c : 4u * c % s.wt_len));
+    }
+    float ss[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const uint32_t c = tid + (uint32_t)j * NT;
+      ss[j] = 0.f;
+      if (c >= n4) continue;
+      if (s.gate_act == 3u)
+#pragma unroll
+        for (int e = 0; e < 4; e++) xv[j][e] *= silu_f(gv[j][e]);
+#pragma unroll
+      for (int e = 0; e < 4; e++) ss[j] = fmaf(xv[j][e], xv[j][e], ss[j]);
+    }
+    float scale[R];
+    if (s.groups) {
+      const float n = (float)(4u * gl);
+      if (gl < 64u) {
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+          if ((uint32_t)j * NT >= n4) break;
+          for (uint32_t o = gl >> 1; o > 0; o >>= 1) ss[j] += __shfl_xor(ss[j], (int)o, 64);
+          scale[j] = 1.0f / sqrtf(ss[j] / n + s.eps);
+        }
+      } else {
+        const uint32_t nb = gl >> 6;
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+          if ((uint32_t)j * NT >= n4) break;
+          const float t = wsum64(ss[j]);
+          if ((tid & 63u) == 0u) part[j * NW + wave] = t;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+          if (tid + (uint32_t)j * NT >= n4) break;
+          const uint32_t b0 = ((uint32_t)j * NW + wave) / nb * nb;
+          float t = 0.f;
+          for (uint32_t b = 0; b < nb; b++) t += part[b0 + b];
+          scale[j] = 1.0f / sqrtf(t / n + s.eps);
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const uint32_t c = tid + (uint32_t)j * NT;
+      if (c >= n4) break;
+      f4_t v = xv[j];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        if (s.groups) v[e] *= scale[j];
+        if (s.wt_len) v[e] *= s.wt_add + wv[j][e];
+        if (s.gate_act == 1u) v[e] *= sigmoid_f(gv[j][e]);
+        else if (s.gate_act == 2u) v[e] *= silu_f(gv[j][e]);
+      }
+      if (kept) *(f4_t*)(keep + 4u * c) = v;
+      put4(c, v);
+    }
   } else if (s.groups) {
     const uint32_t gs = s.k / s.groups;
     const float* gt = act + s.gate + (uint64_t)row * s.gate_stride;
@@ -146,13 +221,22 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
   for (uint32_t i = s.k + tid; i < s.k_stride; i += NT) put(i, 0.f);
 }
 
-template <class T>
-__global__ void __launch_bounds__(256)
+template <class T, int NT>
+__global__ void __launch_bounds__(NT)
 k_operand_rows(const LinSpec s, float* act, T* __restrict__ dst, const uint32_t* __restrict__ row_idx) {
   __shared__ float inv[LIN_MAX_GROUPS];
-  __shared__ float part[8];
+  __shared__ float part[NT / 16];
+  typedef T t4 __attribute__((ext_vector_type(4)));
   T* d = dst + (uint64_t)blockIdx.x * s.k_stride;
-  operand_row<256>(s, act, row_idx ? row_idx[blockIdx.x] : blockIdx.x, true, inv, part, [&](uint32_t i, float v) { d[i] = (T)v; });
+  operand_row<NT>(s, act, row_idx ? row_idx[blockIdx.x] : blockIdx.x, true, inv, part, [&](uint32_t i, float v) { d[i] = (T)v; },
+                  [&](uint32_t c, f4_t v) { *(t4*)(d + 4u * c) = (t4){(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; });
+}
+// Few rows: a row's latency is the launch's, so 1024 threads a row; many rows fill the CUs with 256 each.
+template <class T>
+static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* row_idx, uint32_t rows) {
+  if (rows <= 2u * (uint32_t)g.n_cu) k_operand_rows<T, 1024><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
+  else k_operand_rows<T, 256><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
+  count_launch();
 }
 
 // ---- one row ------------------------------------------------------------------------------------------------------
@@ -166,7 +250,7 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
             float* best_val, uint32_t* best_idx) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ float inv[LIN_MAX_GROUPS];
-  __shared__ float part[16];
+  __shared__ float part[32];
   __shared__ float bv[8];
   __shared__ uint32_t bi[8];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, kp = s.k_stride, half = kp >> 1;
@@ -189,7 +273,8 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
   rows_of(min(task, n_tasks - 1u), r0, r1);
   fetch(r0, r1, k0);
   operand_row<512>(s, act, row_idx ? row_idx[0] : 0u, blockIdx.x == 0u, inv, part,
-                   [&](uint32_t i, float v) { xs[((i >> 2) & 1u) * half + (i >> 3) * 4u + (i & 3u)] = v; });
+                   [&](uint32_t i, float v) { xs[((i >> 2) & 1u) * half + (i >> 3) * 4u + (i & 3u)] = v; },
+                   [&](uint32_t c, f4_t v) { *(f4_t*)(xs + (c & 1u) * half + (c >> 1) * 4u) = v; });
   __syncthreads();
   float top = NEG_MAX_F, a0 = 0.f, a1 = 0.f;
   uint32_t top_i = 0xFFFFFFFFu;
@@ -511,14 +596,14 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   const bf16_t* W = (const bf16_t*)mw->buf + s.w;
   if (mo->dtype == DTYPE_F32) {
     float* op = (float*)mo->buf;
-    if (!s.ready) { k_operand_rows<float><<<rows, 256, 0, g.stream>>>(s, act, op + s.opnd, row_idx); count_launch(); }
+    if (!s.ready) operand_rows<float>(s, act, op + s.opnd, row_idx, rows);
     k_linear_f32<<<dim3(cdiv(s.n, 64), cdiv(rows, 64)), 256, 0, g.stream>>>(W, op + s.opnd, act, op, s, rows);
     count_launch();
     return check_launch();
   }
   bf16_t* op = (bf16_t*)mo->buf;
   const bf16_t* X = op + s.opnd;
-  if (!s.ready) { k_operand_rows<bf16_t><<<rows, 256, 0, g.stream>>>(s, act, op + s.opnd, row_idx); count_launch(); }
+  if (!s.ready) operand_rows<bf16_t>(s, act, op + s.opnd, row_idx, rows);
   if (rows <= 16) k_linear_skinny<1><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows);
   else if (rows <= 32) k_linear_skinny<2><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows);
   else {

@@ -94,6 +94,30 @@ def test_linear_tiles(hip, rows, n, k, biased, add):
     assert np.array_equal(got[:rows, n:], old[:rows, n:]) and np.array_equal(got[rows], old[rows])       # nothing beyond
 
 
+@pytest.mark.parametrize("rows,k,groups,act,per_group", [
+    (1, 2048, 1, 1, 0), (1, 8192, 32, 2, 1), (2, 8196, 1, 0, 0), (3, 4096, 64, 3, 1), (3, 16384, 16, 1, 0), (2, 16640, 1, 2, 0), (5, 768, 3, 3, 0),
+    (5, 768, 1, 0, 1), (7, 256, 64, 1, 1), (4, 1200, 25, 2, 0), (530, 4096, 4, 1, 1), (520, 4352, 1, 3, 0), (515, 36, 0, 0, 0)])
+def test_operand_rows_in_one_trip(hip, rows, k, groups, act, per_group):
+    """Rows and groups that a workgroup's registers hold (and just do not), groups of lanes and of waves, every gate."""
+    note(f"operand rows {rows} k {k} groups {groups} act {act}")
+    rng = np.random.default_rng(k + rows)
+    n, ks = 40, (k + 63) // 64 * 64
+    wt_len = 0 if not groups else k // groups if per_group else k
+    gate, wt, keep = rows * k, 2 * rows * k, 2 * rows * k + k
+    out = keep + rows * k
+    p = Pair(hip, out + rows * n + 64, wt=n * ks, opnd=rows * ks, dtype="float32")
+    W = np.zeros((n, ks), np.uint16)
+    W[:, :k] = f32_to_bf16((rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32))
+    p.put(WT, 0, W)
+    p.put(WS, 0, rng.standard_normal(keep))
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=ks, src=0, src_stride=k, groups=groups, eps=1e-4, wt=wt, wt_len=wt_len, wt_add=0.5, gate=gate,
+                        gate_stride=k, gate_act=act if groups else 0, opnd=0, ready=0, keep=keep, keep_stride=k, kept=1, out=out, out_stride=n)
+    p.call("linear_dev", WS, OP, WT, p.up(spec.words()), 0, rows)
+    # float32 throughout; a group's sum of at most 16640 squares: 2e-5 as for every operand above
+    p.same(WS, keep, rows * k, 2e-5, "operand")
+    p.same(WS, out, rows * n, 2e-5, "out")
+
+
 @pytest.mark.parametrize("rows", [1, 3])
 def test_linear_argmax_takes_the_first_of_equals(hip, rows):
     note(f"linear argmax rows {rows}")
