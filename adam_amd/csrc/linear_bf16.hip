@@ -422,54 +422,72 @@ __device__ __forceinline__ void put_pair_or_tail(const LinSpec& s, float* act, T
 }
 
 // ---- 2 .. 32 rows -------------------------------------------------------------------------------------------------
-// A workgroup owns 32 matrix rows; its 8 waves take 32-column steps of K in turn and add up through LDS.
-template <int MT>
-__global__ void __launch_bounds__(512)
+// Bound by the weights' way in.  A workgroup owns 16 NB matrix rows; its NW waves take 64-column steps of K (a whole line of
+// a row) in turn, two of them in flight, and add up through LDS.  12 rows, 4096 x 14336 (117 MB): 57 us with half the CUs
+// at work, half lines and few loads in flight, 26.8 now (4.4 TB/s); 28672 x 4096 (235 MB): 60.4 and 52.5; 24 rows: 68 and
+// 37, 72 and 64.
+template <int MT, int NB, int NW>
+__global__ void __launch_bounds__(64 * NW)
 k_linear_skinny(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, bf16_t* opnd, const LinSpec s, uint32_t rows) {
-  __shared__ f4_t red[8][2 * MT][64];
+  __shared__ f4_t red[NW][NB * MT][64];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, c = lane & 15u, kg = lane >> 4, kp = s.k_stride;
-  const uint32_t n0 = blockIdx.x * 32u;
-  const bf16_t* wa = W + (uint64_t)min(n0 + c, s.n - 1u) * kp + kg * 8u;
-  const bf16_t* wb = W + (uint64_t)min(n0 + 16u + c, s.n - 1u) * kp + kg * 8u;
-  const bf16_t* xr[MT];
+  const uint32_t n0 = blockIdx.x * (16u * NB);
+  const bf16_t *wr[NB], *xr[MT];
+#pragma unroll
+  for (int i = 0; i < NB; i++) wr[i] = W + (uint64_t)min(n0 + 16u * i + c, s.n - 1u) * kp + kg * 8u;
 #pragma unroll
   for (int m = 0; m < MT; m++) xr[m] = X + (uint64_t)min(16u * m + c, rows - 1u) * kp + kg * 8u;
-  f4_t acc[2][MT];
+  f4_t acc[NB][MT];
 #pragma unroll
-  for (int m = 0; m < MT; m++) { acc[0][m] = (f4_t){0, 0, 0, 0}; acc[1][m] = (f4_t){0, 0, 0, 0}; }
-  constexpr int UN = 4;                                // K steps in flight
-  for (uint32_t k0 = wave * 32u; k0 < kp; k0 += 256u * UN) {
-    bf8_t a[UN], b[UN], x[UN][MT];
+  for (int i = 0; i < NB; i++)
 #pragma unroll
-    for (int u = 0; u < UN; u++) {
-      const uint32_t k = min(k0 + 256u * u, kp - 32u);
-      a[u] = *(const bf8_t*)(wa + k); b[u] = *(const bf8_t*)(wb + k);
+    for (int m = 0; m < MT; m++) acc[i][m] = (f4_t){0, 0, 0, 0};
+  uint32_t k = wave * 64u;
+  const auto steps = [&](auto n) {
+    constexpr int U = decltype(n)::value;
+    bf8_t w[U][2][NB], x[U][2][MT];
 #pragma unroll
-      for (int m = 0; m < MT; m++) x[u][m] = *(const bf8_t*)(xr[m] + k);
-    }
+    for (int u = 0; u < U; u++)
 #pragma unroll
-    for (int u = 0; u < UN; u++) {
-      if (k0 + 256u * u >= kp) break;
+      for (int h = 0; h < 2; h++) {
 #pragma unroll
-      for (int m = 0; m < MT; m++) {
-        acc[0][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], x[u][m], acc[0][m], 0, 0, 0);
-        acc[1][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u], x[u][m], acc[1][m], 0, 0, 0);
+        for (int i = 0; i < NB; i++) w[u][h][i] = *(const bf8_t*)(wr[i] + k + 64 * NW * u + 32 * h);
+#pragma unroll
+        for (int m = 0; m < MT; m++) x[u][h][m] = *(const bf8_t*)(xr[m] + k + 64 * NW * u + 32 * h);
       }
-    }
-  }
+    __builtin_amdgcn_sched_barrier(0);                 // all asked for before the first is waited for
 #pragma unroll
-  for (int m = 0; m < MT; m++) { red[wave][m][lane] = acc[0][m]; red[wave][MT + m][lane] = acc[1][m]; }
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+          for (int i = 0; i < NB; i++) acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][h][i], x[u][h][m], acc[i][m], 0, 0, 0);
+    k += 64u * NW * U;
+  };
+  while (k + 64u * NW < kp) steps(std::integral_constant<int, 2>{});
+  if (k < kp) steps(std::integral_constant<int, 1>{});
+#pragma unroll
+  for (int i = 0; i < NB; i++)
+#pragma unroll
+    for (int m = 0; m < MT; m++) red[wave][i * MT + m][lane] = acc[i][m];
   __syncthreads();
+  const auto sum = [&](uint32_t t) {
+    f4_t v = red[0][t][lane];
+#pragma unroll
+    for (int w = 1; w < NW; w++) v += red[w][t][lane];
+    return v;
+  };
   if (s.epi == 2u) {
-    if (wave < MT) {
-      f4_t gt = red[0][wave][lane], up = red[0][MT + wave][lane];
-      for (int w = 1; w < 8; w++) { gt += red[w][wave][lane]; up += red[w][MT + wave][lane]; }
-      const uint32_t row = 16u * wave + c;
-      if (row < rows) put_pair_or_tail(s, act, opnd, row, n0 + 4u * kg, gt, up);
-    }
-  } else if (wave < 2 * MT) {
-    f4_t v = red[0][wave][lane];
-    for (int w = 1; w < 8; w++) v += red[w][wave][lane];
+    if constexpr (NB == 2)
+      if (wave < MT) {
+        const f4_t gt = sum(wave), up = sum(MT + wave);
+        const uint32_t row = 16u * wave + c;
+        if (row < rows) put_pair_or_tail(s, act, opnd, row, n0 + 4u * kg, gt, up);
+      }
+  } else if (wave < NB * MT) {
+    const f4_t v = sum(wave);
     const uint32_t row = 16u * (wave % MT) + c;
     if (row < rows) put_out(s, act, row, n0 + 16u * (wave / MT) + 4u * kg, v);
   }
@@ -604,8 +622,14 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   bf16_t* op = (bf16_t*)mo->buf;
   const bf16_t* X = op + s.opnd;
   if (!s.ready) operand_rows<bf16_t>(s, act, op + s.opnd, row_idx, rows);
-  if (rows <= 16) k_linear_skinny<1><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows);
-  else if (rows <= 32) k_linear_skinny<2><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows);
+  if (rows <= 32) {
+    // Workgroups of 16 matrix rows as long as no CU gets a second one (12 rows, 4096 x 4096: 9.6 us, of 32: 13.4; 7168 x
+    // 2048: 9.2 to 10.0 and 8.2 to 8.9).
+#define LS(MT) do { if (s.epi != 2u && cdiv(s.n, 16) <= (uint32_t)g.n_cu) k_linear_skinny<MT, 1, 16><<<cdiv(s.n, 16), 1024, 0, g.stream>>>(W, X, act, op, s, rows); \
+      else k_linear_skinny<MT, 2, 8><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows); } while (0)
+    if (rows <= 16) LS(1); else LS(2);
+#undef LS
+  }
   else {
     // The tile that gets through the rows soonest: rounds over the CUs times what a step of 64 columns takes there
     // (1/100 us, measured with all CUs at work on 2048 x 28672 x 4096, 600 x 12672 x 4096, 300 x 10304 x 2048 and
