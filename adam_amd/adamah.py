@@ -170,6 +170,8 @@ _SIGS = {
     "adamah_linear_dev": (i32, [_U] * 6), "adamah_linear_argmax_dev": (i32, [_U] * 6), "adamah_merge_norm_dev": (i32, [_U] * 3),
     "adamah_delta_rule_dev": (i32, [_U] * 10), "adamah_retention_dev": (i32, [_U] * 6),
     "adamah_chunk_attention_dev": (i32, [_U] * 6), "adamah_window_attention_dev": (i32, [_U] * 6),
+    "adamah_hip_delta_rule_seqs_dev": (i32, [_U] * 10), "adamah_hip_retention_seqs_dev": (i32, [_U] * 6),
+    "adamah_hip_chunk_attention_seqs_dev": (i32, [_U] * 6),
     "adamah_state_space_dev": (i32, [_U] * 6), "adamah_experts_dev": (i32, [_U] * 6),
     "adamah_hip_embed_bigram_dev": (i32, [_U] * 8 + [pu32]),
     # timing helpers for benchmarks (HIP events on the library's own stream)
@@ -764,6 +766,17 @@ class Adamah:
 
     def chunk_attention_dev(self, map_act, spec_handle, n_seq, rows, seq0, pos):
         self._op("adamah_chunk_attention_dev", map_act, spec_handle, n_seq, rows, seq0, pos)
+
+    def delta_rule_seqs_dev(self, map_act, map_opnd, map_wt, spec_handle, decay_handle, gate_handle, n_seq, rows, seq0, pos):
+        """A portion of `rows` tokens of each of n_seq sequences, one behind the other in the activation rows."""
+        self._op("adamah_hip_delta_rule_seqs_dev", map_act, map_opnd, map_wt, spec_handle, decay_handle, gate_handle, n_seq, rows,
+                 seq0, pos)
+
+    def retention_seqs_dev(self, map_act, spec_handle, n_seq, rows, seq0, pos):
+        self._op("adamah_hip_retention_seqs_dev", map_act, spec_handle, n_seq, rows, seq0, pos)
+
+    def chunk_attention_seqs_dev(self, map_act, spec_handle, n_seq, rows, seq0, pos):
+        self._op("adamah_hip_chunk_attention_seqs_dev", map_act, spec_handle, n_seq, rows, seq0, pos)
 
     def window_attention_dev(self, map_act, spec_handle, n_seq, rows, seq0, pos):
         self._op("adamah_window_attention_dev", map_act, spec_handle, n_seq, rows, seq0, pos)

@@ -632,14 +632,14 @@ static int run_step(const ASpec& s, float* act, T* cache, uint32_t n_seq, uint32
 #undef STEP
 }
 
-// Ranges and sizes, then one token of each of n_seq sequences or a portion of one.
+// Ranges and sizes, then one token of each of n_seq sequences or a portion of each, one sequence behind the other.
 template <bool WIN>
 static int run_attention(Map* ma, const ASpec& s, uint32_t cache_map, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) {
   Map* mc = get_map(cache_map);
   if (!mc || (mc->dtype != DTYPE_F32 && mc->dtype != DTYPE_BF16)) return ADAMAH_ERR_INVALID;
   const uint64_t D = s.dim, V = s.vdim, H = s.heads, G = s.kv_heads, C = s.size, n_tok = (uint64_t)n_seq * rows;
   const uint64_t D8 = (D + 7) / 8 * 8, V8 = (V + 7) / 8 * 8;
-  if (D == 0 || D > 256 || V == 0 || V > 256 || H == 0 || G == 0 || H % G || C == 0 || (uint64_t)pos + rows + C > 0xFFFFFF00ull) return ADAMAH_ERR_INVALID;
+  if (D == 0 || D > 256 || V == 0 || V > 256 || H == 0 || G == 0 || H % G || C == 0 || (uint64_t)pos + rows + C > 0xFFFFFF00ull || n_tok > 0xFFFFFFFFull) return ADAMAH_ERR_INVALID;
   if (s.x_q + H * D > s.x_stride || s.x_k + G * D > s.x_stride || s.x_v + G * V > s.x_stride ||
       !in_range(s.x, (n_tok - 1) * s.x_stride + s.x_stride, ma->n_elems) ||
       !in_range(s.out, (n_tok - 1) * s.out_stride + H * V, ma->n_elems) ||
@@ -651,8 +651,13 @@ static int run_attention(Map* ma, const ASpec& s, uint32_t cache_map, uint32_t n
   if (rows == 1)
     return mc->dtype == DTYPE_F32 ? run_step<float, WIN>(s, act, (float*)mc->buf, n_seq, seq0, pos)
                                   : run_step<bf16_t, WIN>(s, act, (bf16_t*)mc->buf, n_seq, seq0, pos);
-  return mc->dtype == DTYPE_F32 ? run_portion<float, WIN>(s, act, (float*)mc->buf + slot, rows, pos)
-                                : run_portion<bf16_t, WIN>(s, act, (bf16_t*)mc->buf + slot, rows, pos);
+  ASpec p = s;
+  for (uint32_t q = 0; q < n_seq; q++, p.x += rows * s.x_stride, p.out += rows * s.out_stride) {
+    const uint64_t at = slot + (uint64_t)q * s.seq_stride;
+    if (int r = mc->dtype == DTYPE_F32 ? run_portion<float, WIN>(p, act, (float*)mc->buf + at, rows, pos)
+                                       : run_portion<bf16_t, WIN>(p, act, (bf16_t*)mc->buf + at, rows, pos)) return r;
+  }
+  return ADAMAH_OK;
 }
 
 }  // namespace adamah
@@ -661,13 +666,22 @@ using namespace adamah;
 
 extern "C" {
 
-int adamah_chunk_attention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+static int run_chunk_attention(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) {
   Map* ma = get_f32_map(map_act);
   const AdamahChunkAttnSpec* s = spec_of<AdamahChunkAttnSpec>(h_spec);
-  if (!ma || !s || n_seq == 0 || rows == 0 || (n_seq > 1 && rows > 1)) return ADAMAH_ERR_INVALID;
+  if (!ma || !s || n_seq == 0 || rows == 0) return ADAMAH_ERR_INVALID;
   const ASpec a = {s->heads, s->kv_heads, s->dim, s->vdim, s->chunk, s->x, s->x_stride, s->x_q, s->x_k, s->x_v, s->r1, s->r2, s->scale,
                    s->eps, s->out, s->out_stride, s->k_off, s->v_off, s->seq_stride, 0, 0, 1, 0.f, 0.f};
   return run_attention<false>(ma, a, s->cache_map, n_seq, rows, seq0, pos);
+}
+
+int adamah_chunk_attention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+  if (n_seq > 1 && rows > 1) return ADAMAH_ERR_INVALID;
+  return run_chunk_attention(map_act, h_spec, n_seq, rows, seq0, pos);
+}
+
+int adamah_hip_chunk_attention_seqs_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+  return run_chunk_attention(map_act, h_spec, n_seq, rows, seq0, pos);
 }
 
 int adamah_window_attention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();

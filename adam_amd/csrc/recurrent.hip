@@ -252,9 +252,11 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
   float *qs = lds, *ks = qs + CH * P, *G = ks + CH * P, *vs = G + CH * P;             // G: log2 of the running decay; vs [CH][Vp]
   const uint32_t n_ch = 2u * s.kv_heads * D + s.heads * V, kv = h / (s.heads / s.kv_heads);
   const uint32_t qc = kv * D, kc = s.kv_heads * D + kv * D, vc = 2u * s.kv_heads * D + h * V;
-  const float* x = act + s.x;
-  const float* ring = state + (uint64_t)seq0 * s.seq_stride + s.conv_off;
-  float* out = scratch + ((uint64_t)h * cd.n_chunks + blockIdx.x) * chunk_floats(cd.Dp, cd.Vp);
+  const uint32_t sq = blockIdx.z;                            // sequence: rows sq m ..
+  const float* x = act + s.x + (uint64_t)sq * m * s.x_stride;
+  const float* ring = state + (uint64_t)(seq0 + sq) * s.seq_stride + s.conv_off;
+  const float* dec = act + dec_out + (uint64_t)sq * m * dec_stride;
+  float* out = scratch + (((uint64_t)sq * s.heads + h) * cd.n_chunks + blockIdx.x) * chunk_floats(cd.Dp, cd.Vp);
   float *oW = out, *oQ = oW + CH * cd.Dp, *oK = oQ + CH * cd.Dp, *oB = oK + CH * cd.Dp, *oU = oB + 256u, *oG = oU + CH * cd.Vp;
   for (uint32_t i = tid; i < 2u * D; i += 256u) {
     const bool is_k = i >= D;
@@ -275,7 +277,7 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
       const float bias = act[s.dt_bias + h * D + d];
       float z[CH];
 #pragma unroll
-      for (int t = 0; t < (int)CH; t++) z[t] = c0 + t < m ? act[dec_out + (uint64_t)(c0 + t) * dec_stride + h * D + d] + bias : 0.f;
+      for (int t = 0; t < (int)CH; t++) z[t] = c0 + t < m ? dec[(uint64_t)(c0 + t) * dec_stride + h * D + d] + bias : 0.f;
       float lg = 0.f;
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {
@@ -362,7 +364,8 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
   const uint32_t D = s.dim, V = s.vdim, tid = threadIdx.x, c0 = blockIdx.x * CH, h = blockIdx.y, P = D + 1u, half = s.rot_dims >> 1;
   const uint32_t L = min(CH, m - c0);
   float *qs = lds, *ks = qs + CH * P, *cs = ks + CH * P, *sn = cs + CH * half;
-  float* out = scratch + ((uint64_t)h * cd.n_chunks + blockIdx.x) * chunk_floats(cd.Dp, cd.Vp);
+  const float* x = act + s.x + (uint64_t)blockIdx.z * m * s.x_stride;          // z: the sequence
+  float* out = scratch + (((uint64_t)blockIdx.z * s.heads + h) * cd.n_chunks + blockIdx.x) * chunk_floats(cd.Dp, cd.Vp);
   float *oQ = out + CH * cd.Dp, *oK = oQ + CH * cd.Dp, *oB = oK + CH * cd.Dp, *oU = oB + 256u, *oG = oU + CH * cd.Vp;
   const float kscale = 1.0f / sqrtf((float)D);
   if (tid == 0) {
@@ -373,7 +376,7 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
   for (uint32_t i = tid; i < 2u * D; i += 256u) {
     const bool is_k = i >= D;
     const uint32_t d = is_k ? i - D : i;
-    const float* src = act + s.x + (is_k ? s.x_k : s.x_q) + h * D + d;
+    const float* src = x + (is_k ? s.x_k : s.x_q) + h * D + d;
     float* to = (is_k ? ks : qs) + d;
     float v[CH];
 #pragma unroll
@@ -390,7 +393,7 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
   for (uint32_t v = tid; v < cd.Vp; v += 256u) {
     float y[CH];
 #pragma unroll
-    for (int t = 0; t < (int)CH; t++) y[t] = (c0 + t < m && v < V) ? act[s.x + (uint64_t)(c0 + t) * s.x_stride + s.x_v + h * V + v] : 0.f;
+    for (int t = 0; t < (int)CH; t++) y[t] = (c0 + t < m && v < V) ? x[(uint64_t)(c0 + t) * s.x_stride + s.x_v + h * V + v] : 0.f;
 #pragma unroll
     for (int t = 0; t < (int)CH; t++) oU[t * cd.Vp + v] = y[t];
   }
@@ -434,6 +437,7 @@ struct ScanArgs {
   uint32_t heads, dim, vdim, out, out_stride, s_off, m, pos;
   ChunkDims cd;
   uint32_t kv_heads, taps, conv_off, x, x_stride;     // delta: the convolution's ring is brought up to date here
+  uint32_t seq_stride;                                // of the state; grid z: the sequence, its rows m z .. of the activations
 };
 template <int NT> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], b; float u[4]; };
 
@@ -461,7 +465,9 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, D = a.dim, V = a.vdim, v = v0 + c;
   const uint32_t bs = chunk_floats(a.cd.Dp, a.cd.Vp);
-  const float* blk = scratch + (uint64_t)h * a.cd.n_chunks * bs;
+  const float* blk = scratch + ((uint64_t)blockIdx.z * a.heads + h) * a.cd.n_chunks * bs;
+  state += (uint64_t)blockIdx.z * a.seq_stride;
+  float* out = act + a.out + (uint64_t)blockIdx.z * a.m * a.out_stride;
   float* S = state + a.s_off + (uint64_t)h * D * V;
   f4_t st[NT];
 #pragma unroll
@@ -499,7 +505,7 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const uint32_t r2 = ci * CH + 4u * kg + i;
-        if (r2 < a.m && v < V) act[a.out + (uint64_t)r2 * a.out_stride + h * V + v] = o[i];
+        if (r2 < a.m && v < V) out[(uint64_t)r2 * a.out_stride + h * V + v] = o[i];
       }
     }
 #pragma unroll
@@ -521,7 +527,7 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
   const uint32_t n_ch = 2u * a.kv_heads * D + a.heads * V, rep = a.heads / a.kv_heads, kv = h / rep;
   for (uint32_t r = a.m > a.taps ? a.m - a.taps : 0u; r < a.m; r++) {
     float* slot = state + a.conv_off + (uint64_t)((a.pos + r) % a.taps) * n_ch;
-    const float* x = act + a.x + (uint64_t)r * a.x_stride;
+    const float* x = act + a.x + ((uint64_t)blockIdx.z * a.m + r) * a.x_stride;
     if (blockIdx.y == 0 && h % rep == 0)
       for (uint32_t d = tid; d < D; d += 256u) {
         slot[kv * D + d] = x[kv * D + d];
@@ -540,8 +546,8 @@ static bool rows_ok(uint64_t off, uint64_t stride, uint64_t rows, uint64_t width
 }
 
 template <bool DELTA>
-static int launch_scan(const ScanArgs& a, float* act, float* state) {
-  const dim3 grid(a.heads, cdiv(a.vdim, 16));
+static int launch_scan(const ScanArgs& a, float* act, float* state, uint32_t n_seq) {
+  const dim3 grid(a.heads, cdiv(a.vdim, 16), n_seq);
   const float* sc = (const float*)g_chunks.p;
   switch (a.cd.Dp / 64u) {
     case 1: k_chunk_scan<DELTA, 1><<<grid, 256, 0, g.stream>>>(a, sc, act, state); break;
@@ -556,18 +562,13 @@ static int launch_scan(const ScanArgs& a, float* act, float* state) {
 
 static LowRank low_rank(const LinSpec& s) { return {s.w, s.k, s.k_stride, s.src, s.src_stride, s.out, s.out_stride}; }
 
-}  // namespace adamah
-
-using namespace adamah;
-
-extern "C" {
-
-int adamah_delta_rule_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_decay, uint32_t h_gate,
-                          uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+// n_seq sequences of `rows` tokens each, one behind the other in the activations, their states from slot seq0 on.
+static int run_delta_rule(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_decay, uint32_t h_gate,
+                          uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) {
   Map *ma = get_f32_map(map_act), *mo = get_map(map_opnd), *mw = get_map(map_wt);
   const DSpec* s = spec_of<DSpec>(h_spec);
   const LinSpec *da = spec_of<LinSpec>(h_decay), *ga = spec_of<LinSpec>(h_gate);
-  if (!ma || !mw || mw->dtype != DTYPE_BF16 || !s || !da || !ga || n_seq == 0 || rows == 0 || (n_seq > 1 && rows > 1)) return ADAMAH_ERR_INVALID;
+  if (!ma || !mw || mw->dtype != DTYPE_BF16 || !s || !da || !ga || n_seq == 0 || rows == 0 || (uint64_t)n_seq * rows > 0xFFFFFFFFull) return ADAMAH_ERR_INVALID;
   Map* ms = get_f32_map(s->state_map);
   const uint64_t D = s->dim, V = s->vdim, H = s->heads, KH = s->kv_heads, n_tok = (uint64_t)n_seq * rows;
   if (!ms || D == 0 || D > 256 || V == 0 || H == 0 || KH == 0 || H % KH || s->taps == 0 || s->taps > MAX_TAPS) return ADAMAH_ERR_INVALID;
@@ -597,30 +598,30 @@ int adamah_delta_rule_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, 
     count_launch();
     return check_launch();
   }
-  if (int r = adamah_linear_dev(map_act, map_opnd, map_wt, h_decay, 0, rows)) return r;
-  if (int r = adamah_linear_dev(map_act, map_opnd, map_wt, h_gate, 0, rows)) return r;
+  if (int r = adamah_linear_dev(map_act, map_opnd, map_wt, h_decay, 0, n_seq * rows)) return r;
+  if (int r = adamah_linear_dev(map_act, map_opnd, map_wt, h_gate, 0, n_seq * rows)) return r;
   const ChunkDims cd = {(uint32_t)((D + 63) / 64 * 64), (uint32_t)((V + 15) / 16 * 16), cdiv(rows, CH)};
-  if (int r = scratch_need(g_chunks, (size_t)H * cd.n_chunks * chunk_floats(cd.Dp, cd.Vp) * 4)) return r;
+  if (int r = scratch_need(g_chunks, (size_t)n_seq * H * cd.n_chunks * chunk_floats(cd.Dp, cd.Vp) * 4)) return r;
   const size_t lds = (size_t)CH * (3 * (D + 1) + cd.Vp) * 4;
   if (lds > 120000) return ADAMAH_ERR_INVALID;
 #define PREP(TM)                                                                                                                      \
   do {                                                                                                                                \
     if (lds > 60000) hipFuncSetAttribute((const void*)k_delta_prep<TM>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
-    k_delta_prep<TM><<<dim3(cd.n_chunks, (uint32_t)H), 256, lds, g.stream>>>(*s, da->out, da->out_stride, act, state,                 \
+    k_delta_prep<TM><<<dim3(cd.n_chunks, (uint32_t)H, n_seq), 256, lds, g.stream>>>(*s, da->out, da->out_stride, act, state,                 \
                                                                             (float*)g_chunks.p, cd, rows, seq0, pos);                \
   } while (0)
   if (s->taps <= 4) PREP(4); else PREP(MAX_TAPS);
 #undef PREP
   count_launch();
   if (int r = check_launch()) return r;
-  ScanArgs a = {s->heads, s->dim, s->vdim, s->out, s->out_stride, s->s_off, rows, pos, cd, s->kv_heads, s->taps, s->conv_off, s->x, s->x_stride};
-  return launch_scan<true>(a, act, state + (uint64_t)seq0 * s->seq_stride);
+  ScanArgs a = {s->heads, s->dim, s->vdim, s->out, s->out_stride, s->s_off, rows, pos, cd, s->kv_heads, s->taps, s->conv_off, s->x, s->x_stride, s->seq_stride};
+  return launch_scan<true>(a, act, state + (uint64_t)seq0 * s->seq_stride, n_seq);
 }
 
-int adamah_retention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+static int run_retention(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) {
   Map* ma = get_f32_map(map_act);
   const RSpec* s = spec_of<RSpec>(h_spec);
-  if (!ma || !s || n_seq == 0 || rows == 0 || (n_seq > 1 && rows > 1)) return ADAMAH_ERR_INVALID;
+  if (!ma || !s || n_seq == 0 || rows == 0 || (uint64_t)n_seq * rows > 0xFFFFFFFFull) return ADAMAH_ERR_INVALID;
   Map* ms = get_f32_map(s->state_map);
   const uint64_t D = s->dim, V = s->vdim, H = s->heads, n_tok = (uint64_t)n_seq * rows;
   if (!ms || D == 0 || D > 256 || V == 0 || H == 0 || s->rot_dims > D || (s->rot_dims & 1u)) return ADAMAH_ERR_INVALID;
@@ -640,12 +641,38 @@ int adamah_retention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint
     return check_launch();
   }
   const ChunkDims cd = {(uint32_t)((D + 63) / 64 * 64), (uint32_t)((V + 15) / 16 * 16), cdiv(rows, CH)};
-  if (int r = scratch_need(g_chunks, (size_t)H * cd.n_chunks * chunk_floats(cd.Dp, cd.Vp) * 4)) return r;
-  k_retention_prep<<<dim3(cd.n_chunks, (uint32_t)H), 256, (size_t)CH * (2 * (D + 1) + s->rot_dims) * 4, g.stream>>>(*s, act, (float*)g_chunks.p, cd, rows, pos);
+  if (int r = scratch_need(g_chunks, (size_t)n_seq * H * cd.n_chunks * chunk_floats(cd.Dp, cd.Vp) * 4)) return r;
+  k_retention_prep<<<dim3(cd.n_chunks, (uint32_t)H, n_seq), 256, (size_t)CH * (2 * (D + 1) + s->rot_dims) * 4, g.stream>>>(*s, act, (float*)g_chunks.p, cd, rows, pos);
   count_launch();
   if (int r = check_launch()) return r;
-  ScanArgs a = {s->heads, s->dim, s->vdim, s->out, s->out_stride, s->s_off, rows, pos, cd, 0, 0, 0, 0, 0};
-  return launch_scan<false>(a, act, state + (uint64_t)seq0 * s->seq_stride);
+  ScanArgs a = {s->heads, s->dim, s->vdim, s->out, s->out_stride, s->s_off, rows, pos, cd, 0, 0, 0, 0, 0, s->seq_stride};
+  return launch_scan<false>(a, act, state + (uint64_t)seq0 * s->seq_stride, n_seq);
+}
+
+}  // namespace adamah
+
+using namespace adamah;
+
+extern "C" {
+
+int adamah_delta_rule_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_decay, uint32_t h_gate,
+                          uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+  if (n_seq > 1 && rows > 1) return ADAMAH_ERR_INVALID;
+  return run_delta_rule(map_act, map_opnd, map_wt, h_spec, h_decay, h_gate, n_seq, rows, seq0, pos);
+}
+
+int adamah_hip_delta_rule_seqs_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_decay, uint32_t h_gate,
+                                   uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+  return run_delta_rule(map_act, map_opnd, map_wt, h_spec, h_decay, h_gate, n_seq, rows, seq0, pos);
+}
+
+int adamah_retention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+  if (n_seq > 1 && rows > 1) return ADAMAH_ERR_INVALID;
+  return run_retention(map_act, h_spec, n_seq, rows, seq0, pos);
+}
+
+int adamah_hip_retention_seqs_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) { ADAMAH_API();
+  return run_retention(map_act, h_spec, n_seq, rows, seq0, pos);
 }
 
 }  // extern "C"

@@ -1252,6 +1252,14 @@ class DecodeEngine:
             hi = min(n, lo + self._chunk)
             self._forward_chunk(token_ids[lo:hi], pos0 + lo, sample=sample and hi == n, seq=seq)
 
+    def _prefill_each(self, prompts):
+        """Prompt s into the cache of sequence s; the token that follows each."""
+        first = []
+        for sq, pr in enumerate(prompts):
+            self.prefill(pr, seq=sq)
+            first.append(self.read_token())
+        return first
+
     def read_token(self):
         # reference engine.py:1979-1981: token id crosses the boundary as float32
         tok = self.gpu.gather(self.WS_MAP, self._sample_locs).view(np.float32)
@@ -1276,10 +1284,7 @@ class DecodeEngine:
         ahead = (forced is None and self._lookahead and B == self._batch and B > 1 and max_tokens > 1
                  and self._token_feed() is not None)
         t0 = time.perf_counter()
-        cur = []
-        for sq, pr in enumerate(prompts):
-            self.prefill([int(t) for t in pr], seq=sq)
-            cur.append(self.read_token())
+        cur = self._prefill_each([[int(t) for t in pr] for pr in prompts])
         self.gpu.sync()
         t_pre = time.perf_counter() - t0
         out = [[] for _ in range(B)]

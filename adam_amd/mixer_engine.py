@@ -186,7 +186,7 @@ class MixerEngine(DecodeEngine):
         self._ws['hidden'] = self._ws['normed'] = (0, E, self._rows["hidden"][0])
         self._c_tok_pos = take(M)
         self._c_tok_locs = np.arange(self._c_tok_pos, self._c_tok_pos + M, dtype=np.uint32)
-        self._tok_rows_h = self._up(self._c_tok_locs)
+        self._tok_rows_h, self._tok_row_h = self._up(self._c_tok_locs), []
         self._hid_locs = np.arange(self._rows["hidden"][0], self._rows["hidden"][0] + E, dtype=np.uint32)
         self._alloc_sample_handles()
         self._vec_off = {}
@@ -395,25 +395,34 @@ class MixerEngine(DecodeEngine):
 
     # ------------------------------------------------------------------ running the op list
     def _run_program(self, n_seq, rows, seq0, pos):
-        """`rows` tokens of one sequence, or one token of each of n_seq sequences, from the hidden rows to the hidden rows."""
+        """`rows` tokens of one sequence, or one token of each of n_seq sequences (or, where `_takes_portions`, `rows` of
+        each), from the hidden rows to the hidden rows."""
         g, A, ws, n = self.gpu, self.A, self.WS_MAP, n_seq * rows
+        portions = n_seq > 1 and rows > 1
         for kind, mid, h0, h1, h2 in self._program:
             if kind == A.DECODE_OP_LINEAR:
                 g.linear_dev(ws, self.OPND_MAP, mid, h0, 0, n)
             elif kind == A.DECODE_OP_MERGE_NORM:
                 g.merge_norm_dev(ws, h0, n)
             elif kind == A.DECODE_OP_DELTA_RULE:
-                g.delta_rule_dev(ws, self.OPND_MAP, mid, h0, h1, h2, n_seq, rows, seq0, pos)
+                (g.delta_rule_seqs_dev if portions else g.delta_rule_dev)(ws, self.OPND_MAP, mid, h0, h1, h2, n_seq, rows, seq0, pos)
             elif kind == A.DECODE_OP_RETENTION:
-                g.retention_dev(ws, h0, n_seq, rows, seq0, pos)
+                (g.retention_seqs_dev if portions else g.retention_dev)(ws, h0, n_seq, rows, seq0, pos)
             elif kind == A.DECODE_OP_CHUNK_ATTENTION:
-                g.chunk_attention_dev(ws, h0, n_seq, rows, seq0, pos)
+                (g.chunk_attention_seqs_dev if portions else g.chunk_attention_dev)(ws, h0, n_seq, rows, seq0, pos)
             elif kind == A.DECODE_OP_WINDOW_ATTENTION:
                 g.window_attention_dev(ws, h0, n_seq, rows, seq0, pos)
             elif kind == A.DECODE_OP_STATE_SPACE:
                 g.state_space_dev(ws, h0, n_seq, rows, seq0, pos)
             else:
                 g.experts_dev(ws, self.OPND_MAP, mid, h0, h1, n)
+
+    def _takes_portions(self):
+        """Whether every op can take several tokens of several sequences at once."""
+        A = self.A
+        return self.cfg.pairs is None and hasattr(self.gpu, 'delta_rule_seqs_dev') and all(
+            op[0] in (A.DECODE_OP_LINEAR, A.DECODE_OP_MERGE_NORM, A.DECODE_OP_EXPERTS, A.DECODE_OP_DELTA_RULE, A.DECODE_OP_RETENTION,
+                      A.DECODE_OP_CHUNK_ATTENTION) for op in self._program)
 
     def _ops_for(self, n_seq):
         A, P = self.A, self.A.DECODE_RUNTIME_POS
@@ -540,6 +549,34 @@ class MixerEngine(DecodeEngine):
             g.linear_argmax_dev(ws, self.OPND_MAP, mid, h, self._feed['tok_h'], 1)
             self._sample_token_ready = True
         g.batch_end()
+
+    def _prefill_each(self, prompts):
+        """Prompt s into the state of sequence s; the token that follows each.  As many prompts as the rows hold go through
+        the weights together (sixteen prompts of twelve tokens, one by one: sixteen passes over the weights); a prompt of
+        one token keeps its one-row pass, whose operands stay float32."""
+        P = len(prompts[0])
+        at_once = min(len(prompts), self._chunk // P) if 1 < P <= self._chunk and self._takes_portions() else 1
+        if at_once < 2:
+            return super()._prefill_each(prompts)
+        g, ws, first = self.gpu, self.WS_MAP, []
+        while len(self._tok_row_h) < at_once:
+            n = len(self._tok_row_h)
+            self._tok_row_h.append(self._up(self._c_tok_locs[n:n + 1]))
+        for s0 in range(0, len(prompts), at_once):
+            part = prompts[s0:s0 + at_once]
+            toks = [t for p in part for t in p]
+            self._check_tokens(toks)
+            g.batch_begin()
+            for s in range(s0, s0 + len(part)):
+                self._advance(s, 0, P)
+            self._embed(toks, 1, len(toks), s0, 0)
+            self._run_program(len(part), P, s0, 0)
+            for i in range(len(part)):
+                mid, h = self._head(i * P + P - 1)
+                g.linear_argmax_dev(ws, self.OPND_MAP, mid, h, self._tok_row_h[i], 1)
+            g.batch_end()
+            first += self.read_tokens(len(part))
+        return first
 
     def reset(self):
         keep, self._kept = self._kept, 0

@@ -352,6 +352,14 @@ typedef struct AdamahChunkAttnSpec {
 } AdamahChunkAttnSpec;
 int adamah_chunk_attention_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos);
 
+/* The three above for a portion of each of several sequences at once: n_seq sequences of `rows` tokens, one behind the
+ * other in the activation rows, all at position `pos`, their states from slot seq0 on.  (The calls above take one token of
+ * each of n_seq sequences, or rows tokens of one.) */
+int adamah_hip_delta_rule_seqs_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_decay, uint32_t h_gate,
+                                   uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos);
+int adamah_hip_retention_seqs_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos);
+int adamah_hip_chunk_attention_seqs_dev(uint32_t map_act, uint32_t h_spec, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos);
+
 /* Softmax attention over a sliding window: position i sees the `window` positions i - window + 1 .. i.  qk_norm = 1: q and
  * k are divided by their root mean square first (eps inside).  q is multiplied by 1 + temp_coef * ln(floor((i + 1) /
  * temp_every) + 1) (temp_coef = 0: not).  score = (q . k) * scale, softcap > 0: softcap * tanh(score / softcap), then

@@ -439,6 +439,27 @@ def test_generation(hip):
         assert engine(hip, cfg, W, prefill_chunk=8).generate(prompt, GenerationConfig(max_tokens=12, **kw))[0] == want
 
 
+@pytest.mark.parametrize("name,dtype,P,B", [("odd", "float32", 2, 3), ("odd", "float32", 17, 4), ("odd", "bfloat16", 16, 2),
+                                            ("ones", "float32", 5, 4), ("wide", "bfloat16", 33, 3), ("wide", "float32", 34, 2)])
+def test_prompts_that_share_the_weights(hip, name, dtype, P, B):
+    """Several prompts in one pass (as many as 70 rows hold: all, some and one left over) and one by one."""
+    note(f"prompts together {name} {dtype} {B} x {P}")
+    cfg, got = CONFIGS[name], []
+    prompts = [[int(t) for t in tokens(cfg, P, seed=40 + i)] for i in range(B)]
+    for together in (True, False):
+        eng = engine(hip, cfg, weights(cfg, seed=5), dtype=dtype, prefill_chunk=70, batch=B)
+        assert eng._takes_portions()
+        if not together:
+            eng._takes_portions = lambda: False
+        eng.reset()
+        first = eng._prefill_each(prompts)
+        eng._forward_chunk([1] * B, P, lockstep=True)           # what the states hold shows in the step that follows
+        got.append((first, eng.read_rows("hidden", B)))
+    assert got[0][0] == got[1][0] or dtype == "bfloat16"        # (bfloat16: two best may change places)
+    # a pass of more rows takes other tiles, so float32 sums in another order, and bfloat16 operands that round the other way
+    assert rel(got[0][1], got[1][1]) < TOL[dtype]
+
+
 def test_trace_replay_and_command_line(hip, tmp_path):
     """The programs, each in a process of its own, on a model folder."""
     cfg = CONFIGS["odd"]
