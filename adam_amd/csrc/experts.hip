@@ -288,7 +288,7 @@ k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ 
                                    TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) {
                                      const uint32_t i = min(m0 + r, t.count - 1u);
                                      return opnd + (IN ? s.opnd + (uint64_t)(le[i] / s.top) * kp : s.act_opnd + (uint64_t)(t.first + i) * kp);
-                                   }), kp, la, lb, wave, lane);
+                                   }), kp, 0u, kp, la, lb, wave, lane);
 #pragma unroll
   for (int j = 0; j < NTM; j++) {
     const uint32_t i = m0 + wm + 16u * j + c;

@@ -6,7 +6,8 @@
 //                store + best row of the workgroup (arg-max)
 //   2..32 rows   k_linear_skinny: bf16 matrix instructions straight from memory, K split over the waves of a workgroup
 //   more rows    k_linear_tiled<BM, BN, ...>: bf16 matrix instructions over a ring of LDS tiles filled by direct-to-LDS loads
-//   float32 operand map: k_linear_f32, the float32 matrix instruction over the widened weights
+//   float32 operand map: the same tiles over three bfloat16 pieces of each row (k_split_rows); short rows: k_linear_f32, the
+//                float32 matrix instruction over the widened weights
 // Rows of more than one token pass through the operand map (bf16 or float32, rows k_stride apart, zero beyond k):
 // k_operand_rows writes f(x) there, unless the producer already did.
 #include "linear_common.h"
@@ -494,29 +495,38 @@ k_linear_skinny(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, floa
 }
 
 // ---- tiles --------------------------------------------------------------------------------------------------------
-template <int BM, int BN, int WM, int WN, int ST>
+// Shares of K (part): workgroup plane z takes columns z k_per .. and leaves raw sums, rows of np, for k_linear_sum.
+template <class T, int BM, int BN, int WM, int WN, int ST>
 __global__ void __launch_bounds__(64 * WM * WN)
-k_linear_tiled(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, bf16_t* opnd, const LinSpec s, uint32_t rows,
-               uint32_t tiles_m, uint32_t tiles_n) {
+k_linear_tiled(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, T* opnd, const LinSpec s, uint32_t rows,
+               uint32_t tiles_m, uint32_t tiles_n, uint32_t k_per, float* __restrict__ part, uint32_t np) {
   __shared__ __attribute__((aligned(16))) bf16_t la[ST * BN * 64], lb[ST * BM * 64];
-  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16;
+  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16, PL = sizeof(T) == 4 ? 3 : 1;
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint32_t c = lane & 15u, kg = lane >> 4, kp = s.k_stride;
+  const uint32_t c = lane & 15u, kg = lane >> 4, kp = s.k_stride, kx = PL * kp;
   // workgroups land on the eight dies in turn: give every die a run of neighbouring tiles
   const uint32_t total = tiles_m * tiles_n, per = (total + 7u) / 8u;
   const uint32_t id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if (id >= total || (blockIdx.x >> 3) >= per) return;
-  const uint32_t m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN;
+  const uint32_t m0 = (id % tiles_m) * BM, n0 = (id / tiles_m) * BN, k0 = blockIdx.y * k_per;
   const uint32_t wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
   f4_t acc[NTN][NTM];
-  tile_product<BM, BN, WM, WN, ST>(
+  tile_product<BM, BN, WM, WN, ST, PL>(
       acc, TileRows<BN, WM * WN>(wave, lane, [&](uint32_t r) { return W + (uint64_t)min(n0 + r, s.n - 1u) * kp; }),
-      TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) { return X + (uint64_t)min(m0 + r, rows - 1u) * kp; }), kp, la, lb, wave, lane);
+      TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) { return X + (uint64_t)min(m0 + r, rows - 1u) * kx; }), kp, k0, min(kx, k0 + k_per),
+      la, lb, wave, lane);
 #pragma unroll
   for (int j = 0; j < NTM; j++) {
     const uint32_t row = m0 + wm + 16u * j + c;
     if (row >= rows) continue;
-    if (s.epi == 2u) {
+    if (part) {
+      float* d = part + ((uint64_t)blockIdx.y * rows + row) * np;
+#pragma unroll
+      for (int i = 0; i < NTN; i++) {
+        const uint32_t n = n0 + wn + 16u * i + 4u * kg;
+        if (n < np) *(f4_t*)(d + n) = acc[i][j];
+      }
+    } else if (s.epi == 2u) {
 #pragma unroll
       for (int i = 0; i < NTN; i += 2) put_pair_or_tail(s, act, opnd, row, n0 + wn + 16u * i + 4u * kg, acc[i][j], acc[i + 1][j]);
     } else {
@@ -524,6 +534,43 @@ k_linear_tiled(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float
       for (int i = 0; i < NTN; i++) put_out(s, act, row, n0 + wn + 16u * i + 4u * kg, acc[i][j]);
     }
   }
+}
+// The shares' sums, eight results (four and the four 16 on) a thread, np a multiple of 32.
+template <class T>
+__global__ void __launch_bounds__(256)
+k_linear_sum(const LinSpec s, const float* __restrict__ part, float* act, T* opnd, uint32_t rows, uint32_t shares, uint32_t np) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x, per = np / 8u, row = i / per, q = i % per, n = (q >> 2) * 32u + (q & 3u) * 4u;
+  if (row >= rows) return;
+  f4_t a = {0, 0, 0, 0}, b = a;
+  const float* p = part + (uint64_t)row * np + n;
+  for (uint32_t z = 0; z < shares; z++, p += (uint64_t)rows * np) { a += *(const f4_t*)p; b += *(const f4_t*)(p + 16); }
+  if (s.epi == 2u) put_pair_or_tail(s, act, opnd, row, n, a, b);
+  else { put_out(s, act, row, n, a); put_out(s, act, row, n + 16u, b); }
+}
+// float32 operand rows as three bfloat16 rows whose sum they are exactly (8 significant bits each, so down to 2^-110 in size),
+// the lowest first, as they are added up: the bfloat16 instruction's products of them are exact too, and at sixteen times the
+// float32 instruction's rate three of them take a fifth of its time.  512 rows, 16384 x 2048: 322 -> 111 us (930 TFLOP/s of
+// bfloat16 work), 2048 x 8192: 260 -> 76; 88 rows, 2048 x 2048: 57 -> 18.  Infinities and values that are no numbers stay in
+// the highest piece.
+__global__ void __launch_bounds__(256)
+k_split_rows(const float* __restrict__ x, bf16_t* __restrict__ dst, uint32_t kp, uint32_t rows) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x, per = kp / 4u, row = i / per, c = (i % per) * 4u;
+  if (row >= rows) return;
+  const float4 v = *(const float4*)(x + (uint64_t)row * kp + c);
+  const float e[4] = {v.x, v.y, v.z, v.w};
+  uint32_t p[3][4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const uint32_t u = __float_as_uint(e[j]);
+    const float r = e[j] - __uint_as_float(u & 0xFFFF0000u), t = r - __uint_as_float(__float_as_uint(r) & 0xFFFF0000u);
+    const bool number = (u & 0x7F800000u) != 0x7F800000u;
+    p[0][j] = number ? __float_as_uint(t) >> 16 : 0u;
+    p[1][j] = number ? __float_as_uint(r) >> 16 : 0u;
+    p[2][j] = (u >> 16) | (!number && (u & 0x007FFFFFu) ? 0x40u : 0u);
+  }
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+    *(uint2*)(dst + ((uint64_t)row * 3u + q) * kp + c) = make_uint2(p[q][0] | p[q][1] << 16, p[q][2] | p[q][3] << 16);
 }
 
 // ---- float32 operands ---------------------------------------------------------------------------------------------
@@ -549,8 +596,8 @@ k_linear_f32(const bf16_t* __restrict__ W, const float* __restrict__ X, float* a
 }
 
 // ---- launch -------------------------------------------------------------------------------------------------------
-static Scratch g_best;
-void linear_release() { scratch_free(g_best); }
+static Scratch g_best, g_split, g_shares;
+void linear_release() { scratch_free(g_best); scratch_free(g_split); scratch_free(g_shares); }
 
 static bool span_ok(uint64_t off, uint64_t stride, uint64_t rows, uint64_t width, uint64_t n_elems) {
   return rows == 0 || in_range(off, (rows - 1) * stride + width, n_elems);
@@ -587,6 +634,57 @@ static int check_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, uint32_t ro
   return span_ok(s.out, s.out_stride, rows, s.epi == 2u ? (s.n - s.tail) / 2 : s.n, ma->n_elems) ? ADAMAH_OK : ADAMAH_ERR_INVALID;
 }
 
+// The tile and the shares of K that get through the rows soonest: rounds over the CUs times what a step of 64 columns takes
+// there, measured on 40 .. 600 rows by 2048 .. 28672 x 2048 .. 14336: with one workgroup a CU, with two where two fit, and
+// how much less of the first it is when hardly any CU has one; never faster than the matrix comes in.  Shares pay 4 us for
+// the second launch and the way of the sums out and back (192 rows, 4096 x 14336: 70 us in one, 44 in four shares; 40 rows:
+// 64 and 27; 40 rows, 12576 x 4096: 26 in one, 30 in two).
+template <class T>
+static int launch_tiles(const bf16_t* W, const bf16_t* X, float* act, T* op, const LinSpec& s, uint32_t rows) {
+  struct Tile { uint32_t m, n; double one, idle, more, two; };          // more: hardly any CU has a second workgroup yet
+  static const Tile tile[6] = {{256, 256, 1.70, 0.75, 0, 0}, {256, 128, 1.05, 0.72, 0, 0}, {128, 256, 1.05, 0.72, 0, 0},
+                               {128, 128, 0.63, 0.70, 0, 0}, {64, 128, 0.49, 0.95, 0.80, 0.85}, {64, 64, 0.33, 0.75, 0.33, 0.58}};
+  const uint32_t steps = (sizeof(T) == 4 ? 3u : 1u) * s.k_stride / 64u, np = (s.n + 31u) & ~31u;
+  const uint64_t cu = (uint64_t)g.n_cu;
+  const double out_us = (double)rows * np * 4.0 / 4.5e6, w_us = (double)s.n * s.k_stride * 2.0 / 4.2e6;
+  double best = 1e30;
+  uint32_t pick = 0, shares = 1;
+  for (uint32_t t = 0; t < 6; t++) {
+    const Tile& k = tile[t];
+    const uint64_t tiles = (uint64_t)cdiv(rows, k.m) * cdiv(s.n, k.n), fit = k.two > 0 ? 2 * cu : cu;
+    for (uint32_t sp = 1; sp <= 8 && (sp == 1 || (sp * 8 <= steps && tiles * sp <= fit)); sp++) {
+      const uint64_t wgs = tiles * sp, left = wgs % fit;
+      const double first = k.one * (wgs < cu ? k.idle + (1.0 - k.idle) * (double)wgs / (double)cu : 1.0);
+      const double step = (double)(wgs / fit) * (k.two > 0 ? k.two : k.one) + (left == 0 ? 0.0 : left <= cu ? first : k.more + (k.two - k.more) * (double)(left - cu) / (double)cu);
+      const double us = std::max(w_us, step * cdiv(steps, sp)) + (sp > 1 ? 4.0 + 2.0 * sp * out_us : 0.0);
+      if (us < best) { best = us; pick = t; shares = sp; }
+    }
+  }
+  uint32_t per = cdiv(steps, shares);
+  shares = cdiv(steps, per);
+  if (shares > 1 && scratch_need(g_shares, (size_t)shares * rows * np * sizeof(float)) != ADAMAH_OK) { shares = 1; per = steps; }
+  float* part = shares > 1 ? (float*)g_shares.p : nullptr;
+#define LT(BM, BN, WM, WN, ST) do { const uint32_t t = cdiv(rows, BM) * cdiv(s.n, BN); \
+    k_linear_tiled<T, BM, BN, WM, WN, ST><<<dim3(cdiv(t, 8) * 8, shares), 64 * WM * WN, 0, g.stream>>>(W, X, act, op, s, rows, cdiv(rows, BM), cdiv(s.n, BN), \
+                                                                                                      64 * per, part, np); } while (0)
+  switch (pick) {
+    case 0: LT(256, 256, 2, 4, 2); break;
+    case 1: LT(256, 128, 4, 2, 3); break;
+    case 2: LT(128, 256, 2, 4, 3); break;
+    case 3: LT(128, 128, 2, 4, 4); break;
+    case 4: LT(64, 128, 2, 2, 3); break;
+    default: LT(64, 64, 2, 2, 4); break;
+  }
+#undef LT
+  count_launch();
+  if (part) {
+    if (int r = check_launch()) return r;
+    k_linear_sum<T><<<cdiv((uint64_t)rows * (np / 8), 256), 256, 0, g.stream>>>(s, part, act, op, rows, shares, np);
+    count_launch();
+  }
+  return check_launch();
+}
+
 static uint32_t gemv_grid(uint32_t n_tasks) { return std::min<uint32_t>(cdiv(n_tasks, 8), 2u * (uint32_t)g.n_cu); }
 
 template <int EPI>
@@ -615,6 +713,15 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   if (mo->dtype == DTYPE_F32) {
     float* op = (float*)mo->buf;
     if (!s.ready) operand_rows<float>(s, act, op + s.opnd, row_idx, rows);
+    // Long rows in three bfloat16 pieces (the launch that splits them: 4 us; 88 rows of 512: 15.6 us on the float32
+    // instruction, 11.2 in pieces; of 256: 8.3 and 8.2; of 128: 5.1 and 6.6)
+    if (s.k_stride > 256u && scratch_need(g_split, (size_t)rows * 3 * s.k_stride * sizeof(bf16_t)) == ADAMAH_OK) {
+      bf16_t* X = (bf16_t*)g_split.p;
+      k_split_rows<<<cdiv((uint64_t)rows * s.k_stride / 4, 256), 256, 0, g.stream>>>(op + s.opnd, X, s.k_stride, rows);
+      count_launch();
+      if (int r = check_launch()) return r;
+      return launch_tiles<float>(W, X, act, op, s, rows);
+    }
     k_linear_f32<<<dim3(cdiv(s.n, 64), cdiv(rows, 64)), 256, 0, g.stream>>>(W, op + s.opnd, act, op, s, rows);
     count_launch();
     return check_launch();
@@ -622,36 +729,13 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   bf16_t* op = (bf16_t*)mo->buf;
   const bf16_t* X = op + s.opnd;
   if (!s.ready) operand_rows<bf16_t>(s, act, op + s.opnd, row_idx, rows);
-  if (rows <= 32) {
-    // Workgroups of 16 matrix rows as long as no CU gets a second one (12 rows, 4096 x 4096: 9.6 us, of 32: 13.4; 7168 x
-    // 2048: 9.2 to 10.0 and 8.2 to 8.9).
+  if (rows > 32) return launch_tiles<bf16_t>(W, X, act, op, s, rows);
+  // Workgroups of 16 matrix rows as long as no CU gets a second one (12 rows, 4096 x 4096: 9.6 us, of 32: 13.4; 7168 x
+  // 2048: 9.2 to 10.0 and 8.2 to 8.9).
 #define LS(MT) do { if (s.epi != 2u && cdiv(s.n, 16) <= (uint32_t)g.n_cu) k_linear_skinny<MT, 1, 16><<<cdiv(s.n, 16), 1024, 0, g.stream>>>(W, X, act, op, s, rows); \
-      else k_linear_skinny<MT, 2, 8><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows); } while (0)
-    if (rows <= 16) LS(1); else LS(2);
+    else k_linear_skinny<MT, 2, 8><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows); } while (0)
+  if (rows <= 16) LS(1); else LS(2);
 #undef LS
-  }
-  else {
-    // The tile that gets through the rows soonest: rounds over the CUs times what a step of 64 columns takes there
-    // (1/100 us, measured with all CUs at work on 2048 x 28672 x 4096, 600 x 12672 x 4096, 300 x 10304 x 2048 and
-    // 300 x 4096 x 4096; with at most one workgroup a CU, with two where two fit).
-    const auto cost = [&](uint32_t bm, uint32_t bn, uint32_t one, uint32_t two) {
-      const uint64_t tiles = (uint64_t)cdiv(rows, bm) * cdiv(s.n, bn), cu = (uint64_t)g.n_cu, fit = two ? 2 * cu : cu, left = tiles % fit;
-      return tiles / fit * (two ? two : one) + (left == 0 ? 0 : left <= cu ? one : two);
-    };
-    const uint64_t c[6] = {cost(256, 256, 170, 0), cost(256, 128, 105, 0), cost(128, 256, 105, 0), cost(128, 128, 63, 0), cost(64, 128, 50, 80),
-                           cost(64, 64, 40, 55)};
-#define LT(BM, BN, WM, WN, ST) do { const uint32_t t = cdiv(rows, BM) * cdiv(s.n, BN); \
-      k_linear_tiled<BM, BN, WM, WN, ST><<<cdiv(t, 8) * 8, 64 * WM * WN, 0, g.stream>>>(W, X, act, op, s, rows, cdiv(rows, BM), cdiv(s.n, BN)); } while (0)
-    switch (std::min_element(c, c + 6) - c) {
-      case 0: LT(256, 256, 2, 4, 2); break;
-      case 1: LT(256, 128, 4, 2, 3); break;
-      case 2: LT(128, 256, 2, 4, 3); break;
-      case 3: LT(128, 128, 2, 4, 4); break;
-      case 4: LT(64, 128, 2, 2, 3); break;
-      default: LT(64, 64, 2, 2, 4); break;
-    }
-#undef LT
-  }
   count_launch();
   return check_launch();
 }

@@ -47,7 +47,7 @@ template <int R, int NW> struct TileRows {
       p[i] = row(r) + (((lane & 7u) ^ (r & 7u)) << 3);
     }
   }
-  __device__ __forceinline__ void load(int i, uint32_t k, uint32_t lds, uint32_t wave) const {
+  __device__ __forceinline__ void load(int i, uint32_t k, uint32_t lds, uint32_t wave) const {      // from column k on
     load_to_lds(p[i] + k, lds + ((uint32_t)i * NW + wave) * 1024u);
   }
 };
@@ -56,10 +56,11 @@ template <int R, int NW> struct TileRows {
 // step is two halves of 32 columns; a half's operands are read from LDS under the products of the half before, on both
 // sides of the step's one barrier.  What bounds it (256 x 256, two buffers): of the 1.75 us a step takes on all CUs the
 // products need 1.0, the loads alone 0.7 (23 TB/s out of the L2s), reads of LDS run beside both; loads and reads in a run
-// ahead of the products instead of among them: 1.95 us.
-template <int BM, int BN, int WM, int WN, int ST>
+// ahead of the products instead of among them: 1.95 us.  Columns k0 .. k1 of the tokens; column k of them meets column
+// k mod kp of the matrix (k1 at most PL kp).
+template <int BM, int BN, int WM, int WN, int ST, int PL = 1>
 __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM / 16], const TileRows<BN, WM * WN>& w, const TileRows<BM, WM * WN>& x,
-                                             uint32_t kp, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane) {
+                                             uint32_t kp, uint32_t k0, uint32_t k1, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane) {
   constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16, LOADS = TileRows<BN, WM * WN>::N + TileRows<BM, WM * WN>::N;
   const uint32_t c = lane & 15u, kg = lane >> 4, wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
   const uint32_t ba = lds_byte(la), bb = lds_byte(lb);
@@ -68,8 +69,8 @@ __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM /
 #pragma unroll
     for (int j = 0; j < NTM; j++) acc[i][j] = (f4_t){0, 0, 0, 0};
   const auto load = [&](int i, uint32_t k, uint32_t into) {       // (steps past the end re-read the last: the count in flight stays)
-    const uint32_t kc = min(k, kp - 64u);
-    if (i < TileRows<BN, WM * WN>::N) w.load(i, kc, ba + into * (BN * 128u), wave);
+    const uint32_t kc = min(k, k1 - 64u), kw = PL == 1 ? kc : kc >= 2u * kp ? kc - 2u * kp : kc >= kp ? kc - kp : kc;
+    if (i < TileRows<BN, WM * WN>::N) w.load(i, kw, ba + into * (BN * 128u), wave);
     else x.load(i - TileRows<BN, WM * WN>::N, kc, bb + into * (BM * 128u), wave);
   };
   bf8_t a[2][NTN], b[2][NTM];
@@ -102,12 +103,12 @@ __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM /
 #pragma unroll
   for (int t = 0; t < ST; t++)
 #pragma unroll
-    for (int i = 0; i < LOADS; i++) load(i, (uint32_t)t * 64u, t);
+    for (int i = 0; i < LOADS; i++) load(i, k0 + (uint32_t)t * 64u, t);
   ring_wait<LOADS * (ST - 1)>();
 #pragma unroll
   for (int i = 0; i < NTN + NTM; i++) read(i, 0, 0);
   uint32_t buf = 0;
-  for (uint32_t k = 0; k < kp; k += 64u) {
+  for (uint32_t k = k0; k < k1; k += 64u) {
     const uint32_t next = buf + 1 == ST ? 0 : buf + 1;
     half(0, buf, 0, 0);
     ring_wait<LOADS * (ST - 2)>();                 // the next step's tiles have arrived, this step's are no longer read

@@ -118,6 +118,58 @@ def test_operand_rows_in_one_trip(hip, rows, k, groups, act, per_group):
     p.same(WS, out, rows * n, 2e-5, "out")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows,n,k,epi,tail", [
+    (33, 70, 320, 0, 0), (40, 131, 4096, 1, 0), (64, 96, 1088, 2, 0), (65, 201, 2048, 2, 41), (190, 2050, 1024, 0, 0), (300, 515, 3008, 1, 0),
+    (257, 1000, 576, 2, 8), (3, 45, 512, 0, 0), (512, 2048, 2048, 0, 0)])
+def test_linear_shares_and_pieces(hip, dtype, rows, n, k, epi, tail):
+    """Long rows over shares of K, float32 rows in their bfloat16 pieces (one of them infinite, one huge, one tiny)."""
+    note(f"linear shares {dtype} rows {rows} n {n} k {k} epi {epi}")
+    rng = np.random.default_rng(n + k)
+    f64 = lambda b: (b.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    W = f32_to_bf16(rng.standard_normal((n, k)).astype(np.float32) / np.float32(np.sqrt(k)))
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    x[0] *= np.float32(2.0 ** 100)
+    x[1] *= np.float32(2.0 ** -80)
+    wide = dtype == "float32"
+    if not wide:
+        x = f64(f32_to_bf16(x)).astype(np.float32)
+    x[rows - 1, 5] = np.inf
+    pair_w = (n - tail) // 2 if epi == 2 else 0
+    st, op_at = n + 3, (rows * k + 7) // 8 * 8
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_F32 if wide else A.DTYPE_BF16, 1, op_at + rows * (pair_w + 1) + 8)
+    hip.scatter_contiguous(OP, 0, x.reshape(-1) if wide else f32_to_bf16(x.reshape(-1)))
+    old = rng.standard_normal((rows, st)).astype(np.float32)
+    f32map(hip, WS, old.size, old.reshape(-1))
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=k, opnd=0, ready=1, out=0, out_stride=st, epi=epi, out_opnd=op_at, out_opnd_stride=pair_w + 1,
+                        tail=tail, tail_out=0, tail_stride=st)
+    hip.linear_dev(WS, OP, WT, up(hip, spec.words()), 0, rows)
+    got = read(hip, WS, 0, old.size).reshape(rows, st)
+    with np.errstate(invalid="ignore"):
+        y = x.astype(np.float64) @ f64(W).T
+    body = y[:-1]
+    # exact products; float32 sums of 3 k terms and shares at most: 3 k 2^-24 relative to the terms' root sum of squares
+    tol = 3 * k * 2.0 ** -24
+    each = lambda g, w: max(rel_l2(a, b) for a, b in zip(g, w))
+    if epi < 2:
+        want = body + (old[:-1, :n] if epi else 0.0)
+        assert each(got[:-1, :n], want) < tol
+        assert not np.isfinite(got[-1, :n]).any() and np.array_equal(got[:, n:], old[:, n:])
+        return
+    if tail:
+        assert each(got[:-1, :tail], body[:, n - tail:]) < tol
+    assert np.array_equal(got[:, tail:], old[:, tail:])
+    head = body[1:, :n - tail].reshape(rows - 2, -1, 2, 16)
+    want = (head[:, :, 0] / (1.0 + np.exp(-head[:, :, 0])) * head[:, :, 1]).reshape(rows - 2, pair_w)
+    raw = hip.gather(OP, np.arange(op_at, op_at + rows * (pair_w + 1), dtype=np.uint32))
+    pairs = raw.view(np.float32) if wide else f64(raw.view(np.uint16)[:raw.size])          # (a 16-bit map's values lie packed)
+    pairs = pairs.reshape(rows, -1)[1:-1, :pair_w]
+    # (a row of 2^-80: its pairs are products of two tiny numbers, 2^-161)
+    assert each(pairs[1:], want[1:]) < (4 * tol if wide else 4 * tol + 2.0 ** -8)
+
+
 @pytest.mark.parametrize("rows", [1, 3])
 def test_linear_argmax_takes_the_first_of_equals(hip, rows):
     note(f"linear argmax rows {rows}")
