@@ -85,21 +85,26 @@ k_gemv_block(const float* act, float* act_out, const uint8_t* __restrict__ W,
   __syncthreads();
 
   const uint64_t gbase = b >> 5;                    // first group of the matrix
+  // A row of few blocks takes as many lanes as it has (rounded up to a power of two), so a wave has 64 / lp rows in each of
+  // its ROWS (512 rows of 4 blocks in 2 groups, a row a wave: 37 us of waiting for one load after another, so: 4.8).
+  uint32_t lp = 64u;
+  while (lp > 1u && (lp >> 1) >= nblk) lp >>= 1;
+  const uint32_t at_once = 64u / lp, sub = lane / lp;
   for (uint32_t grp = blockIdx.x; grp < n_groups; grp += gridDim.x) {
     const uint32_t row0 = grp * rows_per_group;
     const uint32_t row1 = min(N, row0 + rows_per_group);
     float best_v = NEG_FLT_MAX;
     uint32_t best_i = INVALID_IDX;
-    for (uint32_t r = row0 + wave * ROWS; r < row1; r += 4u * ROWS) {
+    for (uint32_t r = row0 + wave * ROWS * at_once; r < row1; r += 4u * ROWS * at_once) {
       float acc[ROWS];
 #pragma unroll
       for (int i = 0; i < ROWS; i++) acc[i] = 0.f;
-      for (uint32_t blk = lane; blk < nblk; blk += 64u) {
+      for (uint32_t blk = lane & (lp - 1u); blk < nblk; blk += lp) {
         uint4 q0[ROWS], q1[ROWS];
         float sc[ROWS], zp[ROWS];
 #pragma unroll
         for (int i = 0; i < ROWS; i++) {
-          const uint32_t row = min(r + i, row1 - 1);          // clamp: duplicates are discarded below
+          const uint32_t row = min(r + i * at_once + sub, row1 - 1);          // clamp: duplicates are discarded below
           const uint64_t gidx = gbase + (uint64_t)row * nblk + blk;
           if (Q4) {
             q0[i] = *(const uint4*)(W + (gidx << 4));
@@ -134,15 +139,22 @@ k_gemv_block(const float* act, float* act_out, const uint8_t* __restrict__ W,
       }
 #pragma unroll
       for (int i = 0; i < ROWS; i++) {
-        const float y = wave_sum_to_lane63(acc[i]);   // total valid in lane 63 only
-        const uint32_t row = r + i;
-        if (row < row1 && lane == 63) {
+        float y = acc[i];
+        if (lp == 64u) y = wave_sum_to_lane63(y);     // total valid in the row's last lane only
+        else for (uint32_t o = 1; o < lp; o <<= 1) y += __shfl_xor(y, (int)o, 64);
+        const uint32_t row = r + i * at_once + sub;
+        if (row < row1 && (lane & (lp - 1u)) == lp - 1u) {
           if (EPI == EPI_STORE) act_out[(uint64_t)lc[0] + row] = y;
           else if (better(y, row, best_v, best_i)) { best_v = y; best_i = row; }
         }
       }
     }
     if (EPI == EPI_ARGMAX) {
+      for (uint32_t o = lp; o < 64u; o <<= 1) {       // the best of the wave's rows ends in lane 63
+        const float v = __shfl_xor(best_v, (int)o, 64);
+        const uint32_t at = __shfl_xor(best_i, (int)o, 64);
+        if (better(v, at, best_v, best_i)) { best_v = v; best_i = at; }
+      }
       if (lane == 63) { red_v[wave] = best_v; red_i[wave] = best_i; }
       __syncthreads();
       if (tid == 0) {

@@ -187,6 +187,30 @@ def test_linear_argmax_takes_the_first_of_equals(hip, rows):
     assert a.tolist() == b.tolist() == [2002.0] * rows
 
 
+@pytest.mark.parametrize("n,st", [(16384, 16384), (16385, 16388), (40000, 40001), (49152, 49152)])
+def test_linear_argmax_of_long_rows(hip, n, st):
+    """Runs that are read four floats at a time, their remainder, rows that do not start on sixteen bytes; equals far apart."""
+    note(f"linear argmax n {n}")
+    rows, k = 3, 64
+    rng = np.random.default_rng(n)
+    W = f32_to_bf16(rng.standard_normal((n, k)).astype(np.float32))
+    big = f32_to_bf16(np.full(k, 4.0, np.float32))
+    at = {0: [n - 1, 5000], 1: [n - 1], 2: [12288 + 7, 3, 9000]}
+    x = np.zeros((rows, k), np.float32)
+    for r, places in at.items():                  # row r sees only its own columns
+        x[r, 16 * r:16 * r + 16] = 1.0
+        for p in places:
+            W[p, 16 * r:16 * r + 16] = big[:16]
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * k)
+    f32map(hip, WS, rows * (k + st) + 16, x)
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=k, src=0, src_stride=k, out=rows * k, out_stride=st)
+    tok = rows * (k + st) + np.arange(rows)
+    hip.linear_argmax_dev(WS, OP, WT, up(hip, spec.words()), up(hip, tok), rows)
+    assert read(hip, WS, int(tok[0]), rows).tolist() == [float(min(at[r])) for r in range(rows)]
+
+
 def test_merge_norm(hip):
     note("merge norm")
     rows, dim, st = 5, 77, 80

@@ -299,6 +299,13 @@ def test_matvec_argmax_tail(hip, kind, N, K, rpg):
     assert agree > 0.97, agree
 
 
+@pytest.mark.parametrize("kind,N,K,rpg", [("q4", 100, 32, 7), ("q8", 513, 64, 256), ("q4", 512, 128, 256), ("q8", 300, 96, 64), ("q8", 999, 512, 100),
+                                          ("q4", 70, 1024, 70), ("q8", 130, 1056, 33), ("q4", 64, 2048, 64)])
+def test_matvec_argmax_of_short_rows(hip, kind, N, K, rpg):
+    """Rows of 1 .. 64 blocks (several rows of a wave at once up to 32), groups that end inside a wave's rows."""
+    test_matvec_argmax_tail(hip, kind, N, K, rpg)
+
+
 def test_argmax_plain_ties_nan(hip):
     vals = np.full(5000, -1.0, np.float32)
     vals[[4097, 77, 3000]] = 9.5; vals[5] = np.nan
