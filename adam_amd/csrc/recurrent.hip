@@ -277,11 +277,13 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
       const float bias = act[s.dt_bias + h * D + d];
       float z[CH];
 #pragma unroll
-      for (int t = 0; t < (int)CH; t++) z[t] = c0 + t < m ? dec[(uint64_t)(c0 + t) * dec_stride + h * D + d] + bias : 0.f;
+      for (int t = 0; t < (int)CH; t++) z[t] = dec[(uint64_t)min(c0 + t, m - 1u) * dec_stride + h * D + d];
+#pragma unroll
+      for (int t = 0; t < (int)CH; t++) z[t] = fminf(ea * softplus_f(z[t] + bias), NO_MEMORY) * 1.44269504f;
       float lg = 0.f;
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {
-        if (c0 + t < m) lg -= fminf(ea * softplus_f(z[t]), NO_MEMORY) * 1.44269504f;
+        lg -= c0 + t < m ? z[t] : 0.f;
         G[t * P + d] = lg;
       }
     }
@@ -380,9 +382,9 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
     float* to = (is_k ? ks : qs) + d;
     float v[CH];
 #pragma unroll
-    for (int t = 0; t < (int)CH; t++) v[t] = c0 + t < m ? src[(uint64_t)(c0 + t) * s.x_stride] : 0.f;
+    for (int t = 0; t < (int)CH; t++) v[t] = src[(uint64_t)min(c0 + t, m - 1u) * s.x_stride];      // (a load on every path)
 #pragma unroll
-    for (int t = 0; t < (int)CH; t++) to[t * P] = is_k ? v[t] * kscale : v[t];
+    for (int t = 0; t < (int)CH; t++) to[t * P] = c0 + t >= m ? 0.f : is_k ? v[t] * kscale : v[t];
   }
   for (uint32_t i = tid; i < CH * half; i += 256u) {
     const uint32_t t = i / half, d = i - t * half;
@@ -393,9 +395,9 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
   for (uint32_t v = tid; v < cd.Vp; v += 256u) {
     float y[CH];
 #pragma unroll
-    for (int t = 0; t < (int)CH; t++) y[t] = (c0 + t < m && v < V) ? x[(uint64_t)(c0 + t) * s.x_stride + s.x_v + h * V + v] : 0.f;
+    for (int t = 0; t < (int)CH; t++) y[t] = x[(uint64_t)min(c0 + t, m - 1u) * s.x_stride + s.x_v + h * V + min(v, V - 1u)];
 #pragma unroll
-    for (int t = 0; t < (int)CH; t++) oU[t * cd.Vp + v] = y[t];
+    for (int t = 0; t < (int)CH; t++) oU[t * cd.Vp + v] = c0 + t < m && v < V ? y[t] : 0.f;
   }
   __syncthreads();
   for (uint32_t i = tid; i < 2u * CH * half; i += 256u) {     // turn the pairs in place

@@ -40,22 +40,34 @@ __device__ __forceinline__ float conv_silu_ring(const float* x, const float* rin
 template <int TM, class Put>
 __device__ __forceinline__ void conv_silu_rows(const float* x, uint32_t x_stride, uint32_t r0, uint32_t m, const float* ring, uint32_t n_ch,
                                                uint32_t ch, uint32_t pos, const float* w, uint32_t taps, Put put, float bias = 0.f) {
-  float in[CH + TM - 1], wt[TM];
+  // Every load on every path, rows beyond the portion's end read its last one: a condition around a load made each of the
+  // sixteen wait for the one before (delta_prep of 2048 tokens in 32 heads of 128: 221 us, now 173).
+  float in[CH + TM - 1], wt[TM], y[CH];
 #pragma unroll
   for (int i = 0; i < (int)CH + TM - 1; i++) {
-    const int64_t r = (int64_t)r0 + i - (TM - 1);
-    const bool old = r < 0, on = old ? (uint32_t)-r < taps && (uint32_t)-r <= pos : r < (int64_t)m;
-    in[i] = !on ? 0.f : old ? ring[(uint64_t)((pos + (uint32_t)r) % taps) * n_ch + ch] : x[(uint64_t)r * x_stride + ch];
+    const int32_t r = (int32_t)r0 + i - (TM - 1);
+    in[i] = x[(uint64_t)min((uint32_t)max(r, 0), m - 1u) * x_stride + ch];
   }
 #pragma unroll
-  for (int j = 0; j < TM; j++) wt[j] = (uint32_t)j < taps ? w[taps - 1u - (uint32_t)j] : 0.f;
+  for (int j = 0; j < TM; j++) wt[j] = w[taps - 1u - min((uint32_t)j, taps - 1u)];
+  if (r0 < (uint32_t)TM - 1u) {
+#pragma unroll
+    for (int i = 0; i < TM - 1; i++) {
+      const uint32_t back = (uint32_t)(TM - 1 - i) - r0;      // rows before the portion
+      if (r0 + i < (uint32_t)TM - 1u) in[i] = back < taps && back <= pos ? ring[(uint64_t)((pos - back) % taps) * n_ch + ch] : 0.f;
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < TM; j++) wt[j] = (uint32_t)j < taps ? wt[j] : 0.f;
 #pragma unroll
   for (int t = 0; t < (int)CH; t++) {
     float a = bias;
 #pragma unroll
     for (int j = 0; j < TM; j++) a = fmaf(wt[j], in[t + TM - 1 - j], a);
-    put(t, r0 + (uint32_t)t < m ? silu_f(a) : 0.f);
+    y[t] = silu_f(a);
   }
+#pragma unroll
+  for (int t = 0; t < (int)CH; t++) put(t, r0 + (uint32_t)t < m ? y[t] : 0.f);
 }
 
 }  // namespace adamah
