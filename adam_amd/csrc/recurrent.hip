@@ -433,6 +433,8 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 }
 
 // ---- the walk over the chunks ---------------------------------------------------------------------------------------
+// A serial chain, so what counts is a chunk's latency: 2048 tokens in 32 heads of 128 took 236 us = 1.85 us a chunk with the
+// next one's operands under a condition (the wait at its end is for everything asked for), 144 so.
 // Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
 // is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.
 struct ScanArgs {
@@ -473,16 +475,21 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
   float* S = state + a.s_off + (uint64_t)h * D * V;
   f4_t st[NT];
 #pragma unroll
-  for (int j = 0; j < NT; j++)
+  for (int j = 0; j < NT; j++) st[j] = (f4_t){0, 0, 0, 0};
+  if (a.pos != 0u) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t d = (wave * NT + j) * 16u + 4u * kg + i;
-      st[j][i] = (a.pos != 0u && d < D && v < V) ? S[(uint64_t)d * V + v] : 0.f;
-    }
-  ChunkOps<NT> cur, nxt;
-  load_ops<DELTA, NT>(cur, blk, a.cd, wave, c, kg, v0);
-  for (uint32_t ci = 0; ci < a.cd.n_chunks; ci++) {
-    if (ci + 1u < a.cd.n_chunks) load_ops<DELTA, NT>(nxt, blk + (uint64_t)(ci + 1u) * bs, a.cd, wave, c, kg, v0);
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) st[j][i] = S[(uint64_t)min((wave * NT + j) * 16u + 4u * kg + i, D - 1u) * V + min(v, V - 1u)];
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) if ((wave * NT + j) * 16u + 4u * kg + i >= D || v >= V) st[j][i] = 0.f;
+  }
+  const uint32_t n = a.cd.n_chunks;
+  // the operands of the chunk two ahead, asked for on every path (past the end: the last one's again)
+  const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, c, kg, v0); };
+  const auto chunk = [&](const ChunkOps<NT>& cur, uint32_t ci, f4_t (*pb)[4][64]) {
     f4_t p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < NT; j++)
@@ -491,16 +498,16 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
         if (DELTA) p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], p1, 0, 0, 0);
         p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], p2, 0, 0, 0);
       }
-    if (DELTA) pb[ci & 1u][0][wave][lane] = p1;
-    pb[ci & 1u][1][wave][lane] = p2;
+    if (DELTA) pb[0][wave][lane] = p1;
+    pb[1][wave][lane] = p2;
     __syncthreads();
     f4_t u = {cur.u[0], cur.u[1], cur.u[2], cur.u[3]};
     if (DELTA) {
-      const f4_t* r = &pb[ci & 1u][0][0][0];
+      const f4_t* r = &pb[0][0][0];
       u -= (r[lane] + r[64 + lane]) + (r[128 + lane] + r[192 + lane]);
     }
     if (wave == 0u) {
-      const f4_t* r = &pb[ci & 1u][1][0][0];
+      const f4_t* r = &pb[1][0][0];
       f4_t o = (r[lane] + r[64 + lane]) + (r[128 + lane] + r[192 + lane]);
 #pragma unroll
       for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[i], u[i], o, 0, 0, 0);
@@ -516,7 +523,19 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
 #pragma unroll
       for (int i = 0; i < 4; i++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][i], u[i], st[j], 0, 0, 0);
     }
-    cur = nxt;
+  };
+  ChunkOps<NT> o0, o1, o2;
+  ask(o0, 0); ask(o1, 1); ask(o2, 2);
+  for (uint32_t ci = 0;; ci += 3u) {
+    chunk(o0, ci, pb[ci & 1u]);
+    if (ci + 1u >= n) break;
+    ask(o0, ci + 3u);
+    chunk(o1, ci + 1u, pb[(ci + 1u) & 1u]);
+    if (ci + 2u >= n) break;
+    ask(o1, ci + 4u);
+    chunk(o2, ci + 2u, pb[ci & 1u]);
+    if (ci + 3u >= n) break;
+    ask(o2, ci + 5u);
   }
 #pragma unroll
   for (int j = 0; j < NT; j++)
