@@ -329,8 +329,10 @@ k_attn_keep(const ASpec s, T* cache, const T* __restrict__ K, const T* __restric
 template <bool WIN> __device__ __forceinline__ uint32_t first_seen(const ASpec& s, uint32_t p, uint32_t base) {
   return (WIN ? (p >= s.size ? p + 1u - s.size : 0u) : p / s.size * s.size) - base;
 }
-// 16 queries of a head per wave.  float32 form: keys 16 at a time.
-template <bool WIN, int NV>
+// 16 queries of a head per wave.  float32 form: keys 16 at a time.  Few waves walk a serial chain, so a step's latency
+// counts: queries in registers, keys a step ahead, values asked for at the step's head (read where they were needed, under
+// conditions: 303 us for 512 queries in 16 heads of 128, so: 101).
+template <bool WIN, int NV, int DK>
 __global__ void __launch_bounds__(256)
 k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos) {
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kg = lane >> 4, h = blockIdx.x, kv = h / (s.heads / s.kv_heads);
@@ -343,30 +345,48 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
   const float* kb = K + (uint64_t)kv * sd.np * sd.dp;
   const float* vb = VT + (uint64_t)kv * sd.vp * sd.np;
   const float r1 = act[s.p1 + h], r2 = act[s.p2 + h];
-  f4_t o[NV];
+  f4_t o[NV], q[DK], kk[DK], vv[NV];
 #pragma unroll
   for (int i = 0; i < NV; i++) o[i] = (f4_t){0, 0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < DK; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[t][i] = xq[min(16u * t + 4u * kg + i, s.dim - 1u)];
+  const auto keys = [&](uint32_t j0) {
+#pragma unroll
+    for (int t = 0; t < DK; t++) kk[t] = *(const f4_t*)(kb + (uint64_t)(j0 + c) * sd.dp + min(16u * t, sd.dp - 16u) + 4u * kg);
+  };
+  keys(first);
+#pragma unroll
+  for (int t = 0; t < DK; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[t][i] = 16u * t + 4u * kg + i < s.dim ? q[t][i] : 0.f;
   float mx = ATT_MASKED, sum = 0.f, qs = s.scale;
   if (WIN) {
     if (s.has_sink) { mx = r2; sum = 1.f; }
     if (s.qk_norm) {
       float a = 0.f;
-      for (uint32_t d = kg; d < s.dim; d += 4u) a = fmaf(xq[d], xq[d], a);
+#pragma unroll
+      for (int t = 0; t < DK; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) a = fmaf(q[t][i], q[t][i], a);
       a += __shfl_xor(a, 16, 64); a += __shfl_xor(a, 32, 64);
       qs /= sqrtf(a / (float)s.dim + s.eps);
     }
     qs *= query_temperature(s, pos + qr);
   }
   for (uint32_t j0 = first; j0 < end; j0 += 16u) {
-    f4_t a = {0, 0, 0, 0};
-    for (uint32_t d0 = 0; d0 < sd.dp; d0 += 16u) {
-      const f4_t kk = *(const f4_t*)(kb + (uint64_t)(j0 + c) * sd.dp + d0 + 4u * kg);
+    // everything a step reads is asked for at its head (its keys a step ahead), on every path
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint32_t d = d0 + 4u * kg + i;
-        a = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[i], d < s.dim ? xq[d] : 0.f, a, 0, 0, 0);
-      }
+    for (int v = 0; v < NV; v++) vv[v] = *(const f4_t*)(vb + (uint64_t)(min(v * 16u, sd.vp - 16u) + c) * sd.np + j0 + 4u * kg);
+    f4_t a = {0, 0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < DK; t++) {
+      if (16u * t >= sd.dp) break;
+#pragma unroll
+      for (int i = 0; i < 4; i++) a = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[t][i], q[t][i], a, 0, 0, 0);
     }
+    keys(j0 + 16u < end ? j0 + 16u : j0);
     float t = ATT_MASKED;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -391,10 +411,9 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
 #pragma unroll
     for (int v = 0; v < NV; v++) {
       if ((uint32_t)v * 16u >= sd.vp) break;
-      const f4_t vv = *(const f4_t*)(vb + (uint64_t)(v * 16u + c) * sd.np + j0 + 4u * kg);
       o[v] *= al;
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], a[i], o[v], 0, 0, 0);
+      for (int i = 0; i < 4; i++) o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[v][i], a[i], o[v], 0, 0, 0);
     }
   }
   if (q0 + c >= m) return;
@@ -589,8 +608,10 @@ static int run_portion(const ASpec& s, float* act, T* cache, uint32_t m, uint32_
   if (int r = check_launch()) return r;
   if constexpr (sizeof(T) == 4) {
     const dim3 grid(s.heads, cdiv(m, 64));
-    if (sd.vp <= 64u) k_attn_f32<WIN, 4><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos);
-    else k_attn_f32<WIN, 16><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos);
+#define AF(NV, DK) k_attn_f32<WIN, NV, DK><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos)
+    if (sd.dp <= 128u) { if (sd.vp <= 64u) AF(4, 8); else if (sd.vp <= 128u) AF(8, 8); else AF(16, 8); }
+    else { if (sd.vp <= 64u) AF(4, 16); else if (sd.vp <= 128u) AF(8, 16); else AF(16, 16); }
+#undef AF
   } else {
     switch (sd.dp / 32u) {
       case 1: launch_bf16<WIN, 1>(s, act, K, VT, sd, m, pos); break;
