@@ -331,7 +331,9 @@ template <bool WIN> __device__ __forceinline__ uint32_t first_seen(const ASpec& 
 }
 // 16 queries of a head per wave.  float32 form: keys 16 at a time.  Few waves walk a serial chain, so a step's latency
 // counts: queries in registers, keys a step ahead, values asked for at the step's head (read where they were needed, under
-// conditions: 303 us for 512 queries in 16 heads of 128, so: 101).
+// conditions: 303 us for 512 queries in 16 heads of 128, so: 101).  No loop over q, kk, vv or o ends early: the compiler then
+// leaves it rolled and puts the arrays in memory (512 queries behind 1500 keys, 16 heads of 192 with 256 values: 2470 us,
+// with loads where they were needed 1729, so: 549).
 template <bool WIN, int NV, int DK>
 __global__ void __launch_bounds__(256)
 k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos) {
@@ -381,11 +383,10 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
     for (int v = 0; v < NV; v++) vv[v] = *(const f4_t*)(vb + (uint64_t)(min(v * 16u, sd.vp - 16u) + c) * sd.np + j0 + 4u * kg);
     f4_t a = {0, 0, 0, 0};
 #pragma unroll
-    for (int t = 0; t < DK; t++) {
-      if (16u * t >= sd.dp) break;
+    for (int t = 0; t < DK; t++)
+      if (16u * t < sd.dp)
 #pragma unroll
-      for (int i = 0; i < 4; i++) a = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[t][i], q[t][i], a, 0, 0, 0);
-    }
+        for (int i = 0; i < 4; i++) a = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[t][i], q[t][i], a, 0, 0, 0);
     keys(j0 + 16u < end ? j0 + 16u : j0);
     float t = ATT_MASKED;
 #pragma unroll
@@ -409,12 +410,12 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
     ps += __shfl_xor(ps, 16, 64); ps += __shfl_xor(ps, 32, 64);
     sum = fmaf(sum, al, ps);
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      if ((uint32_t)v * 16u >= sd.vp) break;
-      o[v] *= al;
+    for (int v = 0; v < NV; v++)
+      if ((uint32_t)v * 16u < sd.vp) {
+        o[v] *= al;
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[v][i], a[i], o[v], 0, 0, 0);
-    }
+        for (int i = 0; i < 4; i++) o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[v][i], a[i], o[v], 0, 0, 0);
+      }
   }
   if (q0 + c >= m) return;
   float* out = act + s.out + (uint64_t)qr * s.out_stride + h * s.vdim;
