@@ -189,8 +189,8 @@ def test_prefill_chunk_is_one_causal_launch(hip, chunk_impl, m, seq0, Hq, Hkv, d
     (2, 383, 1, 1, 128, 0.0, 1), (16, 97, 4, 4, 256, 0.0, 0), (100, 650, 5, 1, 64, 0.0, 0), (3, 9000, 2, 1, 128, 0.0, 0)])
 def test_prefill_chunk_over_runs_of_keys(hip, m, seq0, Hq, Hkv, d, softcap, gap):
     """Few heads and tokens behind many keys: runs of keys on workgroups of their own, joined by a third launch.  Against
-    float64 over the same fp16 keys and values; the products take queries and weights as exact two-term sums, so what is
-    left are float32 sums and exponentials (a few 2^-22 of scores of a few units): 4e-6."""
+    float64 over the same fp16 keys and values; queries and weights are two fp16 terms each (2^-22 of a query's largest element,
+    2^-24 of a weight), and what else is left are float32 sums and exponentials (a few 2^-22 of scores of a few units): 4e-6."""
     rng = np.random.default_rng(m * 1000 + seq0)
     cap_len = seq0 + m + 7
     q = rng.standard_normal((m, Hq, d)).astype(np.float32)
@@ -209,6 +209,29 @@ def test_prefill_chunk_over_runs_of_keys(hip, m, seq0, Hq, Hkv, d, softcap, gap)
             assert rel_l2(out[t, h], p / p.sum() @ V16[h // (Hq // Hkv), :seq0 + t]) < 4e-6, (t, h)
             if t == m - 1:
                 assert rel_l2(scores[h], raw) < 1e-5
+
+
+@pytest.mark.parametrize("m,seq0,Hq,Hkv,d,softcap", [(2, 383, 1, 1, 128, 0.0), (17, 700, 3, 1, 64, 30.0), (24, 130, 4, 1, 256, 0.0), (40, 900, 6, 2, 128, 0.0)])
+def test_short_chunk_keeps_the_small_weights(hip, m, seq0, Hq, Hkv, d, softcap):
+    """Weights of about 2^-12 beside one of 1 in every 16 keys, whose own value is zero: the output is made of the small ones
+    alone, so a weight held to a fixed smallest step shows (fp16's, 2^-24: 1e-4).  What is left is float32: an exponential
+    (2^-22 with its argument's rounding), a softmax of at most 940 keys."""
+    rng = np.random.default_rng(m + seq0)
+    n = seq0 + m
+    q, K, V = np.zeros((m, Hq, d), np.float32), (0.1 * rng.standard_normal((Hkv, n + 7, d))).astype(np.float32), rng.standard_normal((Hkv, n + 7, d)).astype(np.float32)
+    q[...] = 0.05 * rng.standard_normal((m, Hq, d))
+    q[:, :, 0] = 4.0
+    K[:, :, 0], K[:, ::16, 0] = 0.0, 2.0789 * (1.1 if softcap else 1.0)
+    V[:, ::16] = 0.0
+    note(f"attention chunk, small weights m={m} seq0={seq0} {Hq}q/{Hkv}kv d={d}")
+    out, _, _ = chunk_case(hip, q, K, V, seq0, n + 7, 1.0, softcap)
+    K16, V16 = (x.astype(np.float16).astype(np.float64) for x in (K, V))
+    for t in range(m):
+        for h in range(Hq):
+            s = K16[h // (Hq // Hkv), :seq0 + t] @ q[t, h].astype(np.float64)
+            s = softcap * np.tanh(s / softcap) if softcap else s
+            p = np.exp(s - s.max())
+            assert rel_l2(out[t, h], p / p.sum() @ V16[h // (Hq // Hkv), :seq0 + t]) < 4e-6, (t, h)
 
 
 def test_causal_rows_entry_point_equals_the_pairs_issued_one_by_one(hip, chunk_impl):
