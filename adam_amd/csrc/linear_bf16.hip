@@ -77,8 +77,9 @@ __device__ __forceinline__ void group_inverse(const LinSpec& s, float* inv, floa
 }
 // f(x) of one row by a workgroup of NT threads; put(i, value) for i in [0, k_stride).  first: this workgroup also stores
 // what the spec wants kept.  put4(c, values): elements 4 c .. 4 c + 3.  inv: LDS, LIN_MAX_GROUPS floats, part: LDS, NT / 16
-// floats.
-template <int NT, class Put, class Put4>
+// floats.  WIDE: for rows of several floats a thread; without it the code is short and needs fewer registers, which is what
+// counts where a thread has one (2048 rows of 64: 4.6 us, with it 5.4).
+template <int NT, bool WIDE, class Put, class Put4>
 __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32_t row, bool first, float* inv, float* part, Put put, Put4 put4) {
   const uint32_t tid = threadIdx.x, gl = s.groups ? s.k / s.groups >> 2 : 64u;          // lanes (of four elements) a group has
   const float* x = act + s.src + (uint64_t)row * s.src_stride;
@@ -124,12 +125,12 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
       if (i < s.k) done(i, xv[j], nv[j]);
     }
     for (uint32_t i = tid + (uint32_t)R * NT; i < s.k; i += NT) done(i, sum_at(i), s.wt_len ? wt[i] : 0.f);
-  } else if (s.k <= 16u * NT && ((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) == 0u &&
+  } else if (WIDE && s.groups && s.k <= 16u * NT && ((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) == 0u &&
              (!s.gate_act || ((s.gate | s.gate_stride) & 3u) == 0u) && (!s.wt_len || ((s.wt | s.wt_len) & 3u) == 0u) &&
-             (!s.groups || ((s.k / s.groups & 3u) == 0u && ((gl & 63u) == 0u || (gl < 64u && (gl & (gl - 1u)) == 0u))))) {
+             (s.k / s.groups & 3u) == 0u && (s.groups == 1u || (gl & 63u) == 0u || (gl < 64u && (gl & (gl - 1u)) == 0u))) {
     // The row makes one trip: up to four times four elements a thread, everything asked for at once (twelve rows of 4096,
     // one float a load and each pass waiting for the one before: 15.8 us; so: 5.0).  A group is a power of two of
-    // neighbouring lanes, or whole waves' worth, whose sums meet in LDS.
+    // neighbouring lanes, or whole waves' worth, whose sums meet in LDS, or all of the row.
     constexpr int R = 4, NW = NT / 64;
     const uint32_t n4 = s.k >> 2, wave = tid >> 6;
     const float* gt = act + s.gate + (uint64_t)row * s.gate_stride;
@@ -155,32 +156,30 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
       for (int e = 0; e < 4; e++) ss[j] = fmaf(xv[j][e], xv[j][e], ss[j]);
     }
     float scale[R];
-    if (s.groups) {
-      const float n = (float)(4u * gl);
-      if (gl < 64u) {
+    const float n = (float)(4u * gl);
+    if (gl < 64u && s.groups != 1u) {
 #pragma unroll
-        for (int j = 0; j < R; j++) {
-          if ((uint32_t)j * NT >= n4) break;
-          for (uint32_t o = gl >> 1; o > 0; o >>= 1) ss[j] += __shfl_xor(ss[j], (int)o, 64);
-          scale[j] = 1.0f / sqrtf(ss[j] / n + s.eps);
-        }
-      } else {
-        const uint32_t nb = gl >> 6;
+      for (int j = 0; j < R; j++) {
+        if ((uint32_t)j * NT >= n4) break;
+        for (uint32_t o = gl >> 1; o > 0; o >>= 1) ss[j] += __shfl_xor(ss[j], (int)o, 64);
+        scale[j] = 1.0f / sqrtf(ss[j] / n + s.eps);
+      }
+    } else {
+      const uint32_t nb = (gl + 63u) >> 6;
 #pragma unroll
-        for (int j = 0; j < R; j++) {
-          if ((uint32_t)j * NT >= n4) break;
-          const float t = wsum64(ss[j]);
-          if ((tid & 63u) == 0u) part[j * NW + wave] = t;
-        }
-        __syncthreads();
+      for (int j = 0; j < R; j++) {
+        if ((uint32_t)j * NT >= n4) break;
+        const float t = wsum64(ss[j]);
+        if ((tid & 63u) == 0u) part[j * NW + wave] = t;
+      }
+      __syncthreads();
 #pragma unroll
-        for (int j = 0; j < R; j++) {
-          if (tid + (uint32_t)j * NT >= n4) break;
-          const uint32_t b0 = ((uint32_t)j * NW + wave) / nb * nb;
-          float t = 0.f;
-          for (uint32_t b = 0; b < nb; b++) t += part[b0 + b];
-          scale[j] = 1.0f / sqrtf(t / n + s.eps);
-        }
+      for (int j = 0; j < R; j++) {
+        if (tid + (uint32_t)j * NT >= n4) break;
+        const uint32_t b0 = ((uint32_t)j * NW + wave) / nb * nb;
+        float t = 0.f;
+        for (uint32_t b = 0; b < nb; b++) t += part[b0 + b];
+        scale[j] = 1.0f / sqrtf(t / n + s.eps);
       }
     }
 #pragma unroll
@@ -190,7 +189,7 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
       f4_t v = xv[j];
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        if (s.groups) v[e] *= scale[j];
+        v[e] *= scale[j];
         if (s.wt_len) v[e] *= s.wt_add + wv[j][e];
         if (s.gate_act == 1u) v[e] *= sigmoid_f(gv[j][e]);
         else if (s.gate_act == 2u) v[e] *= silu_f(gv[j][e]);
@@ -213,6 +212,13 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
       if (kept) keep[i] = v;
       put(i, v);
     }
+  } else if (WIDE && ((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) == 0u) {
+#pragma unroll 4
+    for (uint32_t c = tid; c < s.k >> 2; c += NT) {
+      const f4_t v = *(const f4_t*)(x + 4u * c);
+      if (kept) *(f4_t*)(keep + 4u * c) = v;
+      put4(c, v);
+    }
   } else {
     for (uint32_t i = tid; i < s.k; i += NT) {
       if (kept) keep[i] = x[i];
@@ -222,21 +228,23 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
   for (uint32_t i = s.k + tid; i < s.k_stride; i += NT) put(i, 0.f);
 }
 
-template <class T, int NT>
+template <class T, int NT, bool WIDE>
 __global__ void __launch_bounds__(NT)
 k_operand_rows(const LinSpec s, float* act, T* __restrict__ dst, const uint32_t* __restrict__ row_idx) {
   __shared__ float inv[LIN_MAX_GROUPS];
   __shared__ float part[NT / 16];
   typedef T t4 __attribute__((ext_vector_type(4)));
   T* d = dst + (uint64_t)blockIdx.x * s.k_stride;
-  operand_row<NT>(s, act, row_idx ? row_idx[blockIdx.x] : blockIdx.x, true, inv, part, [&](uint32_t i, float v) { d[i] = (T)v; },
+  operand_row<NT, WIDE>(s, act, row_idx ? row_idx[blockIdx.x] : blockIdx.x, true, inv, part, [&](uint32_t i, float v) { d[i] = (T)v; },
                   [&](uint32_t c, f4_t v) { *(t4*)(d + 4u * c) = (t4){(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; });
 }
-// Few rows: a row's latency is the launch's, so 1024 threads a row; many rows fill the CUs with 256 each.
+// Long rows, few of them: a row's latency is the launch's, so 1024 threads a row; many rows fill the CUs with 256 each, and
+// rows of one float a thread have nothing to gain (12 rows of 256 with 1024 threads: 4.6 us, so: 3.5).
 template <class T>
 static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* row_idx, uint32_t rows) {
-  if (rows <= 2u * (uint32_t)g.n_cu) k_operand_rows<T, 1024><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
-  else k_operand_rows<T, 256><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
+  if (s.k <= 256u) k_operand_rows<T, 256, false><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
+  else if (s.k > 1024u && rows <= 2u * (uint32_t)g.n_cu) k_operand_rows<T, 1024, true><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
+  else k_operand_rows<T, 256, true><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
   count_launch();
 }
 
@@ -273,7 +281,7 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
   uint32_t task = blockIdx.x * 8u + wave, k0 = lane * 8u, r0, r1;
   rows_of(min(task, n_tasks - 1u), r0, r1);
   fetch(r0, r1, k0);
-  operand_row<512>(s, act, row_idx ? row_idx[0] : 0u, blockIdx.x == 0u, inv, part,
+  operand_row<512, (U > 1)>(s, act, row_idx ? row_idx[0] : 0u, blockIdx.x == 0u, inv, part,
                    [&](uint32_t i, float v) { xs[((i >> 2) & 1u) * half + (i >> 3) * 4u + (i & 3u)] = v; },
                    [&](uint32_t c, f4_t v) { *(f4_t*)(xs + (c & 1u) * half + (c >> 1) * 4u) = v; });
   __syncthreads();

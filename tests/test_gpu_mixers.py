@@ -96,7 +96,9 @@ def test_linear_tiles(hip, rows, n, k, biased, add):
 
 @pytest.mark.parametrize("rows,k,groups,act,per_group", [
     (1, 2048, 1, 1, 0), (1, 8192, 32, 2, 1), (2, 8196, 1, 0, 0), (3, 4096, 64, 3, 1), (3, 16384, 16, 1, 0), (2, 16640, 1, 2, 0), (5, 768, 3, 3, 0),
-    (5, 768, 1, 0, 1), (7, 256, 64, 1, 1), (4, 1200, 25, 2, 0), (530, 4096, 4, 1, 1), (520, 4352, 1, 3, 0), (515, 36, 0, 0, 0)])
+    (5, 768, 1, 0, 1), (7, 256, 64, 1, 1), (4, 1200, 25, 2, 0), (530, 4096, 4, 1, 1), (520, 4352, 1, 3, 0), (515, 36, 0, 0, 0),
+    (4, 256, 1, 2, 0), (4, 260, 1, 1, 0), (4, 260, 5, 0, 1), (6, 1024, 8, 1, 1), (6, 1028, 1, 3, 0), (1, 1152, 1, 0, 0), (1, 1022, 1, 2, 0),
+    (1, 1028, 0, 0, 0), (9, 1300, 0, 0, 0), (9, 1302, 0, 0, 0), (600, 1100, 0, 0, 0), (3, 20000, 0, 0, 0)])
 def test_operand_rows_in_one_trip(hip, rows, k, groups, act, per_group):
     """Rows and groups that a workgroup's registers hold (and just do not), groups of lanes and of waves, every gate."""
     note(f"operand rows {rows} k {k} groups {groups} act {act}")
