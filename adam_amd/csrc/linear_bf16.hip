@@ -366,28 +366,28 @@ k_best_pair(const float* __restrict__ val, const uint32_t* __restrict__ idx, uin
 }
 // arg-max of every row of a [rows, n] block.  A row has one workgroup, so its latency counts: sixteen floats a thread asked
 // for at once (16 rows of 100000, one float at a time by 256 threads: 36 us; so: 5.1).
-#define BEST_NT 1024u
-__global__ void __launch_bounds__(BEST_NT)
+template <uint32_t NT>
+__global__ void __launch_bounds__(NT)
 k_best_row(const float* __restrict__ act, uint64_t src, uint32_t stride, uint32_t n, float* out, const uint32_t* __restrict__ dst) {
-  __shared__ float sv[BEST_NT / 64u];
-  __shared__ uint32_t si[BEST_NT / 64u];
+  __shared__ float sv[NT / 64u];
+  __shared__ uint32_t si[NT / 64u];
   const float* x = act + src + (uint64_t)blockIdx.x * stride;
   float v = NEG_MAX_F;
   uint32_t b = 0xFFFFFFFFu, done = 0;
   if (((src | stride) & 3u) == 0u) {
     constexpr uint32_t U = 4;
-    for (; done + 4u * U * BEST_NT <= n; done += 4u * U * BEST_NT) {
+    for (; done + 4u * U * NT <= n; done += 4u * U * NT) {
       f4_t t[U];
 #pragma unroll
-      for (uint32_t u = 0; u < U; u++) t[u] = *(const f4_t*)(x + done + 4u * (u * BEST_NT + threadIdx.x));
+      for (uint32_t u = 0; u < U; u++) t[u] = *(const f4_t*)(x + done + 4u * (u * NT + threadIdx.x));
 #pragma unroll
       for (uint32_t u = 0; u < U; u++)
 #pragma unroll
-        for (uint32_t e = 0; e < 4; e++) if (t[u][e] > v) { v = t[u][e]; b = done + 4u * (u * BEST_NT + threadIdx.x) + e; }
+        for (uint32_t e = 0; e < 4; e++) if (t[u][e] > v) { v = t[u][e]; b = done + 4u * (u * NT + threadIdx.x) + e; }
     }
   }
 #pragma unroll 8
-  for (uint32_t i = done + threadIdx.x; i < n; i += BEST_NT) { const float t = x[i]; if (t > v) { v = t; b = i; } }
+  for (uint32_t i = done + threadIdx.x; i < n; i += NT) { const float t = x[i]; if (t > v) { v = t; b = i; } }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     const float tv = __shfl_xor(v, o, 64);
@@ -397,7 +397,7 @@ k_best_row(const float* __restrict__ act, uint64_t src, uint32_t stride, uint32_
   if ((threadIdx.x & 63u) == 0) { sv[threadIdx.x >> 6] = v; si[threadIdx.x >> 6] = b; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (uint32_t w = 1; w < BEST_NT / 64u; w++) if (sv[w] > v || (sv[w] == v && si[w] < b)) { v = sv[w]; b = si[w]; }
+    for (uint32_t w = 1; w < NT / 64u; w++) if (sv[w] > v || (sv[w] == v && si[w] < b)) { v = sv[w]; b = si[w]; }
     out[dst[blockIdx.x]] = (float)(b == 0xFFFFFFFFu ? 0u : b);
   }
 }
@@ -830,7 +830,9 @@ int adamah_linear_argmax_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_w
     k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0]);
   } else {
     if (int r = run_linear(ma, mo, mw, *s, nullptr, rows)) return r;
-    k_best_row<<<rows, BEST_NT, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
+    // (1024 threads only reduce more: rows of 50 in 3.8 us, with 256 in 3.0; rows of 2000 in 4.5 and 5.1, of 4000 in 5.0 and 8.1)
+    if (s->n > 1024u) k_best_row<1024><<<rows, 1024, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
+    else k_best_row<256><<<rows, 256, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
   }
   count_launch();
   return check_launch();

@@ -189,7 +189,24 @@ def test_linear_argmax_takes_the_first_of_equals(hip, rows):
     assert a.tolist() == b.tolist() == [2002.0] * rows
 
 
-@pytest.mark.parametrize("n,st", [(16384, 16384), (16385, 16388), (40000, 40001), (49152, 49152)])
+@pytest.mark.parametrize("n", [1, 5, 255, 256, 257, 1000, 1023, 1024, 1025, 1028, 2051, 4096, 5000])
+def test_linear_argmax_of_short_rows(hip, n):
+    """Rows around what one float a thread covers, of 256 and of 1024 threads; two equals a wave apart."""
+    note(f"linear argmax n {n}")
+    rng = np.random.default_rng(n)
+    W = f32_to_bf16(rng.uniform(-1, 1, (n, 64)).astype(np.float32))
+    at = (n - 1, max(n - 66, 0))
+    W[list(at)] = f32_to_bf16(np.ones(64, np.float32))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, 128)
+    f32map(hip, WS, 128 + 2 * n + 2, np.ones(128, np.float32))
+    spec = A.LinearSpec(w=0, n=n, k=64, k_stride=64, src=0, src_stride=64, out=128, out_stride=n)
+    hip.linear_argmax_dev(WS, OP, WT, up(hip, spec.words()), up(hip, 128 + 2 * n + np.arange(2)), 2)
+    assert read(hip, WS, 128 + 2 * n, 2).tolist() == [float(min(at))] * 2
+
+
+@pytest.mark.parametrize("n,st", [(16384, 16384), (16385, 16388), (40000, 40001), (49152, 49152), (12296, 12300)])
 def test_linear_argmax_of_long_rows(hip, n, st):
     """Runs that are read four floats at a time, their remainder, rows that do not start on sixteen bytes; equals far apart."""
     note(f"linear argmax n {n}")
