@@ -507,12 +507,12 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
   l_tot += __shfl_xor(l_tot, 32, 64);
   if (splits > 1u) {
     const uint64_t row0 = ((uint64_t)split * H + head) * m + t0;      // [run of keys][head][token]
-    float* const pa = part + 2ull * splits * H * m;                   // (maximum, sum) of all rows, then their values
-    if (g == 0 && n < rows) { part[2 * (row0 + n)] = m_run; part[2 * (row0 + n) + 1] = l_tot; }
+    float* const ms = part + (uint64_t)splits * H * m * D;            // the values of all rows, then their (maximum, sum)
+    if (g == 0 && n < rows) { ms[2 * (row0 + n)] = m_run; ms[2 * (row0 + n) + 1] = l_tot; }
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       if (4u * g + r >= rows) continue;
-      float* dst = pa + (row0 + 4u * g + r) * D + n;
+      float* dst = part + (row0 + 4u * g + r) * D + n;
 #pragma unroll
       for (int b = 0; b < NB; b++) dst[16 * b] = acc[b][r];
     }
@@ -540,17 +540,17 @@ k_attn_prefill_join(const float* __restrict__ part, float* out, const AttpBases 
   const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * 4u, t = blockIdx.y;
   if (i >= H * D) return;
   const uint32_t head = i / D, d = i % D;
-  const float* const pa = part + 2ull * splits * H * m;
+  const float* const ms = part + (uint64_t)splits * H * m * D;
   float M = ATTP_NEG;
-  for (uint32_t s = 0; s < splits; s++) M = fmaxf(M, part[2 * (((uint64_t)s * H + head) * m + t)]);
+  for (uint32_t s = 0; s < splits; s++) M = fmaxf(M, ms[2 * (((uint64_t)s * H + head) * m + t)]);
   float L = 0.f;
   f4p_t o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
   for (uint32_t s = 0; s < splits; s++) {
     const uint64_t row = ((uint64_t)s * H + head) * m + t;
-    const float f = __builtin_amdgcn_exp2f(part[2 * row] - M);
-    const f4p_t v = *(const f4p_t*)(pa + row * D + d);
-    L = fmaf(part[2 * row + 1], f, L);
+    const float f = __builtin_amdgcn_exp2f(ms[2 * row] - M);
+    const f4p_t v = *(const f4p_t*)(part + row * D + d);              // (rows of D floats from the start of the buffer: 16-byte aligned)
+    L = fmaf(ms[2 * row + 1], f, L);
 #pragma unroll
     for (int k = 0; k < 4; k++) o[k] = fmaf(v[k], f, o[k]);
   }

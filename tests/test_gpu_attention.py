@@ -186,7 +186,8 @@ def test_prefill_chunk_is_one_causal_launch(hip, chunk_impl, m, seq0, Hq, Hkv, d
 
 @pytest.mark.parametrize("m,seq0,Hq,Hkv,d,softcap,gap", [
     (24, 4001, 32, 8, 128, 0.0, 0), (17, 513, 4, 1, 256, 50.0, 0), (33, 700, 6, 3, 64, 30.0, 8), (40, 1200, 3, 1, 128, 0.0, 0),
-    (2, 383, 1, 1, 128, 0.0, 1), (16, 97, 4, 4, 256, 0.0, 0), (100, 650, 5, 1, 64, 0.0, 0), (3, 9000, 2, 1, 128, 0.0, 0)])
+    (2, 383, 1, 1, 128, 0.0, 1), (16, 97, 4, 4, 256, 0.0, 0), (100, 650, 5, 1, 64, 0.0, 0), (3, 9000, 2, 1, 128, 0.0, 0),
+    (17, 460, 3, 1, 128, 0.0, 0)])       # (the last: odd heads, tokens and runs)
 def test_prefill_chunk_over_runs_of_keys(hip, m, seq0, Hq, Hkv, d, softcap, gap):
     """Few heads and tokens behind many keys: runs of keys on workgroups of their own, joined by a third launch.  Against
     float64 over the same fp16 keys and values; queries and weights are two fp16 terms each (2^-22 of a query's largest element,
