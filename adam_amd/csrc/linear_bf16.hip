@@ -239,7 +239,8 @@ k_operand_rows(const LinSpec s, float* act, T* __restrict__ dst, const uint32_t*
                   [&](uint32_t c, f4_t v) { *(t4*)(d + 4u * c) = (t4){(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; });
 }
 // Long rows, few of them: a row's latency is the launch's, so 1024 threads a row; many rows fill the CUs with 256 each, and
-// rows of one float a thread have nothing to gain (12 rows of 256 with 1024 threads: 4.6 us, so: 3.5).
+// rows of one float a thread have nothing to gain (300 rows of 64 on the wide form with 1024 threads: 5.7 us, so: 3.6; 12 rows
+// of 100: 4.7 and 3.6).
 template <class T>
 static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* row_idx, uint32_t rows) {
   if (s.k <= 256u) k_operand_rows<T, 256, false><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
@@ -574,7 +575,7 @@ k_linear_sum(const LinSpec s, const float* __restrict__ part, float* act, T* opn
 // the lowest first, as they are added up: the bfloat16 instruction's products of them are exact too, and at sixteen times the
 // float32 instruction's rate three of them take a fifth of its time.  512 rows, 16384 x 2048: 322 -> 111 us (930 TFLOP/s of
 // bfloat16 work), 2048 x 8192: 260 -> 76; 88 rows, 2048 x 2048: 57 -> 18.  Infinities and values that are no numbers stay in
-// the highest piece.
+// the highest piece; tile_product settles what an infinite weight makes of the others.
 __global__ void __launch_bounds__(256)
 k_split_rows(const float* __restrict__ x, bf16_t* __restrict__ dst, uint32_t kp, uint32_t rows) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x, per = kp / 4u, row = i / per, c = (i % per) * 4u;
@@ -830,7 +831,7 @@ int adamah_linear_argmax_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_w
     k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0]);
   } else {
     if (int r = run_linear(ma, mo, mw, *s, nullptr, rows)) return r;
-    // (1024 threads only reduce more: rows of 50 in 3.8 us, with 256 in 3.0; rows of 2000 in 4.5 and 5.1, of 4000 in 5.0 and 8.1)
+    // (1024 threads only reduce more: rows of 50 in 4.1 us, with 256 in 3.0, of 1000 in 4.2 and 3.9; rows of 2000 in 4.5 and 5.1, of 4000 in 5.0 and 8.1)
     if (s->n > 1024u) k_best_row<1024><<<rows, 1024, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
     else k_best_row<256><<<rows, 256, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
   }

@@ -57,7 +57,9 @@ template <int R, int NW> struct TileRows {
 // sides of the step's one barrier.  What bounds it (256 x 256, two buffers): of the 1.75 us a step takes on all CUs the
 // products need 1.0, the loads alone 0.7 (23 TB/s out of the L2s), reads of LDS run beside both; loads and reads in a run
 // ahead of the products instead of among them: 1.95 us.  Columns k0 .. k1 of the tokens; column k of them meets column
-// k mod kp of the matrix (k1 at most PL kp).
+// k mod kp of the matrix (k1 at most PL kp).  PL = 3, tokens in pieces, the largest last: an infinite weight and a lower piece
+// of 0 make no number where the whole product is infinite, so the lower pieces' sum counts only where it is finite (the
+// highest one's is infinite, or no number, exactly where the whole one is).
 template <int BM, int BN, int WM, int WN, int ST, int PL = 1>
 __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM / 16], const TileRows<BN, WM * WN>& w, const TileRows<BM, WM * WN>& x,
                                              uint32_t kp, uint32_t k0, uint32_t k1, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane) {
@@ -107,14 +109,27 @@ __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM /
   ring_wait<LOADS * (ST - 1)>();
 #pragma unroll
   for (int i = 0; i < NTN + NTM; i++) read(i, 0, 0);
-  uint32_t buf = 0;
-  for (uint32_t k = k0; k < k1; k += 64u) {
-    const uint32_t next = buf + 1 == ST ? 0 : buf + 1;
-    half(0, buf, 0, 0);
-    ring_wait<LOADS * (ST - 2)>();                 // the next step's tiles have arrived, this step's are no longer read
-    half(1, next, k + ST * 64u, buf);
-    buf = next;
+  uint32_t buf = 0, k = k0;
+  const auto walk = [&](uint32_t end) {
+    for (; k < end; k += 64u) {
+      const uint32_t next = buf + 1 == ST ? 0 : buf + 1;
+      half(0, buf, 0, 0);
+      ring_wait<LOADS * (ST - 2)>();               // the next step's tiles have arrived, this step's are no longer read
+      half(1, next, k + ST * 64u, buf);
+      buf = next;
+    }
+  };
+  if (PL == 3) {                                   // (a walk of its own: a condition in the steps cost 2 of 10 us at 16 x 512 x 512)
+    walk(min(k1, 2u * kp));
+    if (k0 < 2u * kp)
+#pragma unroll
+      for (int i = 0; i < NTN; i++)
+#pragma unroll
+        for (int j = 0; j < NTM; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[i][j][e] = __builtin_isfinite(acc[i][j][e]) ? acc[i][j][e] : 0.f;
   }
+  walk(k1);
   ring_wait<0>();                                  // nothing is on its way to LDS when the workgroup ends
 }
 // The same in float32: 64 tokens x 64 matrix rows, 32 columns a step, on the float32 matrix instruction.  Within a run of
