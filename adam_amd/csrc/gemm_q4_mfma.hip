@@ -1149,7 +1149,16 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     if (sp > 1 && 3.0 * (double)cdiv64(steps, sp) + 9.0 < (double)steps * (small <= cu / 2 ? 1.3 : small <= cu ? 1.75 : 2.2)) p.shares = (uint32_t)sp;
     return p;
   }
-  if (b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) return p;
+  if (b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {
+    // not the ring (it reads the scales of two blocks as one word): a narrow matrix from 128 rows on in 256 x 128 tiles over
+    // 2 .. 4 shares where they fill the CUs (512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four)
+    const uint64_t w = cdiv64(N, 256) * cdiv64(M, 128);
+    if (M < 128 || w * 4 >= 3 * cu) return p;
+    uint64_t sp = std::min<uint64_t>(4, cu / std::max<uint64_t>(1, w));
+    while (sp > 1 && K / sp < 1024u) sp--;
+    if (w * sp * 4 >= 3 * cu) p.shares = (uint32_t)sp;
+    return p;
+  }
   for (int ma = 2; ma <= 4; ma += 2) {
     const uint64_t tiles = cdiv64(N, 512) * cdiv64(M, 32 * (uint64_t)ma);
     for (uint64_t sp = 1; sp <= 16 && sp * 4 <= pairs && (sp == 1 || tiles * sp <= cu); sp++) {
@@ -1271,9 +1280,11 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     keep();
     return check_launch();
   }
-  if (plan.shares > 1) {                         // 33 .. 64 rows: 256 weight rows a workgroup over shares of K
+  if (plan.shares > 1) {                         // 256 weight rows a workgroup over shares of K
     const uint32_t kper = cdiv(cdiv(K >> 5, plan.shares), 4u) * 4u, shares = cdiv(K >> 5, kper);
-    k_gemm_q4_f16_tiled<4, 2, 8><<<dim3(cdiv(N, 256), cdiv(M, 64), shares), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, shares, kper, g_part_buf);
+#define GS(T) k_gemm_q4_f16_tiled<T, 2, 8><<<dim3(cdiv(N, 256), cdiv(M, 16 * T), shares), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, shares, kper, g_part_buf)
+    if (mt == 4) GS(4); else GS(8);
+#undef GS
     count_launch();
     add_up(shares);
     keep();

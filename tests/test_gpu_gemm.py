@@ -454,6 +454,14 @@ def test_narrow_matrix_under_many_rows_split_over_k(hip, monkeypatch, M, N, K, N
     assert l1 == l0 + 1, (l1, l0)        # the launch that adds the shares
 
 
+def load_from(hip, rng, N, K, base):
+    """A random Q4 matrix [N, K] from element `base` of map 1 on, blocks ahead of it that are weights too (others would take the
+    whole map off the matrix instructions); its values in float64."""
+    qt = quant.quantize_q4_0(rng.standard_normal(((N * K + base) // 32, 32), dtype=np.float32) * np.float32(0.05))
+    load_qtensor(hip, 1, qt)
+    return qt.dequant().astype(np.float64).reshape(-1)[base:].reshape(N, K)
+
+
 @pytest.mark.parametrize("M,N,K,base", [(1000, 3201, 128, 0), (777, 4100, 256, 64), (2049, 1537, 384, 32), (65, 4100, 4096, 0), (97, 1152, 6912, 128),
                                         (341, 13824, 1152, 0), (33, 4100, 4096, 32), (64, 1153, 6912, 0), (130, 515, 14336, 0)])
 def test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base):
@@ -461,14 +469,37 @@ def test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base):
     unequal length, fewer steps of K than the ring has stages, weights that begin at an odd block."""
     note(f"gemm q4 ring M={M} N={N} K={K} base={base}")
     rng = np.random.default_rng(M + N)
-    qt = quant.quantize_q4_0(rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05))
+    W = load_from(hip, rng, N, K, base)
     x = rng.standard_normal((M, K), dtype=np.float32) * np.exp(rng.standard_normal((M, 1))).astype(np.float32)
-    load_qtensor(hip, 1, qt, offset=base, total=base + qt.size)
     f32map(hip, 0, M * K + M * N + N, x.reshape(-1))
     hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [base]), up(hip, [M * K]), M, K, N, 1)
     got = read(hip, 0, M * K, M * N + N)
-    want = x.astype(np.float64) @ qt.dequant().astype(np.float64).T
+    want = x.astype(np.float64) @ W.T
     for m in range(0, M, max(1, M // 64)):
         assert rel_l2(got[m * N:(m + 1) * N], want[m]) < TOL_Q4, m
     assert rel_l2(got[(M - 1) * N:M * N], want[M - 1]) < TOL_Q4 and rel_l2(got[:M * N], want.reshape(-1)) < TOL_Q4
     assert not got[M * N:].any()                   # nothing beyond the last row
+
+
+@pytest.mark.parametrize("M,K,N", [(512, 4096, 4096), (400, 4096, 4100), (256, 4096, 6144)])
+def test_weights_from_an_odd_block_run_over_shares_of_k(hip, M, K, N):
+    """A matrix that begins at an odd block, narrow under many rows: shares of K (conversion, product, sum: three launches) whose
+    sum also stores the add behind the matmul (three again)."""
+    note(f"gemm q4 odd block M={M} N={N} K={K}")
+    rng = np.random.default_rng(M + N)
+    W = load_from(hip, rng, N, K, 32)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    hid = rng.standard_normal((M, N), dtype=np.float32)
+    y0, h0 = M * K, M * K + M * N
+    f32map(hip, 0, h0 + M * N, np.concatenate([x.reshape(-1), np.zeros(M * N, np.float32), hid.reshape(-1)]))
+    hy, hh = up(hip, y0 + np.arange(M * N)), up(hip, h0 + np.arange(M * N))
+    for add in (False, True):
+        hip.batch_begin()
+        hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [32]), up(hip, [y0]), M, K, N, 1)
+        if add:
+            hip.map_op2_dev(0, A.OP_ADD, hh, hy, hh, M * N)
+        hip.batch_end()
+        assert hip.get_last_barrier_count() == 3, add
+    y = x.astype(np.float64) @ W.T
+    assert rel_l2(read(hip, 0, y0, M * N).reshape(M, N), y) < TOL_Q4
+    assert rel_l2(read(hip, 0, h0, M * N).reshape(M, N), y + hid) < TOL_Q4
