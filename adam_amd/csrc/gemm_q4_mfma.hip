@@ -333,7 +333,7 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
 // ---- more than 64 activation rows ------------------------------------------------------------------------------------
 // Eight waves of 64 weight rows each, side by side, over 32 MA activation rows: a wave has 2 x MA results of 32 x 32.  A step
 // is 64 columns (two blocks); its packed weights (16 KB), their scales (2 KB) and both planes of the activations (8 KB per 32
-// rows) go straight to LDS, a ring of three stages and more.  512 x 28672 x 4096: 319 -> 246 us = 489 TFLOP/s (matrix pipe
+// rows) go straight to LDS, a ring of four stages (MA = 2) or three (MA = 4).  512 x 28672 x 4096: 319 -> 246 us = 489 TFLOP/s (matrix pipe
 // 58 % busy on the CUs that have a workgroup).  What bounds it is the vector work beside the matrix instructions (a
 // multiply-add per result and block, the unpacking): they share a wave's issue, so what counts is that no instruction of
 // either kind waits for another.  LDS reads without bank conflicts: 266 -> 246 us.
@@ -351,7 +351,8 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
                uint32_t K, uint32_t N, uint32_t M, uint32_t gbase, uint32_t c_val, uint32_t by_val, uint32_t pairs_per, float* out,
                float* __restrict__ part, const uint32_t* __restrict__ lc, const float* __restrict__ scale, GemmSegs segs) {
   constexpr uint32_t BM = 32u * MA, BN = 512u, RING_STAGE = RING_W + RING_S + MA * 8192u;
-  constexpr int LOADS = 3 + MA, RING_ST = MA == 1 ? 6 : MA == 2 ? 4 : 3;      // loads of a wave and stage: 2 of weights, 1 of scales, MA of activations
+  constexpr int LOADS = 3 + MA, RING_ST = MA == 2 ? 4 : 3;      // loads of a wave and stage: 2 of weights, 1 of scales, MA of activations
+  static_assert(MA == 2 || MA == 4, "stages and schedule");
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING_ST * RING_STAGE];
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t r32 = lane & 31u, h = lane >> 5;
@@ -455,13 +456,9 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
           if (b == 1 && x == 0 && m < 2) read_w(sn, m);
           if (b == 1 && x == 1 && m >= 2) take_w(m - 2);
           if (b == 0 && m == 0) for (int u = x * 4 / NT; u < (x + 1) * 4 / NT; u++) unpack(1, u >> 1, u & 1);
-          if (b == 1 && MA > 1 && x >= 2 && m == 0) for (int u = (x - 2) * 4 / (NT - 2); u < (x - 1) * 4 / (NT - 2); u++) unpack(0, u >> 1, u & 1);
+          if (b == 1 && x >= 2 && m == 0) for (int u = (x - 2) * 4 / (NT - 2); u < (x - 1) * 4 / (NT - 2); u++) unpack(0, u >> 1, u & 1);
           if (b == 1) for (int u = (4 * x + m) * LOADS / (4 * NT); u < (4 * x + m + 1) * LOADS / (4 * NT); u++) load(u, s + RING_ST - 1u, into);
           __builtin_amdgcn_sched_barrier(0);
-        }
-        if (MA == 1 && b == 1 && x == 1) {
-#pragma unroll
-          for (int u = 0; u < 4; u++) unpack(0, u >> 1, u & 1);
         }
       }
     }
