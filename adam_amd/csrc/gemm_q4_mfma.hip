@@ -1119,49 +1119,47 @@ bool launch_attn_merge_rows_f16(const Map* ma, const float* partial, uint32_t o0
 // survive into a later state with the same count).
 void gemm_act_forget() { g_xh_key.valid = false; }
 
-// Preconditions (checked by the caller against the host copies of the handles): Q4 map whose blocks
-// in range are in the block16 layout, K a multiple of 128, weight bases block aligned, all operands
-// in range.
-// How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: MA > 0
-// k_gemm_q4_ring<MA>, 0 the tiled kernel; over how many shares of K.  Estimates in us, fitted to M = 33 .. 512 over 28672 x
-// 4096, 6144 x 4096, 4096 x 4096, 4096 x 14336, 13824 x 1152 and 1152 x 6912 (within 20 %; between near equals either is
-// fine): a ring step takes 1.5 (MA = 2) or 2.3 us (MA = 4) alone and 2.1 or 3.4 with all CUs at work, a 128-column step of
-// the 64 x 64 tile 1.3 .. 2.3, of the 64 x 256 tile 3; shares cost a launch and the passes over the partial sums.
-// Measured either way (us): 48 x 4096 x 14336 137 -> 33 over 16 shares, 100 x 4096 x 4096 43 -> 32, 48 x 13824 x 1152 16
-// (21 over two shares).
+// How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 0
+// k_gemm_q4_ring<ma>, 0 the tiled kernel; over how many shares of K.
+// 33 .. 64 rows: tiled; its 64 x 256 tile over shares takes 3 us a 128-column step where all shares are at work, and 9 for the
+// two launches (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x 2048: 23 -> 17 over four).
+// More: the least of these estimates, in us, fitted to both kernels over 2900 plans of 65 .. 2049 rows by 512 .. 32000 x 128 ..
+// 14336 (the plan it picks takes 0.2 % longer than the best one in the mean, 9 % at most).  Tiled, by the tile it would take
+// (below): 128-column steps of 1.27 us while no CU has a second 64 x 64 tile and 0.72 more for each further one, 4.0 and 2.7
+// more for every two rounds of 64 x 128, 4.6 a round of 256 x 128.  Ring: 64-column steps of 1.7 (ma = 2) or 3.0 us, up to a
+// fifth more as the CUs fill; shares cost their second launch and a pass over the sums each.
+// The ring reads the scales of two blocks as one word and keeps a lane's place in the rows in 32 bits (in the matrix too: a Q4
+// map here has fewer than 2^32 elements): matrices that begin at an odd block stay on the tiled kernel, a narrow one from 128
+// rows on over 2 .. 4 shares (256 x 128 tile; 512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four).
 struct GemmPlan { int ma; uint32_t shares; };
 static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
-  const uint64_t cu = (uint64_t)g.n_cu, steps = cdiv(K, 128), pairs = K / 64;
-  const auto cdiv64 = [](uint64_t x, uint64_t y) { return (x + y - 1) / y; };
-  const uint64_t small = cdiv64(N, 64) * cdiv64(M, 64);
-  const double passes = (double)M * (double)N * 4.0 / 4.5e6;              // one pass over a result
-  double best = (double)steps * (small <= cu / 2 ? 1.3 : small <= cu ? 1.75 : 2.3) * std::max(1.0, (double)small / (3.0 * (double)cu));
-  if (small * 64 * 64 >= 96 * 128 * cu) best = 1e30;                      // (a large product: the ring's)
-  GemmPlan p = {0, 1};
-  if (tuning("ADAMAH_GEMM_SPLITK", 1) == 0) return p;
+  const auto up = [](uint64_t x, uint64_t y) { return (x + y - 1) / y; };
+  const auto wgs = [&](uint64_t n, uint64_t m) { return up(N, n) * up(M, m); };
+  const uint64_t cu = (uint64_t)g.n_cu, steps = up(K, 128), pairs = K / 64, most = 16;
+  if (tuning("ADAMAH_GEMM_SPLITK", 1) == 0) return {0, 1};
+  double best = 0.55 + 0.72 * (double)up(wgs(64, 64), cu);                // (per step)
+  if (M > 64 && wgs(256, 128) * 4 >= 3 * cu) best = 4.6 * (double)up(wgs(256, 128), cu);
+  else if (M > 64 && wgs(64, 128) >= 2 * cu) best = 1.3 + 2.7 * (double)up(wgs(64, 128), 2 * cu);
+  best = 4.5 + best * (double)steps;
   if (M <= 64) {
-    const uint64_t w = cdiv64(N, 256);
-    uint64_t sp = std::min<uint64_t>(16, std::max<uint64_t>(1, 2 * cu / w));
+    uint64_t sp = std::min<uint64_t>(most, std::max<uint64_t>(1, 2 * cu / up(N, 256)));
     while (sp > 1 && K / sp < 512u) sp--;
-    if (sp > 1 && 3.0 * (double)cdiv64(steps, sp) + 9.0 < (double)steps * (small <= cu / 2 ? 1.3 : small <= cu ? 1.75 : 2.2)) p.shares = (uint32_t)sp;
-    return p;
+    return {0, sp > 1 && 3.0 * (double)up(steps, sp) + 9.0 < best ? (uint32_t)sp : 1u};
   }
   if (b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {
-    // not the ring (it reads the scales of two blocks as one word): a narrow matrix from 128 rows on in 256 x 128 tiles over
-    // 2 .. 4 shares where they fill the CUs (512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four)
-    const uint64_t w = cdiv64(N, 256) * cdiv64(M, 128);
-    if (M < 128 || w * 4 >= 3 * cu) return p;
-    uint64_t sp = std::min<uint64_t>(4, cu / std::max<uint64_t>(1, w));
+    const uint64_t w = wgs(256, 128);
+    if (M < 128 || w * 4 >= 3 * cu) return {0, 1};
+    uint64_t sp = std::min<uint64_t>(std::min<uint64_t>(4, most), cu / std::max<uint64_t>(1, w));
     while (sp > 1 && K / sp < 1024u) sp--;
-    if (w * sp * 4 >= 3 * cu) p.shares = (uint32_t)sp;
-    return p;
+    return {0, sp > 1 && w * sp * 4 >= 3 * cu ? (uint32_t)sp : 1u};
   }
+  const double pass = (double)M * (double)N * 4.0 / 4.5e6;                // one pass over a result
+  GemmPlan p = {0, 1};
   for (int ma = 2; ma <= 4; ma += 2) {
-    const uint64_t tiles = cdiv64(N, 512) * cdiv64(M, 32 * (uint64_t)ma);
-    for (uint64_t sp = 1; sp <= 16 && sp * 4 <= pairs && (sp == 1 || tiles * sp <= cu); sp++) {
-      const uint64_t wgs = tiles * sp;
-      const double full = std::min(1.0, (double)wgs / (double)cu), t = ma == 2 ? 1.5 + 0.6 * full : 2.3 + 1.1 * full;
-      const double us = (double)cdiv64(wgs, cu) * ((double)cdiv64(pairs, sp) * t + 10.0) + (sp > 1 ? 4.0 + (2.0 * (double)sp + 1.0) * passes : 0.0);
+    const uint64_t tiles = wgs(512, 32 * (uint64_t)ma);
+    for (uint64_t sp = 1; sp <= most && (sp == 1 || (sp * 4 <= pairs && tiles * sp <= cu)); sp++) {
+      const double full = std::min(1.0, (double)(tiles * sp) / (double)cu), step = ma == 2 ? 1.7 + 0.35 * full : 3.0 + 0.8 * full;
+      const double us = (double)up(tiles * sp, cu) * ((double)up(pairs, sp) * step + 7.0) + (sp > 1 ? 9.0 + (double)(sp + 1) * pass : 0.0);
       if (us < best) { best = us; p = {ma, (uint32_t)sp}; }
     }
   }
@@ -1173,6 +1171,9 @@ bool gemm_q4_adds(uint32_t M, uint32_t K, uint32_t N, int64_t b) {
   return p.ma > 0 || p.shares > 1;
 }
 
+// Preconditions (checked by the caller against the host copies of the handles): Q4 map whose blocks
+// in range are in the block16 layout, K a multiple of 128, weight bases block aligned, all operands
+// in range.
 int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const uint32_t* lb, const uint32_t* lc,
                         uint32_t M, uint32_t K, uint32_t N, uint32_t n_ops, bool q8, float* out, int64_t a_host,
                         int64_t c_host, const GemmSegs* segs, int64_t b_host) {
