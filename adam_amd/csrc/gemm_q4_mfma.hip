@@ -1135,8 +1135,8 @@ struct GemmPlan { int ma; uint32_t shares; };
 static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   const auto up = [](uint64_t x, uint64_t y) { return (x + y - 1) / y; };
   const auto wgs = [&](uint64_t n, uint64_t m) { return up(N, n) * up(M, m); };
-  const uint64_t cu = (uint64_t)g.n_cu, steps = up(K, 128), pairs = K / 64, most = 16;
-  if (tuning("ADAMAH_GEMM_SPLITK", 1) == 0) return {0, 1};
+  const uint64_t cu = (uint64_t)g.n_cu, steps = up(K, 128), pairs = K / 64, most = tuning("ADAMAH_GEMM_SPLITK", 1) ? 16 : 1;
+  const int ring = tuning("ADAMAH_GEMM_RING", 1);
   double best = 0.55 + 0.72 * (double)up(wgs(64, 64), cu);                // (per step)
   if (M > 64 && wgs(256, 128) * 4 >= 3 * cu) best = 4.6 * (double)up(wgs(256, 128), cu);
   else if (M > 64 && wgs(64, 128) >= 2 * cu) best = 1.3 + 2.7 * (double)up(wgs(64, 128), 2 * cu);
@@ -1146,13 +1146,14 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     while (sp > 1 && K / sp < 512u) sp--;
     return {0, sp > 1 && 3.0 * (double)up(steps, sp) + 9.0 < best ? (uint32_t)sp : 1u};
   }
-  if (b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {
+  if (ring == 0 || b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {
     const uint64_t w = wgs(256, 128);
     if (M < 128 || w * 4 >= 3 * cu) return {0, 1};
     uint64_t sp = std::min<uint64_t>(std::min<uint64_t>(4, most), cu / std::max<uint64_t>(1, w));
     while (sp > 1 && K / sp < 1024u) sp--;
     return {0, sp > 1 && w * sp * 4 >= 3 * cu ? (uint32_t)sp : 1u};
   }
+  if (ring == 2) best = 1e30;
   const double pass = (double)M * (double)N * 4.0 / 4.5e6;                // one pass over a result
   GemmPlan p = {0, 1};
   for (int ma = 2; ma <= 4; ma += 2) {

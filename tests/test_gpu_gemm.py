@@ -503,3 +503,74 @@ def test_weights_from_an_odd_block_run_over_shares_of_k(hip, M, K, N):
     y = x.astype(np.float64) @ W.T
     assert rel_l2(read(hip, 0, y0, M * N).reshape(M, N), y) < TOL_Q4
     assert rel_l2(read(hip, 0, h0, M * N).reshape(M, N), y + hid) < TOL_Q4
+
+
+@pytest.mark.parametrize("M,K,Ns,add", [
+    (600, 256, (7200, 7230), False), (513, 256, (100, 14000, 333), False), (65, 128, (500, 36, 700), False), (130, 512, (512, 512), False),
+    (600, 256, (14401,), True), (341, 1152, (13824,), True), (70, 384, (515,), True)])
+def test_ring_stores_stacked_results_and_adds_in_one_share(hip, monkeypatch, M, K, Ns, add):
+    """The ring kernel's own stores (two launches with the conversion: no sum behind it): results of stacked matrices whose border
+    lies inside a workgroup's 512 weight rows, and the add behind a single one; 64 and 128 activation rows a workgroup."""
+    monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
+    monkeypatch.setenv("ADAMAH_GEMM_SPLITK", "0")
+    note(f"gemm q4 ring, one share M={M} K={K} Ns={Ns} add={add}")
+    rng = np.random.default_rng(M + sum(Ns))
+    W = load_from(hip, rng, sum(Ns), K, 0)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    c0, at = [], M * K + 8
+    for n in reversed(Ns):                         # results in reverse order, apart from one another
+        c0.insert(0, at)
+        at += M * n + 24
+    hid = rng.standard_normal(M * Ns[0]).astype(np.float32) if add else np.zeros(0, np.float32)
+    f32map(hip, 0, at + hid.size, np.concatenate([x.reshape(-1), np.zeros(at - M * K, np.float32), hid]))
+    hip.batch_begin()
+    r = 0
+    for n, c in zip(Ns, c0):
+        hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [r * K]), up(hip, [c]), M, K, n, 1)
+        r += n
+    if add:
+        hh = up(hip, at + np.arange(hid.size))
+        hip.map_op2_dev(0, A.OP_ADD, hh, up(hip, c0[0] + np.arange(hid.size)), hh, hid.size)
+    hip.batch_end()
+    assert hip.get_last_barrier_count() == 2
+    got = read(hip, 0, 0, at + hid.size)
+    y, r = x.astype(np.float64) @ W.T, 0
+    for n, c in zip(Ns, c0):
+        for m in range(0, M, 7):
+            assert rel_l2(got[c + m * n:c + (m + 1) * n], y[m, r:r + n]) < TOL_Q4, (n, m)
+        assert rel_l2(got[c:c + M * n].reshape(M, n), y[:, r:r + n]) < TOL_Q4
+        got[c:c + M * n] = 0.0
+        r += n
+    if add:
+        assert rel_l2(got[at:], y.reshape(-1) + hid) < TOL_Q4
+    assert not got[M * K:at].any()                 # nothing beside the results
+
+
+@pytest.mark.parametrize("split", ["0", "1"])
+@pytest.mark.parametrize("M,N,K,base", [(1000, 3201, 128, 0), (777, 4100, 256, 64), (2049, 1537, 384, 64), (65, 515, 128, 0), (129, 511, 14336, 0),
+                                        (300, 9000, 640, 128)])
+def test_ring_at_ragged_ends(hip, monkeypatch, M, N, K, base, split):
+    """The ring kernel where the rule would not take it as well: fewer steps of K than it has stages, rows and weight rows past the
+    last tile, shares of unequal length."""
+    monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
+    monkeypatch.setenv("ADAMAH_GEMM_SPLITK", split)
+    test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
+
+
+def test_ring_off_leaves_the_tiled_kernel_its_shares(hip, monkeypatch):
+    """Either switch alone: without the ring a narrow matrix runs over shares (three launches), without shares in one (two)."""
+    rng = np.random.default_rng(5)
+    M, K, N = 512, 4096, 4096
+    W = load_from(hip, rng, N, K, 0)
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    want = x.astype(np.float64) @ W.T
+    for ring, split, launches in (("0", "1", 3), ("0", "0", 2), ("1", "0", 2), ("2", "0", 2), ("1", "1", 3)):
+        monkeypatch.setenv("ADAMAH_GEMM_RING", ring)
+        monkeypatch.setenv("ADAMAH_GEMM_SPLITK", split)
+        note(f"gemm q4 ring={ring} split={split}")
+        f32map(hip, 0, M * K + M * N, x.reshape(-1))
+        hip.batch_begin()
+        hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [0]), up(hip, [M * K]), M, K, N, 1)
+        hip.batch_end()
+        assert hip.get_last_barrier_count() == launches, (ring, split)
+        assert rel_l2(read(hip, 0, M * K, M * N).reshape(M, N), want) < TOL_Q4, (ring, split)
