@@ -25,9 +25,12 @@ namespace adamah {
 // What the kernels take, from either spec.  size: chunk or window.  p1, p2: chunk: the penalty's two factors per head,
 // window: slope and sink per head.
 struct ASpec {
-  uint32_t heads, kv_heads, dim, vdim, size, x, x_stride, x_q, x_k, x_v, p1, p2;
+  uint32_t heads, kv_heads, dim, vdim, size;
+  uint64_t x;                       // (of the portion at hand: a later sequence's may lie beyond 2^32)
+  uint32_t x_stride, x_q, x_k, x_v, p1, p2;
   float scale, eps;
-  uint32_t out, out_stride, k_off, v_off, seq_stride, has_sink, qk_norm, temp_every;
+  uint64_t out;
+  uint32_t out_stride, k_off, v_off, seq_stride, has_sink, qk_norm, temp_every;
   float softcap, temp_coef;
 };
 #define MAX_SPANS 64u
@@ -674,7 +677,7 @@ static int run_attention(Map* ma, const ASpec& s, uint32_t cache_map, uint32_t n
     return mc->dtype == DTYPE_F32 ? run_step<float, WIN>(s, act, (float*)mc->buf, n_seq, seq0, pos)
                                   : run_step<bf16_t, WIN>(s, act, (bf16_t*)mc->buf, n_seq, seq0, pos);
   ASpec p = s;
-  for (uint32_t q = 0; q < n_seq; q++, p.x += rows * s.x_stride, p.out += rows * s.out_stride) {
+  for (uint32_t q = 0; q < n_seq; q++, p.x += (uint64_t)rows * s.x_stride, p.out += (uint64_t)rows * s.out_stride) {
     const uint64_t at = slot + (uint64_t)q * s.seq_stride;
     if (int r = mc->dtype == DTYPE_F32 ? run_portion<float, WIN>(p, act, (float*)mc->buf + at, rows, pos)
                                        : run_portion<bf16_t, WIN>(p, act, (bf16_t*)mc->buf + at, rows, pos)) return r;

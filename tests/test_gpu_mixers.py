@@ -475,6 +475,32 @@ def test_chunk_attention_over_several_spans_of_keys(hip, dtype):
         run(1, 1, 0, pos)
 
 
+def test_chunk_attention_of_sequences_beyond_2_to_the_32_elements(hip):
+    """Two portions whose border lies at element 2^32 of the activation map (17 GB, two elements a pack): the second sequence's rows
+    are read there and not at the map's start."""
+    note("chunk attention across 2^32 elements")
+    H, G, D, V, C, rows = 2, 1, 16, 16, 32, 5
+    xs, top = H * D + G * (D + V), 1 << 32
+    kv = G * C * D
+    x = np.random.default_rng(3).standard_normal((2 * rows, xs)).astype(np.float32)
+    x0 = top - rows * xs
+    hip.map_create_typed(CA, A.DTYPE_F32, 1, 4 * kv)
+    spec = lambda at: up(hip, A.ChunkAttnSpec(heads=H, kv_heads=G, dim=D, vdim=V, chunk=C, x=at, x_stride=xs, x_q=0, x_k=H * D, x_v=H * D + G * D, r1=8, r2=8,
+                                              scale=0.25, eps=1e-4, out=64, out_stride=H * V, cache_map=CA, k_off=0, v_off=kv, seq_stride=2 * kv).words())
+    got = []
+    try:
+        for packs, at in ((top // 2 + rows * xs, x0), (1 << 12, 2048)):
+            hip.map_create_typed(WS, A.DTYPE_F32, 2, packs)
+            hip.set_dtype(A.DTYPE_F32)
+            assert hip.scatter_contiguous(WS, 4, np.full(4, 0.1, np.float32), n_locs=2) == 0
+            assert hip.scatter_contiguous(WS, at // 2, x.reshape(-1), n_locs=x.size // 2) == 0
+            hip.chunk_attention_seqs_dev(WS, spec(at), 2, rows, 0, 0)
+            got.append(hip.gather(WS, np.arange(32, 32 + rows * H * V, dtype=np.uint32)).view(np.float32).copy())
+    finally:
+        f32map(hip, WS, 64)
+    assert np.abs(got[1]).max() > 0.1 and np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("cut", ["whole", "pairs", "alone"])
 def test_a_standing_out_key_is_seen_inside_its_chunk_only(hip, dtype, cut):
