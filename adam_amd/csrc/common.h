@@ -176,9 +176,10 @@ size_t launch_argmax_run(const std::vector<PendOp>& q, size_t i, int* rc);   // 
 int launch_argmax_direct(const PendOp& p);   // gemv_q.hip: one queued Q8 GEMV + argmax
 int launch_rmsnorm_v(const PendOp& p);
 bool row_op_deferrable(const PendOp& p);                                  // rowprep.hip
-// Element ranges (start, length) of the activation map a queued row op reads or writes; false: not known on the host.
-bool launch_qk_rows(Map* m, const uint32_t* hq, uint32_t hqw, const uint32_t* hk, uint32_t hkw, const uint32_t* hd, uint32_t n_tok,   // rowprep.hip
+// rowprep.hip: QK norm and rotation of consecutive tokens in one launch; false: not a case for it, nothing done
+bool launch_qk_rows(Map* m, const uint32_t* hq, uint32_t hqw, const uint32_t* hk, uint32_t hkw, const uint32_t* hd, uint32_t n_tok,
                     uint32_t q_rows, uint32_t q_dim, uint32_t k_rows, uint32_t k_dim, uint32_t pos0, float base, int* rc);
+// Element ranges (start, length) of the activation map a queued row op reads or writes; false: not known on the host.
 bool row_op_ranges(const PendOp& p, std::vector<std::pair<uint64_t, uint64_t>>* out);   // rowprep.hip
 size_t launch_row_run(const std::vector<PendOp>& q, size_t i, int* rc);   // rowprep.hip
 // a rotation / row copy with more rows than a row run holds (PendOp.op == 1): alone, or rotation + rotation + KV append

@@ -18,6 +18,9 @@
 //
 // Tiled form: workgroup = NW waves, each with R tiles of 16 weight rows = 16 NW R weight rows x 16 MT activation
 // rows; one step = 128 weights of K (four blocks).
+// Ring form (more than 64 activation rows): eight waves of 64 weight rows over 64 or 128 activation rows, on 32x32x16
+// instructions, weights, scales and activations straight to a ring of LDS stages.
+// Either over shares of K, which k_gemm_splitk_sum adds up; gemm_plan says which.
 // K-split form (few activation rows): the waves share R tiles of 16 weight rows and take every NWV-th step of K
 // each, so that small matrices still spread over the whole chip; their partial tiles are summed through LDS in
 // a fixed order.
@@ -333,8 +336,8 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
 // ---- more than 64 activation rows ------------------------------------------------------------------------------------
 // Eight waves of 64 weight rows each, side by side, over 32 MA activation rows: a wave has 2 x MA results of 32 x 32.  A step
 // is 64 columns (two blocks); its packed weights (16 KB), their scales (2 KB) and both planes of the activations (8 KB per 32
-// rows) go straight to LDS, a ring of four stages (MA = 2) or three (MA = 4).  512 x 28672 x 4096: 319 -> 246 us = 489 TFLOP/s (matrix pipe
-// 58 % busy on the CUs that have a workgroup).  What bounds it is the vector work beside the matrix instructions (a
+// rows) go straight to LDS, a ring of four stages (MA = 2) or three (MA = 4).  512 x 28672 x 4096: 317 -> 248 us = 485
+// TFLOP/s.  What bounds it is the vector work beside the matrix instructions (a
 // multiply-add per result and block, the unpacking): they share a wave's issue, so what counts is that no instruction of
 // either kind waits for another.  LDS reads without bank conflicts: 266 -> 246 us.
 // v_mfma_f32_32x32x16_f16: lane l supplies row l % 32, k = 8 (l / 32) .. + 7 of either operand and receives rows

@@ -81,7 +81,7 @@ __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM /
     if (i < NTM) b[h][i] = *(const bf8_t*)(lb + buf * (BM * 64) + (wm + 16u * i + c) * 64u + at);
     else a[h][i - NTM] = *(const bf8_t*)(la + buf * (BN * 64) + (wn + 16u * (i - NTM) + c) * 64u + at);
   };
-  // four products, then a few of the next half's reads and (LD) one of the loads, and so on: the matrix pipe is never
+  // four products, then a few of the next half's reads and (second half) some of the loads, and so on: the matrix pipe is never
   // behind a run of either
   constexpr int NP = NTN * NTM / 4, READS = NP > 1 ? (NTN + NTM + NP - 2) / (NP - 1) : NTN + NTM, LOADS_EACH = (LOADS + NP - 1) / NP;
   const auto half = [&](int h, uint32_t from, uint32_t k, uint32_t into) {
