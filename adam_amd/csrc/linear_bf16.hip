@@ -738,8 +738,8 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
     float* op = (float*)mo->buf;
     if (!s.ready) operand_rows<float>(s, act, op + s.opnd, row_idx, rows);
     // Long rows in three bfloat16 pieces (the launch that splits them: 4 us; 88 rows of 512: 15.6 us on the float32
-    // instruction, 11.2 in pieces; of 256: 8.3 and 8.2; of 128: 5.1 and 6.6)
-    if (s.k_stride > 256u && scratch_need(g_split, (size_t)rows * 3 * s.k_stride * sizeof(bf16_t)) == ADAMAH_OK) {
+    // instruction, 11.2 in pieces; of 256: 8.3 and 8.2; of 128: 5.1 and 6.6).  k_split_rows counts four columns a thread in 32 bits.
+    if (s.k_stride > 256u && (uint64_t)rows * s.k_stride < (1ull << 34) && scratch_need(g_split, (size_t)rows * 3 * s.k_stride * sizeof(bf16_t)) == ADAMAH_OK) {
       bf16_t* X = (bf16_t*)g_split.p;
       k_split_rows<<<cdiv((uint64_t)rows * s.k_stride / 4, 256), 256, 0, g.stream>>>(op + s.opnd, X, s.k_stride, rows);
       count_launch();
