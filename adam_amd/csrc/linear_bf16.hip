@@ -241,9 +241,14 @@ k_operand_rows(const LinSpec s, float* act, T* __restrict__ dst, const uint32_t*
 // Long rows, few of them: a row's latency is the launch's, so 1024 threads a row; many rows fill the CUs with 256 each, and
 // rows of one float a thread have nothing to gain (300 rows of 64 on the wide form with 1024 threads: 5.7 us, so: 3.6; 12 rows
 // of 100: 4.7 and 3.6).
+// Rows with a branch have a form of their own, eight elements a thread: the threads that hold the row, and none of the wide
+// form's registers (with the rule of the others, in us, a product of 16 columns behind them: 300 rows of 2048 20.8, so: 11.9;
+// 2048 rows of 4096 43.6 and 34.4; 2 rows of 4096 12.0 and 10.5; 600 rows of 8192 41.4 and 31.8).
 template <class T>
 static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* row_idx, uint32_t rows) {
-  if (s.k <= 256u) k_operand_rows<T, 256, false><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
+  if (s.k <= 256u || (s.branched && s.k <= 2048u)) k_operand_rows<T, 256, false><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
+  else if (s.branched && s.k <= 4096u) k_operand_rows<T, 512, false><<<rows, 512, 0, g.stream>>>(s, act, dst, row_idx);
+  else if (s.branched) k_operand_rows<T, 1024, false><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
   else if (s.k > 1024u && rows <= 2u * (uint32_t)g.n_cu) k_operand_rows<T, 1024, true><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
   else k_operand_rows<T, 256, true><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
   count_launch();

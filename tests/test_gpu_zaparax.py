@@ -71,6 +71,30 @@ def test_linear_with_a_branch_added_kept_rows_and_a_tail(hip, dtype, rows, n, k,
         p.same(WS, at["out"], rows * (pairs + 1) - 1, tol, "pairs")
 
 
+@pytest.mark.parametrize("rows,k", [(2, 2048), (3, 2050), (600, 2049), (5, 4096), (2, 4098), (600, 4097), (4, 8192), (3, 8201), (530, 300)])
+def test_branched_rows_of_every_thread_count(hip, rows, k):
+    """Rows with a branch on 256, 512 and 1024 threads: as long as their registers hold, and just longer."""
+    note(f"branched rows {rows} k {k}")
+    rng = np.random.default_rng(k + rows)
+    n, ks = 16, r64(k)
+    at, pos = {}, 3
+    for name, sz in (("src", rows * k), ("br", rows * k), ("wt", k), ("bw", k), ("res", rows * k), ("keep", rows * k), ("out", rows * n)):
+        at[name] = pos
+        pos += sz
+    p = Pair(hip, pos + 8, wt=n * ks, opnd=rows * ks, dtype="float32")
+    W = np.zeros((n, ks), np.uint16)
+    W[:, :k] = f32_to_bf16((rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32))
+    p.put(WT, 0, W)
+    p.put(WS, 0, rng.standard_normal(pos))
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=ks, src=at["src"], src_stride=k, groups=1, eps=1e-4, wt=at["wt"], wt_len=k, wt_add=1.0,
+                        branch=at["br"], branch_stride=k, branch_wt=at["bw"], branched=2, res_out=at["res"], res_stride=k,
+                        keep=at["keep"], keep_stride=k, kept=1, opnd=0, out=at["out"], out_stride=n)
+    p.call("linear_dev", WS, OP, WT, p.up(spec.words()), 0, rows)
+    # float32 throughout, sums of at most 8201 squares or products: 2e-5 as for the sums and operands above
+    for name, sz in (("res", rows * k), ("keep", rows * k), ("out", rows * n)):
+        p.same(WS, at[name], sz, 2e-5, name)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows,n,k,groups,epi", [(1, 51, 330, 3, 0), (1, 64, 1100, 10, 1), (3, 70, 64, 2, 0), (40, 129, 96, 1, 1),
                                                  (130, 200, 256, 16, 0)])
