@@ -419,10 +419,17 @@ __device__ __forceinline__ void put_out(const LinSpec& s, float* act, uint32_t r
     *(f4_t*)d = v;
     return;
   }
+  // (a loop for each form: with the form asked for at every value, float32 24 x 1001 x 60 took 4.44 us, so: 4.19)
+  if (s.biased) {
 #pragma unroll
-  for (int i = 0; i < 4; i++) if (n0 + i < s.n) {
-    const float y = s.biased ? v[i] + act[s.bias + n0 + i] : v[i];
-    d[i] = s.epi == 1u ? d[i] + y : y;
+    for (int i = 0; i < 4; i++) if (n0 + i < s.n) v[i] += act[s.bias + n0 + i];
+  }
+  if (s.epi == 1u) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) if (n0 + i < s.n) d[i] += v[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) if (n0 + i < s.n) d[i] = v[i];
   }
 }
 // gate rows n0 .. n0 + 3 and their up rows -> the activation's operand rows
