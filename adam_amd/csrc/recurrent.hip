@@ -278,8 +278,14 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
       float z[CH];
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) z[t] = dec[(uint64_t)min(c0 + t, m - 1u) * dec_stride + h * D + d];
+      const auto decay = [&](int t) { return fminf(ea * softplus_f(z[t] + bias), NO_MEMORY) * 1.44269504f; };
+      if (m - c0 >= CH) {                                    // (as in conv_silu_rows)
 #pragma unroll
-      for (int t = 0; t < (int)CH; t++) z[t] = fminf(ea * softplus_f(z[t] + bias), NO_MEMORY) * 1.44269504f;
+        for (int t = 0; t < (int)CH; t++) z[t] = decay(t);
+      } else {
+#pragma unroll
+        for (int t = 0; t < (int)CH; t++) if (c0 + t < m) z[t] = decay(t);
+      }
       float lg = 0.f;
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {

@@ -59,15 +59,26 @@ __device__ __forceinline__ void conv_silu_rows(const float* x, uint32_t x_stride
   }
 #pragma unroll
   for (int j = 0; j < TM; j++) wt[j] = (uint32_t)j < taps ? wt[j] : 0.f;
-#pragma unroll
-  for (int t = 0; t < (int)CH; t++) {
+  const auto row = [&](int t) {
     float a = bias;
 #pragma unroll
     for (int j = 0; j < TM; j++) a = fmaf(wt[j], in[t + TM - 1 - j], a);
-    y[t] = silu_f(a);
+    return silu_f(a);
+  };
+  // a whole chunk without a condition among its sixteen chains; of a shorter one only its rows (delta rule of 2 rows, 4 heads of
+  // 64: 29.0 us with all sixteen, 25.2 so)
+  if (m - r0 >= CH) {
+#pragma unroll
+    for (int t = 0; t < (int)CH; t++) y[t] = row(t);
+  } else {
+#pragma unroll
+    for (int t = 0; t < (int)CH; t++) {
+      y[t] = 0.f;
+      if (r0 + (uint32_t)t < m) y[t] = row(t);
+    }
   }
 #pragma unroll
-  for (int t = 0; t < (int)CH; t++) put(t, r0 + (uint32_t)t < m ? y[t] : 0.f);
+  for (int t = 0; t < (int)CH; t++) put(t, y[t]);
 }
 
 }  // namespace adamah
