@@ -72,13 +72,14 @@ k_experts_in(const bf16_t* __restrict__ W, float* act, const XSpec s) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ Chosen ch;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, kp = s.k_stride, half = kp >> 1, F = (s.ff + 15u) & ~15u;
-  // (no load under a condition, here and below: each would wait for the one before)
-  for (uint32_t i0 = threadIdx.x; i0 < kp; i0 += XSTEP * 4u) {
-    float v[4];
+  // (no load under a condition, here and below: each would wait for the one before; short rows have two values a thread)
+  constexpr uint32_t R = U == 1 ? 2 : 4;
+  for (uint32_t i0 = threadIdx.x; i0 < kp; i0 += XSTEP * R) {
+    float v[R];
 #pragma unroll
-    for (uint32_t u = 0; u < 4; u++) v[u] = act[s.x + min(i0 + u * XSTEP, s.width - 1u)];
+    for (uint32_t u = 0; u < R; u++) v[u] = act[s.x + min(i0 + u * XSTEP, s.width - 1u)];
 #pragma unroll
-    for (uint32_t u = 0; u < 4; u++) { const uint32_t i = i0 + u * XSTEP; if (i < kp) xs[PLANE(i, half)] = i < s.width ? v[u] : 0.f; }
+    for (uint32_t u = 0; u < R; u++) { const uint32_t i = i0 + u * XSTEP; if (i < kp) xs[PLANE(i, half)] = i < s.width ? v[u] : 0.f; }
   }
   choose_row(s, act, ch);
   const uint32_t n_tasks = ch.n * F;
@@ -117,17 +118,18 @@ k_experts_out(const bf16_t* __restrict__ W, float* act, const XSpec s, uint32_t 
   const uint32_t body = ch.n * fs, kp = body + (s.shared_ff ? s.shared_ff_stride : 0u), half = kp >> 1;
   const float sg = s.shared_ff ? sigmoid_f(act[s.logits + s.experts + s.identity]) : 0.f;
   const uint32_t last = ch.n ? ch.n - 1u : 0u;
-  // Eight values a thread asked for at once and no load under a condition, here and below (2048 rows of
+  // Eight values a thread (of a short row two) asked for at once and no load under a condition, here and below (2048 rows of
   // 6 x 1024 and 2048 columns, 33.5 MB: 17.9 us with each waiting for the one before, so: 14.2).
-  for (uint32_t i0 = threadIdx.x; i0 < kp; i0 += XSTEP * 8u) {
-    float v[8];
+  constexpr uint32_t R = U == 1 ? 2 : 8;
+  for (uint32_t i0 = threadIdx.x; i0 < kp; i0 += XSTEP * R) {
+    float v[R];
 #pragma unroll
-    for (uint32_t u = 0; u < 8; u++) {
+    for (uint32_t u = 0; u < R; u++) {
       const uint32_t i = min(i0 + u * XSTEP, kp - 1u), j = __umulhi(i, magic), c = i - j * fs;
       v[u] = act[i < body ? s.act + j * fs + min(c, s.ff - 1u) : s.shared_act + min(i - body, s.shared_ff - 1u)];
     }
 #pragma unroll
-    for (uint32_t u = 0; u < 8; u++) {
+    for (uint32_t u = 0; u < R; u++) {
       const uint32_t i = i0 + u * XSTEP, j = min(__umulhi(i, magic), last), c = i < body ? i - j * fs : i - body;
       if (i < kp) xs[PLANE(i, half)] = i < body ? (c < s.ff ? v[u] * ch.wt[j] : 0.f) : c < s.shared_ff ? v[u] * sg : 0.f;
     }
