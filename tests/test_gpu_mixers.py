@@ -120,6 +120,26 @@ def test_operand_rows_in_one_trip(hip, rows, k, groups, act, per_group):
     p.same(WS, out, rows * n, 2e-5, "out")
 
 
+@pytest.mark.parametrize("rows,n", [(33, 70), (100, 1001), (300, 515), (700, 2048), (2050, 2100)])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6])
+def test_linear_of_few_steps(hip, rows, n, steps):
+    """Products of as many 64-column steps as the ring of tiles has buffers, one more, one and two fewer, on small and large tiles."""
+    k = 64 * steps
+    note(f"linear rows {rows} n {n} k {k}")
+    rng = np.random.default_rng(rows + k)
+    f64 = lambda b: (b.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    W, x = (f32_to_bf16(rng.standard_normal(s).astype(np.float32)) for s in ((n, k), (rows, k)))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, x.size)
+    hip.scatter_contiguous(OP, 0, x.reshape(-1))
+    f32map(hip, WS, rows * n)
+    hip.linear_dev(WS, OP, WT, up(hip, A.LinearSpec(w=0, n=n, k=k, k_stride=k, opnd=0, ready=1, out=0, out_stride=n).words()), 0, rows)
+    got, want = read(hip, WS, 0, rows * n).reshape(rows, n), f64(x) @ f64(W).T
+    # exact products, float32 sums: k 2^-24 relative to the terms' root sum of squares at most
+    assert max(rel_l2(a, b) for a, b in zip(got, want)) < k * 2.0 ** -24
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows,n,k,epi,tail", [
     (33, 70, 320, 0, 0), (40, 131, 4096, 1, 0), (64, 96, 1088, 2, 0), (65, 201, 2048, 2, 41), (190, 2050, 1024, 0, 0), (300, 515, 3008, 1, 0),
