@@ -54,10 +54,10 @@ template <int R, int NW> struct TileRows {
 // BM tokens x BN matrix rows by WM x WN waves; acc[i][j]: matrix rows wn + 16 i, tokens wm + 16 j of a wave's part; la: ST
 // BN 64, lb: ST BM 64 elements.  A ring of ST buffers of 64 columns: a step's loads are asked for ST - 1 steps ahead.  A
 // step is two halves of 32 columns; a half's operands are read from LDS under the products of the half before, on both
-// sides of the step's one barrier.  What bounds it (256 x 256, two buffers): of the 1.75 us a step takes on all CUs the
-// products need 1.0, the loads alone 0.7 (23 TB/s out of the L2s), reads of LDS run beside both; loads and reads in a run
-// ahead of the products instead of among them: 1.95 us.  Columns k0 .. k1 of the tokens; column k of them meets column
-// k mod kp of the matrix (k1 at most PL kp).  PL = 3, tokens in pieces, the largest last: an infinite weight and a lower piece
+// sides of the step's one barrier.  What bounds it (256 x 256, two buffers): of the 1.7 us a step takes on all CUs the
+// products need 1.0 (matrix pipe 55 .. 62 % busy over a launch of 2048 rows), its loads come out of the L2s at 8.8 TB/s, reads
+// of LDS run beside both; loads and reads in a run ahead of the products instead of among them: 1.95 us.  Columns k0 .. k1 of
+// the tokens; column k of them meets column k mod kp of the matrix (k1 at most PL kp).  PL = 3, tokens in pieces, the largest last: an infinite weight and a lower piece
 // of 0 make no number where the whole product is infinite, so the lower pieces' sum counts only where it is finite (the
 // highest one's is infinite, or no number, exactly where the whole one is).
 template <int BM, int BN, int WM, int WN, int ST, int PL = 1>
