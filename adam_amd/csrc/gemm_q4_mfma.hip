@@ -1124,8 +1124,9 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 
 // How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 0
 // k_gemm_q4_ring<ma>, 0 the tiled kernel; over how many shares of K.
-// 33 .. 64 rows: tiled; its 64 x 256 tile over shares takes 3 us a 128-column step where all shares are at work, and 9 for the
-// two launches (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x 2048: 23 -> 17 over four).
+// 33 .. 64 rows: tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
+// a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x
+// 2048: 23 -> 17 over four; 64 x 28672 x 2048 38 in one, 44 in four, 64 x 28672 x 4096 67 and 62).
 // More: the least of these estimates, in us, fitted to both kernels over 2900 plans of 65 .. 2049 rows by 512 .. 32000 x 128 ..
 // 14336 (the plan it picks takes 0.2 % longer than the best one in the mean, 9 % at most).  Tiled, by the tile it would take
 // (below): 128-column steps of 1.27 us while no CU has a second 64 x 64 tile and 0.72 more for each further one, 4.0 and 2.7
@@ -1140,6 +1141,7 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   const auto wgs = [&](uint64_t n, uint64_t m) { return up(N, n) * up(M, m); };
   const uint64_t cu = (uint64_t)g.n_cu, steps = up(K, 128), pairs = K / 64, most = tuning("ADAMAH_GEMM_SPLITK", 1) ? 16 : 1;
   const int ring = tuning("ADAMAH_GEMM_RING", 1);
+  const double pass = (double)M * (double)N * 4.0 / 4.5e6;                // one pass over a result
   double best = 0.55 + 0.72 * (double)up(wgs(64, 64), cu);                // (per step)
   if (M > 64 && wgs(256, 128) * 4 >= 3 * cu) best = 4.6 * (double)up(wgs(256, 128), cu);
   else if (M > 64 && wgs(64, 128) >= 2 * cu) best = 1.3 + 2.7 * (double)up(wgs(64, 128), 2 * cu);
@@ -1147,7 +1149,9 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   if (M <= 64) {
     uint64_t sp = std::min<uint64_t>(most, std::max<uint64_t>(1, 2 * cu / up(N, 256)));
     while (sp > 1 && K / sp < 512u) sp--;
-    return {0, sp > 1 && 3.0 * (double)up(steps, sp) + 9.0 < best ? (uint32_t)sp : 1u};
+    const bool alone = up(N, 256) * sp <= cu;
+    const double us = (alone ? 3.0 : 4.7) * (double)up(steps, sp) + (alone ? 11.0 : 17.8) + (double)(sp + 1) * pass;
+    return {0, sp > 1 && us < best ? (uint32_t)sp : 1u};
   }
   if (ring == 0 || b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {
     const uint64_t w = wgs(256, 128);
@@ -1157,7 +1161,6 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     return {0, sp > 1 && w * sp * 4 >= 3 * cu ? (uint32_t)sp : 1u};
   }
   if (ring == 2) best = 1e30;
-  const double pass = (double)M * (double)N * 4.0 / 4.5e6;                // one pass over a result
   GemmPlan p = {0, 1};
   for (int ma = 2; ma <= 4; ma += 2) {
     const uint64_t tiles = wgs(512, 32 * (uint64_t)ma);
