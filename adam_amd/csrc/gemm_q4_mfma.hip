@@ -359,7 +359,15 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING_ST * RING_STAGE];
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t r32 = lane & 31u, h = lane >> 5;
-  const uint32_t n0 = blockIdx.x * BN, m0 = blockIdx.y * BM, kz = blockIdx.z;
+  // Workgroups land on the eight dies in turn.  by_val & 4: a die takes a run of tiles, those of one run of weight rows next to each
+  // other, so that its L2 has the weights once (256 x 32000 x 2048, 63 runs of weight rows: 106 us as they come, so: 84).
+  uint32_t tn = blockIdx.x, tm = blockIdx.y;
+  if (by_val & 4u) {
+    const uint32_t rows = (M + BM - 1u) / BM, total = (N + BN - 1u) / BN * rows, id = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (id >= total) return;
+    tn = id / rows; tm = id % rows;
+  }
+  const uint32_t n0 = tn * BN, m0 = tm * BM, kz = blockIdx.z;
   const uint32_t nblk = K >> 5, pairs = K >> 6, p_lo = kz * pairs_per, p_hi = min(pairs, p_lo + pairs_per);
   const uint32_t steps = p_hi - p_lo;
 
@@ -1128,7 +1136,8 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x
 // 2048: 23 -> 17 over four; 64 x 28672 x 2048 38 in one, 44 in four, 64 x 28672 x 4096 67 and 62).
 // More: the least of these estimates, in us, fitted to both kernels over 2900 plans of 65 .. 2049 rows by 512 .. 32000 x 128 ..
-// 14336 (the plan it picks takes 0.2 % longer than the best one in the mean, 9 % at most).  Tiled, by the tile it would take
+// 14336 (the plan it picks takes 0.2 % longer than the best one in the mean, 9 % at most; 12 % for 128 x 32000 x 2048, where the
+// tiled kernel over two shares, which it does not ask for, takes 60 us and one launch 67).  Tiled, by the tile it would take
 // (below): 128-column steps of 1.27 us while no CU has a second 64 x 64 tile and 0.72 more for each further one, 4.0 and 2.7
 // more for every two rounds of 64 x 128, 4.6 a round of 256 x 128.  Ring: 64-column steps of 1.7 (ma = 2) or 3.0 us, up to a
 // fifth more as the CUs fill; shares cost their second launch and a pass over the sums each.
@@ -1276,8 +1285,12 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   }
   if (plan.ma) {
     const uint32_t pairs = K >> 6, per = cdiv(pairs, plan.shares), shares = cdiv(pairs, per);
-    const dim3 grid(cdiv(N, 512), cdiv(M, 32 * plan.ma), shares);
-#define GR(T) k_gemm_q4_ring<T><<<grid, 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, (uint32_t)(b_host >> 5), c_val, by_val, per, act, shares > 1 ? g_part_buf : nullptr, lc, g_scale_buf, sg)
+    // Tiles in runs per die where the dies would not each have whole runs of weight rows anyway, few shares leave the weights
+    // the larger part, and it loads the dies as evenly (400 x 6144 x 4096 over three shares, 33 workgroups on a die: 99 us, 70)
+    const uint32_t tn = cdiv(N, 512), tm = cdiv(M, 32 * plan.ma), tiles = tn * tm, run = cdiv(tiles, 8);
+    const bool runs = tn % 8 != 0 && tm > 1 && shares <= 2 && run * 64 <= tiles * 9 && cdiv(run * shares * 8, g.n_cu) <= cdiv(tiles * shares, g.n_cu);
+    const dim3 grid(runs ? run * 8 : tn, runs ? 1 : tm, shares);
+#define GR(T) k_gemm_q4_ring<T><<<grid, 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, (uint32_t)(b_host >> 5), c_val, by_val | (runs ? 4u : 0u), per, act, shares > 1 ? g_part_buf : nullptr, lc, g_scale_buf, sg)
     if (plan.ma == 2) GR(2); else GR(4);
 #undef GR
     count_launch();

@@ -574,3 +574,18 @@ def test_ring_off_leaves_the_tiled_kernel_its_shares(hip, monkeypatch):
         hip.batch_end()
         assert hip.get_last_barrier_count() == launches, (ring, split)
         assert rel_l2(read(hip, 0, M * K, M * N).reshape(M, N), want) < TOL_Q4, (ring, split)
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 31300, 128), (256, 32000, 256), (100, 31300, 1024), (130, 24100, 256), (1000, 4700, 128)])
+def test_tiles_in_runs_per_die(hip, monkeypatch, M, N, K):
+    """Matrices whose runs of 512 weight rows are no multiple of the dies, under several tiles of activation rows: every result has
+    its place, whatever order the tiles are dealt out in."""
+    monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
+    note(f"gemm q4 ring, tiles in runs M={M} N={N} K={K}")
+    rng = np.random.default_rng(M + N)
+    qt = quant.quantize_q4_0((rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.02)))
+    x = rng.standard_normal((1, M, K), dtype=np.float32)
+    y = run(hip, qt, x)[0]
+    want = x[0].astype(np.float64) @ qt.dequant().astype(np.float64).T
+    for m in range(M):
+        assert rel_l2(y[m], want[m]) < TOL_Q4, m
