@@ -21,9 +21,9 @@
 // Ring form (more than 64 activation rows): eight waves of 64 weight rows over 64 or 128 activation rows, on 32x32x16
 // instructions, weights, scales and activations straight to a ring of LDS stages.
 // Either over shares of K, which k_gemm_splitk_sum adds up; gemm_plan says which.
-// K-split form (few activation rows): the waves share R tiles of 16 weight rows and take every NWV-th step of K
-// each, so that small matrices still spread over the whole chip; their partial tiles are summed through LDS in
-// a fixed order.
+// Few rows (2 .. 64): k_gemm_q4_rows, k_gemm_q4_f16_rows16.  The waves of a workgroup share R tiles of 16 weight rows and take
+// every NWV-th step of K each, so that small matrices still spread over the whole chip; their partial tiles are summed
+// through LDS in a fixed order.  At most 64 rows are converted to operand tiles (ActForm), more to rows.
 #include "gemv_common.h"
 #include "lds_ring.h"
 #include <algorithm>
@@ -65,12 +65,12 @@ __device__ __forceinline__ void split_word(const float* v, uint4* hi, uint4* lo)
 // order (0,4)(1,5)(2,6)(3,7).  The matmul workgroups then copy 16-byte pieces into LDS.  One workgroup per
 // row; also stores (s, 1/s).  xl = second plane (same indexing as xh).
 __global__ void __launch_bounds__(256)
-k_act_f16(const float* act, const uint32_t* __restrict__ la, uint32_t M, uint32_t K, float* scale, uint4* xh, uint4* xl) {
+k_act_f16(const float* act, const uint32_t* __restrict__ la, uint32_t M, uint32_t K, float* scale, uint4* x, ActForm form) {
   __shared__ float red[4];
   const uint32_t row = blockIdx.x, op = blockIdx.y, tid = threadIdx.x;
-  const float* x = act + (uint64_t)la[op] + (uint64_t)row * K;
+  const float* src = act + (uint64_t)la[op] + (uint64_t)row * K;
   float m = 0.f;
-  for (uint32_t i = tid; i < K; i += 256u) m = fmaxf(m, fabsf(x[i]));
+  for (uint32_t i = tid; i < K; i += 256u) m = fmaxf(m, fabsf(src[i]));
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
   if ((tid & 63u) == 0) red[tid >> 6] = m;
@@ -83,14 +83,13 @@ k_act_f16(const float* act, const uint32_t* __restrict__ la, uint32_t M, uint32_
     scale[2 * ((uint64_t)op * M + row)] = s;
     scale[2 * ((uint64_t)op * M + row) + 1] = inv;
   }
-  const uint64_t o0 = ((uint64_t)op * M + row) * (K >> 3);
   for (uint32_t w = tid; w < (K >> 3); w += 256u) {
-    const f4qu_t v0 = *(const f4qu_t*)(x + w * 8u), v1 = *(const f4qu_t*)(x + w * 8u + 4u);
+    const f4qu_t v0 = *(const f4qu_t*)(src + w * 8u), v1 = *(const f4qu_t*)(src + w * 8u + 4u);
     const float v[8] = {v0.x * s, v0.y * s, v0.z * s, v0.w * s, v1.x * s, v1.y * s, v1.z * s, v1.w * s};
     uint4 hi, lo;
     split_word(v, &hi, &lo);
-    xh[o0 + w] = hi;
-    xl[o0 + w] = lo;
+    x[act_piece(form, op, row, w, 0u)] = hi;
+    x[act_piece(form, op, row, w, 1u)] = lo;
   }
 }
 
@@ -133,6 +132,12 @@ __device__ __forceinline__ f4q_t gather_scales(_Float16 d) {
   auto f = [](uint32_t b) { return (float)__builtin_bit_cast(_Float16, (uint16_t)b); };
   return (f4q_t){f(lo.x), f(lo.y), f(hi.x), f(hi.y)};
 }
+// the same as four halves
+__device__ __forceinline__ h4q_t gather_scales16(uint32_t d) {
+  const u2s_t a = __builtin_amdgcn_permlane32_swap(d, d, false, false);
+  const u2s_t lo = __builtin_amdgcn_permlane16_swap(a.x, a.x, false, false), hi = __builtin_amdgcn_permlane16_swap(a.y, a.y, false, false);
+  return __builtin_bit_cast(h4q_t, (u2q_t){lo.x | lo.y << 16, hi.x | hi.y << 16});
+}
 #define DEQK_INIT(c)                                                                           \
   DeqK c = {0x64006400u, 0x54005400u, 0x000F000Fu, 0x00F000F0u,                                \
             {(_Float16)-1032.f, (_Float16)-1032.f}, {(_Float16)-72.f, (_Float16)-72.f}};       \
@@ -148,10 +153,10 @@ __device__ __forceinline__ f4q_t gather_scales(_Float16 d) {
 // of K; the next step's weight words and activation pieces are loaded into registers while the matrix cores work
 // on the current one.  The activation tile is staged by every workgroup, so wide workgroups (eight waves) move
 // fewer bytes per flop: 28672x4096 at M = 512 went 434 -> 344 us with 256 instead of 128 weight rows per workgroup.
-template <int MT, int R, int NW>
+// TILES: the activations come as operand tiles (at most 64 rows), else as rows.
+template <int MT, int R, int NW, bool TILES>
 __global__ void __launch_bounds__(64 * NW)
-k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ xh, const u4q_t* __restrict__ xl,
-                     uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
+k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, ActForm form, uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
                      const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale,
                      GemmSegs segs, uint32_t ksplit, uint32_t kper, float* __restrict__ part) {
   // (the first 14 dwords of the arguments are in registers when a wave starts; by_val bit 0 / 1: the weights' / the
@@ -168,7 +173,7 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
   const uint32_t n0 = blockIdx.x * (16u * NW * R) + wave * (16u * R), m0 = blockIdx.y * BM;
   const uint32_t op = ksplit > 1u ? 0u : blockIdx.z, kz = ksplit > 1u ? blockIdx.z : 0u;
   const uint64_t c_off = (by_val & 2u) ? (uint64_t)c_val : (uint64_t)lc[op], gbase = ((by_val & 1u) ? (uint64_t)b_val : (uint64_t)lb[op]) >> 5;
-  const uint32_t nblk = K >> 5, kw = K >> 3;                   // blocks and 16-byte pieces per row
+  const uint32_t nblk = K >> 5;                                // blocks per row
   const uint32_t kb_lo = kz * kper, kb_hi = min(nblk, kb_lo + kper);   // this workgroup's blocks of K
   uint32_t nrow[R];
 #pragma unroll
@@ -182,11 +187,14 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
   DEQK_INIT(dk);
 
   // staging: the tile's 16 pieces per row, plane and step; thread -> (row, piece) pairs, NP per thread
-  uint64_t xoff[NP];
+  uint64_t xoff[NP], xloff[TILES ? NP : 1];
+  constexpr uint32_t per_blk = TILES ? 64u : 4u;             // pieces from a block of a row to the next one
+  const u4q_t* const xl = x + form.lo;
 #pragma unroll
   for (uint32_t u = 0; u < NP; u++) {
     const uint32_t w = tid + u * NT, row = min(m0 + (w >> 4), M - 1u);   // rows past M: clamped, not stored
-    xoff[u] = ((uint64_t)op * M + row) * kw + (w & 15u);
+    xoff[u] = TILES ? act_piece(form, op, row, w & 15u, 0u) : ((uint64_t)op * M + row) * form.kw + (w & 15u);
+    if (TILES) xloff[u] = act_piece(form, op, row, w & 15u, 1u);
   }
   u4q_t xn[NP], xln[NP], qn[R];
   _Float16 dn[R];
@@ -200,8 +208,8 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
       dn[r] = __builtin_bit_cast(_Float16, d16[gi]);                              \
     }                                                                             \
     _Pragma("unroll") for (uint32_t u = 0; u < NP; u++) {                         \
-      xn[u] = xh[xoff[u] + kb_ * 4u];                                             \
-      xln[u] = xl[xoff[u] + kb_ * 4u];                                            \
+      xn[u] = x[xoff[u] + kb_ * per_blk];                                            \
+      xln[u] = TILES ? x[xloff[u] + kb_ * per_blk] : xl[xoff[u] + kb_ * per_blk];                                            \
     }                                                                             \
   } while (0)
   GEMM_FETCH(kb_lo);
@@ -508,43 +516,203 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
     }
 }
 
-// Few activation rows (M <= 32): the weights are read once and nothing is reused, so the work is
-// bound by how fast they stream.  The NWV waves of a workgroup share R tiles of 16 weight rows and
-// take every NWV-th step of K each (a matrix with few rows still spreads over the whole chip); every
-// wave stages its own activation tile (both planes) from the fp16 copy into its own piece of LDS, so no
-// workgroup barrier sits in the K loop.  The partial tiles are summed in wave order at the end.
-// Eight waves keep twice as many loads in flight for matrices with few weight rows.
-//
-// Q8: the weights are Q8_0 blocks in the same block16 layout (32 code bytes, w = d (code - 128)): two 16-byte
-// loads per block, bytes widened with a byte permute into the fp16 pairs (1024 + code), then -1152 and d
-// (one term each for weights and activations).  `lc` null: the result rows go to out[row * N + n] (a scratch
-// buffer of the caller).
-template <int MT, int R, int NWV, bool Q8>
+// 2 .. 64 activation rows: the weights are read once, so what counts is how fast they stream, and what stands in its way is
+// the activations, of which a 16-row operand of 32 columns is 1 KB beside 288 bytes of weights.  So
+//   * the rows' two planes are stacked: 2 M operand rows (xh of every row, then xl), NT tiles of 16, one instruction per tile and
+//     block -- 8 rows fill one tile, 24 rows three; the planes' sums are added at the end;
+//   * operands go from memory to registers in the instruction's layout, without LDS: a wave reads 16 rows x 64 bytes at a time;
+//   * the NWV waves of a workgroup share R tiles of 16 weight rows and take every NWV-th step of K (128 columns) each, so a
+//     workgroup reads its activations once, and as many weight rows as a CU has share them.
+// Weights are asked for D steps ahead, activations DA.  The waves' tiles are summed through LDS in wave order.
+// What bounds it is the L1's rate for one tile of weights (96 clocks of it a step with one operand tile, of 175 measured) and the
+// vector work for four (75 instructions a step and tile, 36 of them unpacking): more steps ahead only cost their loads (8 rows, 28672
+// x 4096, one tile: 29 us two steps ahead, 45 four).  Before (a tile of activations staged by every wave, both planes apart):
+// 8 rows 4096 x 4096 6.7 -> 5.2 us, 6144 x 4096 10.4 -> 8.3, 4096 x 14336 16.7 -> 14.8, 13824 x 1152 9.0 -> 6.9; 24 rows 13.7 ->
+// 7.9, 19.2 -> 11.0, 39.1 -> 24, 15.2 -> 9.4, 28672 x 4096 48 -> 36; 32 rows 14.4 -> 9.3, 19.7 -> 12.7, 39.6 -> 29, 15.0 -> 10.7, 49.6 -> 40.
+// (segs.glu: tiles of a wave are gate, up, gate, up ...: the gated activation is stored from here.)
+template <int NT, int R, int NWV, int D, int DA>
 __global__ void __launch_bounds__(64 * NWV)
-k_gemm_q4_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ xh, const u4q_t* __restrict__ xl,
-                     uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
-                     const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale,
-                     GemmSegs segs) {
+k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles, uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
+               const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale, GemmSegs segs) {
   // (the first 14 dwords of the arguments are in registers when a wave starts; by_val bit 0 / 1: the weights' / the
   // result's element offset of op 0 is b_val / c_val -- known on the host -- instead of a load from lb / lc, which
   // the first weight loads would have to wait for)
-  constexpr uint32_t BM = 16u * MT, ROWB = 272u, NP = 4u * MT;      // pieces per lane, plane and step
-  constexpr uint32_t PLANES = Q8 ? 1u : 2u;
+  constexpr int RC = R >= 2 ? 2 : 1;
+  static_assert(DA == 1 || DA == D, "activations one step ahead, or as many as the weights");
+  __shared__ float part[NWV * RC * NT * 256];                // [wave][tile of a pair][operand tile][i][lane]
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+  const uint32_t r16 = lane & 15u, g = lane >> 4, op = blockIdx.z;
+  const bool glum = R >= 2 && segs.glu != 0u;
+  const uint64_t c_off = (by_val & 2u) ? (uint64_t)c_val : lc ? (uint64_t)lc[op] : 0ull, gbase = ((by_val & 1u) ? (uint64_t)b_val : (uint64_t)lb[op]) >> 5;
+  const uint32_t nblk = K >> 5, kw = K >> 3, steps = nblk >> 2;
+  const uint8_t* const Wb = W + (gbase << 4);
+  const uint16_t* const Db = (const uint16_t*)d16 + gbase;
+  // Weight loads: lane -> (row lane / 4, block lane % 4 of the step): the four lanes of a quad read 64 contiguous bytes of one
+  // row, one request to the L1 instead of four; a permute brings each block to the lane that consumes it
+  const int perm_addr = (int)((4u * r16 + g) << 2);
+  const auto first_row = [&](int r) {
+    return glum ? (blockIdx.x * (uint32_t)(R / 2) + (uint32_t)(r >> 1)) * 16u + (r & 1 ? N >> 1 : 0u) : (blockIdx.x * (uint32_t)R + (uint32_t)r) * 16u;
+  };
+  uint32_t wo[R];                                            // block index from Wb on (a Q4 map here has fewer than 2^32 elements)
+#pragma unroll
+  for (int r = 0; r < R; r++) wo[r] = min(first_row(r) + (lane >> 2), N - 1u) * nblk + (lane & 3u);
+  const u4q_t* const xb = x + (uint64_t)op * tiles * kw * 16u;
+  f4q_t acc[R][NT];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int t = 0; t < NT; t++) acc[r][t] = (f4q_t){0.f, 0.f, 0.f, 0.f};
+  DEQK_INIT(dk);
+
+  u4q_t qn[D][R], xn[DA][2][NT][2];                          // [steps ahead]; activations by pairs of blocks
+  uint16_t dn[D][R];
+  const auto fetch_w = [&](int slot, uint32_t s) {
+    uint64_t at = min(s, steps - 1u) * 4u;
+    asm volatile("" : "+s"(at));                             // (a wave's base and a lane's offset: no address arithmetic)
+    const uint8_t *wp = Wb + at * 16u, *dp = (const uint8_t*)(Db + at);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      qn[slot][r] = __builtin_nontemporal_load((const u4q_t*)(wp + (wo[r] << 4)));
+      dn[slot][r] = *(const uint16_t*)(dp + (wo[r] << 1));
+    }
+  };
+  const auto fetch_x = [&](int slot, int u, uint32_t s) {
+    const uint64_t at = min(s, steps - 1u) * 256u + u * 128u;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {                           // (a tile past the last: its sums are not used)
+      uint64_t from = (uint64_t)min((uint32_t)t, tiles - 1u) * kw * 16u + at;
+      asm volatile("" : "+s"(from));
+      const uint8_t* p = (const uint8_t*)(xb + from);
+      xn[slot][u][t][0] = *(const u4q_t*)(p + lane * 16u); xn[slot][u][t][1] = *(const u4q_t*)(p + lane * 16u + 1024u);
+    }
+    asm volatile("" ::: "memory");                           // the loads stay here
+  };
+  // one step from slot `ws` / `xs`; more: the loads of the steps that take its place
+  const auto step = [&](int ws, int xs, bool more, uint32_t s) {
+    u4q_t q[R];
+    h4q_t ds[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const u4q_t v = qn[ws][r];
+      q[r] = transpose_blocks((u4q_t){(uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)v.x), (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)v.y),
+                                      (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)v.z), (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)v.w)});
+      ds[r] = gather_scales16((uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)dn[ws][r]));
+    }
+    if (more) fetch_w(ws, s + (uint32_t)D * NWV);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        const int b = 2 * u + e;
+        u4q_t wq[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) wq[r] = deq_word(b == 0 ? q[r].x : b == 1 ? q[r].y : b == 2 ? q[r].z : q[r].w, dk);
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          f4q_t blk[R];
+#pragma unroll
+          for (int r = 0; r < R; r++) blk[r] = MFMA_F16(xn[xs][u][t][e], wq[r], ((f4q_t){0.f, 0.f, 0.f, 0.f}));
+#pragma unroll
+          for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) acc[r][t][i] = fmaf(blk[r][i], (float)ds[r][b], acc[r][t][i]);
+        }
+        __builtin_amdgcn_sched_barrier(0);                   // (blocks overlapped any further cost registers)
+      }
+      if (more || DA < D) fetch_x(xs, u, s + (uint32_t)DA * NWV);
+    }
+  };
+  const uint32_t cnt = wave < steps ? (steps - wave + NWV - 1u) / NWV : 0u;
+  uint32_t i = 0, s = wave;
+#pragma unroll
+  for (int d = 0; d < D; d++) {
+    fetch_w(d, s + (uint32_t)d * NWV);
+    if (d < DA) { fetch_x(d, 0, s + (uint32_t)d * NWV); fetch_x(d, 1, s + (uint32_t)d * NWV); }
+  }
+  for (; i + (uint32_t)D < cnt; i += (uint32_t)D)            // (steps past the end ask for the last one again)
+#pragma unroll
+    for (int d = 0; d < D; d++, s += NWV) step(d, DA == 1 ? 0 : d, true, s);
+#pragma unroll
+  for (int d = 0; d < D; d++, s += NWV)
+    if (i + (uint32_t)d < cnt) step(d, DA == 1 ? 0 : d, false, s);
+
+#pragma unroll
+  for (int r0 = 0; r0 < R; r0 += RC) {
+    if (r0) __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RC; r++)
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) part[((wave * RC + r) * NT + t) * 256u + k * 64u + lane] = acc[r0 + r][t][k];
+    __syncthreads();
+    for (uint32_t idx = tid; idx < M * 16u; idx += 64u * NWV) {
+      // activation row `row` of tile column c: operand rows `row` and M + row of every wave
+      const uint32_t row = idx >> 4, c = idx & 15u, lo = M + row;
+      const auto place = [&](uint32_t v) { return (v >> 4) * 256u + (v & 3u) * 64u + ((v >> 2) & 3u) * 16u + c; };
+      const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
+      float y[RC];
+#pragma unroll
+      for (int r = 0; r < RC; r++) {
+        float a = 0.f, b = 0.f;
+#pragma unroll
+        for (uint32_t w = 0; w < NWV; w++) {
+          const float* p = part + (w * RC + r) * NT * 256u;
+          a += p[place(row)];
+          b += p[place(lo)];
+        }
+        y[r] = (a + b) * inv;
+      }
+#pragma unroll
+      for (int r = 0; r < RC; r++) {
+        const uint32_t n = first_row(r0 + r) + c;
+        if (n >= (glum && !(r & 1) ? N >> 1 : N)) continue;
+        if (segs.count) {   // stacked matrices: the row's own matrix and its result base
+          uint32_t sgi = 0;
+#pragma unroll
+          for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
+          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y[r];
+        } else {
+          out[c_off + (uint64_t)row * N + n] = y[r];
+          if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y[r];
+        }
+      }
+      if (glum && first_row(r0) + c < (N >> 1))   // act(gate) * up, as the element-wise op computes it
+        out[segs.dst + (uint64_t)row * (N >> 1) + first_row(r0) + c] = (segs.glu == 34u ? gelu_tanh(y[0]) : y[0] / (1.0f + expf(-y[0]))) * y[RC - 1];
+    }
+  }
+}
+
+// Q8_0 weights (the LM head of a lockstep batch) under at most 32 activation rows: the weights are read once and nothing is
+// reused, so the work is bound by how fast they stream.  The four waves of a workgroup share R tiles of 16 weight rows and
+// take every fourth step of K each; every wave stages its own activation tile (the first plane) into its own piece of LDS, so
+// no workgroup barrier sits in the K loop.  The partial tiles are summed in wave order at the end.
+// The weights are blocks of 32 code bytes, w = d (code - 128): two 16-byte loads per block, bytes widened with a byte permute
+// into the fp16 pairs (1024 + code), then -1152 and d.  `lc` null: the result rows go to out[row * N + n] (a scratch buffer of
+// the caller).
+template <int MT, int R>
+__global__ void __launch_bounds__(256)
+k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles,
+                     uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
+                     const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale,
+                     GemmSegs segs) {
+  // (by_val bit 0 / 1: the weights' / the result's element offset of op 0 is b_val / c_val -- known on the host -- instead of
+  // a load from lb / lc, which the first weight loads would have to wait for)
+  constexpr uint32_t NWV = 4u, BM = 16u * MT, ROWB = 272u, NP = 4u * MT;      // NP: pieces per lane and step
   constexpr uint32_t TILE = BM * ROWB, PART = (NWV - 1u) * R * MT * 4u * 64u * 4u;
-  __shared__ __attribute__((aligned(16))) uint8_t xs_all[(NWV * PLANES * TILE > PART) ? NWV * PLANES * TILE : PART];
+  __shared__ __attribute__((aligned(16))) uint8_t xs_all[(NWV * TILE > PART) ? NWV * TILE : PART];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t r16 = lane & 15u, g = lane >> 4;
-  uint8_t* xs = xs_all + wave * PLANES * TILE;
-  uint8_t* const xs2 = xs + TILE;
-  const uint32_t n0 = blockIdx.x * (16u * R), m0 = blockIdx.y * BM, op = blockIdx.z;
+  uint8_t* xs = xs_all + wave * TILE;
+  const uint32_t op = blockIdx.z;
   const uint64_t c_off = (by_val & 2u) ? (uint64_t)c_val : lc ? (uint64_t)lc[op] : 0ull;
   const uint64_t gbase = ((by_val & 1u) ? (uint64_t)b_val : (uint64_t)lb[op]) >> 5;
   const uint32_t nblk = K >> 5, kw = K >> 3;
-  // Weight loads: lane -> (row lane / 4, block lane % 4 of the step), so the four lanes of a quad read 64
-  // contiguous bytes of one row -- one request to the L1 instead of one per lane, which is what the
-  // matrix-instruction layout (lane -> row lane % 16, block lane / 16) costs when loaded directly.
-  // A cross-lane permute brings each 16-byte block (and its scale) to the lane that consumes it.
+  // Weight loads: lane -> (row lane / 4, block lane % 4 of the step): the lanes of a quad read neighbouring blocks of one row.
+  // A cross-lane permute brings each 16-byte piece (and its scale) to the lane that consumes it.
   const uint32_t lrow = lane >> 2, lblk = lane & 3u;
   const int perm_addr = (int)((4u * r16 + g) << 2);
   // segs.glu (R = 2, the matrix is [gate rows; up rows], N / 2 a multiple of 16): the workgroup's first tile is 16
@@ -553,7 +721,7 @@ k_gemm_q4_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
   uint32_t trow0[R], nrow[R];
 #pragma unroll
   for (int r = 0; r < R; r++) {
-    trow0[r] = glum ? (uint32_t)r * (N >> 1) + blockIdx.x * 16u : n0 + r * 16u;
+    trow0[r] = glum ? (uint32_t)r * (N >> 1) + blockIdx.x * 16u : blockIdx.x * (16u * R) + r * 16u;
     nrow[r] = min(trow0[r] + lrow, N - 1u);
   }
 
@@ -565,105 +733,69 @@ k_gemm_q4_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
   DEQK_INIT(dk);
   const h2q_t off_q8 = {(_Float16)-1152.f, (_Float16)-1152.f};
 
-  uint64_t xoff[NP];
+  // lane l, piece u: operand tile u / 4, block u % 4 of the step, the tile's row l % 16, piece l / 16 of the block (tiles past
+  // the last: clamped, not stored)
+  const u4q_t* xp[MT];
 #pragma unroll
-  for (uint32_t u = 0; u < NP; u++) {
-    const uint32_t w = lane + u * 64u, row = min(m0 + (w >> 4), M - 1u);
-    xoff[u] = ((uint64_t)op * M + row) * kw + (w & 15u);
-  }
-  u4q_t xn[NP], xln[Q8 ? 1 : NP], qn[R], qn2[Q8 ? R : 1];
+  for (uint32_t t = 0; t < MT; t++) xp[t] = x + ((uint64_t)op * tiles + min(t, tiles - 1u)) * kw * 16u + lane;
+  u4q_t xn[NP], qn[R], qn2[R];
   _Float16 dn[R];
 #define GEMM_FETCH(kb_raw)                                                        \
   do {                                                                            \
     const uint32_t kb_ = min((kb_raw), nblk - 4u);                                \
     _Pragma("unroll") for (int r = 0; r < R; r++) {                               \
       const uint64_t gi = gbase + (uint64_t)nrow[r] * nblk + kb_ + lblk;          \
-      if (Q8) {                                                                   \
-        qn[r] = *(const u4q_t*)(W + (gi << 5));                                   \
-        qn2[r] = *(const u4q_t*)(W + (gi << 5) + 16);                             \
-      } else qn[r] = *(const u4q_t*)(W + (gi << 4));                              \
+      qn[r] = *(const u4q_t*)(W + (gi << 5));                                     \
+      qn2[r] = *(const u4q_t*)(W + (gi << 5) + 16);                               \
       dn[r] = __builtin_bit_cast(_Float16, d16[gi]);                              \
     }                                                                             \
-    _Pragma("unroll") for (uint32_t u = 0; u < NP; u++) {                         \
-      xn[u] = xh[xoff[u] + kb_ * 4u];                                             \
-      if (!Q8) xln[u] = xl[xoff[u] + kb_ * 4u];                                   \
-    }                                                                             \
+    _Pragma("unroll") for (uint32_t u = 0; u < NP; u++)                           \
+      xn[u] = xp[u >> 2][(uint64_t)(kb_ + (u & 3u)) * 64u];                       \
   } while (0)
   GEMM_FETCH(wave * 4u);
 
   for (uint32_t kb0 = wave * 4u; kb0 < nblk; kb0 += 4u * NWV) {
 #pragma unroll
-    for (uint32_t u = 0; u < NP; u++) {
-      const uint32_t w = lane + u * 64u;
-      *(u4q_t*)(xs + (w >> 4) * ROWB + (w & 15u) * 16u) = xn[u];
-      if (!Q8) *(u4q_t*)(xs2 + (w >> 4) * ROWB + (w & 15u) * 16u) = xln[u];
-    }
+    for (uint32_t u = 0; u < NP; u++) *(u4q_t*)(xs + ((u >> 2) * 16u + r16) * ROWB + (u & 3u) * 64u + g * 16u) = xn[u];
     // the step's blocks and scales, moved to the lanes that consume them
-    u4q_t q[R], q2[Q8 ? R : 1];
-    f4q_t ds[Q8 ? 1 : R];
-    h2q_t d2[Q8 ? R : 1];
+    u4q_t q[R], q2[R];
+    h2q_t d2[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
 #define PERM_U4(v) (u4q_t){(uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)(v).x), (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)(v).y), \
                            (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)(v).z), (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)(v).w)}
       q[r] = PERM_U4(qn[r]);
-      if (Q8) q2[r] = PERM_U4(qn2[r]);
+      q2[r] = PERM_U4(qn2[r]);
 #undef PERM_U4
       const uint32_t dbits = (uint32_t)__builtin_amdgcn_ds_bpermute(perm_addr, (int)__builtin_bit_cast(uint16_t, dn[r]));
       const _Float16 dl = __builtin_bit_cast(_Float16, (uint16_t)dbits);
-      if (Q8) d2[r] = (h2q_t){dl, dl};
-      else { q[r] = transpose_blocks(q[r]); ds[r] = gather_scales(dl); }
+      d2[r] = (h2q_t){dl, dl};
     }
     __builtin_amdgcn_wave_barrier();
     GEMM_FETCH(kb0 + 4u * NWV);
-    if (Q8) {
-      // Q8_0 blocks: lane group g holds block g whole; instruction j takes code bytes 8j .. 8j+7 of each of the
-      // four blocks, scaled before the product (one term each for weights and activations)
+    // lane group g holds block g whole; instruction j takes code bytes 8j .. 8j+7 of each of the four blocks, scaled before
+    // the product
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        u4q_t wq[R];
+    for (int j = 0; j < 4; j++) {
+      u4q_t wq[R];
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-          // piece j = code bytes 8j .. 8j+7 in two words; pair p = (byte p of the first, byte p of the second)
-          const uint32_t w0 = j == 0 ? q[r].x : j == 1 ? q[r].z : j == 2 ? q2[r].x : q2[r].z;
-          const uint32_t w1 = j == 0 ? q[r].y : j == 1 ? q[r].w : j == 2 ? q2[r].y : q2[r].w;
-          uint32_t o[4];
+      for (int r = 0; r < R; r++) {
+        // piece j = code bytes 8j .. 8j+7 in two words; pair p = (byte p of the first, byte p of the second)
+        const uint32_t w0 = j == 0 ? q[r].x : j == 1 ? q[r].z : j == 2 ? q2[r].x : q2[r].z;
+        const uint32_t w1 = j == 0 ? q[r].y : j == 1 ? q[r].w : j == 2 ? q2[r].y : q2[r].w;
+        uint32_t o[4];
 #pragma unroll
-          for (uint32_t p = 0; p < 4; p++) {
-            const uint32_t t = __builtin_amdgcn_perm(w1, w0, 0x0C000C00u | ((4u + p) << 16) | p) | dk.magic_lo;
-            o[p] = __builtin_bit_cast(uint32_t, (h2q_t)((__builtin_bit_cast(h2q_t, t) + off_q8) * d2[r]));
-          }
-          wq[r] = (u4q_t){o[0], o[1], o[2], o[3]};
+        for (uint32_t p = 0; p < 4; p++) {
+          const uint32_t t = __builtin_amdgcn_perm(w1, w0, 0x0C000C00u | ((4u + p) << 16) | p) | dk.magic_lo;
+          o[p] = __builtin_bit_cast(uint32_t, (h2q_t)((__builtin_bit_cast(h2q_t, t) + off_q8) * d2[r]));
         }
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-          const u4q_t ah = *(const u4q_t*)(xs + (t * 16u + r16) * ROWB + g * 64u + j * 16u);
-#pragma unroll
-          for (int r = 0; r < R; r++) acc[r][t] = MFMA_F16(ah, wq[r], acc[r][t]);
-        }
+        wq[r] = (u4q_t){o[0], o[1], o[2], o[3]};
       }
-    } else {
 #pragma unroll
-      for (int b = 0; b < 4; b++) {      // one 32-weight block of the step at a time
-        u4q_t wq[R];
+      for (int t = 0; t < MT; t++) {
+        const u4q_t ah = *(const u4q_t*)(xs + (t * 16u + r16) * ROWB + g * 64u + j * 16u);
 #pragma unroll
-        for (int r = 0; r < R; r++) wq[r] = deq_word(b == 0 ? q[r].x : b == 1 ? q[r].y : b == 2 ? q[r].z : q[r].w, dk);
-#pragma unroll
-        for (int t = 0; t < MT; t++) {
-          const uint32_t xo = (t * 16u + r16) * ROWB + b * 64u + g * 16u;
-          const u4q_t ah = *(const u4q_t*)(xs + xo), al = *(const u4q_t*)(xs2 + xo);
-          f4q_t blk[R];
-#pragma unroll
-          for (int r = 0; r < R; r++) blk[r] = MFMA_F16(ah, wq[r], ((f4q_t){0.f, 0.f, 0.f, 0.f}));
-#pragma unroll
-          for (int r = 0; r < R; r++) blk[r] = MFMA_F16(al, wq[r], blk[r]);
-#pragma unroll
-          for (int r = 0; r < R; r++) {
-            const float d = ds[r][b];
-#pragma unroll
-            for (int i = 0; i < 4; i++) acc[r][t][i] = fmaf(blk[r][i], d, acc[r][t][i]);
-          }
-        }
+        for (int r = 0; r < R; r++) acc[r][t] = MFMA_F16(ah, wq[r], acc[r][t]);
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -689,27 +821,26 @@ k_gemm_q4_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
       for (int t = 0; t < MT; t++)
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[r][t][i] += part[(((w * R + r) * MT + t) * 4u + i) * 64u + lane];
-  // lane (r16, g) holds D[4g + i][r16]: activation rows m0 + 16 t + 4g + i, weight row n0 + 16 r + r16
+  // lane (r16, g) holds D[4g + i][r16]: activation rows 16 t + 4g + i, weight row r16 of tile r
 #pragma unroll
   for (int t = 0; t < MT; t++)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint32_t row = m0 + t * 16u + 4u * g + i;
+      const uint32_t row = t * 16u + 4u * g + i;
       if (row >= M) continue;
       const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
-      float* c = out + c_off + (uint64_t)row * N;
 #pragma unroll
       for (int r = 0; r < R; r++) {
         const uint32_t n = trow0[r] + r16;
         if (n >= N) continue;
+        const float y = acc[r][t][i] * inv;
         if (segs.count) {   // stacked matrices: the row's own matrix and its result base
           uint32_t sgi = 0;
 #pragma unroll
           for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = acc[r][t][i] * inv;
+          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y;
         } else {
-          const float y = acc[r][t][i] * inv;
-          c[n] = y;
+          out[c_off + (uint64_t)row * N + n] = y;
           if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;
         }
       }
@@ -736,7 +867,7 @@ k_gemm_q4_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
 #define R16_MS 2u
 template <int NW>
 __global__ void __launch_bounds__(64 * NW)
-k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ xh, const u4q_t* __restrict__ xl,
+k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles,
                      uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
                      const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale,
                      GemmSegs segs) {
@@ -763,14 +894,17 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
   DEQK_INIT(dk);
   f4q_t acc = {0.f, 0.f, 0.f, 0.f};
 
-  // a thread's pieces of a macro tile: piece w -> (step w / 256, row (w / 16) % 16, piece w % 16)
-  uint64_t xoff[NP];
+  // a thread's pieces of a macro tile: piece w -> (step w / 256, block (w / 64) % 4 of the step, piece (w / 16) % 4 of the block,
+  // row w % 16).  Second plane: operand rows M .. 2 M - 1
+  uint64_t xoff[NP], xloff[NP];
   uint32_t xlds[NP], xst[NP];
 #pragma unroll
   for (uint32_t u = 0; u < NP; u++) {
-    const uint32_t w = min(tid + u * NT, PIECES - 1u), row = (w >> 4) & 15u, pc = w & 15u;
+    const uint32_t w = min(tid + u * NT, PIECES - 1u), row = w & 15u, pc = (w >> 4) & 15u, v = min(row, M - 1u), vl = v + M;
     xst[u] = w >> 8;
-    xoff[u] = ((uint64_t)op * M + min(row, M - 1u)) * kw + pc;     // + 16 pieces per step of K
+    const uint64_t at = (uint64_t)op * tiles * kw * 16u + (pc << 4);   // + 256 pieces per step of K
+    xoff[u] = at + v;
+    xloff[u] = at + (uint64_t)(vl >> 4) * kw * 16u + (vl & 15u);
     xlds[u] = xst[u] * TILE + row * ROWB + pc * 16u;
   }
   struct ActR { u4q_t h[NP], l[NP]; };
@@ -781,8 +915,8 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
   auto fetch_a = [&](ActR& a, uint32_t m) {
 #pragma unroll
     for (uint32_t u = 0; u < NP; u++) {
-      const uint64_t at = xoff[u] + min(m * R16_MS + xst[u], steps - 1u) * 16u;
-      a.h[u] = xh[at]; a.l[u] = xl[at];
+      const uint64_t at = (uint64_t)min(m * R16_MS + xst[u], steps - 1u) * 256u;
+      a.h[u] = x[xoff[u] + at]; a.l[u] = x[xloff[u] + at];
     }
   };
   auto fetch_w = [&](WtR& w, uint32_t m) {
@@ -903,8 +1037,8 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
 struct GluSrc { uint32_t op, a, b, d; };
 template <int NW, bool GLU>
 __global__ void __launch_bounds__(1024)
-k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_t a_by_val, uint4* xh, uint4* xl, float* scale,
-               float* act_out, const uint32_t* __restrict__ la, GluSrc glu) {
+k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_t a_by_val, uint4* xf, float* scale,
+               float* act_out, const uint32_t* __restrict__ la, GluSrc glu, ActForm form) {
   // (a_by_val: the rows start at element a_val -- known on the host -- instead of la[op], a load the rows' loads
   // would wait for; with GLU a_val is glu.a)
   __shared__ float red[16];
@@ -946,7 +1080,6 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
     scale[2 * ((uint64_t)op * M + row)] = s;
     scale[2 * ((uint64_t)op * M + row) + 1] = inv;
   }
-  const uint64_t o0 = ((uint64_t)op * M + row) * kw;
 #pragma unroll
   for (int u = 0; u < NW; u++) {
     const uint32_t w = tid + 1024u * u;
@@ -954,8 +1087,8 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
     const float v[8] = {v0[u].x * s, v0[u].y * s, v0[u].z * s, v0[u].w * s, v1[u].x * s, v1[u].y * s, v1[u].z * s, v1[u].w * s};
     uint4 hi, lo;
     split_word(v, &hi, &lo);
-    xh[o0 + w] = hi;
-    xl[o0 + w] = lo;
+    xf[act_piece(form, op, row, w, 0u)] = hi;
+    xf[act_piece(form, op, row, w, 1u)] = lo;
   }
 }
 
@@ -998,14 +1131,21 @@ static bool ensure_act_bufs(size_t scale_floats, size_t xh_bytes) {
   return true;
 }
 
-bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, __half** xh, __half** xl) {
+// The form in which a matmul of M rows reads its activations, and the bytes of n_ops of them
+static ActForm act_form(uint32_t M, uint32_t K, uint32_t n_ops, size_t* bytes) {
+  const uint32_t kw = K >> 3, tiles = M <= 64 && (K & 127u) == 0 ? cdiv(2 * M, 16) : 0u;
+  *bytes = tiles ? (size_t)n_ops * tiles * 32 * K : (size_t)n_ops * M * K * 4;
+  return {M, kw, tiles, (uint64_t)n_ops * M * kw};
+}
+
+bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, uint4** x, ActForm* form) {
   if (tuning("ADAMAH_GEMM_REUSE", 1) == 0) return false;
-  const size_t plane = (size_t)M * K * 2;
-  if (!ensure_act_bufs((size_t)2 * M, 2 * plane)) return false;
+  size_t bytes;
+  *form = act_form(M, K, 1, &bytes);
+  if (!ensure_act_bufs((size_t)2 * M, bytes)) return false;
   g_xh_key.valid = false;   // the buffers are about to be rewritten
   *scale = g_scale_buf;
-  *xh = (__half*)g_xh_buf;
-  *xl = (__half*)((uint8_t*)g_xh_buf + plane);
+  *x = g_xh_buf;
   return true;
 }
 
@@ -1018,12 +1158,12 @@ void gemm_act_mark(const void* buf, uint64_t a, uint32_t M, uint32_t K) {
 // conversion.  false: not taken (nothing launched).
 bool launch_glu_act_f16(const Map* ma, uint32_t op, uint32_t a, uint32_t b, uint32_t d, uint32_t M, uint32_t K) {
   if (K > 16384u || (K & 7u) || M == 0 || knob("ADAMAH_ACT_REGS", 1) == 0) return false;
-  float* scale; __half *xh, *xl;
-  if (!gemm_act_slots(M, K, &scale, &xh, &xl)) return false;
+  float* scale; uint4* xf; ActForm form;
+  if (!gemm_act_slots(M, K, &scale, &xf, &form)) return false;
   float* act = (float*)ma->buf;
   const GluSrc glu = {op, a, b, d};
-  if (K <= 8192) k_act_f16_regs<1, true><<<dim3(M, 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, (uint4*)xh, (uint4*)xl, scale, act, nullptr, glu);
-  else k_act_f16_regs<2, true><<<dim3(M, 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, (uint4*)xh, (uint4*)xl, scale, act, nullptr, glu);
+  if (K <= 8192) k_act_f16_regs<1, true><<<dim3(M, 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form);
+  else k_act_f16_regs<2, true><<<dim3(M, 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form);
   count_launch();
   gemm_act_mark(ma->buf, d, M, K);
   return true;
@@ -1037,7 +1177,7 @@ bool launch_glu_act_f16(const Map* ma, uint32_t op, uint32_t a, uint32_t b, uint
 template <int NW>
 __global__ void __launch_bounds__(1024)
 k_attn_merge_rows_f16(float* out, const float* __restrict__ partial, uint32_t o0, uint32_t M, uint32_t K, uint32_t D,
-                      uint32_t splits, float* scale, uint4* xh, uint4* xl) {
+                      uint32_t splits, float* scale, uint4* xf, ActForm form) {
   __shared__ float red[16];
   const uint32_t row = blockIdx.x, tid = threadIdx.x, kw = K >> 3, heads = K / D, stride = D + 2u, last = splits - 1u;
   float v[NW][8];
@@ -1108,8 +1248,8 @@ k_attn_merge_rows_f16(float* out, const float* __restrict__ partial, uint32_t o0
     const float x[8] = {v[u][0] * s, v[u][1] * s, v[u][2] * s, v[u][3] * s, v[u][4] * s, v[u][5] * s, v[u][6] * s, v[u][7] * s};
     uint4 hi, lo;
     split_word(x, &hi, &lo);
-    xh[(uint64_t)row * kw + w] = hi;
-    xl[(uint64_t)row * kw + w] = lo;
+    xf[act_piece(form, 0u, row, w, 0u)] = hi;
+    xf[act_piece(form, 0u, row, w, 1u)] = lo;
   }
 }
 
@@ -1118,9 +1258,9 @@ k_attn_merge_rows_f16(float* out, const float* __restrict__ partial, uint32_t o0
 bool launch_attn_merge_rows_f16(const Map* ma, const float* partial, uint32_t o0, uint32_t M, uint32_t K, uint32_t D,
                                 uint32_t splits) {
   if (K > 8192u || (K & 7u) || (D & 7u) || K % D || splits < 2 || splits > 8 || M == 0 || knob("ADAMAH_ACT_REGS", 1) == 0) return false;
-  float* scale; __half *xh, *xl;
-  if (!gemm_act_slots(M, K, &scale, &xh, &xl)) return false;
-  k_attn_merge_rows_f16<1><<<M, 1024, 0, g.stream>>>((float*)ma->buf, partial, o0, M, K, D, splits, scale, (uint4*)xh, (uint4*)xl);
+  float* scale; uint4* xf; ActForm form;
+  if (!gemm_act_slots(M, K, &scale, &xf, &form)) return false;
+  k_attn_merge_rows_f16<1><<<M, 1024, 0, g.stream>>>((float*)ma->buf, partial, o0, M, K, D, splits, scale, xf, form);
   count_launch();
   gemm_act_mark(ma->buf, o0, M, K);
   return true;
@@ -1131,8 +1271,10 @@ bool launch_attn_merge_rows_f16(const Map* ma, const float* partial, uint32_t o0
 void gemm_act_forget() { g_xh_key.valid = false; }
 
 // How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 0
-// k_gemm_q4_ring<ma>, 0 the tiled kernel; over how many shares of K.
-// 33 .. 64 rows: tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
+// k_gemm_q4_ring<ma>, 0 the tiled kernel, over how many shares of K; -1 k_gemm_q4_rows.
+// 33 .. 64 rows: k_gemm_q4_rows where a CU has few tiles of 16 weight rows and K is not long, by its time for a round of tiles and
+// a 128-column step (48 rows: 4096 x 4096 12.5 us, tiled 20.8, 6144 x 4096 15.9 and 23.4; 4096 x 14336 38.7 and 33.0; 64 rows:
+// 28672 x 4096 73 and 64).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
 // a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x
 // 2048: 23 -> 17 over four; 64 x 28672 x 2048 38 in one, 44 in four, 64 x 28672 x 4096 67 and 62).
 // More: the least of these estimates, in us, fitted to both kernels over 2900 plans of 65 .. 2049 rows by 512 .. 32000 x 128 ..
@@ -1160,6 +1302,9 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     while (sp > 1 && K / sp < 512u) sp--;
     const bool alone = up(N, 256) * sp <= cu;
     const double us = (alone ? 3.0 : 4.7) * (double)up(steps, sp) + (alone ? 11.0 : 17.8) + (double)(sp + 1) * pass;
+    const uint64_t two = up(N, 16) > cu ? 2 : 1, rounds = up(up(N, 16 * two), cu);
+    const double step = M <= 48 ? (two > 1 ? 0.43 : 0.31) : two > 1 ? 0.53 : 0.40;
+    if (tuning("ADAMAH_GEMM_ROWS", 1) && 4.0 + (double)(rounds * steps) * step < std::min(best, sp > 1 ? us : best)) return {-1, 1};
     return {0, sp > 1 && us < best ? (uint32_t)sp : 1u};
   }
   if (ring == 0 || b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {
@@ -1184,7 +1329,7 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
 // Whether the matmul's launches also store an add that consumes its result (more than 32 rows, one op)
 bool gemm_q4_adds(uint32_t M, uint32_t K, uint32_t N, int64_t b) {
   const GemmPlan p = gemm_plan(M, K, N, b);
-  return p.ma > 0 || p.shares > 1;
+  return p.ma != 0 || p.shares > 1;
 }
 
 // Preconditions (checked by the caller against the host copies of the handles): Q4 map whose blocks
@@ -1203,6 +1348,8 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   if (segs) sg = *segs;
   const size_t need = (size_t)2 * M * n_ops;
   const size_t plane = (size_t)n_ops * M * K * 2;
+  size_t act_bytes;
+  const ActForm form = act_form(M, K, n_ops, &act_bytes);
   const bool reuse = g_xh_key.valid && n_ops == 1 && a_host >= 0 && g_xh_key.buf == ma->buf && g_xh_key.a == (uint64_t)a_host &&
                      g_xh_key.M == M && g_xh_key.K == K && g_xh_key.dispatch == g.stats.dispatch &&
                      g_xh_key.mem_gen == g.mem_gen && g_xh_key.plane == plane && tuning("ADAMAH_GEMM_REUSE", 1) != 0;
@@ -1214,66 +1361,68 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     if (!out && c0 < a1 && a0 < c1) return;
     g_xh_key = {ma->buf, a0, M, K, g.stats.dispatch, g.mem_gen, plane, true};
   };
-  if (!reuse && !ensure_act_bufs(need, 2 * plane)) return ADAMAH_ERR_MEMORY;
+  if (!reuse && !ensure_act_bufs(need, act_bytes)) return ADAMAH_ERR_MEMORY;
   float* act = (float*)ma->buf;
   uint32_t mt = M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8;
   uint4* const xh = g_xh_buf;
   uint4* const xl = (uint4*)((uint8_t*)g_xh_buf + plane);
   if (!reuse) {
     if (K <= 16384 && knob("ADAMAH_ACT_REGS", 1) != 0) {
-      if (K <= 8192) k_act_f16_regs<1, false><<<dim3(M, n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, xl, g_scale_buf, act, la, GluSrc{});
-      else k_act_f16_regs<2, false><<<dim3(M, n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, xl, g_scale_buf, act, la, GluSrc{});
+      if (K <= 8192) k_act_f16_regs<1, false><<<dim3(M, n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form);
+      else k_act_f16_regs<2, false><<<dim3(M, n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form);
     } else
-      k_act_f16<<<dim3(M, n_ops), 256, 0, g.stream>>>(act, la, M, K, g_scale_buf, xh, xl);
+      k_act_f16<<<dim3(M, n_ops), 256, 0, g.stream>>>(act, la, M, K, g_scale_buf, xh, form);
     count_launch();
   }
-  auto wgs = [&](uint32_t rows_per_wg, uint32_t t) { return (uint64_t)cdiv(N, rows_per_wg) * cdiv(M, 16 * t) * n_ops; };
-  const uint64_t want = 2ull * (uint64_t)g.n_cu;
-  if (mt <= 2) {
-    // few activation rows: the K-split form, as many weight-row tiles per workgroup as still fill the chip
-    uint32_t R = wgs(64, mt) >= want ? 4 : wgs(32, mt) >= want ? 2 : 1;
-    R = (uint32_t)knob("ADAMAH_GEMM_R", (int)R);
-    R = R >= 4 ? 4 : R >= 2 ? 2 : 1;
-    if (q8 && R > 2) R = 2;   // a Q8 tile holds twice the registers
-    if (sg.glu) {             // a workgroup pairs one gate tile with its up tile
-      if (sg.count != 2 || sg.n[0] != sg.n[1] || (sg.n[0] & 15u)) return ADAMAH_ERR_INVALID;
-      R = 2;
-    }
-    // many weight rows under at most 16 activation rows: the form whose eight waves share the activation tile, when
-    // its workgroups of 128 weight rows still cover three quarters of the CUs (28672x4096: 28.5 against 32.5 us)
-    {
-      const bool glu_ok = !sg.glu || (sg.count == 2 && sg.n[0] == sg.n[1] && (sg.n[0] & 15u) == 0);
-      const uint32_t wgs16 = cdiv(sg.glu ? N / 2 : N, sg.glu ? 64u : 128u);
-      if (mt == 1 && !q8 && !sg.add && glu_ok && (uint64_t)wgs16 * 4 >= 3ull * (uint64_t)g.n_cu &&
-          tuning("ADAMAH_GEMM_ROWS16", 1) != 0) {
-        dim3 gridr(wgs16, 1, n_ops);
-        k_gemm_q4_f16_rows16<8><<<gridr, 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val,
-                                                            out ? (by_val & 1u) : by_val, out ? out : act, lb, out ? nullptr : lc,
-                                                            g_scale_buf, sg);
-        count_launch();
-        keep();
-        return check_launch();
-      }
-    }
-    dim3 grid(cdiv(N, 16 * R), cdiv(M, 16 * mt), n_ops);
-    float* dst = out ? out : act;
-    const uint32_t* lcd = out ? nullptr : lc;
-    // eight waves where the matrix has too few weight rows for larger tiles (measured: no gain otherwise)
-    const uint32_t nwv = mt == 1 && !q8 ? (uint32_t)knob("ADAMAH_GEMM_NWV", R == 1 ? 8 : 4) : 4u;
-#define GK(T, RR, W, Q) k_gemm_q4_f16_ksplit<T, RR, W, Q><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, out ? (by_val & 1u) : by_val, dst, lb, lcd, g_scale_buf, sg)
-    if (q8) {
-      if (mt == 1) { if (R == 2) GK(1, 2, 4, true); else GK(1, 1, 4, true); }
-      else { if (R == 2) GK(2, 2, 4, true); else GK(2, 1, 4, true); }
-    }
-    else if (mt == 1 && nwv >= 8) { if (R == 4) GK(1, 4, 8, false); else if (R == 2) GK(1, 2, 8, false); else GK(1, 1, 8, false); }
-    else if (mt == 1) { if (R == 4) GK(1, 4, 4, false); else if (R == 2) GK(1, 2, 4, false); else GK(1, 1, 4, false); }
-    else { if (R == 4) GK(2, 4, 4, false); else if (R == 2) GK(2, 2, 4, false); else GK(2, 1, 4, false); }
+  if (sg.glu && (sg.count != 2 || sg.n[0] != sg.n[1] || (sg.n[0] & 15u))) return ADAMAH_ERR_INVALID;
+  float* const dst = out ? out : act;
+  const uint32_t* const lcd = out ? nullptr : lc;
+  const uint32_t by_dst = out ? (by_val & 1u) : by_val, tiles16 = cdiv(N, 16), cu = (uint32_t)g.n_cu;
+  GemmPlan plan = n_ops == 1 && !q8 && !out && M > 32 ? gemm_plan(M, K, N, b_host) : GemmPlan{0, 1};
+  if (q8) {
+    const uint32_t R = sg.glu || (uint64_t)cdiv(N, 32) * cdiv(M, 16 * mt) * n_ops >= 2ull * cu ? 2 : 1;
+    const dim3 grid(cdiv(N, 16 * R), 1, n_ops);
+#define GK(T, RR) k_gemm_q8_f16_ksplit<T, RR><<<grid, 256, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst, dst, lb, lcd, g_scale_buf, sg)
+    if (mt == 1) { if (R == 2) GK(1, 2); else GK(1, 1); }
+    else { if (R == 2) GK(2, 2); else GK(2, 1); }
 #undef GK
     count_launch();
     keep();
     return check_launch();
   }
-  GemmPlan plan = n_ops == 1 && !q8 && !out ? gemm_plan(M, K, N, b_host) : GemmPlan{0, 1};
+  // at most 16 activation rows and workgroups of 128 weight rows for three quarters of the CUs: the form whose eight waves share an
+  // activation tile in LDS (28672 x 4096, 16 rows: 24.8 us, k_gemm_q4_rows 30.4; 8 rows: 24.4 and 24.1)
+  const uint32_t wgs16 = cdiv(sg.glu ? N / 2 : N, sg.glu ? 64u : 128u);
+  if (mt == 1 && !sg.add && (uint64_t)wgs16 * 4 >= 3ull * cu && tuning("ADAMAH_GEMM_ROWS16", 1) != 0) {
+    k_gemm_q4_f16_rows16<8><<<dim3(wgs16, 1, n_ops), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst,
+                                                                        dst, lb, lcd, g_scale_buf, sg);
+    count_launch();
+    keep();
+    return check_launch();
+  }
+  if (M <= 32 || plan.ma < 0) {
+    // As many tiles of 16 weight rows to a workgroup as a CU has: one workgroup per CU reads its activations once (8 rows: 4096 x
+    // 4096 one tile 5.2 us, two 7.8; 6144 x 4096 two 8.2, four 12.7; 13824 x 1152 four 6.9, one 9.7).  One and two tiles
+    // of weights take the same number of waves, so that a stacked matrix has the same sums as its parts; eight where 16 waves
+    // would not have the registers (three and more operand tiles, four tiles of weights)
+    const uint32_t R = tiles16 <= cu && !sg.glu ? 1 : tiles16 <= 2 * cu || form.tiles > 4 ? 2 : 4;
+    const dim3 grid(sg.glu ? cdiv(N / 2, 8 * R) : cdiv(N, 16 * R), 1, n_ops);
+#define GW(T, RR, W, D, DA) k_gemm_q4_rows<T, RR, W, D, DA><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst, dst, lb, lcd, g_scale_buf, sg)
+#define GWT(T) do { if (R == 1) GW(T, 1, 8, 2, 1); else if (R == 2) GW(T, 2, 8, 2, 1); else GW(T, 4, 8, 1, 1); } while (0)
+    if (form.tiles == 1) { if (R == 1) GW(1, 1, 16, 2, 2); else if (R == 2) GW(1, 2, 16, 2, 2); else GW(1, 4, 8, 1, 1); }
+    else if (form.tiles == 2) { if (R == 1) GW(2, 1, 16, 2, 1); else if (R == 2) GW(2, 2, 16, 2, 1); else GW(2, 4, 8, 1, 1); }
+    else if (form.tiles == 3) GWT(3);
+    else if (form.tiles == 4) GWT(4);
+    else if (form.tiles <= 6) { if (R == 1) GW(6, 1, 8, 2, 1); else GW(6, 2, 8, 1, 1); }
+    else { if (R == 1) GW(8, 1, 8, 2, 1); else GW(8, 2, 8, 1, 1); }
+#undef GWT
+#undef GW
+    count_launch();
+    keep();
+    return check_launch();
+  }
+  const auto wgs = [&](uint32_t rows_per_wg, uint32_t t) { return (uint64_t)cdiv(N, rows_per_wg) * cdiv(M, 16 * t) * n_ops; };
+  const uint64_t want = 2ull * (uint64_t)g.n_cu;
   const auto add_up = [&](uint32_t shares) {
     const uint64_t quads = ((uint64_t)M * N + 3) / 4;
     k_gemm_splitk_sum<<<cdiv(quads, 256), 256, 0, g.stream>>>(g_part_buf, shares, M, N, act, c_val, by_val, lc, g_scale_buf, sg);
@@ -1300,8 +1449,8 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   }
   if (plan.shares > 1) {                         // 256 weight rows a workgroup over shares of K
     const uint32_t kper = cdiv(cdiv(K >> 5, plan.shares), 4u) * 4u, shares = cdiv(K >> 5, kper);
-#define GS(T) k_gemm_q4_f16_tiled<T, 2, 8><<<dim3(cdiv(N, 256), cdiv(M, 16 * T), shares), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, shares, kper, g_part_buf)
-    if (mt == 4) GS(4); else GS(8);
+#define GS(T, F) k_gemm_q4_f16_tiled<T, 2, 8, F><<<dim3(cdiv(N, 256), cdiv(M, 16 * T), shares), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, shares, kper, g_part_buf)
+    if (mt == 4) GS(4, true); else GS(8, false);      // (four tiles of rows: at most 64 of them)
 #undef GS
     count_launch();
     add_up(shares);
@@ -1325,12 +1474,14 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   R = R >= 4 && mt == 4 ? 4 : R >= 2 ? 2 : 1;
   if (mt == 4 && NW == 8 && R == 1) R = 2;
   dim3 grid(cdiv(N, 16 * NW * R), cdiv(M, 16 * mt), n_ops);
-#define GT(T, RR, W) k_gemm_q4_f16_tiled<T, RR, W><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, 1, K >> 5, nullptr)
-  if (mt == 4 && NW == 8) { if (R == 4) GT(4, 4, 8); else GT(4, 2, 8); }
-  else if (mt == 4) { if (R == 4) GT(4, 4, 4); else if (R == 2) GT(4, 2, 4); else GT(4, 1, 4); }
-  else if (NW == 8) { if (R == 2) GT(8, 2, 8); else GT(8, 1, 8); }
-  else { if (R == 2) GT(8, 2, 4); else GT(8, 1, 4); }
+#define GTF(T, RR, W, F) k_gemm_q4_f16_tiled<T, RR, W, F><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form, K, N, M, b_val, c_val, by_val, act, lb, lc, g_scale_buf, sg, 1, K >> 5, nullptr)
+#define GT(RR, W) do { if (form.tiles) GTF(4, RR, W, true); else GTF(4, RR, W, false); } while (0)
+  if (mt == 4 && NW == 8) { if (R == 4) GT(4, 8); else GT(2, 8); }
+  else if (mt == 4) { if (R == 4) GT(4, 4); else if (R == 2) GT(2, 4); else GT(1, 4); }
+  else if (NW == 8) { if (R == 2) GTF(8, 2, 8, false); else GTF(8, 1, 8, false); }
+  else { if (R == 2) GTF(8, 2, 4, false); else GTF(8, 1, 4, false); }
 #undef GT
+#undef GTF
   count_launch();
   keep();
   return check_launch();

@@ -146,7 +146,16 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
 // For a kernel that produces the rows [M, K] of a coming batched matmul: the buffers of their fp16 form
 // ((s, 1/s) per row; two planes of K halves per row: fp16(x s) and the fp16 remainder), grown as needed, and -- after that kernel's launch has been
 // counted -- the note that rows [a, a + M K) of `buf` are converted, so the matmul skips its conversion.
-bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, __half** xh, __half** xl);
+// Where the pieces (eight columns, 16 bytes) of those rows go.  tiles == 0: rows of both planes, [plane][op][row][kw], the
+// second plane `lo` pieces behind the first.  Otherwise the matmul's operand tiles: the 2 M rows of both planes of an op, first plane
+// first, 16 to a tile; of a tile and block of 32 columns the 64 pieces are in the order in which a wave's lanes take them.
+struct ActForm { uint32_t M, kw, tiles; uint64_t lo; };
+__device__ __forceinline__ uint64_t act_piece(const ActForm& f, uint32_t op, uint32_t row, uint32_t w, uint32_t plane) {
+  if (!f.tiles) return ((uint64_t)op * f.M + row) * f.kw + w + plane * f.lo;
+  const uint32_t v = plane * f.M + row;
+  return ((uint64_t)op * f.tiles + (v >> 4)) * f.kw * 16u + ((w & ~3u) << 4) + ((w & 3u) << 4) + (v & 15u);
+}
+bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, uint4** x, ActForm* form);
 void gemm_act_forget();
 // Gated activation (op2 34 GEGLU / 35 SWIGLU) of the [M, K] rows at elements a and b into the rows at d, and the fp16
 // form of the result for the batched matmul that follows, in one launch.  false: not taken, nothing launched.

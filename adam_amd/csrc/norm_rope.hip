@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(256)
 k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, uint32_t s0, uint32_t ss_, uint32_t w0, uint32_t ws,
                uint32_t d0, uint32_t ds, uint32_t r0, uint32_t rs, float* out,
                const uint32_t* __restrict__ ls, const uint32_t* __restrict__ lw, const uint32_t* __restrict__ lr,
-               const uint32_t* __restrict__ ld, uint64_t act_elems, uint64_t wt_elems, float* scale, __half* xh, __half* xl) {
+               const uint32_t* __restrict__ ld, uint64_t act_elems, uint64_t wt_elems, float* scale, __half* xf, ActForm form) {
   // (these 14 dwords are in registers when a wave starts.  Top bit of dim_on: row i's source / weights / destination /
   // residual start at x0 + i xs -- the host found the rows evenly spaced -- instead of four loads from the row
   // tables, which the rows' own loads would have to wait for)
@@ -101,17 +101,15 @@ k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, ui
   if (e >= 14u && e <= 254u) { s = __uint_as_float((267u - e) << 23); si = __uint_as_float((e - 13u) << 23); }
   if (tid == 0) { scale[2 * ri] = s; scale[2 * ri + 1] = si; }
   // two planes: fp16(x s) and the fp16 remainder x s - fp16(x s), as the matmul's own conversion writes them
-  __half* dst = xh + (uint64_t)ri * dim;
-  __half* dstl = xl + (uint64_t)ri * dim;
 #pragma unroll
   for (int u = 0; u < NU; u++) {
     const uint32_t i = tid + 256u * u, q = i & 7u;
     if (i < dim) {
-      const uint32_t at = (i & ~7u) + (q < 4u ? 2u * q : 2u * (q - 4u) + 1u);
+      const uint32_t at = q < 4u ? 2u * q : 2u * (q - 4u) + 1u;
       const float v = x[u] * s;
       const __half h = __float2half(v);
-      dst[at] = h;
-      dstl[at] = __float2half(v - __half2float(h));
+      xf[act_piece(form, 0u, ri, i >> 3, 0u) * 8u + at] = h;
+      xf[act_piece(form, 0u, ri, i >> 3, 1u) * 8u + at] = __float2half(v - __half2float(h));
     }
   }
 }
@@ -231,8 +229,9 @@ static int rmsnorm_impl(uint32_t map_act, uint32_t map_wt, uint32_t hs, uint32_t
       emit = in_range(sh[i], dim, ma->n_elems) && in_range(dh[i], dim, ma->n_elems) && in_range(wh[i], dim, mw->n_elems) &&
              (!add || in_range(rh[i], dim, ma->n_elems));
     float* scale = nullptr;
-    __half *xh = nullptr, *xl = nullptr;
-    if (emit) emit = gemm_act_slots(n_rows, dim, &scale, &xh, &xl);
+    uint4* xf = nullptr;
+    ActForm form = {};
+    if (emit) emit = gemm_act_slots(n_rows, dim, &scale, &xf, &form);
     const float* w = (const float*)mw->buf;
     // evenly spaced rows (the usual case: rows of a matrix, one weight vector): their places go by value
     RowsByValue rv = {};
@@ -248,7 +247,7 @@ static int rmsnorm_impl(uint32_t map_act, uint32_t map_wt, uint32_t hs, uint32_t
       }
       if (!even) rv.on = 0u;
     }
-#define RR(A, E, NU) k_rmsnorm_rows<A, E, NU><<<n_rows, 256, 0, g.stream>>>(a, w, dim | (rv.on << 31), eps, rv.s0, rv.ss, rv.w0, rv.ws, rv.d0, rv.ds, rv.r0, rv.rs, a, ls, lw, lr, ld, ma->n_elems, mw->n_elems, scale, xh, xl)
+#define RR(A, E, NU) k_rmsnorm_rows<A, E, NU><<<n_rows, 256, 0, g.stream>>>(a, w, dim | (rv.on << 31), eps, rv.s0, rv.ss, rv.w0, rv.ws, rv.d0, rv.ds, rv.r0, rv.rs, a, ls, lw, lr, ld, ma->n_elems, mw->n_elems, scale, (__half*)xf, form)
 #define RN(A, E) do { if (dim <= 2048) RR(A, E, 8); else if (dim <= 4096) RR(A, E, 16); else RR(A, E, 32); } while (0)
     if (add) { if (emit) RN(true, true); else RN(true, false); }
     else { if (emit) RN(false, true); else RN(false, false); }

@@ -589,3 +589,50 @@ def test_tiles_in_runs_per_die(hip, monkeypatch, M, N, K):
     want = x[0].astype(np.float64) @ qt.dequant().astype(np.float64).T
     for m in range(M):
         assert rel_l2(y[m], want[m]) < TOL_Q4, m
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 16, 128), (3, 8209, 256), (8, 17, 384), (9, 5000, 128), (16, 8210, 640), (17, 40, 2176), (24, 8201, 128),
+                                   (25, 4113, 384), (32, 9000, 256), (33, 100, 128), (40, 4100, 1152), (48, 8200, 256), (49, 4090, 640), (64, 31, 4224)])
+def test_few_rows_on_every_operand_and_weight_tile(hip, M, N, K):
+    """2 .. 64 activation rows: one to eight operand tiles of both planes, one, two and four tiles of weights to a workgroup, ragged
+    in every one; fewer steps of K than waves, and numbers of steps that they do not share evenly.  Rows of very different size keep
+    their own scale, and two ops in one call their own rows and weights."""
+    rng = np.random.default_rng(M + N + K)
+    qt = quant.quantize_q4_0((rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.02)))
+    x = rng.standard_normal((2, M, K), dtype=np.float32)
+    x[:, M - 1] *= 1e4
+    w = qt.dequant().astype(np.float64)
+    for n_ops in (1, 2):
+        note(f"few rows M={M} N={N} K={K} ops={n_ops}")
+        y = run(hip, qt, x[:n_ops], n_ops=n_ops)
+        for op in range(n_ops):
+            want = x[op].astype(np.float64) @ w.T
+            for m in range(M):
+                assert rel_l2(y[op, m], want[m]) < TOL_Q4, (op, m)
+
+
+@pytest.mark.parametrize("M,K,Ns", [(6, 1152, (3000, 3000)), (24, 256, (40, 24, 16)), (48, 640, (4000, 100)), (64, 384, (70,))])
+def test_few_rows_store_stacked_results_and_adds(hip, M, K, Ns):
+    """The kernel of few rows places the results of stacked matrices and, over one matrix, stores the add that consumes them."""
+    rng = np.random.default_rng(M + K)
+    N = sum(Ns)
+    qt = quant.quantize_q4_0(rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05))
+    x, r = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((M, Ns[0]), dtype=np.float32)
+    want = x.astype(np.float64) @ qt.dequant().astype(np.float64).T
+    load_qtensor(hip, 1, qt)
+    at = np.cumsum([0] + [M * n for n in Ns])
+    f32map(hip, 0, M * K + int(at[-1]) + M * Ns[0], np.concatenate([x.reshape(-1), np.zeros(int(at[-1]), np.float32), r.reshape(-1)]))
+    first, res = np.cumsum([0] + list(Ns)), M * K + int(at[-1])
+    note(f"few rows stacked M={M} K={K} Ns={Ns}")
+    hip.batch_begin()
+    for i, n in enumerate(Ns):
+        hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [int(first[i]) * K]), up(hip, [M * K + int(at[i])]), M, K, n, 1)
+    if len(Ns) == 1:
+        span = lambda lo: up(hip, np.arange(lo, lo + M * N))
+        hip.map_op2_dev(0, A.OP_ADD, span(res), span(M * K), span(res), M * N)
+    hip.batch_end()
+    for i, n in enumerate(Ns):
+        got = read(hip, 0, M * K + int(at[i]), M * n).reshape(M, n)
+        assert rel_l2(got, want[:, first[i]:first[i + 1]]) < TOL_Q4, i
+    if len(Ns) == 1:
+        assert rel_l2(read(hip, 0, res, M * N).reshape(M, N), want + r) < TOL_Q4
