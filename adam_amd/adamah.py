@@ -123,6 +123,7 @@ _SIGS = {
     "adamah_clear_decode_plan": (None, [_U]), "adamah_decode_step": (i32, [_U] * 3),
     "adamah_kv_cache_fp16": (i32, [_U] * 3),
     "adamah_attn_causal_rows_dev": (i32, [_U, pu32, _U, _U, _U, pu32, _U, _U, _U, _U, _U, f32c, f32c]),
+    "adamah_hip_rope_append_rows_dev": (i32, [_U] * 12 + [pu32, pu32, _U, _U, f32c, _U]),
     "adamah_qk_norm_rope_rows_dev": (i32, [_U, _U, pu32, _U, pu32, _U, pu32, _U, _U, _U, _U, _U, _U, f32c]),
     "batch_begin": (None, []), "batch_end": (None, []),
     "map_init": (i32, [_U] * 4), "map_init_dtype": (i32, [_U] * 5), "map_destroy": (i32, [_U]),
@@ -468,6 +469,15 @@ class Adamah:
         oa = (ctypes.c_uint32 * m)(*out_handles)
         self._op("adamah_attn_causal_rows_dev", map_id, qa, locs_k_handle, locs_scores_handle, locs_v_handle, oa, m,
                  head_dim, n_keys0, n_heads, value_dim, scale, softcap)
+
+    def rope_append_rows_dev(self, map_id, q, q_step, q_heads, k, k_step, k_heads, v, v_step, head_dim, n_tok, k_cache, v_cache, head_step,
+                             pos0, freq_base, rotate=True):
+        """Extension: for len(k_cache) sequences of n_tok tokens side by side, the rotation of their Q and K heads (rotate) and
+        the append of their K and V rows to the caches, in one native call."""
+        n = len(k_cache)
+        kc, vc = (ctypes.c_uint32 * n)(*k_cache), (ctypes.c_uint32 * n)(*v_cache)
+        self._op("adamah_hip_rope_append_rows_dev", map_id, q, q_step, q_heads, k, k_step, k_heads, v, v_step, head_dim, n_tok, n, kc, vc,
+                 head_step, pos0, freq_base, int(rotate))
 
     def embed_tokens_dev(self, map_act, map_src, locs_tokens_handle, src_row0, dst_start, m, E, V, scale=1.0):
         """Extension: embedding rows of m tokens whose ids (float32) are still on the device, scaled, into

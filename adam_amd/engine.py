@@ -74,6 +74,7 @@ class ModelConfig:
 
 
 class DecodeEngine:
+    _prompts_together = True        # several prompts of a batch in one pass over the weights
     WS_MAP = 0
     Q8_MAP = 2
     EMB_MAP = 15          # float32 copy of an untied embedding table, made when the greedy loops run ahead
@@ -390,6 +391,7 @@ class DecodeEngine:
         self._c_emb_hs = {}
         self._c_wrows = {}
         self._c_kvspec = {}
+        self._c_hidden1 = {}
         if c.emb_scale != 1.0:
             self._c_embscale_h = self._up(np.full(M * c.n_embd, self._pos_emb_scale))
         return pos
@@ -1104,7 +1106,7 @@ class DecodeEngine:
             residual('ffn_out', f'{p}.post_ffw_norm.weight')
         return ops
 
-    def _forward_chunk(self, toks, pos0, sample=True, seq=0, lockstep=False, from_device=False):
+    def _forward_chunk(self, toks, pos0, sample=True, seq=0, lockstep=False, from_device=False, seqs=None):
         """m <= prefill_chunk prompt tokens at positions pos0 .. pos0 + m - 1 in one pass: the row-wise ops
         over m rows, the projections as [m, K] x [N, K]^T matmuls (the fp16 matrix-core kernel for Q4
         blocks), RoPE and the KV append for all tokens at once, attention token by token over the growing
@@ -1115,9 +1117,12 @@ class DecodeEngine:
         position pos0 -- a batched decode step: every row is rotated for pos0, appended to and attended
         over its own sequence's cache, and gets its own LM head pass (tokens in `read_tokens`).
         `from_device` (a lockstep step of the full batch): the rows' tokens are the ones the previous step left in
-        the token slots (`toks` is not looked at); their embedding rows are gathered on the device."""
+        the token slots (`toks` is not looked at); their embedding rows are gathered on the device.
+        `seqs`: the rows are len(toks) / len(seqs) tokens of each of these sequences, one sequence after the other, all from
+        pos0 on; the token that follows row block i is left in the token slot of row i (the last block's in the decode slot)."""
         c, g, A, ws = self.cfg, self.gpu, self.A, self.WS_MAP
         m = self._batch if from_device else len(toks)
+        each = m // len(seqs) if seqs else m            # rows of a sequence
         if not self._chunk or m == 0 or m > self._chunk:
             raise RuntimeError(f"chunk of {m} tokens does not fit prefill_chunk={self._chunk}")
         E, FF = c.n_embd, c.n_ff
@@ -1173,16 +1178,21 @@ class DecodeEngine:
             mm('normed', f'{p}.attn_q.weight', 'q', E, q_dim)
             mm('normed', f'{p}.attn_k.weight', 'k', E, k_dim)
             mm('normed', f'{p}.attn_v.weight', 'v', E, k_dim)
+            append = not lockstep and m > 1 and hasattr(g, 'rope_append_rows_dev')    # rotation and KV append in one call
             if self._chunk_qk and not lockstep and hasattr(g, 'qk_norm_rope_rows_dev'):
-                g.qk_norm_rope_rows_dev(ws, ws, self._c_lq[:m], self._wh[f'{p}.attn_q_norm.weight'], self._c_lk[:m],
-                                        self._wh[f'{p}.attn_k_norm.weight'], self._c_qkdst[:m], c.n_head, c.head_dim,
-                                        c.n_head_kv, c.head_dim_kv, pos0, freq)
+                for lo in range(0, m, each):
+                    hi = lo + each
+                    g.qk_norm_rope_rows_dev(ws, ws, self._c_lq[lo:hi], self._wh[f'{p}.attn_q_norm.weight'], self._c_lk[lo:hi],
+                                            self._wh[f'{p}.attn_k_norm.weight'], self._c_qkdst[lo:hi], c.n_head, c.head_dim,
+                                            c.n_head_kv, c.head_dim_kv, pos0, freq)
             elif self._chunk_qk:
                 qn, kn = self._wh[f'{p}.attn_q_norm.weight'], self._wh[f'{p}.attn_k_norm.weight']
                 for t in range(m):
                     g.map_qk_norm_rope_x_dev(ws, ws, self._c_lq[t], qn, self._c_lk[t], kn, self._c_qkdst[t],
                                              c.n_head, c.head_dim, c.n_head_kv, c.head_dim_kv,
                                              pos0 if lockstep else pos0 + t, freq)
+            elif append:
+                pass
             elif lockstep:
                 # every row sits at the same position: the m rows' heads rotate as the heads of one token
                 g.map_rope_dev(ws, self._c_qbase, self._c_qbase, 1, m * c.n_head, c.head_dim, pos0, freq)
@@ -1190,13 +1200,22 @@ class DecodeEngine:
             else:
                 g.map_rope_dev(ws, CR['q'], CR['q'], m, c.n_head, c.head_dim, pos0, freq)
                 g.map_rope_dev(ws, CR['k'], CR['k'], m, c.n_head_kv, c.head_dim_kv, pos0, freq)
-            g.map_row_copy_offset_dev(ws, self._b_kvspec[L] if lockstep else self._c_kvspec[(seq, L)], self._c_zero, pos0,
-                                      2 * c.n_head_kv * m, c.head_dim_kv)
+            if append:
+                qk_w, D = (q_dim + k_dim, c.head_dim_kv) if self._chunk_qk else (k_dim, c.head_dim)
+                g.rope_append_rows_dev(ws, self._cp['qk'] if self._chunk_qk else self._cp['q'], qk_w if self._chunk_qk else q_dim, c.n_head,
+                                       self._cp['qk'] + q_dim if self._chunk_qk else self._cp['k'], qk_w, c.n_head_kv, self._cp['v'], k_dim, D, each,
+                                       [self._k_base_s[sq][L] for sq in seqs or [seq]], [self._v_base_s[sq][L] for sq in seqs or [seq]],
+                                       self._kv_step, pos0, freq, rotate=not self._chunk_qk)
+            else:
+                g.map_row_copy_offset_dev(ws, self._b_kvspec[L] if lockstep else self._c_kvspec[(seq, L)], self._c_zero, pos0,
+                                          2 * c.n_head_kv * m, c.head_dim_kv)
             if not lockstep and hasattr(g, 'attn_causal_rows_dev'):
-                # the m (scores, softmax . V) pairs of the chunk in one native call
-                g.attn_causal_rows_dev(ws, self._c_qrows[:m], self._k_locs_hs[seq][L], self._scores_row_h,
-                                       self._v_locs_hs[seq][L], self._c_aorows[:m], c.head_dim, pos0 + 1, c.n_head,
-                                       c.head_dim_kv, scale, float(c.attn_softcap))
+                # the (scores, softmax . V) pairs of the chunk, one native call a sequence
+                for i, sq in enumerate(seqs or [seq]):
+                    rows = slice(i * each, (i + 1) * each)
+                    g.attn_causal_rows_dev(ws, self._c_qrows[rows], self._k_locs_hs[sq][L], self._scores_row_h,
+                                           self._v_locs_hs[sq][L], self._c_aorows[rows], c.head_dim, pos0 + 1, c.n_head,
+                                           c.head_dim_kv, scale, float(c.attn_softcap))
             for t in range(0 if not lockstep and hasattr(g, 'attn_causal_rows_dev') else m):
                 n_keys = pos0 + 1 if lockstep else pos0 + t + 1
                 sq = t if lockstep else seq
@@ -1229,6 +1248,15 @@ class DecodeEngine:
                    W['sample_fused_val'][0], self._c_tok1[t], E, c.n_vocab, self._rows_per_group)
             g.batch_end()
             return
+        for i in range(len(seqs or ()) - 1):
+            # the last token of every sequence but the last: output norm and LM head as in a decode step, from its own row
+            row = (i + 1) * each - 1
+            if row not in self._c_hidden1:
+                self._c_hidden1[row] = self._up([self._cp['hidden'] + row * E])
+            self._rms(self._c_hidden1[row], 'output_norm.weight', W['normed'][0], 1, E)
+            fn = (g.map_matvec_argmax_t_xq8_dev if self._kind[self._lm_name] == 'q8' else g.map_matvec_argmax_t_xq4_dev)
+            fn(ws, self._map_of[self._lm_name], W['normed'][0], self._wh[self._lm_name], W['sample_fused_idx'][0],
+               W['sample_fused_val'][0], self._c_tok1[i], E, c.n_vocab, self._rows_per_group)
         # the last token's hidden state -> the decode slots; output norm and LM head as in a decode step
         src_h, _, _, _ = g.map_gather_dev(ws, self._c_last, E)
         g.map_scatter_dev(ws, W['hidden'][0], E, src_h)
@@ -1260,6 +1288,24 @@ class DecodeEngine:
             first.append(self.read_token())
         return first
 
+    def _prefill_prompts(self, prompts):
+        """Prompts of equal length into the caches of sequences 0, 1, ...; the token that follows each.  As many as the rows of a
+        chunk hold go through the weights together (eight prompts of 48 tokens one by one: eight passes over the weights)."""
+        P, g = len(prompts[0]), self.gpu
+        at_once = self._chunk // P if self._prompts_together and P else 1
+        if len(prompts) < 2 or at_once < 2 or not hasattr(g, 'rope_append_rows_dev') or not hasattr(g, 'attn_causal_rows_dev'):
+            return self._prefill_each(prompts)
+        first = []
+        for lo in range(0, len(prompts), at_once):
+            part = prompts[lo:lo + at_once]
+            if len(part) == 1:
+                self.prefill(part[0], seq=lo)
+            else:
+                self._forward_chunk([t for p in part for t in p], 0, seqs=range(lo, lo + len(part)))
+                first += self.read_tokens(len(part) - 1)
+            first.append(self.read_token())
+        return first
+
     def read_token(self):
         # reference engine.py:1979-1981: token id crosses the boundary as float32
         tok = self.gpu.gather(self.WS_MAP, self._sample_locs).view(np.float32)
@@ -1284,7 +1330,7 @@ class DecodeEngine:
         ahead = (forced is None and self._lookahead and B == self._batch and B > 1 and max_tokens > 1
                  and self._token_feed() is not None)
         t0 = time.perf_counter()
-        cur = self._prefill_each([[int(t) for t in pr] for pr in prompts])
+        cur = self._prefill_prompts([[int(t) for t in pr] for pr in prompts])
         self.gpu.sync()
         t_pre = time.perf_counter() - t0
         out = [[] for _ in range(B)]

@@ -53,6 +53,7 @@ class MixerEngine(DecodeEngine):
     WEIGHT_MAPS = [1] + list(range(4, 14))
     LOGIT_ROWS = 16                 # rows of logits a scoring step computes at a time
     MAX_POS = 1 << 24
+    _prompts_together = False       # (`_prefill_each` here does so by itself)
 
     def __init__(self, gpu, cfg, tensors, A=None, dtype="bfloat16", prefill_chunk=512, batch=1, map_elem_limit=(1 << 32) - (1 << 24),
                  decode_plan=True, plan_id=0, lookahead=True, sampling_mode=None, **kw):

@@ -245,6 +245,16 @@ int adamah_qk_norm_rope_rows_dev(uint32_t map_act, uint32_t map_wt, const uint32
                                  const uint32_t* k_src_handles, uint32_t locs_k_wt, const uint32_t* dst_handles,
                                  uint32_t m, uint32_t q_rows, uint32_t q_dim, uint32_t k_rows, uint32_t k_dim,
                                  uint32_t pos0, float freq_base);
+/* Rotation of the Q and K heads of a prompt chunk and the append of its K and V rows to the caches, for n_tok tokens of each of
+ * n_seq sequences side by side: token t of sequence s, at position pos0 + t, is row r = s * n_tok + t, with its Q heads (rotated in place)
+ * at element q + r * q_step, its K heads (rotated in place) at k + r * k_step and its V heads at v + r * v_step; head h of K goes to
+ * k_cache[s] + h * head_step + (pos0 + t) * head_dim, of V likewise.  Exactly map_rope_dev over the Q and over the K rows of every sequence
+ * and map_row_copy_offset_dev of the results.  rotate 0: Q is not touched, K is copied as it is.
+ * ADAMAH_ERR_INVALID where a range leaves the map or two of them touch.  k_cache / v_cache: host arrays of n_seq. */
+int adamah_hip_rope_append_rows_dev(uint32_t map_id, uint32_t q, uint32_t q_step, uint32_t q_heads, uint32_t k, uint32_t k_step,
+                                    uint32_t k_heads, uint32_t v, uint32_t v_step, uint32_t head_dim, uint32_t n_tok, uint32_t n_seq,
+                                    const uint32_t* k_cache, const uint32_t* v_cache, uint32_t head_step, uint32_t pos0, float freq_base,
+                                    uint32_t rotate);
 /* map_matvec_topk_t_xq4_ex_dev for callers that cannot allocate.  No counterpart in the reference: it is for
  * callers under HIP graph capture, tight serving loops and harnesses that forbid hipMalloc.  Same arguments and
  * results; the logits go to a fixed 1 MiB device array that is part of the library's code object (one copy per

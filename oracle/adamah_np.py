@@ -578,6 +578,27 @@ class NumpyAdamah(MixerOps):
             self.map_qk_norm_rope_x_dev(map_act, map_wt, qh, locs_q_wt_handle, kh, locs_k_wt_handle, dh, q_rows, q_dim,
                                         k_rows, k_dim, pos0 + t, freq_base)
 
+    def rope_append_rows_dev(self, map_id, q, q_step, q_heads, k, k_step, k_heads, v, v_step, head_dim, n_tok, k_cache, v_cache, head_step,
+                             pos0, freq_base, rotate=True):
+        """Extension shared with the HIP library: rotation of the Q and K heads and KV append of n_tok tokens of every sequence."""
+        m, D = self._map("rope_append_rows_dev", map_id, DTYPE_F32), head_dim
+        half = D // 2
+
+        def turn(base, heads, pos):
+            c, s = self._rope_cs(half, D, pos, freq_base)
+            i0 = (base + np.arange(heads) * D)[:, None] + np.arange(half)
+            x0, x1 = m.data[i0], m.data[i0 + half]
+            m.data[i0], m.data[i0 + half] = x0 * c - x1 * s, x0 * s + x1 * c
+        for sq, (kc, vc) in enumerate(zip(k_cache, v_cache)):
+            for t in range(n_tok):
+                r = sq * n_tok + t
+                if rotate:
+                    turn(q + r * q_step, q_heads, pos0 + t)
+                    turn(k + r * k_step, k_heads, pos0 + t)
+                for src, cache in ((k + r * k_step, kc), (v + r * v_step, vc)):
+                    dst = (cache + np.arange(k_heads) * head_step + (pos0 + t) * D)[:, None] + np.arange(D)
+                    m.data[dst] = self._kv_round(map_id, dst, m.data[src:src + k_heads * D].reshape(k_heads, D))
+
     def kv_cache_fp16(self, map_id, start, count):
         """Extension shared with the HIP library: elements [start, start+count) of a float32
         map are a KV cache kept in fp16.  Values copied or scattered into that range are rounded

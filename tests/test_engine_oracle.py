@@ -129,3 +129,22 @@ def test_batched_lockstep_decode_equals_independent_sequences(arch):
     assert eng.generate(prompts[1], GenerationConfig(max_tokens=6))[0] == singles[1]
     with pytest.raises(RuntimeError):
         eng.generate_batch([[1, 2], [3]], 2)
+
+
+@pytest.mark.parametrize("arch", ["gemma3", "llama"])
+@pytest.mark.parametrize("chunk", [4, 10, 15])
+def test_prompts_of_a_batch_in_one_pass_equal_one_by_one(arch, chunk):
+    """Prompts of five tokens one by one (four rows), two at a time with one left over, and all three at once: the same tokens, caches
+    and decode slots, exactly, on the oracle."""
+    cfg = synth.tiny_config(arch, n_layer=2, n_embd=64, n_head=4, n_head_kv=2, head_dim=32, n_ff=96, n_vocab=160)
+    tensors = synth.make_model(cfg, seed=3, sigma=0.3)
+    prompts = [[5, 17, 3, 101, 64], [9, 33, 2, 8, 150], [1, 1, 1, 1, 1]]
+    outs = []
+    for together in (False, True):
+        eng = DecodeEngine(oracle.init(), cfg, tensors, A=A, kv_cap=32, kv_fp16=True, batch=3, prefill_chunk=chunk)
+        eng._prompts_together = together
+        first = eng._prefill_prompts(prompts)
+        kv = eng.gpu.gather(0, np.arange(eng._kv_start, eng._kv_start + 3 * eng._kv_per_seq, dtype=np.uint32))
+        outs.append((first, eng.read_token(), kv, eng.read_slot('hidden'), eng.generate_batch(prompts, 4)[0]))
+    assert outs[0][0] == outs[1][0] and outs[0][1] == outs[1][1] and outs[0][4] == outs[1][4]
+    assert np.array_equal(outs[0][2], outs[1][2]) and np.array_equal(outs[0][3], outs[1][3])

@@ -393,3 +393,39 @@ def test_lockstep_sequences_are_one_launch(hip, B, ctx, Hq, Hkv, d, softcap):
         for h in range(Hq):
             assert rel_l2(res[0][0][b, h], res[1][0][b, h]) < TOL, (b, h)
     assert rel_l2(res[0][1], res[1][1]) < 1e-5
+
+
+@pytest.mark.parametrize("m,n_seq,Hq,Hkv,d,softcap", [(2, 2, 4, 1, 64, 0.0), (17, 3, 8, 2, 128, 0.0), (40, 2, 4, 1, 256, 50.0), (16, 5, 32, 8, 128, 0.0)])
+def test_runs_of_several_sequences_are_one_launch(hip, monkeypatch, m, n_seq, Hq, Hkv, d, softcap):
+    """The prompts of several sequences, their causal pairs issued one sequence after the other in one batch: one launch, and the words
+    (outputs of every sequence, score rows of the last one) of a batch for each."""
+    rng = np.random.default_rng(m * 10 + n_seq)
+    cap = m + 5
+    per, sc = 2 * Hkv * cap * d, Hq * cap
+    q0, o0 = sc, sc + n_seq * m * Hq * d
+    kv0 = o0 + n_seq * m * Hq * d
+    kv0 += -kv0 % d
+    x = rng.standard_normal(kv0 + n_seq * per).astype(np.float32)
+    got = []
+    for apart in (True, False):
+        note(f"attention of {n_seq} sequences m={m} apart={apart}")
+        f32map(hip, 0, x.size, x)
+        hip.kv_cache_fp16(0, kv0, n_seq * per)
+        heads = np.arange(Hq) // (Hq // Hkv)
+        calls = []
+        for s in range(n_seq):
+            kb = kv0 + s * per
+            rows = [(s * m + t) * Hq * d + np.arange(Hq) * d for t in range(m)]
+            calls.append(([up(hip, q0 + r) for r in rows], up(hip, kb + heads * cap * d), up(hip, np.arange(Hq) * cap),
+                          up(hip, kb + (Hkv + heads) * cap * d), [up(hip, o0 + r) for r in rows]))
+        launches = 0
+        for s, (qh, k, sr, v, oh) in enumerate(calls):
+            if apart or s == 0:
+                hip.batch_begin()
+            hip.attn_causal_rows_dev(0, qh, k, sr, v, oh, d, 1, Hq, d, d ** -0.5, softcap)
+            if apart or s == n_seq - 1:
+                hip.batch_end()
+                launches += hip.get_last_barrier_count()
+        got.append((read(hip, 0, 0, x.size), launches))
+    assert got[0][1] == n_seq and got[1][1] == 1
+    assert np.array_equal(got[0][0].view(np.uint32), got[1][0].view(np.uint32))

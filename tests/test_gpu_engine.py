@@ -345,3 +345,26 @@ def test_a_plan_called_with_the_same_step_is_not_recorded():
     assert json.loads(p.stdout.strip().split("\n")[-1]) == [True] * 9, p.stdout
     line = [l for l in p.stderr.split("\n") if "steps from graphs" in l]
     assert line and " 0 steps from graphs" in line[-1] and " 0 instantiations" in line[-1], p.stderr[-1000:]
+
+
+@pytest.mark.parametrize("arch", ["gemma3", "llama"])
+@pytest.mark.parametrize("chunk", [64, 45])
+def test_prompts_of_a_batch_go_through_the_weights_together(hip, arch, chunk):
+    """Four prompts of 20 tokens at 64 rows (three at once, one left over) and at 45 (two and two): the tokens that follow and the
+    caches are those of the prompts one by one, up to the rounding of matmuls of other row counts."""
+    cfg = synth.tiny_config(arch, n_layer=3, n_embd=256, n_head=4, n_head_kv=2, head_dim=64, n_ff=512, n_vocab=1000)
+    tensors = synth.make_model(cfg, seed=5, sigma=0.1)
+    rng = np.random.default_rng(3)
+    prompts = [[int(t) for t in rng.integers(0, 1000, 20)] for _ in range(4)]
+    outs = []
+    for together in (False, True):
+        note(f"engine prompts together={together} {arch} chunk={chunk}")
+        dev = DecodeEngine(hip, cfg, tensors, A=A, kv_cap=64, kv_fp16=True, batch=4, prefill_chunk=chunk)
+        dev._prompts_together = together
+        first = dev._prefill_prompts(prompts)
+        outs.append((first, dev.read_token(), dev.gpu.gather(0, np.arange(dev._kv_start, dev._kv_start + 4 * dev._kv_per_seq, dtype=np.uint32)).view(np.float32),
+                     dev.read_slot('hidden')))
+    assert outs[0][0] == outs[1][0] and outs[0][1] == outs[1][1] == outs[1][0][-1]
+    # a cached value is rounded to fp16: neighbours of a rounding edge differ by one unit in the last place
+    assert np.linalg.norm(outs[1][2] - outs[0][2]) < 1e-4 * np.linalg.norm(outs[0][2])
+    assert np.linalg.norm(outs[1][3] - outs[0][3]) < 1e-3 * np.linalg.norm(outs[0][3])

@@ -426,3 +426,52 @@ def test_plain_float_matmuls(hip, M, K, N, n_ops):
     for v in range(3):
         assert rel_l2(out["hip"][v], out["oracle"][v]) < 1e-5
         assert rel_l2(out["hip"][v], want) < 1e-5
+
+
+@pytest.mark.parametrize("n_tok,n_seq,Hq,Hk,D,pos0,rotate,kv16", [(1, 1, 4, 1, 64, 0, True, True), (5, 3, 6, 2, 128, 0, True, True),
+                                                                  (33, 1, 32, 8, 128, 100, True, True), (3, 40, 2, 2, 64, 7, True, False),
+                                                                  (4, 2, 4, 2, 256, 9, False, True)])
+def test_rope_append_rows_equals_rotations_and_row_copies(hip, n_tok, n_seq, Hq, Hk, D, pos0, rotate, kv16):
+    """adamah_hip_rope_append_rows_dev (an extension) leaves, bit for bit, the words of map_rope_dev over the Q and K rows of every
+    sequence and map_row_copy_offset_dev of the results; rows have padding between them, and nothing else is written."""
+    rng = np.random.default_rng(n_tok * 100 + n_seq)
+    cap, rows, qs, ks, vs = pos0 + n_tok + 3, n_tok * n_seq, Hq * D + 8, Hk * D + 4, Hk * D + 12
+    q0 = 16
+    k0, v0 = q0 + rows * qs, q0 + rows * (qs + ks)
+    c0 = -(-(v0 + rows * vs) // D) * D
+    per = 2 * Hk * cap * D
+    total = c0 + n_seq * per + 8
+    x = rng.standard_normal(total).astype(np.float32)
+    kb = [c0 + s * per for s in range(n_seq)]
+    vb = [k + Hk * cap * D for k in kb]
+    got = []
+    for one_call in (False, True):
+        note(f"rope append n_tok={n_tok} n_seq={n_seq} one_call={one_call}")
+        f32map(hip, 0, total, x)
+        if kv16:
+            hip.kv_cache_fp16(0, c0, n_seq * per)
+        if one_call:
+            hip.rope_append_rows_dev(0, q0, qs, Hq, k0, ks, Hk, v0, vs, D, n_tok, kb, vb, cap * D, pos0, 1e4, rotate=rotate)
+        else:
+            for s in range(n_seq):
+                r = s * n_tok + np.arange(n_tok)
+                if rotate:
+                    for at, step, H in ((q0, qs, Hq), (k0, ks, Hk)):
+                        h = up(hip, at + r * step)
+                        hip.map_rope_dev(0, h, h, n_tok, H, D, pos0, 1e4)
+            data = read(hip, 0, 0, total)
+            for s in range(n_seq):
+                for t in range(n_tok):
+                    for at, step, cache in ((k0, ks, kb[s]), (v0, vs, vb[s])):
+                        row = data[at + (s * n_tok + t) * step:][:Hk * D].reshape(Hk, D)
+                        row = row.astype(np.float16).astype(np.float32) if kv16 else row
+                        for h in range(Hk):
+                            put(hip, 0, cache + h * cap * D + (pos0 + t) * D, row[h])
+        got.append(read(hip, 0, 0, total))
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    bad = dict(q=q0, qs=qs, k=k0, v=v0, kb=kb, vb=vb, step=cap * D)
+    for change in (dict(v=k0), dict(kb=vb), dict(vb=[total - 8] * n_seq), dict(k=total - Hk * D + 1), dict(qs=D) if rotate and Hq > 1 else dict(kb=[k0] * n_seq)):
+        a = {**bad, **change}
+        with pytest.raises(RuntimeError):
+            hip.rope_append_rows_dev(0, a["q"], a["qs"], Hq, a["k"], ks, Hk, a["v"], vs, D, n_tok, a["kb"], a["vb"], a["step"], pos0, 1e4, rotate=rotate)
+    assert np.array_equal(read(hip, 0, 0, total).view(np.uint32), got[1].view(np.uint32))
