@@ -1304,7 +1304,7 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     const double us = (alone ? 3.0 : 4.7) * (double)up(steps, sp) + (alone ? 11.0 : 17.8) + (double)(sp + 1) * pass;
     const uint64_t two = up(N, 16) > cu ? 2 : 1, rounds = up(up(N, 16 * two), cu);
     const double step = M <= 48 ? (two > 1 ? 0.43 : 0.31) : two > 1 ? 0.53 : 0.40;
-    if (tuning("ADAMAH_GEMM_ROWS", 1) && 4.0 + (double)(rounds * steps) * step < std::min(best, sp > 1 ? us : best)) return {-1, 1};
+    if (4.0 + (double)(rounds * steps) * step < std::min(best, sp > 1 ? us : best)) return {-1, 1};
     return {0, sp > 1 && us < best ? (uint32_t)sp : 1u};
   }
   if (ring == 0 || b < 0 || ((b >> 5) & 1) || M * K * 2 >= (1ull << 32)) {

@@ -41,23 +41,24 @@ k_rmsnorm(const float* act, const float* wt, float* out, const uint32_t* __restr
   }
 }
 
-// The same row op with the row held in registers (dim <= 256 NU): one trip to memory instead of two
-// dependent passes.  Thread t owns elements t, t + 256, ... and sums their squares in that order, as the
-// kernel above does, so the results are the same bits.  EMIT: the rows are [n_rows, dim] back to back and a
-// batched matmul follows; its fp16 operand form (row scaled by a power of two, two planes, 8-element words in the
-// order (0,4)(1,5)(2,6)(3,7), plus (s, 1/s) per row) is written here as well, which spares that
-// matmul its conversion launch.
+// The same row op with the row held in registers: one trip to memory instead of two dependent passes.  Rows of a multiple of
+// eight, at most 8192: a thread owns the eight neighbours of one word (NT >= dim / 8 threads), loads and stores 16 bytes at a time.
+// EMIT: the rows are [n_rows, dim] back to back and a batched matmul follows; its fp16 operand form (row scaled by a power of two,
+// two planes, 8-element words in the order (0,4)(1,5)(2,6)(3,7), plus (s, 1/s) per row) is written here as well, which spares that
+// matmul its conversion launch.  A launch of few rows is one trip to memory, two sums over the workgroup and the stores: with one
+// element a load and 256 threads a row it was 16 pairs of loads and 48 stores a thread (4096 wide, 8 rows 6.2 us, 24 rows 6.3).
 struct RowsByValue { uint32_t on, s0, ss, w0, ws, d0, ds, r0, rs; };   // host side only
-template <bool ADD, bool EMIT, int NU>
-__global__ void __launch_bounds__(256)
+typedef float f4r_t __attribute__((ext_vector_type(4), aligned(4)));
+template <bool ADD, bool EMIT, int NT>
+__global__ void __launch_bounds__(NT)
 k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, uint32_t s0, uint32_t ss_, uint32_t w0, uint32_t ws,
                uint32_t d0, uint32_t ds, uint32_t r0, uint32_t rs, float* out,
                const uint32_t* __restrict__ ls, const uint32_t* __restrict__ lw, const uint32_t* __restrict__ lr,
-               const uint32_t* __restrict__ ld, uint64_t act_elems, uint64_t wt_elems, float* scale, __half* xf, ActForm form) {
+               const uint32_t* __restrict__ ld, uint64_t act_elems, uint64_t wt_elems, float* scale, uint4* xf, ActForm form) {
   // (these 14 dwords are in registers when a wave starts.  Top bit of dim_on: row i's source / weights / destination /
   // residual start at x0 + i xs -- the host found the rows evenly spaced -- instead of four loads from the row
   // tables, which the rows' own loads would have to wait for)
-  __shared__ float sh[4];
+  __shared__ float sums[NT / 64], tops[NT / 64];
   const uint32_t ri = blockIdx.x, tid = threadIdx.x, dim = dim_on & 0x7FFFFFFFu;
   uint64_t sb, wb, db, rb = 0;
   if (dim_on >> 31) {
@@ -67,51 +68,62 @@ k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, ui
     sb = ls[ri]; wb = lw[ri]; db = ld[ri]; if (ADD) rb = lr[ri];
   }
   if (sb + dim > act_elems || db + dim > act_elems || wb + dim > wt_elems || (ADD && rb + dim > act_elems)) return;
-  float x[NU], w[NU], r[NU];
+  const bool in = tid < (dim >> 3);
+  const uint32_t i = in ? tid * 8u : 0u;                     // (a thread past the row loads its first word)
+  const f4r_t x0 = *(const f4r_t*)(act + sb + i), x1 = *(const f4r_t*)(act + sb + i + 4);
+  const f4r_t g0 = *(const f4r_t*)(wt + wb + i), g1 = *(const f4r_t*)(wt + wb + i + 4);
+  f4r_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
+  if (ADD) { a0 = *(const f4r_t*)(act + rb + i); a1 = *(const f4r_t*)(act + rb + i + 4); }
+  float x[8], ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < NU; u++) {
-    const uint32_t i = tid + 256u * u;
-    const bool in = i < dim;
-    x[u] = in ? act[sb + i] : 0.f;
-    w[u] = in ? wt[wb + i] : 0.f;
-    r[u] = (ADD && in) ? act[rb + i] : 0.f;
+  for (int e = 0; e < 8; e++) {
+    x[e] = e < 4 ? x0[e & 3] : x1[e & 3];
+    ss = in ? fmaf(x[e], x[e], ss) : 0.f;
   }
-  float ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < NU; u++)
-    if (tid + 256u * u < dim) ss = fmaf(x[u], x[u], ss);
-  ss = block_sum_256(ss, sh);
+  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  if ((tid & 63u) == 0) sums[tid >> 6] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int w = 0; w < NT / 64; w++) ss += sums[w];
   const float inv = 1.0f / sqrtf(ss / (float)dim + eps);
   float m = 0.f;
 #pragma unroll
-  for (int u = 0; u < NU; u++) {
-    float y = x[u] * inv * w[u];
-    if (ADD) y += r[u];
-    x[u] = y;
-    if (tid + 256u * u < dim) { out[db + tid + 256u * u] = y; m = fmaxf(m, fabsf(y)); }
+  for (int e = 0; e < 8; e++) {
+    x[e] = x[e] * inv * (e < 4 ? g0[e & 3] : g1[e & 3]);
+    if (ADD) x[e] += e < 4 ? a0[e & 3] : a1[e & 3];
+    m = fmaxf(m, fabsf(x[e]));
+  }
+  if (in) {
+    *(f4r_t*)(out + db + i) = (f4r_t){x[0], x[1], x[2], x[3]};
+    *(f4r_t*)(out + db + i + 4) = (f4r_t){x[4], x[5], x[6], x[7]};
   }
   if (!EMIT) return;
+  if (!in) m = 0.f;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((tid & 63u) == 0) sh[tid >> 6] = m;
+  if ((tid & 63u) == 0) tops[tid >> 6] = m;
   __syncthreads();
-  m = fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
+  m = tops[0];
+#pragma unroll
+  for (int w = 1; w < NT / 64; w++) m = fmaxf(m, tops[w]);
   const uint32_t e = (__float_as_uint(m) >> 23) & 0xFFu;
   float s = 1.f, si = 1.f;
   if (e >= 14u && e <= 254u) { s = __uint_as_float((267u - e) << 23); si = __uint_as_float((e - 13u) << 23); }
   if (tid == 0) { scale[2 * ri] = s; scale[2 * ri + 1] = si; }
+  if (!in) return;
   // two planes: fp16(x s) and the fp16 remainder x s - fp16(x s), as the matmul's own conversion writes them
+  uint32_t hi[4], lo[4];
 #pragma unroll
-  for (int u = 0; u < NU; u++) {
-    const uint32_t i = tid + 256u * u, q = i & 7u;
-    if (i < dim) {
-      const uint32_t at = q < 4u ? 2u * q : 2u * (q - 4u) + 1u;
-      const float v = x[u] * s;
-      const __half h = __float2half(v);
-      xf[act_piece(form, 0u, ri, i >> 3, 0u) * 8u + at] = h;
-      xf[act_piece(form, 0u, ri, i >> 3, 1u) * 8u + at] = __float2half(v - __half2float(h));
-    }
+  for (int p = 0; p < 4; p++) {
+    const float u = x[p] * s, v = x[p + 4] * s;
+    const __half uh = __float2half(u), vh = __float2half(v);
+    hi[p] = (uint32_t)__half_as_ushort(uh) | (uint32_t)__half_as_ushort(vh) << 16;
+    lo[p] = (uint32_t)__half_as_ushort(__float2half(u - __half2float(uh))) | (uint32_t)__half_as_ushort(__float2half(v - __half2float(vh))) << 16;
   }
+  xf[act_piece(form, 0u, ri, tid, 0u)] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+  xf[act_piece(form, 0u, ri, tid, 1u)] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
 }
 
 // theta_i = pos * (1 / base^(2i/dim)).  The exponent and the reciprocal are float32 operations as
@@ -269,7 +281,7 @@ static int rmsnorm_impl(uint32_t map_act, uint32_t map_wt, uint32_t hs, uint32_t
   const uint32_t* lr = add ? res_u32(hr, n_rows) : ls;
   if (!ls || !lw || !ld || !lr) return ADAMAH_ERR_INVALID;
   float* a = (float*)ma->buf;
-  if (n_rows > 1 && dim <= 8192 && tuning("ADAMAH_RMSNORM_ROWS", 1) != 0) {
+  if (n_rows > 1 && dim >= 8 && dim <= 8192 && (dim & 7u) == 0 && tuning("ADAMAH_RMSNORM_ROWS", 1) != 0) {
     // rows in registers; when the results are the rows of a matrix [n_rows, dim], also in the form the
     // batched matmul reads
     const uint32_t* dh = res_host(hd, n_rows);
@@ -300,8 +312,8 @@ static int rmsnorm_impl(uint32_t map_act, uint32_t map_wt, uint32_t hs, uint32_t
       }
       if (!even) rv.on = 0u;
     }
-#define RR(A, E, NU) k_rmsnorm_rows<A, E, NU><<<n_rows, 256, 0, g.stream>>>(a, w, dim | (rv.on << 31), eps, rv.s0, rv.ss, rv.w0, rv.ws, rv.d0, rv.ds, rv.r0, rv.rs, a, ls, lw, lr, ld, ma->n_elems, mw->n_elems, scale, (__half*)xf, form)
-#define RN(A, E) do { if (dim <= 2048) RR(A, E, 8); else if (dim <= 4096) RR(A, E, 16); else RR(A, E, 32); } while (0)
+#define RR(A, E, NT) k_rmsnorm_rows<A, E, NT><<<n_rows, NT, 0, g.stream>>>(a, w, dim | (rv.on << 31), eps, rv.s0, rv.ss, rv.w0, rv.ws, rv.d0, rv.ds, rv.r0, rv.rs, a, ls, lw, lr, ld, ma->n_elems, mw->n_elems, scale, xf, form)
+#define RN(A, E) do { if (dim <= 2048) RR(A, E, 256); else if (dim <= 4096) RR(A, E, 512); else RR(A, E, 1024); } while (0)
     if (add) { if (emit) RN(true, true); else RN(true, false); }
     else { if (emit) RN(false, true); else RN(false, false); }
 #undef RN
@@ -401,7 +413,9 @@ size_t launch_wide_rows(const std::vector<PendOp>& q, size_t i, int* rc) {
   auto fold = [&]() -> bool {
     if (i + 2 >= q.size()) return false;
     const PendOp &pq = q[i], &pk = q[i + 1], &pc = q[i + 2];
-    if (pq.kind != PK_ROPE || pk.kind != PK_ROPE || pc.kind != PK_ROWCOPY || pk.op != 1u || pc.op != 1u ||
+    // (the K rows and the copies may be few enough for a row run of their own: 8 sequences of 32 + 8 heads then took three launches
+    // of 5 us)
+    if (pq.kind != PK_ROPE || pk.kind != PK_ROPE || pc.kind != PK_ROWCOPY ||
         pk.map_act != pq.map_act || pc.map_act != pq.map_act || pq.a != pq.c || pk.a != pk.c || pk.n != pq.n || pk.eps != pq.eps ||
         pc.k != pk.k || !m->kv16)
       return false;

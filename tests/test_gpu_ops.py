@@ -475,3 +475,36 @@ def test_rope_append_rows_equals_rotations_and_row_copies(hip, n_tok, n_seq, Hq,
         with pytest.raises(RuntimeError):
             hip.rope_append_rows_dev(0, a["q"], a["qs"], Hq, a["k"], ks, Hk, a["v"], vs, D, n_tok, a["kb"], a["vb"], a["step"], pos0, 1e4, rotate=rotate)
     assert np.array_equal(read(hip, 0, 0, total).view(np.uint32), got[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("B,Hq,Hk,D", [(8, 32, 8, 128), (5, 16, 2, 64), (3, 32, 8, 128)])
+def test_wide_rotation_takes_few_key_rows_and_copies_along(hip, monkeypatch, B, Hq, Hk, D):
+    """One token of B sequences: more than 64 Q rows beside at most 64 K rows and copies still rotate and append in one launch, and
+    leave the words of separate ones (ADAMAH_ROWS_WIDE=0)."""
+    rng = np.random.default_rng(B * Hq)
+    cap, pos = 9, 4
+    q0, k0 = 0, B * Hq * D
+    v0 = k0 + B * Hk * D
+    c0 = v0 + B * Hk * D
+    per = 2 * Hk * cap * D
+    x = rng.standard_normal(c0 + B * per).astype(np.float32)
+    spec = np.empty((B, 2 * Hk, 2), np.uint32)
+    for s in range(B):
+        for h in range(Hk):
+            spec[s, 2 * h] = ((k0 // D) + s * Hk + h, (c0 + s * per) // D + h * cap)
+            spec[s, 2 * h + 1] = ((v0 // D) + s * Hk + h, (c0 + s * per) // D + (Hk + h) * cap)
+    got = []
+    for wide in ("0", "1"):
+        monkeypatch.setenv("ADAMAH_ROWS_WIDE", wide)
+        note(f"wide rotation B={B} wide={wide}")
+        f32map(hip, 0, x.size, x)
+        hip.kv_cache_fp16(0, c0, B * per)
+        hq, hk, hs, hz = up(hip, [q0]), up(hip, [k0]), up(hip, spec.reshape(-1)), up(hip, [0])
+        hip.batch_begin()
+        hip.map_rope_dev(0, hq, hq, 1, B * Hq, D, pos, 1e4)
+        hip.map_rope_dev(0, hk, hk, 1, B * Hk, D, pos, 1e4)
+        hip.map_row_copy_offset_dev(0, hs, hz, pos, 2 * Hk * B, D)
+        hip.batch_end()
+        got.append((read(hip, 0, 0, x.size), hip.get_last_barrier_count()))
+    assert got[1][1] == 1 and got[0][1] > 1
+    assert np.array_equal(got[0][0].view(np.uint32), got[1][0].view(np.uint32))
