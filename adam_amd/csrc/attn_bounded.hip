@@ -11,7 +11,7 @@
 // its place stores them.  More than one span: k_attn_join.
 //
 // A portion of a prompt: k_attn_stage lays the keys the portion sees -- what the cache holds that its first token sees,
-// then the portion's own -- out as matrix operands, K [np, dp] and V transposed [vp, np]; k_attn_keep then brings the
+// then the portion's own -- out as matrix operands; k_attn_keep then brings the
 // cache up to date; k_attn_f32 / _bf16 take 16 queries of a head per wave through the keys they see.
 // Scores arrive as K . Q^T, so a lane holds four keys of one query, which is also the layout the second
 // product wants its right operand in: no shared memory.  float32: the float32 matrix instruction throughout.  bfloat16:
@@ -66,6 +66,8 @@ template <> struct Eight<bf16_t> {
     o[4] = bf_lo(a.z); o[5] = bf_hi(a.z); o[6] = bf_lo(a.w); o[7] = bf_hi(a.w);
   }
 };
+
+template <class T> using Piece = T __attribute__((ext_vector_type(16 / sizeof(T))));
 
 // cap * tanh(a), the cap in powers of two; bfloat16: by one exponential (an error of 1e-7 of the cap)
 template <class T> __device__ __forceinline__ float capped(float a, float cap) {
@@ -277,7 +279,20 @@ k_attn_join(const ASpec s, float* act, const float* __restrict__ part, uint32_t 
 
 // ---- a portion ------------------------------------------------------------------------------------------------------
 struct StageDims { uint32_t past, n, np, dp, vp, place0; };   // keys from the cache, keys in all, padded counts, first key's place
-// One workgroup per 32 staged keys and key head.  K: [kv_heads, np, dp], VT: [kv_heads, vp, np].
+// The staged keys and values in the order in which a wave's lanes take them: a load of an operand is 1 KB in one piece.  (As
+// rows, K [np, dp] and V transposed [vp, np], four neighbouring lanes read four rows, one request to the L1 each: a step of 32
+// keys and 32 queries took 1500 of its clocks a wave, all of a step's 6000 for the four waves of a CU.)
+// A lane holds E values, 16 bytes; lane 16 kg + c.  Keys: blocks of 16, tiles of 4 E dimensions: key c, dimensions E kg ...  Values:
+// blocks of 4 E keys, tiles of 16 dimensions: dimension c, keys 4 kg .. + 3 (bfloat16: and 16 + 4 kg .. + 3).
+template <class T> __device__ __forceinline__ uint64_t key_place(uint32_t j, uint32_t d, uint32_t dp) {
+  constexpr uint32_t E = 16u / sizeof(T);
+  return (uint64_t)(j >> 4) * 16u * dp + ((d / (4u * E)) * 64u + ((d / E) & 3u) * 16u + (j & 15u)) * E + d % E;
+}
+template <class T> __device__ __forceinline__ uint64_t value_place(uint32_t j, uint32_t d, uint32_t vp) {
+  constexpr uint32_t E = 16u / sizeof(T);
+  return (uint64_t)(j / (4u * E)) * 4u * E * vp + ((d >> 4) * 64u + ((j >> 2) & 3u) * 16u + (d & 15u)) * E + (j / 16u * 4u) % E + (j & 3u);
+}
+// One workgroup per 32 staged keys and key head.  A thread makes 16 bytes at a time.
 template <class T, bool WIN>
 __global__ void __launch_bounds__(256)
 k_attn_stage(const ASpec s, const float* __restrict__ act, const T* cache, T* __restrict__ K, T* __restrict__ VT, StageDims sd) {
@@ -297,11 +312,17 @@ k_attn_stage(const ASpec s, const float* __restrict__ act, const T* cache, T* __
     if ((tid & 7u) == 0) inv[tid >> 3] = !WIN || s.qk_norm ? 1.0f / sqrtf(ss / (float)len + s.eps) : 1.0f;
   }
   __syncthreads();
-  for (uint32_t i = tid; i < 32u * sd.dp; i += 256u) {
-    const uint32_t jj = i / sd.dp, d = i - jj * sd.dp, j = j0 + jj;
-    T v = (T)0.f;
-    if (d < D && j < sd.n) v = j < sd.past ? cK[(uint64_t)((sd.place0 + j) % s.size) * D8 + d] : (T)(xk[(uint64_t)(j - sd.past) * s.x_stride + d] * (WIN ? inv[jj] : 1.0f));
-    K[((uint64_t)kv * sd.np + j) * sd.dp + d] = v;
+  constexpr uint32_t E = 16u / sizeof(T);
+  for (uint32_t i = tid; i < 32u * sd.dp / E; i += 256u) {       // [16-key block][tile of dimensions][lane]
+    const uint32_t jj = i / (16u * sd.dp / E) * 16u + (i & 15u), d0 = i % (16u * sd.dp / E) / 16u * E, j = j0 + jj;
+    Piece<T> v;
+#pragma unroll
+    for (uint32_t e = 0; e < E; e++) {
+      const uint32_t d = d0 + e;
+      v[e] = (T)0.f;
+      if (d < D && j < sd.n) v[e] = j < sd.past ? cK[(uint64_t)((sd.place0 + j) % s.size) * D8 + d] : (T)(xk[(uint64_t)(j - sd.past) * s.x_stride + d] * (WIN ? inv[jj] : 1.0f));
+    }
+    *(Piece<T>*)(K + (uint64_t)kv * sd.np * sd.dp + key_place<T>(j, d0, sd.dp)) = v;
   }
   for (uint32_t i = tid; i < 32u * V; i += 256u) {
     const uint32_t jj = i / V, d = i - jj * V, j = j0 + jj;
@@ -310,9 +331,12 @@ k_attn_stage(const ASpec s, const float* __restrict__ act, const T* cache, T* __
     vt[jj * (V + 1u) + d] = v;
   }
   __syncthreads();
-  for (uint32_t i = tid; i < 32u * sd.vp; i += 256u) {
-    const uint32_t d = i >> 5, jj = i & 31u;
-    VT[((uint64_t)kv * sd.vp + d) * sd.np + j0 + jj] = (T)(d < V ? vt[jj * (V + 1u) + d] : 0.f);
+  for (uint32_t i = tid; i < 32u * sd.vp / E; i += 256u) {       // [block of 4 E keys][tile of dimensions][lane]
+    const uint32_t b = i / (4u * sd.vp), d = i % (4u * sd.vp) / 64u * 16u + (i & 15u), jj = b * 4u * E + (i >> 4 & 3u) * 4u;
+    Piece<T> v;
+#pragma unroll
+    for (uint32_t e = 0; e < E; e++) v[e] = (T)(d < V ? vt[(jj + e / 4u * 16u + (e & 3u)) * (V + 1u) + d] : 0.f);
+    *(Piece<T>*)(VT + (uint64_t)kv * sd.vp * sd.np + value_place<T>(j0 + jj, d, sd.vp)) = v;
   }
 }
 // The cache after the portion: the tokens a later one may see.  A launch of its own, behind the staging that
@@ -324,31 +348,41 @@ k_attn_keep(const ASpec s, T* cache, const T* __restrict__ K, const T* __restric
   const uint32_t place = (sd.place0 + j) % s.size;
   T* cK = cache + s.k_off + ((uint64_t)kv * s.size + place) * D8;
   T* cV = cache + s.v_off + ((uint64_t)kv * s.size + place) * V8;
-  for (uint32_t d = threadIdx.x; d < D8; d += 256u) cK[d] = K[((uint64_t)kv * sd.np + j) * sd.dp + d];
-  for (uint32_t d = threadIdx.x; d < V8; d += 256u) cV[d] = VT[((uint64_t)kv * sd.vp + d) * sd.np + j];
+  for (uint32_t d = threadIdx.x; d < D8; d += 256u) cK[d] = K[(uint64_t)kv * sd.np * sd.dp + key_place<T>(j, d, sd.dp)];
+  for (uint32_t d = threadIdx.x; d < V8; d += 256u) cV[d] = VT[(uint64_t)kv * sd.vp * sd.np + value_place<T>(j, d, sd.vp)];
 }
 
+// The largest of a value over the four key groups (lanes l, l ^ 16, l ^ 32, l ^ 48)
+__device__ __forceinline__ float groups_max(float t) {
+  typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
+  const uint32_t b = __float_as_uint(t);
+  const u2_t x = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  const uint32_t m = __float_as_uint(fmaxf(__uint_as_float(x.x), __uint_as_float(x.y)));
+  const u2_t y = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+  return fmaxf(__uint_as_float(y.x), __uint_as_float(y.y));
+}
 // First staged key that the query at position p sees; base: position of the first staged key.
 template <bool WIN> __device__ __forceinline__ uint32_t first_seen(const ASpec& s, uint32_t p, uint32_t base) {
   return (WIN ? (p >= s.size ? p + 1u - s.size : 0u) : p / s.size * s.size) - base;
 }
-// 16 queries of a head per wave.  float32 form: keys 16 at a time.  Few waves walk a serial chain, so a step's latency
+// 16 queries of a head per wave; KW: waves that part the keys of the same queries, whose sums meet in LDS at the end.  float32
+// form: keys 16 at a time.  Few waves walk a serial chain, so a step's latency
 // counts: queries in registers, keys a step ahead, values asked for at the step's head (read where they were needed, under
 // conditions: 303 us for 512 queries in 16 heads of 128, so: 101).  No loop over q, kk, vv or o ends early: the compiler then
 // leaves it rolled and puts the arrays in memory (512 queries behind 1500 keys, 16 heads of 192 with 256 values: 2470 us,
 // with loads where they were needed 1729, so: 549).
-template <bool WIN, int NV, int DK>
+template <bool WIN, int NV, int DK, int KW>
 __global__ void __launch_bounds__(256)
 k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos) {
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kg = lane >> 4, h = blockIdx.x, kv = h / (s.heads / s.kv_heads);
-  const uint32_t q0 = (blockIdx.y * 4u + (threadIdx.x >> 6)) * 16u;
+  const uint32_t wave = threadIdx.x >> 6, part = wave % KW, q0 = (blockIdx.y * (4u / KW) + wave / KW) * 16u;
   if (q0 >= m) return;
   const uint32_t qr = min(q0 + c, m - 1u), base = pos - sd.past;           // key j of the stage sits at position base + j
   const uint32_t qj = sd.past + qr, lo = first_seen<WIN>(s, pos + qr, base);   // visible: lo .. qj
-  const uint32_t first = first_seen<WIN>(s, pos + q0, base) & ~15u, end = sd.past + min(q0 + 16u, m);
+  const uint32_t end = sd.past + min(q0 + 16u, m), from = (first_seen<WIN>(s, pos + q0, base) & ~15u) + 16u * part, first = min(from, (end - 1u) & ~15u);
   const float* xq = act + s.x + (uint64_t)qr * s.x_stride + s.x_q + h * s.dim;
-  const float* kb = K + (uint64_t)kv * sd.np * sd.dp;
-  const float* vb = VT + (uint64_t)kv * sd.vp * sd.np;
+  const float* kb = K + (uint64_t)kv * sd.np * sd.dp + 4u * lane;
+  const float* vb = VT + (uint64_t)kv * sd.vp * sd.np + 4u * lane;
   const float r1 = act[s.p1 + h], r2 = act[s.p2 + h];
   f4_t o[NV], q[DK], kk[DK], vv[NV];
 #pragma unroll
@@ -359,7 +393,7 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
     for (int i = 0; i < 4; i++) q[t][i] = xq[min(16u * t + 4u * kg + i, s.dim - 1u)];
   const auto keys = [&](uint32_t j0) {
 #pragma unroll
-    for (int t = 0; t < DK; t++) kk[t] = *(const f4_t*)(kb + (uint64_t)(j0 + c) * sd.dp + min(16u * t, sd.dp - 16u) + 4u * kg);
+    for (int t = 0; t < DK; t++) kk[t] = *(const f4_t*)(kb + (uint64_t)j0 * sd.dp + min(16u * t, sd.dp - 16u) * 16u);
   };
   keys(first);
 #pragma unroll
@@ -368,7 +402,7 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
     for (int i = 0; i < 4; i++) q[t][i] = 16u * t + 4u * kg + i < s.dim ? q[t][i] : 0.f;
   float mx = ATT_MASKED, sum = 0.f, qs = s.scale;
   if (WIN) {
-    if (s.has_sink) { mx = r2; sum = 1.f; }
+    if (s.has_sink && part == 0u) { mx = r2; sum = 1.f; }
     if (s.qk_norm) {
       float a = 0.f;
 #pragma unroll
@@ -380,31 +414,32 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
     }
     qs *= query_temperature(s, pos + qr);
   }
-  for (uint32_t j0 = first; j0 < end; j0 += 16u) {
+  for (uint32_t j0 = from; j0 < end; j0 += 16u * KW) {
     // everything a step reads is asked for at its head (its keys a step ahead), on every path
 #pragma unroll
-    for (int v = 0; v < NV; v++) vv[v] = *(const f4_t*)(vb + (uint64_t)(min(v * 16u, sd.vp - 16u) + c) * sd.np + j0 + 4u * kg);
+    for (int v = 0; v < NV; v++) vv[v] = *(const f4_t*)(vb + (uint64_t)j0 * sd.vp + min(v * 16u, sd.vp - 16u) * 16u);
     f4_t a = {0, 0, 0, 0};
 #pragma unroll
     for (int t = 0; t < DK; t++)
       if (16u * t < sd.dp)
 #pragma unroll
         for (int i = 0; i < 4; i++) a = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[t][i], q[t][i], a, 0, 0, 0);
-    keys(j0 + 16u < end ? j0 + 16u : j0);
+    keys(j0 + 16u * KW < end ? j0 + 16u * KW : j0);
     float t = ATT_MASKED;
+    a *= WIN ? qs : s.scale;
+    if (WIN && s.softcap > 0.f) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < 4; i++) a[i] = s.softcap * tanhf(a[i] / s.softcap);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {                            // (no branch for a score: the keys it does not see are masked behind)
       const uint32_t j = j0 + 4u * kg + i;
-      const bool ok = j >= lo && j <= qj;
-      if (WIN) {
-        float z = a[i] * qs;
-        if (s.softcap > 0.f) z = s.softcap * tanhf(z / s.softcap);
-        a[i] = ok ? z - r1 * (float)(qj - j) : ATT_MASKED;
-      } else
-        a[i] = ok ? a[i] * s.scale - r1 * log1pf(r2 * (float)(qj - j)) : ATT_MASKED;
+      const float away = (float)(int32_t)(qj - j);
+      const float z = a[i] - r1 * (WIN ? away : log1pf(r2 * fmaxf(away, 0.f)));
+      a[i] = (j >= lo) & (j <= qj) ? z : ATT_MASKED;
       t = fmaxf(t, a[i]);
     }
-    t = fmaxf(t, __shfl_xor(t, 16, 64)); t = fmaxf(t, __shfl_xor(t, 32, 64));
+    t = groups_max(t);
     const float nm = fmaxf(mx, t), al = expf(mx - nm);
     mx = nm;
     float ps = 0.f;
@@ -420,8 +455,34 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
         for (int i = 0; i < 4; i++) o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[v][i], a[i], o[v], 0, 0, 0);
       }
   }
-  if (q0 + c >= m) return;
   float* out = act + s.out + (uint64_t)qr * s.out_stride + h * s.vdim;
+  if constexpr (KW > 1) {                                    // the waves' parts of the keys, brought to their common maximum
+    __shared__ float os[KW][NV][4][64], ms[KW][2][16];
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) os[part][v][i][lane] = o[v][i];
+    if (kg == 0u) { ms[part][0][c] = mx; ms[part][1][c] = sum; }
+    __syncthreads();
+    float top = ms[0][0][c], e[KW];
+#pragma unroll
+    for (int w = 1; w < KW; w++) top = fmaxf(top, ms[w][0][c]);
+    sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < KW; w++) { e[w] = expf(ms[w][0][c] - top); sum = fmaf(ms[w][1][c], e[w], sum); }
+    if (q0 + c >= m) return;
+    for (uint32_t v = part; v < NV; v += KW)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const uint32_t d = v * 16u + 4u * kg + i;
+        float a = 0.f;
+#pragma unroll
+        for (int w = 0; w < KW; w++) a = fmaf(os[w][v][i][lane], e[w], a);
+        if (d < s.vdim) out[d] = a / sum;
+      }
+    return;
+  }
+  if (q0 + c >= m) return;
 #pragma unroll
   for (int v = 0; v < NV; v++)
 #pragma unroll
@@ -433,7 +494,10 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
 
 // bfloat16 form: QT tiles of 16 queries a wave, keys 32 at a time (two tiles of 16); DK: k-steps of 32 dimensions.  Scores
 // and the penalty are kept in powers of two.  A step's values and the next step's keys are in flight under the products.
-template <bool WIN, int DK, int NV, int QT>
+// What bounds it is issue (350 vector instructions a step, 50 of them exponentials and reciprocals, beside 64 matrix instructions),
+// and, with one wave a SIMD, their latency.  2048 queries in 16 heads of 128, window form: 209 us; operands in one piece 183; no
+// branch for a score, products that are rescaled only behind a new maximum 110.  Chunk form, 32 heads, 1953 behind 2048: 444, 284, 204.
+template <bool WIN, int DK, int NV, int QT, int KW>
 __global__ void __launch_bounds__(256, DK * QT <= 8 && NV * QT <= 16 ? 2 : 1)
 k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_t* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos) {
   // workgroups land on the eight dies in turn: the query heads of a key head share one; late query tiles, which see more
@@ -441,13 +505,13 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
   const uint32_t nx = gridDim.x, h = (nx & 7u) == 0u ? (blockIdx.x & 7u) * (nx >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const uint32_t ny = gridDim.y, by = blockIdx.y < (ny >> 1) ? blockIdx.y : ny - 1u - (blockIdx.y - (ny >> 1));
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kg = lane >> 4, kv = h / (s.heads / s.kv_heads);
-  const uint32_t q0 = (by * 4u + (threadIdx.x >> 6)) * 16u * QT;
+  const uint32_t wave = threadIdx.x >> 6, part = wave % KW, q0 = (by * (4u / KW) + wave / KW) * 16u * QT;
   if (q0 >= m) return;
   const uint32_t base = pos - sd.past, qlast = min(q0 + 16u * QT, m) - 1u;
-  const uint32_t first = first_seen<WIN>(s, pos + q0, base) & ~31u, end = sd.past + qlast + 1u;
+  const uint32_t end = sd.past + qlast + 1u, from = (first_seen<WIN>(s, pos + q0, base) & ~31u) + 32u * part;
   const uint32_t lo_all = first_seen<WIN>(s, pos + qlast, base);           // seen by every query from here to past + q0
-  const bf16_t* kb = K + (uint64_t)kv * sd.np * sd.dp + (uint64_t)c * sd.dp + 8u * kg;
-  const bf16_t* vb = VT + (uint64_t)kv * sd.vp * sd.np + (uint64_t)c * sd.np + 4u * kg;
+  const bf16_t* kb = K + (uint64_t)kv * sd.np * sd.dp + 8u * lane;
+  const bf16_t* vb = VT + (uint64_t)kv * sd.vp * sd.np + 8u * lane;
   const float r1 = act[s.p1 + h] * (WIN ? LOG2E : 1.0f), r2 = act[s.p2 + h] * (WIN ? LOG2E : 1.0f);
   const float cap = WIN ? s.softcap * LOG2E : 0.f;
   uint32_t qr[QT], qj[QT], lo[QT];
@@ -483,7 +547,7 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
   float mx[QT], sum[QT];
 #pragma unroll
   for (int g = 0; g < QT; g++) {
-    mx[g] = WIN && s.has_sink ? r2 : ATT_MASKED; sum[g] = WIN && s.has_sink && kg == 0u ? 1.f : 0.f;
+    mx[g] = WIN && s.has_sink && part == 0u ? r2 : ATT_MASKED; sum[g] = WIN && s.has_sink && part == 0u && kg == 0u ? 1.f : 0.f;
 #pragma unroll
     for (int i = 0; i < NV; i++) o[g][i] = (f4_t){0, 0, 0, 0};
   }
@@ -492,16 +556,13 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
-      for (int t = 0; t < DK; t++) kf[u][t] = *(const bf8_t*)(kb + (uint64_t)(j0 + 16u * u) * sd.dp + 32u * t);
+      for (int t = 0; t < DK; t++) kf[u][t] = *(const bf8_t*)(kb + (uint64_t)(j0 + 16u * u) * sd.dp + 512u * t);
   };
-  keys(first);
-  for (uint32_t j0 = first; j0 < end; j0 += 32u) {
-    bf4_t vf[NV][2];
+  keys(min(from, (end - 1u) & ~31u));
+  for (uint32_t j0 = from; j0 < end; j0 += 32u * KW) {
+    bf8_t vf[NV];
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      vf[v][0] = *(const bf4_t*)(vb + (uint64_t)v * 16u * sd.np + j0);
-      vf[v][1] = *(const bf4_t*)(vb + (uint64_t)v * 16u * sd.np + j0 + 16u);
-    }
+    for (int v = 0; v < NV; v++) vf[v] = *(const bf8_t*)(vb + (uint64_t)j0 * sd.vp + 512u * v);
     f4_t a[QT][2];
 #pragma unroll
     for (int g = 0; g < QT; g++)
@@ -514,45 +575,116 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
           a[g][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[u][t], qh[g][t], a[g][u], 0, 0, 0);
         }
       }
-    if (j0 + 32u < end) keys(j0 + 32u);
-    const bool all = j0 >= lo_all && j0 + 31u <= sd.past + q0;
+    if (j0 + 32u * KW < end) keys(j0 + 32u * KW);
+    // No condition inside the loops over scores (a branch for each kept the exponentials from overlapping): the cap's and the
+    // mask's are around them
+    if (WIN && cap > 0.f) {
+#pragma unroll
+      for (int g = 0; g < QT; g++)
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) a[g][u][i] = fmaf(-2.0f * cap, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a[g][u][i]) + 1.0f), cap);
+    }
 #pragma unroll
     for (int g = 0; g < QT; g++) {
       const float dist = (float)(int32_t)(qj[g] - j0 - 4u * kg);
-      float t = ATT_MASKED;
 #pragma unroll
       for (int u = 0; u < 2; u++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const float away = dist - (float)(16 * u + i), pen = r1 * (WIN ? away : __builtin_amdgcn_logf(fmaf(r2, away, 1.0f)));
-          if (WIN && cap > 0.f) a[g][u][i] = fmaf(-2.0f * cap, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a[g][u][i]) + 1.0f), cap);
-          const uint32_t j = j0 + 16u * u + 4u * kg + i;
-          a[g][u][i] = all || (j >= lo[g] && j <= qj[g]) ? a[g][u][i] - pen : ATT_MASKED;
-          t = fmaxf(t, a[g][u][i]);
+          const float away = dist - (float)(16 * u + i);
+          a[g][u][i] -= r1 * (WIN ? away : __builtin_amdgcn_logf(fmaf(r2, away, 1.0f)));
         }
-      t = fmaxf(t, __shfl_xor(t, 16, 64)); t = fmaxf(t, __shfl_xor(t, 32, 64));
-      const float nm = fmaxf(mx[g], t), al = __builtin_amdgcn_exp2f(mx[g] - nm);
-      mx[g] = nm;
-      float ps = 0.f;
-      bf8_t ph, pl;
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float p = all || a[g][u][i] > 0.5f * ATT_MASKED ? __builtin_amdgcn_exp2f(a[g][u][i] - nm) : 0.f;
-          ps += p;
-          ph[4 * u + i] = (bf16_t)p;
-          pl[4 * u + i] = (bf16_t)(p - (float)ph[4 * u + i]);
-        }
-      sum[g] = fmaf(sum[g], al, ps);                       // per lane: the four key groups are added up at the end
-#pragma unroll
-      for (int v = 0; v < NV; v++) {
-        const bf8_t vv = {vf[v][0][0], vf[v][0][1], vf[v][0][2], vf[v][0][3], vf[v][1][0], vf[v][1][1], vf[v][1][2], vf[v][1][3]};
-        o[g][v] *= al;
-        o[g][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, pl, o[g][v], 0, 0, 0);
-        o[g][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, ph, o[g][v], 0, 0, 0);
-      }
     }
+    const bool all = j0 >= lo_all && j0 + 31u <= sd.past + q0;               // seen by every query of the wave
+    if (!all) {
+#pragma unroll
+      for (int g = 0; g < QT; g++)
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const uint32_t j = j0 + 16u * u + 4u * kg + i;
+            a[g][u][i] = (j >= lo[g]) & (j <= qj[g]) ? a[g][u][i] : ATT_MASKED;
+          }
+    }
+    float al[QT];
+    bool same = true;
+#pragma unroll
+    for (int g = 0; g < QT; g++) {
+      float t = fmaxf(fmaxf(fmaxf(a[g][0][0], a[g][0][1]), fmaxf(a[g][0][2], a[g][0][3])), fmaxf(fmaxf(a[g][1][0], a[g][1][1]), fmaxf(a[g][1][2], a[g][1][3])));
+      t = groups_max(t);
+      const float nm = fmaxf(mx[g], t);
+      al[g] = __builtin_amdgcn_exp2f(mx[g] - nm);
+      same = same & (nm == mx[g]);
+      mx[g] = nm;
+    }
+    bf8_t ph[QT], pl[QT];
+#pragma unroll
+    for (int g = 0; g < QT; g++) {
+      // (a query that has seen no key yet has the maximum of the masked: its weights have to be zeros, not exp2(0))
+      const float zero = mx[g] > 0.5f * ATT_MASKED ? mx[g] : 0.f;
+      float ps = 0.f;
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float p = __builtin_amdgcn_exp2f(a[g][u][i] - zero);
+          ps += p;
+          ph[g][4 * u + i] = (bf16_t)p;
+          pl[g][4 * u + i] = (bf16_t)(p - (float)ph[g][4 * u + i]);
+        }
+      sum[g] = fmaf(sum[g], al[g], ps);                    // per lane: the four key groups are added up at the end
+    }
+    if (__builtin_amdgcn_ballot_w64(!same)) {              // the maxima of most steps are old ones
+#pragma unroll
+      for (int g = 0; g < QT; g++)
+#pragma unroll
+        for (int v = 0; v < NV; v++) o[g][v] *= al[g];
+    }
+#pragma unroll
+    for (int g = 0; g < QT; g++)
+#pragma unroll
+      for (int v = 0; v < NV; v++) o[g][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v], pl[g], o[g][v], 0, 0, 0);
+#pragma unroll
+    for (int g = 0; g < QT; g++)
+#pragma unroll
+      for (int v = 0; v < NV; v++) o[g][v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v], ph[g], o[g][v], 0, 0, 0);
+  }
+  if constexpr (KW > 1) {                                    // the waves' parts of the keys, brought to their common maximum
+    __shared__ float os[KW][QT][NV][4][64], ms[KW][QT][2][16];
+#pragma unroll
+    for (int g = 0; g < QT; g++) {
+      sum[g] += __shfl_xor(sum[g], 16, 64); sum[g] += __shfl_xor(sum[g], 32, 64);
+#pragma unroll
+      for (int v = 0; v < NV; v++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) os[part][g][v][i][lane] = o[g][v][i];
+      if (kg == 0u) { ms[part][g][0][c] = mx[g]; ms[part][g][1][c] = sum[g]; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < QT; g++) {
+      float top = ms[0][g][0][c], e[KW], all_sum = 0.f;
+#pragma unroll
+      for (int w = 1; w < KW; w++) top = fmaxf(top, ms[w][g][0][c]);
+#pragma unroll
+      for (int w = 0; w < KW; w++) { e[w] = __builtin_amdgcn_exp2f(ms[w][g][0][c] - top); all_sum = fmaf(ms[w][g][1][c], e[w], all_sum); }
+      if (q0 + 16u * g + c >= m) continue;
+      const float inv = 1.0f / all_sum;
+      float* out = act + s.out + (uint64_t)qr[g] * s.out_stride + h * s.vdim;
+      for (uint32_t v = part; v < NV; v += KW)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const uint32_t d = v * 16u + 4u * kg + i;
+          float a = 0.f;
+#pragma unroll
+          for (int w = 0; w < KW; w++) a = fmaf(os[w][g][v][i][lane], e[w], a);
+          if (d < s.vdim) out[d] = a * inv;
+        }
+    }
+    return;
   }
 #pragma unroll
   for (int g = 0; g < QT; g++) {
@@ -573,13 +705,23 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
 static Scratch g_stage, g_parts;
 void attn_bounded_release() { scratch_free(g_stage); scratch_free(g_parts); }
 
+// Whether the four waves of a workgroup share their queries and part the keys, instead of taking queries each: where workgroups of
+// queries would not give every CU one, and a wave has keys enough to pay for the sum through LDS.  952 queries behind 2048 keys, 16
+// heads: 151 -> 98 us; float32, 512 queries in 16 heads: 88 -> 39, 88 behind 512 keys: 98 -> 33.  (With one for every CU the waves
+// of a workgroup are better off reading the same keys: 2048 queries in 16 heads 110 us, so: 116; in 32 heads 193 and 200.)
+static bool shared_keys(const ASpec& s, const StageDims& sd, uint32_t wgs_y) {
+  return (uint64_t)s.heads * wgs_y < (uint64_t)g.n_cu && sd.n >= 256u;
+}
 template <bool WIN, int DK>
 static void launch_bf16(const ASpec& s, float* act, const bf16_t* K, const bf16_t* VT, const StageDims& sd, uint32_t m, uint32_t pos) {
   switch (sd.vp / 16u) {
 #define CASE(N)                                                                                                     \
   case N: {                                                                                                         \
     constexpr int QT = DK <= 4 && N <= 8 ? 2 : 1;                                                                   \
-    k_attn_bf16<WIN, DK, N, QT><<<dim3(s.heads, cdiv(m, 64 * QT)), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos); \
+    if (shared_keys(s, sd, cdiv(m, 64 * QT)))                                                                       \
+      k_attn_bf16<WIN, DK, N, QT, 4><<<dim3(s.heads, cdiv(m, 16 * QT)), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos); \
+    else                                                                                                            \
+      k_attn_bf16<WIN, DK, N, QT, 1><<<dim3(s.heads, cdiv(m, 64 * QT)), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos); \
   } break
     CASE(2); CASE(4); CASE(6); CASE(8); CASE(12); CASE(16);
 #undef CASE
@@ -611,8 +753,13 @@ static int run_portion(const ASpec& s, float* act, T* cache, uint32_t m, uint32_
   count_launch();
   if (int r = check_launch()) return r;
   if constexpr (sizeof(T) == 4) {
-    const dim3 grid(s.heads, cdiv(m, 64));
-#define AF(NV, DK) k_attn_f32<WIN, NV, DK><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos)
+    const bool apart = shared_keys(s, sd, cdiv(m, 64));
+    const dim3 grid(s.heads, cdiv(m, apart ? 16 : 64));
+#define AF(NV, DK)                                                                                                  \
+  do {                                                                                                              \
+    if (apart) k_attn_f32<WIN, NV, DK, 4><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos);                   \
+    else k_attn_f32<WIN, NV, DK, 1><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos);                         \
+  } while (0)
     if (sd.dp <= 128u) { if (sd.vp <= 64u) AF(4, 8); else if (sd.vp <= 128u) AF(8, 8); else AF(16, 8); }
     else { if (sd.vp <= 64u) AF(4, 16); else if (sd.vp <= 128u) AF(8, 16); else AF(16, 16); }
 #undef AF

@@ -710,3 +710,16 @@ def test_calls_with_impossible_operands_are_refused(hip):
     for bad in (dict(dim=300), dict(rot_dims=9), dict(seq_stride=63), dict(x_v=30), dict(state_map=9)):
         with pytest.raises(RuntimeError, match="-3"):
             hip.retention_dev(0, up(A.RetentionSpec(**{**r, **bad})), 1, 1, 0, 0)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,G,D,V,C,ms", [(64, 8, 40, 24, 900, (520, 260, 31, 200)), (6, 2, 128, 128, 290, (250, 33, 300)), (3, 1, 200, 72, 700, (300, 300))])
+def test_chunk_attention_with_the_keys_parted_among_waves(hip, H, G, D, V, C, ms, dtype):
+    """Portions that give every compute unit a workgroup of queries and ones that do not (the waves of a workgroup part the keys, some of
+    them with none), across a chunk's edge as well."""
+    note(f"chunk attention, keys parted, H {H} D {D} chunk {C} {dtype}")
+    run, _, _ = attention_pair(hip, H, G, D, V, C, dtype, 520, 1, seed=C)
+    pos = 0
+    for m in ms:
+        run(1, m, 0, pos)
+        pos += m

@@ -538,3 +538,16 @@ def test_calls_with_impossible_operands_are_refused(hip):
     for bad in (dict(branched=3), dict(branched=2, res_out=k - 1), dict(groups=2), dict(tail=3), dict(branch=(1 << 32) - 2), dict(kept=1, keep=(1 << 32) - 2)):
         with pytest.raises(RuntimeError, match="-3"):
             hip.linear_dev(0, 2, mid, up(A.LinearSpec(**{**good, **bad})), 0, 1)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,G,D,V,R,ms", [(64, 8, 40, 24, 900, (520, 260, 31, 2)), (6, 2, 128, 128, 290, (250, 33, 300, 17)), (3, 1, 200, 72, 260, (300, 300))])
+def test_window_attention_with_the_keys_parted_among_waves(hip, H, G, D, V, R, ms, dtype):
+    """Portions that give every compute unit a workgroup of queries and ones that do not: there the waves of a workgroup part the keys,
+    some of them with none, a window's edge inside the first wave's, and the sink counted once."""
+    note(f"window attention, keys parted, H {H} D {D} window {R} {dtype}")
+    run, _, _ = window_pair(hip, H, G, D, V, R, dtype, 520, 1, seed=R, scale=0.6)
+    pos = 0
+    for m in ms:
+        run(1, m, 0, pos)
+        pos += m
