@@ -279,6 +279,9 @@ k_attn_join(const ASpec s, float* act, const float* __restrict__ part, uint32_t 
 
 // ---- a portion ------------------------------------------------------------------------------------------------------
 struct StageDims { uint32_t past, n, np, dp, vp, place0; };   // keys from the cache, keys in all, padded counts, first key's place
+// One after the other in the grid's third dimension, the portions of several sequences of one length: elements from one's rows,
+// outputs, cache, staged keys and values to the next one's.
+struct SeqSteps { uint64_t x, out, cache, k, v; };
 // The staged keys and values in the order in which a wave's lanes take them: a load of an operand is 1 KB in one piece.  (As
 // rows, K [np, dp] and V transposed [vp, np], four neighbouring lanes read four rows, one request to the L1 each: a step of 32
 // keys and 32 queries took 1500 of its clocks a wave, all of a step's 6000 for the four waves of a CU.)
@@ -295,9 +298,10 @@ template <class T> __device__ __forceinline__ uint64_t value_place(uint32_t j, u
 // One workgroup per 32 staged keys and key head.  A thread makes 16 bytes at a time.
 template <class T, bool WIN>
 __global__ void __launch_bounds__(256)
-k_attn_stage(const ASpec s, const float* __restrict__ act, const T* cache, T* __restrict__ K, T* __restrict__ VT, StageDims sd) {
+k_attn_stage(const ASpec s, const float* __restrict__ act, const T* cache, T* __restrict__ K, T* __restrict__ VT, StageDims sd, SeqSteps by) {
   extern __shared__ float vt[];                    // [32][V + 1]
   __shared__ float inv[32];
+  act += blockIdx.z * by.x; cache += blockIdx.z * by.cache; K += blockIdx.z * by.k; VT += blockIdx.z * by.v;
   const uint32_t D = s.dim, V = s.vdim, D8 = (D + 7u) & ~7u, V8 = (V + 7u) & ~7u, tid = threadIdx.x, kv = blockIdx.y, j0 = blockIdx.x * 32u;
   const T* cK = cache + s.k_off + (uint64_t)kv * s.size * D8;
   const T* cV = cache + s.v_off + (uint64_t)kv * s.size * V8;
@@ -343,7 +347,8 @@ k_attn_stage(const ASpec s, const float* __restrict__ act, const T* cache, T* __
 // still reads the places it writes.
 template <class T>
 __global__ void __launch_bounds__(256)
-k_attn_keep(const ASpec s, T* cache, const T* __restrict__ K, const T* __restrict__ VT, StageDims sd, uint32_t first) {
+k_attn_keep(const ASpec s, T* cache, const T* __restrict__ K, const T* __restrict__ VT, StageDims sd, uint32_t first, SeqSteps by) {
+  cache += blockIdx.z * by.cache; K += blockIdx.z * by.k; VT += blockIdx.z * by.v;
   const uint32_t D8 = (s.dim + 7u) & ~7u, V8 = (s.vdim + 7u) & ~7u, kv = blockIdx.y, j = first + blockIdx.x;
   const uint32_t place = (sd.place0 + j) % s.size;
   T* cK = cache + s.k_off + ((uint64_t)kv * s.size + place) * D8;
@@ -373,14 +378,17 @@ template <bool WIN> __device__ __forceinline__ uint32_t first_seen(const ASpec& 
 // with loads where they were needed 1729, so: 549).
 template <bool WIN, int NV, int DK, int KW>
 __global__ void __launch_bounds__(256)
-k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos) {
+k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos, SeqSteps by) {
+  const float* const rows = act + blockIdx.z * by.x + s.x;
+  float* const outs = act + blockIdx.z * by.out + s.out;
+  K += blockIdx.z * by.k; VT += blockIdx.z * by.v;
   const uint32_t lane = threadIdx.x & 63u, c = lane & 15u, kg = lane >> 4, h = blockIdx.x, kv = h / (s.heads / s.kv_heads);
   const uint32_t wave = threadIdx.x >> 6, part = wave % KW, q0 = (blockIdx.y * (4u / KW) + wave / KW) * 16u;
   if (q0 >= m) return;
   const uint32_t qr = min(q0 + c, m - 1u), base = pos - sd.past;           // key j of the stage sits at position base + j
   const uint32_t qj = sd.past + qr, lo = first_seen<WIN>(s, pos + qr, base);   // visible: lo .. qj
   const uint32_t end = sd.past + min(q0 + 16u, m), from = (first_seen<WIN>(s, pos + q0, base) & ~15u) + 16u * part, first = min(from, (end - 1u) & ~15u);
-  const float* xq = act + s.x + (uint64_t)qr * s.x_stride + s.x_q + h * s.dim;
+  const float* xq = rows + (uint64_t)qr * s.x_stride + s.x_q + h * s.dim;
   const float* kb = K + (uint64_t)kv * sd.np * sd.dp + 4u * lane;
   const float* vb = VT + (uint64_t)kv * sd.vp * sd.np + 4u * lane;
   const float r1 = act[s.p1 + h], r2 = act[s.p2 + h];
@@ -455,7 +463,7 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
         for (int i = 0; i < 4; i++) o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[v][i], a[i], o[v], 0, 0, 0);
       }
   }
-  float* out = act + s.out + (uint64_t)qr * s.out_stride + h * s.vdim;
+  float* out = outs + (uint64_t)qr * s.out_stride + h * s.vdim;
   if constexpr (KW > 1) {                                    // the waves' parts of the keys, brought to their common maximum
     __shared__ float os[KW][NV][4][64], ms[KW][2][16];
 #pragma unroll
@@ -499,7 +507,10 @@ k_attn_f32(const ASpec s, float* act, const float* __restrict__ K, const float* 
 // branch for a score, products that are rescaled only behind a new maximum 110.  Chunk form, 32 heads, 1953 behind 2048: 444, 284, 204.
 template <bool WIN, int DK, int NV, int QT, int KW>
 __global__ void __launch_bounds__(256, DK * QT <= 8 && NV * QT <= 16 ? 2 : 1)
-k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_t* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos) {
+k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_t* __restrict__ VT, StageDims sd, uint32_t m, uint32_t pos, SeqSteps sq) {
+  const float* const rows = act + blockIdx.z * sq.x + s.x;
+  float* const outs = act + blockIdx.z * sq.out + s.out;
+  K += blockIdx.z * sq.k; VT += blockIdx.z * sq.v;
   // workgroups land on the eight dies in turn: the query heads of a key head share one; late query tiles, which see more
   // keys, go with early ones
   const uint32_t nx = gridDim.x, h = (nx & 7u) == 0u ? (blockIdx.x & 7u) * (nx >> 3) + (blockIdx.x >> 3) : blockIdx.x;
@@ -521,7 +532,7 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
     qr[g] = min(q0 + 16u * g + c, m - 1u);
     qj[g] = sd.past + qr[g];
     lo[g] = first_seen<WIN>(s, pos + qr[g], base);
-    const float* xq = act + s.x + (uint64_t)qr[g] * s.x_stride + s.x_q + h * s.dim;
+    const float* xq = rows + (uint64_t)qr[g] * s.x_stride + s.x_q + h * s.dim;
     float qs = s.scale * LOG2E;
     if (WIN) {                                               // capped: the exponent of the cap's own exponential
       if (s.softcap > 0.f) qs *= 2.0f / s.softcap;
@@ -673,7 +684,7 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
       for (int w = 0; w < KW; w++) { e[w] = __builtin_amdgcn_exp2f(ms[w][g][0][c] - top); all_sum = fmaf(ms[w][g][1][c], e[w], all_sum); }
       if (q0 + 16u * g + c >= m) continue;
       const float inv = 1.0f / all_sum;
-      float* out = act + s.out + (uint64_t)qr[g] * s.out_stride + h * s.vdim;
+      float* out = outs + (uint64_t)qr[g] * s.out_stride + h * s.vdim;
       for (uint32_t v = part; v < NV; v += KW)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -691,7 +702,7 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
     sum[g] += __shfl_xor(sum[g], 16, 64); sum[g] += __shfl_xor(sum[g], 32, 64);
     if (q0 + 16u * g + c >= m) continue;
     const float inv = 1.0f / sum[g];
-    float* out = act + s.out + (uint64_t)qr[g] * s.out_stride + h * s.vdim;
+    float* out = outs + (uint64_t)qr[g] * s.out_stride + h * s.vdim;
 #pragma unroll
     for (int v = 0; v < NV; v++)
 #pragma unroll
@@ -709,19 +720,20 @@ void attn_bounded_release() { scratch_free(g_stage); scratch_free(g_parts); }
 // queries would not give every CU one, and a wave has keys enough to pay for the sum through LDS.  952 queries behind 2048 keys, 16
 // heads: 151 -> 98 us; float32, 512 queries in 16 heads: 88 -> 39, 88 behind 512 keys: 98 -> 33.  (With one for every CU the waves
 // of a workgroup are better off reading the same keys: 2048 queries in 16 heads 110 us, so: 116; in 32 heads 193 and 200.)
-static bool shared_keys(const ASpec& s, const StageDims& sd, uint32_t wgs_y) {
-  return (uint64_t)s.heads * wgs_y < (uint64_t)g.n_cu && sd.n >= 256u;
+static bool shared_keys(const ASpec& s, const StageDims& sd, uint64_t wgs) {
+  return s.heads * wgs < (uint64_t)g.n_cu && sd.n >= 256u;
 }
 template <bool WIN, int DK>
-static void launch_bf16(const ASpec& s, float* act, const bf16_t* K, const bf16_t* VT, const StageDims& sd, uint32_t m, uint32_t pos) {
+static void launch_bf16(const ASpec& s, float* act, const bf16_t* K, const bf16_t* VT, const StageDims& sd, uint32_t m, uint32_t pos, uint32_t n_seq,
+                        const SeqSteps& by) {
   switch (sd.vp / 16u) {
 #define CASE(N)                                                                                                     \
   case N: {                                                                                                         \
     constexpr int QT = DK <= 4 && N <= 8 ? 2 : 1;                                                                   \
-    if (shared_keys(s, sd, cdiv(m, 64 * QT)))                                                                       \
-      k_attn_bf16<WIN, DK, N, QT, 4><<<dim3(s.heads, cdiv(m, 16 * QT)), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos); \
+    if (shared_keys(s, sd, (uint64_t)cdiv(m, 64 * QT) * n_seq))                                                                     \
+      k_attn_bf16<WIN, DK, N, QT, 4><<<dim3(s.heads, cdiv(m, 16 * QT), n_seq), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos, by); \
     else                                                                                                            \
-      k_attn_bf16<WIN, DK, N, QT, 1><<<dim3(s.heads, cdiv(m, 64 * QT)), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos); \
+      k_attn_bf16<WIN, DK, N, QT, 1><<<dim3(s.heads, cdiv(m, 64 * QT), n_seq), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos, by); \
   } break
     CASE(2); CASE(4); CASE(6); CASE(8); CASE(12); CASE(16);
 #undef CASE
@@ -733,7 +745,7 @@ static uint32_t vtiles(uint32_t v) {
 }
 
 template <class T, bool WIN>
-static int run_portion(const ASpec& s, float* act, T* cache, uint32_t m, uint32_t pos) {
+static int run_portion(const ASpec& s, float* act, T* cache, uint32_t n_seq, uint32_t m, uint32_t pos) {
   StageDims sd;
   sd.past = WIN ? std::min(pos, s.size - 1u) : pos % s.size;
   sd.place0 = (pos - sd.past) % s.size;
@@ -742,35 +754,46 @@ static int run_portion(const ASpec& s, float* act, T* cache, uint32_t m, uint32_
   sd.dp = 32u * (s.dim <= 128u ? cdiv(s.dim, 32) : s.dim <= 192u ? 6u : 8u);
   sd.vp = vtiles(s.vdim) * 16u;
   const uint64_t nk = (uint64_t)s.kv_heads * sd.np * sd.dp, nv = (uint64_t)s.kv_heads * sd.np * sd.vp;
-  if (int r = scratch_need(g_stage, (nk + nv) * sizeof(T) + 64)) return r;
-  T *K = (T*)g_stage.p, *VT = K + nk;
-  k_attn_stage<T, WIN><<<dim3(sd.np / 32u, s.kv_heads), 256, (size_t)32 * (s.vdim + 1) * 4, g.stream>>>(s, act, cache, K, VT, sd);
+  // the sequences that one set of launches takes (their staged operands are to stay below 256 MB; the grid's limit)
+  const uint32_t at_once = (uint32_t)std::min<uint64_t>(std::min<uint64_t>(n_seq, 65535u), std::max<uint64_t>(1u, ((uint64_t)256 << 20) / ((nk + nv) * sizeof(T))));
+  const SeqSteps by = {(uint64_t)m * s.x_stride, (uint64_t)m * s.out_stride, s.seq_stride, nk, nv};
+  if (at_once < n_seq) {
+    for (uint32_t q = 0; q < n_seq; q += at_once) {
+      ASpec p = s;
+      p.x += q * by.x; p.out += q * by.out;
+      if (int r = run_portion<T, WIN>(p, act, cache + q * by.cache, std::min(at_once, n_seq - q), m, pos)) return r;
+    }
+    return ADAMAH_OK;
+  }
+  if (int r = scratch_need(g_stage, n_seq * (nk + nv) * sizeof(T) + 64)) return r;
+  T *K = (T*)g_stage.p, *VT = K + n_seq * nk;
+  k_attn_stage<T, WIN><<<dim3(sd.np / 32u, s.kv_heads, n_seq), 256, (size_t)32 * (s.vdim + 1) * 4, g.stream>>>(s, act, cache, K, VT, sd, by);
   count_launch();
   if (int r = check_launch()) return r;
   // positions still wanted after the portion: the last token's chunk, or a window up to it; from its first new token on
   const uint32_t end = pos + m, from = std::max(pos, WIN ? end - std::min(end, s.size) : (end - 1u) / s.size * s.size);
-  k_attn_keep<T><<<dim3(end - from, s.kv_heads), 256, 0, g.stream>>>(s, cache, K, VT, sd, from - (pos - sd.past));
+  k_attn_keep<T><<<dim3(end - from, s.kv_heads, n_seq), 256, 0, g.stream>>>(s, cache, K, VT, sd, from - (pos - sd.past), by);
   count_launch();
   if (int r = check_launch()) return r;
   if constexpr (sizeof(T) == 4) {
-    const bool apart = shared_keys(s, sd, cdiv(m, 64));
-    const dim3 grid(s.heads, cdiv(m, apart ? 16 : 64));
+    const bool apart = shared_keys(s, sd, (uint64_t)cdiv(m, 64) * n_seq);
+    const dim3 grid(s.heads, cdiv(m, apart ? 16 : 64), n_seq);
 #define AF(NV, DK)                                                                                                  \
   do {                                                                                                              \
-    if (apart) k_attn_f32<WIN, NV, DK, 4><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos);                   \
-    else k_attn_f32<WIN, NV, DK, 1><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos);                         \
+    if (apart) k_attn_f32<WIN, NV, DK, 4><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos, by);                   \
+    else k_attn_f32<WIN, NV, DK, 1><<<grid, 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos, by);                         \
   } while (0)
     if (sd.dp <= 128u) { if (sd.vp <= 64u) AF(4, 8); else if (sd.vp <= 128u) AF(8, 8); else AF(16, 8); }
     else { if (sd.vp <= 64u) AF(4, 16); else if (sd.vp <= 128u) AF(8, 16); else AF(16, 16); }
 #undef AF
   } else {
     switch (sd.dp / 32u) {
-      case 1: launch_bf16<WIN, 1>(s, act, K, VT, sd, m, pos); break;
-      case 2: launch_bf16<WIN, 2>(s, act, K, VT, sd, m, pos); break;
-      case 3: launch_bf16<WIN, 3>(s, act, K, VT, sd, m, pos); break;
-      case 4: launch_bf16<WIN, 4>(s, act, K, VT, sd, m, pos); break;
-      case 6: launch_bf16<WIN, 6>(s, act, K, VT, sd, m, pos); break;
-      default: launch_bf16<WIN, 8>(s, act, K, VT, sd, m, pos); break;
+      case 1: launch_bf16<WIN, 1>(s, act, K, VT, sd, m, pos, n_seq, by); break;
+      case 2: launch_bf16<WIN, 2>(s, act, K, VT, sd, m, pos, n_seq, by); break;
+      case 3: launch_bf16<WIN, 3>(s, act, K, VT, sd, m, pos, n_seq, by); break;
+      case 4: launch_bf16<WIN, 4>(s, act, K, VT, sd, m, pos, n_seq, by); break;
+      case 6: launch_bf16<WIN, 6>(s, act, K, VT, sd, m, pos, n_seq, by); break;
+      default: launch_bf16<WIN, 8>(s, act, K, VT, sd, m, pos, n_seq, by); break;
     }
   }
   count_launch();
@@ -804,7 +827,8 @@ static int run_step(const ASpec& s, float* act, T* cache, uint32_t n_seq, uint32
 #undef STEP
 }
 
-// Ranges and sizes, then one token of each of n_seq sequences or a portion of each, one sequence behind the other.
+// Ranges and sizes, then one token of each of n_seq sequences or a portion of each (12 tokens of 16 sequences, 32 heads: 16 times three
+// launches of 11, 9 and 5 us one sequence behind the other).
 template <bool WIN>
 static int run_attention(Map* ma, const ASpec& s, uint32_t cache_map, uint32_t n_seq, uint32_t rows, uint32_t seq0, uint32_t pos) {
   Map* mc = get_map(cache_map);
@@ -823,13 +847,8 @@ static int run_attention(Map* ma, const ASpec& s, uint32_t cache_map, uint32_t n
   if (rows == 1)
     return mc->dtype == DTYPE_F32 ? run_step<float, WIN>(s, act, (float*)mc->buf, n_seq, seq0, pos)
                                   : run_step<bf16_t, WIN>(s, act, (bf16_t*)mc->buf, n_seq, seq0, pos);
-  ASpec p = s;
-  for (uint32_t q = 0; q < n_seq; q++, p.x += (uint64_t)rows * s.x_stride, p.out += (uint64_t)rows * s.out_stride) {
-    const uint64_t at = slot + (uint64_t)q * s.seq_stride;
-    if (int r = mc->dtype == DTYPE_F32 ? run_portion<float, WIN>(p, act, (float*)mc->buf + at, rows, pos)
-                                       : run_portion<bf16_t, WIN>(p, act, (bf16_t*)mc->buf + at, rows, pos)) return r;
-  }
-  return ADAMAH_OK;
+  return mc->dtype == DTYPE_F32 ? run_portion<float, WIN>(s, act, (float*)mc->buf + slot, n_seq, rows, pos)
+                                : run_portion<bf16_t, WIN>(s, act, (bf16_t*)mc->buf + slot, n_seq, rows, pos);
 }
 
 }  // namespace adamah
