@@ -172,7 +172,7 @@ _SIGS = {
     "adamah_delta_rule_dev": (i32, [_U] * 10), "adamah_retention_dev": (i32, [_U] * 6),
     "adamah_chunk_attention_dev": (i32, [_U] * 6), "adamah_window_attention_dev": (i32, [_U] * 6),
     "adamah_hip_delta_rule_seqs_dev": (i32, [_U] * 10), "adamah_hip_retention_seqs_dev": (i32, [_U] * 6),
-    "adamah_hip_chunk_attention_seqs_dev": (i32, [_U] * 6),
+    "adamah_hip_chunk_attention_seqs_dev": (i32, [_U] * 6), "adamah_hip_linear_argmax_rows_dev": (i32, [_U] * 7),
     "adamah_state_space_dev": (i32, [_U] * 6), "adamah_experts_dev": (i32, [_U] * 6),
     "adamah_hip_embed_bigram_dev": (i32, [_U] * 8 + [pu32]),
     # timing helpers for benchmarks (HIP events on the library's own stream)
@@ -760,6 +760,10 @@ class Adamah:
     # ---- layered mixers over bfloat16 weights (include/adamah_hip.h; argument order as there) ----------
     def linear_dev(self, map_act, map_opnd, map_wt, spec_handle, rows_handle, rows):
         self._op("adamah_linear_dev", map_act, map_opnd, map_wt, spec_handle, rows_handle, rows)
+
+    def linear_argmax_rows_dev(self, map_act, map_opnd, map_wt, spec_handle, rows_handle, dst_handle, rows):
+        """Extension: linear_argmax_dev over one row for each of the listed rows in turn, the weights read once for several."""
+        self._op("adamah_hip_linear_argmax_rows_dev", map_act, map_opnd, map_wt, spec_handle, rows_handle, dst_handle, rows)
 
     def linear_argmax_dev(self, map_act, map_opnd, map_wt, spec_handle, dst_handle, rows):
         self._op("adamah_linear_argmax_dev", map_act, map_opnd, map_wt, spec_handle, dst_handle, rows)

@@ -348,9 +348,110 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
     best_val[blockIdx.x] = top; best_idx[blockIdx.x] = top_i;
   }
 }
-// best of n (value, index) pairs; ties to the lower index -> float(index)
+// The one-row head over NR rows at a time (their operand, float32, ready at X): the weights go by once instead of once a row, 32768 x
+// 4096 for 16 rows 697 us one by one.  Four matrix rows a wave, so that a value of x read from LDS meets four weights; a result's sums
+// are the one-row kernel's, in its order.  Rows past the last are zeros; the logits at `out` are the row `kept`'s, if it is among them.
+template <int NR>
+__global__ void __launch_bounds__(512)
+k_head_rows(const bf16_t* __restrict__ W, float* act, const LinSpec s, const float* __restrict__ X, uint32_t rows, uint32_t kept, uint32_t n_tasks,
+            float* best_val, uint32_t* best_idx) {
+  constexpr int U = 2;
+  extern __shared__ __attribute__((aligned(16))) float xs[];  // [row][two planes: elements 0..3 / 4..7 of every eight]
+  __shared__ float bv[8][NR];
+  __shared__ uint32_t bi[8][NR];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, kp = s.k_stride, half = kp >> 1;
+  uint4 p[4][U];
+  auto fetch = [&](uint32_t task, uint32_t k0) {
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const uint32_t k = k0 + 512u * u;
+        p[j][u] = k < kp ? *(const uint4*)(W + (uint64_t)min(task * 4u + j, s.n - 1u) * kp + k) : make_uint4(0, 0, 0, 0);
+      }
+  };
+  uint32_t task = blockIdx.x * 8u + wave, k0 = lane * 8u;
+  fetch(min(task, n_tasks - 1u), k0);
+  for (uint32_t i = threadIdx.x; i < NR * (kp >> 2); i += 512u) {
+    const uint32_t r = i / (kp >> 2), c = i % (kp >> 2);
+    const f4_t v = r < rows ? *(const f4_t*)(X + (uint64_t)r * kp + 4u * c) : (f4_t){0, 0, 0, 0};
+    *(f4_t*)(xs + r * kp + (c & 1u) * half + (c >> 1) * 4u) = v;
+  }
+  __syncthreads();
+  float a[NR][4], top[NR];
+  uint32_t top_i[NR];
+#pragma unroll
+  for (int r = 0; r < NR; r++) {
+    top[r] = NEG_MAX_F; top_i[r] = 0xFFFFFFFFu;
+#pragma unroll
+    for (int j = 0; j < 4; j++) a[r][j] = 0.f;
+  }
+  while (task < n_tasks) {
+    uint4 c[4][U];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+      for (int u = 0; u < U; u++) c[j][u] = p[j][u];
+    const bool last = k0 - lane * 8u + 512u * U >= kp;        // of these four rows
+    const uint32_t next = last ? task + gridDim.x * 8u : task, kn = last ? lane * 8u : k0 + 512u * U;
+    if (next < n_tasks) fetch(next, kn);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t k = k0 + 512u * u;
+      if (k >= kp) break;
+      float w[4][8];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        w[j][0] = bf_lo(c[j][u].x); w[j][1] = bf_hi(c[j][u].x); w[j][2] = bf_lo(c[j][u].y); w[j][3] = bf_hi(c[j][u].y);
+        w[j][4] = bf_lo(c[j][u].z); w[j][5] = bf_hi(c[j][u].z); w[j][6] = bf_lo(c[j][u].w); w[j][7] = bf_hi(c[j][u].w);
+      }
+#pragma unroll
+      for (int r = 0; r < NR; r++) {
+        const f4_t lo = *(const f4_t*)(xs + r * kp + (k >> 1)), hi = *(const f4_t*)(xs + r * kp + half + (k >> 1));
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) a[r][j] = fmaf(w[j][e], lo[e], a[r][j]);
+#pragma unroll
+          for (int e = 0; e < 4; e++) a[r][j] = fmaf(w[j][4 + e], hi[e], a[r][j]);
+        }
+      }
+    }
+    if (last) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const uint32_t n = task * 4u + j;
+        const float bias = s.biased && n < s.n ? act[s.bias + n] : 0.f;
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+          float y = wsum64(a[r][j]);
+          if (s.biased) y += bias;
+          a[r][j] = 0.f;
+          if (n < s.n && r == (int)kept && lane == 0) act[s.out + n] = y;
+          if (n < s.n && !isnan(y) && y > top[r]) { top[r] = y; top_i[r] = n; }
+        }
+      }
+    }
+    task = next; k0 = kn;
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int r = 0; r < NR; r++) { bv[wave][r] = top[r]; bi[wave][r] = top_i[r]; }
+  }
+  __syncthreads();
+  if (threadIdx.x < min(rows, (uint32_t)NR)) {
+    const uint32_t r = threadIdx.x;
+    float v = bv[0][r];
+    uint32_t b = bi[0][r];
+    for (int w = 1; w < 8; w++) if (bv[w][r] > v || (bv[w][r] == v && bi[w][r] < b)) { v = bv[w][r]; b = bi[w][r]; }
+    best_val[r * gridDim.x + blockIdx.x] = v; best_idx[r * gridDim.x + blockIdx.x] = b;
+  }
+}
+// best of n (value, index) pairs, a workgroup a row of them; ties to the lower index -> float(index) at dst_list[row] (or at dst)
 __global__ void __launch_bounds__(256)
-k_best_pair(const float* __restrict__ val, const uint32_t* __restrict__ idx, uint32_t n, float* dst) {
+k_best_pair(const float* __restrict__ val, const uint32_t* __restrict__ idx, uint32_t n, float* dst, const uint32_t* __restrict__ dst_list) {
+  val += (uint64_t)blockIdx.x * n; idx += (uint64_t)blockIdx.x * n;
+  if (dst_list) dst += dst_list[blockIdx.x];
   __shared__ float sv[4];
   __shared__ uint32_t si[4];
   float v = NEG_MAX_F;
@@ -632,8 +733,8 @@ k_linear_f32(const bf16_t* __restrict__ W, const float* __restrict__ X, float* a
 }
 
 // ---- launch -------------------------------------------------------------------------------------------------------
-static Scratch g_best, g_split, g_shares;
-void linear_release() { scratch_free(g_best); scratch_free(g_split); scratch_free(g_shares); }
+static Scratch g_best, g_split, g_shares, g_rows;
+void linear_release() { scratch_free(g_best); scratch_free(g_split); scratch_free(g_shares); scratch_free(g_rows); }
 
 static bool span_ok(uint64_t off, uint64_t stride, uint64_t rows, uint64_t width, uint64_t n_elems) {
   return rows == 0 || in_range(off, (rows - 1) * stride + width, n_elems);
@@ -842,13 +943,66 @@ int adamah_linear_argmax_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_w
     const uint32_t n_tasks = cdiv(s->n, 2), grid = gemv_grid(n_tasks);
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
     gemv_launch<LEPI_ARGMAX>(ma, mw, *s, nullptr, n_tasks);
-    k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0]);
+    k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0], nullptr);
   } else {
     if (int r = run_linear(ma, mo, mw, *s, nullptr, rows)) return r;
     // (1024 threads only reduce more: rows of 50 in 4.1 us, with 256 in 3.0, of 1000 in 4.2 and 3.9; rows of 2000 in 4.5 and 5.1, of 4000 in 5.0 and 8.1)
     if (s->n > 1024u) k_best_row<1024><<<rows, 1024, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
     else k_best_row<256><<<rows, 256, 0, g.stream>>>(act, s->out, s->out_stride, s->n, act, res_u32(h_dst, rows));
   }
+  count_launch();
+  return check_launch();
+}
+
+// What adamah_linear_argmax_dev over one row gives, for each of the listed rows in turn
+int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_rows, uint32_t h_dst, uint32_t rows) { ADAMAH_API();
+  Map *ma = get_f32_map(map_act), *mo = get_map(map_opnd), *mw = get_map(map_wt);
+  const LinSpec* s = spec_of<LinSpec>(h_spec);
+  const uint32_t* dev;
+  uint32_t src_rows;
+  if (!s || s->epi != 0u || rows == 0) return ADAMAH_ERR_INVALID;
+  if (int r = row_list(h_rows, rows, &dev, &src_rows)) return r;
+  if (int r = check_linear(ma, mo, mw, *s, 1, src_rows)) return r;
+  const uint32_t *dst = res_host(h_dst, rows), *dst_dev = res_u32(h_dst, rows);
+  if (!dst || !dst_dev) return ADAMAH_ERR_INVALID;
+  for (uint32_t i = 0; i < rows; i++) if (dst[i] >= ma->n_elems) return ADAMAH_ERR_INVALID;
+  float* act = (float*)ma->buf;
+  // rows at a time: as many as 144 KB of LDS hold (a workgroup a CU), none of them for nothing
+  const size_t row_bytes = (size_t)s->k_stride * 4;
+  const uint32_t fit = (uint32_t)(((size_t)144 << 10) / row_bytes), nr = fit >= 8 && rows > 4 ? 8 : fit >= 4 && rows > 2 ? 4 : fit >= 2 && rows > 1 ? 2 : 1;
+  if (nr == 1) {
+    const uint32_t n_tasks = cdiv(s->n, 2), grid = gemv_grid(n_tasks);
+    if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
+    for (uint32_t i = 0; i < rows; i++) {
+      LinSpec one = *s;                                       // (row i of no list)
+      if (!dev) { one.src += i * s->src_stride; one.gate += i * s->gate_stride; one.branch += i * s->branch_stride; one.res_out += i * s->res_stride; one.keep += i * s->keep_stride; }
+      gemv_launch<LEPI_ARGMAX>(ma, mw, one, dev ? dev + i : nullptr, n_tasks);
+      k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[i], nullptr);
+      count_launch();
+    }
+    return check_launch();
+  }
+  const uint32_t n_tasks = cdiv(s->n, 4), grid = std::min<uint32_t>(cdiv(n_tasks, 8), (uint32_t)g.n_cu);
+  if (int r = scratch_need(g_best, (size_t)grid * rows * 8)) return r;
+  if (int r = scratch_need(g_rows, rows * row_bytes)) return r;
+  float* const X = (float*)g_rows.p;
+  float* const bv = (float*)g_best.p;
+  uint32_t* const bi = (uint32_t*)(bv + (size_t)grid * rows);
+  operand_rows<float>(*s, act, X, dev, rows);
+  const bf16_t* W = (const bf16_t*)mw->buf + s->w;
+  for (uint32_t i = 0; i < rows; i += nr) {
+    const uint32_t n = std::min(nr, rows - i), kept = i + n == rows ? n - 1u : 0xFFFFFFFFu;
+#define HEAD(NR)                                                                                                    \
+  do {                                                                                                              \
+    hipFuncSetAttribute((const void*)k_head_rows<NR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NR * row_bytes)); \
+    k_head_rows<NR><<<grid, 512, NR * row_bytes, g.stream>>>(W, act, *s, X + (size_t)i * s->k_stride, n, kept, n_tasks, bv + (size_t)i * grid, bi + (size_t)i * grid); \
+  } while (0)
+    if (nr == 8) HEAD(8); else if (nr == 4) HEAD(4); else HEAD(2);
+#undef HEAD
+    count_launch();
+  }
+  if (int r = check_launch()) return r;
+  k_best_pair<<<rows, 256, 0, g.stream>>>(bv, bi, grid, act, dst_dev);
   count_launch();
   return check_launch();
 }

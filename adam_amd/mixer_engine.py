@@ -188,6 +188,7 @@ class MixerEngine(DecodeEngine):
         self._c_tok_pos = take(M)
         self._c_tok_locs = np.arange(self._c_tok_pos, self._c_tok_pos + M, dtype=np.uint32)
         self._tok_rows_h, self._tok_row_h = self._up(self._c_tok_locs), []
+        self._last_rows_h = self._up(np.zeros(self._batch, np.uint32))
         self._hid_locs = np.arange(self._rows["hidden"][0], self._rows["hidden"][0] + E, dtype=np.uint32)
         self._alloc_sample_handles()
         self._vec_off = {}
@@ -560,9 +561,12 @@ class MixerEngine(DecodeEngine):
         if at_once < 2:
             return super()._prefill_each(prompts)
         g, ws, first = self.gpu, self.WS_MAP, []
-        while len(self._tok_row_h) < at_once:
+        heads = hasattr(g, 'linear_argmax_rows_dev')          # one row's head for each of the last rows, in one call
+        while not heads and len(self._tok_row_h) < at_once:
             n = len(self._tok_row_h)
             self._tok_row_h.append(self._up(self._c_tok_locs[n:n + 1]))
+        if heads:
+            g.upload_dev((np.arange(self._batch, dtype=np.uint32) + 1) * np.uint32(P) - np.uint32(1), handle=self._last_rows_h)
         for s0 in range(0, len(prompts), at_once):
             part = prompts[s0:s0 + at_once]
             toks = [t for p in part for t in p]
@@ -572,9 +576,12 @@ class MixerEngine(DecodeEngine):
                 self._advance(s, 0, P)
             self._embed(toks, 1, len(toks), s0, 0)
             self._run_program(len(part), P, s0, 0)
-            for i in range(len(part)):
+            for i in range(0 if heads else len(part)):
                 mid, h = self._head(i * P + P - 1)
                 g.linear_argmax_dev(ws, self.OPND_MAP, mid, h, self._tok_row_h[i], 1)
+            if heads:
+                mid, h = self._head(0)
+                g.linear_argmax_rows_dev(ws, self.OPND_MAP, mid, h, self._last_rows_h, self._tok_rows_h, len(part))
             g.batch_end()
             first += self.read_tokens(len(part))
         return first

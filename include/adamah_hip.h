@@ -321,6 +321,10 @@ typedef struct AdamahLinearSpec {
 int adamah_linear_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_rows, uint32_t rows);
 /* The same (epi 0), then float(arg-max of row r) to element dst[r] of the activation map (h_dst: `rows` offsets). */
 int adamah_linear_argmax_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_dst, uint32_t rows);
+/* adamah_linear_argmax_dev over ONE row (float32 operands), for each of `rows` rows in turn -- row h_rows[i] of the source (h_rows 0: row i),
+ * its best column to h_dst[i], the logits of the last one left at `out` --, the weights read once for up to eight of them. */
+int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_rows, uint32_t h_dst,
+                                      uint32_t rows);
 
 /* dst += scale * (a / rms(a) * wa + b / rms(b) * wb) per row (store = 1: dst =). */
 typedef struct AdamahMergeSpec { uint32_t a, b, stride, wa, wb, dst, dst_stride, dim; float eps, scale; uint32_t store; } AdamahMergeSpec;

@@ -116,6 +116,14 @@ class MixerOps:
         for r, d in enumerate(self.res[h_dst].view(np.uint32)[:rows]):
             self._put(map_act, int(d), [np.argmax(self._get(map_act, s.out + r * s.out_stride, s.n))])
 
+    def linear_argmax_rows_dev(self, map_act, map_opnd, map_wt, h, h_rows, h_dst, rows):
+        """linear_argmax_dev over one row for each listed row."""
+        at = self.res[h_rows].view(np.uint32)[:rows] if h_rows else np.arange(rows)
+        s = self._spec(h, _LINEAR)
+        for r, d in zip(at, self.res[h_dst].view(np.uint32)[:rows]):
+            self.linear_dev(map_act, map_opnd, map_wt, h, self.upload_dev(np.array([r], np.uint32))[0], 1)
+            self._put(map_act, int(d), [np.argmax(self._get(map_act, s.out, s.n))])
+
     def merge_norm_dev(self, map_act, h, rows):
         s = self._spec(h, _MERGE)
         for r in range(rows):

@@ -723,3 +723,40 @@ def test_chunk_attention_with_the_keys_parted_among_waves(hip, H, G, D, V, C, ms
     for m in ms:
         run(1, m, 0, pos)
         pos += m
+
+
+@pytest.mark.parametrize("k,n,rows,listed,branched", [(64, 40, 2, False, False), (200, 1003, 5, True, False), (4096, 517, 9, True, True), (4608, 70, 16, False, False),
+                                                      (4672, 33, 6, True, False), (9216, 66, 3, True, True), (20000, 21, 2, True, False), (1000, 8, 1, True, False)])
+def test_heads_of_several_rows_are_the_one_row_head(hip, k, n, rows, listed, branched):
+    """adamah_hip_linear_argmax_rows_dev, at every number of rows a workgroup takes at a time (k bounds it): the best columns and the
+    logits left behind are, but for the order of the norm's sums, those of the one-row head called for each row."""
+    rng = np.random.default_rng(k + n)
+    ks = -(-k // 64) * 64
+    src_rows = rows + 3
+    at = rng.permutation(src_rows)[:rows] if listed else np.arange(rows)
+    w = np.zeros((n, ks), np.float32)
+    w[:, :k] = rng.standard_normal((n, k)) / np.sqrt(k)
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * ks)
+    hip.scatter_contiguous(WT, 0, f32_to_bf16(w.reshape(-1)))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, 8)
+    x0, b0, wt, bw, bias, out, tok = np.cumsum([0] + [src_rows * k] * 2 + [k, k, n, n]).tolist()
+    f32map(hip, WS, tok + src_rows, rng.standard_normal(tok + src_rows).astype(np.float32))
+    s = dict(n=n, k=k, k_stride=ks, w=0, src=x0, src_stride=k, out=out, out_stride=n, groups=1, eps=1e-5, wt=wt, wt_len=k, wt_add=0.5, bias=bias, biased=1)
+    if branched:
+        s.update(branched=1, branch=b0, branch_stride=k, branch_wt=bw)
+    note(f"heads of several rows k={k} n={n} rows={rows}")
+    want, last = [], None
+    for r in at:
+        one = dict(s, src=x0 + int(r) * k)
+        if branched:
+            one["branch"] = b0 + int(r) * k
+        hip.linear_argmax_dev(WS, OP, WT, up(hip, A.LinearSpec(**one).words()), up(hip, [tok]), 1)
+        want.append(int(read(hip, WS, tok, 1)[0]))
+        last = read(hip, WS, out, n)
+    hip.scatter_contiguous(WS, out, np.zeros(n, np.float32))
+    hip.linear_argmax_rows_dev(WS, OP, WT, up(hip, A.LinearSpec(**s).words()), up(hip, at) if listed else 0, up(hip, tok + 1 + np.arange(rows)), rows)
+    assert [int(t) for t in read(hip, WS, tok + 1, rows)] == want
+    got = read(hip, WS, out, n)
+    assert np.abs(got - last).max() < 64 * 2.0 ** -24 * np.abs(last).max()
+    with pytest.raises(RuntimeError):
+        hip.linear_argmax_rows_dev(WS, OP, WT, up(hip, A.LinearSpec(**dict(s, src=tok)).words()), up(hip, at) if listed else 0, up(hip, tok + 1 + np.arange(rows)), rows)
