@@ -357,6 +357,33 @@ k_experts_sum(const XSpec s, float* act, const float* __restrict__ parts, const 
   const float *x = act + s.x + (uint64_t)row * s.x_stride, *sh = act + shared + (uint64_t)row * shared_stride;
   const float* p = parts + (uint64_t)row * s.top * s.width;
   float* d = act + s.out + (uint64_t)row * s.out_stride;
+  // Four columns a thread and no load under a condition (an entry that gives the row back has no result: what lies there is read and
+  // left out): 2048 rows of 2048, 6 of 34: 45 us with a float a load and a branch for each, so: 25; 10 rows 26 and 6.
+  if (((s.width | s.x | s.x_stride | shared | shared_stride | s.out | s.out_stride) & 3u) == 0u) {
+    for (uint32_t i = tid * 4u; i < s.width; i += 1024u) {
+      const f4_t xv = *(const f4_t*)(x + i), hv = *(const f4_t*)(sh + i);
+      f4_t y = {back * xv[0], back * xv[1], back * xv[2], back * xv[3]};
+      for (uint32_t j0 = 0; j0 < s.top; j0 += 6u) {
+        f4_t v[6];
+#pragma unroll
+        for (uint32_t u = 0; u < 6u; u++) v[u] = *(const f4_t*)(p + (uint64_t)min(j0 + u, s.top - 1u) * s.width + i);
+#pragma unroll
+        for (uint32_t u = 0; u < 6u; u++) {
+          const uint32_t j = min(j0 + u, s.top - 1u);
+          const bool on = j0 + u < s.top && real[j];
+          const float wj = w[j];
+#pragma unroll
+          for (int e = 0; e < 4; e++) y[e] = on ? fmaf(wj, v[u][e], y[e]) : y[e];
+        }
+      }
+      if (s.shared_ff)
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[e] = fmaf(sg, hv[e], y[e]);
+      if (s.epi) { const f4_t o = *(const f4_t*)(d + i); y = (f4_t){o[0] + y[0], o[1] + y[1], o[2] + y[2], o[3] + y[3]}; }
+      *(f4_t*)(d + i) = y;
+    }
+    return;
+  }
   for (uint32_t i = tid; i < s.width; i += 256u) {
     float y = back * x[i];
 #pragma unroll 4

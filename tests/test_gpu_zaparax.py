@@ -14,7 +14,7 @@ from adam_amd.engine import GenerationConfig
 from adam_amd.mixer_engine import MixerEngine
 from adam_amd.models import zaparax_config
 from adam_amd.safetensors_file import f32_to_bf16
-from gpu_util import note
+from gpu_util import f32map, note, read, up
 from mixer_cases import floats, rel, write_model
 from mixer_pair import CA, OP, ST, WS, WT, Pair
 from oracle import zaparax_np as Z
@@ -551,3 +551,42 @@ def test_window_attention_with_the_keys_parted_among_waves(hip, H, G, D, V, R, m
     for m in ms:
         run(1, m, 0, pos)
         pos += m
+
+
+@pytest.mark.parametrize("E,I,top,shared,width,epi", [(5, 4, 7, 28, 64, 1), (20, 9, 13, 0, 1028, 0), (3, 1, 1, 16, 2052, 1), (30, 2, 6, 64, 1024, 0)])
+def test_sums_of_aligned_rows_are_those_of_shifted_ones(hip, E, I, top, shared, width, epi):
+    """Rows that start on four floats are added up four columns a thread (any number of choices, some of them giving the row back, whose
+    results are never written); moved by one float they are not: the same words."""
+    note(f"experts, aligned sums E {E} top {top} width {width}")
+    rng = np.random.default_rng(E + width)
+    n, ks, F, rows = E + I, r64(width), 64, 9
+    S = r64(shared)
+    xs = width + 4
+    W = f32_to_bf16((rng.standard_normal(E * 32 * ks + E * width * F + width * max(S, 1)) / 32).astype(np.float32))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size + 8)
+    hip.scatter_contiguous(WT, 0, W)
+    act_at = rows * ks
+    sact = act_at + rows * top * F
+    OPN = sact + rows * max(S, 1) + 8
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, OPN)
+    hip.scatter_contiguous(OP, 0, f32_to_bf16(rng.standard_normal(OPN).astype(np.float32)))
+    got = []
+    vals = {k: rng.standard_normal(s).astype(np.float32) for k, s in (("h", rows * xs), ("out", rows * xs), ("log", rows * (n + 1)))}
+    for shift in (0, 1):
+        at, pos = {}, 0
+        for name, sz in (("corr", n + -n % 4), ("log", rows * (n + 1) + -rows * (n + 1) % 4), ("act", top * F), ("sact", 64 + S), ("h", rows * xs + 4), ("sout", rows * xs + 4),
+                         ("out", rows * xs + 4)):
+            at[name] = pos + (shift if name in ("h", "sout", "out") else 0)
+            pos += sz
+        f32map(hip, WS, pos + 8, np.zeros(pos, np.float32))
+        for name, v in vals.items():
+            hip.scatter_contiguous(WS, at[name], v)
+        spec = A.ExpertsSpec(experts=E, identity=I, top=top, ff=16, ff_stride=F, width=width, k_stride=ks, gate_up=0, gate_up_step=32 * ks, down=E * 32 * ks,
+                             down_step=width * F, logits=at["log"], logits_stride=n + 1, correction=at["corr"], x=at["h"], x_stride=xs, opnd=0, act=at["act"],
+                             act_opnd=act_at, shared_ff=shared, shared_ff_stride=S, shared_down=E * 32 * ks + E * width * F, shared_act=at["sact"], out=at["out"],
+                             out_stride=xs, epi=epi)
+        sh = up(hip, A.LinearSpec(w=E * 32 * ks + E * width * F, n=width, k=shared, k_stride=S, src=at["h"], src_stride=xs, out=at["sout"], out_stride=xs, opnd=sact,
+                                  ready=1).words()) if shared else 0
+        hip.experts_dev(WS, OP, WT, up(hip, spec.words()), sh, rows)
+        got.append(read(hip, WS, at["out"], rows * xs).reshape(rows, xs)[:, :width])
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
