@@ -71,36 +71,44 @@ __device__ __forceinline__ float dot8_regs(const uint4 (&w)[NC], const float* x,
 // One token of one sequence per blockIdx.z; DN: state rows a thread holds (dim <= 16 DN); TM >= taps.  Everything a
 // workgroup reads is asked for at the start: the state, the convolution's inputs, the rows of the low-rank factors (in
 // registers where their rank is at most 128).
+//
+// CW: value columns of a thread, VC of them beside each other in a workgroup.  With one, a head of 128 columns is four
+// workgroups, each of which repeats the head's decay and convolution: latency decides, and more of them is better.  With
+// four, one workgroup does the head: a quarter of the repeated work, and the state moves 16 bytes a lane.  The state's
+// rows go to the same sums in the same order either way, so a result does not depend on the sequences beside it.
 #define DSTEP 512u
-template <int DN, int TM>
+template <int CW> struct alignas(4 * CW) Cols { float x[CW]; };
+template <int DN, int TM, int CW>
 __global__ void __launch_bounds__(DSTEP)
 k_delta_step(const DSpec s, const LowRank da, const LowRank ga, float* act, const bf16_t* __restrict__ W, float* state, uint32_t seq0,
              uint32_t pos) {
   constexpr int NP = DN / 4 > 0 ? DN / 4 : 1;          // decay rows of 8 lanes: 64 a pass
-  constexpr uint32_t NG = DSTEP / VC;
+  constexpr uint32_t NG = DSTEP / VC, NV = VC * CW;
+  constexpr int NR = CW > 2 ? CW / 2 : 1;              // gate rows of 8 lanes: 64 a pass
   extern __shared__ float lds[];
   __shared__ float sh[3 * DSTEP / 64];
-  __shared__ float red[2][NG][VC];
-  __shared__ float vs[VC];
-  const uint32_t D = s.dim, V = s.vdim, tid = threadIdx.x, h = blockIdx.x, v0 = blockIdx.y * VC, row = blockIdx.z;
+  __shared__ __align__(16) float red[2][NG][NV];
+  __shared__ __align__(16) float vs[NV];
+  const uint32_t D = s.dim, V = s.vdim, tid = threadIdx.x, h = blockIdx.x, v0 = blockIdx.y * NV, row = blockIdx.z;
   float *qs = lds, *ks = qs + D, *gs = ks + D, *la = gs + D, *lg = la + da.k_stride;
   const uint32_t n_ch = 2u * s.kv_heads * D + s.heads * V, rep = s.heads / s.kv_heads, kv = h / rep, sub = tid & 7u;
   const float* x = act + s.x + (uint64_t)row * s.x_stride;
   float* ring = state + (uint64_t)(seq0 + row) * s.seq_stride + s.conv_off;
   float* S = state + (uint64_t)(seq0 + row) * s.seq_stride + s.s_off + (uint64_t)h * D * V;
   const uint32_t qc = kv * D, kc = s.kv_heads * D + kv * D, vc = 2u * s.kv_heads * D + h * V;
-  const uint32_t col = tid & (VC - 1u), dg = tid / VC, v = v0 + col;
+  const uint32_t col = (tid & (VC - 1u)) * CW, dg = tid / VC, v = v0 + col;
   const bool small = da.k_stride <= 128u && ga.k_stride <= 128u;
-  const uint32_t gt = DSTEP - 1u - tid, gv = v0 + (gt >> 3), grow = h * V + min(gv, V - 1u);   // gate rows: the last threads
-  float st[DN];
+  const uint32_t gt = DSTEP - 1u - tid;                // gate rows: the last threads
+  Cols<CW> st[DN];
 #pragma unroll
   for (int i = 0; i < DN; i++) {
     const uint32_t d = dg + NG * i;
-    st[i] = (pos != 0u && d < D && v < V) ? S[(uint64_t)d * V + v] : 0.f;
+    st[i] = {};
+    if (pos != 0u && d < D && v < V) st[i] = *(const Cols<CW>*)(S + (uint64_t)d * V + v);
   }
   for (uint32_t i = tid; i < da.k_stride; i += DSTEP) la[i] = i < da.k ? act[da.src + (uint64_t)row * da.src_stride + i] : 0.f;
   for (uint32_t i = gt; i < ga.k_stride; i += DSTEP) lg[i] = i < ga.k ? act[ga.src + (uint64_t)row * ga.src_stride + i] : 0.f;
-  uint4 wa[NP][2], wg[2];
+  uint4 wa[NP][2], wg[NR][2];
   float bias[NP];
 #pragma unroll
   for (int i = 0; i < NP; i++) {
@@ -112,10 +120,13 @@ k_delta_step(const DSpec s, const LowRank da, const LowRank ga, float* act, cons
         wa[i][n] = sub * 8u + 64u * n < da.k_stride ? *(const uint4*)(W + da.w + (uint64_t)r * da.k_stride + sub * 8u + 64u * n) : make_uint4(0, 0, 0, 0);
   }
   const float a_log = act[s.a_log + h], step = x[s.x_b + h];
-  if (small && gt < 8u * VC)
+  const auto gate_row = [&](int i) { return h * V + min(v0 + (gt >> 3) + 64u * i, V - 1u); };
+  if (small && gt < 8u * NV)
 #pragma unroll
-    for (int n = 0; n < 2; n++)
-      wg[n] = (gt & 7u) * 8u + 64u * n < ga.k_stride ? *(const uint4*)(W + ga.w + (uint64_t)grow * ga.k_stride + (gt & 7u) * 8u + 64u * n) : make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < NR; i++)
+#pragma unroll
+      for (int n = 0; n < 2; n++)
+        wg[i][n] = (gt & 7u) * 8u + 64u * n < ga.k_stride ? *(const uint4*)(W + ga.w + (uint64_t)gate_row(i) * ga.k_stride + (gt & 7u) * 8u + 64u * n) : make_uint4(0, 0, 0, 0);
   float sq = 0.f, sk = 0.f, qk = 0.f;
   for (uint32_t i = tid; i < 2u * D; i += DSTEP) {
     const bool is_k = i >= D;
@@ -124,7 +135,7 @@ k_delta_step(const DSpec s, const LowRank da, const LowRank ga, float* act, cons
     (is_k ? ks : qs)[d] = a;
     if (is_k) sk = fmaf(a, a, sk); else sq = fmaf(a, a, sq);
   }
-  if (gt < VC && v0 + gt < V)
+  if (gt < NV && v0 + gt < V)
     vs[gt] = conv_silu_ring<TM>(x, ring, n_ch, vc + v0 + gt, pos, act + s.cv + (uint64_t)(h * V + v0 + gt) * s.taps, s.taps);
   const float ea = expf(a_log), beta = sigmoid_f(step);
   __syncthreads();
@@ -143,41 +154,61 @@ k_delta_step(const DSpec s, const LowRank da, const LowRank ga, float* act, cons
       if (sub == 0 && d < D) gs[d] = expf(-ea * softplus_f(a + act[s.dt_bias + r]));
     }
   }
-  if (gt < 8u * VC) {
-    const float a = small ? dot8_regs<2>(wg, lg, ga.k_stride, gt & 7u) : dot8(W + ga.w + (uint64_t)grow * ga.k_stride, lg, ga.k_stride, gt & 7u);
-    if ((gt & 7u) == 0 && gv < V) act[ga.out + (uint64_t)row * ga.out_stride + grow] = a;
-  }
+  if (gt < 8u * NV)
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+      const uint32_t grow = gate_row(i);
+      const float a = small ? dot8_regs<2>(wg[i], lg, ga.k_stride, gt & 7u) : dot8(W + ga.w + (uint64_t)grow * ga.k_stride, lg, ga.k_stride, gt & 7u);
+      if ((gt & 7u) == 0 && v0 + (gt >> 3) + 64u * i < V) act[ga.out + (uint64_t)row * ga.out_stride + grow] = a;
+    }
   block_add3<DSTEP / 64>(sq, sk, qk, sh);      // (its barriers also publish gs)
   const float iq = 1.0f / sqrtf(sq + 1e-6f) / sqrtf((float)D), ik = 1.0f / sqrtf(sk + 1e-6f);
   qk = qk * iq * ik;
-  float pk = 0.f, pq = 0.f;
+  Cols<CW> pk = {}, pq = {};
 #pragma unroll
   for (int i = 0; i < DN; i++) {
     const uint32_t d = dg + NG * i;
     if (d < D) {
-      st[i] *= gs[d];
-      pk = fmaf(st[i], ks[d], pk); pq = fmaf(st[i], qs[d], pq);
+      const float g = gs[d], k = ks[d], q = qs[d];
+#pragma unroll
+      for (int c = 0; c < CW; c++) {
+        st[i].x[c] *= g;
+        pk.x[c] = fmaf(st[i].x[c], k, pk.x[c]); pq.x[c] = fmaf(st[i].x[c], q, pq.x[c]);
+      }
     }
   }
-  red[0][dg][col] = pk; red[1][dg][col] = pq;
+  *(Cols<CW>*)&red[0][dg][col] = pk; *(Cols<CW>*)&red[1][dg][col] = pq;
   __syncthreads();
-  pk = 0.f; pq = 0.f;
+  pk = {}; pq = {};
+#pragma unroll CW == 1 ? 16 : 4
+  for (int i = 0; i < (int)NG; i++) {
+    const Cols<CW> a = *(const Cols<CW>*)&red[0][i][col], b = *(const Cols<CW>*)&red[1][i][col];
 #pragma unroll
-  for (int i = 0; i < (int)NG; i++) { pk += red[0][i][col]; pq += red[1][i][col]; }
+    for (int c = 0; c < CW; c++) { pk.x[c] += a.x[c]; pq.x[c] += b.x[c]; }
+  }
   if (v < V) {
-    const float u = beta * (vs[col] - pk * ik);
-    if (dg == 0) act[s.out + (uint64_t)row * s.out_stride + h * V + v] = fmaf(u, qk, pq * iq);
-    const float uk = u * ik;
+    float uk[CW];
+#pragma unroll
+    for (int c = 0; c < CW; c++) {
+      const float u = beta * (vs[col + c] - pk.x[c] * ik);
+      if (dg == 0) act[s.out + (uint64_t)row * s.out_stride + h * V + v + c] = fmaf(u, qk, pq.x[c] * iq);
+      uk[c] = u * ik;
+    }
 #pragma unroll
     for (int i = 0; i < DN; i++) {
       const uint32_t d = dg + NG * i;
-      if (d < D) S[(uint64_t)d * V + v] = fmaf(ks[d], uk, st[i]);
+      if (d < D) {
+        const float k = ks[d];
+#pragma unroll
+        for (int c = 0; c < CW; c++) st[i].x[c] = fmaf(k, uk[c], st[i].x[c]);
+        *(Cols<CW>*)(S + (uint64_t)d * V + v) = st[i];
+      }
     }
   }
   float* slot = ring + (uint64_t)(pos % s.taps) * n_ch;
   if (blockIdx.y == 0 && h % rep == 0)
     for (uint32_t d = tid; d < D; d += DSTEP) { slot[qc + d] = x[qc + d]; slot[kc + d] = x[kc + d]; }
-  if (tid < VC && v0 + tid < V) slot[vc + v0 + tid] = x[vc + v0 + tid];
+  if (tid < NV && v0 + tid < V) slot[vc + v0 + tid] = x[vc + v0 + tid];
 }
 
 __device__ __forceinline__ float rotated(const float* x, const float* freq, uint32_t d, uint32_t dims, uint32_t p) {
@@ -616,11 +647,18 @@ static int run_delta_rule(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, 
   if (rows == 1) {
     const size_t lds = (size_t)(3 * D + da->k_stride + ga->k_stride) * 4;
     if (lds > 48000) return ADAMAH_ERR_INVALID;
-    const dim3 grid((uint32_t)H, cdiv(V, VC), n_seq);
     const bf16_t* W = (const bf16_t*)mw->buf;
-#define STEP(DN, TM) k_delta_step<DN, TM><<<grid, DSTEP, lds, g.stream>>>(*s, low_rank(*da), low_rank(*ga), act, W, state, seq0, pos)
-    if (s->taps <= 4) { if (D <= 64) STEP(4, 4); else if (D <= 128) STEP(8, 4); else STEP(16, 4); }
-    else { if (D <= 64) STEP(4, MAX_TAPS); else if (D <= 128) STEP(8, MAX_TAPS); else STEP(16, MAX_TAPS); }
+    // Four columns a thread once that alone gives more than every other compute unit a workgroup, and rows start on 16
+    // bytes.  Heads of 128 x 128, us with one and four (the state at a large copy's rate): 32 heads 1 sequence 8.4 / 9.6 (0.9),
+    // 4 12.0 / 11.6 (3.5), 8 21.6 / 14.7 (6.9), 16 38.5 / 20.9 (13.8), 32 77 / 45 (28); 16 heads 4 8.9 / 10.0, 16 21.8 / 14.6.
+    // Beyond 128 rows of state a thread's part of it would leave one workgroup a compute unit.
+    const bool wide = s->taps <= 4 && D <= 128 && V > 2 * VC && !((V | s->s_off | s->seq_stride) & 3u) &&
+                      2 * H * cdiv(V, 4 * VC) * n_seq > (uint64_t)g.n_cu;
+    const dim3 grid((uint32_t)H, cdiv(V, wide ? 4 * VC : VC), n_seq);
+#define STEP(DN, TM, CW) k_delta_step<DN, TM, CW><<<grid, DSTEP, lds, g.stream>>>(*s, low_rank(*da), low_rank(*ga), act, W, state, seq0, pos)
+    if (wide) { if (D <= 64) STEP(4, 4, 4); else STEP(8, 4, 4); }
+    else if (s->taps <= 4) { if (D <= 64) STEP(4, 4, 1); else if (D <= 128) STEP(8, 4, 1); else STEP(16, 4, 1); }
+    else { if (D <= 64) STEP(4, MAX_TAPS, 1); else if (D <= 128) STEP(8, MAX_TAPS, 1); else STEP(16, MAX_TAPS, 1); }
 #undef STEP
     count_launch();
     return check_launch();

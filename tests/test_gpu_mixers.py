@@ -317,7 +317,7 @@ def test_merge_norm(hip):
 
 
 # ---- recurrences -----------------------------------------------------------------------------------------------------
-def delta_pair(hip, H, KH, D, V, taps, rank, rows, seqs, strong, seed):
+def delta_pair(hip, H, KH, D, V, taps, rank, rows, seqs, strong, seed, off=1, pad=5):
     rng = np.random.default_rng(seed)
     n_ch = 2 * KH * D + H * V
     xs = n_ch + H + 2 * rank + 1
@@ -326,7 +326,7 @@ def delta_pair(hip, H, KH, D, V, taps, rank, rows, seqs, strong, seed):
         at[n] = pos
         pos += sz
     ks = (rank + 63) // 64 * 64
-    state = H * D * V + taps * n_ch + 5
+    state = H * D * V + taps * n_ch + pad
     p = Pair(hip, pos + 16, wt=(H * D + H * V) * ks, opnd=2 * rows * ks, state=seqs * state)
     W = np.zeros((H * D + H * V, ks), np.uint16)
     W[:, :rank] = f32_to_bf16((rng.standard_normal((H * D + H * V, rank)) / np.sqrt(rank)).astype(np.float32))
@@ -341,7 +341,7 @@ def delta_pair(hip, H, KH, D, V, taps, rank, rows, seqs, strong, seed):
     c = at["conv"]
     spec = p.up(A.DeltaSpec(heads=H, kv_heads=KH, dim=D, vdim=V, taps=taps, x=at["x"], x_stride=xs, x_b=n_ch, cq=c, ck=c + KH * D * taps,
                             cv=c + 2 * KH * D * taps, a_log=at["A"], dt_bias=at["dt"], out=at["o"], out_stride=H * V, state_map=ST,
-                            s_off=1, conv_off=1 + H * D * V, seq_stride=state).words())
+                            s_off=off, conv_off=off + H * D * V, seq_stride=state).words())
     fresh = lambda n: p.put(WS, at["x"], rng.standard_normal((n, xs)))
 
     def run(n_seq, m, seq0, pos0):
@@ -349,7 +349,8 @@ def delta_pair(hip, H, KH, D, V, taps, rank, rows, seqs, strong, seed):
         p.call("delta_rule_dev", WS, OP, WT, spec, dec, gate, n_seq, m, seq0, pos0)
         p.same(WS, at["o"], n_seq * m * H * V, 2e-5, f"outputs {n_seq}x{m} at {pos0}")
         p.same(WS, at["g"], n_seq * m * H * V, 2e-5, "gate")
-        p.same(ST, seq0 * state + 1, H * D * V, 2e-5, f"state after {pos0 + m}")
+        for i in range(n_seq):
+            p.same(ST, (seq0 + i) * state + off, H * D * V, 2e-5, f"state of sequence {i} after {pos0 + m}")
     return run
 
 
@@ -371,6 +372,18 @@ def test_delta_rule(hip, H, KH, D, V, taps, rank, strong):
         run(3, 1, 0, 5 + t)
     run(1, 1, 2, 0)                                  # a sequence that starts with a single token
     run(1, 2, 2, 1)
+
+
+@pytest.mark.parametrize("H,KH,D,V,taps,rank,seqs", [
+    (8, 8, 128, 128, 4, 128, 17), (8, 4, 128, 96, 3, 20, 17), (4, 2, 100, 132, 4, 140, 17), (9, 3, 17, 68, 4, 16, 16), (2, 1, 64, 256, 1, 64, 33),
+    (8, 8, 129, 128, 4, 8, 17), (8, 8, 64, 128, 5, 8, 17)])
+def test_delta_rule_steps_of_many_sequences(hip, H, KH, D, V, taps, rank, seqs):
+    """Enough heads for four columns a thread, rows of state on 16 bytes; one column where dim or taps are beyond its registers."""
+    note(f"delta rule of {seqs} sequences, H {H} KH {KH} D {D} V {V} taps {taps} rank {rank}")
+    n_ch = 2 * KH * D + H * V
+    run = delta_pair(hip, H, KH, D, V, taps, rank, seqs, seqs, False, seed=V, off=4, pad=8 + -(taps * n_ch) % 4)
+    for pos in (0, 1, 2, 3, 9):
+        run(seqs, 1, 0, pos)
 
 
 def test_delta_rule_keeps_a_key_over_a_long_gap(hip):
