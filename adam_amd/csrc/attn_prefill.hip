@@ -267,34 +267,57 @@ k_attn_prefill(const float* data, float* out, const __half* kv, uint64_t kv_shif
 // Workgroup b serves head quad b % (H / 4): with eight KV heads, XCD x (workgroups x, x + 8, ...) walks the cache of
 // KV head x only, which fits its L2; the token tiles with the longest walks come first.
 typedef _Float16 h8p_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u4p_t __attribute__((ext_vector_type(4)));
 typedef float f4pu_t __attribute__((ext_vector_type(4), aligned(4)));
 struct AttpVt { uint32_t grp[ATTP_MAX_HEADS]; };   // head -> index of its KV head's part of the transposed scratch
 struct AttpVtSrc { uint32_t vb[ATTP_MAX_HEADS], kb[ATTP_MAX_HEADS]; };  // group -> bases of its V and K cache (element offsets in the map)
 
+// A workgroup per tile of 32 rows and KV head; D / 2 threads take V, as many K, with eight 16-byte loads each that wait for
+// nothing (rows past the end read the last one and are then put to zero: a condition around each load made every one wait for
+// the one before, and a V value was a load of its own).  Latency bounds the launch where few KV heads leave few workgroups:
+// 700 rows of 1 head of 256 12.4 us before, 4.6 now; of 8 heads of 128, 1877 rows 8.9 and 5.8, 4024 rows 11.7 and 9.9 (6.8 at a
+// large copy's rate).
 template <int D>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(D)
 k_kv_tile_arrange(const __half* kv, uint64_t kv_shift, const AttpVtSrc src, uint32_t nkeys, uint32_t tiles, uint4* vt, uint4* kt) {
-  constexpr uint32_t NB = D / 16, KS = D / 32;
+  constexpr uint32_t NB = D / 16, KS = D / 32, Q = D / 8;
   const uint32_t T = blockIdx.x, grp = blockIdx.y;
-  const unsigned short* v = (const unsigned short*)(kv + ((uint64_t)src.vb[grp] - kv_shift));
-  for (uint32_t idx = threadIdx.x; idx < NB * 64u; idx += 256u) {
-    const uint32_t b = idx >> 6, g = (idx >> 4) & 3u, n = idx & 15u;
-    uint32_t w[4];
+  u4p_t x[8];
+  if (threadIdx.x < D / 2u) {
+    // V: eight rows by eight dims, turned over: dims c .. c + 7 of one g are consecutive pieces
+    const u4p_t* v = (const u4p_t*)(kv + ((uint64_t)src.vb[grp] - kv_shift));
+    const uint32_t c = threadIdx.x % Q, g = threadIdx.x / Q;
 #pragma unroll
     for (uint32_t j = 0; j < 8; j++) {
       const uint32_t key = 32u * T + (j < 4u ? 4u * g + j : 16u + 4u * g + (j - 4u));
-      const uint32_t x = key < nkeys ? (uint32_t)v[(uint64_t)key * D + 16u * b + n] : 0u;
-      if (j & 1u) w[j >> 1] |= x << 16; else w[j >> 1] = x;
+      x[j] = v[(uint64_t)min(key, nkeys - 1u) * Q + c];
+      if (key >= nkeys) x[j] = (u4p_t)(0u);
     }
-    vt[((((uint64_t)grp * tiles + T) * NB + b) * 4u + g) * 16u + n] = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-  // K: piece (step st, half kb, lane (g, n)) = dims 32 st + 8 g .. + 7 of row 32 T + 16 kb + n (rows past the end: zeros)
-  const uint4* k = (const uint4*)(kv + ((uint64_t)src.kb[grp] - kv_shift));
-  for (uint32_t idx = threadIdx.x; idx < 2u * KS * 64u; idx += 256u) {
-    const uint32_t st = idx >> 7, kb = (idx >> 6) & 1u, g = (idx >> 4) & 3u, n = idx & 15u;
-    const uint32_t key = 32u * T + 16u * kb + n;
-    kt[((uint64_t)grp * tiles + T) * (2u * KS * 64u) + idx] =
-        key < nkeys ? k[(uint64_t)key * (D / 8) + 4u * st + g] : make_uint4(0u, 0u, 0u, 0u);
+    u4p_t* out = (u4p_t*)vt + ((((uint64_t)grp * tiles + T) * NB + c / 2u) * 4u + g) * 16u + (c & 1u) * 8u;
+#pragma unroll
+    for (uint32_t d = 0; d < 8; d++) {
+      u4p_t w;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t lo = x[2 * j][d / 2u], hi = x[2 * j + 1][d / 2u];
+        w[j] = d & 1u ? lo >> 16 | (hi & 0xFFFF0000u) : (lo & 0xFFFFu) | hi << 16;
+      }
+      out[d] = w;
+    }
+  } else {
+    // K: piece (step st, half kb, lane (g, n)) = dims 32 st + 8 g .. + 7 of row 32 T + 16 kb + n
+    const u4p_t* k = (const u4p_t*)(kv + ((uint64_t)src.kb[grp] - kv_shift));
+    u4p_t* out = (u4p_t*)kt + ((uint64_t)grp * tiles + T) * (2u * KS * 64u);
+    const uint32_t i0 = threadIdx.x - D / 2u;
+#pragma unroll
+    for (uint32_t j = 0; j < 8; j++) {
+      const uint32_t idx = i0 + j * (D / 2u), st = idx >> 7, kb = (idx >> 6) & 1u, g = (idx >> 4) & 3u, n = idx & 15u;
+      const uint32_t key = 32u * T + 16u * kb + n;
+      x[j] = k[(uint64_t)min(key, nkeys - 1u) * Q + 4u * st + g];
+      if (key >= nkeys) x[j] = (u4p_t)(0u);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 8; j++) out[i0 + j * (D / 2u)] = x[j];
   }
 }
 
@@ -538,26 +561,55 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
 }
 
 // The runs of keys of a split launch, brought to their common maximum and added up in order (a run that a query sees
-// nothing of has the maximum -1e30: its factor is exactly 0).  Four values per thread, a row of the grid per token.
+// nothing of has the maximum -1e30: its factor is exactly 0).  Four values per thread, a row of the grid per token.  Bound by
+// latency: the runs are asked for eight at a time, the first eight before the maximum is known (past the last run the last one
+// again, with no part in the sum).  24 tokens of 32 heads of 128, 16 runs: 8.0 us with four at a time after it, 4.1 so.
 __global__ void __launch_bounds__(256)
 k_attn_prefill_join(const float* __restrict__ part, float* out, const AttpBases bs, uint32_t H, uint32_t D, uint32_t m, uint32_t splits,
                     uint32_t o_stride) {
+  constexpr uint32_t NS = 8;
   const uint32_t i = (blockIdx.x * 256u + threadIdx.x) * 4u, t = blockIdx.y;
   if (i >= H * D) return;
   const uint32_t head = i / D, d = i % D;
-  const float* const ms = part + (uint64_t)splits * H * m * D;
+  const float2* const ms = (const float2*)(part + (uint64_t)splits * H * m * D) + (uint64_t)head * m + t;
+  const float* const rows = part + ((uint64_t)head * m + t) * D + d;                 // (rows of D floats from the start of the buffer: 16-byte aligned)
+  const uint64_t step = (uint64_t)H * m;
+  float2 ml[NS];
+  f4p_t v[NS];
+  const auto ask = [&](uint32_t s0) {
+#pragma unroll
+    for (uint32_t j = 0; j < NS; j++) {
+      const uint32_t s = min(s0 + j, splits - 1u);
+      ml[j] = ms[s * step];
+      v[j] = *(const f4p_t*)(rows + s * step * D);
+    }
+  };
+  ask(0);
   float M = ATTP_NEG;
-  for (uint32_t s = 0; s < splits; s++) M = fmaxf(M, ms[2 * (((uint64_t)s * H + head) * m + t)]);
+#pragma unroll
+  for (uint32_t j = 0; j < NS; j++) M = fmaxf(M, ml[j].x);
+  for (uint32_t s0 = NS; s0 < splits; s0 += NS) {
+    float x[NS];
+#pragma unroll
+    for (uint32_t j = 0; j < NS; j++) x[j] = ms[min(s0 + j, splits - 1u) * step].x;
+#pragma unroll
+    for (uint32_t j = 0; j < NS; j++) M = fmaxf(M, x[j]);
+  }
   float L = 0.f;
   f4p_t o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (uint32_t s = 0; s < splits; s++) {
-    const uint64_t row = ((uint64_t)s * H + head) * m + t;
-    const float f = __builtin_amdgcn_exp2f(ms[2 * row] - M);
-    const f4p_t v = *(const f4p_t*)(part + row * D + d);              // (rows of D floats from the start of the buffer: 16-byte aligned)
-    L = fmaf(ms[2 * row + 1], f, L);
+  for (uint32_t s0 = 0;;) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = fmaf(v[k], f, o[k]);
+    for (uint32_t j = 0; j < NS; j++) {
+      const float f = __builtin_amdgcn_exp2f(ml[j].x - M);
+      if (s0 + j < splits) {
+        L = fmaf(ml[j].y, f, L);
+#pragma unroll
+        for (int k = 0; k < 4; k++) o[k] = fmaf(v[j][k], f, o[k]);
+      }
+    }
+    s0 += NS;
+    if (s0 >= splits) break;
+    ask(s0);
   }
   float* dst = out + (uint64_t)bs.o[head] + (uint64_t)t * o_stride + d;
   const float il = 1.0f / L;
@@ -688,7 +740,7 @@ size_t launch_attn_chunk(const std::vector<PendOp>& q, size_t i, int* rc) {
   } while (0)
 #define APM(DD)                                                                                                   \
   do {                                                                                                            \
-    k_kv_tile_arrange<DD><<<dim3(tiles, n_grp), 256, 0, g.stream>>>(mp->kv16, mp->kv_start, src, seq_last, tiles, g_vt, g_kt); \
+    k_kv_tile_arrange<DD><<<dim3(tiles, n_grp), DD, 0, g.stream>>>(mp->kv16, mp->kv_start, src, seq_last, tiles, g_vt, g_kt); \
     const dim3 gr_(n_quads * n_tt * splits);                                                                      \
     if (wph == 2 && DD <= 128) {   /* (D = 256 needs more registers than two waves per SIMD have) */              \
       constexpr int D2_ = DD <= 128 ? DD : 128;                                                                   \
