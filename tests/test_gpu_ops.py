@@ -477,6 +477,30 @@ def test_rope_append_rows_equals_rotations_and_row_copies(hip, n_tok, n_seq, Hq,
     assert np.array_equal(read(hip, 0, 0, total).view(np.uint32), got[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n_tok,n_seq,Hq,Hk,D,pos0", [(3, 2, 32, 8, 256, 5), (2, 1, 3, 1, 6, 0), (1, 33, 5, 2, 8, 1), (2, 1, 1, 1, 2, 3), (4, 1, 40, 12, 72, 2)])
+def test_rope_append_rows_of_any_start(hip, n_tok, n_seq, Hq, Hk, D, pos0, shift):
+    """Rows that start on four values and rows that do not, more pairs than a workgroup takes at once and fewer than it has threads."""
+    rng = np.random.default_rng(D)
+    cap, rows = pos0 + n_tok + 1, n_tok * n_seq
+    qs, ks, vs = Hq * D, Hk * D + 4, Hk * D
+    q0 = shift
+    k0, v0 = q0 + rows * qs, q0 + rows * (qs + ks)
+    c0, per = v0 + rows * vs, 2 * Hk * cap * D
+    x = rng.standard_normal(c0 + n_seq * per).astype(np.float32)
+    kb = [c0 + s * per for s in range(n_seq)]
+    out = []
+    for g in (hip, oracle.init()):
+        note(f"rope append {n_tok} x {n_seq}, {Hq} + {Hk} heads of {D}, shift {shift}")
+        f32map(g, 0, x.size, x)
+        g.kv_cache_fp16(0, c0, n_seq * per)
+        g.rope_append_rows_dev(0, q0, qs, Hq, k0, ks, Hk, v0, vs, D, n_tok, kb, [k + Hk * cap * D for k in kb], cap * D, pos0, 1e4, rotate=True)
+        out.append(read(g, 0, 0, x.size))
+    assert rel_l2(out[0][:c0], out[1][:c0]) < 1e-6
+    assert np.array_equal(out[0][k0 + rows * ks:c0], x[k0 + rows * ks:c0])
+    assert np.abs(out[0][c0:] - out[1][c0:]).max() <= 2.0 ** -10 * np.abs(x).max() * 1.5 + 1e-7     # one fp16 step where the rotations round apart
+
+
 @pytest.mark.parametrize("B,Hq,Hk,D", [(8, 32, 8, 128), (5, 16, 2, 64), (3, 32, 8, 128)])
 def test_wide_rotation_takes_few_key_rows_and_copies_along(hip, monkeypatch, B, Hq, Hk, D):
     """One token of B sequences: more than 64 Q rows beside at most 64 K rows and copies still rotate and append in one launch, and
