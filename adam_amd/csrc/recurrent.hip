@@ -272,6 +272,8 @@ struct ChunkDims { uint32_t Dp, Vp, n_chunks; };
 __host__ __device__ inline uint32_t chunk_floats(uint32_t Dp, uint32_t Vp) { return 49u * Dp + 256u + 16u * Vp; }
 
 // Columns of q and k (a thread each) run through their convolution in registers, then those of v and of the decay.
+// Exponentials and LDS reads bound it; four workgroups a compute unit (by LDS) hide one another's barriers as long as a thread has
+// at most 128 registers (2048 tokens in 32 heads of 128: 194 us with 201 registers, two workgroups; 143 with 69).
 template <int TM>
 __global__ void __launch_bounds__(256)
 k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* __restrict__ act, const float* __restrict__ state,
@@ -387,6 +389,7 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
       const uint32_t os = is_u ? cd.Vp : cd.Dp;
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {
+        if (!(t & 3)) asm volatile("" ::: "memory");         // four rows of M at a time: all of them would take 136 registers
         float a = 0.f;
 #pragma unroll
         for (int r = 0; r <= t; r++) a = fmaf(M[t][r], y[r], a);
