@@ -348,7 +348,7 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
       }
     }
     A[t][r] = r < t ? a * ik[t] * ik[r] * beta[t] : 0.f;
-    oB[t * 16u + r] = b * iq[t] * ik[r];
+    oB[place16(t, r)] = b * iq[t] * ik[r];
   }
   __syncthreads();
   if (tid < CH) {                                            // column tid of the inverse, forward substitution
@@ -368,15 +368,15 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
       const uint32_t d = i;
       const bool in = d < D;
       const float gl = in ? G[15u * P + d] : 0.f;
-      float kt[CH];
+      float qt[CH], kt[CH];
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {
         const float lg = in ? G[t * P + d] : 0.f;
-        oQ[t * cd.Dp + d] = in ? qs[t * P + d] * iq[t] * __builtin_amdgcn_exp2f(lg) : 0.f;
+        qt[t] = in ? qs[t * P + d] * iq[t] * __builtin_amdgcn_exp2f(lg) : 0.f;
         kt[t] = in ? ks[t * P + d] * ik[t] * __builtin_amdgcn_exp2f(gl - lg) : 0.f;
       }
-#pragma unroll
-      for (int t = 0; t < (int)CH; t += 4) *(f4_t*)(oK + d * 16u + t) = (f4_t){kt[t], kt[t + 1], kt[t + 2], kt[t + 3]};
+      store_rows(oQ, d, qt);
+      store_cols(oK, d, kt);
       oG[d] = __builtin_amdgcn_exp2f(gl);
     } else {
       const bool is_u = i >= 2u * cd.Dp;
@@ -385,16 +385,16 @@ k_delta_prep(const DSpec s, uint32_t dec_out, uint32_t dec_stride, const float* 
 #pragma unroll
       for (int t = 0; t < (int)CH; t++)
         y[t] = is_u ? (d < V ? vs[t * cd.Vp + d] : 0.f) : d < D ? ks[t * P + d] * ik[t] * __builtin_amdgcn_exp2f(G[t * P + d]) : 0.f;
-      float* o = is_u ? oU + d : oW + d;
-      const uint32_t os = is_u ? cd.Vp : cd.Dp;
+      float o[CH];
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {
         if (!(t & 3)) asm volatile("" ::: "memory");         // four rows of M at a time: all of them would take 136 registers
         float a = 0.f;
 #pragma unroll
         for (int r = 0; r <= t; r++) a = fmaf(M[t][r], y[r], a);
-        o[t * os] = a;
+        o[t] = a;
       }
+      if (is_u) store_cols(oU, d, o); else store_rows(oW, d, o);
     }
   }
 }
@@ -437,7 +437,8 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 #pragma unroll
     for (int t = 0; t < (int)CH; t++) y[t] = x[(uint64_t)min(c0 + t, m - 1u) * s.x_stride + s.x_v + h * V + min(v, V - 1u)];
 #pragma unroll
-    for (int t = 0; t < (int)CH; t++) oU[t * cd.Vp + v] = c0 + t < m && v < V ? y[t] : 0.f;
+    for (int t = 0; t < (int)CH; t++) y[t] = c0 + t < m && v < V ? y[t] : 0.f;
+    store_cols(oU, v, y);
   }
   __syncthreads();
   for (uint32_t i = tid; i < 2u * CH * half; i += 256u) {     // turn the pairs in place
@@ -457,17 +458,17 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
       for (uint32_t d = 0; d < D; d++) b = fmaf(qs[t * P + d], ks[r * P + d], b);
       b *= pw[t - r];
     }
-    oB[t * 16u + r] = b;
+    oB[place16(t, r)] = b;
   }
   for (uint32_t d = tid; d < cd.Dp; d += 256u) {
-    float kt[CH];
+    float qt[CH], kt[CH];
 #pragma unroll
     for (int t = 0; t < (int)CH; t++) {
-      oQ[t * cd.Dp + d] = d < D ? qs[t * P + d] * pw[t + 1] : 0.f;
+      qt[t] = d < D ? qs[t * P + d] * pw[t + 1] : 0.f;
       kt[t] = (d < D && (uint32_t)t < L) ? ks[t * P + d] * pw[L - 1u - min((uint32_t)t, L - 1u)] : 0.f;
     }
-#pragma unroll
-    for (int t = 0; t < (int)CH; t += 4) *(f4_t*)(oK + d * 16u + t) = (f4_t){kt[t], kt[t + 1], kt[t + 2], kt[t + 3]};
+    store_rows(oQ, d, qt);
+    store_cols(oK, d, kt);
     oG[d] = pw[L];
   }
 }
@@ -483,23 +484,21 @@ struct ScanArgs {
   uint32_t kv_heads, taps, conv_off, x, x_stride;     // delta: the convolution's ring is brought up to date here
   uint32_t seq_stride;                                // of the state; grid z: the sequence, its rows m z .. of the activations
 };
-template <int NT> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], b; float u[4]; };
+template <int NT> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], b, u; };
 
 template <bool DELTA, int NT>
-__device__ __forceinline__ void load_ops(ChunkOps<NT>& o, const float* blk, const ChunkDims& cd, uint32_t wave, uint32_t c, uint32_t kg,
-                                         uint32_t v0) {
+__device__ __forceinline__ void load_ops(ChunkOps<NT>& o, const float* blk, const ChunkDims& cd, uint32_t wave, uint32_t lane, uint32_t v0) {
   const float *pQ = blk + CH * cd.Dp, *pK = pQ + CH * cd.Dp, *pB = pK + CH * cd.Dp, *pU = pB + 256u, *pG = pU + CH * cd.Vp;
 #pragma unroll
   for (int j = 0; j < NT; j++) {
-    const uint32_t d0 = (wave * NT + j) * 16u;
-    if (DELTA) o.w[j] = *(const f4_t*)(blk + c * cd.Dp + d0 + 4u * kg);
-    o.q[j] = *(const f4_t*)(pQ + c * cd.Dp + d0 + 4u * kg);
-    o.k[j] = *(const f4_t*)(pK + (d0 + c) * 16u + 4u * kg);
-    o.gl[j] = *(const f4_t*)(pG + d0 + 4u * kg);
+    const uint32_t T = wave * NT + j, at = T * 256u + lane * 4u;
+    if (DELTA) o.w[j] = *(const f4_t*)(blk + at);
+    o.q[j] = *(const f4_t*)(pQ + at);
+    o.k[j] = *(const f4_t*)(pK + at);
+    o.gl[j] = *(const f4_t*)(pG + T * 16u + (lane >> 4) * 4u);
   }
-  o.b = *(const f4_t*)(pB + c * 16u + 4u * kg);
-#pragma unroll
-  for (int i = 0; i < 4; i++) o.u[i] = pU[(4u * kg + i) * cd.Vp + v0 + c];
+  o.b = *(const f4_t*)(pB + lane * 4u);
+  o.u = *(const f4_t*)(pU + v0 * 16u + lane * 4u);
 }
 
 template <bool DELTA, int NT>
@@ -528,7 +527,7 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
   }
   const uint32_t n = a.cd.n_chunks;
   // the operands of the chunk two ahead, asked for on every path (past the end: the last one's again)
-  const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, c, kg, v0); };
+  const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, lane, v0); };
   const auto chunk = [&](const ChunkOps<NT>& cur, uint32_t ci, f4_t (*pb)[4][64]) {
     f4_t p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0};
 #pragma unroll
@@ -541,7 +540,7 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
     if (DELTA) pb[0][wave][lane] = p1;
     pb[1][wave][lane] = p2;
     __syncthreads();
-    f4_t u = {cur.u[0], cur.u[1], cur.u[2], cur.u[3]};
+    f4_t u = cur.u;
     if (DELTA) {
       const f4_t* r = &pb[0][0][0];
       u -= (r[lane] + r[64 + lane]) + (r[128 + lane] + r[192 + lane]);

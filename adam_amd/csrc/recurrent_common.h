@@ -81,4 +81,38 @@ __device__ __forceinline__ void conv_silu_rows(const float* x, uint32_t x_stride
   for (int t = 0; t < (int)CH; t++) put(t, y[t]);
 }
 
+// Operands of the walk over the chunks: tiles of 16 x 16 in the order in which a wave's lanes take them, four consecutive floats a
+// lane, so that a load is 1 KB in one piece.  In rows (element (t, d) by t) a quad of lanes lay in four rows, each a request of its
+// own to the L1: a chunk's operands were 2200 clocks of requests of a compute unit, more than the chain they feed.
+//   rows of tokens by d (left operand, tokens its rows):  d / 16, d / 4 % 4, t, d % 4
+//   rows of d by tokens (left operand, d its rows; also a right operand, d its columns):  d / 16, t / 4, d % 16, t % 4
+__device__ __forceinline__ uint32_t place16(uint32_t row, uint32_t k) { return (k >> 2) * 64u + row * 4u + (k & 3u); }   // of one tile
+// A thread has the CH tokens of its d; the quad's four lanes turn theirs over four by four.  Whole quads, d % 4 a lane's place in its own.
+__device__ __forceinline__ void store_rows(float* o, uint32_t d, const float (&y)[CH]) {
+  const bool odd = d & 1u, high = d & 2u;
+  float* to = o + (d >> 4) * 256u + ((d >> 2) & 3u) * 64u;
+#pragma unroll
+  for (uint32_t b = 0; b < CH; b += 4u) {
+    float r[4] = {y[b], y[b + 1], y[b + 2], y[b + 3]};
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(odd ? r[i] : r[i + 1]), 0xB1, 0xF, 0xF, false));
+      r[i] = odd ? got : r[i];
+      r[i + 1] = odd ? r[i + 1] : got;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(high ? r[i] : r[i + 2]), 0x4E, 0xF, 0xF, false));
+      r[i] = high ? got : r[i];
+      r[i + 2] = high ? r[i + 2] : got;
+    }
+    *(f4_t*)(to + (b + (d & 3u)) * 4u) = (f4_t){r[0], r[1], r[2], r[3]};
+  }
+}
+__device__ __forceinline__ void store_cols(float* o, uint32_t d, const float (&y)[CH]) {
+  float* to = o + (d >> 4) * 256u + (d & 15u) * 4u;
+#pragma unroll
+  for (uint32_t b = 0; b < CH; b += 4u) *(f4_t*)(to + b * 16u) = (f4_t){y[b], y[b + 1], y[b + 2], y[b + 3]};
+}
+
 }  // namespace adamah

@@ -117,17 +117,17 @@ k_space_prep(const SSpec s, const float* __restrict__ act, const float* __restri
 #pragma unroll 4
         for (uint32_t d = 0; d < N; d++) a = fmaf(cs[t * P + d], bs[r * P + d], a);
       }
-      oD[t * 16u + r] = a;
+      oD[place16(t, r)] = a;
     }
     for (uint32_t d = tid; d < sd.Np; d += 256u) {
-      float b[CH];
+      float c[CH], b[CH];
 #pragma unroll
       for (int t = 0; t < (int)CH; t++) {
-        oC[t * sd.Np + d] = d < N ? cs[t * P + d] : 0.f;
+        c[t] = d < N ? cs[t * P + d] : 0.f;
         b[t] = d < N ? bs[t * P + d] : 0.f;
       }
-#pragma unroll
-      for (int t = 0; t < (int)CH; t += 4) *(f4_t*)(oB + d * 16u + t) = (f4_t){b[t], b[t + 1], b[t + 2], b[t + 3]};
+      store_rows(oC, d, c);
+      store_cols(oB, d, b);
     }
     return;
   }
@@ -142,11 +142,9 @@ k_space_prep(const SSpec s, const float* __restrict__ act, const float* __restri
     if (tid < CH) { dt[t] = d; lg[t] = -fminf(expf(act[s.a_log + h]) * d, NO_MEMORY) * 1.44269504f; }
   }
   for (uint32_t i = tid; i < sd.Vp; i += 256u) {
-    if (i < V) conv(h * V + i, [&](int t, float v) { oX[t * sd.Vp + i] = v; });
-    else {
-#pragma unroll
-      for (int t = 0; t < (int)CH; t++) oX[t * sd.Vp + i] = 0.f;
-    }
+    float y[CH] = {};
+    if (i < V) conv(h * V + i, [&](int t, float v) { y[t] = v; });
+    store_cols(oX, i, y);
   }
   __syncthreads();
   // Decays between two tokens from the logarithms between them: the difference of two long sums would keep the rounding of
@@ -156,30 +154,29 @@ k_space_prep(const SSpec s, const float* __restrict__ act, const float* __restri
 #pragma unroll
   for (uint32_t i = 0; i < CH; i++) { l += i > r && i <= t ? lg[i] : 0.f; e += i <= r ? lg[i] : 0.f; }
   l = r <= t ? __builtin_amdgcn_exp2f(l) * dt[r] : 0.f;
-  oM[t * 16u + r] = l;
+  oM[place16(t, r)] = l;
   if (t == CH - 1u) { oE[r] = __builtin_amdgcn_exp2f(e); oG[r] = l; }
 }
 
 // Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
 // is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.
-template <int NT> struct SpaceOps { f4_t c[NT], b[NT], cb, m, e, g; float u[4], last; };
+template <int NT> struct SpaceOps { f4_t c[NT], b[NT], cb, m, e, g, u; float last; };
 template <int NT>
-__device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const float* hb, const SpaceDims& sd, uint32_t wave, uint32_t c,
-                                         uint32_t kg, uint32_t v0) {
+__device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const float* hb, const SpaceDims& sd, uint32_t wave, uint32_t lane,
+                                         uint32_t v0) {
   const float *pB = gb + 16u * sd.Np, *pD = pB + 16u * sd.Np, *pM = hb + 16u * sd.Vp, *pE = pM + 256u, *pG = pE + 16u;
 #pragma unroll
   for (int j = 0; j < NT; j++) {
-    const uint32_t d0 = (wave * NT + j) * 16u;
-    o.c[j] = *(const f4_t*)(gb + c * sd.Np + d0 + 4u * kg);
-    o.b[j] = *(const f4_t*)(pB + (d0 + c) * 16u + 4u * kg);
+    const uint32_t at = (wave * NT + j) * 256u + lane * 4u;
+    o.c[j] = *(const f4_t*)(gb + at);
+    o.b[j] = *(const f4_t*)(pB + at);
   }
-  o.cb = *(const f4_t*)(pD + c * 16u + 4u * kg);
-  o.m = *(const f4_t*)(pM + c * 16u + 4u * kg);
-  o.e = *(const f4_t*)(pE + 4u * kg);
-  o.g = *(const f4_t*)(pG + 4u * kg);
+  o.cb = *(const f4_t*)(pD + lane * 4u);
+  o.m = *(const f4_t*)(pM + lane * 4u);
+  o.e = *(const f4_t*)(pE + (lane >> 4) * 4u);
+  o.g = *(const f4_t*)(pG + (lane >> 4) * 4u);
   o.last = pE[15];
-#pragma unroll
-  for (int i = 0; i < 4; i++) o.u[i] = hb[(4u * kg + i) * sd.Vp + v0 + c];
+  o.u = *(const f4_t*)(hb + v0 * 16u + lane * 4u);
 }
 
 template <int NT>
@@ -212,7 +209,7 @@ k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float
   // the wait at its end was for everything asked for (2048 tokens in 64 heads of 64 by 128: 162 us, now 109).
   const auto ask = [&](SpaceOps<NT>& o, uint32_t ci) {
     const uint64_t at = min(ci, n - 1u);
-    load_ops<NT>(o, gb + at * gs, hb + at * hs, sd, wave, c, kg, v0);
+    load_ops<NT>(o, gb + at * gs, hb + at * hs, sd, wave, lane, v0);
   };
   const auto chunk = [&](const SpaceOps<NT>& cur, uint32_t ci, f4_t (*pb)[64]) {
     f4_t p = {0, 0, 0, 0};
