@@ -135,13 +135,16 @@ k_topk_merge(float* data, const float* __restrict__ part_v, const uint32_t* __re
 // the candidates that agree with the digits fixed so far, a suffix scan over the bins finds the bin the k-th falls in --
 // and everything at or above that key is gathered and put in order by counting.  One workgroup of 1024 threads, the
 // values in registers (at most 40 per thread).  Same results as the rounds (tests/test_gpu_sampling.py); the partial
-// lists of the sampled LM head (40960 candidates, k = 40): 145 -> 20 us.
+// lists of the sampled LM head (40960 candidates, k = 40) take 145 us in rounds; here 59 with each load under a condition and one
+// count a bin, 41 with loads on every path, TSEL_ASK at a time, and four counts a bin (the values share few bins of the first
+// passes, and a wave's counts of one address go one behind the other).
 #define TSEL_THREADS 1024u
 #define TSEL_PER 40u
+#define TSEL_ASK 20u
 __global__ void __launch_bounds__(1024)
 k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __restrict__ li, const uint32_t* __restrict__ lv,
               uint32_t n, uint32_t k, uint64_t n_elems) {
-  __shared__ uint32_t hist[2048];
+  __shared__ uint4 hist[2048];                  // a bin's counts of the lanes with the same two last bits
   __shared__ uint32_t wtot[16];
   __shared__ uint32_t sel_bin, sel_rem, n_win;
   __shared__ float win_v[SMP_MAX];
@@ -150,15 +153,23 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
   const uint32_t per = (n + TSEL_THREADS - 1u) / TSEL_THREADS;
   uint32_t vk[TSEL_PER];   // orderable value bits of candidate u * 1024 + tid
 #pragma unroll
-  for (uint32_t u0 = 0; u0 < TSEL_PER; u0 += 8u) {   // eight at a time: the loads' temporaries stay within the budget
+  for (uint32_t u0 = 0; u0 < TSEL_PER; u0 += TSEL_ASK) {
+    if (u0 < per) {
+      uint32_t l[TSEL_ASK];
+      float x[TSEL_ASK];
 #pragma unroll
-    for (uint32_t u = u0; u < u0 + 8u; u++) {
-      const uint32_t i = u * TSEL_THREADS + tid;
-      float x = SMP_NEG_INF;
-      if (u < per && i < n) { const uint32_t l = ls[i]; if (l < n_elems) x = data[l]; }
-      x = x != x ? SMP_NEG_INF : x;
-      const uint32_t b = __float_as_uint(x);
-      vk[u] = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+      for (uint32_t j = 0; j < TSEL_ASK; j++) l[j] = ls[min((u0 + j) * TSEL_THREADS + tid, n - 1u)];
+#pragma unroll
+      for (uint32_t j = 0; j < TSEL_ASK; j++) x[j] = data[min((uint64_t)l[j], n_elems - 1u)];
+#pragma unroll
+      for (uint32_t j = 0; j < TSEL_ASK; j++) {
+        const float y = l[j] < n_elems && x[j] == x[j] ? x[j] : SMP_NEG_INF;
+        const uint32_t b = __float_as_uint(y);
+        vk[u0 + j] = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+      }
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < TSEL_ASK; j++) vk[u0 + j] = 0u;
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -171,7 +182,7 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
     const bool on_idx = pass >= 3u;             // passes 0..2: value bits 31..21, 20..10, 9..0; 3, 4: index bits 15..8, 7..0
     const uint32_t sh = pass == 0u ? 21u : pass == 1u ? 10u : pass == 3u ? 8u : 0u;
     const uint32_t bm = pass < 2u ? 2047u : pass == 2u ? 1023u : 255u;
-    hist[2u * tid] = 0u; hist[2u * tid + 1u] = 0u;
+    hist[2u * tid] = make_uint4(0u, 0u, 0u, 0u); hist[2u * tid + 1u] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     uint32_t inv = inv0, idx = tid;
     asm volatile("" : "+v"(inv), "+v"(idx));   // per pass, so that the 40 index digits are not all kept in registers
@@ -180,12 +191,13 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
       if (u < per && idx + u * TSEL_THREADS < n) {
         const uint32_t iv = inv - u * TSEL_THREADS;
         const bool in = on_idx ? (vk[u] == prefix && (iv & imask) == iprefix) : ((vk[u] & mask) == prefix);
-        if (in) atomicAdd(&hist[((on_idx ? iv : vk[u]) >> sh) & bm], 1u);
+        if (in) atomicAdd((uint32_t*)&hist[((on_idx ? iv : vk[u]) >> sh) & bm] + (tid & 3u), 1u);
       }
     }
     __syncthreads();
     // suffix sums over the bins (two per thread), top down: the bin in which the count reaches `remaining`
-    const uint32_t h0 = hist[2u * tid], h1 = hist[2u * tid + 1u], own = h0 + h1;
+    const uint4 c0 = hist[2u * tid], c1 = hist[2u * tid + 1u];
+    const uint32_t h0 = c0.x + c0.y + c0.z + c0.w, h1 = c1.x + c1.y + c1.z + c1.w, own = h0 + h1;
     uint32_t suf = own;   // inclusive suffix sum within the wave
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
