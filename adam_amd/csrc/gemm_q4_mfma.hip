@@ -854,8 +854,8 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
 #undef GEMM_FETCH
 
 // M <= 16 and many weight rows: the waves of a workgroup take 16 weight rows each and share ONE activation tile per
-// step of K, staged through LDS once for all of them (the K-split form above stages a tile per wave: the tile, both
-// planes of all 16 rows, is 7x the bytes of a wave's weights, and those requests to the L1, not HBM, set its pace).
+// step of K, staged through LDS once for all of them (the tile, both planes of all 16 rows, is 7x the bytes of a wave's
+// weights: fetched by every wave, those requests to the L1, not HBM, would set the pace).
 // A macro step is two steps of K (256 weights).  Registers hold rings of what is on its way: the workgroup's next
 // four activation macro tiles (a thread's share: one or two pieces per plane each) and each wave's weights of the next
 // four macro steps, so a CU keeps ~10 KB per wave in flight; LDS holds two macro tiles, one being read by the matrix

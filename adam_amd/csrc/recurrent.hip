@@ -475,7 +475,8 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 
 // ---- the walk over the chunks ---------------------------------------------------------------------------------------
 // A serial chain, so what counts is a chunk's latency: 2048 tokens in 32 heads of 128 took 236 us = 1.85 us a chunk with the
-// next one's operands under a condition (the wait at its end is for everything asked for), 144 so.
+// next one's operands under a condition (the wait at its end is for everything asked for), 157-170 so, 144 with the operands in
+// lane order (16 sequences of 12 tokens 54 and 39.5).
 // Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
 // is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.
 struct ScanArgs {
