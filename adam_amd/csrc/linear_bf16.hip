@@ -351,7 +351,8 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
 // The one-row head over NR rows at a time (their operand, float32, ready at X): the weights go by once instead of once a row, 32768 x
 // 4096 for 16 rows 697 us one by one.  Four matrix rows a wave, so that a value of x read from LDS meets four weights; a result's sums
 // are the one-row kernel's, in its order.  32768 x 4096 for eight rows 95 us (55 at a large copy's rate): multiply-adds and memory in
-// turn; 115 with loads, maxima and logits under conditions and the rows staged one load at a time.  Rows past the last are zeros; the logits at `out` are the row `kept`'s, if it is among them.
+// turn; 115 with loads, maxima and logits under conditions and the rows staged one load at a time.  Rows past the last are zeros;
+// the logits at `out` are the row `kept`'s, if it is among them.
 template <int NR>
 __global__ void __launch_bounds__(512)
 k_head_rows(const bf16_t* __restrict__ W, float* act, const LinSpec s, const float* __restrict__ X, uint32_t rows, uint32_t kept, uint32_t n_tasks,
