@@ -524,11 +524,15 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 //   * the NWV waves of a workgroup share R tiles of 16 weight rows and take every NWV-th step of K (128 columns) each, so a
 //     workgroup reads its activations once, and as many weight rows as a CU has share them.
 // Weights are asked for D steps ahead, activations DA.  The waves' tiles are summed through LDS in wave order.
-// What bounds it is the L1's rate for one tile of weights (96 clocks of it a step with one operand tile, of 175 measured) and the
-// vector work for four (75 instructions a step and tile, 36 of them unpacking): more steps ahead only cost their loads (8 rows, 28672
-// x 4096, one tile: 29 us two steps ahead, 45 four).  Before (a tile of activations staged by every wave, both planes apart):
-// 8 rows 4096 x 4096 6.7 -> 5.2 us, 6144 x 4096 10.4 -> 8.3, 4096 x 14336 16.7 -> 14.8, 13824 x 1152 9.0 -> 6.9; 24 rows 13.7 ->
-// 7.9, 19.2 -> 11.0, 39.1 -> 24, 15.2 -> 9.4, 28672 x 4096 48 -> 36; 32 rows 14.4 -> 9.3, 19.7 -> 12.7, 39.6 -> 29, 15.0 -> 10.7, 49.6 -> 40.
+// The weights come by ordinary loads: a step takes half a line of a row and another wave's step the other half, which it finds in
+// the L1.  Marked as read once, every line was asked of the L2 twice (8 rows, 4096 x 4096: 68,000 of 422,000 requests; the same
+// bytes from memory), and 8 rows took 6.0 us for 4096 x 4096 (5.0 so), 8.2 for 6144 x 4096 (7.2), 16.6 for 4096 x 14336 (14.2), 8.3
+// for 1152 x 6912 (6.15); 24 rows 8.6 (7.7), 11.7 (10.3), 26 (24), 13.0 (10.2).
+// What bounds it is the way from the L2 for one tile of weights (of a 128-column step 4 KB are activations, 1.2 KB weights) and the
+// vector work for four (75 instructions a step and tile, 36 of them unpacking).
+// us, rows ready, the K-split kernel before (a tile of activations staged by every wave, both planes apart) and this one: 8 rows
+// 4096 x 4096 6.5 and 5.0, 6144 x 4096 9.6 and 7.2, 4096 x 14336 16.3 and 14.2, 13824 x 1152 8.7 and 6.4; 24 rows 13.3 and 7.7, 18.5 and 10.3,
+// 39 and 24, 15.0 and 8.7, 28672 x 4096 48 and 32; 32 rows 13.2 and 8.8, 19.2 and 12.1, 39.6 and 28.9, 14.9 and 9.9, 50 and 37.
 // (segs.glu: tiles of a wave are gate, up, gate, up ...: the gated activation is stored from here.)
 template <int NT, int R, int NWV, int D, int DA>
 __global__ void __launch_bounds__(64 * NWV)
@@ -572,7 +576,7 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
     const uint8_t *wp = Wb + at * 16u, *dp = (const uint8_t*)(Db + at);
 #pragma unroll
     for (int r = 0; r < R; r++) {
-      qn[slot][r] = __builtin_nontemporal_load((const u4q_t*)(wp + (wo[r] << 4)));
+      qn[slot][r] = *(const u4q_t*)(wp + (wo[r] << 4));
       dn[slot][r] = *(const uint16_t*)(dp + (wo[r] << 1));
     }
   };
@@ -853,7 +857,7 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
 }
 #undef GEMM_FETCH
 
-// M <= 16 and many weight rows: the waves of a workgroup take 16 weight rows each and share ONE activation tile per
+// 9 .. 16 rows and many weight rows: the waves of a workgroup take 16 weight rows each and share ONE activation tile per
 // step of K, staged through LDS once for all of them (the tile, both planes of all 16 rows, is 7x the bytes of a wave's
 // weights: fetched by every wave, those requests to the L1, not HBM, would set the pace).
 // A macro step is two steps of K (256 weights).  Registers hold rings of what is on its way: the workgroup's next
@@ -1273,8 +1277,8 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 0
 // k_gemm_q4_ring<ma>, 0 the tiled kernel, over how many shares of K; -1 k_gemm_q4_rows.
 // 33 .. 64 rows: k_gemm_q4_rows where a CU has few tiles of 16 weight rows and K is not long, by its time for a round of tiles and
-// a 128-column step (48 rows: 4096 x 4096 12.5 us, tiled 20.8, 6144 x 4096 15.9 and 23.4; 4096 x 14336 38.7 and 33.0; 64 rows:
-// 28672 x 4096 73 and 64).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
+// a 128-column step (48 rows: 4096 x 4096 12.3 us, tiled 21.7, 6144 x 4096 14.9 and 23.8; 4096 x 14336 38.0 and 34.1; 64 rows:
+// 28672 x 4096 71.9 and 67.7).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
 // a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x
 // 2048: 23 -> 17 over four; 64 x 28672 x 2048 38 in one, 44 in four, 64 x 28672 x 4096 67 and 62).
 // More: the least of these estimates, in us, fitted to both kernels over 2900 plans of 65 .. 2049 rows by 512 .. 32000 x 128 ..
@@ -1390,10 +1394,11 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     keep();
     return check_launch();
   }
-  // at most 16 activation rows and workgroups of 128 weight rows for three quarters of the CUs: the form whose eight waves share an
-  // activation tile in LDS (28672 x 4096, 16 rows: 24.8 us, k_gemm_q4_rows 30.4; 8 rows: 24.4 and 24.1)
+  // 9 .. 16 activation rows and workgroups of 128 weight rows for three quarters of the CUs: the form whose eight waves share an
+  // activation tile in LDS (16 rows: 28672 x 4096 25.3 us, k_gemm_q4_rows 26.9, 65536 x 2048 25.5 and 33.0; 8 rows: 24.9 and 19.9,
+  // 25.1 and 21.3)
   const uint32_t wgs16 = cdiv(sg.glu ? N / 2 : N, sg.glu ? 64u : 128u);
-  if (mt == 1 && !sg.add && (uint64_t)wgs16 * 4 >= 3ull * cu && tuning("ADAMAH_GEMM_ROWS16", 1) != 0) {
+  if (form.tiles == 2 && !sg.add && (uint64_t)wgs16 * 4 >= 3ull * cu && tuning("ADAMAH_GEMM_ROWS16", 1) != 0) {
     k_gemm_q4_f16_rows16<8><<<dim3(wgs16, 1, n_ops), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst,
                                                                         dst, lb, lcd, g_scale_buf, sg);
     count_launch();
@@ -1402,7 +1407,7 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   }
   if (M <= 32 || plan.ma < 0) {
     // As many tiles of 16 weight rows to a workgroup as a CU has: one workgroup per CU reads its activations once (8 rows: 4096 x
-    // 4096 one tile 5.2 us, two 7.8; 6144 x 4096 two 8.2, four 12.7; 13824 x 1152 four 6.9, one 9.7).  One and two tiles
+    // 4096 one tile 4.9 us, two 6.8; 6144 x 4096 two 6.7, four 10.0; 13824 x 1152 four 6.4, one 9.2).  One and two tiles
     // of weights take the same number of waves, so that a stacked matrix has the same sums as its parts; eight where 16 waves
     // would not have the registers (three and more operand tiles, four tiles of weights)
     const uint32_t R = tiles16 <= cu && !sg.glu ? 1 : tiles16 <= 2 * cu || form.tiles > 4 ? 2 : 4;

@@ -352,7 +352,7 @@ def test_gated_activation_feeds_the_matmul_without_a_conversion_launch(hip, op, 
 
 
 @pytest.mark.parametrize("kind,op,M,K,F", [("q4", "swiglu", 16, 4096, 14336), ("q4", "geglu", 5, 256, 48), ("q8", "swiglu", 32, 512, 80),
-                                           ("q4", "swiglu", 16, 256, 40), ("q4", "geglu", 40, 256, 48)])
+                                           ("q4", "swiglu", 16, 256, 40), ("q4", "geglu", 40, 256, 48), ("q4", "swiglu", 8, 256, 12304)])
 def test_gated_activation_stored_by_the_stacked_gate_up_matmul(hip, kind, op, M, K, F):
     """gate = X Wg^T, up = X Wu^T (matrices back to back), act = GLU(gate, up), then a matmul over act, as a
     batched decode step issues them: for M <= 32 and F a multiple of 16 the stacked launch stores act as well
@@ -592,7 +592,7 @@ def test_tiles_in_runs_per_die(hip, monkeypatch, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(2, 16, 128), (3, 8209, 256), (8, 17, 384), (9, 5000, 128), (16, 8210, 640), (17, 40, 2176), (24, 8201, 128),
-                                   (25, 4113, 384), (32, 9000, 256), (33, 100, 128), (40, 4100, 1152), (48, 8200, 256), (49, 4090, 640), (64, 31, 4224)])
+                                   (25, 4113, 384), (32, 9000, 256), (6, 24700, 128), (33, 100, 128), (40, 4100, 1152), (48, 8200, 256), (49, 4090, 640), (64, 31, 4224)])
 def test_few_rows_on_every_operand_and_weight_tile(hip, M, N, K):
     """2 .. 64 activation rows: one to eight operand tiles of both planes, one, two and four tiles of weights to a workgroup, ragged
     in every one; fewer steps of K than waves, and numbers of steps that they do not share evenly.  Rows of very different size keep
