@@ -691,8 +691,12 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 
 // Q8_0 weights (the LM head of a lockstep batch) under at most 32 activation rows: the weights are read once and nothing is
 // reused, so the work is bound by how fast they stream.  The four waves of a workgroup share R tiles of 16 weight rows and
-// take every fourth step of K each; every wave stages its own activation tile (the first plane) into its own piece of LDS, so
-// no workgroup barrier sits in the K loop.  The partial tiles are summed in wave order at the end.
+// take every fourth step of K each; the partial tiles are summed in wave order at the end.
+// Lane group g wants block g of the step whole, piece j of it for instruction j: of the operand tiles those are 256 bytes in one
+// piece, so the first plane's go straight to registers, refilled behind the instructions that used them; a lane past the last row
+// reads that row again.  us, rows ready: staged through LDS a step ahead, whole tiles of both planes, 128256 x 4096 8 rows 128, 32 rows
+// 165, 16000 x 8192 40.8 and 57.5, 4096 x 4096 32 rows 14.1; so 114, 157, 32, 52, 10.3 (from rows of the first plane, staged: 114, 158,
+// 33.3, 51.8, 10.4).
 // The weights are blocks of 32 code bytes, w = d (code - 128): two 16-byte loads per block, bytes widened with a byte permute
 // into the fp16 pairs (1024 + code), then -1152 and d.  `lc` null: the result rows go to out[row * N + n] (a scratch buffer of
 // the caller).
@@ -704,13 +708,11 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
                      GemmSegs segs) {
   // (by_val bit 0 / 1: the weights' / the result's element offset of op 0 is b_val / c_val -- known on the host -- instead of
   // a load from lb / lc, which the first weight loads would have to wait for)
-  constexpr uint32_t NWV = 4u, BM = 16u * MT, ROWB = 272u, NP = 4u * MT;      // NP: pieces per lane and step
-  constexpr uint32_t TILE = BM * ROWB, PART = (NWV - 1u) * R * MT * 4u * 64u * 4u;
-  __shared__ __attribute__((aligned(16))) uint8_t xs_all[(NWV * TILE > PART) ? NWV * TILE : PART];
+  constexpr uint32_t NWV = 4u;
+  __shared__ float part[(NWV - 1u) * R * MT * 4u * 64u];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t r16 = lane & 15u, g = lane >> 4;
-  uint8_t* xs = xs_all + wave * TILE;
   const uint32_t op = blockIdx.z;
   const uint64_t c_off = (by_val & 2u) ? (uint64_t)c_val : lc ? (uint64_t)lc[op] : 0ull;
   const uint64_t gbase = ((by_val & 1u) ? (uint64_t)b_val : (uint64_t)lb[op]) >> 5;
@@ -737,30 +739,32 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
   DEQK_INIT(dk);
   const h2q_t off_q8 = {(_Float16)-1152.f, (_Float16)-1152.f};
 
-  // lane l, piece u: operand tile u / 4, block u % 4 of the step, the tile's row l % 16, piece l / 16 of the block (tiles past
-  // the last: clamped, not stored)
+  // (rows 16 t .. of the first plane; the grid has a tile of them for every t)
   const u4q_t* xp[MT];
 #pragma unroll
-  for (uint32_t t = 0; t < MT; t++) xp[t] = x + ((uint64_t)op * tiles + min(t, tiles - 1u)) * kw * 16u + lane;
-  u4q_t xn[NP], qn[R], qn2[R];
+  for (uint32_t t = 0; t < MT; t++) xp[t] = x + (((uint64_t)op * tiles + t) * kw + g * 4u) * 16u + min(r16, M - 1u - t * 16u);
+  u4q_t xn[MT][4], qn[R], qn2[R];
   _Float16 dn[R];
-#define GEMM_FETCH(kb_raw)                                                        \
-  do {                                                                            \
-    const uint32_t kb_ = min((kb_raw), nblk - 4u);                                \
-    _Pragma("unroll") for (int r = 0; r < R; r++) {                               \
-      const uint64_t gi = gbase + (uint64_t)nrow[r] * nblk + kb_ + lblk;          \
-      qn[r] = *(const u4q_t*)(W + (gi << 5));                                     \
-      qn2[r] = *(const u4q_t*)(W + (gi << 5) + 16);                               \
-      dn[r] = __builtin_bit_cast(_Float16, d16[gi]);                              \
-    }                                                                             \
-    _Pragma("unroll") for (uint32_t u = 0; u < NP; u++)                           \
-      xn[u] = xp[u >> 2][(uint64_t)(kb_ + (u & 3u)) * 64u];                       \
-  } while (0)
-  GEMM_FETCH(wave * 4u);
+  const auto fetch_w = [&](uint32_t kb) {
+    kb = min(kb, nblk - 4u);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const uint64_t gi = gbase + (uint64_t)nrow[r] * nblk + kb + lblk;
+      qn[r] = *(const u4q_t*)(W + (gi << 5));
+      qn2[r] = *(const u4q_t*)(W + (gi << 5) + 16);
+      dn[r] = __builtin_bit_cast(_Float16, d16[gi]);
+    }
+  };
+  const auto fetch_x = [&](uint32_t kb, int j) {
+    kb = min(kb, nblk - 4u);
+#pragma unroll
+    for (int t = 0; t < MT; t++) xn[t][j] = xp[t][(uint64_t)kb * 64u + (uint32_t)j * 16u];
+  };
+  fetch_w(wave * 4u);
+#pragma unroll
+  for (int j = 0; j < 4; j++) fetch_x(wave * 4u, j);
 
   for (uint32_t kb0 = wave * 4u; kb0 < nblk; kb0 += 4u * NWV) {
-#pragma unroll
-    for (uint32_t u = 0; u < NP; u++) *(u4q_t*)(xs + ((u >> 2) * 16u + r16) * ROWB + (u & 3u) * 64u + g * 16u) = xn[u];
     // the step's blocks and scales, moved to the lanes that consume them
     u4q_t q[R], q2[R];
     h2q_t d2[R];
@@ -775,8 +779,9 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
       const _Float16 dl = __builtin_bit_cast(_Float16, (uint16_t)dbits);
       d2[r] = (h2q_t){dl, dl};
     }
-    __builtin_amdgcn_wave_barrier();
-    GEMM_FETCH(kb0 + 4u * NWV);
+    fetch_w(kb0 + 4u * NWV);
+    asm volatile("" ::: "memory");                           // the loads stay here
+    __builtin_amdgcn_sched_barrier(0);
     // lane group g holds block g whole; instruction j takes code bytes 8j .. 8j+7 of each of the four blocks, scaled before
     // the product
 #pragma unroll
@@ -796,17 +801,15 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
         wq[r] = (u4q_t){o[0], o[1], o[2], o[3]};
       }
 #pragma unroll
-      for (int t = 0; t < MT; t++) {
-        const u4q_t ah = *(const u4q_t*)(xs + (t * 16u + r16) * ROWB + g * 64u + j * 16u);
+      for (int t = 0; t < MT; t++)
 #pragma unroll
-        for (int r = 0; r < R; r++) acc[r][t] = MFMA_F16(ah, wq[r], acc[r][t]);
-      }
+        for (int r = 0; r < R; r++) acc[r][t] = MFMA_F16(xn[t][j], wq[r], acc[r][t]);
+      fetch_x(kb0 + 4u * NWV, j);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_wave_barrier();
   }
   // sum the waves' tiles in wave order; wave 0 stores
-  __syncthreads();
-  float* part = (float*)xs_all;
   if (wave > 0) {
 #pragma unroll
     for (int r = 0; r < R; r++)
@@ -855,7 +858,6 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
       }
     }
 }
-#undef GEMM_FETCH
 
 // 9 .. 16 rows and many weight rows: the waves of a workgroup take 16 weight rows each and share ONE activation tile per
 // step of K, staged through LDS once for all of them (the tile, both planes of all 16 rows, is 7x the bytes of a wave's

@@ -88,7 +88,8 @@ def test_batched_matmul_other_layouts_take_generic_path(hip):
         assert rel_l2(run(hip, qt, x, scale=s, zp=z), run(oracle.init(), qt, x, scale=s, zp=z)) < TOL
 
 
-@pytest.mark.parametrize("M,N,K", [(16, 3000, 4096), (2, 64, 128), (23, 130, 256), (32, 1000, 1152)])
+@pytest.mark.parametrize("M,N,K", [(16, 3000, 4096), (2, 64, 128), (23, 130, 256), (32, 1000, 1152), (3, 16399, 128), (9, 33, 640), (12, 16400, 384),
+                                   (17, 16385, 256), (31, 16389, 640)])
 def test_batched_q8_matmul_matches_oracle(hip, M, N, K):
     """Up to 32 rows over Q8_0 blocks take the matrix cores as well (the LM head of a lockstep batch)."""
     rng = np.random.default_rng(M + N + K)
