@@ -519,7 +519,10 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 // 2 .. 64 activation rows: the weights are read once, so what counts is how fast they stream, and what stands in its way is
 // the activations, of which a 16-row operand of 32 columns is 1 KB beside 288 bytes of weights.  So
 //   * the rows' two planes are stacked: 2 M operand rows (xh of every row, then xl), NT tiles of 16, one instruction per tile and
-//     block -- 8 rows fill one tile, 24 rows three; the planes' sums are added at the end;
+//     block -- 8 rows fill one tile, 24 rows three; the planes' sums are added at the end.  9 .. 16 rows (PAIR): a tile a plane, and
+//     both instructions of a block go to one sum;
+//   * one tile has 4, 8 or 16 rows in memory, two as many as there are in fours: every CU reads them all, and over long K that is what
+//     counts (9 rows, 4096 x 14336: 19.7 us with both planes in stacked tiles of 16, 16.1 so; 2 rows 14.2 and 10.4);
 //   * operands go from memory to registers in the instruction's layout, without LDS: a wave reads 16 rows x 64 bytes at a time;
 //   * the NWV waves of a workgroup share R tiles of 16 weight rows and take every NWV-th step of K (128 columns) each, so a
 //     workgroup reads its activations once, and as many weight rows as a CU has share them.
@@ -532,18 +535,21 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 // vector work for four (75 instructions a step and tile, 36 of them unpacking).
 // us, rows ready, the K-split kernel before (a tile of activations staged by every wave, both planes apart) and this one: 8 rows
 // 4096 x 4096 6.5 and 5.0, 6144 x 4096 9.6 and 7.2, 4096 x 14336 16.3 and 14.2, 13824 x 1152 8.7 and 6.4; 24 rows 13.3 and 7.7, 18.5 and 10.3,
-// 39 and 24, 15.0 and 8.7, 28672 x 4096 48 and 32; 32 rows 13.2 and 8.8, 19.2 and 12.1, 39.6 and 28.9, 14.9 and 9.9, 50 and 37.
+// 39 and 24, 15.0 and 8.7, 28672 x 4096 48 and 32; 32 rows 13.2 and 8.8, 19.2 and 12.1, 39.6 and 28.9, 14.9 and 9.9, 50 and 37; 9 rows 6.6
+// and 5.25, 9.5 and 7.2, 16.2 and 16.1, 8.7 and 6.8, 1152 x 6912 8.1 and 6.7; 16 rows 7.2 and 6.0, 10.8 and 7.6, 20.2 and 19.2, 9.1 and 6.9,
+// 8.3 and 7.3 (eight waves a step ahead; 16 waves two steps ahead 4096 x 14336 20.1).
 // (segs.glu: tiles of a wave are gate, up, gate, up ...: the gated activation is stored from here.)
-template <int NT, int R, int NWV, int D, int DA>
+template <int NT, int R, int NWV, int D, int DA, bool PAIR>
 __global__ void __launch_bounds__(64 * NWV)
-k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles, uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
+k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles_r, uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
                const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale, GemmSegs segs) {
   // (the first 14 dwords of the arguments are in registers when a wave starts; by_val bit 0 / 1: the weights' / the
   // result's element offset of op 0 is b_val / c_val -- known on the host -- instead of a load from lb / lc, which
   // the first weight loads would have to wait for)
   constexpr int RC = R >= 2 ? 2 : 1;
   static_assert(DA == 1 || DA == D, "activations one step ahead, or as many as the weights");
-  __shared__ float part[NWV * RC * NT * 256];                // [wave][tile of a pair][operand tile][i][lane]
+  constexpr int NA = PAIR ? NT / 2 : NT;                     // sums of a tile of weights
+  __shared__ float part[NWV * RC * NA * 256];                // [wave][tile of a pair][sums][i][lane]
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t r16 = lane & 15u, g = lane >> 4, op = blockIdx.z;
   const bool glum = R >= 2 && segs.glu != 0u;
@@ -560,12 +566,14 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
   uint32_t wo[R];                                            // block index from Wb on (a Q4 map here has fewer than 2^32 elements)
 #pragma unroll
   for (int r = 0; r < R; r++) wo[r] = min(first_row(r) + (lane >> 2), N - 1u) * nblk + (lane & 3u);
-  const u4q_t* const xb = x + (uint64_t)op * tiles * kw * 16u;
-  f4q_t acc[R][NT];
+  const uint32_t tiles = tiles_r & 255u, rt = tiles_r >> 8;  // operand tiles and their rows (lanes past them: the last one's again)
+  const u4q_t* const xb = x + (uint64_t)op * tiles * kw * rt;
+  const uint32_t xlane = (g * rt + min(r16, rt - 1u)) * 16u;
+  f4q_t acc[R][NA];
 #pragma unroll
   for (int r = 0; r < R; r++)
 #pragma unroll
-    for (int t = 0; t < NT; t++) acc[r][t] = (f4q_t){0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < NA; t++) acc[r][t] = (f4q_t){0.f, 0.f, 0.f, 0.f};
   DEQK_INIT(dk);
 
   u4q_t qn[D][R], xn[DA][2][NT][2];                          // [steps ahead]; activations by pairs of blocks
@@ -581,13 +589,13 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
     }
   };
   const auto fetch_x = [&](int slot, int u, uint32_t s) {
-    const uint64_t at = min(s, steps - 1u) * 256u + u * 128u;
+    const uint64_t at = (uint64_t)(min(s, steps - 1u) * 16u + u * 8u) * rt;
 #pragma unroll
     for (int t = 0; t < NT; t++) {                           // (a tile past the last: its sums are not used)
-      uint64_t from = (uint64_t)min((uint32_t)t, tiles - 1u) * kw * 16u + at;
+      uint64_t from = (uint64_t)min((uint32_t)t, tiles - 1u) * kw * rt + at;
       asm volatile("" : "+s"(from));
       const uint8_t* p = (const uint8_t*)(xb + from);
-      xn[slot][u][t][0] = *(const u4q_t*)(p + lane * 16u); xn[slot][u][t][1] = *(const u4q_t*)(p + lane * 16u + 1024u);
+      xn[slot][u][t][0] = *(const u4q_t*)(p + xlane); xn[slot][u][t][1] = *(const u4q_t*)(p + rt * 64u + xlane);
     }
     asm volatile("" ::: "memory");                           // the loads stay here
   };
@@ -614,10 +622,13 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 #pragma unroll
         for (int r = 0; r < R; r++) wq[r] = deq_word(b == 0 ? q[r].x : b == 1 ? q[r].y : b == 2 ? q[r].z : q[r].w, dk);
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
+        for (int t = 0; t < NA; t++) {
           f4q_t blk[R];
 #pragma unroll
           for (int r = 0; r < R; r++) blk[r] = MFMA_F16(xn[xs][u][t][e], wq[r], ((f4q_t){0.f, 0.f, 0.f, 0.f}));
+          if (PAIR)
+#pragma unroll
+            for (int r = 0; r < R; r++) blk[r] = MFMA_F16(xn[xs][u][NT - NA + t][e], wq[r], blk[r]);
 #pragma unroll
           for (int r = 0; r < R; r++)
 #pragma unroll
@@ -648,12 +659,12 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 #pragma unroll
     for (int r = 0; r < RC; r++)
 #pragma unroll
-      for (int t = 0; t < NT; t++)
+      for (int t = 0; t < NA; t++)
 #pragma unroll
-        for (int k = 0; k < 4; k++) part[((wave * RC + r) * NT + t) * 256u + k * 64u + lane] = acc[r0 + r][t][k];
+        for (int k = 0; k < 4; k++) part[((wave * RC + r) * NA + t) * 256u + k * 64u + lane] = acc[r0 + r][t][k];
     __syncthreads();
     for (uint32_t idx = tid; idx < M * 16u; idx += 64u * NWV) {
-      // activation row `row` of tile column c: operand rows `row` and M + row of every wave
+      // activation row `row` of tile column c: operand rows `row` and M + row of every wave (PAIR: row `row` of the one sum)
       const uint32_t row = idx >> 4, c = idx & 15u, lo = M + row;
       const auto place = [&](uint32_t v) { return (v >> 4) * 256u + (v & 3u) * 64u + ((v >> 2) & 3u) * 16u + c; };
       const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
@@ -663,9 +674,9 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
         float a = 0.f, b = 0.f;
 #pragma unroll
         for (uint32_t w = 0; w < NWV; w++) {
-          const float* p = part + (w * RC + r) * NT * 256u;
+          const float* p = part + (w * RC + r) * NA * 256u;
           a += p[place(row)];
-          b += p[place(lo)];
+          if (!PAIR) b += p[place(lo)];
         }
         y[r] = (a + b) * inv;
       }
@@ -702,7 +713,7 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 // the caller).
 template <int MT, int R>
 __global__ void __launch_bounds__(256)
-k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles,
+k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles_r,
                      uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
                      const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale,
                      GemmSegs segs) {
@@ -739,10 +750,11 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
   DEQK_INIT(dk);
   const h2q_t off_q8 = {(_Float16)-1152.f, (_Float16)-1152.f};
 
-  // (rows 16 t .. of the first plane; the grid has a tile of them for every t)
+  // (rows 16 t .. of the first plane; there is a tile of them for every t)
+  const uint32_t tiles = tiles_r & 255u, rt = tiles_r >> 8;  // operand tiles and their rows
   const u4q_t* xp[MT];
 #pragma unroll
-  for (uint32_t t = 0; t < MT; t++) xp[t] = x + (((uint64_t)op * tiles + t) * kw + g * 4u) * 16u + min(r16, M - 1u - t * 16u);
+  for (uint32_t t = 0; t < MT; t++) xp[t] = x + (((uint64_t)op * tiles + t) * kw + g * 4u) * rt + min(r16, M - 1u - t * 16u);
   u4q_t xn[MT][4], qn[R], qn2[R];
   _Float16 dn[R];
   const auto fetch_w = [&](uint32_t kb) {
@@ -758,7 +770,7 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
   const auto fetch_x = [&](uint32_t kb, int j) {
     kb = min(kb, nblk - 4u);
 #pragma unroll
-    for (int t = 0; t < MT; t++) xn[t][j] = xp[t][(uint64_t)kb * 64u + (uint32_t)j * 16u];
+    for (int t = 0; t < MT; t++) xn[t][j] = xp[t][(uint64_t)kb * (4u * rt) + (uint32_t)j * rt];
   };
   fetch_w(wave * 4u);
 #pragma unroll
@@ -873,7 +885,7 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
 #define R16_MS 2u
 template <int NW>
 __global__ void __launch_bounds__(64 * NW)
-k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles,
+k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ x, uint32_t tiles_r,
                      uint32_t K, uint32_t N, uint32_t M, uint32_t b_val, uint32_t c_val, uint32_t by_val, float* out,
                      const uint32_t* __restrict__ lb, const uint32_t* __restrict__ lc, const float* __restrict__ scale,
                      GemmSegs segs) {
@@ -901,16 +913,16 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
   f4q_t acc = {0.f, 0.f, 0.f, 0.f};
 
   // a thread's pieces of a macro tile: piece w -> (step w / 256, block (w / 64) % 4 of the step, piece (w / 16) % 4 of the block,
-  // row w % 16).  Second plane: operand rows M .. 2 M - 1
+  // row w % 16).  Second plane: the second tile
+  const uint32_t rt = tiles_r >> 8;                          // rows of a tile
   uint64_t xoff[NP], xloff[NP];
   uint32_t xlds[NP], xst[NP];
 #pragma unroll
   for (uint32_t u = 0; u < NP; u++) {
-    const uint32_t w = min(tid + u * NT, PIECES - 1u), row = w & 15u, pc = (w >> 4) & 15u, v = min(row, M - 1u), vl = v + M;
+    const uint32_t w = min(tid + u * NT, PIECES - 1u), row = w & 15u, pc = (w >> 4) & 15u;
     xst[u] = w >> 8;
-    const uint64_t at = (uint64_t)op * tiles * kw * 16u + (pc << 4);   // + 256 pieces per step of K
-    xoff[u] = at + v;
-    xloff[u] = at + (uint64_t)(vl >> 4) * kw * 16u + (vl & 15u);
+    xoff[u] = ((uint64_t)op * 2u * kw + pc) * rt + min(row, M - 1u);   // + 16 rt pieces per step of K
+    xloff[u] = xoff[u] + (uint64_t)kw * rt;
     xlds[u] = xst[u] * TILE + row * ROWB + pc * 16u;
   }
   struct ActR { u4q_t h[NP], l[NP]; };
@@ -921,7 +933,7 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
   auto fetch_a = [&](ActR& a, uint32_t m) {
 #pragma unroll
     for (uint32_t u = 0; u < NP; u++) {
-      const uint64_t at = (uint64_t)min(m * R16_MS + xst[u], steps - 1u) * 256u;
+      const uint64_t at = (uint64_t)min(m * R16_MS + xst[u], steps - 1u) * (16u * rt);
       a.h[u] = x[xoff[u] + at]; a.l[u] = x[xloff[u] + at];
     }
   };
@@ -1139,9 +1151,10 @@ static bool ensure_act_bufs(size_t scale_floats, size_t xh_bytes) {
 
 // The form in which a matmul of M rows reads its activations, and the bytes of n_ops of them
 static ActForm act_form(uint32_t M, uint32_t K, uint32_t n_ops, size_t* bytes) {
-  const uint32_t kw = K >> 3, tiles = M <= 64 && (K & 127u) == 0 ? cdiv(2 * M, 16) : 0u;
-  *bytes = tiles ? (size_t)n_ops * tiles * 32 * K : (size_t)n_ops * M * K * 4;
-  return {M, kw, tiles, (uint64_t)n_ops * M * kw};
+  const uint32_t kw = K >> 3, tiles = M <= 64 && (K & 127u) == 0 ? cdiv(2 * M, 16) : 0u, second = tiles == 2 ? 16u : M;
+  const uint32_t rows = tiles == 2 ? cdiv(M, 4) * 4 : M <= 2 ? 4u : M <= 4 ? 8u : 16u;
+  *bytes = tiles ? (size_t)n_ops * tiles * rows * 2 * K : (size_t)n_ops * M * K * 4;
+  return {M, kw, tiles, second, rows, (uint64_t)n_ops * M * kw};
 }
 
 bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, uint4** x, ActForm* form) {
@@ -1388,7 +1401,10 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   if (q8) {
     const uint32_t R = sg.glu || (uint64_t)cdiv(N, 32) * cdiv(M, 16 * mt) * n_ops >= 2ull * cu ? 2 : 1;
     const dim3 grid(cdiv(N, 16 * R), 1, n_ops);
-#define GK(T, RR) k_gemm_q8_f16_ksplit<T, RR><<<grid, 256, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst, dst, lb, lcd, g_scale_buf, sg)
+    // Two tiles of weights over long rows: LDS that nothing uses, so that a CU takes four workgroups and not five (128256 x 4096, 2, 8,
+    // 9 and 16 rows: 111, 116, 130 and 135 us with five, 106, 113, 123 and 131 with four; 262144 x 1152: 60, 69, 75, 79 and 67, 77, 81, 84)
+    const size_t spare = mt == 1 && R == 2 && K >= 2048 ? 28000 : 0;
+#define GK(T, RR) k_gemm_q8_f16_ksplit<T, RR><<<grid, 256, spare, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles | form.rows << 8, K, N, M, b_val, c_val, by_dst, dst, lb, lcd, g_scale_buf, sg)
     if (mt == 1) { if (R == 2) GK(1, 2); else GK(1, 1); }
     else { if (R == 2) GK(2, 2); else GK(2, 1); }
 #undef GK
@@ -1397,11 +1413,11 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     return check_launch();
   }
   // 9 .. 16 activation rows and workgroups of 128 weight rows for three quarters of the CUs: the form whose eight waves share an
-  // activation tile in LDS (16 rows: 28672 x 4096 25.3 us, k_gemm_q4_rows 26.9, 65536 x 2048 25.5 and 33.0; 8 rows: 24.9 and 19.9,
-  // 25.1 and 21.3)
+  // activation tile in LDS (us, this and k_gemm_q4_rows: 16 rows 28672 x 4096 23.8 and 24.1, 65536 x 2048 25.3 and 30.1; 9 rows 24.8 and
+  // 24.1, 24.9 and 29.5; 8 rows 24.9 and 19.9, 25.1 and 21.3)
   const uint32_t wgs16 = cdiv(sg.glu ? N / 2 : N, sg.glu ? 64u : 128u);
   if (form.tiles == 2 && !sg.add && (uint64_t)wgs16 * 4 >= 3ull * cu && tuning("ADAMAH_GEMM_ROWS16", 1) != 0) {
-    k_gemm_q4_f16_rows16<8><<<dim3(wgs16, 1, n_ops), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst,
+    k_gemm_q4_f16_rows16<8><<<dim3(wgs16, 1, n_ops), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles | form.rows << 8, K, N, M, b_val, c_val, by_dst,
                                                                         dst, lb, lcd, g_scale_buf, sg);
     count_launch();
     keep();
@@ -1411,13 +1427,13 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     // As many tiles of 16 weight rows to a workgroup as a CU has: one workgroup per CU reads its activations once (8 rows: 4096 x
     // 4096 one tile 4.9 us, two 6.8; 6144 x 4096 two 6.7, four 10.0; 13824 x 1152 four 6.4, one 9.2).  One and two tiles
     // of weights take the same number of waves, so that a stacked matrix has the same sums as its parts; eight where 16 waves
-    // would not have the registers (three and more operand tiles, four tiles of weights)
+    // are slower (9 .. 16 rows) or would not have the registers (more operand tiles, four tiles of weights)
     const uint32_t R = tiles16 <= cu && !sg.glu ? 1 : tiles16 <= 2 * cu || form.tiles > 4 ? 2 : 4;
     const dim3 grid(sg.glu ? cdiv(N / 2, 8 * R) : cdiv(N, 16 * R), 1, n_ops);
-#define GW(T, RR, W, D, DA) k_gemm_q4_rows<T, RR, W, D, DA><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles, K, N, M, b_val, c_val, by_dst, dst, lb, lcd, g_scale_buf, sg)
+#define GW(T, RR, W, D, DA) k_gemm_q4_rows<T, RR, W, D, DA, T == 2><<<grid, 64 * W, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles | form.rows << 8, K, N, M, b_val, c_val, by_dst, dst, lb, lcd, g_scale_buf, sg)
 #define GWT(T) do { if (R == 1) GW(T, 1, 8, 2, 1); else if (R == 2) GW(T, 2, 8, 2, 1); else GW(T, 4, 8, 1, 1); } while (0)
     if (form.tiles == 1) { if (R == 1) GW(1, 1, 16, 2, 2); else if (R == 2) GW(1, 2, 16, 2, 2); else GW(1, 4, 8, 1, 1); }
-    else if (form.tiles == 2) { if (R == 1) GW(2, 1, 16, 2, 1); else if (R == 2) GW(2, 2, 16, 2, 1); else GW(2, 4, 8, 1, 1); }
+    else if (form.tiles == 2) { if (R == 1) GW(2, 1, 8, 1, 1); else if (R == 2) GW(2, 2, 8, 1, 1); else GW(2, 4, 8, 1, 1); }
     else if (form.tiles == 3) GWT(3);
     else if (form.tiles == 4) GWT(4);
     else if (form.tiles <= 6) { if (R == 1) GW(6, 1, 8, 2, 1); else GW(6, 2, 8, 1, 1); }

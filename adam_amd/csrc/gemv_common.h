@@ -147,13 +147,14 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
 // ((s, 1/s) per row; two planes of K halves per row: fp16(x s) and the fp16 remainder), grown as needed, and -- after that kernel's launch has been
 // counted -- the note that rows [a, a + M K) of `buf` are converted, so the matmul skips its conversion.
 // Where the pieces (eight columns, 16 bytes) of those rows go.  tiles == 0: rows of both planes, [plane][op][row][kw], the
-// second plane `lo` pieces behind the first.  Otherwise the matmul's operand tiles: the 2 M rows of both planes of an op, first plane
-// first, 16 to a tile; of a tile and block of 32 columns the 64 pieces are in the order in which a wave's lanes take them.
-struct ActForm { uint32_t M, kw, tiles; uint64_t lo; };
+// second plane `lo` pieces behind the first.  Otherwise the matmul's operand tiles: operand row v is row v of the first plane, v -
+// `second` of the second one, 16 to a tile; a tile is [piece of a row][row], in the order in which a wave's lanes take a block of
+// 32 columns, with as many rows as it has (to four of them: 64 bytes) where there are one or two tiles.
+struct ActForm { uint32_t M, kw, tiles, second, rows; uint64_t lo; };
 __device__ __forceinline__ uint64_t act_piece(const ActForm& f, uint32_t op, uint32_t row, uint32_t w, uint32_t plane) {
   if (!f.tiles) return ((uint64_t)op * f.M + row) * f.kw + w + plane * f.lo;
-  const uint32_t v = plane * f.M + row;
-  return ((uint64_t)op * f.tiles + (v >> 4)) * f.kw * 16u + ((w & ~3u) << 4) + ((w & 3u) << 4) + (v & 15u);
+  const uint32_t v = plane * f.second + row;
+  return (((uint64_t)op * f.tiles + (v >> 4)) * f.kw + w) * f.rows + (v & 15u);
 }
 bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, uint4** x, ActForm* form);
 void gemm_act_forget();

@@ -593,7 +593,7 @@ def test_tiles_in_runs_per_die(hip, monkeypatch, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(2, 16, 128), (3, 8209, 256), (8, 17, 384), (9, 5000, 128), (16, 8210, 640), (17, 40, 2176), (24, 8201, 128),
-                                   (25, 4113, 384), (32, 9000, 256), (6, 24700, 128), (33, 100, 128), (40, 4100, 1152), (48, 8200, 256), (49, 4090, 640), (64, 31, 4224)])
+                                   (25, 4113, 384), (32, 9000, 256), (6, 24700, 128), (4, 130, 2176), (12, 8200, 256), (15, 24600, 128), (33, 100, 128), (40, 4100, 1152), (48, 8200, 256), (49, 4090, 640), (64, 31, 4224)])
 def test_few_rows_on_every_operand_and_weight_tile(hip, M, N, K):
     """2 .. 64 activation rows: one to eight operand tiles of both planes, one, two and four tiles of weights to a workgroup, ragged
     in every one; fewer steps of K than waves, and numbers of steps that they do not share evenly.  Rows of very different size keep
