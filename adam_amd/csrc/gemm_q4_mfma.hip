@@ -186,15 +186,18 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
     for (int t = 0; t < MT; t++) acc[r][t] = (f4q_t){0.f, 0.f, 0.f, 0.f};
   DEQK_INIT(dk);
 
-  // staging: the tile's 16 pieces per row, plane and step; thread -> (row, piece) pairs, NP per thread
+  // staging: the tile's 16 pieces per row, plane and step; thread -> (row, piece) pairs, NP per thread, in the order they lie in
+  // (of operand tiles a row's neighbouring pieces are a request to the L1 each: 64 x 28672 x 4096 68.3 us by rows, 66.2 so)
+  const auto srow = [](uint32_t w) { return TILES ? (w >> 8) * 16u + (w & 15u) : w >> 4; };
+  const auto spiece = [](uint32_t w) { return TILES ? (w >> 4) & 15u : w & 15u; };
   uint64_t xoff[NP], xloff[TILES ? NP : 1];
   constexpr uint32_t per_blk = TILES ? 64u : 4u;             // pieces from a block of a row to the next one
   const u4q_t* const xl = x + form.lo;
 #pragma unroll
   for (uint32_t u = 0; u < NP; u++) {
-    const uint32_t w = tid + u * NT, row = min(m0 + (w >> 4), M - 1u);   // rows past M: clamped, not stored
-    xoff[u] = TILES ? act_piece(form, op, row, w & 15u, 0u) : ((uint64_t)op * M + row) * form.kw + (w & 15u);
-    if (TILES) xloff[u] = act_piece(form, op, row, w & 15u, 1u);
+    const uint32_t w = tid + u * NT, row = min(m0 + srow(w), M - 1u);   // rows past M: clamped, not stored
+    xoff[u] = TILES ? act_piece(form, op, row, spiece(w), 0u) : ((uint64_t)op * M + row) * form.kw + spiece(w);
+    if (TILES) xloff[u] = act_piece(form, op, row, spiece(w), 1u);
   }
   u4q_t xn[NP], xln[NP], qn[R];
   _Float16 dn[R];
@@ -218,8 +221,8 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
 #pragma unroll
     for (uint32_t u = 0; u < NP; u++) {
       const uint32_t w = tid + u * NT;
-      *(u4q_t*)(xs + (w >> 4) * ROWB + (w & 15u) * 16u) = xn[u];
-      *(u4q_t*)(xs2 + (w >> 4) * ROWB + (w & 15u) * 16u) = xln[u];
+      *(u4q_t*)(xs + srow(w) * ROWB + spiece(w) * 16u) = xn[u];
+      *(u4q_t*)(xs2 + srow(w) * ROWB + spiece(w) * 16u) = xln[u];
     }
     u4q_t q[R];
     f4q_t ds[R];
@@ -1056,11 +1059,18 @@ struct GluSrc { uint32_t op, a, b, d; };
 template <int NW, bool GLU>
 __global__ void __launch_bounds__(1024)
 k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_t a_by_val, uint4* xf, float* scale,
-               float* act_out, const uint32_t* __restrict__ la, GluSrc glu, ActForm form) {
+               float* act_out, const uint32_t* __restrict__ la, GluSrc glu, ActForm form, uint32_t parts) {
   // (a_by_val: the rows start at element a_val -- known on the host -- instead of la[op], a load the rows' loads
   // would wait for; with GLU a_val is glu.a)
   __shared__ float red[16];
-  const uint32_t row = blockIdx.x, op = blockIdx.y, tid = threadIdx.x, kw = K >> 3;
+  const uint32_t op = blockIdx.y, tid = threadIdx.x, kw = K >> 3;
+  uint32_t row = blockIdx.x, w0 = 0, w1 = kw;                // the words this workgroup stores
+  if (parts) {
+    const uint32_t unit = (blockIdx.x >> 6) * 8u + (blockIdx.x & 7u), share = (kw / parts + 8u) & ~7u;
+    row = unit / parts * 8u + ((blockIdx.x >> 3) & 7u);
+    w0 = unit % parts * share; w1 = min(kw, w0 + share);
+    if (row >= M || w0 >= kw) return;
+  }
   const float* x = act + (a_by_val ? (uint64_t)a_val : (uint64_t)la[op]) + (uint64_t)row * K;
   f4qu_t v0[NW], v1[NW];
   float m = 0.f;
@@ -1077,8 +1087,7 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
         v0[u] = (f4qu_t){f(v0[u].x, y0.x), f(v0[u].y, y0.y), f(v0[u].z, y0.z), f(v0[u].w, y0.w)};
         v1[u] = (f4qu_t){f(v1[u].x, y1.x), f(v1[u].y, y1.y), f(v1[u].z, y1.z), f(v1[u].w, y1.w)};
         float* d = act_out + (uint64_t)glu.d + (uint64_t)row * K + w * 8u;
-        *(f4qu_t*)d = v0[u];
-        *(f4qu_t*)(d + 4) = v1[u];
+        if (w >= w0 && w < w1) { *(f4qu_t*)d = v0[u]; *(f4qu_t*)(d + 4) = v1[u]; }
       }
       m = fmaxf(m, fmaxf(fmaxf(fmaxf(fabsf(v0[u].x), fabsf(v0[u].y)), fmaxf(fabsf(v0[u].z), fabsf(v0[u].w))),
                          fmaxf(fmaxf(fabsf(v1[u].x), fabsf(v1[u].y)), fmaxf(fabsf(v1[u].z), fabsf(v1[u].w)))));
@@ -1094,14 +1103,14 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
   const uint32_t e = (__float_as_uint(m) >> 23) & 0xFFu;
   float s = 1.f, inv = 1.f;
   if (e >= 14u && e <= 254u) { s = __uint_as_float((267u - e) << 23); inv = __uint_as_float((e - 13u) << 23); }
-  if (tid == 0) {
+  if (tid == 0 && w0 == 0) {
     scale[2 * ((uint64_t)op * M + row)] = s;
     scale[2 * ((uint64_t)op * M + row) + 1] = inv;
   }
 #pragma unroll
   for (int u = 0; u < NW; u++) {
     const uint32_t w = tid + 1024u * u;
-    if (w >= kw) continue;
+    if (w < w0 || w >= w1) continue;
     const float v[8] = {v0[u].x * s, v0[u].y * s, v0[u].z * s, v0[u].w * s, v1[u].x * s, v1[u].y * s, v1[u].z * s, v1[u].w * s};
     uint4 hi, lo;
     split_word(v, &hi, &lo);
@@ -1157,6 +1166,15 @@ static ActForm act_form(uint32_t M, uint32_t K, uint32_t n_ops, size_t* bytes) {
   return {M, kw, tiles, second, rows, (uint64_t)n_ops * M * kw};
 }
 
+// Workgroups a row of k_act_f16_regs, 0: one, in the grid's order.  In operand tiles a row's pieces lie apart, a store of 64 of them 64
+// requests where a row in one piece takes 16, and eight rows share a line: so several workgroups read a row and store a share of it
+// each, and those of eight rows and a share follow each other on one die (workgroups land on the eight in turn), whose L2 then has
+// the line whole.  us, conversion and matmul, one workgroup a row anywhere and so: 8 rows 4096 x 14336 20.4 and 18.8, 4096 x 4096 8.6
+// and 8.1; 16 rows 24.6 and 22.9, 9.5 and 9.1, 1152 x 6912 12.3 and 11.4; 32 rows 35.2 and 32.3, 13.6 and 12.5, 18.0 and 17.0; 64 rows 43.2
+// and 41.0, 21.8 and 20.1, 29.2 and 27.9.
+static uint32_t act_parts(const ActForm& f) { return !f.tiles ? 0u : f.M <= 8 ? 8u : 4u; }
+static uint32_t act_grid(const ActForm& f) { return f.tiles ? cdiv(cdiv(f.M, 8) * act_parts(f), 8) * 64u : f.M; }
+
 bool gemm_act_slots(uint32_t M, uint32_t K, float** scale, uint4** x, ActForm* form) {
   if (tuning("ADAMAH_GEMM_REUSE", 1) == 0) return false;
   size_t bytes;
@@ -1181,8 +1199,9 @@ bool launch_glu_act_f16(const Map* ma, uint32_t op, uint32_t a, uint32_t b, uint
   if (!gemm_act_slots(M, K, &scale, &xf, &form)) return false;
   float* act = (float*)ma->buf;
   const GluSrc glu = {op, a, b, d};
-  if (K <= 8192) k_act_f16_regs<1, true><<<dim3(M, 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form);
-  else k_act_f16_regs<2, true><<<dim3(M, 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form);
+  // (the caller has seen to it that d touches neither a nor b: several workgroups may read a row)
+  if (K <= 8192) k_act_f16_regs<1, true><<<dim3(act_grid(form), 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form, act_parts(form));
+  else k_act_f16_regs<2, true><<<dim3(act_grid(form), 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form, act_parts(form));
   count_launch();
   gemm_act_mark(ma->buf, d, M, K);
   return true;
@@ -1387,8 +1406,8 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   uint4* const xl = (uint4*)((uint8_t*)g_xh_buf + plane);
   if (!reuse) {
     if (K <= 16384 && knob("ADAMAH_ACT_REGS", 1) != 0) {
-      if (K <= 8192) k_act_f16_regs<1, false><<<dim3(M, n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form);
-      else k_act_f16_regs<2, false><<<dim3(M, n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form);
+      if (K <= 8192) k_act_f16_regs<1, false><<<dim3(act_grid(form), n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form, act_parts(form));
+      else k_act_f16_regs<2, false><<<dim3(act_grid(form), n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form, act_parts(form));
     } else
       k_act_f16<<<dim3(M, n_ops), 256, 0, g.stream>>>(act, la, M, K, g_scale_buf, xh, form);
     count_launch();
