@@ -1106,6 +1106,11 @@ class DecodeEngine:
             residual('ffn_out', f'{p}.post_ffw_norm.weight')
         return ops
 
+    def _rope_appends(self):
+        """Whether one call rotates and appends the rows of a chunk: it takes one head size, an even one of at most 4096."""
+        c = self.cfg
+        return hasattr(self.gpu, 'rope_append_rows_dev') and c.head_dim == c.head_dim_kv and c.head_dim % 2 == 0 and c.head_dim <= 4096
+
     def _forward_chunk(self, toks, pos0, sample=True, seq=0, lockstep=False, from_device=False, seqs=None):
         """m <= prefill_chunk prompt tokens at positions pos0 .. pos0 + m - 1 in one pass: the row-wise ops
         over m rows, the projections as [m, K] x [N, K]^T matmuls (the fp16 matrix-core kernel for Q4
@@ -1178,7 +1183,7 @@ class DecodeEngine:
             mm('normed', f'{p}.attn_q.weight', 'q', E, q_dim)
             mm('normed', f'{p}.attn_k.weight', 'k', E, k_dim)
             mm('normed', f'{p}.attn_v.weight', 'v', E, k_dim)
-            append = not lockstep and m > 1 and hasattr(g, 'rope_append_rows_dev')    # rotation and KV append in one call
+            append = not lockstep and m > 1 and self._rope_appends()    # rotation and KV append in one call
             if self._chunk_qk and not lockstep and hasattr(g, 'qk_norm_rope_rows_dev'):
                 for lo in range(0, m, each):
                     hi = lo + each
@@ -1293,7 +1298,7 @@ class DecodeEngine:
         chunk hold go through the weights together (eight prompts of 48 tokens one by one: eight passes over the weights)."""
         P, g = len(prompts[0]), self.gpu
         at_once = self._chunk // P if self._prompts_together and P else 1
-        if len(prompts) < 2 or at_once < 2 or not hasattr(g, 'rope_append_rows_dev') or not hasattr(g, 'attn_causal_rows_dev'):
+        if len(prompts) < 2 or at_once < 2 or not self._rope_appends() or not hasattr(g, 'attn_causal_rows_dev'):
             return self._prefill_each(prompts)
         first = []
         for lo in range(0, len(prompts), at_once):

@@ -111,6 +111,22 @@ def test_chunked_prefill_equals_token_by_token(arch, chunk):
     assert np.array_equal(outs[0][1], outs[1][1]) and np.array_equal(outs[0][2], outs[1][2])
 
 
+@pytest.mark.parametrize("head_dim,head_dim_kv", [(16, 32), (5, 5)])
+def test_chunks_of_unequal_and_odd_heads_equal_token_by_token(head_dim, head_dim_kv):
+    """Heads of Q smaller than those of K and V, and of an odd size: what a chunk rotates and appends is what single tokens do."""
+    cfg = synth.tiny_config("llama", n_layer=2, n_embd=64, n_head=32, n_head_kv=32, head_dim=head_dim, n_ff=96, n_vocab=160)
+    cfg.head_dim_kv = head_dim_kv
+    tensors = synth.make_model(cfg, seed=3, sigma=0.3)
+    outs = []
+    for m in (0, 4):
+        eng = DecodeEngine(oracle.init(), cfg, tensors, A=A, kv_cap=32, kv_fp16=True, prefill_chunk=m, batch=2 if m else 1)
+        assert not eng._rope_appends()
+        out, _ = eng.generate([5, 17, 3, 101, 64, 9], GenerationConfig(max_tokens=4))
+        outs.append((out, eng.read_slot('hidden')))
+    assert outs[0][0] == outs[1][0] and np.array_equal(outs[0][1], outs[1][1])
+    assert eng.generate_batch([[5, 17], [3, 101]], 3)[0] == [eng.generate(p, GenerationConfig(max_tokens=3))[0] for p in ([5, 17], [3, 101])]
+
+
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
 def test_batched_lockstep_decode_equals_independent_sequences(arch):
     """Several sequences decoded in lockstep (rows of one [B, K] matmul, own KV cache each) give, on the

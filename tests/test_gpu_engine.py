@@ -198,6 +198,21 @@ def test_chunked_prefill_on_the_matrix_cores(hip, arch, chunk):
         assert dev_tok[i] == ref_tok[i] or margins[i] < 1e-4, (i, dev_tok[i], ref_tok[i], margins[i])
 
 
+@pytest.mark.parametrize("head_dim,head_dim_kv", [(16, 32), (5, 5)])
+def test_chunks_of_unequal_and_odd_heads(hip, head_dim, head_dim_kv):
+    """Heads of Q smaller than those of K and V, and of an odd size, in chunks: as token by token on the oracle."""
+    cfg = synth.tiny_config("llama", n_layer=2, n_embd=64, n_head=32, n_head_kv=32, head_dim=head_dim, n_ff=96, n_vocab=160)
+    cfg.head_dim_kv = head_dim_kv
+    tensors = synth.make_model(cfg, seed=3, sigma=0.1)
+    prompt = [5, 17, 3, 101, 64, 9]
+    ref = DecodeEngine(oracle.init(), cfg, tensors, A=A, kv_cap=32, kv_fp16=True)
+    ref.prefill(prompt)
+    note(f"engine chunks of heads {head_dim} / {head_dim_kv}")
+    dev = DecodeEngine(hip, cfg, tensors, A=A, kv_cap=32, kv_fp16=True, prefill_chunk=4)
+    dev.prefill(prompt)
+    assert rel_l2(dev.read_slot('hidden'), ref.read_slot('hidden')) < 1e-3
+
+
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
 def test_batched_lockstep_decode(hip, arch):
     """Four sequences in lockstep on the HIP library (projections as [4, K] matmuls on the matrix cores,
