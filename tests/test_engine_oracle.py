@@ -148,13 +148,14 @@ def test_batched_lockstep_decode_equals_independent_sequences(arch):
 
 
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
-@pytest.mark.parametrize("chunk", [4, 10, 15])
-def test_prompts_of_a_batch_in_one_pass_equal_one_by_one(arch, chunk):
-    """Prompts of five tokens one by one (four rows), two at a time with one left over, and all three at once: the same tokens, caches
-    and decode slots, exactly, on the oracle."""
+@pytest.mark.parametrize("chunk,P", [(4, 5), (10, 5), (15, 5), (3, 1), (2, 1)])
+def test_prompts_of_a_batch_in_one_pass_equal_one_by_one(arch, chunk, P):
+    """Prompts of five tokens one by one (four rows), two at a time with one left over, and all three at once; prompts of one token: the same
+    tokens, caches and decode slots, exactly, on the oracle."""
     cfg = synth.tiny_config(arch, n_layer=2, n_embd=64, n_head=4, n_head_kv=2, head_dim=32, n_ff=96, n_vocab=160)
     tensors = synth.make_model(cfg, seed=3, sigma=0.3)
     prompts = [[5, 17, 3, 101, 64], [9, 33, 2, 8, 150], [1, 1, 1, 1, 1]]
+    prompts = [p[:P] for p in prompts]
     outs = []
     for together in (False, True):
         eng = DecodeEngine(oracle.init(), cfg, tensors, A=A, kv_cap=32, kv_fp16=True, batch=3, prefill_chunk=chunk)

@@ -363,14 +363,16 @@ def test_a_plan_called_with_the_same_step_is_not_recorded():
 
 
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
-@pytest.mark.parametrize("chunk", [64, 45])
-def test_prompts_of_a_batch_go_through_the_weights_together(hip, arch, chunk):
-    """Four prompts of 20 tokens at 64 rows (three at once, one left over) and at 45 (two and two): the tokens that follow and the
-    caches are those of the prompts one by one, up to the rounding of matmuls of other row counts."""
+@pytest.mark.parametrize("chunk,P", [(64, 20), (45, 20), (160, 40), (110, 35), (4, 1)])
+def test_prompts_of_a_batch_go_through_the_weights_together(hip, monkeypatch, arch, chunk, P):
+    """Four prompts of 20 tokens at 64 rows (three at once, one left over) and at 45 (two and two), of 40 and 35 at 160 and 105 rows on
+    the ring matmul, and of one token: the tokens that follow and the caches are those of the prompts one by one, up to the rounding of
+    matmuls of other row counts."""
+    monkeypatch.setenv("ADAMAH_GEMM_RING", "2")              # more than 64 rows: always the ring
     cfg = synth.tiny_config(arch, n_layer=3, n_embd=256, n_head=4, n_head_kv=2, head_dim=64, n_ff=512, n_vocab=1000)
     tensors = synth.make_model(cfg, seed=5, sigma=0.1)
     rng = np.random.default_rng(3)
-    prompts = [[int(t) for t in rng.integers(0, 1000, 20)] for _ in range(4)]
+    prompts = [[int(t) for t in rng.integers(0, 1000, P)] for _ in range(4)]
     outs = []
     for together in (False, True):
         note(f"engine prompts together={together} {arch} chunk={chunk}")
