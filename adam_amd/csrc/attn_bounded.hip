@@ -716,8 +716,8 @@ k_attn_bf16(const ASpec s, float* act, const bf16_t* __restrict__ K, const bf16_
 static Scratch g_stage, g_parts;
 void attn_bounded_release() { scratch_free(g_stage); scratch_free(g_parts); }
 
-// Whether the four waves of a workgroup share their queries and part the keys, instead of taking queries each: where workgroups of
-// queries would not give every CU one, and a wave has keys enough to pay for the sum through LDS.  952 queries behind 2048 keys, 16
+// Whether the four waves of a workgroup share their queries and part the keys, instead of taking queries each: where a portion's
+// workgroups of queries would not give every CU one (the portion's alone: its sums do not depend on the sequences beside it), and a wave has keys enough to pay for the sum through LDS.  952 queries behind 2048 keys, 16
 // heads: 151 -> 98 us; float32, 512 queries in 16 heads: 88 -> 39, 88 behind 512 keys: 98 -> 33.  (With one for every CU the waves
 // of a workgroup are better off reading the same keys: 2048 queries in 16 heads 110 us, so: 116; in 32 heads 193 and 200.)
 static bool shared_keys(const ASpec& s, const StageDims& sd, uint64_t wgs) {
@@ -730,7 +730,7 @@ static void launch_bf16(const ASpec& s, float* act, const bf16_t* K, const bf16_
 #define CASE(N)                                                                                                     \
   case N: {                                                                                                         \
     constexpr int QT = DK <= 4 && N <= 8 ? 2 : 1;                                                                   \
-    if (shared_keys(s, sd, (uint64_t)cdiv(m, 64 * QT) * n_seq))                                                                     \
+    if (shared_keys(s, sd, cdiv(m, 64 * QT)))                                                                       \
       k_attn_bf16<WIN, DK, N, QT, 4><<<dim3(s.heads, cdiv(m, 16 * QT), n_seq), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos, by); \
     else                                                                                                            \
       k_attn_bf16<WIN, DK, N, QT, 1><<<dim3(s.heads, cdiv(m, 64 * QT), n_seq), 256, 0, g.stream>>>(s, act, K, VT, sd, m, pos, by); \
@@ -754,8 +754,9 @@ static int run_portion(const ASpec& s, float* act, T* cache, uint32_t n_seq, uin
   sd.dp = 32u * (s.dim <= 128u ? cdiv(s.dim, 32) : s.dim <= 192u ? 6u : 8u);
   sd.vp = vtiles(s.vdim) * 16u;
   const uint64_t nk = (uint64_t)s.kv_heads * sd.np * sd.dp, nv = (uint64_t)s.kv_heads * sd.np * sd.vp;
-  // the sequences that one set of launches takes (their staged operands are to stay below 256 MB; the grid's limit)
-  const uint32_t at_once = (uint32_t)std::min<uint64_t>(std::min<uint64_t>(n_seq, 65535u), std::max<uint64_t>(1u, ((uint64_t)256 << 20) / ((nk + nv) * sizeof(T))));
+  // the sequences that one set of launches takes (their staged operands, kept between calls, are to stay below 64 MB, eight of 2048
+  // keys in 8 heads of 128; the grid's limit)
+  const uint32_t at_once = (uint32_t)std::min<uint64_t>(std::min<uint64_t>(n_seq, 65535u), std::max<uint64_t>(1u, ((uint64_t)64 << 20) / ((nk + nv) * sizeof(T))));
   const SeqSteps by = {(uint64_t)m * s.x_stride, (uint64_t)m * s.out_stride, s.seq_stride, nk, nv};
   if (at_once < n_seq) {
     for (uint32_t q = 0; q < n_seq; q += at_once) {
@@ -776,7 +777,7 @@ static int run_portion(const ASpec& s, float* act, T* cache, uint32_t n_seq, uin
   count_launch();
   if (int r = check_launch()) return r;
   if constexpr (sizeof(T) == 4) {
-    const bool apart = shared_keys(s, sd, (uint64_t)cdiv(m, 64) * n_seq);
+    const bool apart = shared_keys(s, sd, cdiv(m, 64));
     const dim3 grid(s.heads, cdiv(m, apart ? 16 : 64), n_seq);
 #define AF(NV, DK)                                                                                                  \
   do {                                                                                                              \

@@ -738,6 +738,39 @@ def test_chunk_attention_with_the_keys_parted_among_waves(hip, H, G, D, V, C, ms
         pos += m
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("H,G,D,V,C,rows,n_seq", [(16, 4, 64, 64, 400, 150, 9), (40, 8, 32, 48, 600, 290, 3)])
+def test_a_portion_has_the_same_sums_beside_others(hip, H, G, D, V, C, rows, n_seq, dtype):
+    """Portions that by themselves leave compute units idle (the waves of a workgroup part the keys) and together do not: outputs and
+    caches are, bit for bit, those of each sequence alone."""
+    note(f"chunk attention of {n_seq} sequences, H {H} D {D} chunk {C} {dtype}")
+    rng = np.random.default_rng(C)
+    xs, kc, vc = H * D + G * (D + V), G * C * D, G * C * V
+    oo = n_seq * rows * xs
+    ro = oo + n_seq * rows * H * V
+    ss = kc + vc
+    x = [rng.standard_normal(oo).astype(np.float32) for _ in range(2)]
+    spec = lambda i: up(hip, A.ChunkAttnSpec(heads=H, kv_heads=G, dim=D, vdim=V, chunk=C, x=i * rows * xs, x_stride=xs, x_q=0, x_k=H * D, x_v=(H + G) * D, r1=ro,
+                                             r2=ro + H, scale=0.25, eps=1e-4, out=oo + i * rows * H * V, out_stride=H * V, cache_map=CA, k_off=0, v_off=kc,
+                                             seq_stride=ss).words())
+    got = []
+    for together in (False, True):
+        hip.map_create_typed(CA, A.DTYPE_F32 if dtype == "float32" else A.DTYPE_BF16, 1, n_seq * ss)
+        f32map(hip, WS, ro + 2 * H, np.concatenate([np.zeros(ro, np.float32), np.linspace(0.02, 1.5, H), np.full(H, 0.3)]).astype(np.float32))
+        words = []
+        for i, xi in enumerate(x):
+            hip.scatter_contiguous(WS, 0, xi)
+            if together:
+                hip.chunk_attention_seqs_dev(WS, spec(0), n_seq, rows, 0, i * rows)
+            else:
+                for q in range(n_seq):
+                    hip.chunk_attention_dev(WS, spec(q), 1, rows, q, i * rows)
+            words.append(read(hip, WS, oo, n_seq * rows * H * V).view(np.uint32).copy())
+        got.append(words)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("k,n,rows,listed,branched", [(64, 40, 2, False, False), (200, 1003, 5, True, False), (4096, 517, 9, True, True), (4608, 70, 16, False, False),
                                                       (4672, 33, 6, True, False), (9216, 66, 3, True, True), (20000, 21, 2, True, False), (1000, 8, 1, True, False)])
 def test_heads_of_several_rows_are_the_one_row_head(hip, k, n, rows, listed, branched):
