@@ -41,15 +41,19 @@ k_rmsnorm(const float* act, const float* wt, float* out, const uint32_t* __restr
   }
 }
 
-// The same row op with the row held in registers: one trip to memory instead of two dependent passes.  Rows of a multiple of
-// eight, at most 8192: a thread owns the eight neighbours of one word (NT >= dim / 8 threads), loads and stores 16 bytes at a time.
+// The same row op with the row held in registers: one trip to memory instead of two dependent passes, for rows of at most 8192.
+// WIDE: rows of a multiple of eight, a thread owns the eight neighbours of one word (PER = 8, NT >= dim / 8 threads), loads and
+// stores 16 bytes at a time; the squares pass through LDS, where 256 threads add them up in the order of the kernel above.
+// Otherwise 256 threads own elements 256 apart (dim <= 256 PER), that kernel's order by itself.  The results are the same bits.
 // EMIT: the rows are [n_rows, dim] back to back and a batched matmul follows; its fp16 operand form (row scaled by a power of two,
 // two planes, 8-element words in the order (0,4)(1,5)(2,6)(3,7), plus (s, 1/s) per row) is written here as well, which spares that
 // matmul its conversion launch.  A launch of few rows is one trip to memory, two sums over the workgroup and the stores: with one
-// element a load and 256 threads a row it was 16 pairs of loads and 48 stores a thread (4096 wide, 8 rows 6.2 us, 24 rows 6.3).
+// element a load and 256 threads a row it was 16 pairs of loads and 48 stores a thread.  us behind each other, operand form included,
+// that and this: 8 rows of 4096 4.55 and 4.35, of 8192 6.5 and 6.1, 512 rows 7.5 and 7.3, 12.0 and 11.6; 2 rows of 4096 with a residual
+// 4.7 and 4.2.  (Each thread's squares summed by itself, in another order: 4.0, 4.8, 6.4 and 10.1.)
 struct RowsByValue { uint32_t on, s0, ss, w0, ws, d0, ds, r0, rs; };   // host side only
 typedef float f4r_t __attribute__((ext_vector_type(4), aligned(4)));
-template <bool ADD, bool EMIT, int NT>
+template <bool ADD, bool EMIT, bool WIDE, int NT, int PER>
 __global__ void __launch_bounds__(NT)
 k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, uint32_t s0, uint32_t ss_, uint32_t w0, uint32_t ws,
                uint32_t d0, uint32_t ds, uint32_t r0, uint32_t rs, float* out,
@@ -58,7 +62,9 @@ k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, ui
   // (these 14 dwords are in registers when a wave starts.  Top bit of dim_on: row i's source / weights / destination /
   // residual start at x0 + i xs -- the host found the rows evenly spaced -- instead of four loads from the row
   // tables, which the rows' own loads would have to wait for)
-  __shared__ float sums[NT / 64], tops[NT / 64];
+  static_assert(WIDE ? PER == 8 : NT == 256 && !EMIT, "the operand form is made of whole words");
+  __shared__ __attribute__((aligned(16))) float row[WIDE ? 8 * NT : 4];
+  __shared__ float sums[4], tops[NT / 64];
   const uint32_t ri = blockIdx.x, tid = threadIdx.x, dim = dim_on & 0x7FFFFFFFu;
   uint64_t sb, wb, db, rb = 0;
   if (dim_on >> 31) {
@@ -68,62 +74,84 @@ k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, ui
     sb = ls[ri]; wb = lw[ri]; db = ld[ri]; if (ADD) rb = lr[ri];
   }
   if (sb + dim > act_elems || db + dim > act_elems || wb + dim > wt_elems || (ADD && rb + dim > act_elems)) return;
-  const bool in = tid < (dim >> 3);
-  const uint32_t i = in ? tid * 8u : 0u;                     // (a thread past the row loads its first word)
-  const f4r_t x0 = *(const f4r_t*)(act + sb + i), x1 = *(const f4r_t*)(act + sb + i + 4);
-  const f4r_t g0 = *(const f4r_t*)(wt + wb + i), g1 = *(const f4r_t*)(wt + wb + i + 4);
-  f4r_t a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
-  if (ADD) { a0 = *(const f4r_t*)(act + rb + i); a1 = *(const f4r_t*)(act + rb + i + 4); }
-  float x[8], ss = 0.f;
+  const bool in = tid < (dim >> 3);                          // WIDE: the thread has a word
+  float x[PER], w[PER], r[PER], ss = 0.f;
+  if (WIDE) {
+    const uint32_t i = in ? tid * 8u : 0u;                   // (a thread past the row loads its first word)
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    x[e] = e < 4 ? x0[e & 3] : x1[e & 3];
-    ss = in ? fmaf(x[e], x[e], ss) : 0.f;
+    for (int h = 0; h < 2; h++) {
+      const f4r_t xv = *(const f4r_t*)(act + sb + i + 4 * h), wv = *(const f4r_t*)(wt + wb + i + 4 * h);
+      f4r_t rv = {0.f, 0.f, 0.f, 0.f};
+      if (ADD) rv = *(const f4r_t*)(act + rb + i + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; e++) { x[4 * h + e] = xv[e]; w[4 * h + e] = wv[e]; r[4 * h + e] = rv[e]; }
+    }
+    *(f4r_t*)(row + tid * 8u) = (f4r_t){x[0], x[1], x[2], x[3]};
+    *(f4r_t*)(row + tid * 8u + 4) = (f4r_t){x[4], x[5], x[6], x[7]};
+    __syncthreads();
+    if (tid < 256u) {
+#pragma unroll
+      for (uint32_t u = 0; u < 8u * NT / 256u; u++) {
+        const float v = row[tid + 256u * u];
+        ss = tid + 256u * u < dim ? fmaf(v, v, ss) : ss;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < PER; e++) {
+      const uint32_t i = min(tid + 256u * e, dim - 1u);
+      x[e] = act[sb + i]; w[e] = wt[wb + i]; r[e] = ADD ? act[rb + i] : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < PER; e++) ss = tid + 256u * e < dim ? fmaf(x[e], x[e], ss) : ss;
   }
+  if (tid < 256u) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-  if ((tid & 63u) == 0) sums[tid >> 6] = ss;
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    if ((tid & 63u) == 0) sums[tid >> 6] = ss;
+  }
   __syncthreads();
-  ss = 0.f;
-#pragma unroll
-  for (int w = 0; w < NT / 64; w++) ss += sums[w];
-  const float inv = 1.0f / sqrtf(ss / (float)dim + eps);
+  const float inv = 1.0f / sqrtf(((sums[0] + sums[1]) + (sums[2] + sums[3])) / (float)dim + eps);
   float m = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; e++) {
-    x[e] = x[e] * inv * (e < 4 ? g0[e & 3] : g1[e & 3]);
-    if (ADD) x[e] += e < 4 ? a0[e & 3] : a1[e & 3];
+  for (int e = 0; e < PER; e++) {
+    x[e] = x[e] * inv * w[e];
+    if (ADD) x[e] += r[e];
     m = fmaxf(m, fabsf(x[e]));
   }
-  if (in) {
-    *(f4r_t*)(out + db + i) = (f4r_t){x[0], x[1], x[2], x[3]};
-    *(f4r_t*)(out + db + i + 4) = (f4r_t){x[4], x[5], x[6], x[7]};
+  if (!WIDE) {
+#pragma unroll
+    for (int e = 0; e < PER; e++) if (tid + 256u * e < dim) out[db + tid + 256u * e] = x[e];
+  } else if (in) {
+    *(f4r_t*)(out + db + tid * 8u) = (f4r_t){x[0], x[1], x[2], x[3]};
+    *(f4r_t*)(out + db + tid * 8u + 4) = (f4r_t){x[4], x[5], x[6], x[7]};
   }
-  if (!EMIT) return;
-  if (!in) m = 0.f;
+  if constexpr (EMIT) {
+    if (!in) m = 0.f;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-  if ((tid & 63u) == 0) tops[tid >> 6] = m;
-  __syncthreads();
-  m = tops[0];
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    if ((tid & 63u) == 0) tops[tid >> 6] = m;
+    __syncthreads();
+    m = tops[0];
 #pragma unroll
-  for (int w = 1; w < NT / 64; w++) m = fmaxf(m, tops[w]);
-  const uint32_t e = (__float_as_uint(m) >> 23) & 0xFFu;
-  float s = 1.f, si = 1.f;
-  if (e >= 14u && e <= 254u) { s = __uint_as_float((267u - e) << 23); si = __uint_as_float((e - 13u) << 23); }
-  if (tid == 0) { scale[2 * ri] = s; scale[2 * ri + 1] = si; }
-  if (!in) return;
-  // two planes: fp16(x s) and the fp16 remainder x s - fp16(x s), as the matmul's own conversion writes them
-  uint32_t hi[4], lo[4];
+    for (int w = 1; w < NT / 64; w++) m = fmaxf(m, tops[w]);
+    const uint32_t e = (__float_as_uint(m) >> 23) & 0xFFu;
+    float s = 1.f, si = 1.f;
+    if (e >= 14u && e <= 254u) { s = __uint_as_float((267u - e) << 23); si = __uint_as_float((e - 13u) << 23); }
+    if (tid == 0) { scale[2 * ri] = s; scale[2 * ri + 1] = si; }
+    if (!in) return;
+    // two planes: fp16(x s) and the fp16 remainder x s - fp16(x s), as the matmul's own conversion writes them
+    uint32_t hi[4], lo[4];
 #pragma unroll
-  for (int p = 0; p < 4; p++) {
-    const float u = x[p] * s, v = x[p + 4] * s;
-    const __half uh = __float2half(u), vh = __float2half(v);
-    hi[p] = (uint32_t)__half_as_ushort(uh) | (uint32_t)__half_as_ushort(vh) << 16;
-    lo[p] = (uint32_t)__half_as_ushort(__float2half(u - __half2float(uh))) | (uint32_t)__half_as_ushort(__float2half(v - __half2float(vh))) << 16;
+    for (int p = 0; p < 4; p++) {
+      const float u = x[p] * s, v = x[p + 4] * s;
+      const __half uh = __float2half(u), vh = __float2half(v);
+      hi[p] = (uint32_t)__half_as_ushort(uh) | (uint32_t)__half_as_ushort(vh) << 16;
+      lo[p] = (uint32_t)__half_as_ushort(__float2half(u - __half2float(uh))) | (uint32_t)__half_as_ushort(__float2half(v - __half2float(vh))) << 16;
+    }
+    xf[act_piece(form, 0u, ri, tid, 0u)] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    xf[act_piece(form, 0u, ri, tid, 1u)] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
   }
-  xf[act_piece(form, 0u, ri, tid, 0u)] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-  xf[act_piece(form, 0u, ri, tid, 1u)] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
 }
 
 // theta_i = pos * (1 / base^(2i/dim)).  The exponent and the reciprocal are float32 operations as
@@ -307,7 +335,7 @@ static int rmsnorm_impl(uint32_t map_act, uint32_t map_wt, uint32_t hs, uint32_t
   const uint32_t* lr = add ? res_u32(hr, n_rows) : ls;
   if (!ls || !lw || !ld || !lr) return ADAMAH_ERR_INVALID;
   float* a = (float*)ma->buf;
-  if (n_rows > 1 && dim >= 8 && dim <= 8192 && (dim & 7u) == 0 && tuning("ADAMAH_RMSNORM_ROWS", 1) != 0) {
+  if (n_rows > 1 && dim > 0 && dim <= 8192 && tuning("ADAMAH_RMSNORM_ROWS", 1) != 0) {
     // rows in registers; when the results are the rows of a matrix [n_rows, dim], also in the form the
     // batched matmul reads
     const uint32_t* dh = res_host(hd, n_rows);
@@ -338,10 +366,13 @@ static int rmsnorm_impl(uint32_t map_act, uint32_t map_wt, uint32_t hs, uint32_t
       }
       if (!even) rv.on = 0u;
     }
-#define RR(A, E, NT) k_rmsnorm_rows<A, E, NT><<<n_rows, NT, 0, g.stream>>>(a, w, dim | (rv.on << 31), eps, rv.s0, rv.ss, rv.w0, rv.ws, rv.d0, rv.ds, rv.r0, rv.rs, a, ls, lw, lr, ld, ma->n_elems, mw->n_elems, scale, xf, form)
-#define RN(A, E) do { if (dim <= 2048) RR(A, E, 256); else if (dim <= 4096) RR(A, E, 512); else RR(A, E, 1024); } while (0)
-    if (add) { if (emit) RN(true, true); else RN(true, false); }
+#define RR(A, E, V, NT, PER) k_rmsnorm_rows<A, E, V, NT, PER><<<n_rows, NT, 0, g.stream>>>(a, w, dim | (rv.on << 31), eps, rv.s0, rv.ss, rv.w0, rv.ws, rv.d0, rv.ds, rv.r0, rv.rs, a, ls, lw, lr, ld, ma->n_elems, mw->n_elems, scale, xf, form)
+#define RN(A, E) do { if (dim <= 2048) RR(A, E, true, 256, 8); else if (dim <= 4096) RR(A, E, true, 512, 8); else RR(A, E, true, 1024, 8); } while (0)
+#define RO(A) do { if (dim <= 2048) RR(A, false, false, 256, 8); else if (dim <= 4096) RR(A, false, false, 256, 16); else RR(A, false, false, 256, 32); } while (0)
+    if (dim & 7u) { if (add) RO(true); else RO(false); }
+    else if (add) { if (emit) RN(true, true); else RN(true, false); }
     else { if (emit) RN(false, true); else RN(false, false); }
+#undef RO
 #undef RN
 #undef RR
     count_launch();

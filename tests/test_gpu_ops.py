@@ -74,6 +74,32 @@ def test_rmsnorm_rows_at_irregular_places(hip, dim, add):
         assert rel_l2(outs[0][dst[i]:dst[i] + dim], y) < 1e-5, i
 
 
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("dim", [1, 7, 100, 256, 1001, 1152, 2050, 4096, 5000, 8191, 8192])
+def test_rmsnorm_of_several_rows_has_the_bits_of_one(hip, dim, add):
+    """Rows held in registers, of any width, whole words or not: the sums of the one-row kernel in its order."""
+    rng = np.random.default_rng(dim)
+    n = 24
+    x = rng.standard_normal(dim * (2 * n + 2)).astype(np.float32) * np.float32(3)
+    src, wt, res = dim * np.arange(n), np.full(n, n * dim), np.full(n, (n + 1) * dim)
+    dst = (n + 2) * dim + src
+    got = []
+    for rows in (n, 1):
+        note(f"rmsnorm dim={dim} add={add} rows={rows}")
+        f32map(hip, 0, x.size, x)
+        for i in range(0, n, rows):
+            h = [up(hip, v[i:i + rows]) for v in (src, wt, res, dst)]
+            if add:
+                hip.map_rmsnorm_add_dev(0, h[0], h[1], h[2], h[3], rows, dim, 1e-5)
+            else:
+                hip.map_rmsnorm_dev(0, h[0], h[1], h[3], rows, dim, 1e-5)
+        got.append(read(hip, 0, 0, x.size))
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    y = x[:n * dim].reshape(n, dim).astype(np.float64)
+    want = y / np.sqrt((y * y).mean(1, keepdims=True) + 1e-5) * x[n * dim:][:dim] + (x[(n + 1) * dim:][:dim] if add else 0)
+    assert rel_l2(got[0][(n + 2) * dim:], want.reshape(-1)) < 1e-5
+
+
 @pytest.mark.parametrize("heads,dim,pos,base", [(32, 128, 0, 500000.0), (8, 128, 4095, 500000.0),
                                                (4, 256, 639, 1e6), (1, 256, 16383, 1e4)])
 def test_rope(hip, heads, dim, pos, base):
