@@ -193,7 +193,8 @@ k_rope(float* data, const uint32_t* __restrict__ ls, const uint32_t* __restrict_
 // 32 + 2 x 8 heads of 128: 24 tokens 8.4 us a pair at a time in a loop, 4.5 so; 512 tokens 11.3 and 8.7.
 #define APPEND_SEQS 32u
 #define APPEND_UNITS 4
-struct AppendRows { uint32_t q, q_step, q_heads, k, k_step, k_heads, v, v_step, dim, n_tok, head_step, pos0, rotate; float base;
+// (q, k, v: of the first sequence of the launch, which may lie beyond 2^32)
+struct AppendRows { uint64_t q, k, v; uint32_t q_step, q_heads, k_step, k_heads, v_step, dim, n_tok, head_step, pos0, rotate; float base;
                     uint32_t kc[APPEND_SEQS], vc[APPEND_SEQS]; };
 template <int W>
 __global__ void __launch_bounds__(256)
@@ -641,7 +642,8 @@ int adamah_hip_rope_append_rows_dev(uint32_t map_id, uint32_t q, uint32_t q_step
   for (uint32_t s = 0; s < n_seq; s++) starts |= k_cache[s] | v_cache[s];
   for (uint32_t s0 = 0; s0 < n_seq; s0 += APPEND_SEQS) {
     const uint32_t part = std::min(n_seq - s0, APPEND_SEQS);
-    AppendRows a = {q + s0 * n_tok * q_step, q_step, q_heads, k + s0 * n_tok * k_step, k_step, k_heads, v + s0 * n_tok * v_step, v_step, head_dim,
+    const uint64_t row = (uint64_t)s0 * n_tok;
+    AppendRows a = {q + row * q_step, k + row * k_step, v + row * v_step, q_step, q_heads, k_step, k_heads, v_step, head_dim,
                     n_tok, head_step, pos0, rotate, freq_base, {}, {}};
     for (uint32_t s = 0; s < part; s++) { a.kc[s] = k_cache[s0 + s]; a.vc[s] = v_cache[s0 + s]; }
 #define APPEND(W) k_rope_append_rows<W><<<dim3(n_tok, part), 256, D * sizeof(float), g.stream>>>((float*)m->buf, a, m->kv16, m->kv_start, m->kv_count)

@@ -527,6 +527,31 @@ def test_rope_append_rows_of_any_start(hip, n_tok, n_seq, Hq, Hk, D, pos0, shift
     assert np.abs(out[0][c0:] - out[1][c0:]).max() <= 2.0 ** -10 * np.abs(x).max() * 1.5 + 1e-7     # one fp16 step where the rotations round apart
 
 
+def test_rope_append_rows_of_sequences_beyond_2_to_the_32_elements(hip):
+    """The 33rd sequence, where a second launch begins, with its Q row at element 2^32 of the map (17 GB, two elements a pack)."""
+    note("rope append across 2^32 elements")
+    n_seq, D, cap = 35, 8, 4
+    k0, v0 = 1024, 2048
+    kb = [4096 + s * 2 * cap * D for s in range(n_seq)]
+    top = 1 << 32
+    rng = np.random.default_rng(4)
+    q, kv = rng.standard_normal((n_seq, D)).astype(np.float32), rng.standard_normal((2, n_seq, D)).astype(np.float32)
+    got = []
+    try:
+        for packs, q0 in ((top // 2 + 64, top - 32 * D), (1 << 13, 12288)):
+            hip.map_create_typed(0, A.DTYPE_F32, 2, packs)
+            hip.set_dtype(A.DTYPE_F32)
+            for at, x in ((q0, q), (k0, kv[0]), (v0, kv[1])):
+                assert hip.scatter_contiguous(0, at // 2, x.reshape(-1), n_locs=x.size // 2) == 0
+            hip.rope_append_rows_dev(0, q0, D, 1, k0, D, 1, v0, D, D, 1, kb, [k + cap * D for k in kb], cap * D, 3, 1e4, rotate=True)
+            part = lambda at, n: hip.gather(0, np.arange(at // 2, (at + n) // 2, dtype=np.uint32)).view(np.float32).copy()
+            got.append((part(q0, q.size), part(0, 4096 + n_seq * 2 * cap * D)))
+    finally:
+        f32map(hip, 0, 64)
+    assert not np.array_equal(got[0][0], q.reshape(-1))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("B,Hq,Hk,D", [(8, 32, 8, 128), (5, 16, 2, 64), (3, 32, 8, 128)])
 def test_wide_rotation_takes_few_key_rows_and_copies_along(hip, monkeypatch, B, Hq, Hk, D):
     """One token of B sequences: more than 64 Q rows beside at most 64 K rows and copies still rotate and append in one launch, and
