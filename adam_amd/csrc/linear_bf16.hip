@@ -262,7 +262,7 @@ enum { LEPI_STORE = 0, LEPI_ADD = 1, LEPI_PAIR = 2, LEPI_ARGMAX = 3 };
 template <int EPI, int U>
 __global__ void __launch_bounds__(512)
 k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t n_tasks, const uint32_t* __restrict__ row_idx,
-            float* best_val, uint32_t* best_idx) {
+            float* best_val, uint32_t* best_idx, uint32_t row) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ float inv[LIN_MAX_GROUPS];
   __shared__ float part[32];
@@ -287,7 +287,7 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
   uint32_t task = blockIdx.x * 8u + wave, k0 = lane * 8u, r0, r1;
   rows_of(min(task, n_tasks - 1u), r0, r1);
   fetch(r0, r1, k0);
-  operand_row<512, (U > 1)>(s, act, row_idx ? row_idx[0] : 0u, blockIdx.x == 0u, inv, part,
+  operand_row<512, (U > 1)>(s, act, row_idx ? row_idx[0] : row, blockIdx.x == 0u, inv, part,
                    [&](uint32_t i, float v) { xs[((i >> 2) & 1u) * half + (i >> 3) * 4u + (i & 3u)] = v; },
                    [&](uint32_t c, f4_t v) { *(f4_t*)(xs + (c & 1u) * half + (c >> 1) * 4u) = v; });
   __syncthreads();
@@ -834,7 +834,7 @@ static int launch_tiles(const bf16_t* W, const bf16_t* X, float* act, T* op, con
 static uint32_t gemv_grid(uint32_t n_tasks) { return std::min<uint32_t>(cdiv(n_tasks, 8), 2u * (uint32_t)g.n_cu); }
 
 template <int EPI>
-static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_idx, uint32_t n_tasks) {
+static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_idx, uint32_t n_tasks, uint32_t row = 0u) {
   const uint32_t grid = gemv_grid(n_tasks);
   const size_t lds = (size_t)s.k_stride * 4;
   const bf16_t* W = (const bf16_t*)mw->buf + s.w;
@@ -842,8 +842,8 @@ static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_
   uint32_t* bi = bv ? (uint32_t*)(bv + grid) : nullptr;
   if (s.k_stride >= 1024u) {
     if (lds > 60000) hipFuncSetAttribute((const void*)k_gemv_bf16<EPI, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    k_gemv_bf16<EPI, 4><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi);
-  } else k_gemv_bf16<EPI, 1><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi);
+    k_gemv_bf16<EPI, 4><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi, row);
+  } else k_gemv_bf16<EPI, 1><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi, row);
   count_launch();
 }
 
@@ -981,9 +981,7 @@ int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint3
     const uint32_t n_tasks = cdiv(s->n, 2), grid = gemv_grid(n_tasks);
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
     for (uint32_t i = 0; i < rows; i++) {
-      LinSpec one = *s;                                       // (row i of no list)
-      if (!dev) { one.src += i * s->src_stride; one.gate += i * s->gate_stride; one.branch += i * s->branch_stride; one.res_out += i * s->res_stride; one.keep += i * s->keep_stride; }
-      gemv_launch<LEPI_ARGMAX>(ma, mw, one, dev ? dev + i : nullptr, n_tasks);
+      gemv_launch<LEPI_ARGMAX>(ma, mw, *s, dev ? dev + i : nullptr, n_tasks, i);
       k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[i], nullptr);
       count_launch();
     }

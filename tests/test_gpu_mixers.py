@@ -13,7 +13,7 @@ from adam_amd import adamah as A
 from adam_amd.engine import GenerationConfig
 from adam_amd.mixer_engine import MixerEngine
 from adam_amd.models import load_engine, vomotar_config
-from adam_amd.safetensors_file import f32_to_bf16
+from adam_amd.safetensors_file import bf16_to_f32, f32_to_bf16
 from gpu_util import f32map, note, read, rel_l2, up
 from mixer_cases import CONFIGS, config, delta, floats, par, rel, weights, write_model
 from mixer_pair import CA, OP, ST, WS, WT, Pair
@@ -806,3 +806,31 @@ def test_heads_of_several_rows_are_the_one_row_head(hip, k, n, rows, listed, bra
     assert np.abs(got - last).max() < 64 * 2.0 ** -24 * np.abs(last).max()
     with pytest.raises(RuntimeError):
         hip.linear_argmax_rows_dev(WS, OP, WT, up(hip, A.LinearSpec(**dict(s, src=tok)).words()), up(hip, at) if listed else 0, up(hip, tok + 1 + np.arange(rows)), rows)
+
+
+def test_heads_of_rows_beyond_2_to_the_32_elements(hip):
+    """Rows too long to go several at a time, the second one at element 2^32 of the activation map (17 GB, two elements a pack), with no
+    list of rows."""
+    note("heads of rows across 2^32 elements")
+    k, ks, n, top = 20000, 20032, 40, 1 << 32
+    rng = np.random.default_rng(6)
+    w = np.zeros((n, ks), np.float32)
+    w[:, :k] = rng.standard_normal((n, k))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * ks)
+    hip.scatter_contiguous(WT, 0, f32_to_bf16(w.reshape(-1)))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, 8)
+    x = rng.standard_normal((2, k)).astype(np.float32)
+    got = []
+    try:
+        for packs, at in ((top // 2 + k, top - k), (1 << 16, 4096)):
+            hip.map_create_typed(WS, A.DTYPE_F32, 2, packs)
+            hip.set_dtype(A.DTYPE_F32)
+            assert hip.scatter_contiguous(WS, at // 2, x.reshape(-1), n_locs=x.size // 2) == 0
+            s = A.LinearSpec(n=n, k=k, k_stride=ks, w=0, src=at, src_stride=k, out=64, out_stride=n, groups=1, eps=1e-5)
+            hip.linear_argmax_rows_dev(WS, OP, WT, up(hip, s.words()), 0, up(hip, [0, 1]), 2)
+            got.append(hip.gather(WS, np.arange(0, 32 + n // 2, dtype=np.uint32)).view(np.float32).copy())
+    finally:
+        f32map(hip, WS, 64)
+    want = (x / np.sqrt((x.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-5)) @ bf16_to_f32(f32_to_bf16(w[:, :k].reshape(-1))).reshape(n, k).T.astype(np.float64)
+    assert got[0][:2].tolist() == want.argmax(1).tolist() == got[1][:2].tolist()
+    assert np.array_equal(got[0], got[1]) and rel_l2(got[0][64:64 + n], want[1]) < 1e-5
