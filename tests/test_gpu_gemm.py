@@ -612,9 +612,11 @@ def test_few_rows_on_every_operand_and_weight_tile(hip, M, N, K):
                 assert rel_l2(y[op, m], want[m]) < TOL_Q4, (op, m)
 
 
-@pytest.mark.parametrize("M,K,Ns", [(6, 1152, (3000, 3000)), (24, 256, (40, 24, 16)), (48, 640, (4000, 100)), (64, 384, (70,))])
+@pytest.mark.parametrize("M,K,Ns", [(6, 1152, (3000, 3000)), (24, 256, (40, 24, 16)), (48, 640, (4000, 100)), (64, 384, (70,)), (3, 256, (8209,)), (13, 640, (90,)),
+                                    (33, 128, (100,)), (40, 1152, (4100,)), (48, 256, (8200,)), (49, 640, (4090,)), (64, 4224, (31,))])
 def test_few_rows_store_stacked_results_and_adds(hip, M, K, Ns):
-    """The kernel of few rows places the results of stacked matrices and, over one matrix, stores the add that consumes them."""
+    """The kernel of few rows places the results of stacked matrices and, over one matrix, stores the add that consumes them: the
+    conversion and one launch (of 33 to 64 rows the tiled kernel would leave the add, or take a launch for its shares' sums)."""
     rng = np.random.default_rng(M + K)
     N = sum(Ns)
     qt = quant.quantize_q4_0(rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05))
@@ -632,6 +634,7 @@ def test_few_rows_store_stacked_results_and_adds(hip, M, K, Ns):
         span = lambda lo: up(hip, np.arange(lo, lo + M * N))
         hip.map_op2_dev(0, A.OP_ADD, span(res), span(M * K), span(res), M * N)
     hip.batch_end()
+    assert hip.get_last_barrier_count() == 2
     for i, n in enumerate(Ns):
         got = read(hip, 0, M * K + int(at[i]), M * n).reshape(M, n)
         assert rel_l2(got, want[:, first[i]:first[i + 1]]) < TOL_Q4, i

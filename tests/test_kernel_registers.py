@@ -35,7 +35,11 @@ def descriptions():
 
 
 @pytest.mark.parametrize("part,most", [("k_attn_f32", 0), ("k_chunk_scan", 0), ("k_space_scan", 0), ("k_linear_tiled", 0), ("k_linear_skinny", 0),
-                                       ("k_experts", 0), ("k_operand_rows", 0), ("k_gemm_q4_ring", 16)])
+                                       ("k_experts", 0), ("k_operand_rows", 0), ("k_gemm_q4_ring", 16), ("k_gemm_q4_rows", 0), ("k_gemm_q8_f16", 0),
+                                       ("k_head_rows", 0), ("k_delta", 0), ("k_rmsnorm_rows", 0), ("k_rope_append_rows", 0), ("k_kv_tile_arrange", 0),
+                                       ("k_attn_prefill", 0), ("k_topk_select", 0),
+                                       # heads of up to 128 two tiles of queries a wave; wider ones spill at 256 registers, heads of 256 by 256 most
+                                       ("k_attn_bf16ILb0ELi4ELi8E", 0), ("k_attn_bf16ILb1ELi4ELi8E", 12), ("k_attn_bf16", 412)])
 def test_arrays_stay_in_registers(part, most):
     """An array that a loop indexes and the compiler does not unroll lands in memory and is read from there in every step (the
     float32 attention of heads wider than 128 ran 1.4 times slower than with its loads in place).  `most`: bytes a lane."""
