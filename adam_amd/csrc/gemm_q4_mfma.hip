@@ -1058,12 +1058,13 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
 struct GluSrc { uint32_t op, a, b, d; };
 template <int NW, bool GLU>
 __global__ void __launch_bounds__(1024)
-k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_t a_by_val, uint4* xf, float* scale,
-               float* act_out, const uint32_t* __restrict__ la, GluSrc glu, ActForm form, uint32_t parts) {
-  // (a_by_val: the rows start at element a_val -- known on the host -- instead of la[op], a load the rows' loads
-  // would wait for; with GLU a_val is glu.a)
+k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_t by_parts, uint4* xf, float* scale,
+               float* act_out, const uint32_t* __restrict__ la, GluSrc glu, ActForm form) {
+  // (by_parts: act_parts, and below it one bit: the rows start at element a_val -- known on the host -- instead of la[op], a load
+  // the rows' loads would wait for; with GLU a_val is glu.a.  Both are in registers when a wave starts)
   __shared__ float red[16];
   const uint32_t op = blockIdx.y, tid = threadIdx.x, kw = K >> 3;
+  const uint32_t parts = by_parts >> 1;
   uint32_t row = blockIdx.x, w0 = 0, w1 = kw;                // the words this workgroup stores
   if (parts) {
     const uint32_t unit = (blockIdx.x >> 6) * 8u + (blockIdx.x & 7u), share = (kw / parts + 8u) & ~7u;
@@ -1071,7 +1072,7 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
     w0 = unit % parts * share; w1 = min(kw, w0 + share);
     if (row >= M || w0 >= kw) return;
   }
-  const float* x = act + (a_by_val ? (uint64_t)a_val : (uint64_t)la[op]) + (uint64_t)row * K;
+  const float* x = act + (by_parts & 1u ? (uint64_t)a_val : (uint64_t)la[op]) + (uint64_t)row * K;
   f4qu_t v0[NW], v1[NW];
   float m = 0.f;
 #pragma unroll
@@ -1200,8 +1201,8 @@ bool launch_glu_act_f16(const Map* ma, uint32_t op, uint32_t a, uint32_t b, uint
   float* act = (float*)ma->buf;
   const GluSrc glu = {op, a, b, d};
   // (the caller has seen to it that d touches neither a nor b: several workgroups may read a row)
-  if (K <= 8192) k_act_f16_regs<1, true><<<dim3(act_grid(form), 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form, act_parts(form));
-  else k_act_f16_regs<2, true><<<dim3(act_grid(form), 1), 1024, 0, g.stream>>>(act, K, M, a, 1u, xf, scale, act, nullptr, glu, form, act_parts(form));
+  if (K <= 8192) k_act_f16_regs<1, true><<<dim3(act_grid(form), 1), 1024, 0, g.stream>>>(act, K, M, a, 1u | act_parts(form) << 1, xf, scale, act, nullptr, glu, form);
+  else k_act_f16_regs<2, true><<<dim3(act_grid(form), 1), 1024, 0, g.stream>>>(act, K, M, a, 1u | act_parts(form) << 1, xf, scale, act, nullptr, glu, form);
   count_launch();
   gemm_act_mark(ma->buf, d, M, K);
   return true;
@@ -1406,8 +1407,8 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   uint4* const xl = (uint4*)((uint8_t*)g_xh_buf + plane);
   if (!reuse) {
     if (K <= 16384 && knob("ADAMAH_ACT_REGS", 1) != 0) {
-      if (K <= 8192) k_act_f16_regs<1, false><<<dim3(act_grid(form), n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form, act_parts(form));
-      else k_act_f16_regs<2, false><<<dim3(act_grid(form), n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, (a_host >= 0 && n_ops == 1) ? 1u : 0u, xh, g_scale_buf, act, la, GluSrc{}, form, act_parts(form));
+      if (K <= 8192) k_act_f16_regs<1, false><<<dim3(act_grid(form), n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, ((a_host >= 0 && n_ops == 1) ? 1u : 0u) | act_parts(form) << 1, xh, g_scale_buf, act, la, GluSrc{}, form);
+      else k_act_f16_regs<2, false><<<dim3(act_grid(form), n_ops), 1024, 0, g.stream>>>(act, K, M, a_host >= 0 ? (uint32_t)a_host : 0u, ((a_host >= 0 && n_ops == 1) ? 1u : 0u) | act_parts(form) << 1, xh, g_scale_buf, act, la, GluSrc{}, form);
     } else
       k_act_f16<<<dim3(M, n_ops), 256, 0, g.stream>>>(act, la, M, K, g_scale_buf, xh, form);
     count_launch();
