@@ -198,21 +198,6 @@ def test_chunked_prefill_on_the_matrix_cores(hip, arch, chunk):
         assert dev_tok[i] == ref_tok[i] or margins[i] < 1e-4, (i, dev_tok[i], ref_tok[i], margins[i])
 
 
-@pytest.mark.parametrize("head_dim,head_dim_kv", [(16, 32), (5, 5)])
-def test_chunks_of_unequal_and_odd_heads(hip, head_dim, head_dim_kv):
-    """Heads of Q smaller than those of K and V, and of an odd size, in chunks: as token by token on the oracle."""
-    cfg = synth.tiny_config("llama", n_layer=2, n_embd=64, n_head=32, n_head_kv=32, head_dim=head_dim, n_ff=96, n_vocab=160)
-    cfg.head_dim_kv = head_dim_kv
-    tensors = synth.make_model(cfg, seed=3, sigma=0.1)
-    prompt = [5, 17, 3, 101, 64, 9]
-    ref = DecodeEngine(oracle.init(), cfg, tensors, A=A, kv_cap=32, kv_fp16=True)
-    ref.prefill(prompt)
-    note(f"engine chunks of heads {head_dim} / {head_dim_kv}")
-    dev = DecodeEngine(hip, cfg, tensors, A=A, kv_cap=32, kv_fp16=True, prefill_chunk=4)
-    dev.prefill(prompt)
-    assert rel_l2(dev.read_slot('hidden'), ref.read_slot('hidden')) < 1e-3
-
-
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
 def test_batched_lockstep_decode(hip, arch):
     """Four sequences in lockstep on the HIP library (projections as [4, K] matmuls on the matrix cores,
@@ -363,16 +348,14 @@ def test_a_plan_called_with_the_same_step_is_not_recorded():
 
 
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
-@pytest.mark.parametrize("chunk,P", [(64, 20), (45, 20), (160, 40), (110, 35), (4, 1)])
-def test_prompts_of_a_batch_go_through_the_weights_together(hip, monkeypatch, arch, chunk, P):
-    """Four prompts of 20 tokens at 64 rows (three at once, one left over) and at 45 (two and two), of 40 and 35 at 160 and 105 rows on
-    the ring matmul, and of one token: the tokens that follow and the caches are those of the prompts one by one, up to the rounding of
-    matmuls of other row counts."""
-    monkeypatch.setenv("ADAMAH_GEMM_RING", "2")              # more than 64 rows: always the ring
+@pytest.mark.parametrize("chunk", [64, 45])
+def test_prompts_of_a_batch_go_through_the_weights_together(hip, arch, chunk):
+    """Four prompts of 20 tokens at 64 rows (three at once, one left over) and at 45 (two and two): the tokens that follow and the
+    caches are those of the prompts one by one, up to the rounding of matmuls of other row counts."""
     cfg = synth.tiny_config(arch, n_layer=3, n_embd=256, n_head=4, n_head_kv=2, head_dim=64, n_ff=512, n_vocab=1000)
     tensors = synth.make_model(cfg, seed=5, sigma=0.1)
     rng = np.random.default_rng(3)
-    prompts = [[int(t) for t in rng.integers(0, 1000, P)] for _ in range(4)]
+    prompts = [[int(t) for t in rng.integers(0, 1000, 20)] for _ in range(4)]
     outs = []
     for together in (False, True):
         note(f"engine prompts together={together} {arch} chunk={chunk}")
@@ -385,3 +368,59 @@ def test_prompts_of_a_batch_go_through_the_weights_together(hip, monkeypatch, ar
     # a cached value is rounded to fp16: neighbours of a rounding edge differ by one unit in the last place
     assert np.linalg.norm(outs[1][2] - outs[0][2]) < 1e-4 * np.linalg.norm(outs[0][2])
     assert np.linalg.norm(outs[1][3] - outs[0][3]) < 1e-3 * np.linalg.norm(outs[0][3])
+
+
+_PACKED_SNIPPET = """
+import sys, json
+sys.path.insert(0, {root!r})
+import numpy as np
+from adam_amd import adamah as A, synth
+from adam_amd.engine import DecodeEngine
+gpu, out = A.init(), []
+for arch, chunk, P in (("llama", 70, 35), ("gemma3", 99, 33), ("llama", 4, 1), ("gemma3", 3, 1)):
+    cfg = synth.tiny_config(arch, n_layer=3, n_embd=256, n_head=4, n_head_kv=2, head_dim=64, n_ff=512, n_vocab=1000)
+    tensors = synth.make_model(cfg, seed=5, sigma=0.1)
+    rng = np.random.default_rng(3)
+    prompts = [[int(t) for t in rng.integers(0, 1000, P)] for _ in range(4)]
+    runs = []
+    for together in (False, True):
+        print("prompts", arch, chunk, P, together, file=sys.stderr, flush=True)
+        dev = DecodeEngine(gpu, cfg, tensors, A=A, kv_cap=64, kv_fp16=True, batch=4, prefill_chunk=chunk)
+        dev._prompts_together = together
+        first = dev._prefill_prompts(prompts)
+        kv = gpu.gather(0, np.arange(dev._kv_start, dev._kv_start + 4 * dev._kv_per_seq, dtype=np.uint32)).view(np.float32)
+        runs.append((first, dev.read_token(), kv, dev.read_slot('hidden')))
+    (f0, t0, k0, h0), (f1, t1, k1, h1) = runs
+    d = lambda a, b: float(np.linalg.norm(a.astype(np.float64) - b) / np.linalg.norm(a.astype(np.float64)))
+    out.append([f0 == f1 and t0 == t1 == f1[-1], d(k0, k1), d(h0, h1)])
+heads = []
+import oracle
+for head_dim, head_dim_kv in ((16, 32), (5, 5)):
+    print("heads", head_dim, head_dim_kv, file=sys.stderr, flush=True)
+    cfg = synth.tiny_config("llama", n_layer=2, n_embd=64, n_head=32, n_head_kv=32, head_dim=head_dim, n_ff=96, n_vocab=160)
+    cfg.head_dim_kv = head_dim_kv
+    tensors = synth.make_model(cfg, seed=3, sigma=0.1)
+    ref = DecodeEngine(oracle.init(), cfg, tensors, A=A, kv_cap=32, kv_fp16=True)
+    ref.prefill([5, 17, 3, 101, 64, 9])
+    dev = DecodeEngine(gpu, cfg, tensors, A=A, kv_cap=32, kv_fp16=True, prefill_chunk=4)
+    dev.prefill([5, 17, 3, 101, 64, 9])
+    heads.append(d(ref.read_slot('hidden'), dev.read_slot('hidden')))
+gpu.shutdown()
+print(json.dumps([out, heads]))
+"""
+
+
+def test_packed_prompts_on_the_ring_matmul_of_one_token_and_chunks_of_odd_heads():
+    """Prompts of 35 and 33 tokens two and three at a time, 70 and 99 rows on the ring matmul (ADAMAH_GEMM_RING=2: always beyond 64 rows;
+    one by one they have no more than 64), and prompts of one token: as one by one.  Heads of Q smaller than those of K and V, and of
+    an odd size, in chunks: as token by token on the oracle.  In a process with handles of its own."""
+    import json, os, subprocess, sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    note("packed prompts on the ring matmul")
+    p = subprocess.run([sys.executable, "-c", _PACKED_SNIPPET.format(root=root)], capture_output=True, text=True, timeout=100,
+                       env=dict(os.environ, ADAMAH_GEMM_RING="2"))
+    assert p.returncode == 0, p.stderr[-2000:]
+    packed, heads = json.loads(p.stdout.strip().splitlines()[-1])
+    for same, kv, hidden in packed:
+        assert same and kv < 1e-4 and hidden < 1e-3
+    assert max(heads) < 1e-3

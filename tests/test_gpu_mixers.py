@@ -753,6 +753,7 @@ def test_a_portion_has_the_same_sums_beside_others(hip, H, G, D, V, C, rows, n_s
     spec = lambda i: up(hip, A.ChunkAttnSpec(heads=H, kv_heads=G, dim=D, vdim=V, chunk=C, x=i * rows * xs, x_stride=xs, x_q=0, x_k=H * D, x_v=(H + G) * D, r1=ro,
                                              r2=ro + H, scale=0.25, eps=1e-4, out=oo + i * rows * H * V, out_stride=H * V, cache_map=CA, k_off=0, v_off=kc,
                                              seq_stride=ss).words())
+    specs = [spec(i) for i in range(n_seq)]
     got = []
     for together in (False, True):
         hip.map_create_typed(CA, A.DTYPE_F32 if dtype == "float32" else A.DTYPE_BF16, 1, n_seq * ss)
@@ -761,10 +762,10 @@ def test_a_portion_has_the_same_sums_beside_others(hip, H, G, D, V, C, rows, n_s
         for i, xi in enumerate(x):
             hip.scatter_contiguous(WS, 0, xi)
             if together:
-                hip.chunk_attention_seqs_dev(WS, spec(0), n_seq, rows, 0, i * rows)
+                hip.chunk_attention_seqs_dev(WS, specs[0], n_seq, rows, 0, i * rows)
             else:
                 for q in range(n_seq):
-                    hip.chunk_attention_dev(WS, spec(q), 1, rows, q, i * rows)
+                    hip.chunk_attention_dev(WS, specs[q], 1, rows, q, i * rows)
             words.append(read(hip, WS, oo, n_seq * rows * H * V).view(np.uint32).copy())
         got.append(words)
     for a, b in zip(*got):
