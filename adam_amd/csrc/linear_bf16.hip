@@ -262,7 +262,7 @@ enum { LEPI_STORE = 0, LEPI_ADD = 1, LEPI_PAIR = 2, LEPI_ARGMAX = 3 };
 template <int EPI, int U>
 __global__ void __launch_bounds__(512)
 k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t n_tasks, const uint32_t* __restrict__ row_idx,
-            float* best_val, uint32_t* best_idx, uint32_t row) {
+            float* best_val, uint32_t* best_idx) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ float inv[LIN_MAX_GROUPS];
   __shared__ float part[32];
@@ -287,7 +287,7 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t 
   uint32_t task = blockIdx.x * 8u + wave, k0 = lane * 8u, r0, r1;
   rows_of(min(task, n_tasks - 1u), r0, r1);
   fetch(r0, r1, k0);
-  operand_row<512, (U > 1)>(s, act, row_idx ? row_idx[0] : row, blockIdx.x == 0u, inv, part,
+  operand_row<512, (U > 1)>(s, act, row_idx ? row_idx[0] : 0u, blockIdx.x == 0u, inv, part,
                    [&](uint32_t i, float v) { xs[((i >> 2) & 1u) * half + (i >> 3) * 4u + (i & 3u)] = v; },
                    [&](uint32_t c, f4_t v) { *(f4_t*)(xs + (c & 1u) * half + (c >> 1) * 4u) = v; });
   __syncthreads();
@@ -834,7 +834,7 @@ static int launch_tiles(const bf16_t* W, const bf16_t* X, float* act, T* op, con
 static uint32_t gemv_grid(uint32_t n_tasks) { return std::min<uint32_t>(cdiv(n_tasks, 8), 2u * (uint32_t)g.n_cu); }
 
 template <int EPI>
-static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_idx, uint32_t n_tasks, uint32_t row = 0u) {
+static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_idx, uint32_t n_tasks) {
   const uint32_t grid = gemv_grid(n_tasks);
   const size_t lds = (size_t)s.k_stride * 4;
   const bf16_t* W = (const bf16_t*)mw->buf + s.w;
@@ -842,8 +842,8 @@ static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_
   uint32_t* bi = bv ? (uint32_t*)(bv + grid) : nullptr;
   if (s.k_stride >= 1024u) {
     if (lds > 60000) hipFuncSetAttribute((const void*)k_gemv_bf16<EPI, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    k_gemv_bf16<EPI, 4><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi, row);
-  } else k_gemv_bf16<EPI, 1><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi, row);
+    k_gemv_bf16<EPI, 4><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi);
+  } else k_gemv_bf16<EPI, 1><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi);
   count_launch();
 }
 
@@ -977,14 +977,12 @@ int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint3
   // rows at a time: as many as 144 KB of LDS hold (a workgroup a CU), none of them for nothing
   const size_t row_bytes = (size_t)s->k_stride * 4;
   const uint32_t fit = (uint32_t)(((size_t)144 << 10) / row_bytes), nr = fit >= 8 && rows > 4 ? 8 : fit >= 4 && rows > 2 ? 4 : fit >= 2 && rows > 1 ? 2 : 1;
-  if (nr == 1) {
+  if (rows == 1) {
     const uint32_t n_tasks = cdiv(s->n, 2), grid = gemv_grid(n_tasks);
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
-    for (uint32_t i = 0; i < rows; i++) {
-      gemv_launch<LEPI_ARGMAX>(ma, mw, *s, dev ? dev + i : nullptr, n_tasks, i);
-      k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[i], nullptr);
-      count_launch();
-    }
+    gemv_launch<LEPI_ARGMAX>(ma, mw, *s, dev, n_tasks);
+    k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0], nullptr);
+    count_launch();
     return check_launch();
   }
   const uint32_t n_tasks = cdiv(s->n, 4), grid = std::min<uint32_t>(cdiv(n_tasks, 8), (uint32_t)g.n_cu);
@@ -1002,7 +1000,7 @@ int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint3
     hipFuncSetAttribute((const void*)k_head_rows<NR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(NR * row_bytes)); \
     k_head_rows<NR><<<grid, 512, NR * row_bytes, g.stream>>>(W, act, *s, X + (size_t)i * s->k_stride, n, kept, n_tasks, bv + (size_t)i * grid, bi + (size_t)i * grid); \
   } while (0)
-    if (nr == 8) HEAD(8); else if (nr == 4) HEAD(4); else HEAD(2);
+    if (nr == 8) HEAD(8); else if (nr == 4) HEAD(4); else if (nr == 2) HEAD(2); else HEAD(1);
 #undef HEAD
     count_launch();
   }
