@@ -62,8 +62,8 @@ __device__ __forceinline__ void split_word(const float* v, uint4* hi, uint4* lo)
 
 // The activations are converted once per matmul (or by the kernel that produced them) to the two fp16
 // planes the matrix cores consume: rows scaled by their power of two, elements of every 8-word in the
-// order (0,4)(1,5)(2,6)(3,7).  The matmul workgroups then copy 16-byte pieces into LDS.  One workgroup per
-// row; also stores (s, 1/s).  xl = second plane (same indexing as xh).
+// order (0,4)(1,5)(2,6)(3,7), in the places that `form` gives them (rows of both planes, or operand tiles).  One workgroup per
+// row; also stores (s, 1/s).
 __global__ void __launch_bounds__(256)
 k_act_f16(const float* act, const uint32_t* __restrict__ la, uint32_t M, uint32_t K, float* scale, uint4* x, ActForm form) {
   __shared__ float red[4];
@@ -1121,13 +1121,13 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
 }
 
 static float* g_scale_buf = nullptr;
-static uint4* g_xh_buf = nullptr;     // fp16 activations: first plane, then the second plane at g_xh_plane bytes
-static size_t g_xh_cap = 0;           // in bytes (both planes)
+static uint4* g_xh_buf = nullptr;     // fp16 activations, both planes, as their ActForm places them
+static size_t g_xh_cap = 0;           // in bytes
 static size_t g_scale_cap = 0;
 // The rows last converted into g_xh_buf / g_scale_buf, and the launch and upload counts right after the
 // matmul that used them: while both counts stand still nothing has written device memory since, so a
-// matmul over the same rows (K and V after Q, up after gate) skips the conversion launch.  plane = byte
-// offset of the second plane those rows were written with.
+// matmul over the same rows (K and V after Q, up after gate) skips the conversion launch.  (The form
+// follows from M and K; plane = bytes of one plane.)
 static struct { const void* buf; uint64_t a; uint32_t M, K; uint64_t dispatch, mem_gen; size_t plane; bool valid; } g_xh_key = {};
 
 static float* g_part_buf = nullptr;   // raw sums of the shares of a K-split launch
@@ -1433,8 +1433,9 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     return check_launch();
   }
   // 9 .. 16 activation rows and workgroups of 128 weight rows for three quarters of the CUs: the form whose eight waves share an
-  // activation tile in LDS (us, this and k_gemm_q4_rows: 16 rows 28672 x 4096 23.8 and 24.1, 65536 x 2048 25.3 and 30.1; 9 rows 24.8 and
-  // 24.1, 24.9 and 29.5; 8 rows 24.9 and 19.9, 25.1 and 21.3)
+  // activation tile in LDS (us, this and k_gemm_q4_rows with four tiles: 16 rows 28672 x 4096 23.8 and 24.1, 65536 x 2048 25.3 and 30.1; 9 rows 24.8 and
+  // 24.1, 24.9 and 29.5; 8 rows 24.9 and 19.9, 25.1 and 21.3.  With two tiles a workgroup k_gemm_q4_rows takes 22.7, 24.0, 22.0 and 22.5
+  // for the four of 16 and 9 rows: the line is older than that)
   const uint32_t wgs16 = cdiv(sg.glu ? N / 2 : N, sg.glu ? 64u : 128u);
   if (form.tiles == 2 && !sg.add && (uint64_t)wgs16 * 4 >= 3ull * cu && tuning("ADAMAH_GEMM_ROWS16", 1) != 0) {
     k_gemm_q4_f16_rows16<8><<<dim3(wgs16, 1, n_ops), 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, form.tiles | form.rows << 8, K, N, M, b_val, c_val, by_dst,
