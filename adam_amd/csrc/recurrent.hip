@@ -474,18 +474,24 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 }
 
 // ---- the walk over the chunks ---------------------------------------------------------------------------------------
-// A serial chain, so what counts is a chunk's latency: 2048 tokens in 32 heads of 128 took 236 us = 1.85 us a chunk with the
-// next one's operands under a condition (the wait at its end is for everything asked for), 157-170 so, 144 with the operands in
-// lane order (16 sequences of 12 tokens 54 and 39.5).
-// Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
-// is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.
+// A serial chain, so what counts is a chunk's latency.  Four waves share the state rows (NT tiles of 16 each); a tile's
+// accumulator holds rows 4 g + i of lane group g, which is also how instruction i wants its right operand when the left one is
+// read as four consecutive columns per lane.  On their chain are only the products that the state needs (delta: W S, its sum
+// through LDS, K u); Q S and a quarter of B u, the wave's share of the outputs, go out while that sum is on its way.  A fifth
+// wave adds up the shares and stores them, a chunk behind: loads and stores share a counter, and a wave that does both waits
+// for its stores.  2048 tokens in 32 heads of 128, warm: outputs by the first of four waves, ahead of its part of the state, 127 us,
+// retention 93; so 105 and 76 (without any output 96 and 68, without loads either 86 and 61: what is left is 25 instructions
+// of 32 clocks, an exchange through LDS and its barrier a chunk).
+// FEW: one or two chunks, whose operands are not asked for ahead, so that a compute unit has three workgroups instead of two (16
+// sequences of 12 tokens 26.5 us, 48.5 with the other form, 38.6 before).
 struct ScanArgs {
   uint32_t heads, dim, vdim, out, out_stride, s_off, m, pos;
   ChunkDims cd;
   uint32_t kv_heads, taps, conv_off, x, x_stride;     // delta: the convolution's ring is brought up to date here
   uint32_t seq_stride;                                // of the state; grid z: the sequence, its rows m z .. of the activations
 };
-template <int NT> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], b, u; };
+#define SCAN_T 320u          // four waves of state rows and the one of the outputs
+template <int NT> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], u; float b; };
 
 template <bool DELTA, int NT>
 __device__ __forceinline__ void load_ops(ChunkOps<NT>& o, const float* blk, const ChunkDims& cd, uint32_t wave, uint32_t lane, uint32_t v0) {
@@ -498,99 +504,119 @@ __device__ __forceinline__ void load_ops(ChunkOps<NT>& o, const float* blk, cons
     o.k[j] = *(const f4_t*)(pK + at);
     o.gl[j] = *(const f4_t*)(pG + T * 16u + (lane >> 4) * 4u);
   }
-  o.b = *(const f4_t*)(pB + lane * 4u);
   o.u = *(const f4_t*)(pU + v0 * 16u + lane * 4u);
+  o.b = pB[lane * 4u + wave];
 }
 
-template <bool DELTA, int NT>
-__global__ void __launch_bounds__(256)
+template <bool DELTA, int NT, bool FEW>
+__global__ void __launch_bounds__(SCAN_T)
 k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, float* state) {
-  __shared__ f4_t pb[2][2][4][64];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, c = lane & 15u, kg = lane >> 4;
+  __shared__ f4_t p1[2][4][64], p2[2][4][64];                // [chunk & 1][wave][lane]
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, D = a.dim, V = a.vdim, v = v0 + c;
-  const uint32_t bs = chunk_floats(a.cd.Dp, a.cd.Vp);
-  const float* blk = scratch + ((uint64_t)blockIdx.z * a.heads + h) * a.cd.n_chunks * bs;
+  const uint32_t bs = chunk_floats(a.cd.Dp, a.cd.Vp), n = a.cd.n_chunks;
+  const float* blk = scratch + ((uint64_t)blockIdx.z * a.heads + h) * n * bs;
   state += (uint64_t)blockIdx.z * a.seq_stride;
-  float* out = act + a.out + (uint64_t)blockIdx.z * a.m * a.out_stride;
-  float* S = state + a.s_off + (uint64_t)h * D * V;
-  f4_t st[NT];
+  const auto sum4 = [&](const f4_t (*p)[64]) { return (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]); };
+  if (wave == 4u) {
+    float* out = act + a.out + (uint64_t)blockIdx.z * a.m * a.out_stride + h * V + v;
+    for (uint32_t ci = 0; ci <= n; ci++) {
+      __syncthreads();
+      if (ci == 0u) continue;
+      const f4_t o = sum4(p2[(ci - 1u) & 1u]);
 #pragma unroll
-  for (int j = 0; j < NT; j++) st[j] = (f4_t){0, 0, 0, 0};
-  if (a.pos != 0u) {
+      for (int i = 0; i < 4; i++) {
+        const uint32_t r = (ci - 1u) * CH + 4u * kg + i;
+        if (r < a.m && v < V) out[(uint64_t)r * a.out_stride] = o[i];
+      }
+    }
+  } else {
+    float* S = state + a.s_off + (uint64_t)h * D * V;
+    f4_t st[NT];
 #pragma unroll
-    for (int j = 0; j < NT; j++)
+    for (int j = 0; j < NT; j++) st[j] = (f4_t){0, 0, 0, 0};
+    if (a.pos != 0u) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) st[j][i] = S[(uint64_t)min((wave * NT + j) * 16u + 4u * kg + i, D - 1u) * V + min(v, V - 1u)];
+      for (int j = 0; j < NT; j++)
 #pragma unroll
-    for (int j = 0; j < NT; j++)
+        for (int i = 0; i < 4; i++) st[j][i] = S[(uint64_t)min((wave * NT + j) * 16u + 4u * kg + i, D - 1u) * V + min(v, V - 1u)];
 #pragma unroll
-      for (int i = 0; i < 4; i++) if ((wave * NT + j) * 16u + 4u * kg + i >= D || v >= V) st[j][i] = 0.f;
-  }
-  const uint32_t n = a.cd.n_chunks;
-  // the operands of the chunk two ahead, asked for on every path (past the end: the last one's again)
-  const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, lane, v0); };
-  const auto chunk = [&](const ChunkOps<NT>& cur, uint32_t ci, f4_t (*pb)[4][64]) {
-    f4_t p1 = {0, 0, 0, 0}, p2 = {0, 0, 0, 0};
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) if ((wave * NT + j) * 16u + 4u * kg + i >= D || v >= V) st[j][i] = 0.f;
+    }
+    // the operands of the chunk two ahead, asked for on every path (past the end: the last one's again)
+    const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, lane, v0); __builtin_amdgcn_sched_barrier(0); };
+    const auto chunk = [&](const ChunkOps<NT>& cur, uint32_t x) {
+      f4_t u = cur.u;
+      if (DELTA) {                                           // (two sums: an instruction waits for the one that it adds to)
+        f4_t s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) s[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], s[i & 1], 0, 0, 0);
+        p1[x][wave][lane] = s[0] + s[1];
+      }
+      __syncthreads();
+      f4_t r[4];
+      if (DELTA)
+#pragma unroll
+        for (int w = 0; w < 4; w++) r[w] = p1[x][w][lane];
+      __builtin_amdgcn_sched_barrier(0);                     // Q S behind them, not ahead of the barrier
+      f4_t s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], s[i & 1], 0, 0, 0);
+      if (DELTA) u -= (r[0] + r[1]) + (r[2] + r[3]);
+#pragma unroll
+      for (int j = 0; j < NT; j++) st[j] *= cur.gl[j];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][i], u[i], st[j], 0, 0, 0);
+      s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b, wave & 2u ? (wave & 1u ? u[3] : u[2]) : (wave & 1u ? u[1] : u[0]), s[0], 0, 0, 0);
+      p2[x][wave][lane] = s[0] + s[1];
+    };
+    ChunkOps<NT> o0;
+    ask(o0, 0);
+    if constexpr (FEW) {
+      for (uint32_t ci = 0; ci < n; ci++) {
+        if (ci) ask(o0, ci);
+        chunk(o0, ci & 1u);
+      }
+    } else {
+      // (a loop in one piece: with a way out behind each chunk the loads were moved down to where only the rest of the loop needs them)
+      ChunkOps<NT> o1, o2;
+      ask(o1, 1); ask(o2, 2);
+      uint32_t ci = 0;
+      for (; ci + 3u <= n; ci += 3u) {
+        chunk(o0, ci & 1u);
+        ask(o0, ci + 3u);
+        chunk(o1, (ci + 1u) & 1u);
+        ask(o1, ci + 4u);
+        chunk(o2, ci & 1u);
+        ask(o2, ci + 5u);
+      }
+      if (ci < n) chunk(o0, ci & 1u);
+      if (ci + 1u < n) chunk(o1, (ci + 1u) & 1u);
+    }
+    __syncthreads();                                         // the last chunk's Q S is there
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        if (DELTA) p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], p1, 0, 0, 0);
-        p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], p2, 0, 0, 0);
+        const uint32_t d = (wave * NT + j) * 16u + 4u * kg + i;
+        if (d < D && v < V) S[(uint64_t)d * V + v] = st[j][i];
       }
-    if (DELTA) pb[0][wave][lane] = p1;
-    pb[1][wave][lane] = p2;
-    __syncthreads();
-    f4_t u = cur.u;
-    if (DELTA) {
-      const f4_t* r = &pb[0][0][0];
-      u -= (r[lane] + r[64 + lane]) + (r[128 + lane] + r[192 + lane]);
-    }
-    if (wave == 0u) {
-      const f4_t* r = &pb[1][0][0];
-      f4_t o = (r[lane] + r[64 + lane]) + (r[128 + lane] + r[192 + lane]);
-#pragma unroll
-      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[i], u[i], o, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint32_t r2 = ci * CH + 4u * kg + i;
-        if (r2 < a.m && v < V) out[(uint64_t)r2 * a.out_stride + h * V + v] = o[i];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-      st[j] *= cur.gl[j];
-#pragma unroll
-      for (int i = 0; i < 4; i++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][i], u[i], st[j], 0, 0, 0);
-    }
-  };
-  ChunkOps<NT> o0, o1, o2;
-  ask(o0, 0); ask(o1, 1); ask(o2, 2);
-  for (uint32_t ci = 0;; ci += 3u) {
-    chunk(o0, ci, pb[ci & 1u]);
-    if (ci + 1u >= n) break;
-    ask(o0, ci + 3u);
-    chunk(o1, ci + 1u, pb[(ci + 1u) & 1u]);
-    if (ci + 2u >= n) break;
-    ask(o1, ci + 4u);
-    chunk(o2, ci + 2u, pb[ci & 1u]);
-    if (ci + 3u >= n) break;
-    ask(o2, ci + 5u);
   }
-#pragma unroll
-  for (int j = 0; j < NT; j++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t d = (wave * NT + j) * 16u + 4u * kg + i;
-      if (d < D && v < V) S[(uint64_t)d * V + v] = st[j][i];
-    }
   if (!DELTA) return;
   const uint32_t n_ch = 2u * a.kv_heads * D + a.heads * V, rep = a.heads / a.kv_heads, kv = h / rep;
   for (uint32_t r = a.m > a.taps ? a.m - a.taps : 0u; r < a.m; r++) {
     float* slot = state + a.conv_off + (uint64_t)((a.pos + r) % a.taps) * n_ch;
     const float* x = act + a.x + ((uint64_t)blockIdx.z * a.m + r) * a.x_stride;
     if (blockIdx.y == 0 && h % rep == 0)
-      for (uint32_t d = tid; d < D; d += 256u) {
+      for (uint32_t d = tid; d < D; d += SCAN_T) {
         slot[kv * D + d] = x[kv * D + d];
         slot[(a.kv_heads + kv) * D + d] = x[(a.kv_heads + kv) * D + d];
       }
@@ -610,13 +636,17 @@ template <bool DELTA>
 static int launch_scan(const ScanArgs& a, float* act, float* state, uint32_t n_seq) {
   const dim3 grid(a.heads, cdiv(a.vdim, 16), n_seq);
   const float* sc = (const float*)g_chunks.p;
+  const bool few = a.cd.n_chunks <= 2u;        // (above)
+#define SCAN(NT) do { if (few) k_chunk_scan<DELTA, NT, true><<<grid, SCAN_T, 0, g.stream>>>(a, sc, act, state); \
+                      else k_chunk_scan<DELTA, NT, false><<<grid, SCAN_T, 0, g.stream>>>(a, sc, act, state); } while (0)
   switch (a.cd.Dp / 64u) {
-    case 1: k_chunk_scan<DELTA, 1><<<grid, 256, 0, g.stream>>>(a, sc, act, state); break;
-    case 2: k_chunk_scan<DELTA, 2><<<grid, 256, 0, g.stream>>>(a, sc, act, state); break;
-    case 3: k_chunk_scan<DELTA, 3><<<grid, 256, 0, g.stream>>>(a, sc, act, state); break;
-    case 4: k_chunk_scan<DELTA, 4><<<grid, 256, 0, g.stream>>>(a, sc, act, state); break;
+    case 1: SCAN(1); break;
+    case 2: SCAN(2); break;
+    case 3: SCAN(3); break;
+    case 4: SCAN(4); break;
     default: return ADAMAH_ERR_INVALID;
   }
+#undef SCAN
   count_launch();
   return check_launch();
 }

@@ -159,8 +159,12 @@ k_space_prep(const SSpec s, const float* __restrict__ act, const float* __restri
 }
 
 // Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
-// is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.
-template <int NT> struct SpaceOps { f4_t c[NT], b[NT], cb, m, e, g, u; float last; };
+// is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.  A wave's
+// share of the outputs is its rows' part of C S and a quarter of the chunk's own part; a fifth wave adds up the shares and
+// stores them, a chunk behind: loads and stores share a counter, and a wave that does both waits for its stores (2048 tokens in
+// 64 heads of 64 by 128, the waves taking turns with the outputs 80.7 us, so 67).  FEW: one or two chunks, no operands ahead.
+#define SCAN_T 320u          // four waves of state rows and the one of the outputs
+template <int NT> struct SpaceOps { f4_t c[NT], b[NT], e, g, u; float cb, m, last; };
 template <int NT>
 __device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const float* hb, const SpaceDims& sd, uint32_t wave, uint32_t lane,
                                          uint32_t v0) {
@@ -171,100 +175,112 @@ __device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const
     o.c[j] = *(const f4_t*)(gb + at);
     o.b[j] = *(const f4_t*)(pB + at);
   }
-  o.cb = *(const f4_t*)(pD + lane * 4u);
-  o.m = *(const f4_t*)(pM + lane * 4u);
   o.e = *(const f4_t*)(pE + (lane >> 4) * 4u);
   o.g = *(const f4_t*)(pG + (lane >> 4) * 4u);
-  o.last = pE[15];
   o.u = *(const f4_t*)(hb + v0 * 16u + lane * 4u);
+  o.cb = pD[lane * 4u + wave];
+  o.m = pM[lane * 4u + wave];
+  o.last = pE[15];
 }
 
-template <int NT>
-__global__ void __launch_bounds__(256)
+template <int NT, bool FEW>
+__global__ void __launch_bounds__(SCAN_T)
 k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float* state, SpaceDims sd, uint32_t m, uint32_t seq0, uint32_t pos) {
-  __shared__ f4_t pb[2][4][64];
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, c = lane & 15u, kg = lane >> 4;
+  __shared__ f4_t pb[2][4][64];                              // [chunk & 1][wave][lane]
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, N = s.state, V = s.vdim, v = v0 + c, rep = s.heads / s.groups, grp = h / rep;
-  const uint32_t gs = group_floats(sd), hs = head_floats(sd);
-  const float* gb = scratch + (uint64_t)grp * sd.n_chunks * gs;
-  const float* hb = scratch + (uint64_t)s.groups * sd.n_chunks * gs + (uint64_t)h * sd.n_chunks * hs;
+  const uint32_t gs = group_floats(sd), hs = head_floats(sd), n = sd.n_chunks;
   state += (uint64_t)seq0 * s.seq_stride;
-  float* S = state + s.s_off + (uint64_t)h * N * V;
-  const float skip = act[s.skip + h];
-  f4_t st[NT];
-#pragma unroll
-  for (int j = 0; j < NT; j++) st[j] = (f4_t){0, 0, 0, 0};
-  if (pos != 0u) {
-#pragma unroll
-    for (int j = 0; j < NT; j++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) st[j][i] = S[(uint64_t)min((wave * NT + j) * 16u + 4u * kg + i, N - 1u) * V + min(v, V - 1u)];
-#pragma unroll
-    for (int j = 0; j < NT; j++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) if ((wave * NT + j) * 16u + 4u * kg + i >= N || v >= V) st[j][i] = 0.f;
-  }
-  const uint32_t n = sd.n_chunks;
-  // The operands of the chunk two ahead, asked for on every path (past the end: the last one's again): under a condition
-  // the wait at its end was for everything asked for (2048 tokens in 64 heads of 64 by 128: 162 us, 94 so, 83 with
-  // the operands in lane order).
-  const auto ask = [&](SpaceOps<NT>& o, uint32_t ci) {
-    const uint64_t at = min(ci, n - 1u);
-    load_ops<NT>(o, gb + at * gs, hb + at * hs, sd, wave, lane, v0);
-  };
-  const auto chunk = [&](const SpaceOps<NT>& cur, uint32_t ci, f4_t (*pb)[64]) {
-    f4_t p = {0, 0, 0, 0};
-#pragma unroll
-    for (int j = 0; j < NT; j++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) p = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.c[j][i], st[j][i], p, 0, 0, 0);
-    pb[wave][lane] = p;
-#pragma unroll
-    for (int j = 0; j < NT; j++) {
-      st[j] *= cur.last;
-#pragma unroll
-      for (int i = 0; i < 4; i++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[j][i], cur.g[i] * cur.u[i], st[j], 0, 0, 0);
-    }
-    __syncthreads();
-    if (wave == (ci & 3u)) {                                  // the waves take turns with the outputs
-      const f4_t* r = &pb[0][0];
-      f4_t o = ((r[lane] + r[64 + lane]) + (r[128 + lane] + r[192 + lane])) * cur.e;
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        o = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.cb[i] * cur.m[i] + (c == 4u * kg + i ? skip : 0.f), cur.u[i], o, 0, 0, 0);
+  if (wave == 4u) {
+    float* out = act + s.out + h * V + v;
+    for (uint32_t ci = 0; ci < n; ci++) {
+      __syncthreads();
+      const f4_t (*p)[64] = pb[ci & 1u];
+      const f4_t o = (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const uint32_t r2 = ci * CH + 4u * kg + i;
-        if (r2 < m && v < V) act[s.out + (uint64_t)r2 * s.out_stride + h * V + v] = o[i];
+        const uint32_t r = ci * CH + 4u * kg + i;
+        if (r < m && v < V) out[(uint64_t)r * s.out_stride] = o[i];
       }
     }
-  };
-  SpaceOps<NT> o0, o1, o2;
-  ask(o0, 0); ask(o1, 1); ask(o2, 2);
-  for (uint32_t ci = 0;; ci += 3u) {
-    chunk(o0, ci, pb[ci & 1u]);
-    if (ci + 1u >= n) break;
-    ask(o0, ci + 3u);
-    chunk(o1, ci + 1u, pb[(ci + 1u) & 1u]);
-    if (ci + 2u >= n) break;
-    ask(o1, ci + 4u);
-    chunk(o2, ci + 2u, pb[ci & 1u]);
-    if (ci + 3u >= n) break;
-    ask(o2, ci + 5u);
-  }
+  } else {
+    const float* gb = scratch + (uint64_t)grp * n * gs;
+    const float* hb = scratch + (uint64_t)s.groups * n * gs + (uint64_t)h * n * hs;
+    float* S = state + s.s_off + (uint64_t)h * N * V;
+    const float skip = c == 4u * kg + wave ? act[s.skip + h] : 0.f;      // of this wave's columns of the chunk's own part
+    f4_t st[NT];
 #pragma unroll
-  for (int j = 0; j < NT; j++)
+    for (int j = 0; j < NT; j++) st[j] = (f4_t){0, 0, 0, 0};
+    if (pos != 0u) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t d = (wave * NT + j) * 16u + 4u * kg + i;
-      if (d < N && v < V) S[(uint64_t)d * V + v] = st[j][i];
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) st[j][i] = S[(uint64_t)min((wave * NT + j) * 16u + 4u * kg + i, N - 1u) * V + min(v, V - 1u)];
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) if ((wave * NT + j) * 16u + 4u * kg + i >= N || v >= V) st[j][i] = 0.f;
     }
+    // The operands of the chunk two ahead, asked for on every path (past the end: the last one's again): under a condition
+    // the wait at its end was for everything asked for (162 us for 94).
+    const auto ask = [&](SpaceOps<NT>& o, uint32_t ci) {
+      const uint64_t at = min(ci, n - 1u);
+      load_ops<NT>(o, gb + at * gs, hb + at * hs, sd, wave, lane, v0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const auto chunk = [&](const SpaceOps<NT>& cur, uint32_t x) {
+      f4_t p[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.c[j][i], st[j][i], p[i & 1], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < NT; j++) st[j] *= cur.last;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[j][i], cur.g[i] * cur.u[i], st[j], 0, 0, 0);
+      const float u = wave & 2u ? (wave & 1u ? cur.u[3] : cur.u[2]) : (wave & 1u ? cur.u[1] : cur.u[0]);
+      pb[x][wave][lane] = __builtin_amdgcn_mfma_f32_16x16x4f32(fmaf(cur.cb, cur.m, skip), u, (p[0] + p[1]) * cur.e, 0, 0, 0);
+      __syncthreads();
+    };
+    SpaceOps<NT> o0;
+    ask(o0, 0);
+    if constexpr (FEW) {
+      for (uint32_t ci = 0; ci < n; ci++) {
+        if (ci) ask(o0, ci);
+        chunk(o0, ci & 1u);
+      }
+    } else {
+      // (a loop in one piece: with a way out behind each chunk the loads were moved down to where only the rest of the loop needs them)
+      SpaceOps<NT> o1, o2;
+      ask(o1, 1); ask(o2, 2);
+      uint32_t ci = 0;
+      for (; ci + 3u <= n; ci += 3u) {
+        chunk(o0, ci & 1u);
+        ask(o0, ci + 3u);
+        chunk(o1, (ci + 1u) & 1u);
+        ask(o1, ci + 4u);
+        chunk(o2, ci & 1u);
+        ask(o2, ci + 5u);
+      }
+      if (ci < n) chunk(o0, ci & 1u);
+      if (ci + 1u < n) chunk(o1, (ci + 1u) & 1u);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const uint32_t d = (wave * NT + j) * 16u + 4u * kg + i;
+        if (d < N && v < V) S[(uint64_t)d * V + v] = st[j][i];
+      }
+  }
   const uint32_t inner = s.heads * V, n_ch = inner + 2u * s.groups * N;      // the convolution's ring
   for (uint32_t r = m > s.taps ? m - s.taps : 0u; r < m; r++) {
     float* slot = state + s.conv_off + (uint64_t)((pos + r) % s.taps) * n_ch;
     const float* x = act + s.x + s.x_c + (uint64_t)r * s.x_stride;
     if (blockIdx.y == 0 && h % rep == 0)
-      for (uint32_t d = tid; d < N; d += 256u) {
+      for (uint32_t d = tid; d < N; d += SCAN_T) {
         const uint32_t b = inner + grp * N + d, cc = inner + (s.groups + grp) * N + d;
         slot[b] = x[b];
         slot[cc] = x[cc];
@@ -314,12 +330,16 @@ extern "C" int adamah_state_space_dev(uint32_t map_act, uint32_t h_spec, uint32_
   count_launch();
   if (int r = check_launch()) return r;
   const dim3 grid((uint32_t)H, cdiv(V, 16));
+  const bool few = sd.n_chunks <= 2u;
+#define SCAN(NT) do { if (few) k_space_scan<NT, true><<<grid, SCAN_T, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); \
+                      else k_space_scan<NT, false><<<grid, SCAN_T, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); } while (0)
   switch (sd.Np / 64u) {
-    case 1: k_space_scan<1><<<grid, 256, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); break;
-    case 2: k_space_scan<2><<<grid, 256, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); break;
-    case 3: k_space_scan<3><<<grid, 256, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); break;
-    default: k_space_scan<4><<<grid, 256, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); break;
+    case 1: SCAN(1); break;
+    case 2: SCAN(2); break;
+    case 3: SCAN(3); break;
+    default: SCAN(4); break;
   }
+#undef SCAN
   count_launch();
   return check_launch();
 }

@@ -449,6 +449,34 @@ def test_retention(hip, H, D, V, rot):
     run(3, 1, 0, 7)
 
 
+CHUNK_ROWS = (16, 17, 33, 48, 64, 65, 96, 7)      # 1, 2, 3, 3, 4, 5, 6 and 1 chunks: two kernels, and every remainder of three
+
+
+@pytest.mark.parametrize("D,V", [(24, 20), (100, 16), (180, 33)])
+def test_walk_of_few_and_of_many_chunks(hip, D, V):
+    note(f"walk over the chunks, D {D} V {V}")
+    run = delta_pair(hip, 2, 1, D, V, 3, 9, 96, 2, False, seed=D)
+    pos = 0
+    for m in CHUNK_ROWS:
+        run(1, m, 1, pos)
+        pos += m
+    rng = np.random.default_rng(V)
+    H, xs = 2, 2 * (2 * D + V)
+    state, oo = H * D * V, 96 * xs
+    p = Pair(hip, oo + 96 * H * V + H, state=state)
+    p.put(ST, 0, np.zeros(state))
+    p.put(WS, oo + 96 * H * V, [0.9, 0.999])
+    spec = p.up(A.RetentionSpec(heads=H, dim=D, vdim=V, rot_dims=0, freq=0, decay=oo + 96 * H * V, x=0, x_stride=xs, x_q=0, x_k=H * D,
+                                x_v=2 * H * D, out=oo, out_stride=H * V, state_map=ST, s_off=0, seq_stride=state).words())
+    pos = 0
+    for m in CHUNK_ROWS:
+        p.put(WS, 0, rng.standard_normal((m, xs)))
+        p.call("retention_dev", WS, spec, 1, m, 0, pos)
+        p.same(WS, oo, m * H * V, 5e-5, f"outputs of {m} at {pos}")
+        p.same(ST, 0, state, 5e-5, f"state after {pos + m}")
+        pos += m
+
+
 # ---- attention -------------------------------------------------------------------------------------------------------
 def attention_pair(hip, H, G, D, V, C, dtype, rows, seqs, seed, scale=0.25):
     rng = np.random.default_rng(seed)

@@ -191,6 +191,17 @@ def test_state_space(hip, H, G, N, V, taps, strong):
     run(1, 2, 2, 1)
 
 
+@pytest.mark.parametrize("N,V", [(24, 20), (100, 16), (180, 33)])
+def test_walk_of_few_and_of_many_chunks(hip, N, V):
+    """1, 2, 3, 3, 4, 5, 6 and 1 chunks: two kernels, and every remainder of three."""
+    note(f"state space walk over the chunks, N {N} V {V}")
+    run, _ = space_pair(hip, 2, 1, N, V, 3, 96, 2, False, seed=N)
+    pos = 0
+    for m in (16, 17, 33, 48, 64, 65, 96, 7):
+        run(1, m, 1, pos)
+        pos += m
+
+
 def test_state_space_keeps_an_input_over_a_long_gap(hip):
     """Steps close to zero leave the state alone: what the first token wrote is read 300 tokens later."""
     note("state space, long gap")
