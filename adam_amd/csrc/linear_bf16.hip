@@ -48,29 +48,29 @@ __device__ __forceinline__ float block_sum(float v, float* sh) {
 }
 // Root mean squares of the row's groups -> inv (with a barrier behind them).
 template <int NT, class Val>
-__device__ __forceinline__ void group_inverse(const LinSpec& s, float* inv, float* part, Val val) {
+__device__ __forceinline__ void group_inverse(uint32_t k, uint32_t groups, float eps, float* inv, float* part, Val val) {
   constexpr uint32_t NW = NT / 64;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, gs = s.k / s.groups;
-  if (s.groups >= NW) {
-    for (uint32_t gi = wave; gi < s.groups; gi += NW) {
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, gs = k / groups;
+  if (groups >= NW) {
+    for (uint32_t gi = wave; gi < groups; gi += NW) {
       float ss = 0.f;
       for (uint32_t i = lane; i < gs; i += 64u) { const float v = val(gi * gs + i); ss = fmaf(v, v, ss); }
       ss = wsum64(ss);
-      if (lane == 0) inv[gi] = 1.0f / sqrtf(ss / (float)gs + s.eps);
+      if (lane == 0) inv[gi] = 1.0f / sqrtf(ss / (float)gs + eps);
     }
     __syncthreads();
   } else {                                    // fewer groups than waves: `sub` waves share a group
-    const uint32_t sub = NW / s.groups, gi = wave / sub, sp = wave % sub;
+    const uint32_t sub = NW / groups, gi = wave / sub, sp = wave % sub;
     float ss = 0.f;
-    if (gi < s.groups)
+    if (gi < groups)
       for (uint32_t i = sp * 64u + lane; i < gs; i += sub * 64u) { const float v = val(gi * gs + i); ss = fmaf(v, v, ss); }
     ss = wsum64(ss);
     if (lane == 0) part[wave] = ss;
     __syncthreads();
-    if (tid < s.groups) {
+    if (tid < groups) {
       float t = 0.f;
       for (uint32_t j = 0; j < sub; j++) t += part[tid * sub + j];
-      inv[tid] = 1.0f / sqrtf(t / (float)gs + s.eps);
+      inv[tid] = 1.0f / sqrtf(t / (float)gs + eps);
     }
     __syncthreads();
   }
@@ -78,78 +78,160 @@ __device__ __forceinline__ void group_inverse(const LinSpec& s, float* inv, floa
 // f(x) of one row by a workgroup of NT threads; put(i, value) for i in [0, k_stride).  first: this workgroup also stores
 // what the spec wants kept.  put4(c, values): elements 4 c .. 4 c + 3.  inv: LDS, LIN_MAX_GROUPS floats, part: LDS, NT / 16
 // floats.  WIDE: for rows of several floats a thread; without it the code is short and needs fewer registers, which is what
-// counts where a thread has one (2048 rows of 64: 4.6 us, with it 5.4).
-template <int NT, bool WIDE, class Put, class Put4>
-__device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32_t row, bool first, float* inv, float* part, Put put, Put4 put4) {
-  const uint32_t tid = threadIdx.x, gl = s.groups ? s.k / s.groups >> 2 : 64u;          // lanes (of four elements) a group has
-  const float* x = act + s.src + (uint64_t)row * s.src_stride;
-  float* keep = act + s.keep + (uint64_t)row * s.keep_stride;
-  const bool kept = first && s.kept;
-  const float* wt = act + s.wt;
-  if (s.branched) {
+// counts where a thread has one (2048 rows of 64: 4.6 us, with it 5.4).  path: operand_path of the spec.  ahead(): called once,
+// behind the row's first loads -- loads arrive in order, and what is asked for there (the first weights) must not hold the row up.
+enum { ROW_ANY = 0, ROW_NORM = 1, ROW_BRANCH = 2, ROW_PLAIN = 3 };      // anything; four elements a load
+static uint32_t operand_path(const LinSpec& s, uint32_t nt) {
+  if (((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) != 0u) return ROW_ANY;
+  if (s.branched)
+    return s.k <= 8u * nt && ((s.branch | s.branch_stride | s.branch_wt | (s.wt_len ? s.wt : 0u) | (s.branched == 2u ? s.res_out | s.res_stride : 0u)) & 3u) == 0u
+               ? ROW_BRANCH : ROW_ANY;
+  if (!s.groups) return ROW_PLAIN;
+  const uint32_t gl = s.k / s.groups >> 2;                   // lanes (of four elements) a group has
+  return s.k <= 16u * nt && (!s.gate_act || ((s.gate | s.gate_stride) & 3u) == 0u) && (!s.wt_len || ((s.wt | s.wt_len) & 3u) == 0u) &&
+         (s.k / s.groups & 3u) == 0u && (s.groups == 1u || (gl & 63u) == 0u || (gl < 64u && (gl & (gl - 1u)) == 0u)) ? ROW_NORM : ROW_ANY;
+}
+// What a row is found by, apart from the spec: it is in registers when a wave starts, the spec's fields are a trip to memory (and
+// loaded where they are used: a copy of the spec would load them all first).  mode: below; at: the weight's place, of a
+// branched row the branch's weight's.
+struct RowArgs { uint32_t src, k, kp, branch, at, mode, row, src_stride, branch_stride, gate_stride, res_stride, keep_stride; };
+#define MODE_GROUPS(m) ((m) & 2047u)
+#define MODE_BRANCHED(m) ((m) >> 11 & 3u)
+#define MODE_GATED(m) ((m) >> 13 & 1u)
+#define MODE_PATH(m) ((m) >> 14 & 3u)
+#define MODE_WT(m) ((m) >> 16 & 1u)                  // there is a weight
+#define MODE_WHOLE(m) ((m) >> 17 & 1u)               // as long as the row
+#define MODE_GL(m) ((m) >> 18)                       // lanes (of four elements) a group has
+static uint32_t operand_mode(const LinSpec& s, uint32_t nt) {
+  return s.groups | s.branched << 11 | (s.gate_act ? 1u << 13 : 0u) | operand_path(s, nt) << 14 | (s.wt_len ? 1u << 16 : 0u) | (s.wt_len == s.k ? 1u << 17 : 0u) |
+         (s.groups ? s.k / s.groups >> 2 : 64u) << 18;
+}
+template <int NT, bool WIDE, class Put, class Put4, class Ahead>
+__device__ __forceinline__ void operand_row(const RowArgs& r, const LinSpec& s, float* act, bool first, float* inv, float* part, Put put, Put4 put4, Ahead ahead) {
+  const uint32_t tid = threadIdx.x, mode = r.mode, path = MODE_PATH(mode), gl = MODE_GL(mode);
+  const float* x = act + r.src + (uint64_t)r.row * r.src_stride;
+  const auto keep = [&] { return act + s.keep + (uint64_t)r.row * r.keep_stride; };
+  const auto kept = [&] { return first && s.kept; };
+  const auto gate_act = [&] { return MODE_GATED(mode) ? s.gate_act : 0u; };
+  const auto weight = [&] { return act + (MODE_BRANCHED(mode) ? s.wt : r.at); };
+  if (WIDE && path == ROW_BRANCH) {
+    // x + the branch's row behind a norm of its own, twice four elements a thread, everything asked for at once (past the end: the
+    // last four again, whose squares count for nothing)
+    constexpr int R = 2;
+    const uint32_t n4 = r.k >> 2;
+    const float *b = act + r.branch + (uint64_t)r.row * r.branch_stride, *bw = act + r.at;
+    f4_t xv[R], bv[R], wv[R], nv[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const uint32_t at = min(tid + (uint32_t)j * NT, n4 - 1u) * 4u;
+      xv[j] = *(const f4_t*)(x + at); bv[j] = *(const f4_t*)(b + at); wv[j] = *(const f4_t*)(bw + at);
+    }
+    ahead();
+    if (MODE_WT(mode)) {
+      const float* wt = weight();
+#pragma unroll
+      for (int j = 0; j < R; j++) nv[j] = *(const f4_t*)(wt + min(tid + (uint32_t)j * NT, n4 - 1u) * 4u);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const bool on = tid + (uint32_t)j * NT < n4;
+#pragma unroll
+      for (int e = 0; e < 4; e++) { bv[j][e] = on ? bv[j][e] : 0.f; ss = fmaf(bv[j][e], bv[j][e], ss); }
+    }
+    const float ib = 1.0f / sqrtf(block_sum<NT / 64>(ss, part) / (float)r.k + s.eps);
+    ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const bool on = tid + (uint32_t)j * NT < n4;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        xv[j][e] = fmaf(bv[j][e] * ib, s.wt_add + wv[j][e], xv[j][e]);
+        const float v = on ? xv[j][e] : 0.f;
+        ss = fmaf(v, v, ss);
+      }
+    }
+    const float ix = 1.0f / sqrtf(block_sum<NT / 64>(ss, part + NT / 64) / (float)r.k + s.eps);
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const uint32_t c = tid + (uint32_t)j * NT;
+      if (c >= n4) break;
+      if (first && MODE_BRANCHED(mode) == 2u) *(f4_t*)(act + s.res_out + (uint64_t)r.row * r.res_stride + 4u * c) = xv[j];
+      f4_t v = xv[j];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        v[e] *= ix;
+        if (MODE_WT(mode)) v[e] *= s.wt_add + nv[j][e];
+      }
+      if (kept()) *(f4_t*)(keep() + 4u * c) = v;
+      put4(c, v);
+    }
+  } else if (MODE_BRANCHED(mode)) {
+    ahead();
     // x + the branch's row behind a norm of its own: eight elements a thread stay in registers (a longer row is read again)
     constexpr int R = 8;
-    const float *b = act + s.branch + (uint64_t)row * s.branch_stride, *bw = act + s.branch_wt;
-    float* res = act + s.res_out + (uint64_t)row * s.res_stride;
+    const float *b = act + r.branch + (uint64_t)r.row * r.branch_stride, *bw = act + r.at;
+    float* res = act + s.res_out + (uint64_t)r.row * r.res_stride;
+    const float* wt = weight();
+    const bool keeps = kept();
     float xv[R], bv[R], wv[R], nv[R], ss = 0.f;
 #pragma unroll
     for (int j = 0; j < R; j++) {
       const uint32_t i = tid + (uint32_t)j * NT;
-      const bool on = i < s.k;
-      bv[j] = on ? b[i] : 0.f; xv[j] = on ? x[i] : 0.f; wv[j] = on ? bw[i] : 0.f; nv[j] = on && s.wt_len ? wt[i] : 0.f;
+      const bool on = i < r.k;
+      bv[j] = on ? b[i] : 0.f; xv[j] = on ? x[i] : 0.f; wv[j] = on ? bw[i] : 0.f; nv[j] = on && MODE_WT(mode) ? wt[i] : 0.f;
     }
 #pragma unroll
     for (int j = 0; j < R; j++) ss = fmaf(bv[j], bv[j], ss);
-    for (uint32_t i = tid + (uint32_t)R * NT; i < s.k; i += NT) ss = fmaf(b[i], b[i], ss);
-    const float ib = 1.0f / sqrtf(block_sum<NT / 64>(ss, part) / (float)s.k + s.eps);
+    for (uint32_t i = tid + (uint32_t)R * NT; i < r.k; i += NT) ss = fmaf(b[i], b[i], ss);
+    const float ib = 1.0f / sqrtf(block_sum<NT / 64>(ss, part) / (float)r.k + s.eps);
     ss = 0.f;
 #pragma unroll
     for (int j = 0; j < R; j++) {
       const uint32_t i = tid + (uint32_t)j * NT;
       xv[j] = fmaf(bv[j] * ib, s.wt_add + wv[j], xv[j]);
-      if (i < s.k) ss = fmaf(xv[j], xv[j], ss);
+      if (i < r.k) ss = fmaf(xv[j], xv[j], ss);
     }
     const auto sum_at = [&](uint32_t i) { return fmaf(b[i] * ib, s.wt_add + bw[i], x[i]); };
-    for (uint32_t i = tid + (uint32_t)R * NT; i < s.k; i += NT) { const float v = sum_at(i); ss = fmaf(v, v, ss); }
-    const float ix = 1.0f / sqrtf(block_sum<NT / 64>(ss, part + NT / 64) / (float)s.k + s.eps);
+    for (uint32_t i = tid + (uint32_t)R * NT; i < r.k; i += NT) { const float v = sum_at(i); ss = fmaf(v, v, ss); }
+    const float ix = 1.0f / sqrtf(block_sum<NT / 64>(ss, part + NT / 64) / (float)r.k + s.eps);
     const auto done = [&](uint32_t i, float v, float w) {
-      if (first && s.branched == 2u) res[i] = v;
+      if (first && MODE_BRANCHED(mode) == 2u) res[i] = v;
       v *= ix;
-      if (s.wt_len) v *= s.wt_add + w;
-      if (kept) keep[i] = v;
+      if (MODE_WT(mode)) v *= s.wt_add + w;
+      if (keeps) keep()[i] = v;
       put(i, v);
     };
 #pragma unroll
     for (int j = 0; j < R; j++) {
       const uint32_t i = tid + (uint32_t)j * NT;
-      if (i < s.k) done(i, xv[j], nv[j]);
+      if (i < r.k) done(i, xv[j], nv[j]);
     }
-    for (uint32_t i = tid + (uint32_t)R * NT; i < s.k; i += NT) done(i, sum_at(i), s.wt_len ? wt[i] : 0.f);
-  } else if (WIDE && s.groups && s.k <= 16u * NT && ((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) == 0u &&
-             (!s.gate_act || ((s.gate | s.gate_stride) & 3u) == 0u) && (!s.wt_len || ((s.wt | s.wt_len) & 3u) == 0u) &&
-             (s.k / s.groups & 3u) == 0u && (s.groups == 1u || (gl & 63u) == 0u || (gl < 64u && (gl & (gl - 1u)) == 0u))) {
+    for (uint32_t i = tid + (uint32_t)R * NT; i < r.k; i += NT) done(i, sum_at(i), MODE_WT(mode) ? wt[i] : 0.f);
+  } else if (WIDE && path == ROW_NORM) {
     // The row makes one trip: up to four times four elements a thread, everything asked for at once (twelve rows of 4096,
     // one float a load and each pass waiting for the one before: 15.8 us; so: 5.0).  A group is a power of two of
     // neighbouring lanes, or whole waves' worth, whose sums meet in LDS, or all of the row.
     constexpr int R = 4, NW = NT / 64;
-    const uint32_t n4 = s.k >> 2, wave = tid >> 6;
-    const float* gt = act + s.gate + (uint64_t)row * s.gate_stride;
+    const uint32_t n4 = r.k >> 2, wave = tid >> 6;
+    const float *gt = MODE_GATED(mode) ? act + s.gate + (uint64_t)r.row * r.gate_stride : act, *wt = weight();
     f4_t xv[R], gv[R], wv[R];
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const uint32_t c = tid + (uint32_t)j * NT;
-      if (c >= n4) break;
+      const uint32_t c = min(tid + (uint32_t)j * NT, n4 - 1u);
+      if ((uint32_t)j * NT >= n4) break;
       xv[j] = *(const f4_t*)(x + 4u * c);
-      if (s.gate_act) gv[j] = *(const f4_t*)(gt + 4u * c);
-      if (s.wt_len) wv[j] = *(const f4_t*)(wt + (s.wt_len == s.k ? 4u * c : 4u * c % s.wt_len));
+      if (MODE_GATED(mode)) gv[j] = *(const f4_t*)(gt + 4u * c);
+      if (MODE_WT(mode)) wv[j] = *(const f4_t*)(wt + (MODE_WHOLE(mode) ? 4u * c : 4u * c % s.wt_len));
     }
+    ahead();
     float ss[R];
 #pragma unroll
     for (int j = 0; j < R; j++) {
       const uint32_t c = tid + (uint32_t)j * NT;
       ss[j] = 0.f;
       if (c >= n4) continue;
-      if (s.gate_act == 3u)
+      if (gate_act() == 3u)
 #pragma unroll
         for (int e = 0; e < 4; e++) xv[j][e] *= silu_f(gv[j][e]);
 #pragma unroll
@@ -157,7 +239,7 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
     }
     float scale[R];
     const float n = (float)(4u * gl);
-    if (gl < 64u && s.groups != 1u) {
+    if (gl < 64u && MODE_GROUPS(mode) != 1u) {
 #pragma unroll
       for (int j = 0; j < R; j++) {
         if ((uint32_t)j * NT >= n4) break;
@@ -175,11 +257,10 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < R; j++) {
-        if (tid + (uint32_t)j * NT >= n4) break;
-        const uint32_t b0 = ((uint32_t)j * NW + wave) / nb * nb;
-        float t = 0.f;
-        for (uint32_t b = 0; b < nb; b++) t += part[b0 + b];
-        scale[j] = 1.0f / sqrtf(t / n + s.eps);
+        if ((uint32_t)j * NT >= n4) break;                   // (all lanes or none: they add up together)
+        if (j > 0 && MODE_GROUPS(mode) == 1u) { scale[j] = scale[0]; continue; }
+        const uint32_t lane = tid & 63u, b0 = ((uint32_t)j * NW + wave) / nb * nb;         // (a partial sum a lane)
+        scale[j] = 1.0f / sqrtf(wsum64(lane < nb ? part[min(b0 + lane, (uint32_t)(R * NW) - 1u)] : 0.f) / n + s.eps);
       }
     }
 #pragma unroll
@@ -190,53 +271,73 @@ __device__ __forceinline__ void operand_row(const LinSpec& s, float* act, uint32
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         v[e] *= scale[j];
-        if (s.wt_len) v[e] *= s.wt_add + wv[j][e];
-        if (s.gate_act == 1u) v[e] *= sigmoid_f(gv[j][e]);
-        else if (s.gate_act == 2u) v[e] *= silu_f(gv[j][e]);
+        if (MODE_WT(mode)) v[e] *= s.wt_add + wv[j][e];
+        if (gate_act() == 1u) v[e] *= sigmoid_f(gv[j][e]);
+        else if (gate_act() == 2u) v[e] *= silu_f(gv[j][e]);
       }
-      if (kept) *(f4_t*)(keep + 4u * c) = v;
+      if (kept()) *(f4_t*)(keep() + 4u * c) = v;
       put4(c, v);
     }
-  } else if (s.groups) {
-    const uint32_t gs = s.k / s.groups;
-    const float* gt = act + s.gate + (uint64_t)row * s.gate_stride;
-    if (s.gate_act == 3u) group_inverse<NT>(s, inv, part, [&](uint32_t i) { return x[i] * silu_f(gt[i]); });
-    else group_inverse<NT>(s, inv, part, [&](uint32_t i) { return x[i]; });
-    for (uint32_t i = tid; i < s.k; i += NT) {
+  } else if (MODE_GROUPS(mode)) {
+    ahead();
+    const uint32_t gs = r.k / MODE_GROUPS(mode);
+    const float *gt = act + s.gate + (uint64_t)r.row * r.gate_stride, *wt = weight();
+    const bool keeps = kept();
+    if (gate_act() == 3u) group_inverse<NT>(r.k, MODE_GROUPS(mode), s.eps, inv, part, [&](uint32_t i) { return x[i] * silu_f(gt[i]); });
+    else group_inverse<NT>(r.k, MODE_GROUPS(mode), s.eps, inv, part, [&](uint32_t i) { return x[i]; });
+    for (uint32_t i = tid; i < r.k; i += NT) {
       float v = x[i];
-      if (s.gate_act == 3u) v *= silu_f(gt[i]);
+      if (gate_act() == 3u) v *= silu_f(gt[i]);
       v *= inv[i / gs];
-      if (s.wt_len) v *= s.wt_add + wt[s.wt_len == s.k ? i : i % s.wt_len];
-      if (s.gate_act == 1u) v *= sigmoid_f(gt[i]);
-      else if (s.gate_act == 2u) v *= silu_f(gt[i]);
-      if (kept) keep[i] = v;
+      if (MODE_WT(mode)) v *= s.wt_add + wt[MODE_WHOLE(mode) ? i : i % s.wt_len];
+      if (gate_act() == 1u) v *= sigmoid_f(gt[i]);
+      else if (gate_act() == 2u) v *= silu_f(gt[i]);
+      if (keeps) keep()[i] = v;
       put(i, v);
     }
-  } else if (WIDE && ((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) == 0u) {
-#pragma unroll 4
-    for (uint32_t c = tid; c < s.k >> 2; c += NT) {
-      const f4_t v = *(const f4_t*)(x + 4u * c);
-      if (kept) *(f4_t*)(keep + 4u * c) = v;
-      put4(c, v);
+  } else if (WIDE && path == ROW_PLAIN) {
+    constexpr int R = 4;                                     // of the row; a longer one's rest behind ahead()
+    const uint32_t n4 = r.k >> 2;
+    f4_t v[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      if ((uint32_t)j * NT >= n4) break;
+      v[j] = *(const f4_t*)(x + 4u * min(tid + (uint32_t)j * NT, n4 - 1u));
     }
+    ahead();
+    const auto done = [&](uint32_t c, f4_t v) {
+      if (kept()) *(f4_t*)(keep() + 4u * c) = v;
+      put4(c, v);
+    };
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const uint32_t c = tid + (uint32_t)j * NT;
+      if (c < n4) done(c, v[j]);
+    }
+#pragma unroll 4
+    for (uint32_t c = tid + (uint32_t)R * NT; c < n4; c += NT) done(c, *(const f4_t*)(x + 4u * c));
   } else {
-    for (uint32_t i = tid; i < s.k; i += NT) {
-      if (kept) keep[i] = x[i];
+    ahead();
+    const bool keeps = kept();
+    for (uint32_t i = tid; i < r.k; i += NT) {
+      if (keeps) keep()[i] = x[i];
       put(i, x[i]);
     }
   }
-  for (uint32_t i = s.k + tid; i < s.k_stride; i += NT) put(i, 0.f);
+  for (uint32_t i = r.k + tid; i < r.kp; i += NT) put(i, 0.f);
 }
 
 template <class T, int NT, bool WIDE>
 __global__ void __launch_bounds__(NT)
-k_operand_rows(const LinSpec s, float* act, T* __restrict__ dst, const uint32_t* __restrict__ row_idx) {
+k_operand_rows(float* act, T* __restrict__ dst, const uint32_t* __restrict__ row_idx, uint32_t src, uint32_t src_stride, uint32_t k, uint32_t kp, uint32_t mode,
+               uint32_t at, uint32_t branch, const LinSpec s) {
   __shared__ float inv[LIN_MAX_GROUPS];
   __shared__ float part[NT / 16];
   typedef T t4 __attribute__((ext_vector_type(4)));
-  T* d = dst + (uint64_t)blockIdx.x * s.k_stride;
-  operand_row<NT, WIDE>(s, act, row_idx ? row_idx[blockIdx.x] : blockIdx.x, true, inv, part, [&](uint32_t i, float v) { d[i] = (T)v; },
-                  [&](uint32_t c, f4_t v) { *(t4*)(d + 4u * c) = (t4){(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; });
+  T* d = dst + (uint64_t)blockIdx.x * kp;
+  const RowArgs r = {src, k, kp, branch, at, mode, row_idx ? row_idx[blockIdx.x] : blockIdx.x, src_stride, s.branch_stride, s.gate_stride, s.res_stride, s.keep_stride};
+  operand_row<NT, WIDE>(r, s, act, true, inv, part, [&](uint32_t i, float v) { d[i] = (T)v; },
+                        [&](uint32_t c, f4_t v) { *(t4*)(d + 4u * c) = (t4){(T)v[0], (T)v[1], (T)v[2], (T)v[3]}; }, [] {});
 }
 // Long rows, few of them: a row's latency is the launch's, so 1024 threads a row; many rows fill the CUs with 256 each, and
 // rows of one float a thread have nothing to gain (300 rows of 64 on the wide form with 1024 threads: 5.7 us, so: 3.6; 12 rows
@@ -246,92 +347,110 @@ k_operand_rows(const LinSpec s, float* act, T* __restrict__ dst, const uint32_t*
 // 2048 rows of 4096 43.6 and 34.4; 2 rows of 4096 12.0 and 10.5; 600 rows of 8192 41.4 and 31.8).
 template <class T>
 static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* row_idx, uint32_t rows) {
-  if (s.k <= 256u || (s.branched && s.k <= 2048u)) k_operand_rows<T, 256, false><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
-  else if (s.branched && s.k <= 4096u) k_operand_rows<T, 512, false><<<rows, 512, 0, g.stream>>>(s, act, dst, row_idx);
-  else if (s.branched) k_operand_rows<T, 1024, false><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
-  else if (s.k > 1024u && rows <= 2u * (uint32_t)g.n_cu) k_operand_rows<T, 1024, true><<<rows, 1024, 0, g.stream>>>(s, act, dst, row_idx);
-  else k_operand_rows<T, 256, true><<<rows, 256, 0, g.stream>>>(s, act, dst, row_idx);
+#define ROWS(NT, WIDE) k_operand_rows<T, NT, WIDE><<<rows, NT, 0, g.stream>>>(act, dst, row_idx, s.src, s.src_stride, s.k, s.k_stride, operand_mode(s, NT), \
+                                                                              s.branched ? s.branch_wt : s.wt, s.branch, s)
+  if (s.k <= 256u || (s.branched && s.k <= 2048u)) ROWS(256, false);
+  else if (s.branched && s.k <= 4096u) ROWS(512, false);
+  else if (s.branched) ROWS(1024, false);
+  else if (s.k > 1024u && rows <= 2u * (uint32_t)g.n_cu) ROWS(1024, true);
+  else ROWS(256, true);
+#undef ROWS
   count_launch();
 }
 
 // ---- one row ------------------------------------------------------------------------------------------------------
-// A wave takes two matrix rows at a time (for gate / up pairs: row 32 b + j and its partner 16 further on) and walks
+// A wave takes R matrix rows at a time (two; for gate / up pairs row 32 b + j and its partner 16 further on) and walks
 // along K, 512 columns a step, U steps in flight.  x in LDS as two planes (elements 0..3 / 4..7 of every eight), so that
 // a lane's two 16-byte reads are conflict free.
+// What bounds it is the weights' way in and, for the smaller matrices, what a workgroup does before it can use them: x and the
+// first weights behind it are asked for from the leading arguments alone (in registers when a wave starts; the spec is a
+// trip to memory, 0.5 us), sums of a norm stay in the vector unit.  us, weights cold, before and so: 2048 x 2048 4.9 and 4.1,
+// 2048 x 4096 7.2 and 6.2, behind a norm 9.2 and 7.7, 4096 x 4096 behind a norm 11.8 and 9.2, 10304 x 2048 behind a branch
+// 13.8 and 11.4, 4131 x 2048 (pairs, a tail) 10.4 and 8.7, 28672 x 4096 (pairs) 44.3 and 42, 4096 x 14336 24.7 and 23.6.
 enum { LEPI_STORE = 0, LEPI_ADD = 1, LEPI_PAIR = 2, LEPI_ARGMAX = 3 };
-template <int EPI, int U>
+template <int EPI, int U, int R>
 __global__ void __launch_bounds__(512)
-k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const LinSpec s, uint32_t n_tasks, const uint32_t* __restrict__ row_idx,
-            float* best_val, uint32_t* best_idx) {
+k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const uint32_t* __restrict__ row_idx, uint32_t kp, uint32_t n, uint32_t pairs, uint32_t src,
+            uint32_t k_in, uint32_t mode, uint32_t branch, uint32_t at, const LinSpec s, float* best_val, uint32_t* best_idx) {
+  static_assert(R == 2 || EPI == LEPI_STORE || EPI == LEPI_ADD, "one row");
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ float inv[LIN_MAX_GROUPS];
   __shared__ float part[32];
   __shared__ float bv[8];
   __shared__ uint32_t bi[8];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, kp = s.k_stride, half = kp >> 1;
-  const uint32_t pairs = EPI == LEPI_PAIR ? (s.n - s.tail) >> 1 : 0u;        // the tail's rows come two a task behind the pairs
-  auto rows_of = [&](uint32_t task, uint32_t& r0, uint32_t& r1) {
-    if (EPI == LEPI_PAIR && task < pairs) { r0 = (task >> 4) * 32u + (task & 15u); r1 = r0 + 16u; }
-    else { r0 = task * 2u; r1 = min(r0 + 1u, s.n - 1u); }     // (2 pairs + 2 (task - pairs) for the tail)
+  RowArgs ra = {src, k_in, kp, branch, at, mode, 0u, 0u, 0u, 0u, 0u, 0u};
+  if (row_idx) {                                             // (an asm: not to be loaded, and waited for, where there is no list)
+    ra.row = row_idx[0];
+    ra.src_stride = s.src_stride; ra.branch_stride = s.branch_stride; ra.gate_stride = s.gate_stride; ra.res_stride = s.res_stride; ra.keep_stride = s.keep_stride;
+    asm volatile("" : "+s"(ra.src_stride), "+s"(ra.branch_stride), "+s"(ra.gate_stride), "+s"(ra.res_stride), "+s"(ra.keep_stride));
+  }
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, half = kp >> 1, n_tasks = R == 1 ? n : pairs + ((n - 2u * pairs + 1u) >> 1);
+  // pairs: tasks of gate / up; the tail's rows come two a task behind them
+  auto rows_of = [&](uint32_t task, uint32_t (&r)[R]) {
+    if constexpr (R == 1) r[0] = task;
+    else if (EPI == LEPI_PAIR && task < pairs) { r[0] = (task >> 4) * 32u + (task & 15u); r[1] = r[0] + 16u; }
+    else { r[0] = task * 2u; r[1] = min(r[0] + 1u, n - 1u); }     // (2 pairs + 2 (task - pairs) for the tail)
   };
-  uint4 p[U], q[U];
-  auto fetch = [&](uint32_t r0, uint32_t r1, uint32_t k0) {
+  uint4 p[R][U];
+  auto fetch = [&](const uint32_t (&r)[R], uint32_t k0) {    // (past the row's end its last columns, which nothing uses)
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const uint32_t k = k0 + 512u * u;
-      p[u] = k < kp ? *(const uint4*)(W + (uint64_t)r0 * kp + k) : make_uint4(0, 0, 0, 0);
-      q[u] = k < kp ? *(const uint4*)(W + (uint64_t)r1 * kp + k) : make_uint4(0, 0, 0, 0);
+      const uint32_t k = min(k0 + 512u * u, kp - 8u);
+#pragma unroll
+      for (int q = 0; q < R; q++) p[q][u] = *(const uint4*)(W + (uint64_t)r[q] * kp + k);
     }
   };
   // the first weights are on their way while x is staged, each further step's under the products of the one before
-  uint32_t task = blockIdx.x * 8u + wave, k0 = lane * 8u, r0, r1;
-  rows_of(min(task, n_tasks - 1u), r0, r1);
-  fetch(r0, r1, k0);
-  operand_row<512, (U > 1)>(s, act, row_idx ? row_idx[0] : 0u, blockIdx.x == 0u, inv, part,
+  uint32_t task = blockIdx.x * 8u + wave, k0 = lane * 8u, r[R];
+  rows_of(min(task, n_tasks - 1u), r);
+  operand_row<512, (U > 1)>(ra, s, act, blockIdx.x == 0u, inv, part,
                    [&](uint32_t i, float v) { xs[((i >> 2) & 1u) * half + (i >> 3) * 4u + (i & 3u)] = v; },
-                   [&](uint32_t c, f4_t v) { *(f4_t*)(xs + (c & 1u) * half + (c >> 1) * 4u) = v; });
+                   [&](uint32_t c, f4_t v) { *(f4_t*)(xs + (c & 1u) * half + (c >> 1) * 4u) = v; },
+                   [&] { fetch(r, k0); __builtin_amdgcn_sched_barrier(0); });
   __syncthreads();
-  float top = NEG_MAX_F, a0 = 0.f, a1 = 0.f;
+  float top = NEG_MAX_F, a[R] = {};
   uint32_t top_i = 0xFFFFFFFFu;
   while (task < n_tasks) {
-    uint4 cp[U], cq[U];
+    uint4 cur[R][U];
 #pragma unroll
-    for (int u = 0; u < U; u++) { cp[u] = p[u]; cq[u] = q[u]; }
-    const bool last = k0 - lane * 8u + 512u * U >= kp;              // of this pair of rows
-    const uint32_t next = last ? task + gridDim.x * 8u : task, kn = last ? lane * 8u : k0 + 512u * U, c0 = r0;
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int q = 0; q < R; q++) cur[q][u] = p[q][u];
+    const bool last = k0 - lane * 8u + 512u * U >= kp;              // of these rows
+    const uint32_t next = last ? task + gridDim.x * 8u : task, kn = last ? lane * 8u : k0 + 512u * U, c0 = r[0];
     if (next < n_tasks) {
-      if (last) rows_of(next, r0, r1);
-      fetch(r0, r1, kn);
+      if (last) rows_of(next, r);
+      fetch(r, kn);
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const uint32_t k = k0 + 512u * u;
       if (k >= kp) break;
       const float4 lo = *(const float4*)(xs + (k >> 1)), hi = *(const float4*)(xs + half + (k >> 1));
-      a0 = fmaf(bf_lo(cp[u].x), lo.x, a0); a1 = fmaf(bf_lo(cq[u].x), lo.x, a1);
-      a0 = fmaf(bf_hi(cp[u].x), lo.y, a0); a1 = fmaf(bf_hi(cq[u].x), lo.y, a1);
-      a0 = fmaf(bf_lo(cp[u].y), lo.z, a0); a1 = fmaf(bf_lo(cq[u].y), lo.z, a1);
-      a0 = fmaf(bf_hi(cp[u].y), lo.w, a0); a1 = fmaf(bf_hi(cq[u].y), lo.w, a1);
-      a0 = fmaf(bf_lo(cp[u].z), hi.x, a0); a1 = fmaf(bf_lo(cq[u].z), hi.x, a1);
-      a0 = fmaf(bf_hi(cp[u].z), hi.y, a0); a1 = fmaf(bf_hi(cq[u].z), hi.y, a1);
-      a0 = fmaf(bf_lo(cp[u].w), hi.z, a0); a1 = fmaf(bf_lo(cq[u].w), hi.z, a1);
-      a0 = fmaf(bf_hi(cp[u].w), hi.w, a0); a1 = fmaf(bf_hi(cq[u].w), hi.w, a1);
+#pragma unroll
+      for (int q = 0; q < R; q++) {
+        const uint4 w = cur[q][u];
+        a[q] = fmaf(bf_lo(w.x), lo.x, a[q]); a[q] = fmaf(bf_hi(w.x), lo.y, a[q]); a[q] = fmaf(bf_lo(w.y), lo.z, a[q]); a[q] = fmaf(bf_hi(w.y), lo.w, a[q]);
+        a[q] = fmaf(bf_lo(w.z), hi.x, a[q]); a[q] = fmaf(bf_hi(w.z), hi.y, a[q]); a[q] = fmaf(bf_lo(w.w), hi.z, a[q]); a[q] = fmaf(bf_hi(w.w), hi.w, a[q]);
+      }
     }
     if (last) {
-      a0 = wsum64(a0); a1 = wsum64(a1);
+#pragma unroll
+      for (int q = 0; q < R; q++) a[q] = wsum64(a[q]);
       if (EPI == LEPI_PAIR && task < pairs) {
-        if (lane == 0) act[s.out + task] = silu_f(a0) * a1;
+        if (lane == 0) act[s.out + task] = silu_f(a[0]) * a[R - 1];
       } else {
-        const uint32_t r = c0 + lane;
-        float y = lane ? a1 : a0;
-        if (lane < 2u && r < s.n) {
-          if (s.biased) y += act[s.bias + r];
-          float* d = EPI == LEPI_PAIR ? act + s.tail_out + (r - 2u * pairs) : act + s.out + r;
+        const uint32_t i = c0 + lane;
+        float y = lane ? a[R - 1] : a[0];
+        if (lane < (uint32_t)R && i < n) {
+          if (s.biased) y += act[s.bias + i];
+          float* d = EPI == LEPI_PAIR ? act + s.tail_out + (i - 2u * pairs) : act + s.out + i;
           *d = EPI == LEPI_ADD ? *d + y : y;
-          if (EPI == LEPI_ARGMAX && !isnan(y) && y > top) { top = y; top_i = r; }
+          if (EPI == LEPI_ARGMAX && !isnan(y) && y > top) { top = y; top_i = i; }
         }
       }
-      a0 = a1 = 0.f;
+#pragma unroll
+      for (int q = 0; q < R; q++) a[q] = 0.f;
     }
     task = next; k0 = kn;
   }
@@ -833,26 +952,36 @@ static int launch_tiles(const bf16_t* W, const bf16_t* X, float* act, T* op, con
 
 static uint32_t gemv_grid(uint32_t n_tasks) { return std::min<uint32_t>(cdiv(n_tasks, 8), 2u * (uint32_t)g.n_cu); }
 
+// tasks of two rows (pairs of gate / up ahead of the tail's)
+static uint32_t gemv_tasks(const LinSpec& s) { return s.epi == 2u ? (s.n - s.tail) / 2 + cdiv(s.tail, 2) : cdiv(s.n, 2); }
+
 template <int EPI>
-static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_idx, uint32_t n_tasks) {
-  const uint32_t grid = gemv_grid(n_tasks);
-  const size_t lds = (size_t)s.k_stride * 4;
+static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_idx) {
   const bf16_t* W = (const bf16_t*)mw->buf + s.w;
-  float* bv = (float*)g_best.p;
-  uint32_t* bi = bv ? (uint32_t*)(bv + grid) : nullptr;
-  if (s.k_stride >= 1024u) {
-    if (lds > 60000) hipFuncSetAttribute((const void*)k_gemv_bf16<EPI, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    k_gemv_bf16<EPI, 4><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi);
-  } else k_gemv_bf16<EPI, 1><<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, s, n_tasks, row_idx, bv, bi);
-  count_launch();
+  const size_t lds = (size_t)s.k_stride * 4;
+  const uint32_t mode = operand_mode(s, 512);
+  const auto go = [&](auto* kernel, uint32_t n_tasks) {
+    const uint32_t grid = gemv_grid(n_tasks);
+    float* bv = (float*)g_best.p;
+    if (lds > 60000) hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    kernel<<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, row_idx, s.k_stride, s.n, s.epi == 2u ? (s.n - s.tail) / 2 : 0u, s.src, s.k, mode, s.branch,
+                                         s.branched ? s.branch_wt : s.wt, s, bv, bv ? (uint32_t*)(bv + grid) : nullptr);
+    count_launch();
+  };
+  if (s.k_stride < 1024u) return go(k_gemv_bf16<EPI, 1, 2>, gemv_tasks(s));
+  // A row a wave while that is a workgroup a CU at most: with two, half the CUs or less would have one (2048 x 2048 4.8 us, so 4.05;
+  // 4096 x 4096 in two workgroups a CU 12.2, two rows a wave 9.8)
+  if constexpr (EPI == LEPI_STORE || EPI == LEPI_ADD)
+    if (s.n <= 8u * (uint32_t)g.n_cu) return s.k_stride > 2048u ? go(k_gemv_bf16<EPI, 8, 1>, s.n) : go(k_gemv_bf16<EPI, 4, 1>, s.n);
+  go(k_gemv_bf16<EPI, 4, 2>, gemv_tasks(s));
 }
 
 int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_idx, uint32_t rows) {
   float* act = (float*)ma->buf;
   if (rows == 1) {
-    if (s.epi == 2u) gemv_launch<LEPI_PAIR>(ma, mw, s, row_idx, (s.n - s.tail) / 2 + cdiv(s.tail, 2));
-    else if (s.epi == 1u) gemv_launch<LEPI_ADD>(ma, mw, s, row_idx, cdiv(s.n, 2));
-    else gemv_launch<LEPI_STORE>(ma, mw, s, row_idx, cdiv(s.n, 2));
+    if (s.epi == 2u) gemv_launch<LEPI_PAIR>(ma, mw, s, row_idx);
+    else if (s.epi == 1u) gemv_launch<LEPI_ADD>(ma, mw, s, row_idx);
+    else gemv_launch<LEPI_STORE>(ma, mw, s, row_idx);
     return check_launch();
   }
   const bf16_t* W = (const bf16_t*)mw->buf + s.w;
@@ -947,9 +1076,9 @@ int adamah_linear_argmax_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_w
   for (uint32_t i = 0; i < rows; i++) if (dst[i] >= ma->n_elems) return ADAMAH_ERR_INVALID;
   float* act = (float*)ma->buf;
   if (rows == 1) {
-    const uint32_t n_tasks = cdiv(s->n, 2), grid = gemv_grid(n_tasks);
+    const uint32_t grid = gemv_grid(gemv_tasks(*s));
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
-    gemv_launch<LEPI_ARGMAX>(ma, mw, *s, nullptr, n_tasks);
+    gemv_launch<LEPI_ARGMAX>(ma, mw, *s, nullptr);
     k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0], nullptr);
   } else {
     if (int r = run_linear(ma, mo, mw, *s, nullptr, rows)) return r;
@@ -978,9 +1107,9 @@ int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint3
   const size_t row_bytes = (size_t)s->k_stride * 4;
   const uint32_t fit = (uint32_t)(((size_t)144 << 10) / row_bytes), nr = fit >= 8 && rows > 4 ? 8 : fit >= 4 && rows > 2 ? 4 : fit >= 2 && rows > 1 ? 2 : 1;
   if (rows == 1) {
-    const uint32_t n_tasks = cdiv(s->n, 2), grid = gemv_grid(n_tasks);
+    const uint32_t grid = gemv_grid(gemv_tasks(*s));
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
-    gemv_launch<LEPI_ARGMAX>(ma, mw, *s, dev, n_tasks);
+    gemv_launch<LEPI_ARGMAX>(ma, mw, *s, dev);
     k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0], nullptr);
     count_launch();
     return check_launch();

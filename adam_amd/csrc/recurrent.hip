@@ -27,7 +27,7 @@ typedef AdamahRetentionSpec RSpec;
 // sums over a workgroup of NW waves of up to three values at once; sh: 3 NW floats
 template <int NW>
 __device__ __forceinline__ void block_add3(float& a, float& b, float& c, float* sh) {
-  a = wave_add(a); b = wave_add(b); c = wave_add(c);
+  a = wsum64(a); b = wsum64(b); c = wsum64(c);
   const uint32_t w = threadIdx.x >> 6;
   __syncthreads();
   if ((threadIdx.x & 63u) == 0) { sh[w] = a; sh[NW + w] = b; sh[2 * NW + w] = c; }
@@ -479,9 +479,9 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 // read as four consecutive columns per lane.  On their chain are only the products that the state needs (delta: W S, its sum
 // through LDS, K u); Q S and a quarter of B u, the wave's share of the outputs, go out while that sum is on its way.  A fifth
 // wave adds up the shares and stores them, a chunk behind: loads and stores share a counter, and a wave that does both waits
-// for its stores.  2048 tokens in 32 heads of 128, warm: outputs by the first of four waves, ahead of its part of the state, 127 us,
-// retention 93; so 105 and 76 (without any output 96 and 68, without loads either 86 and 61: what is left is 25 instructions
-// of 32 clocks, an exchange through LDS and its barrier a chunk).
+// for its stores.  2048 tokens in 32 heads of 128: outputs by the first of four waves, ahead of its part of the state, 127 us warm
+// (148 in a first pass), retention 93 (110); so 105 (115) and 76 (91).  Of the 115, with parts taken out: 106 without any output, 91
+// without loads either: what is left is 25 instructions of 32 clocks, an exchange through LDS and its barrier a chunk.
 // FEW: one or two chunks, whose operands are not asked for ahead, so that a compute unit has three workgroups instead of two (16
 // sequences of 12 tokens 26.5 us, 48.5 with the other form, 38.6 before).
 struct ScanArgs {

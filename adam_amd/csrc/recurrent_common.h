@@ -13,11 +13,6 @@ namespace adamah {
 #define NO_MEMORY 110.0f  // exp(-110) is zero in float32: a stronger decay per token changes nothing, and the sums stay small
 
 __device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
-__device__ __forceinline__ float wave_add(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 // silu of the causal convolution at token position p for channel ch, older inputs from the ring only.  The taps' loads do
 // not depend on each other: up to TM of them are asked for at once (TM >= taps).
 template <int TM>

@@ -66,6 +66,35 @@ def test_linear(hip, dtype, rows, n, k, groups, epi):
     p.same(WS, out, rows * (out_w + 3) - 3, tol, "out")
 
 
+@pytest.mark.parametrize("n,k,groups,epi,branched,act", [
+    (1, 1088, 1, 0, 0, 0), (2047, 1024, 0, 1, 0, 0), (2048, 2048, 1, 0, 2, 0), (2049, 2048, 4, 0, 0, 2), (2048, 2112, 1, 1, 1, 0),
+    (130, 4096, 1024, 0, 0, 3), (7, 4104, 1, 0, 2, 0), (2051, 4160, 1, 1, 0, 1), (67, 2048, 1, 2, 2, 0), (2050, 4096, 1, 0, 1, 0), (9, 8192, 2, 1, 0, 0),
+    (5, 32768, 1, 0, 0, 0), (3, 9000, 0, 0, 0, 0), (40, 960, 1, 0, 2, 0)])
+@pytest.mark.parametrize("listed,shift", [(False, 0), (True, 1)])
+def test_one_row_products(hip, n, k, groups, epi, branched, act, listed, shift):
+    """A wave has one row up to 2048 of them and two beyond, eight steps in flight beyond 2048 columns; rows on four floats (shift 0) and off."""
+    note(f"one row n {n} k {k} groups {groups} epi {epi} branched {branched} act {act} listed {listed} shift {shift}")
+    rng = np.random.default_rng(n + k)
+    ks, st, at, pos = (k + 63) // 64 * 64, (k + 3) // 4 * 4 + 4 + shift, {}, 4 + shift
+    tail = 3 if epi == 2 else 0
+    for name, sz in (("x", 3 * st), ("br", 3 * st), ("gate", 3 * st), ("wt", k), ("bw", k), ("res", 3 * st), ("keep", 3 * st), ("bias", n), ("out", n), ("tail", n)):
+        at[name] = pos
+        pos += (sz + 3) // 4 * 4 + (4 if shift == 0 else 3)
+    p = Pair(hip, pos, wt=n * ks)
+    W = np.zeros((n, ks), np.uint16)
+    W[:, :k] = f32_to_bf16((rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32))
+    p.put(WT, 0, W)
+    p.put(WS, 0, rng.standard_normal(pos))
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=ks, src=at["x"], src_stride=st, groups=groups, eps=1e-4, wt=at["wt"], wt_len=k if groups else 0, wt_add=0.5,
+                        gate=at["gate"], gate_stride=st, gate_act=act, branched=branched, branch=at["br"], branch_stride=st, branch_wt=at["bw"],
+                        res_out=at["res"], res_stride=st, keep=at["keep"], keep_stride=st, kept=1, bias=at["bias"], biased=int(epi == 0), out=at["out"],
+                        out_stride=n, epi=epi, tail=tail, tail_out=at["tail"], tail_stride=n)
+    p.call("linear_dev", WS, OP, WT, p.up(spec.words()), p.up([2]) if listed else 0, 1)
+    # float32 throughout: as for the operands above
+    for name, sz in (("out", (n - tail) // 2 if epi == 2 else n), ("keep", 3 * st), ("res", 3 * st), ("tail", max(tail, 1))):
+        p.same(WS, at[name], sz, 2e-5, name)
+
+
 @pytest.mark.parametrize("rows,n,k,biased,add", [
     (2000, 8170, 64, 0, 0), (2048, 4096, 128, 1, 1), (1999, 4090, 192, 1, 0), (600, 12600, 64, 0, 1), (300, 10300, 128, 1, 0),
     (300, 6001, 320, 0, 0), (40, 300, 256, 1, 1), (33, 64, 64, 0, 0), (100, 131, 1024, 0, 1)])
