@@ -3,8 +3,8 @@
 //
 // One row: two launches.  Every workgroup chooses the experts for itself (a row of logits is small: each candidate counts
 // those that beat it), so nothing has to wait for a launch that only chooses.  k_experts_in: gate and up rows of the chosen
-// experts, two matrix rows a wave; k_experts_out: a row of the result is one dot product over the chosen experts'
-// activations, already weighted, and the shared expert's behind each other; the row itself times the weights of those that
+// experts, two matrix rows a wave; k_experts_out: a row of the result is one dot product over the shared expert's activations
+// and the chosen experts', each run times its expert's weight; the row itself times the weights of those that
 // give it back is added at the end.
 //
 // More rows: k_experts_choose (a wave per row), k_experts_list (a workgroup per expert: its rows in order), then the two
@@ -23,11 +23,39 @@ typedef AdamahExpertsSpec XSpec;
 #define XSTEP 512u
 
 // ---- one row --------------------------------------------------------------------------------------------------------
-struct Chosen { float score[MAX_CHOICES], by[MAX_CHOICES]; uint32_t id[MAX_TOP]; float wt[MAX_TOP]; uint32_t n; float back; };
+struct Choice { uint32_t id[MAX_TOP]; float wt[MAX_TOP]; uint32_t n; float back; };
+struct Chosen : Choice { float score[MAX_CHOICES], by[MAX_CHOICES]; };
 // The chosen experts with matrices, best first, and their weights; n of them; back: what the row itself is multiplied by.
-__device__ __forceinline__ void choose_row(const XSpec& s, const float* act, Chosen& ch) {
+// Up to 64 candidates every wave chooses among by itself, one a lane, and all write the same words: no barrier (a wave may read
+// them at once), and what it needs (choose_ask) can be asked for ahead of everything else.
+struct Asked { float z, c; };
+__device__ __forceinline__ Asked choose_ask(const XSpec& s, const float* act) {
+  const uint32_t i = min(threadIdx.x & 63u, s.experts + s.identity - 1u);
+  return {act[s.logits + i], act[s.correction + i]};
+}
+__device__ __forceinline__ void choose_row(const XSpec& s, const float* act, const Asked& q, Chosen& ch) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, n = s.experts + s.identity;
   const float *z = act + s.logits, *corr = act + s.correction;
+  if (n <= 64u) {
+    const float mx = wmax64(q.z), e = lane < n ? expf(q.z - mx) : 0.f, p = e * (1.0f / wsum64(e)), me = p + q.c;
+    uint32_t rank = 0;
+#pragma unroll 8
+    for (uint32_t j = 0; j < n; j++) {
+      const float by = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(me), (int)j));
+      rank += by > me || (by == me && j < lane) ? 1u : 0u;
+    }
+    const int to = (int)((lane < n ? rank : lane) * 4u);     // lane r gets the candidate of rank r (nothing: 0)
+    const uint32_t id = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)(lane + 1u)) - 1u;
+    const float w = __uint_as_float((uint32_t)__builtin_amdgcn_ds_permute(to, (int)__float_as_uint(p)));
+    const bool real = lane < s.top && id < s.experts;
+    const uint64_t mask = __ballot(real);
+    const float back = wsum64(lane < s.top && !real ? w : 0.f);
+    const uint32_t at = __popcll(mask & ((1ull << lane) - 1ull));
+    if (real) { ch.id[at] = id; ch.wt[at] = w; }
+    if (lane == 0) { ch.n = __popcll(mask); ch.back = back; }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    return;
+  }
   float mx = -3.4e38f, sum = 0.f;
   for (uint32_t i = lane; i < n; i += 64u) mx = fmaxf(mx, z[i]);
 #pragma unroll
@@ -66,106 +94,158 @@ __device__ __forceinline__ void fma8(float& a, const uint4& w, const float4& lo,
 // x in LDS as two planes (elements 0..3 / 4..7 of every eight), so that a lane's two 16-byte reads are conflict free.
 #define PLANE(i, half) ((((i) >> 2) & 1u) * (half) + ((i) >> 3) * 4u + ((i) & 3u))
 
+// `left` runs of two buffers, both asked for already: each is asked for again behind its use while there are more
+#define RUNS_OF_TWO(left, run, fetch)                          \
+  do {                                                         \
+    for (; left > 3u; left -= 2u) { run(0); fetch(0); run(1); fetch(1); } \
+    if (left == 3u) { run(0); fetch(0); run(1); run(0); }      \
+    else if (left == 2u) { run(0); run(1); }                   \
+    else if (left == 1u) run(0);                               \
+  } while (0)
+// The first run of columns is asked for before x is staged, as soon as the choice is known; not two at a time (6 x 1024 pairs of rows
+// of 2048, 50 MB: 15.2 us, so 13.5).
 template <int U>
 __global__ void __launch_bounds__(XSTEP)
-k_experts_in(const bf16_t* __restrict__ W, float* act, const XSpec s) {
+k_experts_in(const bf16_t* __restrict__ W, float* act, Choice* choice, const XSpec s) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ Chosen ch;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, kp = s.k_stride, half = kp >> 1, F = (s.ff + 15u) & ~15u;
+  const Asked q = choose_ask(s, act);
   // (no load under a condition, here and below: each would wait for the one before; short rows have two values a thread)
   constexpr uint32_t R = U == 1 ? 2 : 4;
-  for (uint32_t i0 = threadIdx.x; i0 < kp; i0 += XSTEP * R) {
-    float v[R];
+  float v[R];
 #pragma unroll
-    for (uint32_t u = 0; u < R; u++) v[u] = act[s.x + min(i0 + u * XSTEP, s.width - 1u)];
-#pragma unroll
-    for (uint32_t u = 0; u < R; u++) { const uint32_t i = i0 + u * XSTEP; if (i < kp) xs[PLANE(i, half)] = i < s.width ? v[u] : 0.f; }
-  }
-  choose_row(s, act, ch);
+  for (uint32_t u = 0; u < R; u++) v[u] = act[s.x + min(threadIdx.x + u * XSTEP, s.width - 1u)];
+  choose_row(s, act, q, ch);
   const uint32_t n_tasks = ch.n * F;
-  for (uint32_t task = blockIdx.x * (XSTEP / 64u) + wave; task < n_tasks; task += gridDim.x * (XSTEP / 64u)) {
+  uint32_t task = blockIdx.x * (XSTEP / 64u) + wave, k0 = lane * 8u;
+  uint4 g[U], h[U];
+  const auto fetch = [&] {
     const uint32_t j = task / F, t = task - j * F;
     const bf16_t* wg = W + s.gate_up + (uint64_t)ch.id[j] * s.gate_up_step + (uint64_t)((t >> 4) * 32u + (t & 15u)) * kp;
-    const bf16_t* wu = wg + (uint64_t)16u * kp;
-    float a = 0.f, b = 0.f;
-    const auto steps = [&](auto n, uint32_t k0) {            // n runs of 512 columns, asked for together
-      constexpr int N = decltype(n)::value;
-      uint4 p[N], q[N];
 #pragma unroll
-      for (int u = 0; u < N; u++) { p[u] = *(const uint4*)(wg + k0 + 512u * u); q[u] = *(const uint4*)(wu + k0 + 512u * u); }
+    for (int u = 0; u < U; u++) {
+      const uint32_t k = min(k0 + 512u * u, kp - 8u);
+      g[u] = *(const uint4*)(wg + k); h[u] = *(const uint4*)(wg + (uint64_t)16u * kp + k);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (task < n_tasks) fetch();
 #pragma unroll
-      for (int u = 0; u < N; u++) {
-        const uint32_t k = k0 + 512u * u;
-        const float4 lo = *(const float4*)(xs + (k >> 1)), hi = *(const float4*)(xs + half + (k >> 1));
-        fma8(a, p[u], lo, hi); fma8(b, q[u], lo, hi);
-      }
-    };
-    uint32_t k0 = 0;
-    for (; k0 + 512u * U <= kp; k0 += 512u * U) steps(std::integral_constant<int, U>{}, k0 + lane * 8u);
-    for (k0 += lane * 8u; k0 < kp; k0 += 512u) steps(std::integral_constant<int, 1>{}, k0);
-    a = wsum64(a); b = wsum64(b);
-    if (lane == 0) act[s.act + j * s.ff_stride + t] = silu_f(a) * b;
+  for (uint32_t u = 0; u < R; u++) {
+    const uint32_t i = threadIdx.x + u * XSTEP;
+    if (i < kp) xs[PLANE(i, half)] = i < s.width ? v[u] : 0.f;
+  }
+  for (uint32_t i = threadIdx.x + R * XSTEP; i < kp; i += XSTEP) xs[PLANE(i, half)] = i < s.width ? act[s.x + i] : 0.f;
+  __syncthreads();
+  float a = 0.f, b = 0.f;
+  while (task < n_tasks) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t k = k0 + 512u * u;
+      if (k >= kp) break;
+      const float4 lo = *(const float4*)(xs + (k >> 1)), hi = *(const float4*)(xs + half + (k >> 1));
+      fma8(a, g[u], lo, hi); fma8(b, h[u], lo, hi);
+    }
+    const uint32_t done = task;
+    const bool last = k0 - lane * 8u + 512u * U >= kp;
+    if (last) { k0 = lane * 8u; task += gridDim.x * (XSTEP / 64u); } else k0 += 512u * U;
+    if (task < n_tasks) fetch();
+    if (last) {
+      a = wsum64(a); b = wsum64(b);
+      const uint32_t j = done / F;
+      if (lane == 0) act[s.act + j * s.ff_stride + done - j * F] = silu_f(a) * b;
+      a = b = 0.f;
+    }
+  }
+  if (blockIdx.x == 0u && threadIdx.x < MAX_TOP) {           // for the launch behind this one
+    choice->id[threadIdx.x] = ch.id[threadIdx.x]; choice->wt[threadIdx.x] = ch.wt[threadIdx.x];
+    if (threadIdx.x == 0u) { choice->n = ch.n; choice->back = ch.back; }
   }
 }
 
+// A row of the result a wave, the shared expert's columns first: they do not wait for the choice, nor do the activations, which
+// lie by place in the choice and get their weights in the sums.  Two runs of U times 512 columns in flight.
+// What bounds it is the weights' way in and what stands ahead of it (2048 rows of 6 x 1024 and 2048 columns, 33.5 MB, 6.9 us at a
+// large copy's rate: 14.2 us with two rows a wave, half the CUs at work and the activations weighted as they are staged, 12.5 so).
 template <int U>
 __global__ void __launch_bounds__(XSTEP)
-k_experts_out(const bf16_t* __restrict__ W, float* act, const XSpec s, uint32_t magic) {
+k_experts_out(const bf16_t* __restrict__ W, float* act, const Choice* __restrict__ choice, const XSpec s, uint32_t magic) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
-  __shared__ Chosen ch;
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, fs = s.ff_stride;
-  choose_row(s, act, ch);
-  const uint32_t body = ch.n * fs, kp = body + (s.shared_ff ? s.shared_ff_stride : 0u), half = kp >> 1;
-  const float sg = s.shared_ff ? sigmoid_f(act[s.logits + s.experts + s.identity]) : 0.f;
-  const uint32_t last = ch.n ? ch.n - 1u : 0u;
-  // Eight values a thread (of a short row two) asked for at once and no load under a condition, here and below (2048 rows of
-  // 6 x 1024 and 2048 columns, 33.5 MB: 17.9 us with each waiting for the one before, so: 14.2).
-  constexpr uint32_t R = U == 1 ? 2 : 8;
-  for (uint32_t i0 = threadIdx.x; i0 < kp; i0 += XSTEP * R) {
-    float v[R];
+  __shared__ Choice ch;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, fs = s.ff_stride, stride = gridDim.x * (XSTEP / 64u);
+  const uint32_t sk = s.shared_ff ? s.shared_ff_stride : 0u, held = sk + min(s.top, s.experts) * fs, half = held >> 1;
+  uint4 p[2][U];
+  uint32_t row = blockIdx.x * (XSTEP / 64u) + wave, k0 = lane * 8u, from = min(row, s.width - 1u), fk = k0, end = 0u;
+  // the next run: within the shared expert's columns, or anywhere once the choice is known
+  const auto fetch = [&](uint4 (&to)[U], bool chosen) {
 #pragma unroll
-    for (uint32_t u = 0; u < R; u++) {
-      const uint32_t i = min(i0 + u * XSTEP, kp - 1u), j = __umulhi(i, magic), c = i - j * fs;
-      v[u] = act[i < body ? s.act + j * fs + min(c, s.ff - 1u) : s.shared_act + min(i - body, s.shared_ff - 1u)];
+    for (int u = 0; u < U; u++) {
+      const uint32_t k = chosen ? min(fk + 512u * u, end - 8u) : fk + 512u * u, c = max(k, sk) - sk, j = __umulhi(c, magic);
+      const uint64_t at = !chosen || k < sk ? s.shared_down + (uint64_t)from * s.shared_ff_stride + k
+                                            : s.down + (uint64_t)ch.id[j] * s.down_step + (uint64_t)from * fs + (c - j * fs);
+      to[u] = *(const uint4*)(W + at);
     }
+    fk += 512u * U;
+    if (chosen && fk - lane * 8u >= end) { fk = lane * 8u; from += stride; }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const bool early = sk >= 512u * U;
+  const uint32_t id = choice->id[lane], n_ch = choice->n;    // (a word a lane: MAX_TOP of them)
+  const float wt = choice->wt[lane], back = choice->back;
+  const float gate = act[s.logits + s.experts + s.identity - (s.shared_ff ? 0u : 1u)];
+  // Sixteen values a thread (of a short row two) asked for at once and no load under a condition
+  constexpr uint32_t R = U == 1 ? 2 : 16;
+  const auto value = [&](uint32_t i0) {
+    const uint32_t i = min(i0, held - 1u), c = max(i, sk) - sk, j = __umulhi(c, magic);
+    return act[i < sk ? s.shared_act + min(i, s.shared_ff - 1u) : s.act + j * fs + min(c - j * fs, s.ff - 1u)];
+  };
+  float v[R];
 #pragma unroll
-    for (uint32_t u = 0; u < R; u++) {
-      const uint32_t i = i0 + u * XSTEP, j = min(__umulhi(i, magic), last), c = i < body ? i - j * fs : i - body;
-      if (i < kp) xs[PLANE(i, half)] = i < body ? (c < s.ff ? v[u] * ch.wt[j] : 0.f) : c < s.shared_ff ? v[u] * sg : 0.f;
-    }
+  for (uint32_t u = 0; u < R; u++) v[u] = value(threadIdx.x + u * XSTEP);
+  if (early) fetch(p[0], false);
+  ch.id[lane] = id; ch.wt[lane] = wt;                        // (every wave the same words, for itself)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  end = sk + n_ch * fs;
+  uint32_t left = row < s.width ? ((s.width - 1u - row) / stride + 1u) * max(1u, (end + 512u * U - 1u) / (512u * U)) : 0u;
+  if (end && left > 0u) {
+    if (!early) fetch(p[0], true);
+    else if (fk - lane * 8u >= end) { fk = lane * 8u; from += stride; }
+    if (left > 1u) fetch(p[1], true);
   }
+  const float sg = sigmoid_f(gate);
+  const auto put = [&](uint32_t i, float x) {
+    const uint32_t c = max(i, sk) - sk, j = __umulhi(c, magic);
+    if (i < held) xs[PLANE(i, half)] = i < sk ? (i < s.shared_ff ? x * sg : 0.f) : c - j * fs < s.ff ? x : 0.f;
+  };
+#pragma unroll
+  for (uint32_t u = 0; u < R; u++) put(threadIdx.x + u * XSTEP, v[u]);
+  for (uint32_t i = threadIdx.x + R * XSTEP; i < held; i += XSTEP) put(i, value(i));
   __syncthreads();
-  const uint32_t n_tasks = (s.width + 1u) >> 1;
-  for (uint32_t task = blockIdx.x * (XSTEP / 64u) + wave; task < n_tasks; task += gridDim.x * (XSTEP / 64u)) {
-    const uint32_t r0 = task * 2u, r1 = min(r0 + 1u, s.width - 1u);
-    float a = 0.f, b = 0.f;
-    const auto steps = [&](auto n, uint32_t k0) {
-      constexpr int N = decltype(n)::value;
-      uint4 p[N], q[N];
+  float a = 0.f;
+  const auto more = [&](int x) { if (end) fetch(p[x], true); };
+  const auto run = [&](int x) {
+    if (end)
 #pragma unroll
-      for (int u = 0; u < N; u++) {
-        const uint32_t k = k0 + 512u * u, j = min(__umulhi(k, magic), last), st = k < body ? fs : s.shared_ff_stride;
-        const uint64_t at = k < body ? s.down + (uint64_t)ch.id[j] * s.down_step + (k - j * fs) : s.shared_down + (uint64_t)(k - body);
-        p[u] = *(const uint4*)(W + at + (uint64_t)r0 * st); q[u] = *(const uint4*)(W + at + (uint64_t)r1 * st);
-      }
-#pragma unroll
-      for (int u = 0; u < N; u++) {
-        const uint32_t k = k0 + 512u * u;
+      for (int u = 0; u < U; u++) {
+        const uint32_t k = k0 + 512u * u, j = __umulhi(max(k, sk) - sk, magic);
+        if (k >= end) break;
         const float4 lo = *(const float4*)(xs + (k >> 1)), hi = *(const float4*)(xs + half + (k >> 1));
-        fma8(a, p[u], lo, hi); fma8(b, q[u], lo, hi);
+        float t = 0.f;
+        fma8(t, p[x][u], lo, hi);
+        a = fmaf(k < sk ? 1.f : ch.wt[j], t, a);
       }
-    };
-    uint32_t k0 = 0;
-    for (; k0 + 512u * U <= kp; k0 += 512u * U) steps(std::integral_constant<int, U>{}, k0 + lane * 8u);
-    for (k0 += lane * 8u; k0 < kp; k0 += 512u) steps(std::integral_constant<int, 1>{}, k0);
-    a = wsum64(a); b = wsum64(b);
-    if (lane < 2u && r0 + lane < s.width) {
-      const uint32_t r = r0 + lane;
-      const float y = fmaf(ch.back, act[s.x + r], lane ? b : a);
-      float* d = act + s.out + r;
+    k0 += 512u * U;
+    if (k0 - lane * 8u < end) return;
+    a = wsum64(a);
+    if (lane == 0) {
+      const float y = fmaf(back, act[s.x + row], a);
+      float* d = act + s.out + row;
       *d = s.epi ? *d + y : y;
     }
-  }
+    a = 0.f; k0 = lane * 8u; row += stride;
+  };
+  RUNS_OF_TWO(left, run, more);
 }
 
 // ---- more rows ------------------------------------------------------------------------------------------------------
@@ -438,16 +518,18 @@ extern "C" int adamah_experts_dev(uint32_t map_act, uint32_t map_opnd, uint32_t 
     if (held > MAX_STEP || !in_range(s->act, most * fs, ma->n_elems)) return ADAMAH_ERR_INVALID;
     if (s->shared_ff && (s->shared_ff_stride < s->shared_ff || (s->shared_ff_stride & 63u) || (s->shared_down & 7u) ||
                          !in_range(s->shared_down, wd * s->shared_ff_stride, mw->n_elems) || !in_range(s->shared_act, s->shared_ff, ma->n_elems))) return ADAMAH_ERR_INVALID;
+    if (int r = scratch_need(g_experts, sizeof(Choice))) return r;
+    Choice* choice = (Choice*)g_experts.p;
     const uint32_t cu2 = 2u * (uint32_t)g.n_cu, in_grid = std::min<uint32_t>(cdiv(most * F16, XSTEP / 64), cu2), in_lds = s->k_stride * 4u;
-    const uint32_t out_grid = std::min<uint32_t>(cdiv(cdiv(wd, 2), XSTEP / 64), cu2), out_lds = (uint32_t)held * 4u;
+    const uint32_t out_grid = std::min<uint32_t>(cdiv(wd, XSTEP / 64), cu2), out_lds = (uint32_t)held * 4u;
     const uint32_t magic = (uint32_t)((0x100000000ull + fs - 1) / fs);       // i / fs = umulhi(i, magic) for i <= MAX_STEP
 #define LDS_FOR(K, B) if ((B) > 48000) hipFuncSetAttribute((const void*)(K), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(B))
-    if (s->k_stride >= 1024u) { LDS_FOR(k_experts_in<4>, in_lds); k_experts_in<4><<<in_grid, XSTEP, in_lds, g.stream>>>(W, act, *s); }
-    else k_experts_in<1><<<in_grid, XSTEP, in_lds, g.stream>>>(W, act, *s);
+    if (s->k_stride >= 1024u) { LDS_FOR(k_experts_in<4>, in_lds); k_experts_in<4><<<in_grid, XSTEP, in_lds, g.stream>>>(W, act, choice, *s); }
+    else k_experts_in<1><<<in_grid, XSTEP, in_lds, g.stream>>>(W, act, choice, *s);
     count_launch();
     if (int r = check_launch()) return r;
-    if (held >= 1024u) { LDS_FOR(k_experts_out<4>, out_lds); k_experts_out<4><<<out_grid, XSTEP, out_lds, g.stream>>>(W, act, *s, magic); }
-    else k_experts_out<1><<<out_grid, XSTEP, out_lds, g.stream>>>(W, act, *s, magic);
+    if (held >= 1024u) { LDS_FOR(k_experts_out<4>, out_lds); k_experts_out<4><<<out_grid, XSTEP, out_lds, g.stream>>>(W, act, choice, *s, magic); }
+    else k_experts_out<1><<<out_grid, XSTEP, out_lds, g.stream>>>(W, act, choice, *s, magic);
 #undef LDS_FOR
     count_launch();
     return check_launch();

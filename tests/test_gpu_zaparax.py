@@ -363,6 +363,13 @@ def test_experts(hip, E, I, top, ff, shared, width, epi, dtype):
         p.same(WS, at["out"], rows * width, 5e-5 if dtype == "float32" or rows == 1 else 4e-2, f"rows {rows}")
 
 
+@pytest.mark.parametrize("E,I,top,ff,shared,width,epi", [(4, 2, 3, 1000, 2100, 300, 0), (2, 30, 2, 512, 0, 70, 1), (2, 60, 3, 500, 2048, 33, 0),
+                                                         (3, 1, 2, 64, 576, 4200, 1), (33, 31, 8, 700, 0, 2070, 0)])
+def test_experts_of_every_schedule(hip, E, I, top, ff, shared, width, epi):
+    """One row: shared columns of a whole run and less, no chosen expert with a matrix, one and more rows a wave, 64 candidates."""
+    test_experts(hip, E, I, top, ff, shared, width, epi, "float32")
+
+
 def test_experts_with_equal_scores_take_the_first(hip):
     note("experts, equal scores")
     E, w = 6, 32
