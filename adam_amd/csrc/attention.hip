@@ -22,13 +22,11 @@ __device__ __forceinline__ float ld(const float* p, uint64_t i) { return p[i]; }
 __device__ __forceinline__ float ld(const __half* p, uint64_t i) { return __half2float(p[i]); }
 
 __device__ __forceinline__ float wave_sum64(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_add(v);
   return v;
 }
 __device__ __forceinline__ float wave_max64(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  v = wave_max(v);
   return v;
 }
 

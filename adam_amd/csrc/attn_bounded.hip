@@ -116,12 +116,12 @@ k_attn_step(const ASpec s, float* act, T* cache, float* part, uint32_t seq0, uin
   if (own && !WIN) {
     iv = 0.f;
     for (uint32_t d = lane; d < V; d += 64u) iv = fmaf(xv[d], xv[d], iv);
-    iv = 1.0f / sqrtf(wsum64(iv) / (float)V + s.eps);
+    iv = 1.0f / sqrtf(wave_add(iv) / (float)V + s.eps);
   }
   if (own && WIN && s.qk_norm) {
     ik = 0.f;
     for (uint32_t d = lane; d < D; d += 64u) ik = fmaf(xk[d], xk[d], ik);
-    ik = 1.0f / sqrtf(wsum64(ik) / (float)D + s.eps);
+    ik = 1.0f / sqrtf(wave_add(ik) / (float)D + s.eps);
   }
   if (WIN && wave < nh) {                                       // a wave per query head: what its scores are multiplied by
     const float* xq = x + s.x_q + (h0 + wave) * D;
@@ -129,7 +129,7 @@ k_attn_step(const ASpec s, float* act, T* cache, float* part, uint32_t seq0, uin
     if (s.qk_norm) {
       float a = 0.f;
       for (uint32_t d = lane; d < D; d += 64u) a = fmaf(xq[d], xq[d], a);
-      f /= sqrtf(wsum64(a) / (float)D + s.eps);
+      f /= sqrtf(wave_add(a) / (float)D + s.eps);
     }
     if (lane == 0) qi[wave] = s.softcap > 0.f ? f / s.softcap : f * LOG2E;
   }
@@ -266,7 +266,7 @@ k_attn_join(const ASpec s, float* act, const float* __restrict__ part, uint32_t 
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     const float e = lane < n_part ? __builtin_amdgcn_exp2f(m - mx) : 0.f;
-    w[lane] = e / (wsum64(e * l) + (s.has_sink ? __builtin_amdgcn_exp2f(sk - mx) : 0.f));
+    w[lane] = e / (wave_add(e * l) + (s.has_sink ? __builtin_amdgcn_exp2f(sk - mx) : 0.f));
   }
   __syncthreads();
   for (uint32_t d = threadIdx.x; d < V; d += 256u) {

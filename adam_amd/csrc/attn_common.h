@@ -2,6 +2,7 @@
 // decode kernel.
 #pragma once
 #include "common.h"
+#include "lanes.h"
 #include <vector>
 
 namespace adamah {

@@ -180,8 +180,7 @@ k_attn_decode(const float* data, const __half* kv, uint64_t kv_shift, uint32_t r
         if (i < (uint32_t)(G * D)) {
           qs[i] = qraw[u];
           float m = fabsf(qraw[u]);
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+          m = wave_max(m);
           if (lane == 0u) atomicMax(&hmax[i / D], __float_as_uint(m));
         }
       }
@@ -231,8 +230,7 @@ k_attn_decode(const float* data, const __half* kv, uint64_t kv_shift, uint32_t r
           qs[i] = qraw[u];
           if (rp.flags & 1u) {
             float ss = fmaf(qraw[u], qraw[u], 0.f);
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+            ss = wave_add(ss);
             if (lane == 0u) ssq[i >> 6] = ss;
           }
         }
@@ -241,8 +239,7 @@ k_attn_decode(const float* data, const __half* kv, uint64_t kv_shift, uint32_t r
         kraw_s[tid] = kraw;
         if (rp.flags & 1u) {
           float ss = fmaf(kraw, kraw, 0.f);
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+          ss = wave_add(ss);
           if (lane == 0u) ssk[tid >> 6] = ss;
         }
         // the V row: rounded to fp16 for the copy, and the rounded value into the float32 row
@@ -280,8 +277,7 @@ k_attn_decode(const float* data, const __half* kv, uint64_t kv_shift, uint32_t r
             qd[i] = r0; qd[i + half] = r1;
           }
           float m = fmaxf(fabsf(r0), fabsf(r1));
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+          m = wave_max(m);
           if (lane == 0u) atomicMax(&hmax[h], __float_as_uint(m));
           if (u == 0u && tail_wg && tid < half) {
             // the new K row: same angle as this thread's query pair (tid = i); stored as the row tasks store it

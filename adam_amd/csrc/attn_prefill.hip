@@ -98,8 +98,7 @@ k_attn_prefill(const float* data, float* out, const __half* kv, uint64_t kv_shif
       const float x = r < rows ? data[(uint64_t)bs.q[head] + (uint64_t)(t0 + r) * q_stride + i % D] : 0.f;
       qs[i] = x;
       float mx = fabsf(x);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+      mx = wave_max(mx);
       if (lane == 0u) atomicMax(&hmax[r], __float_as_uint(mx));
     }
     if (rbase < nkeys) fetch(kA, vA, rbase);
@@ -373,7 +372,7 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
 #pragma unroll
       for (int t = 0; t < 8; t++) { if (n >= rows) x[st][t] = 0.f; mx = fmaxf(mx, fabsf(x[st][t])); }
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64)); mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_x32(max_x16(mx));
     const uint32_t e = (__float_as_uint(mx) >> 23) & 0xFFu;
     float s = 1.f;
     inv_s = 1.f;
@@ -458,7 +457,7 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
           if (key < lim && last) out[sc_row + key] = ((RUNS ? s[kb][0][r] + s[kb][2][r] : s[kb][0][r]) + s[kb][1][r]) * inv_s;
         }
     }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64)); mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = max_x32(max_x16(mt));
     const float m_new = fmaxf(m_run, RUNS ? ceilf(mt) : mt);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     const bool moved = m_new > m_run;
@@ -531,8 +530,7 @@ k_attn_prefill_mfma(const float* data, float* out, const uint4* __restrict__ kt,
       for (int r = 0; r < 4; r++) acc[b][r] = acc[b][r] * g0[r] + mine[(2 + 4 * b + r) * 64] * g1[r];
   }
 
-  float l_tot = l_run + __shfl_xor(l_run, 16, 64);
-  l_tot += __shfl_xor(l_tot, 32, 64);
+  const float l_tot = add_x32(add_x16(l_run));
   if (splits > 1u) {
     const uint64_t row0 = ((uint64_t)split * H + head) * m + t0;      // [run of keys][head][token]
     float* const ms = part + (uint64_t)splits * H * m * D;            // the values of all rows, then their (maximum, sum)

@@ -37,7 +37,7 @@ __device__ __forceinline__ void choose_row(const XSpec& s, const float* act, con
   const uint32_t tid = threadIdx.x, lane = tid & 63u, n = s.experts + s.identity;
   const float *z = act + s.logits, *corr = act + s.correction;
   if (n <= 64u) {
-    const float mx = wmax64(q.z), e = lane < n ? expf(q.z - mx) : 0.f, p = e * (1.0f / wsum64(e)), me = p + q.c;
+    const float mx = wave_max(q.z), e = lane < n ? expf(q.z - mx) : 0.f, p = e * (1.0f / wave_add(e)), me = p + q.c;
     uint32_t rank = 0;
 #pragma unroll 8
     for (uint32_t j = 0; j < n; j++) {
@@ -49,7 +49,7 @@ __device__ __forceinline__ void choose_row(const XSpec& s, const float* act, con
     const float w = __uint_as_float((uint32_t)__builtin_amdgcn_ds_permute(to, (int)__float_as_uint(p)));
     const bool real = lane < s.top && id < s.experts;
     const uint64_t mask = __ballot(real);
-    const float back = wsum64(lane < s.top && !real ? w : 0.f);
+    const float back = wave_add(lane < s.top && !real ? w : 0.f);
     const uint32_t at = __popcll(mask & ((1ull << lane) - 1ull));
     if (real) { ch.id[at] = id; ch.wt[at] = w; }
     if (lane == 0) { ch.n = __popcll(mask); ch.back = back; }
@@ -58,10 +58,9 @@ __device__ __forceinline__ void choose_row(const XSpec& s, const float* act, con
   }
   float mx = -3.4e38f, sum = 0.f;
   for (uint32_t i = lane; i < n; i += 64u) mx = fmaxf(mx, z[i]);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
   for (uint32_t i = lane; i < n; i += 64u) sum += expf(z[i] - mx);
-  const float inv = 1.0f / wsum64(sum);
+  const float inv = 1.0f / wave_add(sum);
   for (uint32_t i = tid; i < n; i += XSTEP) { const float p = expf(z[i] - mx) * inv; ch.score[i] = p; ch.by[i] = p + corr[i]; }
   if (tid < MAX_TOP) { ch.id[tid] = 0xFFFFFFFFu; ch.wt[tid] = 0.f; }
   __syncthreads();
@@ -78,7 +77,7 @@ __device__ __forceinline__ void choose_row(const XSpec& s, const float* act, con
     const float w = ch.wt[lane];
     const bool real = e < s.experts;
     const uint64_t mask = __ballot(real);
-    const float back = wsum64(real ? 0.f : w);
+    const float back = wave_add(real ? 0.f : w);
     const uint32_t at = __popcll(mask & ((1ull << lane) - 1ull));
     if (real) { ch.id[at] = e; ch.wt[at] = w; }              // (one wave: every lane has read its own before)
     if (lane == 0) { ch.n = __popcll(mask); ch.back = back; }
@@ -152,7 +151,7 @@ k_experts_in(const bf16_t* __restrict__ W, float* act, Choice* choice, const XSp
     if (last) { k0 = lane * 8u; task += gridDim.x * (XSTEP / 64u); } else k0 += 512u * U;
     if (task < n_tasks) fetch();
     if (last) {
-      a = wsum64(a); b = wsum64(b);
+      a = wave_add(a); b = wave_add(b);
       const uint32_t j = done / F;
       if (lane == 0) act[s.act + j * s.ff_stride + done - j * F] = silu_f(a) * b;
       a = b = 0.f;
@@ -237,7 +236,7 @@ k_experts_out(const bf16_t* __restrict__ W, float* act, const Choice* __restrict
       }
     k0 += 512u * U;
     if (k0 - lane * 8u < end) return;
-    a = wsum64(a);
+    a = wave_add(a);
     if (lane == 0) {
       const float y = fmaf(back, act[s.x + row], a);
       float* d = act + s.out + row;
@@ -259,11 +258,10 @@ k_experts_choose(const XSpec s, const float* __restrict__ act, uint32_t* __restr
   float p[NV], by[NV], mx = -3.4e38f, sum = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; i++) { const uint32_t e = lane + 64u * i; p[i] = e < n ? z[e] : -3.4e38f; mx = fmaxf(mx, p[i]); }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
 #pragma unroll
   for (int i = 0; i < NV; i++) { p[i] = lane + 64u * i < n ? expf(p[i] - mx) : 0.f; sum += p[i]; }
-  const float inv = 1.0f / wsum64(sum);
+  const float inv = 1.0f / wave_add(sum);
 #pragma unroll
   for (int i = 0; i < NV; i++) { const uint32_t e = lane + 64u * i; p[i] *= inv; by[i] = e < n ? p[i] + act[s.correction + e] : -3.4e38f; }
   uint32_t gone = 0;                                        // bit i: candidate lane + 64 i has been taken

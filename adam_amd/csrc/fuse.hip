@@ -51,8 +51,7 @@ k_rmsnorm_v(const float* act, const float* wt, float* out, uint32_t src, uint32_
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   float ss = 0.f;
   for (uint32_t i = tid; i < dim; i += 1024u) { const float x = act[(uint64_t)src + i]; ss = fmaf(x, x, ss); }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+  ss = wave_add(ss);
   if (lane == 0) sh[wave] = ss;
   __syncthreads();
   ss = 0.f;

@@ -71,8 +71,7 @@ k_act_f16(const float* act, const uint32_t* __restrict__ la, uint32_t M, uint32_
   const float* src = act + (uint64_t)la[op] + (uint64_t)row * K;
   float m = 0.f;
   for (uint32_t i = tid; i < K; i += 256u) m = fmaxf(m, fabsf(src[i]));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  m = wave_max(m);
   if ((tid & 63u) == 0) red[tid >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -1094,8 +1093,7 @@ k_act_f16_regs(const float* act, uint32_t K, uint32_t M, uint32_t a_val, uint32_
                          fmaxf(fmaxf(fabsf(v1[u].x), fabsf(v1[u].y)), fmaxf(fabsf(v1[u].z), fabsf(v1[u].w)))));
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  m = wave_max(m);
   if ((tid & 63u) == 0) red[tid >> 6] = m;
   __syncthreads();
   m = red[0];
@@ -1269,8 +1267,7 @@ k_attn_merge_rows_f16(float* out, const float* __restrict__ partial, uint32_t o0
       for (int k = 0; k < 8; k++) m = fmaxf(m, fabsf(v[u][k]));
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  m = wave_max(m);
   if ((tid & 63u) == 0) red[tid >> 6] = m;
   __syncthreads();
   m = red[0];

@@ -1,6 +1,7 @@
 // Device helpers and launch declarations shared by the quantised GEMV translation units.
 #pragma once
 #include "common.h"
+#include "lanes.h"
 
 namespace adamah {
 
@@ -18,8 +19,7 @@ __device__ __forceinline__ bool better(float cv, uint32_t ci, float bv, uint32_t
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_add(v);
   return v;
 }
 

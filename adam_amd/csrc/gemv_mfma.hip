@@ -264,14 +264,21 @@ k_gemv_mfma(const float* xp, const uint8_t* __restrict__ W, const __half* __rest
     const f4u_t v0 = ((const f4u_t*)p)[0], v1 = ((const f4u_t*)p)[1];
     v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w; v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
   };
+  // the waves' sums in order (all sixteen asked for at once; a loop over them waited for each)
+  auto add_waves = [&](const float* red) {
+    float r[16], t = 0.f;
+#pragma unroll
+    for (uint32_t w = 0; w < 16u; w++) r[w] = red[w];
+#pragma unroll
+    for (uint32_t w = 0; w < 16u; w++) t += w < nwav ? r[w] : 0.f;
+    return t;
+  };
   auto block_sum = [&](float v) {     // sum over the workgroup, same value in every thread
     v = wave_sum_to_lane63(v);
     __syncthreads();                  // red_f may still be read from the previous use
     if (lane == 63u) red_f[wave] = v;
     __syncthreads();
-    float t = 0.f;
-    for (uint32_t w = 0; w < nwav; w++) t += red_f[w];
-    return t;
+    return add_waves(red_f);
   };
 
   float nrm1 = 1.f, nrm_late = 1.f;   // nrm_late: the prologue's last norm, applied to the row sums
@@ -473,8 +480,7 @@ k_gemv_mfma(const float* xp, const uint8_t* __restrict__ W, const __half* __rest
     ss_last = wave_sum_to_lane63(ss_last);
     if (lane == 63u) red_g[wave] = ss_last;
     __syncthreads();          // the staged activations and the waves' partial sums are in LDS
-    float tot = 0.f;
-    for (uint32_t w = 0; w < nwav; w++) tot += red_g[w];
+    const float tot = add_waves(red_g);
     nrm_late = 1.0f / sqrtf(tot / (float)K + (PRO == PRO_NORM2 ? fz.p_eps2 : fz.p_eps));
     if (blockIdx.x == 0) {    // the normalised vector itself, where the norm op would have stored it
 #pragma unroll
@@ -565,8 +571,8 @@ k_gemv_mfma(const float* xp, const uint8_t* __restrict__ W, const __half* __rest
       if (chunk + ks >= C) { part[wave * 64u + lane] = acc; res_keep = Rl.res; }   // this wave's share of the bundle is done
     } else if (chunk == C - 1u) {   // row bundle complete: sum the 16 lanes that share a row
       float y = acc;
-      y += __shfl_xor(y, 4, 64); y += __shfl_xor(y, 8, 64);
-      y += __shfl_xor(y, 16, 64); y += __shfl_xor(y, 32, 64);
+      y += lane_x4(y); y += LANE_X8(y);
+      y = add_x32(add_x16(y));
       if (PRO == PRO_RMSNORM || PRO == PRO_NORM2) y *= nrm_late;
       acc = 0.f;
       if (glu) {
@@ -645,8 +651,8 @@ k_gemv_mfma(const float* xp, const uint8_t* __restrict__ W, const __half* __rest
       if (kpart == 0u && first < N) {
         float y = part[wave * 64u + lane];
         for (uint32_t pk = 1; pk < ks; pk++) y += part[(wave + pk) * 64u + lane];
-        y += __shfl_xor(y, 4, 64); y += __shfl_xor(y, 8, 64);
-        y += __shfl_xor(y, 16, 64); y += __shfl_xor(y, 32, 64);
+        y += lane_x4(y); y += LANE_X8(y);
+        y = add_x32(add_x16(y));
         if (PRO == PRO_RMSNORM || PRO == PRO_NORM2) y *= nrm_late;
         const uint32_t row = first + l;
         if (row < N && bcol == 0u) {

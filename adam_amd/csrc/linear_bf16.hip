@@ -38,7 +38,7 @@ void scratch_free(Scratch& s) {
 // Sum over a workgroup of NW waves; sh: NW floats that no earlier sum still reads.
 template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* sh) {
-  v = wsum64(v);
+  v = wave_add(v);
   if ((threadIdx.x & 63u) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   v = 0.f;
@@ -55,7 +55,7 @@ __device__ __forceinline__ void group_inverse(uint32_t k, uint32_t groups, float
     for (uint32_t gi = wave; gi < groups; gi += NW) {
       float ss = 0.f;
       for (uint32_t i = lane; i < gs; i += 64u) { const float v = val(gi * gs + i); ss = fmaf(v, v, ss); }
-      ss = wsum64(ss);
+      ss = wave_add(ss);
       if (lane == 0) inv[gi] = 1.0f / sqrtf(ss / (float)gs + eps);
     }
     __syncthreads();
@@ -64,7 +64,7 @@ __device__ __forceinline__ void group_inverse(uint32_t k, uint32_t groups, float
     float ss = 0.f;
     if (gi < groups)
       for (uint32_t i = sp * 64u + lane; i < gs; i += sub * 64u) { const float v = val(gi * gs + i); ss = fmaf(v, v, ss); }
-    ss = wsum64(ss);
+    ss = wave_add(ss);
     if (lane == 0) part[wave] = ss;
     __syncthreads();
     if (tid < groups) {
@@ -251,7 +251,7 @@ __device__ __forceinline__ void operand_row(const RowArgs& r, const LinSpec& s, 
 #pragma unroll
       for (int j = 0; j < R; j++) {
         if ((uint32_t)j * NT >= n4) break;
-        const float t = wsum64(ss[j]);
+        const float t = wave_add(ss[j]);
         if ((tid & 63u) == 0u) part[j * NW + wave] = t;
       }
       __syncthreads();
@@ -260,7 +260,7 @@ __device__ __forceinline__ void operand_row(const RowArgs& r, const LinSpec& s, 
         if ((uint32_t)j * NT >= n4) break;                   // (all lanes or none: they add up together)
         if (j > 0 && MODE_GROUPS(mode) == 1u) { scale[j] = scale[0]; continue; }
         const uint32_t lane = tid & 63u, b0 = ((uint32_t)j * NW + wave) / nb * nb;         // (a partial sum a lane)
-        scale[j] = 1.0f / sqrtf(wsum64(lane < nb ? part[min(b0 + lane, (uint32_t)(R * NW) - 1u)] : 0.f) / n + s.eps);
+        scale[j] = 1.0f / sqrtf(wave_add(lane < nb ? part[min(b0 + lane, (uint32_t)(R * NW) - 1u)] : 0.f) / n + s.eps);
       }
     }
 #pragma unroll
@@ -436,7 +436,7 @@ k_gemv_bf16(const bf16_t* __restrict__ W, float* act, const uint32_t* __restrict
     }
     if (last) {
 #pragma unroll
-      for (int q = 0; q < R; q++) a[q] = wsum64(a[q]);
+      for (int q = 0; q < R; q++) a[q] = wave_add(a[q]);
       if (EPI == LEPI_PAIR && task < pairs) {
         if (lane == 0) act[s.out + task] = silu_f(a[0]) * a[R - 1];
       } else {
@@ -548,7 +548,7 @@ k_head_rows(const bf16_t* __restrict__ W, float* act, const LinSpec s, const flo
         float logit = 0.f;
 #pragma unroll
         for (int r = 0; r < NR; r++) {
-          float y = wsum64(a[r][j]);
+          float y = wave_add(a[r][j]);
           y = s.biased ? y + bias : y;
           a[r][j] = 0.f;
           logit = r == (int)kept ? y : logit;
@@ -1038,7 +1038,7 @@ k_merge_norm(const AdamahMergeSpec s, float* act) {
   float sa = 0.f, sb = 0.f;
 #pragma unroll 4
   for (uint32_t i = tid; i < s.dim; i += NT) { sa = fmaf(a[i], a[i], sa); sb = fmaf(b[i], b[i], sb); }
-  sa = wsum64(sa); sb = wsum64(sb);
+  sa = wave_add(sa); sb = wave_add(sb);
   if (lane == 0) { sh[0][wave] = sa; sh[1][wave] = sb; }
   __syncthreads();
   sa = sb = 0.f;

@@ -1,5 +1,6 @@
 // Products with bfloat16 weight maps: the operand structs shared by the launchers and the ops built on them.
 #pragma once
+#include "lanes.h"
 #include "lds_ring.h"
 #include "../../include/adamah_hip.h"
 
@@ -22,28 +23,6 @@ __device__ __forceinline__ float row16_sum(float v) {
   ROW16_ADD(0xB1); ROW16_ADD(0x4E); ROW16_ADD(0x141); ROW16_ADD(0x140);   // quads, then the row's halves and the row mirrored
 #undef ROW16_ADD
   return v;
-}
-
-// The same over all 64 lanes: rows change places in the vector unit too (six exchanges through LDS, each waiting for the one
-// before, took a norm of a row and its two barriers 0.5 us longer).
-__device__ __forceinline__ float wsum64(float v) {
-  typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
-  const uint32_t r = __float_as_uint(row16_sum(v));
-  const u2_t a = __builtin_amdgcn_permlane16_swap(r, r, false, false);
-  const uint32_t h = __float_as_uint(__uint_as_float(a.x) + __uint_as_float(a.y));
-  const u2_t b = __builtin_amdgcn_permlane32_swap(h, h, false, false);
-  return __uint_as_float(b.x) + __uint_as_float(b.y);
-}
-
-__device__ __forceinline__ float wmax64(float v) {
-  typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
-#define ROW16_MAX(ctrl) v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, false)))
-  ROW16_MAX(0xB1); ROW16_MAX(0x4E); ROW16_MAX(0x141); ROW16_MAX(0x140);
-#undef ROW16_MAX
-  const u2_t a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const uint32_t h = __float_as_uint(fmaxf(__uint_as_float(a.x), __uint_as_float(a.y)));
-  const u2_t b = __builtin_amdgcn_permlane32_swap(h, h, false, false);
-  return fmaxf(__uint_as_float(b.x), __uint_as_float(b.y));
 }
 
 // ---- tiles of the many-row products ---------------------------------------------------------------------------------

@@ -11,8 +11,7 @@
 namespace adamah {
 
 __device__ __forceinline__ float block_sum_256(float v, float* sh) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = wave_add(v);
   if ((threadIdx.x & 63u) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   float t = (sh[0] + sh[1]) + (sh[2] + sh[3]);
@@ -106,8 +105,7 @@ k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, ui
     for (int e = 0; e < PER; e++) ss = tid + 256u * e < dim ? fmaf(x[e], x[e], ss) : ss;
   }
   if (tid < 256u) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    ss = wave_add(ss);
     if ((tid & 63u) == 0) sums[tid >> 6] = ss;
   }
   __syncthreads();
@@ -128,8 +126,7 @@ k_rmsnorm_rows(const float* act, const float* wt, uint32_t dim_on, float eps, ui
   }
   if constexpr (EMIT) {
     if (!in) m = 0.f;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    m = wave_max(m);
     if ((tid & 63u) == 0) tops[tid >> 6] = m;
     __syncthreads();
     m = tops[0];

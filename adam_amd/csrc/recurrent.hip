@@ -27,7 +27,7 @@ typedef AdamahRetentionSpec RSpec;
 // sums over a workgroup of NW waves of up to three values at once; sh: 3 NW floats
 template <int NW>
 __device__ __forceinline__ void block_add3(float& a, float& b, float& c, float* sh) {
-  a = wsum64(a); b = wsum64(b); c = wsum64(c);
+  a = wave_add(a); b = wave_add(b); c = wave_add(c);
   const uint32_t w = threadIdx.x >> 6;
   __syncthreads();
   if ((threadIdx.x & 63u) == 0) { sh[w] = a; sh[NW + w] = b; sh[2 * NW + w] = c; }

@@ -42,8 +42,7 @@ __device__ __forceinline__ void run_row_task(float* act, const RowTask& t, __hal
   if (t.flags & 1u) {
     float ss = 0.f;
     for (uint32_t i = tid; i < dim; i += 256u) { const float x = act[(uint64_t)t.src + i]; ss = fmaf(x, x, ss); }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    ss = wave_add(ss);
     if ((tid & 63u) == 0) sh[tid >> 6] = ss;
     __syncthreads();
     ss = (sh[0] + sh[1]) + (sh[2] + sh[3]);

@@ -280,8 +280,7 @@ k_topp(float* data, const uint32_t* __restrict__ ls, const uint32_t* __restrict_
   const float temp = fmaxf(temperature, 1e-6f);
   const float keep_p = fminf(fmaxf(top_p, 0.f), 1.f);
   float mx = lg[tid];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  mx = wave_max(mx);
   if (mx == SMP_NEG_INF) { if (tid < n) put(tid, 0.f); return; }
   if (tid < n) pr[tid] = lg[tid] == SMP_NEG_INF ? 0.f : expf((lg[tid] - mx) / temp);
   __syncthreads();
