@@ -18,7 +18,7 @@
 //
 // Tiled form: workgroup = NW waves, each with R tiles of 16 weight rows = 16 NW R weight rows x 16 MT activation
 // rows; one step = 128 weights of K (four blocks).
-// Ring form (more than 64 activation rows): eight waves of 64 weight rows over 64 or 128 activation rows, on 32x32x16
+// Ring form (more than 64 activation rows): eight waves of 64 weight rows over 64, 96 or 128 activation rows, on 32x32x16
 // instructions, weights, scales and activations straight to a ring of LDS stages.
 // Either over shares of K, which k_gemm_splitk_sum adds up; gemm_plan says which.
 // Few rows (2 .. 64): k_gemm_q4_rows, k_gemm_q4_f16_rows16.  The waves of a workgroup share R tiles of 16 weight rows and take
@@ -346,8 +346,9 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
 // ---- more than 64 activation rows ------------------------------------------------------------------------------------
 // Eight waves of 64 weight rows each, side by side, over 32 MA activation rows: a wave has 2 x MA results of 32 x 32.  A step
 // is 64 columns (two blocks); its packed weights (16 KB), their scales (2 KB) and both planes of the activations (8 KB per 32
-// rows) go straight to LDS, a ring of four stages (MA = 2) or three (MA = 4).  512 x 28672 x 4096: 317 -> 248 us = 485
-// TFLOP/s.  What bounds it is the vector work beside the matrix instructions (a
+// rows) go straight to LDS, a ring of four stages (MA = 2) or three (MA = 3, 4).  512 x 28672 x 4096: 317 -> 248 us = 485
+// TFLOP/s.  96 rows a workgroup give every CU one where 128 leave a third of them without (384 x 28672 x 4096, 168 workgroups and
+// 224: 216 us and 197, not in proportion: with all CUs at work the clock falls from 2.3 to 2.0 GHz, the products' power).  What bounds it is the vector work beside the matrix instructions (a
 // multiply-add per result and block, the unpacking): they share a wave's issue, so what counts is that no instruction of
 // either kind waits for another.  LDS reads without bank conflicts: 266 -> 246 us.
 // v_mfma_f32_32x32x16_f16: lane l supplies row l % 32, k = 8 (l / 32) .. + 7 of either operand and receives rows
@@ -365,7 +366,7 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
                float* __restrict__ part, const uint32_t* __restrict__ lc, const float* __restrict__ scale, GemmSegs segs) {
   constexpr uint32_t BM = 32u * MA, BN = 512u, RING_STAGE = RING_W + RING_S + MA * 8192u;
   constexpr int LOADS = 3 + MA, RING_ST = MA == 2 ? 4 : 3;      // loads of a wave and stage: 2 of weights, 1 of scales, MA of activations
-  static_assert(MA == 2 || MA == 4, "stages and schedule");
+  static_assert(MA >= 2 && MA <= 4, "stages and schedule");
   __shared__ __attribute__((aligned(16))) uint8_t ring[RING_ST * RING_STAGE];
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t r32 = lane & 31u, h = lane >> 5;
@@ -1317,8 +1318,10 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // 14336 (the plan it picks takes 0.2 % longer than the best one in the mean, 9 % at most; 12 % for 128 x 32000 x 2048, where the
 // tiled kernel over two shares, which it does not ask for, takes 60 us and one launch 67).  Tiled, by the tile it would take
 // (below): 128-column steps of 1.27 us while no CU has a second 64 x 64 tile and 0.72 more for each further one, 4.0 and 2.7
-// more for every two rounds of 64 x 128, 4.6 a round of 256 x 128.  Ring: 64-column steps of 1.7 (ma = 2) or 3.0 us, up to a
-// fifth more as the CUs fill; shares cost their second launch and a pass over the sums each.
+// more for every two rounds of 64 x 128, 4.6 a round of 256 x 128.  Ring: 64-column steps of 1.7 (ma = 2), 2.35 (3) or 3.0 us (4), up to a
+// quarter more as the CUs fill; shares cost their second launch and a pass over the sums each.  (us, conversion included, without
+// and with 96 rows a workgroup: 28672 x 4096 under 96 rows 88 and 76, 150 129 and 114, 192 129 and 118, 288 231 and 184, 384 241 and
+// 212; 4096 x 14336 288 116 and 105, 384 139 and 128; 6144 x 4096 480 90 and 83.)
 // The ring reads the scales of two blocks as one word and keeps a lane's place in the rows in 32 bits (in the matrix too: a Q4
 // map here has fewer than 2^32 elements): matrices that begin at an odd block stay on the tiled kernel, a narrow one from 128
 // rows on over 2 .. 4 shares (256 x 128 tile; 512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four).
@@ -1352,10 +1355,10 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   }
   if (ring == 2) best = 1e30;
   GemmPlan p = {0, 1};
-  for (int ma = 2; ma <= 4; ma += 2) {
+  for (int ma = 2; ma <= 4; ma++) {
     const uint64_t tiles = wgs(512, 32 * (uint64_t)ma);
     for (uint64_t sp = 1; sp <= most && (sp == 1 || (sp * 4 <= pairs && tiles * sp <= cu)); sp++) {
-      const double full = std::min(1.0, (double)(tiles * sp) / (double)cu), step = ma == 2 ? 1.7 + 0.35 * full : 3.0 + 0.8 * full;
+      const double full = std::min(1.0, (double)(tiles * sp) / (double)cu), step = ma == 2 ? 1.7 + 0.35 * full : ma == 3 ? 2.35 + 0.6 * full : 3.0 + 0.8 * full;
       const double us = (double)up(tiles * sp, cu) * ((double)up(pairs, sp) * step + 7.0) + (sp > 1 ? 9.0 + (double)(sp + 1) * pass : 0.0);
       if (us < best) { best = us; p = {ma, (uint32_t)sp}; }
     }
@@ -1481,7 +1484,7 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     const bool runs = tn % 8 != 0 && tm > 1 && shares <= 2 && run * 64 <= tiles * 9 && cdiv(run * shares * 8, g.n_cu) <= cdiv(tiles * shares, g.n_cu);
     const dim3 grid(runs ? run * 8 : tn, runs ? 1 : tm, shares);
 #define GR(T) k_gemm_q4_ring<T><<<grid, 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, (uint32_t)(b_host >> 5), c_val, by_val | (runs ? 4u : 0u), per, act, shares > 1 ? g_part_buf : nullptr, lc, g_scale_buf, sg)
-    if (plan.ma == 2) GR(2); else GR(4);
+    if (plan.ma == 2) GR(2); else if (plan.ma == 3) GR(3); else GR(4);
 #undef GR
     count_launch();
     if (shares > 1) add_up(shares);

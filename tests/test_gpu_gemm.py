@@ -558,6 +558,14 @@ def test_ring_at_ragged_ends(hip, monkeypatch, M, N, K, base, split):
     test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
 
 
+@pytest.mark.parametrize("M,N,K,base,split", [(288, 35837, 128, 0, "0"), (257, 35840, 384, 64, "0"), (96, 28001, 1024, 0, "1"), (341, 9000, 2048, 128, "1")])
+def test_ring_of_96_rows(hip, monkeypatch, M, N, K, base, split):
+    """Sizes at which 96 activation rows a workgroup fill the CUs in one round and 64 or 128 do not; ragged in both directions."""
+    monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
+    monkeypatch.setenv("ADAMAH_GEMM_SPLITK", split)
+    test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
+
+
 def test_ring_off_leaves_the_tiled_kernel_its_shares(hip, monkeypatch):
     """Either switch alone: without the ring a narrow matrix runs over shares (three launches), without shares in one (two)."""
     rng = np.random.default_rng(5)
