@@ -18,6 +18,11 @@ __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
+// the same, or nothing (the same for all lanes)
+__device__ __forceinline__ void load_to_lds_unless(uint32_t skip, const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_cmp_lg_u32 %3, 0\n\ts_cbranch_scc1 .Lskip%=\n\ts_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n.Lskip%=:"
+               ::"s"(lds), "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane((int)skip)) : "memory", "m0", "scc");
+}
 __device__ __forceinline__ void load4_to_lds(const void* base, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }

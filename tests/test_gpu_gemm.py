@@ -558,9 +558,11 @@ def test_ring_at_ragged_ends(hip, monkeypatch, M, N, K, base, split):
     test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
 
 
-@pytest.mark.parametrize("M,N,K,base,split", [(288, 35837, 128, 0, "0"), (257, 35840, 384, 64, "0"), (96, 28001, 1024, 0, "1"), (341, 9000, 2048, 128, "1")])
+@pytest.mark.parametrize("M,N,K,base,split", [(288, 35837, 128, 0, "0"), (257, 35840, 384, 64, "0"), (96, 28001, 1024, 0, "1"), (341, 9000, 2048, 128, "1"),
+                                                (777, 4100, 256, 256, "0"), (1000, 3201, 512, 512, "1"), (341, 4100, 3328, 0, "1")])
 def test_ring_of_96_rows(hip, monkeypatch, M, N, K, base, split):
-    """Sizes at which 96 activation rows a workgroup fill the CUs in one round and 64 or 128 do not; ragged in both directions."""
+    """Sizes at which 96 activation rows a workgroup fill the CUs in one round and 64 or 128 do not, ragged in both directions; scales of one
+    run of 256 columns and of several, shares that begin inside a run."""
     monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
     monkeypatch.setenv("ADAMAH_GEMM_SPLITK", split)
     test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
