@@ -354,9 +354,9 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
 // v_mfma_f32_32x32x16_f16: lane l supplies row l % 32, k = 8 (l / 32) .. + 7 of either operand and receives rows
 // 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32 -- here the columns are weight rows, so a block's scale is one number per
 // lane.  S16 (rows of whole runs of 256 columns that begin on 16 bytes of scales): the scales of four steps come in one 16-byte piece a row.
-// A step's own four bytes of every row each took a line from the L2, 40 % of the requests (512 x 28672 x 4096: 18.9 to 13.2 million; the
-// clock, which the chip's power sets, rises from 1.92 to 1.96 GHz).  4096 x 14336 under 341 rows 116 -> 110 us, 4096 x 4096 under 512 56.5
-// -> 55; 1877 tokens through the Llama 8B shape 79.9 -> 79.2 ms.
+// A step's own four bytes of every row each took a line from the L2, 40 % of the requests (7.6 of 18.9 million for 512 x 28672 x 4096; now
+// a quarter of that).  4096 x 14336 under 341 rows 116 -> 110 us, 4096 x 4096 under 512 56.5 -> 55; 1877 tokens through the Llama 8B
+// shape 79.9 -> 79.2 ms.
 // An instruction covers half a block; two permutes bring a block's words to the half of the wave that owns them.
 typedef float f16q_t __attribute__((ext_vector_type(16)));
 #define RING_W 16384u
