@@ -4,7 +4,8 @@
 //   one row      k_gemv_bf16: f is computed by every workgroup while it stages x in LDS (float32), weights stream
 //                through registers, float32 multiply-adds; store, add to the residual, gate / up pairs combined, or
 //                store + best row of the workgroup (arg-max)
-//   2..32 rows   k_linear_skinny: bf16 matrix instructions straight from memory, K split over the waves of a workgroup
+//   2..32 rows   bf16 matrix instructions straight from memory, K split over the waves of a workgroup: k_linear_few, a workgroup a
+//                CU with the tokens in its registers, where those hold them; k_linear_skinny for shorter and longer rows
 //   more rows    k_linear_tiled<BM, BN, ...>: bf16 matrix instructions over a ring of LDS tiles filled by direct-to-LDS loads
 //   float32 operand map: the same tiles over three bfloat16 pieces of each row (k_split_rows); short rows: k_linear_f32, the
 //                float32 matrix instruction over the widened weights
@@ -757,6 +758,141 @@ k_linear_skinny(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, floa
   }
 }
 
+// Four results of one token, units j0 .. j0 + 3 of a workgroup's own (below end): a unit is a matrix row, of an epi 2 product two of
+// them, gate / up or two of the tail.
+__device__ __forceinline__ void put_units(const LinSpec& s, float* act, uint32_t row, uint32_t j0, uint32_t end, f4_t v) {
+  float* d = act + s.out + (uint64_t)row * s.out_stride + j0;
+  if (s.biased) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) if (j0 + i < end) v[i] += act[s.bias + j0 + i];
+  }
+  if (s.epi == 1u) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] += j0 + i < end ? d[i] : 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) if (j0 + i < end) d[i] = v[i];
+}
+typedef uint32_t words_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint32_t pair_row(uint32_t j) { return (j >> 4) * 32u + (j & 15u); }
+__device__ __forceinline__ void put_units(const LinSpec& s, float* act, bf16_t* opnd, uint32_t row, uint32_t j0, uint32_t end, f4_t gt, f4_t up) {
+  const uint32_t head = s.n - s.tail;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint32_t r = pair_row(j0 + i);
+    if (j0 + i >= end || r >= s.n) continue;
+    if (r < head) { opnd[s.out_opnd + (uint64_t)row * s.out_opnd_stride + j0 + i] = (bf16_t)(silu_f(gt[i]) * up[i]); continue; }
+    float* d = act + s.tail_out + (uint64_t)row * s.tail_stride + (r - head);
+    d[0] = gt[i];
+    if (r + 16u < s.n) d[16] = up[i];
+  }
+}
+
+// Rows of 1025 .. 4096 columns.  Bound by the weights' way in.  One workgroup a CU, each an equal share of the units (the kernel above
+// put 28672 rows into 896 workgroups, of which three fit a CU: the last 128 ran alone), in passes of 16 matrix rows.  A wave's S steps
+// of K are the same in every pass, so its columns of the tokens stay in registers (they were read again for every 32 matrix rows:
+// half as many bytes as the weights at 16 tokens, as many at 32), and a step's weights are asked for as soon as its own of the pass
+// before (of two passes before where rows are short) have been used: 64 .. 128 KB of a CU in flight throughout, without a wait for
+// all of them.  A pass leaves its sums over K in LDS; no barrier before there is no room for more.  What remains is the tokens' way
+// in, 128 KB a CU for 16 of 4096 columns: 2 us at the rate of the L2s.
+// us, the kernel above and this one: 12 tokens, 28672 x 4096 (pairs) 54.3 and 41.5 (5.7 TB/s), 12576 x 4096 27.2 and 22, 32768 x 4096 58.2 and
+// 48.3, 10304 x 2048 14.4 and 10.3, 2048 x 2048 5.5 and 4.7, 14336 x 2560 (pairs) 18.9 and 16.9; 32 tokens, the same: 68 and 47, 34.3 and
+// 26.4, 71.5 and 54.4, 18.6 and 12.9, 7.7 and 6.9, 24.5 and 19.4.
+template <int MT, int S>
+__global__ void __launch_bounds__(512)
+k_linear_few(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, bf16_t* opnd, uint32_t kp, uint32_t n, uint32_t rows,
+             uint32_t units, uint32_t per, uint32_t pair, const LinSpec s) {
+  constexpr int NW = 8, D = S <= 4 ? 2 : 1, P = 16 / MT;
+  __shared__ f4_t red[P][MT][NW][64];
+  const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), c = lane & 15u, kg = lane >> 4;
+  const uint32_t begin = blockIdx.x * per, end = min(begin + per, units), passes = ((end - begin + 15u) >> 4) << pair;
+  // step u of this wave: columns 64 (wave + 8 u) ..; some waves' last lies beyond the row's end: they read their first again, and `keep` makes zeros of it
+  const bool over = 64u * (wave + NW * (S - 1)) >= kp;
+  const uint32_t last = over ? 64u * wave : 64u * (wave + NW * (S - 1)), keep = over ? 0u : ~0u;
+  const auto kept = [&](bf8_t v) { return __builtin_bit_cast(bf8_t, __builtin_bit_cast(words_t, v) & (words_t){keep, keep, keep, keep}); };
+  const auto column = [&](int u) { return u == S - 1 ? last : 64u * (wave + NW * (uint32_t)u); };
+  const auto row_of = [&](uint32_t p) {
+    const uint32_t j = min(begin + 16u * (p >> pair) + c, end - 1u);
+    return W + (uint64_t)min(pair ? pair_row(j) + 16u * (p & 1u) : j, n - 1u) * kp + kg * 8u;
+  };
+  bf8_t w[D][S][2], x[S][2][MT];
+  const auto ask = [&](const bf16_t* r, int d, int u) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) w[d][u][h] = *(const bf8_t*)(r + column(u) + 32 * h);
+  };
+  {
+    const bf16_t *r = row_of(0), *xr[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) xr[m] = X + (uint64_t)min(16u * m + c, rows - 1u) * kp + kg * 8u;
+#pragma unroll
+    for (int u = 0; u < S; u++) {
+      ask(r, 0, u);
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int m = 0; m < MT; m++) x[u][h][m] = *(const bf8_t*)(xr[m] + column(u) + 32 * h);
+    }
+    if (D == 2 && passes > 1u) {
+      r = row_of(1);
+#pragma unroll
+      for (int u = 0; u < S; u++) ask(r, D - 1, u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  uint32_t first = 0;
+  const auto sums = [&](uint32_t to) {      // passes first .. to - 1 lie in LDS
+    __syncthreads();
+    const uint32_t tasks = ((to - first) >> pair) * MT;
+    for (uint32_t t = wave; t < tasks; t += NW) {
+      const uint32_t m = t % MT, p = (t / MT) << pair, row = 16u * m + c, j0 = begin + 16u * ((first + p) >> pair) + 4u * kg;
+      const auto sum = [&](uint32_t q) {
+        f4_t v = red[q][m][0][lane];
+#pragma unroll
+        for (int i = 1; i < NW; i++) v += red[q][m][i][lane];
+        return v;
+      };
+      const f4_t a = sum(p), b = pair ? sum(p + 1u) : a;
+      if (row >= rows) continue;
+      if (pair) put_units(s, act, opnd, row, j0, end, a, b);
+      else put_units(s, act, row, j0, end, a);
+    }
+  };
+  const auto pass = [&](uint32_t p, auto place, auto more) {
+    constexpr int d = decltype(place)::value;
+    if (p - first == (uint32_t)P) { sums(p); __syncthreads(); first = p; }
+    const bf16_t* next = row_of(p + D);
+    f4_t acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++) acc[m] = (f4_t){0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < S; u++) {
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+          if (u == S - 1) { w[d][u][h] = kept(w[d][u][h]); x[u][h][m] = kept(x[u][h][m]); }
+          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[d][u][h], x[u][h][m], acc[m], 0, 0, 0);
+        }
+      if (more) ask(next, d, u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; m++) red[p - first][m][wave][lane] = acc[m];
+  };
+  typedef std::integral_constant<int, 0> A;
+  typedef std::integral_constant<int, D - 1> B;
+  uint32_t p = 0;
+  if (D == 2) {
+    for (; p + 3u < passes; p += 2u) { pass(p, A{}, std::true_type{}); pass(p + 1u, B{}, std::true_type{}); }
+    if (p + 2u < passes) { pass(p, A{}, std::true_type{}); pass(p + 1u, B{}, std::false_type{}); pass(p + 2u, A{}, std::false_type{}); }
+    else { pass(p, A{}, std::false_type{}); if (p + 1u < passes) pass(p + 1u, B{}, std::false_type{}); }
+  } else {
+    for (; p + 1u < passes; p++) pass(p, A{}, std::true_type{});
+    pass(p, A{}, std::false_type{});
+  }
+  sums(passes);
+}
+
 // ---- tiles --------------------------------------------------------------------------------------------------------
 // Shares of K (part): workgroup plane z takes columns z k_per .. and leaves raw sums, rows of np, for k_linear_sum.
 template <class T, int BM, int BN, int WM, int WN, int ST>
@@ -1007,6 +1143,26 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   if (rows > 32) return launch_tiles<bf16_t>(W, X, act, op, s, rows);
   // Workgroups of 16 matrix rows as long as no CU gets a second one (12 rows, 4096 x 4096: 9.6 us, of 32: 13.4; 7168 x
   // 2048: 9.2 to 10.0 and 8.2 to 8.9).
+  const uint32_t pair = s.epi == 2u, units = pair ? cdiv(s.n, 32) * 16u : s.n, per = cdiv(units, g.n_cu), grid = cdiv(units, per);
+  // Up to 1024 columns a launch is over before its registers are worth filling (8192 x 1024 under 16 rows: 5.7 us as it is, 9.7 with
+  // one step of four used); beyond 4096 the tokens do not fit them.  One pass of nearly all its 16 matrix rows on every CU has nothing
+  // to stream behind: 16 waves in two lots of loads do it as well or better (12 rows, 4096 x 4096: 9.75 and 10.1, of 32 rows 14.3 and
+  // 14.4; 13 matrix rows a CU, 3328 x 4096: 9.7 and 9.3, 14.4 and 13.6).
+  if (s.k_stride > 1024u && s.k_stride <= 4096u && (pair || per <= 14u || per > 16u || s.k_stride <= 2048u)) {
+    const auto go = [&](auto* one, auto* two) {
+      (rows <= 16 ? one : two)<<<grid, 512, 0, g.stream>>>(W, X, act, op, s.k_stride, s.n, rows, units, per, pair, s);
+    };
+    switch (cdiv(s.k_stride, 512)) {
+      case 3: go(k_linear_few<1, 3>, k_linear_few<2, 3>); break;
+      case 4: go(k_linear_few<1, 4>, k_linear_few<2, 4>); break;
+      case 5: go(k_linear_few<1, 5>, k_linear_few<2, 5>); break;
+      case 6: go(k_linear_few<1, 6>, k_linear_few<2, 6>); break;
+      case 7: go(k_linear_few<1, 7>, k_linear_few<2, 7>); break;
+      default: go(k_linear_few<1, 8>, k_linear_few<2, 8>); break;
+    }
+    count_launch();
+    return check_launch();
+  }
 #define LS(MT) do { if (s.epi != 2u && cdiv(s.n, 16) <= (uint32_t)g.n_cu) k_linear_skinny<MT, 1, 16><<<cdiv(s.n, 16), 1024, 0, g.stream>>>(W, X, act, op, s, rows); \
     else k_linear_skinny<MT, 2, 8><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows); } while (0)
   if (rows <= 16) LS(1); else LS(2);

@@ -123,6 +123,54 @@ def test_linear_tiles(hip, rows, n, k, biased, add):
     assert np.array_equal(got[:rows, n:], old[:rows, n:]) and np.array_equal(got[rows], old[rows])       # nothing beyond
 
 
+@pytest.mark.parametrize("rows,n,k,epi,tail", [
+    (2, 1, 1088, 0, 0), (16, 4095, 1536, 1, 0), (17, 4097, 2048, 0, 0), (32, 8195, 1600, 1, 0), (12, 12300, 2048, 0, 0), (3, 16390, 1088, 1, 0),
+    (31, 36901, 1088, 0, 0), (5, 70003, 1088, 1, 0), (16, 8200, 2560, 0, 0), (32, 300, 2624, 1, 0), (9, 4100, 3072, 0, 0), (20, 515, 3520, 1, 0),
+    (16, 8208, 4096, 0, 0), (29, 4099, 4032, 0, 0), (12, 32, 1088, 2, 0), (32, 8227, 2048, 2, 35), (2, 8257, 4096, 2, 1), (18, 16448, 1216, 2, 64),
+    (13, 34000, 1344, 2, 16), (7, 3601, 2112, 0, 0)])
+def test_products_of_few_rows(hip, rows, n, k, epi, tail):
+    """One pass of 16 matrix rows a workgroup up to more than LDS holds the sums of, rows of every count of steps, whole and ragged; an
+    infinite value of a token whose columns a wave reads twice."""
+    note(f"few rows {rows} n {n} k {k} epi {epi} tail {tail}")
+    rng = np.random.default_rng(n + k)
+    f64 = lambda b: (b.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    W = f32_to_bf16(rng.standard_normal((n, k), dtype=np.float32) / np.float32(np.sqrt(k)))
+    x = rng.standard_normal((rows, k), dtype=np.float32)
+    x[rows - 1, 5] = np.inf
+    xb = f32_to_bf16(x)
+    pair_w, st, op_at = (n - tail) // 2 if epi == 2 else 0, max(tail, 1) + 2 if epi == 2 else n + 3, (rows * k + 7) // 8 * 8
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, W.size)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, op_at + rows * (pair_w + 1) + 8)
+    hip.scatter_contiguous(OP, 0, xb.reshape(-1))
+    old = rng.standard_normal((rows + 1, st)).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    f32map(hip, WS, old.size + n, np.concatenate([old.reshape(-1), bias]))
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=k, opnd=0, ready=1, out=0, out_stride=st, epi=epi, out_opnd=op_at, out_opnd_stride=pair_w + 1,
+                        tail=tail, tail_out=0, tail_stride=st, bias=old.size, biased=int(epi == 0))
+    hip.linear_dev(WS, OP, WT, up(hip, spec.words()), 0, rows)
+    got = read(hip, WS, 0, old.size).reshape(rows + 1, st)
+    y = f64(xb[:-1]) @ f64(W).T
+    tol = k * 2.0 ** -24                          # exact products, float32 sums of k terms: relative to the terms' root sum of squares
+    held = n if epi < 2 else tail
+    assert np.array_equal(got[:, held:], old[:, held:]) and np.array_equal(got[rows], old[rows])             # nothing beyond
+    inf = np.sign(f64(W[:, 5])) * np.inf          # (a weight of 0 meets it: no number)
+    with np.errstate(invalid="ignore"):
+        inf[f64(W[:, 5]) == 0.0] = np.nan
+    if epi < 2:
+        want = y + (old[:rows - 1, :n] if epi else bias)
+        assert rel_l2(got[:rows - 1, :n], want) < tol and np.array_equal(got[rows - 1, :n], inf.astype(np.float32), equal_nan=True)
+        return
+    if tail:
+        assert rel_l2(got[:rows - 1, :tail], y[:, n - tail:]) < tol
+        assert np.array_equal(got[rows - 1, :tail], inf[n - tail:].astype(np.float32), equal_nan=True)
+    head = y[:, :n - tail].reshape(rows - 1, -1, 2, 16)
+    want = (head[:, :, 0] / (1.0 + np.exp(-head[:, :, 0])) * head[:, :, 1]).reshape(rows - 1, pair_w)
+    raw = hip.gather(OP, np.arange(op_at, op_at + rows * (pair_w + 1), dtype=np.uint32))
+    pairs = f64(raw.view(np.uint16)[:raw.size]).reshape(rows, -1)[:-1, :pair_w]
+    assert rel_l2(pairs, want) < 4 * tol + 2.0 ** -8
+
+
 @pytest.mark.parametrize("rows,k,groups,act,per_group", [
     (1, 2048, 1, 1, 0), (1, 8192, 32, 2, 1), (2, 8196, 1, 0, 0), (3, 4096, 64, 3, 1), (3, 16384, 16, 1, 0), (2, 16640, 1, 2, 0), (5, 768, 3, 3, 0),
     (5, 768, 1, 0, 1), (7, 256, 64, 1, 1), (4, 1200, 25, 2, 0), (530, 4096, 4, 1, 1), (520, 4352, 1, 3, 0), (515, 36, 0, 0, 0),
