@@ -311,6 +311,37 @@ def test_residual_add_stored_by_the_matmul(hip, M, K, N, in_place):
         assert rel_l2(fused[d0:d0 + M * N].reshape(M, N), y + hid) < TOL
 
 
+@pytest.mark.parametrize("twice", [False, True])
+@pytest.mark.parametrize("off,d_off", [(0, 0), (1, 0), (0, 2)])
+@pytest.mark.parametrize("M,N,K", [(70, 512, 14336), (130, 1024, 8192), (300, 1536, 6912), (487, 4096, 4096), (512, 6144, 4096), (257, 1025, 4096)])
+def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice):
+    """Two shares of K to more than eight, results and residual on 16 bytes and off them, the result added to itself: every sum is the
+    stored product plus the residual."""
+    note(f"sums of shares M={M} K={K} N={N} off={off} {d_off} twice={twice}")
+    rng = np.random.default_rng(M + N)
+    qt = quant.quantize_q4_0(rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05))
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    hid = rng.standard_normal((M, N), dtype=np.float32)
+    y0 = M * K + off
+    h0 = y0 + M * N + 8 - (y0 + M * N) % 4 + d_off
+    d0 = h0 + M * N
+    old = np.zeros(d0 + M * N + 4, np.float32)
+    old[:M * K], old[h0:h0 + M * N] = x.reshape(-1), hid.reshape(-1)
+    load_qtensor(hip, 1, qt)
+    f32map(hip, 0, old.size, old)
+    hy, hh, hd = up(hip, y0 + np.arange(M * N)), up(hip, h0 + np.arange(M * N)), up(hip, d0 + np.arange(M * N))
+    hip.batch_begin()
+    hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [0]), up(hip, [y0]), M, K, N, 1)
+    hip.map_op2_dev(0, A.OP_ADD, hy if twice else hh, hy, hd, M * N)
+    hip.batch_end()
+    got = read(hip, 0, 0, old.size)
+    y = got[y0:y0 + M * N]
+    assert rel_l2(y.reshape(M, N), x.astype(np.float64) @ qt.dequant().astype(np.float64).T) < TOL
+    assert np.array_equal(got[d0:d0 + M * N], y + (y if twice else hid.reshape(-1)))
+    got[y0:y0 + M * N] = got[d0:d0 + M * N] = 0
+    assert np.array_equal(got, old)                # nothing beside the results
+
+
 @pytest.mark.parametrize("op,M,K,N,in_place", [("swiglu", 16, 14336, 96, False), ("geglu", 5, 6912, 64, False), ("swiglu", 40, 256, 50, False),
                                                ("geglu", 16, 1024, 96, True)])
 def test_gated_activation_feeds_the_matmul_without_a_conversion_launch(hip, op, M, K, N, in_place):
