@@ -1086,7 +1086,13 @@ static int launch_tiles(const bf16_t* W, const bf16_t* X, float* act, T* op, con
   return check_launch();
 }
 
-static uint32_t gemv_grid(uint32_t n_tasks) { return std::min<uint32_t>(cdiv(n_tasks, 8), 2u * (uint32_t)g.n_cu); }
+// A few workgroups more than CUs would each read and norm x first, on a CU that another one keeps busy: where x is normed, some waves
+// take a second task instead, whose weights are asked for under the products of the first (2066 pairs of 2048, branched: 259 workgroups
+// 8.7 us, so 8.1; 4600 x 4096 behind a norm 12.0 and 11.4.  Without one 4200 x 2048 6.75 and 6.85).
+static uint32_t gemv_grid(const LinSpec& s, uint32_t n_tasks) {
+  const uint32_t grid = cdiv(n_tasks, 8), cu = (uint32_t)g.n_cu;
+  return (s.groups || s.branched) && grid > cu && grid <= cu + cu / 8u ? cu : std::min(grid, 2u * cu);
+}
 
 // tasks of two rows (pairs of gate / up ahead of the tail's)
 static uint32_t gemv_tasks(const LinSpec& s) { return s.epi == 2u ? (s.n - s.tail) / 2 + cdiv(s.tail, 2) : cdiv(s.n, 2); }
@@ -1097,7 +1103,7 @@ static void gemv_launch(Map* ma, Map* mw, const LinSpec& s, const uint32_t* row_
   const size_t lds = (size_t)s.k_stride * 4;
   const uint32_t mode = operand_mode(s, 512);
   const auto go = [&](auto* kernel, uint32_t n_tasks) {
-    const uint32_t grid = gemv_grid(n_tasks);
+    const uint32_t grid = gemv_grid(s, n_tasks);
     float* bv = (float*)g_best.p;
     if (lds > 60000) hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     kernel<<<grid, 512, lds, g.stream>>>(W, (float*)ma->buf, row_idx, s.k_stride, s.n, s.epi == 2u ? (s.n - s.tail) / 2 : 0u, s.src, s.k, mode, s.branch,
@@ -1232,7 +1238,7 @@ int adamah_linear_argmax_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_w
   for (uint32_t i = 0; i < rows; i++) if (dst[i] >= ma->n_elems) return ADAMAH_ERR_INVALID;
   float* act = (float*)ma->buf;
   if (rows == 1) {
-    const uint32_t grid = gemv_grid(gemv_tasks(*s));
+    const uint32_t grid = gemv_grid(*s, gemv_tasks(*s));
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
     gemv_launch<LEPI_ARGMAX>(ma, mw, *s, nullptr);
     k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0], nullptr);
@@ -1263,7 +1269,7 @@ int adamah_hip_linear_argmax_rows_dev(uint32_t map_act, uint32_t map_opnd, uint3
   const size_t row_bytes = (size_t)s->k_stride * 4;
   const uint32_t fit = (uint32_t)(((size_t)144 << 10) / row_bytes), nr = fit >= 8 && rows > 4 ? 8 : fit >= 4 && rows > 2 ? 4 : fit >= 2 && rows > 1 ? 2 : 1;
   if (rows == 1) {
-    const uint32_t grid = gemv_grid(gemv_tasks(*s));
+    const uint32_t grid = gemv_grid(*s, gemv_tasks(*s));
     if (int r = scratch_need(g_best, (size_t)grid * 8)) return r;
     gemv_launch<LEPI_ARGMAX>(ma, mw, *s, dev);
     k_best_pair<<<1, 256, 0, g.stream>>>((const float*)g_best.p, (const uint32_t*)g_best.p + grid, grid, act + dst[0], nullptr);
