@@ -367,7 +367,7 @@ static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* r
 // first weights behind it are asked for from the leading arguments alone (in registers when a wave starts; the spec is a
 // trip to memory, 0.5 us), sums of a norm stay in the vector unit.  us, weights cold, before and so: 2048 x 2048 4.9 and 4.1,
 // 2048 x 4096 7.2 and 6.2, behind a norm 9.2 and 7.7, 4096 x 4096 behind a norm 11.8 and 9.2, 10304 x 2048 behind a branch
-// 13.8 and 11.4, 4131 x 2048 (pairs, a tail) 10.4 and 8.7, 28672 x 4096 (pairs) 44.3 and 42, 4096 x 14336 24.7 and 23.6.
+// 13.8 and 11.4, 4131 x 2048 (pairs, a tail) 10.4 and 8.1, 28672 x 4096 (pairs) 44.3 and 42, 4096 x 14336 24.7 and 23.6.
 enum { LEPI_STORE = 0, LEPI_ADD = 1, LEPI_PAIR = 2, LEPI_ARGMAX = 3 };
 template <int EPI, int U, int R>
 __global__ void __launch_bounds__(512)
