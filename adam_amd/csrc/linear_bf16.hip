@@ -689,8 +689,7 @@ __device__ __forceinline__ void put_pair_or_tail(const LinSpec& s, float* act, T
 // ---- 2 .. 32 rows -------------------------------------------------------------------------------------------------
 // Bound by the weights' way in.  A workgroup owns 16 NB matrix rows; its NW waves take 64-column steps of K (a whole line of
 // a row) in turn, two of them in flight, and add up through LDS.  12 rows, 4096 x 14336 (117 MB): 57 us with half the CUs
-// at work, half lines and few loads in flight, 26.8 now (4.4 TB/s); 28672 x 4096 (235 MB): 60.4 and 52.5; 24 rows: 68 and
-// 37, 72 and 64.
+// at work, half lines and few loads in flight, 26.8 now (4.4 TB/s); 24 rows: 68 and 37.
 template <int MT, int NB, int NW>
 __global__ void __launch_bounds__(64 * NW)
 k_linear_skinny(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, bf16_t* opnd, const LinSpec s, uint32_t rows) {
@@ -1147,8 +1146,6 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   const bf16_t* X = op + s.opnd;
   if (!s.ready) operand_rows<bf16_t>(s, act, op + s.opnd, row_idx, rows);
   if (rows > 32) return launch_tiles<bf16_t>(W, X, act, op, s, rows);
-  // Workgroups of 16 matrix rows as long as no CU gets a second one (12 rows, 4096 x 4096: 9.6 us, of 32: 13.4; 7168 x
-  // 2048: 9.2 to 10.0 and 8.2 to 8.9).
   const uint32_t pair = s.epi == 2u, units = pair ? cdiv(s.n, 32) * 16u : s.n, per = cdiv(units, g.n_cu), grid = cdiv(units, per);
   // Up to 1024 columns a launch is over before its registers are worth filling (8192 x 1024 under 16 rows: 5.7 us as it is, 9.7 with
   // one step of four used); beyond 4096 the tokens do not fit them.  One pass of nearly all its 16 matrix rows on every CU has nothing
@@ -1169,6 +1166,7 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
     count_launch();
     return check_launch();
   }
+  // Workgroups of 16 matrix rows as long as no CU gets a second one (12 rows, 4096 x 4096: 9.6 us, of 32: 13.4)
 #define LS(MT) do { if (s.epi != 2u && cdiv(s.n, 16) <= (uint32_t)g.n_cu) k_linear_skinny<MT, 1, 16><<<cdiv(s.n, 16), 1024, 0, g.stream>>>(W, X, act, op, s, rows); \
     else k_linear_skinny<MT, 2, 8><<<cdiv(s.n, 32), 512, 0, g.stream>>>(W, X, act, op, s, rows); } while (0)
   if (rows <= 16) LS(1); else LS(2);
