@@ -311,9 +311,8 @@ def test_residual_add_stored_by_the_matmul(hip, M, K, N, in_place):
         assert rel_l2(fused[d0:d0 + M * N].reshape(M, N), y + hid) < TOL
 
 
-@pytest.mark.parametrize("twice", [False, True])
-@pytest.mark.parametrize("off,d_off", [(0, 0), (1, 0), (0, 2)])
-@pytest.mark.parametrize("M,N,K", [(70, 512, 14336), (130, 1024, 8192), (300, 1536, 6912), (487, 4096, 4096), (512, 6144, 4096), (257, 1025, 4096)])
+@pytest.mark.parametrize("M,N,K,off,d_off,twice", [(70, 512, 14336, 0, 0, False), (130, 1024, 8192, 0, 2, False), (300, 1536, 6912, 1, 0, False),
+                                                   (487, 4096, 4096, 0, 0, True), (512, 6144, 4096, 0, 0, False), (257, 1025, 4096, 0, 0, False)])
 def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice):
     """Two shares of K to more than eight, results and residual on 16 bytes and off them, the result added to itself: every sum is the
     stored product plus the residual."""
@@ -329,10 +328,11 @@ def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice):
     old[:M * K], old[h0:h0 + M * N] = x.reshape(-1), hid.reshape(-1)
     load_qtensor(hip, 1, qt)
     f32map(hip, 0, old.size, old)
-    hy, hh, hd = up(hip, y0 + np.arange(M * N)), up(hip, h0 + np.arange(M * N)), up(hip, d0 + np.arange(M * N))
+    zero, hy, hd = up(hip, [0]), up(hip, y0 + np.arange(M * N)), up(hip, d0 + np.arange(M * N))
+    hh = hy if twice else up(hip, h0 + np.arange(M * N))
     hip.batch_begin()
-    hip.map_matmul_t_xq4_dev(0, 1, up(hip, [0]), up(hip, [0]), up(hip, [y0]), M, K, N, 1)
-    hip.map_op2_dev(0, A.OP_ADD, hy if twice else hh, hy, hd, M * N)
+    hip.map_matmul_t_xq4_dev(0, 1, zero, zero, hy, M, K, N, 1)         # (the result begins at the first of its places)
+    hip.map_op2_dev(0, A.OP_ADD, hh, hy, hd, M * N)
     hip.batch_end()
     got = read(hip, 0, 0, old.size)
     y = got[y0:y0 + M * N]
