@@ -13,9 +13,9 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X and the built libadamah_hip.so")
 
 
-@pytest.fixture(scope="session")
+@pytest.fixture(scope="module")
 def hip():
-    """One library context for the whole session (the library keeps one global context)."""
+    """A library context a file (the library keeps one at a time): its table of 65536 handles then holds a file's, not the whole suite's."""
     from adam_amd import adamah
     g = adamah.init()
     yield g
