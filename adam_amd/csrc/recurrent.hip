@@ -477,11 +477,12 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 // A serial chain, so what counts is a chunk's latency.  Four waves share the state rows (NT tiles of 16 each); a tile's
 // accumulator holds rows 4 g + i of lane group g, which is also how instruction i wants its right operand when the left one is
 // read as four consecutive columns per lane.  On their chain are only the products that the state needs (delta: W S, its sum
-// through LDS, K u); Q S and a quarter of B u, the wave's share of the outputs, go out while that sum is on its way.  A fifth
-// wave adds up the shares and stores them, a chunk behind: loads and stores share a counter, and a wave that does both waits
-// for its stores.  2048 tokens in 32 heads of 128: outputs by the first of four waves, ahead of its part of the state, 127 us warm
-// (148 in a first pass), retention 93 (110); so 105 (115) and 76 (91).  Of the 115, with parts taken out: 106 without any output, 91
-// without loads either: what is left is 25 instructions of 32 clocks, an exchange through LDS and its barrier a chunk.
+// through LDS, K u); Q S goes out while that sum is on its way.  A fifth wave adds up the four shares of Q S, adds B u from what they
+// leave in LDS and stores, a chunk behind: loads and stores share a counter, and a wave that does both waits for its stores.
+// 2048 tokens in 32 heads of 128: outputs by the first of four waves, ahead of its part of the state, 136 us, retention 97; so 114 and 86.
+// One product behind the other by wave, the waves' parts as (0 + 1) + (2 + 3), B u behind that sum in order: a router behind these sums
+// turns another order into another choice of experts (with two sums a wave and a quarter of B u in each share 111 and 79 us, and 3e-2
+// in a mixture's logits).
 // FEW: one or two chunks, whose operands are not asked for ahead, so that a compute unit has three workgroups instead of two (16
 // sequences of 12 tokens 26.5 us, 48.5 with the other form, 38.6 before).
 struct ScanArgs {
@@ -512,6 +513,7 @@ template <bool DELTA, int NT, bool FEW>
 __global__ void __launch_bounds__(SCAN_T)
 k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, float* state) {
   __shared__ f4_t p1[2][4][64], p2[2][4][64];                // [chunk & 1][wave][lane]
+  __shared__ float pb[2][4][64], pu[2][4][64];               // B and u, a quarter of the four a lane has by each wave
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, D = a.dim, V = a.vdim, v = v0 + c;
   const uint32_t bs = chunk_floats(a.cd.Dp, a.cd.Vp), n = a.cd.n_chunks;
@@ -523,7 +525,10 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
     for (uint32_t ci = 0; ci <= n; ci++) {
       __syncthreads();
       if (ci == 0u) continue;
-      const f4_t o = sum4(p2[(ci - 1u) & 1u]);
+      const uint32_t x = (ci - 1u) & 1u;
+      f4_t o = sum4(p2[x]);
+#pragma unroll
+      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(pb[x][i][lane], pu[x][i][lane], o, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const uint32_t r = (ci - 1u) * CH + 4u * kg + i;
@@ -549,13 +554,14 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
     const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, lane, v0); __builtin_amdgcn_sched_barrier(0); };
     const auto chunk = [&](const ChunkOps<NT>& cur, uint32_t x) {
       f4_t u = cur.u;
-      if (DELTA) {                                           // (two sums: an instruction waits for the one that it adds to)
-        f4_t s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+      f4_t s = {0, 0, 0, 0};
+      if (DELTA) {
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
-          for (int i = 0; i < 4; i++) s[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], s[i & 1], 0, 0, 0);
-        p1[x][wave][lane] = s[0] + s[1];
+          for (int i = 0; i < 4; i++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], s, 0, 0, 0);
+        p1[x][wave][lane] = s;
+        s = (f4_t){0, 0, 0, 0};
       }
       __syncthreads();
       f4_t r[4];
@@ -563,11 +569,10 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
 #pragma unroll
         for (int w = 0; w < 4; w++) r[w] = p1[x][w][lane];
       __builtin_amdgcn_sched_barrier(0);                     // Q S behind them, not ahead of the barrier
-      f4_t s[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
       for (int j = 0; j < NT; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) s[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], s[i & 1], 0, 0, 0);
+        for (int i = 0; i < 4; i++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], s, 0, 0, 0);
       if (DELTA) u -= (r[0] + r[1]) + (r[2] + r[3]);
 #pragma unroll
       for (int j = 0; j < NT; j++) st[j] *= cur.gl[j];
@@ -575,8 +580,9 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
       for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < NT; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][i], u[i], st[j], 0, 0, 0);
-      s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b, wave & 2u ? (wave & 1u ? u[3] : u[2]) : (wave & 1u ? u[1] : u[0]), s[0], 0, 0, 0);
-      p2[x][wave][lane] = s[0] + s[1];
+      p2[x][wave][lane] = s;
+      pb[x][wave][lane] = cur.b;
+      pu[x][wave][lane] = wave & 2u ? (wave & 1u ? u[3] : u[2]) : (wave & 1u ? u[1] : u[0]);
     };
     ChunkOps<NT> o0;
     ask(o0, 0);

@@ -159,12 +159,14 @@ k_space_prep(const SSpec s, const float* __restrict__ act, const float* __restri
 }
 
 // Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
-// is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.  A wave's
-// share of the outputs is its rows' part of C S and a quarter of the chunk's own part; a fifth wave adds up the shares and
-// stores them, a chunk behind: loads and stores share a counter, and a wave that does both waits for its stores (2048 tokens in
-// 64 heads of 64 by 128, the waves taking turns with the outputs 80.7 us, so 67).  FEW: one or two chunks, no operands ahead.
+// is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.  Each leaves
+// its rows' part of C S in LDS and its quarter of what the chunk's own part needs; a fifth wave adds up, multiplies and stores, a
+// chunk behind: loads and stores share a counter, and a wave that does both waits for its stores (2048 tokens in
+// 64 heads of 64 by 128, the waves taking turns with the outputs 104 us, so 85).  The order of the sums is that of the other walks (the
+// chunk's own part behind the sum over the waves, in order), and C B times its decay is rounded before the skip is added.
+// FEW: one or two chunks, no operands ahead.
 #define SCAN_T 320u          // four waves of state rows and the one of the outputs
-template <int NT> struct SpaceOps { f4_t c[NT], b[NT], e, g, u; float cb, m, last; };
+template <int NT> struct SpaceOps { f4_t c[NT], b[NT], g, u; float cb, m, e, last; };
 template <int NT>
 __device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const float* hb, const SpaceDims& sd, uint32_t wave, uint32_t lane,
                                          uint32_t v0) {
@@ -175,11 +177,11 @@ __device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const
     o.c[j] = *(const f4_t*)(gb + at);
     o.b[j] = *(const f4_t*)(pB + at);
   }
-  o.e = *(const f4_t*)(pE + (lane >> 4) * 4u);
   o.g = *(const f4_t*)(pG + (lane >> 4) * 4u);
   o.u = *(const f4_t*)(hb + v0 * 16u + lane * 4u);
   o.cb = pD[lane * 4u + wave];
   o.m = pM[lane * 4u + wave];
+  o.e = pE[(lane >> 4) * 4u + wave];
   o.last = pE[15];
 }
 
@@ -187,6 +189,7 @@ template <int NT, bool FEW>
 __global__ void __launch_bounds__(SCAN_T)
 k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float* state, SpaceDims sd, uint32_t m, uint32_t seq0, uint32_t pos) {
   __shared__ f4_t pb[2][4][64];                              // [chunk & 1][wave][lane]
+  __shared__ float pc[2][3][4][64];                          // C B and skip, x, decay: a quarter of the four a lane has by each wave
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, N = s.state, V = s.vdim, v = v0 + c, rep = s.heads / s.groups, grp = h / rep;
   const uint32_t gs = group_floats(sd), hs = head_floats(sd), n = sd.n_chunks;
@@ -196,7 +199,10 @@ k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float
     for (uint32_t ci = 0; ci < n; ci++) {
       __syncthreads();
       const f4_t (*p)[64] = pb[ci & 1u];
-      const f4_t o = (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]);
+      const float (*q)[4][64] = pc[ci & 1u];
+      f4_t o = ((p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane])) * (f4_t){q[2][0][lane], q[2][1][lane], q[2][2][lane], q[2][3][lane]};
+#pragma unroll
+      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q[0][i][lane], q[1][i][lane], o, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const uint32_t r = ci * CH + 4u * kg + i;
@@ -229,19 +235,21 @@ k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float
       __builtin_amdgcn_sched_barrier(0);
     };
     const auto chunk = [&](const SpaceOps<NT>& cur, uint32_t x) {
-      f4_t p[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+      f4_t p = {0, 0, 0, 0};
 #pragma unroll
       for (int j = 0; j < NT; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) p[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.c[j][i], st[j][i], p[i & 1], 0, 0, 0);
+        for (int i = 0; i < 4; i++) p = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.c[j][i], st[j][i], p, 0, 0, 0);
 #pragma unroll
       for (int j = 0; j < NT; j++) st[j] *= cur.last;
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < NT; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[j][i], cur.g[i] * cur.u[i], st[j], 0, 0, 0);
-      const float u = wave & 2u ? (wave & 1u ? cur.u[3] : cur.u[2]) : (wave & 1u ? cur.u[1] : cur.u[0]);
-      pb[x][wave][lane] = __builtin_amdgcn_mfma_f32_16x16x4f32(fmaf(cur.cb, cur.m, skip), u, (p[0] + p[1]) * cur.e, 0, 0, 0);
+      pb[x][wave][lane] = p;
+      pc[x][0][wave][lane] = cur.cb * cur.m + skip;
+      pc[x][1][wave][lane] = wave & 2u ? (wave & 1u ? cur.u[3] : cur.u[2]) : (wave & 1u ? cur.u[1] : cur.u[0]);
+      pc[x][2][wave][lane] = cur.e;
       __syncthreads();
     };
     SpaceOps<NT> o0;

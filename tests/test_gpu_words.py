@@ -1,0 +1,116 @@
+"""Results that keep their words.  Ahead of a router a sum in another order is another choice of experts: 1e-6 in one layer's output moved
+the logits of a mixture's prompt by 3e-2.  What these kernels add up in which order is therefore part of what they promise."""
+import zlib
+
+import numpy as np
+import pytest
+
+from adam_amd import adamah as A
+from adam_amd.safetensors_file import f32_to_bf16
+from gpu_util import note, up, f32map, read
+
+pytestmark = pytest.mark.gpu
+
+WS, OP, WT, ST = 0, 2, 1, 3
+
+
+def places(first, **sizes):
+    """Offsets of regions one behind the other, each on four floats; the last entry is the end."""
+    at, pos = {}, first
+    for name, n in sizes.items():
+        at[name] = pos
+        pos += (n + 3) // 4 * 4
+    return at, pos
+
+
+# ---- walks over the chunks ---------------------------------------------------------------------------------------------
+def walk(hip, kind, H, G, D, V, seqs, rows):
+    """CRC of the outputs and of the states behind a portion of `rows` tokens of each sequence, from a state that is not empty."""
+    rng = np.random.default_rng(H * 1000 + D + rows)
+    n, taps = seqs * rows, 4
+    if kind == "delta":
+        ch = 2 * G * D + H * V
+        xs, state, rank = ch + H + 2 * 16, H * D * V + taps * ch, 16
+        at, end = places(4, x=n * xs, a=n * H * D, g=n * H * V, o=n * H * V, conv=ch * taps, A=H, dt=H * D)
+        hip.map_create_typed(WT, A.DTYPE_BF16, 1, (H * D + H * V) * 64)
+        W = np.zeros((H * D + H * V, 64), np.float32)
+        W[:, :rank] = rng.standard_normal((H * D + H * V, rank)) / 4
+        hip.scatter_contiguous(WT, 0, f32_to_bf16(W).reshape(-1))
+        hip.map_create_typed(OP, A.DTYPE_BF16, 1, 2 * n * 64)
+    elif kind == "retention":
+        xs, state = H * (2 * D + V), H * D * V
+        at, end = places(4, x=n * xs, o=n * H * V, decay=H)
+    else:
+        ch = H * V + 2 * G * D
+        xs, state = H * V + ch + H, H * D * V + taps * ch
+        at, end = places(4, x=n * xs, o=n * H * V, conv=ch * taps, b=ch, dt=H, A=H, D=H)
+    hip.set_dtype(A.DTYPE_F32)
+    put = lambda m, off, v: hip.scatter_contiguous(m, off, np.ascontiguousarray(v, np.float32).reshape(-1))
+    hip.map_create(WS, 1, end + 4)
+    hip.map_create(ST, 1, seqs * state)
+    put(WS, at["x"], rng.standard_normal(n * xs, dtype=np.float32))
+    put(ST, 0, rng.standard_normal(seqs * state, dtype=np.float32))
+    if "conv" in at:
+        put(WS, at["conv"], rng.standard_normal(ch * taps, dtype=np.float32) * np.float32(0.7))
+        put(WS, at["A"], np.linspace(-3.0, 0.5, H))
+        put(WS, at["dt"], rng.standard_normal(H * D if kind == "delta" else H, dtype=np.float32))
+    if kind == "delta":
+        low = lambda w, m, col, out: up(hip, A.LinearSpec(w=w, n=m, k=rank, k_stride=64, src=at["x"] + ch + H + col, src_stride=xs, opnd=0,
+                                                          out=at[out], out_stride=m).words())
+        dec, gate, c = low(0, H * D, 0, "a"), low(H * D * 64, H * V, rank, "g"), at["conv"]
+        spec = A.DeltaSpec(heads=H, kv_heads=G, dim=D, vdim=V, taps=taps, x=at["x"], x_stride=xs, x_b=ch, cq=c, ck=c + G * D * taps,
+                           cv=c + 2 * G * D * taps, a_log=at["A"], dt_bias=at["dt"], out=at["o"], out_stride=H * V, state_map=ST, s_off=0,
+                           conv_off=H * D * V, seq_stride=state)
+        hip.delta_rule_seqs_dev(WS, OP, WT, up(hip, spec.words()), dec, gate, seqs, rows, 0, 9)
+    elif kind == "retention":
+        put(WS, at["decay"], 1.0 - 2.0 ** -np.linspace(3, 9, H))
+        spec = A.RetentionSpec(heads=H, dim=D, vdim=V, rot_dims=0, freq=0, decay=at["decay"], x=at["x"], x_stride=xs, x_q=0, x_k=H * D,
+                               x_v=2 * H * D, out=at["o"], out_stride=H * V, state_map=ST, s_off=0, seq_stride=state)
+        hip.retention_seqs_dev(WS, up(hip, spec.words()), seqs, rows, 0, 9)
+    else:
+        put(WS, at["b"], rng.standard_normal(ch, dtype=np.float32))
+        put(WS, at["D"], rng.standard_normal(H, dtype=np.float32))
+        spec = A.StateSpaceSpec(heads=H, groups=G, state=D, vdim=V, taps=taps, x=at["x"], x_stride=xs, x_c=H * V, x_dt=H * V + ch, conv=at["conv"],
+                                conv_b=at["b"], dt_bias=at["dt"], a_log=at["A"], skip=at["D"], out=at["o"], out_stride=H * V, state_map=ST,
+                                s_off=0, conv_off=H * D * V, seq_stride=state)
+        hip.state_space_dev(WS, up(hip, spec.words()), seqs, rows, 0, 9)
+    return [f"{zlib.crc32(read(hip, m, off, size).tobytes()):08x}" for m, off, size in ((WS, at["o"], n * H * V), (ST, 0, seqs * state))]
+
+
+# Recorded with this library's walks of four waves (W S and Q S one product behind the other by wave, the waves' parts added as
+# (0 + 1) + (2 + 3), the chunk's own products behind that sum, in order) and ROCm 7.2's expf and exp2f.
+WALKS = {
+    ("delta", 2, 1, 24, 20, 1, 7): "98665651 5837517d",
+    ("delta", 3, 3, 100, 33, 2, 77): "7b2191fd f986b388",
+    ("delta", 2, 2, 128, 16, 1, 170): "76175282 56bba8ef",
+    ("delta", 4, 2, 180, 40, 1, 65): "a5a30d12 b19d4695",
+    ("delta", 1, 1, 256, 64, 1, 50): "387a19e7 42e9a6b8",
+    ("delta", 16, 16, 64, 64, 5, 40): "493b53b8 b70306d0",
+    ("delta", 16, 8, 64, 64, 9, 150): "dbd6aaa7 f7dfe3cb",
+    ("delta", 16, 16, 128, 100, 3, 150): "049324e3 55f86e0d",
+    ("delta", 20, 20, 192, 100, 2, 90): "83ab5318 3183c87b",
+    ("delta", 20, 20, 256, 100, 2, 90): "202dd06b ffd35d1a",
+    ("retention", 2, 0, 24, 20, 1, 7): "0fb25b32 c4b37fec",
+    ("retention", 3, 0, 100, 33, 2, 77): "aea11587 7cbdea86",
+    ("retention", 2, 0, 180, 40, 1, 65): "5fe31224 6db0836f",
+    ("retention", 1, 0, 256, 64, 1, 50): "ff24d1bc 2825e1d2",
+    ("retention", 16, 0, 64, 64, 9, 150): "2a6fe897 cd358e76",
+    ("retention", 16, 0, 128, 100, 5, 150): "8367e4e7 6f540275",
+    ("retention", 20, 0, 192, 100, 2, 90): "cc94d0f8 bd48135c",
+    ("retention", 20, 0, 250, 100, 2, 90): "175f578f d42d027b",
+    ("space", 2, 1, 24, 20, 1, 7): "e1e179c3 23146a8a",
+    ("space", 4, 2, 100, 33, 1, 77): "b600b15f 33b552db",
+    ("space", 4, 4, 180, 40, 1, 65): "6e7f7d9b 4d4ec6db",
+    ("space", 2, 1, 256, 64, 1, 50): "a40188e0 b260f797",
+    ("space", 130, 10, 64, 100, 1, 150): "a9b6b790 e153d87c",
+    ("space", 130, 10, 128, 100, 1, 150): "46180f9e 57ce785f",
+    ("space", 64, 8, 192, 100, 1, 90): "db1be02e 968e6ca1",
+    ("space", 64, 8, 250, 100, 1, 90): "a74b3f51 e9cf6a5c",
+}
+
+
+@pytest.mark.parametrize("case", WALKS, ids=lambda c: "-".join(map(str, c)))
+def test_walk_keeps_its_words(hip, case):
+    """One chunk to ten, one head to more workgroups than two a compute unit, every tile count, ragged in all directions."""
+    note(f"words of a walk {case}")
+    assert walk(hip, *case) == WALKS[case].split()
