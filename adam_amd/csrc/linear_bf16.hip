@@ -81,12 +81,10 @@ __device__ __forceinline__ void group_inverse(uint32_t k, uint32_t groups, float
 // floats.  WIDE: for rows of several floats a thread; without it the code is short and needs fewer registers, which is what
 // counts where a thread has one (2048 rows of 64: 4.6 us, with it 5.4).  path: operand_path of the spec.  ahead(): called once,
 // behind the row's first loads -- loads arrive in order, and what is asked for there (the first weights) must not hold the row up.
-enum { ROW_ANY = 0, ROW_NORM = 1, ROW_BRANCH = 2, ROW_PLAIN = 3 };      // anything; four elements a load
+enum { ROW_ANY = 0, ROW_NORM = 1, ROW_BRANCH = 2, ROW_PLAIN = 3 };      // NORM, PLAIN: four elements a load; BRANCH: one
 static uint32_t operand_path(const LinSpec& s, uint32_t nt) {
+  if (s.branched) return s.k <= 8u * nt ? ROW_BRANCH : ROW_ANY;
   if (((s.src | s.src_stride | s.k | (s.kept ? s.keep | s.keep_stride : 0u)) & 3u) != 0u) return ROW_ANY;
-  if (s.branched)
-    return s.k <= 8u * nt && ((s.branch | s.branch_stride | s.branch_wt | (s.wt_len ? s.wt : 0u) | (s.branched == 2u ? s.res_out | s.res_stride : 0u)) & 3u) == 0u
-               ? ROW_BRANCH : ROW_ANY;
   if (!s.groups) return ROW_PLAIN;
   const uint32_t gl = s.k / s.groups >> 2;                   // lanes (of four elements) a group has
   return s.k <= 16u * nt && (!s.gate_act || ((s.gate | s.gate_stride) & 3u) == 0u) && (!s.wt_len || ((s.wt | s.wt_len) & 3u) == 0u) &&
@@ -116,56 +114,51 @@ __device__ __forceinline__ void operand_row(const RowArgs& r, const LinSpec& s, 
   const auto gate_act = [&] { return MODE_GATED(mode) ? s.gate_act : 0u; };
   const auto weight = [&] { return act + (MODE_BRANCHED(mode) ? s.wt : r.at); };
   if (WIDE && path == ROW_BRANCH) {
-    // x + the branch's row behind a norm of its own, twice four elements a thread, everything asked for at once (past the end: the
-    // last four again, whose squares count for nothing)
-    constexpr int R = 2;
-    const uint32_t n4 = r.k >> 2;
+    // x + the branch's row behind a norm of its own, eight elements a thread, everything asked for at once (past the end: the
+    // last one again, whose square counts for nothing)
+    constexpr int R = 8;
     const float *b = act + r.branch + (uint64_t)r.row * r.branch_stride, *bw = act + r.at;
-    f4_t xv[R], bv[R], wv[R], nv[R];
+    float xv[R], bv[R], wv[R], nv[R];
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const uint32_t at = min(tid + (uint32_t)j * NT, n4 - 1u) * 4u;
-      xv[j] = *(const f4_t*)(x + at); bv[j] = *(const f4_t*)(b + at); wv[j] = *(const f4_t*)(bw + at);
+      if ((uint32_t)j * NT >= r.k) break;
+      const uint32_t i = min(tid + (uint32_t)j * NT, r.k - 1u);
+      xv[j] = x[i]; bv[j] = b[i]; wv[j] = bw[i];
     }
     ahead();
     if (MODE_WT(mode)) {
       const float* wt = weight();
 #pragma unroll
-      for (int j = 0; j < R; j++) nv[j] = *(const f4_t*)(wt + min(tid + (uint32_t)j * NT, n4 - 1u) * 4u);
+      for (int j = 0; j < R; j++) {
+        if ((uint32_t)j * NT >= r.k) break;
+        nv[j] = wt[min(tid + (uint32_t)j * NT, r.k - 1u)];
+      }
     }
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const bool on = tid + (uint32_t)j * NT < n4;
-#pragma unroll
-      for (int e = 0; e < 4; e++) { bv[j][e] = on ? bv[j][e] : 0.f; ss = fmaf(bv[j][e], bv[j][e], ss); }
+      if ((uint32_t)j * NT >= r.k) break;
+      ss = tid + (uint32_t)j * NT < r.k ? fmaf(bv[j], bv[j], ss) : ss;
     }
     const float ib = 1.0f / sqrtf(block_sum<NT / 64>(ss, part) / (float)r.k + s.eps);
     ss = 0.f;
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const bool on = tid + (uint32_t)j * NT < n4;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        xv[j][e] = fmaf(bv[j][e] * ib, s.wt_add + wv[j][e], xv[j][e]);
-        const float v = on ? xv[j][e] : 0.f;
-        ss = fmaf(v, v, ss);
-      }
+      if ((uint32_t)j * NT >= r.k) break;
+      xv[j] = fmaf(bv[j] * ib, s.wt_add + wv[j], xv[j]);
+      ss = tid + (uint32_t)j * NT < r.k ? fmaf(xv[j], xv[j], ss) : ss;
     }
     const float ix = 1.0f / sqrtf(block_sum<NT / 64>(ss, part + NT / 64) / (float)r.k + s.eps);
+    const bool keeps = kept();
 #pragma unroll
     for (int j = 0; j < R; j++) {
-      const uint32_t c = tid + (uint32_t)j * NT;
-      if (c >= n4) break;
-      if (first && MODE_BRANCHED(mode) == 2u) *(f4_t*)(act + s.res_out + (uint64_t)r.row * r.res_stride + 4u * c) = xv[j];
-      f4_t v = xv[j];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        v[e] *= ix;
-        if (MODE_WT(mode)) v[e] *= s.wt_add + nv[j][e];
-      }
-      if (kept()) *(f4_t*)(keep() + 4u * c) = v;
-      put4(c, v);
+      const uint32_t i = tid + (uint32_t)j * NT;
+      if (i >= r.k) break;
+      if (first && MODE_BRANCHED(mode) == 2u) act[s.res_out + (uint64_t)r.row * r.res_stride + i] = xv[j];
+      float v = xv[j] * ix;
+      if (MODE_WT(mode)) v *= s.wt_add + nv[j];
+      if (keeps) keep()[i] = v;
+      put(i, v);
     }
   } else if (MODE_BRANCHED(mode)) {
     ahead();
@@ -260,8 +253,13 @@ __device__ __forceinline__ void operand_row(const RowArgs& r, const LinSpec& s, 
       for (int j = 0; j < R; j++) {
         if ((uint32_t)j * NT >= n4) break;                   // (all lanes or none: they add up together)
         if (j > 0 && MODE_GROUPS(mode) == 1u) { scale[j] = scale[0]; continue; }
-        const uint32_t lane = tid & 63u, b0 = ((uint32_t)j * NW + wave) / nb * nb;         // (a partial sum a lane)
-        scale[j] = 1.0f / sqrtf(wave_add(lane < nb ? part[min(b0 + lane, (uint32_t)(R * NW) - 1u)] : 0.f) / n + s.eps);
+        // (read a partial sum a lane, added up one behind the other)
+        const uint32_t lane = tid & 63u, b0 = ((uint32_t)j * NW + wave) / nb * nb;
+        const uint32_t own = __float_as_uint(part[min(b0 + min(lane, nb - 1u), (uint32_t)(R * NW) - 1u)]);
+        float t = 0.f;
+#pragma unroll 8
+        for (uint32_t b = 0; b < nb; b++) t += __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)own, (int)b));
+        scale[j] = 1.0f / sqrtf(t / n + s.eps);
       }
     }
 #pragma unroll
@@ -365,9 +363,11 @@ static void operand_rows(const LinSpec& s, float* act, T* dst, const uint32_t* r
 // a lane's two 16-byte reads are conflict free.
 // What bounds it is the weights' way in and, for the smaller matrices, what a workgroup does before it can use them: x and the
 // first weights behind it are asked for from the leading arguments alone (in registers when a wave starts; the spec is a
-// trip to memory, 0.5 us), sums of a norm stay in the vector unit.  us, weights cold, before and so: 2048 x 2048 4.9 and 4.1,
-// 2048 x 4096 7.2 and 6.2, behind a norm 9.2 and 7.7, 4096 x 4096 behind a norm 11.8 and 9.2, 10304 x 2048 behind a branch
-// 13.8 and 11.4, 4131 x 2048 (pairs, a tail) 10.4 and 8.1, 28672 x 4096 (pairs) 44.3 and 42, 4096 x 14336 24.7 and 23.6.
+// trip to memory, 0.5 us), sums of a norm stay in the vector unit.  us, weights cold, before and so: 2048 x 2048 5.0 and 4.1,
+// 2048 x 4096 7.3 and 6.3, behind a norm 9.3 and 7.8, 4096 x 4096 behind a norm 11.8 and 9.4, 10304 x 2048 behind a branch
+// 13.8 and 12.0, 4131 x 2048 (pairs, a tail) 10.4 and 8.0, 28672 x 4096 (pairs) 44.9 and 43.2, 4096 x 14336 25.4 and 24.0.
+// A norm's sums keep the order that they had before (partial sums of the waves in turn; a branched row's columns by thread): four
+// neighbours a load and the partial sums in pairs would take 0.2 us less, and behind a router that is another choice of experts.
 enum { LEPI_STORE = 0, LEPI_ADD = 1, LEPI_PAIR = 2, LEPI_ARGMAX = 3 };
 template <int EPI, int U, int R>
 __global__ void __launch_bounds__(512)

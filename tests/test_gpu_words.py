@@ -114,3 +114,91 @@ def test_walk_keeps_its_words(hip, case):
     """One chunk to ten, one head to more workgroups than two a compute unit, every tile count, ragged in all directions."""
     note(f"words of a walk {case}")
     assert walk(hip, *case) == WALKS[case].split()
+
+
+# ---- norms of operand rows -------------------------------------------------------------------------------------------------
+fma = lambda a, b, c: (np.float64(1) * a * b + c).astype(np.float32)
+
+
+def wave_sum(v):
+    """[..., 64] lanes -> [...]: lane ^ 32, ^ 16, ... ^ 1."""
+    while v.shape[-1] > 1:
+        v = v[..., :v.shape[-1] // 2] + v[..., v.shape[-1] // 2:]
+    return v[..., 0]
+
+
+def in_turn(v):
+    """Along the last axis, one behind the other."""
+    t = np.zeros(v.shape[:-1], np.float32)
+    for i in range(v.shape[-1]):
+        t = t + v[..., i]
+    return t
+
+
+def inverse(total, n, eps):
+    return np.float32(1) / np.sqrt(total / np.float32(n) + np.float32(eps))
+
+
+def normed(x, groups, eps):
+    """Rows by groups of whole waves' worth (four columns a lane) or one: 256 columns a wave, the waves' sums in turn."""
+    y = np.empty_like(x)
+    gs = x.shape[1] // groups
+    for i, row in enumerate(x):
+        g = np.zeros((groups, (gs + 255) // 256 * 256), np.float32)
+        g[:, :gs] = row.reshape(groups, gs)
+        q, ss = g.reshape(groups, -1, 64, 4), np.float32(0)
+        for e in range(4):
+            ss = fma(q[..., e], q[..., e], ss)
+        y[i] = (row.reshape(groups, gs) * inverse(in_turn(wave_sum(ss)), gs, eps)[:, None]).reshape(-1)
+    return y
+
+
+@pytest.mark.parametrize("rows,k,groups", [(rows, *shape) for rows in (1, 3, 600) for shape in
+                                           [(1024, 1), (2048, 1), (4096, 1), (4096, 2), (4096, 4), (2052, 1), (8192, 1), (8192, 8), (4100, 1)]
+                                           if rows < 512 or shape[0] <= 4096])             # (many longer rows: another form)
+def test_norm_adds_up_in_turn(hip, rows, k, groups):
+    """What the product keeps of its normed row, to the bit."""
+    note(f"words of a norm, rows {rows} k {k} groups {groups}")
+    rng = np.random.default_rng(k + groups)
+    ks, n = (k + 63) // 64 * 64, 40
+    at, end = places(4, x=rows * k, keep=rows * k, out=rows * n)
+    x = rng.standard_normal((rows, k), dtype=np.float32)
+    f32map(hip, WS, end, x, at["x"])
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * ks)
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * ks)
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=ks, src=at["x"], src_stride=k, groups=groups, eps=1e-6, keep=at["keep"], keep_stride=k, kept=1,
+                        opnd=0, out=at["out"], out_stride=n)
+    hip.linear_dev(WS, OP, WT, up(hip, spec.words()), 0, rows)
+    at_most = min(rows, 20)
+    got = read(hip, WS, at["keep"], rows * k).reshape(rows, k)[-at_most:]
+    assert np.array_equal(got.view(np.uint32), normed(x[-at_most:], groups, 1e-6).view(np.uint32))
+
+
+@pytest.mark.parametrize("k,shift,twice", [(1024, 0, True), (2048, 0, True), (2048, 1, False), (1501, 3, True), (4096, 0, True), (4095, 0, False)])
+def test_branched_norms_of_one_row_add_up_by_thread(hip, k, shift, twice):
+    """x + the branch's row behind a norm of its own, then a norm: 512 threads, each its columns in turn, then wave by wave."""
+    note(f"words of a branched norm, k {k} shift {shift} twice {twice}")
+    rng = np.random.default_rng(k)
+    ks, n, eps = (k + 63) // 64 * 64, 24, np.float32(1e-5)
+    at, end = places(4, **{name: k + 4 for name in ("x", "b", "bw", "wt", "res", "keep")}, out=n)
+    at = {name: off + (shift if name != "out" else 0) for name, off in at.items()}
+    x, b, bw, wt = (rng.standard_normal(k, dtype=np.float32) for _ in range(4))
+    f32map(hip, WS, end + 4)
+    for name, v in (("out", np.zeros(n)), ("keep", np.zeros(k)), ("res", np.zeros(k)), ("wt", wt), ("bw", bw), ("b", b), ("x", x)):
+        hip.scatter_contiguous(WS, at[name], np.ascontiguousarray(v, np.float32))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * ks)
+    spec = A.LinearSpec(w=0, n=n, k=k, k_stride=ks, src=at["x"], src_stride=k, groups=1, eps=eps, wt=at["wt"], wt_len=k if twice else 0, wt_add=0.5,
+                        branched=2, branch=at["b"], branch_stride=k, branch_wt=at["bw"], res_out=at["res"], res_stride=k,
+                        keep=at["keep"], keep_stride=k, kept=1, out=at["out"], out_stride=n)
+    hip.linear_dev(WS, OP, WT, up(hip, spec.words()), 0, 1)
+
+    def norm(v):
+        ss = np.zeros(512, np.float32)
+        for c in np.pad(v, (0, -k % 512)).reshape(-1, 512):
+            ss = fma(c, c, ss)
+        return inverse(in_turn(wave_sum(ss.reshape(8, 64))), k, eps)
+    half = np.float32(0.5)
+    res = fma(b * norm(b), half + bw, x)
+    kept = res * norm(res) * (half + wt if twice else np.float32(1))
+    for name, want in (("res", res), ("keep", kept)):
+        assert np.array_equal(read(hip, WS, at[name], k).view(np.uint32), want.view(np.uint32)), name
