@@ -794,15 +794,18 @@ __device__ __forceinline__ void put_units(const LinSpec& s, float* act, bf16_t* 
 // before (of two passes before where rows are short) have been used: 64 .. 128 KB of a CU in flight throughout, without a wait for
 // all of them.  A pass leaves its sums over K in LDS; no barrier before there is no room for more.  What remains is the tokens' way
 // in, 128 KB a CU for 16 of 4096 columns: 2 us at the rate of the L2s.
+// The order of the sums over K is the other kernel's, to the bit (a router behind them turns another order into another expert): steps of
+// K in turn by wave, the waves' sums in order.  ODD: a pass at most, where that kernel has sixteen waves: a wave here has two of them, their
+// steps the even and the odd ones of its own.
 // us, the kernel above and this one: 12 tokens, 28672 x 4096 (pairs) 54.3 and 41.5 (5.7 TB/s), 12576 x 4096 27.2 and 22, 32768 x 4096 58.2 and
 // 48.3, 10304 x 2048 14.4 and 10.3, 2048 x 2048 5.5 and 4.7, 14336 x 2560 (pairs) 18.9 and 16.9; 32 tokens, the same: 68 and 47, 34.3 and
 // 26.4, 71.5 and 54.4, 18.6 and 12.9, 7.7 and 6.9, 24.5 and 19.4.
-template <int MT, int S>
+template <int MT, int S, bool ODD>
 __global__ void __launch_bounds__(512)
 k_linear_few(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* act, bf16_t* opnd, uint32_t kp, uint32_t n, uint32_t rows,
              uint32_t units, uint32_t per, uint32_t pair, const LinSpec s) {
-  constexpr int NW = 8, D = S <= 4 ? 2 : 1, P = 16 / MT;
-  __shared__ f4_t red[P][MT][NW][64];
+  constexpr int NW = 8, D = S <= 4 && !ODD ? 2 : 1, P = ODD ? 1 : 16 / MT, NS = ODD ? 2 : 1;
+  __shared__ f4_t red[P][MT][NS * NW][64];
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t begin = blockIdx.x * per, end = min(begin + per, units), passes = ((end - begin + 15u) >> 4) << pair;
   // step u of this wave: columns 64 (wave + 8 u) ..; some waves' last lies beyond the row's end: they read their first again, and `keep` makes zeros of it
@@ -847,7 +850,7 @@ k_linear_few(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* 
       const auto sum = [&](uint32_t q) {
         f4_t v = red[q][m][0][lane];
 #pragma unroll
-        for (int i = 1; i < NW; i++) v += red[q][m][i][lane];
+        for (int i = 1; i < NS * NW; i++) v += red[q][m][i][lane];
         return v;
       };
       const f4_t a = sum(p), b = pair ? sum(p + 1u) : a;
@@ -860,9 +863,9 @@ k_linear_few(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* 
     constexpr int d = decltype(place)::value;
     if (p - first == (uint32_t)P) { sums(p); __syncthreads(); first = p; }
     const bf16_t* next = row_of(p + D);
-    f4_t acc[MT];
+    f4_t acc[NS][MT];
 #pragma unroll
-    for (int m = 0; m < MT; m++) acc[m] = (f4_t){0, 0, 0, 0};
+    for (int m = 0; m < MT; m++) acc[0][m] = acc[NS - 1][m] = (f4_t){0, 0, 0, 0};
 #pragma unroll
     for (int u = 0; u < S; u++) {
 #pragma unroll
@@ -870,13 +873,15 @@ k_linear_few(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X, float* 
 #pragma unroll
         for (int m = 0; m < MT; m++) {
           if (u == S - 1) { w[d][u][h] = kept(w[d][u][h]); x[u][h][m] = kept(x[u][h][m]); }
-          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[d][u][h], x[u][h][m], acc[m], 0, 0, 0);
+          acc[u % NS][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[d][u][h], x[u][h][m], acc[u % NS][m], 0, 0, 0);
         }
       if (more) ask(next, d, u);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int m = 0; m < MT; m++) red[p - first][m][wave][lane] = acc[m];
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+      for (int q = 0; q < NS; q++) red[p - first][m][q * NW + wave][lane] = acc[q][m];
   };
   typedef std::integral_constant<int, 0> A;
   typedef std::integral_constant<int, D - 1> B;
@@ -1155,14 +1160,16 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
     const auto go = [&](auto* one, auto* two) {
       (rows <= 16 ? one : two)<<<grid, 512, 0, g.stream>>>(W, X, act, op, s.k_stride, s.n, rows, units, per, pair, s);
     };
+#define FEW(S) do { if (pair || per > 16u) go(k_linear_few<1, S, false>, k_linear_few<2, S, false>); else go(k_linear_few<1, S, true>, k_linear_few<2, S, true>); } while (0)
     switch (cdiv(s.k_stride, 512)) {
-      case 3: go(k_linear_few<1, 3>, k_linear_few<2, 3>); break;
-      case 4: go(k_linear_few<1, 4>, k_linear_few<2, 4>); break;
-      case 5: go(k_linear_few<1, 5>, k_linear_few<2, 5>); break;
-      case 6: go(k_linear_few<1, 6>, k_linear_few<2, 6>); break;
-      case 7: go(k_linear_few<1, 7>, k_linear_few<2, 7>); break;
-      default: go(k_linear_few<1, 8>, k_linear_few<2, 8>); break;
+      case 3: FEW(3); break;
+      case 4: FEW(4); break;
+      case 5: FEW(5); break;
+      case 6: FEW(6); break;
+      case 7: FEW(7); break;
+      default: FEW(8); break;
     }
+#undef FEW
     count_launch();
     return check_launch();
   }

@@ -202,3 +202,30 @@ def test_branched_norms_of_one_row_add_up_by_thread(hip, k, shift, twice):
     kept = res * norm(res) * (half + wt if twice else np.float32(1))
     for name, want in (("res", res), ("keep", kept)):
         assert np.array_equal(read(hip, WS, at[name], k).view(np.uint32), want.view(np.uint32)), name
+
+
+# ---- products of few rows ----------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("k", [2112, 2560, 3008, 4096])
+@pytest.mark.parametrize("rows,epi", [(2, 0), (16, 1), (19, 0), (32, 0)])
+def test_a_narrow_product_does_not_hang_on_its_width(hip, rows, epi, k):
+    """Up to 16 matrix rows a compute unit the sums are those of sixteen waves, whichever kernel takes the width: 13 of them, 15 of them and
+    a few rows of the same matrix, the same words."""
+    note(f"words of a narrow product, rows {rows} k {k} epi {epi}")
+    rng = np.random.default_rng(k + rows)
+    cu = 256
+    widths = (15 * cu, 13 * cu, 6 * cu + 5, 33)
+    n = widths[0]
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * k)
+    hip.scatter_contiguous(WT, 0, f32_to_bf16(rng.standard_normal(n * k, dtype=np.float32)))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * k)
+    hip.scatter_contiguous(OP, 0, f32_to_bf16(rng.standard_normal(rows * k, dtype=np.float32)))
+    old = rng.standard_normal((rows, n), dtype=np.float32)
+    got = []
+    for w in widths:
+        f32map(hip, WS, rows * n, old)
+        spec = A.LinearSpec(w=0, n=w, k=k, k_stride=k, opnd=0, ready=1, out=0, out_stride=n, epi=epi)
+        hip.linear_dev(WS, OP, WT, up(hip, spec.words()), 0, rows)
+        got.append(read(hip, WS, 0, rows * n).reshape(rows, n))
+    for w, y in zip(widths[1:], got[1:]):
+        assert np.array_equal(y[:, :w].view(np.uint32), got[0][:, :w].view(np.uint32)), w
+        assert np.array_equal(y[:, w:], old[:, w:])
