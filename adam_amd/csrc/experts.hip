@@ -163,88 +163,104 @@ k_experts_in(const bf16_t* __restrict__ W, float* act, Choice* choice, const XSp
   }
 }
 
-// A row of the result a wave, the shared expert's columns first: they do not wait for the choice, nor do the activations, which
-// lie by place in the choice and get their weights in the sums.  Two runs of U times 512 columns in flight.
+// A row of the result a wave: the chosen experts' columns, then the shared expert's.  LDS holds the activations times their experts'
+// weights, by place in the choice (whatever its length), the shared expert's behind all places.  Activations and the choice are asked for
+// together; so are the shared expert's first columns where which ones a lane has does not hang on the choice, ahead of all others.  Two
+// runs of U times 512 columns in flight besides.
 // What bounds it is the weights' way in and what stands ahead of it (2048 rows of 6 x 1024 and 2048 columns, 33.5 MB, 6.9 us at a
-// large copy's rate: 14.2 us with two rows a wave, half the CUs at work and the activations weighted as they are staged, 12.5 so).
+// large copy's rate: 14.2 us with two rows a wave, half the CUs at work and nothing ahead of the choice, 12.5 so).
 template <int U>
 __global__ void __launch_bounds__(XSTEP)
 k_experts_out(const bf16_t* __restrict__ W, float* act, const Choice* __restrict__ choice, const XSpec s, uint32_t magic) {
   extern __shared__ __attribute__((aligned(16))) float xs[];
   __shared__ Choice ch;
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, fs = s.ff_stride, stride = gridDim.x * (XSTEP / 64u);
-  const uint32_t sk = s.shared_ff ? s.shared_ff_stride : 0u, held = sk + min(s.top, s.experts) * fs, half = held >> 1;
-  uint4 p[2][U];
-  uint32_t row = blockIdx.x * (XSTEP / 64u) + wave, k0 = lane * 8u, from = min(row, s.width - 1u), fk = k0, end = 0u;
-  // the next run: within the shared expert's columns, or anywhere once the choice is known
-  const auto fetch = [&](uint4 (&to)[U], bool chosen) {
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const uint32_t k = chosen ? min(fk + 512u * u, end - 8u) : fk + 512u * u, c = max(k, sk) - sk, j = __umulhi(c, magic);
-      const uint64_t at = !chosen || k < sk ? s.shared_down + (uint64_t)from * s.shared_ff_stride + k
-                                            : s.down + (uint64_t)ch.id[j] * s.down_step + (uint64_t)from * fs + (c - j * fs);
-      to[u] = *(const uint4*)(W + at);
-    }
-    fk += 512u * U;
-    if (chosen && fk - lane * 8u >= end) { fk = lane * 8u; from += stride; }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  const bool early = sk >= 512u * U;
+  const uint32_t sk = s.shared_ff ? s.shared_ff_stride : 0u, places = min(s.top, s.experts) * fs, held = places + sk, half = held >> 1;
+  const uint32_t row0 = blockIdx.x * (XSTEP / 64u) + wave;
   const uint32_t id = choice->id[lane], n_ch = choice->n;    // (a word a lane: MAX_TOP of them)
   const float wt = choice->wt[lane], back = choice->back;
   const float gate = act[s.logits + s.experts + s.identity - (s.shared_ff ? 0u : 1u)];
   // Sixteen values a thread (of a short row two) asked for at once and no load under a condition
   constexpr uint32_t R = U == 1 ? 2 : 16;
   const auto value = [&](uint32_t i0) {
-    const uint32_t i = min(i0, held - 1u), c = max(i, sk) - sk, j = __umulhi(c, magic);
-    return act[i < sk ? s.shared_act + min(i, s.shared_ff - 1u) : s.act + j * fs + min(c - j * fs, s.ff - 1u)];
+    const uint32_t i = min(i0, held - 1u), j = __umulhi(i, magic);
+    return act[i < places ? s.act + j * fs + min(i - j * fs, s.ff - 1u) : s.shared_act + min(i - places, s.shared_ff - 1u)];
   };
   float v[R];
 #pragma unroll
   for (uint32_t u = 0; u < R; u++) v[u] = value(threadIdx.x + u * XSTEP);
-  if (early) fetch(p[0], false);
+  // runs of a row: `chosen` of them up to column `edge`, the others behind it; the first of these is at hand for the wave's first row
+  const bool early = (fs & 511u) == 0u && sk >= 512u * U;
+  uint4 p[2][U], e[U];
+  if (early)
+#pragma unroll
+    for (int u = 0; u < U; u++) e[u] = *(const uint4*)(W + s.shared_down + (uint64_t)min(row0, s.width - 1u) * sk + lane * 8u + 512u * u);
+  __builtin_amdgcn_sched_barrier(0);
   ch.id[lane] = id; ch.wt[lane] = wt;                        // (every wave the same words, for itself)
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  end = sk + n_ch * fs;
-  uint32_t left = row < s.width ? ((s.width - 1u - row) / stride + 1u) * max(1u, (end + 512u * U - 1u) / (512u * U)) : 0u;
-  if (end && left > 0u) {
-    if (!early) fetch(p[0], true);
-    else if (fk - lane * 8u >= end) { fk = lane * 8u; from += stride; }
-    if (left > 1u) fetch(p[1], true);
-  }
+  const auto runs_of = [](uint32_t columns) { return (columns + 512u * U - 1u) / (512u * U); };
+  const uint32_t body = n_ch * fs, end = body + sk, edge = early ? body : end, chosen = runs_of(edge), all = chosen + runs_of(end - edge);
+  const auto base = [&](uint32_t run) { return (run < chosen ? run * (512u * U) : edge + (run - chosen) * (512u * U)) + lane * 8u; };
+  const auto limit = [&](uint32_t run) { return run < chosen ? edge : end; };
+  const auto skip = [&](uint32_t row, uint32_t run) { return early && row == row0 && run == chosen; };
+  uint32_t from = row0, fr = skip(row0, 0u) ? 1u : 0u;       // the run to be asked for
+  const auto wrap = [&](uint32_t& row, uint32_t& run) { if (run >= all) { run = 0u; row += stride; } };
+  wrap(from, fr);
+  const auto fetch = [&](int x) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t k = min(base(fr) + 512u * u, limit(fr) - 8u), j = min(__umulhi(k, magic), (uint32_t)MAX_TOP - 1u);
+      const uint64_t at = k < body ? s.down + (uint64_t)ch.id[j] * s.down_step + (uint64_t)from * fs + (k - j * fs)
+                                   : s.shared_down + (uint64_t)from * sk + (k - body);
+      p[x][u] = *(const uint4*)(W + at);
+    }
+    fr++;
+    if (skip(from, fr)) fr++;
+    wrap(from, fr);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  uint32_t left = row0 < s.width ? ((s.width - 1u - row0) / stride + 1u) * all - (early ? 1u : 0u) : 0u;
+  if (left > 0u) fetch(0);
+  if (left > 1u) fetch(1);
   const float sg = sigmoid_f(gate);
   const auto put = [&](uint32_t i, float x) {
-    const uint32_t c = max(i, sk) - sk, j = __umulhi(c, magic);
-    if (i < held) xs[PLANE(i, half)] = i < sk ? (i < s.shared_ff ? x * sg : 0.f) : c - j * fs < s.ff ? x : 0.f;
+    const uint32_t j = min(__umulhi(i, magic), (uint32_t)MAX_TOP - 1u);
+    if (i < held) xs[PLANE(i, half)] = i < places ? (i - j * fs < s.ff ? x * ch.wt[j] : 0.f) : i - places < s.shared_ff ? x * sg : 0.f;
   };
 #pragma unroll
   for (uint32_t u = 0; u < R; u++) put(threadIdx.x + u * XSTEP, v[u]);
   for (uint32_t i = threadIdx.x + R * XSTEP; i < held; i += XSTEP) put(i, value(i));
   __syncthreads();
   float a = 0.f;
-  const auto more = [&](int x) { if (end) fetch(p[x], true); };
-  const auto run = [&](int x) {
-    if (end)
+  uint32_t row = row0, r = 0u;
+  const auto add = [&](const uint4 (&w)[U]) {                // run r of the row
 #pragma unroll
-      for (int u = 0; u < U; u++) {
-        const uint32_t k = k0 + 512u * u, j = __umulhi(max(k, sk) - sk, magic);
-        if (k >= end) break;
-        const float4 lo = *(const float4*)(xs + (k >> 1)), hi = *(const float4*)(xs + half + (k >> 1));
-        float t = 0.f;
-        fma8(t, p[x][u], lo, hi);
-        a = fmaf(k < sk ? 1.f : ch.wt[j], t, a);
-      }
-    k0 += 512u * U;
-    if (k0 - lane * 8u < end) return;
+    for (int u = 0; u < U; u++) {
+      const uint32_t k = base(r) + 512u * u, i = k < body ? k : k - body + places;
+      if (k >= limit(r)) break;
+      const float4 lo = *(const float4*)(xs + (i >> 1)), hi = *(const float4*)(xs + half + (i >> 1));
+      fma8(a, w[u], lo, hi);
+    }
+    r++;
+  };
+  const auto done = [&] {
+    if (r < all) return;
     a = wave_add(a);
     if (lane == 0) {
       const float y = fmaf(back, act[s.x + row], a);
       float* d = act + s.out + row;
       *d = s.epi ? *d + y : y;
     }
-    a = 0.f; k0 = lane * 8u; row += stride;
+    a = 0.f; r = 0u; row += stride;
   };
-  RUNS_OF_TWO(left, run, more);
+  const auto at_hand = [&] { if (skip(row, r)) add(e); };
+  if (all == 0u) {                                           // nothing chosen has a matrix, and nothing is shared
+    while (row < s.width) done();
+    return;
+  }
+  if (row < s.width) { at_hand(); done(); }
+  const auto run = [&](int x) { add(p[x]); at_hand(); done(); };
+  RUNS_OF_TWO(left, run, fetch);
 }
 
 // ---- more rows ------------------------------------------------------------------------------------------------------

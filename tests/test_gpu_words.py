@@ -229,3 +229,57 @@ def test_a_narrow_product_does_not_hang_on_its_width(hip, rows, epi, k):
     for w, y in zip(widths[1:], got[1:]):
         assert np.array_equal(y[:, :w].view(np.uint32), got[0][:, :w].view(np.uint32)), w
         assert np.array_equal(y[:, w:], old[:, w:])
+
+
+# ---- one row through the experts -----------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("E,I,top,ff,shared,width,epi", [(4, 0, 4, 1024, 2048, 300, 0), (3, 1, 4, 1000, 2500, 2070, 1), (2, 2, 4, 512, 0, 70, 0),
+                                                         (7, 1, 8, 576, 2048, 33, 1), (4, 4, 2, 448, 2112, 50, 0), (1, 1, 2, 2048, 4096, 4200, 0),
+                                                         (2, 6, 2, 1536, 2048, 100, 1), (8, 0, 1, 64, 128, 40, 0)])
+def test_one_row_of_the_experts_adds_up_in_the_order_of_its_columns(hip, E, I, top, ff, shared, width, epi):
+    """Equal logits, so that every weight is a power of two; the correction decides who is chosen and in which order.  A lane has columns
+    8 lane .. of every 512 of the chosen experts' activations (weighted) and the shared expert's behind them, in turn."""
+    note(f"words of the experts, {E} + {I} top {top} ff {ff} shared {shared} width {width} epi {epi}")
+    rng = np.random.default_rng(E * ff + width)
+    n, ks, F, F16, S = E + I, (width + 63) // 64 * 64, (ff + 63) // 64 * 64, (ff + 15) // 16 * 16, (shared + 63) // 64 * 64
+    assert n & (n - 1) == 0
+    at, end = places(4, h=width, log=n + 1, corr=n, out=width, act=top * F, sact=max(S, 4))
+    gu, dn, sd = 0, E * 2 * F16 * ks, E * 2 * F16 * ks + E * width * F
+    bf = lambda w: (w.astype(np.uint32) << 16).view(np.float32)
+    W = f32_to_bf16(rng.standard_normal((E, 2 * F16, ks), dtype=np.float32) / np.float32(np.sqrt(width)))
+    W[:, :, width:] = 0
+    D = f32_to_bf16(rng.standard_normal((E, width, F), dtype=np.float32))
+    sh = f32_to_bf16(rng.standard_normal((width, S), dtype=np.float32))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, sd + width * S + 8)
+    for off, w in ((gu, W), (dn, D)) + (((sd, sh),) if shared else ()):
+        hip.scatter_contiguous(WT, off, w.reshape(-1))
+    x, old = rng.standard_normal(width, dtype=np.float32), rng.standard_normal(width, dtype=np.float32)
+    corr, sact = rng.permutation(n).astype(np.float32), rng.standard_normal(max(S, 4), dtype=np.float32)
+    f32map(hip, WS, end + 4)
+    log = np.zeros(n + 1)
+    log[n] = 120.0                                             # the shared expert's gate: exactly one
+    for name, v in (("h", x), ("log", log), ("corr", corr), ("out", old), ("sact", sact)):
+        hip.scatter_contiguous(WS, at[name], np.ascontiguousarray(v, np.float32))
+    spec = A.ExpertsSpec(experts=E, identity=I, top=top, ff=ff, ff_stride=F, width=width, k_stride=ks, gate_up=gu, gate_up_step=2 * F16 * ks,
+                         down=dn, down_step=width * F, logits=at["log"], logits_stride=n + 1, correction=at["corr"], x=at["h"], x_stride=width,
+                         act=at["act"], shared_ff=shared, shared_ff_stride=S, shared_down=sd, shared_act=at["sact"], out=at["out"],
+                         out_stride=width, epi=epi)
+    hip.experts_dev(WS, OP, WT, up(hip, spec.words()), 0, 1)
+    first = [int(e) for e in np.argsort(-corr)[:top]]
+    chosen, p = [e for e in first if e < E], np.float32(1.0 / n)
+    act = read(hip, WS, at["act"], top * F).reshape(top, F)
+    cols = [np.where(np.arange(F) < ff, act[j] * p, np.float32(0)) for j in range(len(chosen))]
+    mats = [bf(D[e]) for e in chosen]
+    if shared:
+        cols.append(np.where(np.arange(S) < shared, sact[:S], np.float32(0)))
+        mats.append(bf(sh))
+    a = np.zeros((width, 64), np.float32)
+    if cols:
+        v, m = np.concatenate(cols), np.concatenate(mats, axis=1)
+        pad = -len(v) % 512
+        for b, w in zip(np.pad(v, (0, pad)).reshape(-1, 64, 8), np.pad(m, ((0, 0), (0, pad))).reshape(width, -1, 64, 8).transpose(1, 0, 2, 3)):
+            for e in range(8):
+                a = fma(w[..., e], b[:, e], a)
+    back = np.float32(p * (top - len(chosen)))
+    want = fma(np.broadcast_to(back, x.shape), x, wave_sum(a))
+    want = old + want if epi else want
+    assert np.array_equal(read(hip, WS, at["out"], width).view(np.uint32), want.view(np.uint32))
