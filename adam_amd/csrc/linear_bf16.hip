@@ -787,7 +787,7 @@ __device__ __forceinline__ void put_units(const LinSpec& s, float* act, bf16_t* 
   }
 }
 
-// Rows of 1025 .. 4096 columns.  Bound by the weights' way in.  One workgroup a CU, each an equal share of the units (the kernel above
+// Rows of 1152 .. 4096 columns.  Bound by the weights' way in.  One workgroup a CU, each an equal share of the units (the kernel above
 // put 28672 rows into 896 workgroups, of which three fit a CU: the last 128 ran alone), in passes of 16 matrix rows.  A wave's S steps
 // of K are the same in every pass, so its columns of the tokens stay in registers (they were read again for every 32 matrix rows:
 // half as many bytes as the weights at 16 tokens, as many at 32), and a step's weights are asked for as soon as its own of the pass
@@ -1152,11 +1152,21 @@ int run_linear(Map* ma, Map* mo, Map* mw, const LinSpec& s, const uint32_t* row_
   if (!s.ready) operand_rows<bf16_t>(s, act, op + s.opnd, row_idx, rows);
   if (rows > 32) return launch_tiles<bf16_t>(W, X, act, op, s, rows);
   const uint32_t pair = s.epi == 2u, units = pair ? cdiv(s.n, 32) * 16u : s.n, per = cdiv(units, g.n_cu), grid = cdiv(units, per);
-  // Up to 1024 columns a launch is over before its registers are worth filling (8192 x 1024 under 16 rows: 5.7 us as it is, 9.7 with
-  // one step of four used); beyond 4096 the tokens do not fit them.  One pass of nearly all its 16 matrix rows on every CU has nothing
-  // to stream behind: 16 waves in two lots of loads do it as well or better (12 rows, 4096 x 4096: 9.75 and 10.1, of 32 rows 14.3 and
-  // 14.4; 13 matrix rows a CU, 3328 x 4096: 9.7 and 9.3, 14.4 and 13.6).
-  if (s.k_stride > 1024u && s.k_stride <= 4096u && (pair || per <= 14u || per > 16u || s.k_stride <= 2048u)) {
+  // Below 1152 columns a launch is over before its registers are worth filling, and of three steps the third is nearly empty (32 rows,
+  // 3584 x 1088: 5.4 us as it is, 6.5 with this kernel; 8192 x 1024 under 16 rows 5.7, 9.7 with one step of four used); beyond 4096 the
+  // tokens do not fit them.  In between a wave whose last step lies beyond the row's end reads its first columns again; where that is
+  // more than a twentieth of the row, it costs more than it brings unless a CU has hardly a pass or more than two (16 rows, us, the kernel
+  // below and this one: 4096 x 1216 4.5 and 5.1, 8192 x 2112 9.8 and 11.2, 4096 x 3648 9.2 and 10.6; but 1536 x 2112 6.0 and 5.8, 9216 x 2112 14.7 and
+  // 12.4, 28671 x 2112 27.9 and 25.4; of pairs, whose CUs have twice the rows, 8192 x 2112 9.7 and 11.5, 512 x 2112 8.0 and 6.1).
+  // One pass of nearly all its 16 matrix rows on every CU has nothing to stream behind: 16 waves in two lots of loads do it
+  // as well or better (12 rows, 4096 x 4096: 9.4 and 10.4, of 32 rows 13.8 and 13.9; 13 matrix rows a CU, 3328 x 4096: 9.95 and 8.4, 14.1 and 13);
+  // nor do two of them with one step of each in flight beat one workgroup of 32 a CU (8192 x 3072 12.2 and 13.9, 8192 x 4032 14.6 and 16.4).
+  // The words are the same either way.
+  const uint32_t room = 512u * cdiv(s.k_stride, 512), each = pair ? 2u * per : per;       // columns that the steps have room for; matrix rows a CU
+  const bool whole = s.k_stride * 20u >= room * 19u;
+  if (s.k_stride >= 1152u && s.k_stride <= 4096u &&
+      (whole ? pair || s.k_stride <= 2048u || per <= 14u || (per > 16u && !(per > 28u && per <= 32u && s.k_stride > 2560u))
+             : each <= 8u || each > (pair ? 64u : 34u))) {
     const auto go = [&](auto* one, auto* two) {
       (rows <= 16 ? one : two)<<<grid, 512, 0, g.stream>>>(W, X, act, op, s.k_stride, s.n, rows, units, per, pair, s);
     };

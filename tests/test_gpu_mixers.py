@@ -128,7 +128,10 @@ def test_linear_tiles(hip, rows, n, k, biased, add):
     (2, 1, 1088, 0, 0), (16, 4095, 1536, 1, 0), (17, 4097, 2048, 0, 0), (32, 8195, 1600, 1, 0), (12, 12300, 2048, 0, 0), (3, 16390, 1088, 1, 0),
     (31, 36901, 1088, 0, 0), (5, 70003, 1088, 1, 0), (16, 8200, 2560, 0, 0), (32, 300, 2624, 1, 0), (9, 4100, 3072, 0, 0), (20, 515, 3520, 1, 0),
     (16, 8208, 4096, 0, 0), (29, 4099, 4032, 0, 0), (12, 32, 1088, 2, 0), (32, 8227, 2048, 2, 35), (2, 8257, 4096, 2, 1), (18, 16448, 1216, 2, 64),
-    (13, 34000, 1344, 2, 16), (7, 3601, 2112, 0, 0)])
+    (13, 34000, 1344, 2, 16), (7, 3601, 2112, 0, 0),
+    # columns read twice in passes behind one another; sums of gate and up that LDS does not hold at once
+    (31, 36901, 1216, 0, 0), (5, 70003, 1344, 1, 0), (32, 12300, 1600, 0, 0), (20, 33859, 1152, 2, 35), (32, 40000, 1280, 2, 64), (9, 9222, 2624, 0, 0),
+    (3, 1500, 1216, 0, 0)])
 def test_products_of_few_rows(hip, rows, n, k, epi, tail):
     """One pass of 16 matrix rows a workgroup up to more than LDS holds the sums of, rows of every count of steps, whole and ragged; an
     infinite value of a token whose columns a wave reads twice."""

@@ -231,6 +231,26 @@ def test_a_narrow_product_does_not_hang_on_its_width(hip, rows, epi, k):
         assert np.array_equal(y[:, w:], old[:, w:])
 
 
+@pytest.mark.parametrize("rows,k", [(2, 1152), (16, 1216), (19, 2112), (32, 2624), (12, 3072), (17, 3648), (9, 1472)])
+def test_a_wide_product_does_not_hang_on_its_width(hip, rows, k):
+    """Beyond 16 matrix rows a compute unit the sums are those of eight waves: two kernels share the widths, the same words."""
+    note(f"words of a wide product, rows {rows} k {k}")
+    rng = np.random.default_rng(k + rows)
+    widths = tuple(256 * w + 5 for w in (36, 31, 24, 16))
+    n = widths[0]
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * k)
+    hip.scatter_contiguous(WT, 0, f32_to_bf16(rng.standard_normal(n * k, dtype=np.float32)))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * k)
+    hip.scatter_contiguous(OP, 0, f32_to_bf16(rng.standard_normal(rows * k, dtype=np.float32)))
+    f32map(hip, WS, rows * n)
+    got = []
+    for w in widths:
+        hip.linear_dev(WS, OP, WT, up(hip, A.LinearSpec(w=0, n=w, k=k, k_stride=k, opnd=0, ready=1, out=0, out_stride=n).words()), 0, rows)
+        got.append(read(hip, WS, 0, rows * n).reshape(rows, n))
+    for w, y in zip(widths[1:], got[1:]):
+        assert np.array_equal(y[:, :w].view(np.uint32), got[0][:, :w].view(np.uint32)), w
+
+
 # ---- one row through the experts -----------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("E,I,top,ff,shared,width,epi", [(4, 0, 4, 1024, 2048, 300, 0), (3, 1, 4, 1000, 2500, 2070, 1), (2, 2, 4, 512, 0, 70, 0),
                                                          (7, 1, 8, 576, 2048, 33, 1), (4, 4, 2, 448, 2112, 50, 0), (1, 1, 2, 2048, 4096, 4200, 0),
