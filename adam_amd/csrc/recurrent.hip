@@ -474,28 +474,26 @@ k_retention_prep(const RSpec s, const float* __restrict__ act, float* __restrict
 }
 
 // ---- the walk over the chunks ---------------------------------------------------------------------------------------
-// A serial chain, so what counts is a chunk's latency.  Four waves share the state rows (NT tiles of 16 each); a tile's
-// accumulator holds rows 4 g + i of lane group g, which is also how instruction i wants its right operand when the left one is
-// read as four consecutive columns per lane.  On their chain are only the products that the state needs (delta: W S, its sum
-// through LDS, K u); Q S goes out while that sum is on its way.  A fifth wave adds up the four shares of Q S, adds B u from what they
-// leave in LDS and stores, a chunk behind: loads and stores share a counter, and a wave that does both waits for its stores.
-// 2048 tokens in 32 heads of 128: outputs by the first of four waves, ahead of its part of the state, 136 us, retention 97; so 114 and 86.
-// One product behind the other by wave, the waves' parts as (0 + 1) + (2 + 3), B u behind that sum in order: a router behind these sums
-// turns another order into another choice of experts (with two sums a wave and a quarter of B u in each share 111 and 79 us, and 3e-2
-// in a mixture's logits).
-// FEW: one or two chunks, whose operands are not asked for ahead, so that a compute unit has three workgroups instead of two (16
-// sequences of 12 tokens 26.5 us, 48.5 with the other form, 38.6 before).
+// A serial chain, so what counts is a chunk's latency, or how much of it other workgroups hide (scan_form).  Four waves share the
+// state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which is also how instruction i wants its
+// right operand when the left one is read as four consecutive columns per lane.  On their chain are only the products that the state
+// needs (delta: W S, its sum through LDS, K u); Q S goes out while that sum is on its way.  A fifth wave adds up the four shares of
+// Q S, adds B u from what they leave in LDS and stores: loads and stores share a counter, and a wave that does both waits
+// for its stores.  2048 tokens in 32 heads of 128: outputs by the first of four waves, ahead of its part of the state, 136 us,
+// retention 97; so 114 and 79.
+// In every form one product behind the other by wave, the waves' parts as (0 + 1) + (2 + 3), B u behind that sum in order: a router behind
+// these sums turns another order into another choice of experts (with two sums a wave and a quarter of B u in each share 111 and 79
+// us, and 3e-2 in a mixture's logits).
 struct ScanArgs {
   uint32_t heads, dim, vdim, out, out_stride, s_off, m, pos;
   ChunkDims cd;
   uint32_t kv_heads, taps, conv_off, x, x_stride;     // delta: the convolution's ring is brought up to date here
   uint32_t seq_stride;                                // of the state; grid z: the sequence, its rows m z .. of the activations
 };
-#define SCAN_T 320u          // four waves of state rows and the one of the outputs
-template <int NT> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], u; float b; };
+template <int NT, int FORM> struct ChunkOps { f4_t w[NT], q[NT], k[NT], gl[NT], u; std::conditional_t<FORM == SCAN_TURNS, f4_t, float> b; };
 
-template <bool DELTA, int NT>
-__device__ __forceinline__ void load_ops(ChunkOps<NT>& o, const float* blk, const ChunkDims& cd, uint32_t wave, uint32_t lane, uint32_t v0) {
+template <bool DELTA, int NT, int FORM>
+__device__ __forceinline__ void load_ops(ChunkOps<NT, FORM>& o, const float* blk, const ChunkDims& cd, uint32_t wave, uint32_t lane, uint32_t v0) {
   const float *pQ = blk + CH * cd.Dp, *pK = pQ + CH * cd.Dp, *pB = pK + CH * cd.Dp, *pU = pB + 256u, *pG = pU + CH * cd.Vp;
 #pragma unroll
   for (int j = 0; j < NT; j++) {
@@ -506,34 +504,37 @@ __device__ __forceinline__ void load_ops(ChunkOps<NT>& o, const float* blk, cons
     o.gl[j] = *(const f4_t*)(pG + T * 16u + (lane >> 4) * 4u);
   }
   o.u = *(const f4_t*)(pU + v0 * 16u + lane * 4u);
-  o.b = pB[lane * 4u + wave];
+  if constexpr (FORM == SCAN_TURNS) o.b = *(const f4_t*)(pB + lane * 4u);
+  else o.b = pB[lane * 4u + wave];
 }
 
-template <bool DELTA, int NT, bool FEW>
-__global__ void __launch_bounds__(SCAN_T)
+template <bool DELTA, int NT, int FORM>
+__global__ void __launch_bounds__(SCAN_T(FORM), FORM == SCAN_TURNS ? 2 : 1)
 k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, float* state) {
   __shared__ f4_t p1[2][4][64], p2[2][4][64];                // [chunk & 1][wave][lane]
-  __shared__ float pb[2][4][64], pu[2][4][64];               // B and u, a quarter of the four a lane has by each wave
+  __shared__ f4_t pb[2][64], pu[2][64];                      // B and u for the fifth wave, one of a lane's four by each wave
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, D = a.dim, V = a.vdim, v = v0 + c;
   const uint32_t bs = chunk_floats(a.cd.Dp, a.cd.Vp), n = a.cd.n_chunks;
   const float* blk = scratch + ((uint64_t)blockIdx.z * a.heads + h) * n * bs;
   state += (uint64_t)blockIdx.z * a.seq_stride;
-  const auto sum4 = [&](const f4_t (*p)[64]) { return (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]); };
-  if (wave == 4u) {
-    float* out = act + a.out + (uint64_t)blockIdx.z * a.m * a.out_stride + h * V + v;
-    for (uint32_t ci = 0; ci <= n; ci++) {
+  float* out = act + a.out + (uint64_t)blockIdx.z * a.m * a.out_stride + h * V + v;
+  const auto put = [&](uint32_t ci, f4_t b, f4_t u) {        // the outputs of chunk ci
+    const f4_t (*p)[64] = p2[ci & 1u];
+    f4_t o = (p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(b[i], u[i], o, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t r = ci * CH + 4u * kg + i;
+      if (r < a.m && v < V) out[(uint64_t)r * a.out_stride] = o[i];
+    }
+  };
+  if (FORM != SCAN_TURNS && wave == 4u) {
+    if (DELTA) __syncthreads();                              // (there a chunk's shares are whole at the next one's barrier)
+    for (uint32_t ci = 0; ci < n; ci++) {
       __syncthreads();
-      if (ci == 0u) continue;
-      const uint32_t x = (ci - 1u) & 1u;
-      f4_t o = sum4(p2[x]);
-#pragma unroll
-      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(pb[x][i][lane], pu[x][i][lane], o, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint32_t r = (ci - 1u) * CH + 4u * kg + i;
-        if (r < a.m && v < V) out[(uint64_t)r * a.out_stride] = o[i];
-      }
+      put(ci, pb[ci & 1u][lane], pu[ci & 1u][lane]);
     }
   } else {
     float* S = state + a.s_off + (uint64_t)h * D * V;
@@ -551,63 +552,82 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
         for (int i = 0; i < 4; i++) if ((wave * NT + j) * 16u + 4u * kg + i >= D || v >= V) st[j][i] = 0.f;
     }
     // the operands of the chunk two ahead, asked for on every path (past the end: the last one's again)
-    const auto ask = [&](ChunkOps<NT>& o, uint32_t ci) { load_ops<DELTA, NT>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, lane, v0); __builtin_amdgcn_sched_barrier(0); };
-    const auto chunk = [&](const ChunkOps<NT>& cur, uint32_t x) {
-      f4_t u = cur.u;
-      f4_t s = {0, 0, 0, 0};
-      if (DELTA) {
+    const auto ask = [&](ChunkOps<NT, FORM>& o, uint32_t ci) { load_ops<DELTA, NT, FORM>(o, blk + (uint64_t)min(ci, n - 1u) * bs, a.cd, wave, lane, v0); __builtin_amdgcn_sched_barrier(0); };
+    const auto chunk = [&](const ChunkOps<NT, FORM>& cur, uint32_t ci) {
+      const uint32_t x = ci & 1u;
+      f4_t u = cur.u, s = {0, 0, 0, 0}, q_s = {0, 0, 0, 0}, r[4], was[NT];
+      const auto k_u = [&](int t) { st[t % NT] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[t % NT][t / NT], u[t / NT], st[t % NT], 0, 0, 0); };
+      const auto share = [&] {                               // of the outputs
+        p2[x][wave][lane] = q_s;
+        if constexpr (FORM != SCAN_TURNS) {
+          ((float*)&pb[x][lane])[wave] = cur.b;
+          ((float*)&pu[x][lane])[wave] = wave & 2u ? (wave & 1u ? u[3] : u[2]) : (wave & 1u ? u[1] : u[0]);
+        }
+      };
+      constexpr bool Q_AHEAD = FORM == SCAN_TURNS;           // of the barrier
+      if (DELTA || Q_AHEAD)
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
-          for (int i = 0; i < 4; i++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], s, 0, 0, 0);
-        p1[x][wave][lane] = s;
-        s = (f4_t){0, 0, 0, 0};
+          for (int i = 0; i < 4; i++) {
+            if (DELTA) s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.w[j][i], st[j][i], s, 0, 0, 0);
+            if (Q_AHEAD) q_s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], q_s, 0, 0, 0);
+          }
+      if (DELTA) p1[x][wave][lane] = s;
+      else if (!Q_AHEAD) {                                   // (an instruction waits for the one that it adds to: two sums in turn)
+#pragma unroll
+        for (int j = 0; j < NT; j++) { was[j] = st[j]; st[j] *= cur.gl[j]; }
+#pragma unroll
+        for (int t = 0; t < 4 * NT; t++) {
+          q_s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[t / 4][t % 4], was[t / 4][t % 4], q_s, 0, 0, 0);
+          k_u(t);
+        }
       }
+      if (!DELTA || Q_AHEAD) share();
       __syncthreads();
-      f4_t r[4];
       if (DELTA)
 #pragma unroll
         for (int w = 0; w < 4; w++) r[w] = p1[x][w][lane];
       __builtin_amdgcn_sched_barrier(0);                     // Q S behind them, not ahead of the barrier
+      if (DELTA && !Q_AHEAD)
 #pragma unroll
-      for (int j = 0; j < NT; j++)
+        for (int j = 0; j < NT; j++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], s, 0, 0, 0);
+          for (int i = 0; i < 4; i++) q_s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.q[j][i], st[j][i], q_s, 0, 0, 0);
       if (DELTA) u -= (r[0] + r[1]) + (r[2] + r[3]);
+      if constexpr (FORM == SCAN_TURNS) if (wave == (ci & 3u)) put(ci, cur.b, u);
+      if (DELTA || Q_AHEAD) {
 #pragma unroll
-      for (int j = 0; j < NT; j++) st[j] *= cur.gl[j];
+        for (int j = 0; j < NT; j++) st[j] *= cur.gl[j];
 #pragma unroll
-      for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][i], u[i], st[j], 0, 0, 0);
-      p2[x][wave][lane] = s;
-      pb[x][wave][lane] = cur.b;
-      pu[x][wave][lane] = wave & 2u ? (wave & 1u ? u[3] : u[2]) : (wave & 1u ? u[1] : u[0]);
+        for (int t = 0; t < 4 * NT; t++) k_u(t);
+        if (!Q_AHEAD) share();
+      }
     };
-    ChunkOps<NT> o0;
+    ChunkOps<NT, FORM> o0;
     ask(o0, 0);
-    if constexpr (FEW) {
+    if constexpr (FORM == SCAN_FEW) {
       for (uint32_t ci = 0; ci < n; ci++) {
         if (ci) ask(o0, ci);
-        chunk(o0, ci & 1u);
+        chunk(o0, ci);
       }
     } else {
       // (a loop in one piece: with a way out behind each chunk the loads were moved down to where only the rest of the loop needs them)
-      ChunkOps<NT> o1, o2;
+      ChunkOps<NT, FORM> o1, o2;
       ask(o1, 1); ask(o2, 2);
       uint32_t ci = 0;
       for (; ci + 3u <= n; ci += 3u) {
-        chunk(o0, ci & 1u);
+        chunk(o0, ci);
         ask(o0, ci + 3u);
-        chunk(o1, (ci + 1u) & 1u);
+        chunk(o1, ci + 1u);
         ask(o1, ci + 4u);
-        chunk(o2, ci & 1u);
+        chunk(o2, ci + 2u);
         ask(o2, ci + 5u);
       }
-      if (ci < n) chunk(o0, ci & 1u);
-      if (ci + 1u < n) chunk(o1, (ci + 1u) & 1u);
+      if (ci < n) chunk(o0, ci);
+      if (ci + 1u < n) chunk(o1, ci + 1u);
     }
-    __syncthreads();                                         // the last chunk's Q S is there
+    if (DELTA && FORM != SCAN_TURNS) __syncthreads();        // the last chunk's shares are there
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
@@ -622,7 +642,7 @@ k_chunk_scan(const ScanArgs a, const float* __restrict__ scratch, float* act, fl
     float* slot = state + a.conv_off + (uint64_t)((a.pos + r) % a.taps) * n_ch;
     const float* x = act + a.x + ((uint64_t)blockIdx.z * a.m + r) * a.x_stride;
     if (blockIdx.y == 0 && h % rep == 0)
-      for (uint32_t d = tid; d < D; d += SCAN_T) {
+      for (uint32_t d = tid; d < D; d += SCAN_T(FORM)) {
         slot[kv * D + d] = x[kv * D + d];
         slot[(a.kv_heads + kv) * D + d] = x[(a.kv_heads + kv) * D + d];
       }
@@ -642,17 +662,21 @@ template <bool DELTA>
 static int launch_scan(const ScanArgs& a, float* act, float* state, uint32_t n_seq) {
   const dim3 grid(a.heads, cdiv(a.vdim, 16), n_seq);
   const float* sc = (const float*)g_chunks.p;
-  const bool few = a.cd.n_chunks <= 2u;        // (above)
-#define SCAN(NT) do { if (few) k_chunk_scan<DELTA, NT, true><<<grid, SCAN_T, 0, g.stream>>>(a, sc, act, state); \
-                      else k_chunk_scan<DELTA, NT, false><<<grid, SCAN_T, 0, g.stream>>>(a, sc, act, state); } while (0)
+  const auto go = [&](auto tiles) {
+    constexpr int NT = decltype(tiles)::value;
+    constexpr bool turns = !DELTA || NT < 4;                 // (that one would spill)
+    const int form = scan_form((uint64_t)grid.x * grid.y * grid.z, a.cd.n_chunks, NT, NT == 1 || (!DELTA && NT == 2), turns);
+    if (form == SCAN_FEW) k_chunk_scan<DELTA, NT, SCAN_FEW><<<grid, SCAN_T(SCAN_FEW), 0, g.stream>>>(a, sc, act, state);
+    else if (form == SCAN_DEEP) k_chunk_scan<DELTA, NT, SCAN_DEEP><<<grid, SCAN_T(SCAN_DEEP), 0, g.stream>>>(a, sc, act, state);
+    else if constexpr (turns) k_chunk_scan<DELTA, NT, SCAN_TURNS><<<grid, SCAN_T(SCAN_TURNS), 0, g.stream>>>(a, sc, act, state);
+  };
   switch (a.cd.Dp / 64u) {
-    case 1: SCAN(1); break;
-    case 2: SCAN(2); break;
-    case 3: SCAN(3); break;
-    case 4: SCAN(4); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
     default: return ADAMAH_ERR_INVALID;
   }
-#undef SCAN
   count_launch();
   return check_launch();
 }

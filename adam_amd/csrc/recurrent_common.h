@@ -12,6 +12,25 @@ namespace adamah {
 #define VC 32u            // value columns of a decode workgroup
 #define NO_MEMORY 110.0f  // exp(-110) is zero in float32: a stronger decay per token changes nothing, and the sums stay small
 
+// Forms of the walk over a portion's chunks (a workgroup: 16 value columns of a head).  FEW and DEEP have four waves of state rows and
+// a fifth that adds up and stores the outputs; FEW asks for a chunk's operands when it needs them, DEEP two chunks ahead.  TURNS: as
+// DEEP without the fifth wave, the four take turns with the outputs.
+enum { SCAN_FEW = 0, SCAN_DEEP = 1, SCAN_TURNS = 2 };
+#define SCAN_T(form) ((form) == SCAN_TURNS ? 256u : 320u)
+// nt: tiles of 16 state rows a wave; two: a second workgroup of DEEP fits a CU (128 registers a lane, 4 waves a SIMD; its five do not go
+// twice into 3); turns: there is such a form.  Up to a workgroup a CU a chunk's latency is all: DEEP, but for one or two chunks, whose operands
+// would arrive no sooner.  Beyond, workgroups hide each other's latency: FEW, of which most fit, while the first loads count, TURNS for
+// longer walks.  us, four waves of which the first has the outputs / FEW / DEEP / TURNS, delta rule, dim 128, 2048 value columns
+// (256 workgroups): 1 chunk 5.8 / 4.8 / 5.4 / 5.9, 4 8.9 / 9.0 / 8.4 / 8.8, 64 71 / 78 / 60 / 68; 8192 columns: 1 12.7 / 9.7 / 15.2 / 11.4, 8 35 / 33 / 41 / 36,
+// 64 219 / 238 / 247 / 221; 192 state rows, 8192 columns: 4 31 / 32 / 38 / 30, 16 78 / 95 / 91 / 77, 64 300 / 389 / 336 / 292; state space, 256 rows,
+// 16384 columns: 4 27 / 29 / 33 / 28, 16 67 / 86 / 83 / 68.  DEEP twice on a CU: state space, 64 rows, 8192 columns, 64 chunks 55 / 55 / 47 / 53.
+static inline int scan_form(uint64_t workgroups, uint32_t chunks, int nt, bool two, bool turns) {
+  const uint64_t cu = (uint64_t)g.n_cu;
+  if (workgroups <= cu) return chunks <= 2u ? SCAN_FEW : SCAN_DEEP;
+  if (two && workgroups <= 2u * cu) return chunks <= 4u ? SCAN_FEW : SCAN_DEEP;
+  return chunks <= (nt <= 2 ? 8u : nt == 3 || !turns ? 4u : 2u) ? SCAN_FEW : turns ? SCAN_TURNS : SCAN_DEEP;
+}
+
 __device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 // silu of the causal convolution at token position p for channel ch, older inputs from the ring only.  The taps' loads do
 // not depend on each other: up to TM of them are asked for at once (TM >= taps).

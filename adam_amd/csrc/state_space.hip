@@ -161,14 +161,13 @@ k_space_prep(const SSpec s, const float* __restrict__ act, const float* __restri
 // Four waves share the state rows (NT tiles of 16 each); a tile's accumulator holds rows 4 g + i of lane group g, which
 // is also how instruction i wants its right operand when the left one is read as four consecutive columns per lane.  Each leaves
 // its rows' part of C S in LDS and its quarter of what the chunk's own part needs; a fifth wave adds up, multiplies and stores, a
-// chunk behind: loads and stores share a counter, and a wave that does both waits for its stores (2048 tokens in
-// 64 heads of 64 by 128, the waves taking turns with the outputs 104 us, so 85).  The order of the sums is that of the other walks (the
-// chunk's own part behind the sum over the waves, in order), and C B times its decay is rounded before the skip is added.
-// FEW: one or two chunks, no operands ahead.
-#define SCAN_T 320u          // four waves of state rows and the one of the outputs
-template <int NT> struct SpaceOps { f4_t c[NT], b[NT], g, u; float cb, m, e, last; };
-template <int NT>
-__device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const float* hb, const SpaceDims& sd, uint32_t wave, uint32_t lane,
+// chunk behind: loads and stores share a counter, and a wave that does both waits for its stores (2048 tokens in 64 heads of 64 by
+// 128, the waves taking turns with the outputs 104 us, so 85; scan_form says where they do all the same).  In every form one product
+// behind the other by wave, the waves' parts as (0 + 1) + (2 + 3) times the decay, the chunk's own part behind that sum in order; C B
+// times its decay is rounded before the skip is added.
+template <int NT, int FORM> struct SpaceOps { f4_t c[NT], b[NT], g, u; std::conditional_t<FORM == SCAN_TURNS, f4_t, float> cb, m, e; float last; };
+template <int NT, int FORM>
+__device__ __forceinline__ void load_ops(SpaceOps<NT, FORM>& o, const float* gb, const float* hb, const SpaceDims& sd, uint32_t wave, uint32_t lane,
                                          uint32_t v0) {
   const float *pB = gb + 16u * sd.Np, *pD = pB + 16u * sd.Np, *pM = hb + 16u * sd.Vp, *pE = pM + 256u, *pG = pE + 16u;
 #pragma unroll
@@ -179,41 +178,45 @@ __device__ __forceinline__ void load_ops(SpaceOps<NT>& o, const float* gb, const
   }
   o.g = *(const f4_t*)(pG + (lane >> 4) * 4u);
   o.u = *(const f4_t*)(hb + v0 * 16u + lane * 4u);
-  o.cb = pD[lane * 4u + wave];
-  o.m = pM[lane * 4u + wave];
-  o.e = pE[(lane >> 4) * 4u + wave];
+  if constexpr (FORM == SCAN_TURNS) {
+    o.cb = *(const f4_t*)(pD + lane * 4u); o.m = *(const f4_t*)(pM + lane * 4u); o.e = *(const f4_t*)(pE + (lane >> 4) * 4u);
+  } else {
+    o.cb = pD[lane * 4u + wave]; o.m = pM[lane * 4u + wave]; o.e = pE[(lane >> 4) * 4u + wave];
+  }
   o.last = pE[15];
 }
 
-template <int NT, bool FEW>
-__global__ void __launch_bounds__(SCAN_T)
+template <int NT, int FORM>
+__global__ void __launch_bounds__(SCAN_T(FORM), FORM == SCAN_TURNS ? 2 : 1)
 k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float* state, SpaceDims sd, uint32_t m, uint32_t seq0, uint32_t pos) {
   __shared__ f4_t pb[2][4][64];                              // [chunk & 1][wave][lane]
-  __shared__ float pc[2][3][4][64];                          // C B and skip, x, decay: a quarter of the four a lane has by each wave
+  __shared__ f4_t pc[2][3][64];                              // C B and skip, x, decay for the fifth wave, one of a lane's four by each wave
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), c = lane & 15u, kg = lane >> 4;
   const uint32_t h = blockIdx.x, v0 = blockIdx.y * 16u, N = s.state, V = s.vdim, v = v0 + c, rep = s.heads / s.groups, grp = h / rep;
   const uint32_t gs = group_floats(sd), hs = head_floats(sd), n = sd.n_chunks;
   state += (uint64_t)seq0 * s.seq_stride;
-  if (wave == 4u) {
-    float* out = act + s.out + h * V + v;
+  float* out = act + s.out + h * V + v;
+  const auto put = [&](uint32_t ci, f4_t cb, f4_t u, f4_t e) {         // the outputs of chunk ci
+    const f4_t (*p)[64] = pb[ci & 1u];
+    f4_t o = ((p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane])) * e;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(cb[i], u[i], o, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t r = ci * CH + 4u * kg + i;
+      if (r < m && v < V) out[(uint64_t)r * s.out_stride] = o[i];
+    }
+  };
+  if (FORM != SCAN_TURNS && wave == 4u) {
     for (uint32_t ci = 0; ci < n; ci++) {
       __syncthreads();
-      const f4_t (*p)[64] = pb[ci & 1u];
-      const float (*q)[4][64] = pc[ci & 1u];
-      f4_t o = ((p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane])) * (f4_t){q[2][0][lane], q[2][1][lane], q[2][2][lane], q[2][3][lane]};
-#pragma unroll
-      for (int i = 0; i < 4; i++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(q[0][i][lane], q[1][i][lane], o, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint32_t r = ci * CH + 4u * kg + i;
-        if (r < m && v < V) out[(uint64_t)r * s.out_stride] = o[i];
-      }
+      put(ci, pc[ci & 1u][0][lane], pc[ci & 1u][1][lane], pc[ci & 1u][2][lane]);
     }
   } else {
     const float* gb = scratch + (uint64_t)grp * n * gs;
     const float* hb = scratch + (uint64_t)s.groups * n * gs + (uint64_t)h * n * hs;
     float* S = state + s.s_off + (uint64_t)h * N * V;
-    const float skip = c == 4u * kg + wave ? act[s.skip + h] : 0.f;      // of this wave's columns of the chunk's own part
+    const float skip = act[s.skip + h];
     f4_t st[NT];
 #pragma unroll
     for (int j = 0; j < NT; j++) st[j] = (f4_t){0, 0, 0, 0};
@@ -229,12 +232,13 @@ k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float
     }
     // The operands of the chunk two ahead, asked for on every path (past the end: the last one's again): under a condition
     // the wait at its end was for everything asked for (162 us for 94).
-    const auto ask = [&](SpaceOps<NT>& o, uint32_t ci) {
+    const auto ask = [&](SpaceOps<NT, FORM>& o, uint32_t ci) {
       const uint64_t at = min(ci, n - 1u);
-      load_ops<NT>(o, gb + at * gs, hb + at * hs, sd, wave, lane, v0);
+      load_ops<NT, FORM>(o, gb + at * gs, hb + at * hs, sd, wave, lane, v0);
       __builtin_amdgcn_sched_barrier(0);
     };
-    const auto chunk = [&](const SpaceOps<NT>& cur, uint32_t x) {
+    const auto chunk = [&](const SpaceOps<NT, FORM>& cur, uint32_t ci) {
+      const uint32_t x = ci & 1u;
       f4_t p = {0, 0, 0, 0};
 #pragma unroll
       for (int j = 0; j < NT; j++)
@@ -247,33 +251,43 @@ k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float
 #pragma unroll
         for (int j = 0; j < NT; j++) st[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.b[j][i], cur.g[i] * cur.u[i], st[j], 0, 0, 0);
       pb[x][wave][lane] = p;
-      pc[x][0][wave][lane] = cur.cb * cur.m + skip;
-      pc[x][1][wave][lane] = wave & 2u ? (wave & 1u ? cur.u[3] : cur.u[2]) : (wave & 1u ? cur.u[1] : cur.u[0]);
-      pc[x][2][wave][lane] = cur.e;
-      __syncthreads();
+      if constexpr (FORM == SCAN_TURNS) {
+        __syncthreads();
+        if (wave == (ci & 3u)) {
+          f4_t cb = cur.cb * cur.m;
+#pragma unroll
+          for (int i = 0; i < 4; i++) cb[i] += c == 4u * kg + i ? skip : 0.f;
+          put(ci, cb, cur.u, cur.e);
+        }
+      } else {
+        ((float*)&pc[x][0][lane])[wave] = cur.cb * cur.m + (c == 4u * kg + wave ? skip : 0.f);
+        ((float*)&pc[x][1][lane])[wave] = wave & 2u ? (wave & 1u ? cur.u[3] : cur.u[2]) : (wave & 1u ? cur.u[1] : cur.u[0]);
+        ((float*)&pc[x][2][lane])[wave] = cur.e;
+        __syncthreads();
+      }
     };
-    SpaceOps<NT> o0;
+    SpaceOps<NT, FORM> o0;
     ask(o0, 0);
-    if constexpr (FEW) {
+    if constexpr (FORM == SCAN_FEW) {
       for (uint32_t ci = 0; ci < n; ci++) {
         if (ci) ask(o0, ci);
-        chunk(o0, ci & 1u);
+        chunk(o0, ci);
       }
     } else {
       // (a loop in one piece: with a way out behind each chunk the loads were moved down to where only the rest of the loop needs them)
-      SpaceOps<NT> o1, o2;
+      SpaceOps<NT, FORM> o1, o2;
       ask(o1, 1); ask(o2, 2);
       uint32_t ci = 0;
       for (; ci + 3u <= n; ci += 3u) {
-        chunk(o0, ci & 1u);
+        chunk(o0, ci);
         ask(o0, ci + 3u);
-        chunk(o1, (ci + 1u) & 1u);
+        chunk(o1, ci + 1u);
         ask(o1, ci + 4u);
-        chunk(o2, ci & 1u);
+        chunk(o2, ci + 2u);
         ask(o2, ci + 5u);
       }
-      if (ci < n) chunk(o0, ci & 1u);
-      if (ci + 1u < n) chunk(o1, (ci + 1u) & 1u);
+      if (ci < n) chunk(o0, ci);
+      if (ci + 1u < n) chunk(o1, ci + 1u);
     }
 #pragma unroll
     for (int j = 0; j < NT; j++)
@@ -288,7 +302,7 @@ k_space_scan(const SSpec s, const float* __restrict__ scratch, float* act, float
     float* slot = state + s.conv_off + (uint64_t)((pos + r) % s.taps) * n_ch;
     const float* x = act + s.x + s.x_c + (uint64_t)r * s.x_stride;
     if (blockIdx.y == 0 && h % rep == 0)
-      for (uint32_t d = tid; d < N; d += SCAN_T) {
+      for (uint32_t d = tid; d < N; d += SCAN_T(FORM)) {
         const uint32_t b = inner + grp * N + d, cc = inner + (s.groups + grp) * N + d;
         slot[b] = x[b];
         slot[cc] = x[cc];
@@ -338,16 +352,19 @@ extern "C" int adamah_state_space_dev(uint32_t map_act, uint32_t h_spec, uint32_
   count_launch();
   if (int r = check_launch()) return r;
   const dim3 grid((uint32_t)H, cdiv(V, 16));
-  const bool few = sd.n_chunks <= 2u;
-#define SCAN(NT) do { if (few) k_space_scan<NT, true><<<grid, SCAN_T, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); \
-                      else k_space_scan<NT, false><<<grid, SCAN_T, 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos); } while (0)
+  const auto go = [&](auto tiles) {
+    constexpr int NT = decltype(tiles)::value;
+    const int form = scan_form((uint64_t)grid.x * grid.y, sd.n_chunks, NT, NT <= 2, true);
+    if (form == SCAN_FEW) k_space_scan<NT, SCAN_FEW><<<grid, SCAN_T(SCAN_FEW), 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos);
+    else if (form == SCAN_DEEP) k_space_scan<NT, SCAN_DEEP><<<grid, SCAN_T(SCAN_DEEP), 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos);
+    else k_space_scan<NT, SCAN_TURNS><<<grid, SCAN_T(SCAN_TURNS), 0, g.stream>>>(*s, sc, act, state, sd, rows, seq0, pos);
+  };
   switch (sd.Np / 64u) {
-    case 1: SCAN(1); break;
-    case 2: SCAN(2); break;
-    case 3: SCAN(3); break;
-    default: SCAN(4); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    default: go(std::integral_constant<int, 4>{}); break;
   }
-#undef SCAN
   count_launch();
   return check_launch();
 }
