@@ -178,7 +178,7 @@ _SIGS = {
     # timing helpers for benchmarks (HIP events on the library's own stream)
     "adamah_hip_timer_begin": (i32, []), "adamah_hip_timer_end": (f32c, []),
     "adamah_hip_debug_dequant": (i32, [_U, u64, u64, pf32]),
-    "adamah_hip_map_layout": (i32, [_U]),
+    "adamah_hip_map_layout": (i32, [_U]), "adamah_hip_matmul_plan": (i32, [_U, _U, _U, u64, pu32, pu32]),
     "adamah_hip_stream_probe": (f32c, [u64, u64, _U, _U, _U]),
 }
 
@@ -841,6 +841,14 @@ class Adamah:
     def map_layout(self, map_id):
         """0 = generic affine qparams, 1 = fp16-scale block plane (Q4_0 / Q8_0 recognised)."""
         return int(self._lib.adamah_hip_map_layout(map_id))
+
+    def matmul_plan(self, rows, k, n, base=0):
+        """(activation rows a workgroup of the ring kernel or 0 for the tiled one, shares of K) of a Q4 matmul of more than 64 rows."""
+        tile, shares = ctypes.c_uint32(), ctypes.c_uint32()
+        ret = self._lib.adamah_hip_matmul_plan(rows, k, n, base, ctypes.byref(tile), ctypes.byref(shares))
+        if ret != 0:
+            raise RuntimeError(f"adamah_hip_matmul_plan failed with code {ret}")
+        return tile.value, shares.value
 
     # ---- misc ------------------------------------------------------------------------
     def reset_metrics(self):

@@ -1608,3 +1608,13 @@ void gemm_q4_mfma_release() {
 }
 
 }  // namespace adamah
+
+using namespace adamah;
+extern "C" int adamah_hip_matmul_plan(uint32_t rows, uint32_t k, uint32_t n, uint64_t base, uint32_t* tile, uint32_t* shares) {
+  if (g.n_cu <= 0 || rows <= 64u || k == 0u || (k & 127u) || n == 0u || (base & 31u) || !tile || !shares) return ADAMAH_ERR_INVALID;
+  const GemmPlan p = gemm_plan(rows, k, n, (int64_t)base);
+  const uint32_t units = p.ma ? k >> 6 : cdiv(k, 128), per = cdiv(units, p.shares);      // (of the ring 64 columns, of the tiled kernel 128)
+  *tile = 32u * (uint32_t)p.ma;
+  *shares = cdiv(units, per);
+  return ADAMAH_OK;
+}

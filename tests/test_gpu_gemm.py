@@ -311,12 +311,15 @@ def test_residual_add_stored_by_the_matmul(hip, M, K, N, in_place):
         assert rel_l2(fused[d0:d0 + M * N].reshape(M, N), y + hid) < TOL
 
 
-@pytest.mark.parametrize("M,N,K,off,d_off,twice", [(70, 512, 14336, 0, 0, False), (130, 1024, 8192, 0, 2, False), (300, 1536, 6912, 1, 0, False),
-                                                   (487, 4096, 4096, 0, 0, True), (512, 6144, 4096, 0, 0, False), (257, 1025, 4096, 0, 0, False)])
-def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice):
+@pytest.mark.parametrize("M,N,K,off,d_off,twice,shares", [
+    (70, 512, 14336, 0, 0, False, 16), (130, 1024, 8192, 0, 2, False, 16), (300, 1536, 6912, 1, 0, False, 16), (487, 4096, 4096, 0, 0, True, 4),
+    (512, 6144, 4096, 0, 0, False, 5), (257, 1025, 4096, 0, 0, False, 16), (341, 9000, 2048, 0, 0, False, 2), (341, 6144, 2048, 1, 0, False, 3),
+    (341, 4096, 2304, 0, 1, False, 5), (130, 6144, 2304, 0, 0, True, 6), (130, 6144, 2048, 0, 2, False, 7), (70, 512, 2048, 3, 0, False, 8)])
+def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice, shares):
     """Two shares of K to more than eight, results and residual on 16 bytes and off them, the result added to itself: every sum is the
     stored product plus the residual."""
     note(f"sums of shares M={M} K={K} N={N} off={off} {d_off} twice={twice}")
+    assert hip.matmul_plan(M, K, N)[1] == shares
     rng = np.random.default_rng(M + N)
     qt = quant.quantize_q4_0(rng.standard_normal((N, K), dtype=np.float32) * np.float32(0.05))
     x = rng.standard_normal((M, K), dtype=np.float32)
@@ -537,14 +540,17 @@ def test_weights_from_an_odd_block_run_over_shares_of_k(hip, M, K, N):
     assert rel_l2(read(hip, 0, h0, M * N).reshape(M, N), y + hid) < TOL_Q4
 
 
-@pytest.mark.parametrize("M,K,Ns,add", [
-    (600, 256, (7200, 7230), False), (513, 256, (100, 14000, 333), False), (65, 128, (500, 36, 700), False), (130, 512, (512, 512), False),
-    (600, 256, (14401,), True), (341, 1152, (13824,), True), (70, 384, (515,), True)])
-def test_ring_stores_stacked_results_and_adds_in_one_share(hip, monkeypatch, M, K, Ns, add):
+@pytest.mark.parametrize("M,K,Ns,add,tile", [
+    (600, 256, (7200, 7230), False, 96), (513, 256, (100, 14000, 333), False, 96), (65, 128, (500, 36, 700), False, 64),
+    (130, 512, (512, 512), False, 64), (600, 256, (14401,), True, 96), (341, 1152, (13824,), True, 64), (70, 384, (515,), True, 64),
+    (512, 512, (15800, 15944), False, 128), (385, 256, (31700,), True, 128), (500, 640, (100, 31000, 600), False, 128), (512, 384, (31744,), True, 128)])
+def test_ring_stores_stacked_results_and_adds_in_one_share(hip, monkeypatch, M, K, Ns, add, tile):
     """The ring kernel's own stores (two launches with the conversion: no sum behind it): results of stacked matrices whose border
-    lies inside a workgroup's 512 weight rows, and the add behind a single one; 64 and 128 activation rows a workgroup."""
+    lies inside a workgroup's 512 weight rows, and the add behind a single one; 64, 96 and 128 activation rows a workgroup, scales by the step and
+    by four steps."""
     monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
     monkeypatch.setenv("ADAMAH_GEMM_SPLITK", "0")
+    assert hip.matmul_plan(M, K, sum(Ns)) == (tile, 1)
     note(f"gemm q4 ring, one share M={M} K={K} Ns={Ns} add={add}")
     rng = np.random.default_rng(M + sum(Ns))
     W = load_from(hip, rng, sum(Ns), K, 0)
@@ -580,7 +586,8 @@ def test_ring_stores_stacked_results_and_adds_in_one_share(hip, monkeypatch, M, 
 
 @pytest.mark.parametrize("split", ["0", "1"])
 @pytest.mark.parametrize("M,N,K,base", [(1000, 3201, 128, 0), (777, 4100, 256, 64), (2049, 1537, 384, 64), (65, 515, 128, 0), (129, 511, 14336, 0),
-                                        (300, 9000, 640, 128)])
+                                        (300, 9000, 640, 128), (96, 28001, 1024, 0), (341, 9000, 2048, 128), (777, 4100, 256, 256), (1000, 3201, 512, 512),
+                                        (341, 4100, 3328, 0)])
 def test_ring_at_ragged_ends(hip, monkeypatch, M, N, K, base, split):
     """The ring kernel where the rule would not take it as well: fewer steps of K than it has stages, rows and weight rows past the
     last tile, shares of unequal length."""
@@ -589,13 +596,15 @@ def test_ring_at_ragged_ends(hip, monkeypatch, M, N, K, base, split):
     test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
 
 
-@pytest.mark.parametrize("M,N,K,base,split", [(288, 35837, 128, 0, "0"), (257, 35840, 384, 64, "0"), (96, 28001, 1024, 0, "1"), (341, 9000, 2048, 128, "1"),
-                                                (777, 4100, 256, 256, "0"), (1000, 3201, 512, 512, "1"), (341, 4100, 3328, 0, "1")])
-def test_ring_of_96_rows(hip, monkeypatch, M, N, K, base, split):
-    """Sizes at which 96 activation rows a workgroup fill the CUs in one round and 64 or 128 do not, ragged in both directions; scales of one
-    run of 256 columns and of several, shares that begin inside a run."""
+@pytest.mark.parametrize("M,N,K,base,split,shares", [
+    (288, 35837, 128, 0, "0", 1), (257, 35840, 384, 64, "0", 1), (600, 14401, 512, 0, "0", 1), (600, 14401, 1280, 256, "0", 1), (288, 9000, 1280, 0, "1", 4),
+    (288, 9000, 1280, 64, "1", 4), (96, 9000, 3328, 512, "1", 13), (280, 7000, 2304, 0, "1", 6), (341, 6144, 4096, 0, "1", 5)])
+def test_ring_of_96_rows(hip, monkeypatch, M, N, K, base, split, shares):
+    """Sizes at which the rule takes 96 activation rows a workgroup, ragged in both directions; scales by the step, of one run of 256 columns
+    and of several, shares that begin inside a run."""
     monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
     monkeypatch.setenv("ADAMAH_GEMM_SPLITK", split)
+    assert hip.matmul_plan(M, K, N, base) == (96, shares)
     test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
 
 
