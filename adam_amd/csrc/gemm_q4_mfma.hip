@@ -1364,14 +1364,16 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // 28672 x 4096 71.9 and 67.7).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
 // a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x
 // 2048: 23 -> 17 over four; 64 x 28672 x 2048 38 in one, 44 in four, 64 x 28672 x 4096 67 and 62).
-// More: the least of these estimates, in us, fitted to both kernels over 2900 plans of 65 .. 2049 rows by 512 .. 32000 x 128 ..
-// 14336 (the plan it picks takes 0.2 % longer than the best one in the mean, 9 % at most; 12 % for 128 x 32000 x 2048, where the
-// tiled kernel over two shares, which it does not ask for, takes 60 us and one launch 67).  Tiled, by the tile it would take
+// More: the least of these estimates, in us.  Over 360 products of 65 .. 2049 rows by 512 .. 32000 x 128 .. 14336 the plan it picks takes
+// 0.9 % longer than the best one in the mean where N is a multiple of four (15 % at most, 357 rows of 10092 x 1536: 53 us tiled,
+// 46 over two shares), else 1.2 % (20 %, 134 rows of 3575 x 9344: 66 us over 12 shares, 55 over 9).  Tiled, by the tile it would take
 // (below): 128-column steps of 1.27 us while no CU has a second 64 x 64 tile and 0.72 more for each further one, 4.0 and 2.7
 // more for every two rounds of 64 x 128, 4.6 a round of 256 x 128.  Ring: 64-column steps of 1.7 (ma = 2), 2.35 (3) or 3.0 us (4), up to a
-// quarter more as the CUs fill; shares cost their second launch and a pass over the sums each.  (us, conversion included, without
-// and with 96 rows a workgroup: 28672 x 4096 under 96 rows 88 and 76, 150 129 and 114, 192 129 and 118, 288 231 and 184, 384 241 and
-// 212; 4096 x 14336 288 116 and 105, 384 139 and 128; 6144 x 4096 480 90 and 83.)
+// quarter more as the CUs fill; shares cost their second launch and a pass over the sums each, where N is no multiple of four two and a
+// half (a result at a time, one share behind the other: 88 rows of 9007 x 5760 57 us over 7 shares of 64 rows a workgroup, 65 over
+// 13 of 96, of 9008 x 5760 50 and 48; 730 of 559 x 11904 69 over 10, 81 over 16, of 560 61 and 63).  (us, conversion included, without and
+// with 96 rows a workgroup: 28672 x 4096 under 96 rows 88 and 76, 150 129 and 114, 192 129 and 118, 288 231 and 184, 384 241 and 212;
+// 4096 x 14336 288 116 and 105, 384 139 and 128; 6144 x 4096 480 90 and 83.)
 // The ring reads the scales of two blocks as one word and keeps a lane's place in the rows in 32 bits (in the matrix too: a Q4
 // map here has fewer than 2^32 elements): matrices that begin at an odd block stay on the tiled kernel, a narrow one from 128
 // rows on over 2 .. 4 shares (256 x 128 tile; 512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four).
@@ -1409,7 +1411,8 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     const uint64_t tiles = wgs(512, 32 * (uint64_t)ma);
     for (uint64_t sp = 1; sp <= most && (sp == 1 || (sp * 4 <= pairs && tiles * sp <= cu)); sp++) {
       const double full = std::min(1.0, (double)(tiles * sp) / (double)cu), step = ma == 2 ? 1.7 + 0.35 * full : ma == 3 ? 2.35 + 0.6 * full : 3.0 + 0.8 * full;
-      const double us = (double)up(tiles * sp, cu) * ((double)up(pairs, sp) * step + 7.0) + (sp > 1 ? 9.0 + (double)(sp + 1) * pass : 0.0);
+      const double sums = sp == 1 ? 0.0 : N % 4 == 0 ? 9.0 + (double)(sp + 1) * pass : 7.0 + (2.5 * (double)sp - 3.0) * pass;
+      const double us = (double)up(tiles * sp, cu) * ((double)up(pairs, sp) * step + 7.0) + sums;
       if (us < best) { best = us; p = {ma, (uint32_t)sp}; }
     }
   }

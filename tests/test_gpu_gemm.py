@@ -313,7 +313,7 @@ def test_residual_add_stored_by_the_matmul(hip, M, K, N, in_place):
 
 @pytest.mark.parametrize("M,N,K,off,d_off,twice,shares", [
     (70, 512, 14336, 0, 0, False, 16), (130, 1024, 8192, 0, 2, False, 16), (300, 1536, 6912, 1, 0, False, 16), (487, 4096, 4096, 0, 0, True, 4),
-    (512, 6144, 4096, 0, 0, False, 5), (257, 1025, 4096, 0, 0, False, 16), (341, 9000, 2048, 0, 0, False, 2), (341, 6144, 2048, 1, 0, False, 3),
+    (512, 6144, 4096, 0, 0, False, 5), (257, 1025, 4096, 0, 0, False, 13), (341, 9000, 2048, 0, 0, False, 2), (341, 6144, 2048, 1, 0, False, 3),
     (341, 4096, 2304, 0, 1, False, 5), (130, 6144, 2304, 0, 0, True, 6), (130, 6144, 2048, 0, 2, False, 7), (70, 512, 2048, 3, 0, False, 8)])
 def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice, shares):
     """Two shares of K to more than eight, results and residual on 16 bytes and off them, the result added to itself: every sum is the
@@ -343,6 +343,12 @@ def test_sums_of_shares_on_and_off_a_line(hip, M, N, K, off, d_off, twice, share
     assert np.array_equal(got[d0:d0 + M * N], y + (y if twice else hid.reshape(-1)))
     got[y0:y0 + M * N] = got[d0:d0 + M * N] = 0
     assert np.array_equal(got, old)                # nothing beside the results
+
+
+@pytest.mark.parametrize("M,N,K", [(88, 9007, 5760), (541, 2606, 4480), (730, 559, 11904), (70, 10865, 2304)])
+def test_sums_of_single_results_are_planned_as_dear(hip, M, N, K):
+    """A row that is no multiple of four results long is added up a result at a time: fewer shares than of the next length that is one."""
+    assert hip.matmul_plan(M, K, N)[1] < hip.matmul_plan(M, K, (N + 3) // 4 * 4)[1]
 
 
 @pytest.mark.parametrize("op,M,K,N,in_place", [("swiglu", 16, 14336, 96, False), ("geglu", 5, 6912, 64, False), ("swiglu", 40, 256, 50, False),
