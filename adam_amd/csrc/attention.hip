@@ -21,15 +21,6 @@ namespace adamah {
 __device__ __forceinline__ float ld(const float* p, uint64_t i) { return p[i]; }
 __device__ __forceinline__ float ld(const __half* p, uint64_t i) { return __half2float(p[i]); }
 
-__device__ __forceinline__ float wave_sum64(float v) {
-  v = wave_add(v);
-  return v;
-}
-__device__ __forceinline__ float wave_max64(float v) {
-  v = wave_max(v);
-  return v;
-}
-
 // C[M,N] = A[M,K] . B[N,K]^T per op; one wave per output column, lanes over K.
 // B is read through `bsrc` (float map or fp16 KV copy, index = element - b_shift).
 template <typename TB>
@@ -45,7 +36,7 @@ k_matmul_t(const float* A, float* C, const TB* bsrc, uint64_t b_shift, const uin
   float s = 0.f;
   if (a + K <= a_elems && b >= b_shift && b - b_shift + K <= b_elems)
     for (uint32_t k = lane; k < K; k += 64u) s = fmaf(A[a + k], ld(bsrc, b - b_shift + k), s);
-  s = wave_sum64(s);
+  s = wave_add(s);
   if (lane == 0 && c < a_elems) C[c] = s;
 }
 
@@ -114,7 +105,7 @@ k_matmul_nt(const float* A, float* C, const float* B, const uint32_t* __restrict
     const uint64_t bi = b + (uint64_t)k * N + col;
     if (a + k < a_elems && bi < b_elems) s = fmaf(A[a + k], B[bi], s);
   }
-  s = wave_sum64(s);
+  s = wave_add(s);
   if (lane == 0 && c < a_elems) C[c] = s;
 }
 
@@ -146,7 +137,7 @@ k_attn_softmax_value(const float* data, float* out, const TV* vsrc, uint64_t v_s
       p[t] = v;
       mx = fmaxf(mx, v);
     }
-  mx = wave_max64(mx);
+  mx = wave_max(mx);
   if (lane == 0) red[wave] = mx;
   __syncthreads();
   mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -159,7 +150,7 @@ k_attn_softmax_value(const float* data, float* out, const TV* vsrc, uint64_t v_s
       p[t] = e;
       sum += e;
     }
-  sum = wave_sum64(sum);
+  sum = wave_add(sum);
   if (lane == 0) red[wave] = sum;
   __syncthreads();
   sum = (red[0] + red[1]) + (red[2] + red[3]);
@@ -363,7 +354,7 @@ k_attn_fused(const float* data, float* out, const __half* kv, uint64_t kv_shift,
     p[t] = v;
     mx = fmaxf(mx, v);
   }
-  mx = wave_max64(mx);
+  mx = wave_max(mx);
   if (lane == 0) red[wave] = mx;
   __syncthreads();
   mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -374,7 +365,7 @@ k_attn_fused(const float* data, float* out, const __half* kv, uint64_t kv_shift,
     p[t] = e;
     sum += e;
   }
-  sum = wave_sum64(sum);
+  sum = wave_add(sum);
   if (lane == 0) red[wave] = sum;
   __syncthreads();
   sum = (red[0] + red[1]) + (red[2] + red[3]);
@@ -457,9 +448,9 @@ k_attn_combine(float* out, const float* partial, const uint32_t* __restrict__ lo
     for (uint32_t k = 0; k < 8u; k++) v[k] = pp[(uint64_t)min(sg + 8u * k, last) * stride + 2 + dc];
     const float qv = (q_n ? q_src : partial)[q_n ? min(gi, q_n - 1u) : 0u];   // (a load on every path)
     const uint64_t ob = lo[op];
-    const float M = wave_max64(lane < n_splits ? m_own : -9.99999968e+37f);
+    const float M = wave_max(lane < n_splits ? m_own : -9.99999968e+37f);
     const float e = lane < n_splits ? expf(m_own - M) : 0.f;
-    const float invL = 1.0f / wave_sum64(lane < n_splits ? fmaf(l_own, e, 0.f) : 0.f);
+    const float invL = 1.0f / wave_add(lane < n_splits ? fmaf(l_own, e, 0.f) : 0.f);
     float o0 = 0.f, o1 = 0.f;
 #pragma unroll
     for (uint32_t k = 0; k < 4u; k++) {
@@ -487,7 +478,7 @@ k_attn_combine(float* out, const float* partial, const uint32_t* __restrict__ lo
   if (ob + value_dim > n_elems) return;
   float M = -9.99999968e+37f;
   for (uint32_t s = tid; s < n_splits; s += 256u) M = fmaxf(M, pp[(uint64_t)s * stride]);
-  M = wave_max64(M);
+  M = wave_max(M);
   if (lane == 0) red[wave] = M;
   __syncthreads();
   M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -498,7 +489,7 @@ k_attn_combine(float* out, const float* partial, const uint32_t* __restrict__ lo
     w[s] = e;
     L = fmaf(pp[(uint64_t)s * stride + 1], e, L);
   }
-  L = wave_sum64(L);
+  L = wave_add(L);
   if (lane == 0) red[wave] = L;
   __syncthreads();
   const float invL = 1.0f / ((red[0] + red[1]) + (red[2] + red[3]));
@@ -534,14 +525,14 @@ k_softmax_rows(float* data, const uint32_t* __restrict__ ls, const uint32_t* __r
   if (sb + row_size > n_elems || db + row_size > n_elems) return;
   float mx = -9.99999968e+37f;
   for (uint32_t i = tid; i < row_size; i += 256u) mx = fmaxf(mx, prep(data[sb + i], scale, cap));
-  mx = wave_max64(mx);
+  mx = wave_max(mx);
   if (lane == 0) red[wave] = mx;
   __syncthreads();
   mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
   __syncthreads();
   float sum = 0.f;
   for (uint32_t i = tid; i < row_size; i += 256u) sum += expf(prep(data[sb + i], scale, cap) - mx);
-  sum = wave_sum64(sum);
+  sum = wave_add(sum);
   if (lane == 0) red[wave] = sum;
   __syncthreads();
   sum = (red[0] + red[1]) + (red[2] + red[3]);

@@ -51,8 +51,8 @@ k_gateup_act(float* act, const uint8_t* __restrict__ W, const float2* __restrict
     if (bg + k < wt_elems) sg = fmaf(x, deq_elem(W, qp, bg + k, group, Q4), sg);
     if (bu + k < wt_elems) su = fmaf(x, deq_elem(W, qp, bu + k, group, Q4), su);
   }
-  sg = wave_sum(sg);
-  su = wave_sum(su);
+  sg = wave_add(sg);
+  su = wave_add(su);
   const uint64_t c = (uint64_t)lco[0] + row;
   if (lane == 0 && c < act_elems) act[c] = (sg / (1.0f + expf(-sg))) * su;
 }

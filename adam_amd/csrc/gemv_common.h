@@ -18,11 +18,6 @@ __device__ __forceinline__ bool better(float cv, uint32_t ci, float bv, uint32_t
   return (cv > bv) || ((cv == bv) && (ci < bi));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-  v = wave_add(v);
-  return v;
-}
-
 // byte n of a 32-bit register -> float, one VALU op
 template <int N> __device__ __forceinline__ float ubyte_f32(uint32_t w) {
   float r;

@@ -328,7 +328,7 @@ k_matmul_xq_generic(const float* act, float* out, const uint8_t* __restrict__ W,
     const uint64_t wi = TRANSPOSED ? b + (uint64_t)col * K + k : b + (uint64_t)k * N + col;
     if (a + k < act_elems && wi < wt_elems) s = fmaf(act[a + k], deq_elem(W, qp, wi, group, Q4), s);
   }
-  s = wave_sum(s);
+  s = wave_add(s);
   if (lane == 0 && c < act_elems) out[c] = s;
 }
 
@@ -350,7 +350,7 @@ k_matvec_argmax_generic(const float* act, float* out, const uint8_t* __restrict_
       const uint64_t wi = b + (uint64_t)r * K + k;
       if (a + k < act_elems && wi < wt_elems) s = fmaf(act[a + k], deq_elem(W, qp, wi, group, Q4), s);
     }
-    s = wave_sum(s);
+    s = wave_add(s);
     if (better(s, r, bv, bi)) { bv = s; bi = r; }
   }
   if (lane == 0) { red_v[wave] = bv; red_i[wave] = bi; }

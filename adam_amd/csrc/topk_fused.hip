@@ -68,7 +68,7 @@ k_matvec_rows(const float* act, const uint8_t* __restrict__ W, const float2* __r
   float s = 0.f;
   for (uint32_t k = lane; k < K; k += 64u)
     if (a + k < act_elems && b + k < wt_elems) s = fmaf(act[a + k], deq_elem(W, qp, b + k, group, Q4), s);
-  s = wave_sum(s);
+  s = wave_add(s);
   if (lane == 0) out[row] = s;
 }
 
@@ -203,7 +203,7 @@ k_rerank_q8(float* act, const uint8_t* __restrict__ W, const float2* __restrict_
   float s = 0.f;
   for (uint32_t k = lane; k < K; k += 64u)
     if (a + k < act_elems && b + k < wt_elems) s = fmaf(act[a + k], deq_elem(W, qp, b + k, group, false), s);
-  s = wave_sum(s);
+  s = wave_add(s);
   if (lane == 0) {
     bool hit = false;
     for (uint32_t i = 0; i < n_pen; i++) hit = hit || pen[i] == tok;
