@@ -1090,12 +1090,16 @@ static int launch_tiles(const bf16_t* W, const bf16_t* X, float* act, T* op, con
   return check_launch();
 }
 
-// A few workgroups more than CUs would each read and norm x first, on a CU that another one keeps busy: where x is normed, some waves
-// take a second task instead, whose weights are asked for under the products of the first (2066 pairs of 2048, branched: 259 workgroups
-// 8.7 us, so 8.1; 4600 x 4096 behind a norm 12.0 and 11.4.  Without one 4200 x 2048 6.75 and 6.85).
+// A few workgroups more than CUs would each read and norm x first, on a CU that another one keeps busy: where x is normed and rows have 1024
+// to 4096 columns, some waves take a second task instead, whose weights are asked for under the products of the first.  us, 264 to 288
+// workgroups and 256 of them: behind a norm 1024 columns 6.1 and 5.6, 2048 8.3 and 7.95, 3072 11.0 and 9.9, 4096 11.95 and 11.65; behind a branch 6.3 and
+// 5.8, 8.65 and 8.2, 11.5 and 10.5, 12.55 and 12.1; 2066 pairs of 2048, branched, 8.7 and 7.7.  Without a norm nothing waits (2048 columns 6.9 and 7.0); a
+// short row's second task is a trip to memory that nothing hides (768 columns behind a norm 5.3 and 6.0); of a longer row, which a branch
+// does not find in registers any more, a task is most of a wave's time (7168 columns behind a norm 17.7 and 18.2, behind a branch 22.6 and 23.6).
 static uint32_t gemv_grid(const LinSpec& s, uint32_t n_tasks) {
   const uint32_t grid = cdiv(n_tasks, 8), cu = (uint32_t)g.n_cu;
-  return (s.groups || s.branched) && grid > cu && grid <= cu + cu / 8u ? cu : std::min(grid, 2u * cu);
+  const bool once = (s.groups || s.branched) && s.k_stride >= 1024u && s.k_stride <= 4096u;
+  return once && grid > cu && grid <= cu + cu / 8u ? cu : std::min(grid, 2u * cu);
 }
 
 // tasks of two rows (pairs of gate / up ahead of the tail's)

@@ -251,6 +251,45 @@ def test_a_wide_product_does_not_hang_on_its_width(hip, rows, k):
         assert np.array_equal(y[:, :w].view(np.uint32), got[0][:, :w].view(np.uint32)), w
 
 
+# ---- products of one row -------------------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("k", [960, 1024, 2100, 4096, 4160])
+@pytest.mark.parametrize("kind", ["norm", "branch", "pairs"])
+def test_one_row_does_not_hang_on_the_workgroups(hip, kind, k):
+    """A few workgroups beyond one a compute unit, more of them, and none: what a matrix row gives is the same word, whether its wave has it
+    as its first task or its second."""
+    note(f"words of one row, {kind} k {k}")
+    rng = np.random.default_rng(k)
+    ks = (k + 63) // 64 * 64
+    widths = [2 * 8 * w for w in (300, 290, 288, 264, 258, 256, 140)]          # rows: two a wave, eight waves
+    n = widths[0]
+    at, end = places(4, x=k, wt=k, b=k, bw=k, res=k, out=n)
+    W = f32_to_bf16(rng.standard_normal((n, ks), dtype=np.float32))
+    W[:, k:] = 0
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, n * ks)
+    hip.scatter_contiguous(WT, 0, W.reshape(-1))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, ks)
+    f32map(hip, WS, end, rng.standard_normal(end, dtype=np.float32))
+    got = []
+    for w in widths:
+        spec = dict(w=0, n=w, k=k, k_stride=ks, src=at["x"], src_stride=k, groups=1, eps=1e-5, wt=at["wt"], wt_len=k, opnd=0, out=at["out"], out_stride=w)
+        if kind != "norm":
+            spec.update(branched=2, branch=at["b"], branch_stride=k, branch_wt=at["bw"], res_out=at["res"], res_stride=k)
+        if kind == "pairs":
+            spec.update(epi=2, out_opnd=0, out_opnd_stride=w // 2)
+        hip.linear_dev(WS, OP, WT, up(hip, A.LinearSpec(**spec).words()), 0, 1)
+        got.append(read(hip, WS, at["out"], w // 2 if kind == "pairs" else w))
+    x, b, bw, wt = (read(hip, WS, at[name], k).astype(np.float64) for name in ("x", "b", "bw", "wt"))
+    if kind != "norm":
+        x = x + b / np.sqrt(np.mean(b * b) + 1e-5) * bw
+    y = (W.astype(np.uint32) << 16).view(np.float32)[:, :k].astype(np.float64) @ (x / np.sqrt(np.mean(x * x) + 1e-5) * wt)
+    if kind == "pairs":
+        g, u = y.reshape(-1, 2, 16).transpose(1, 0, 2).reshape(2, -1)
+        y = g / (1 + np.exp(-g)) * u
+    assert np.linalg.norm(got[0] - y) < 1e-5 * np.linalg.norm(y)               # sums of k terms in float32, by 64 lanes: about 1e-6
+    for w, v in zip(widths[1:], got[1:]):
+        assert np.array_equal(v.view(np.uint32), got[0][:len(v)].view(np.uint32)), w
+
+
 # ---- one row through the experts -----------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("E,I,top,ff,shared,width,epi", [(4, 0, 4, 1024, 2048, 300, 0), (3, 1, 4, 1000, 2500, 2070, 1), (2, 2, 4, 512, 0, 70, 0),
                                                          (7, 1, 8, 576, 2048, 33, 1), (4, 4, 2, 448, 2112, 50, 0), (1, 1, 2, 2048, 4096, 4200, 0),
