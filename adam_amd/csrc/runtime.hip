@@ -885,6 +885,7 @@ static int replay_plan(uint32_t plan_id, uint32_t pos, uint32_t seq_len) {
 #define PLAN_EXECS 3
 struct PlanGraph {
   hipGraphExec_t exec[PLAN_EXECS] = {nullptr, nullptr, nullptr};
+  uint32_t exec_nodes[PLAN_EXECS] = {0, 0, 0};
   hipEvent_t done[PLAN_EXECS] = {nullptr, nullptr, nullptr};   // recorded behind the last launch of exec[i]
   bool launched[PLAN_EXECS] = {false, false, false};
   int cur = 0;               // exec[cur] holds the recorded step when ready
@@ -899,6 +900,44 @@ struct PlanGraph {
 };
 static PlanGraph g_pg[MAX_PLANS];
 
+// An executable graph is never destroyed.  Its kernels' arguments lie in device memory of the runtime's, and where that memory had been
+// freed, what is allocated later has now and then held wrong values: of 1750 library contexts made behind one that had used graphs, 17
+// had one decode step off by about 1e-3 of a layer's output in their second or third pass; of 948 without the free none, nor 5000
+// passes of a process's first context.  What no plan holds any more waits here and serves the next plan with as many launches (an
+// update, where it had been an instantiation); with PARKED_MOST of them waiting, a plan that none of them fits is replayed the
+// ordinary way.
+#define PARKED_MOST 256u
+#define PARKED_TRIES 8             // an update that does not fit costs as much as one that does
+struct Parked { hipGraphExec_t exec; uint32_t n_nodes; };
+static std::vector<Parked> g_parked;
+
+static void plan_graph_park(PlanGraph& pg, int slot) {       // (its last launch has finished)
+  if (pg.exec[slot]) g_parked.push_back({pg.exec[slot], pg.exec_nodes[slot]});
+  pg.exec[slot] = nullptr;
+}
+
+static bool graph_update(hipGraphExec_t exec, hipGraph_t graph) {
+  hipGraphNode_t bad = nullptr;
+  hipGraphExecUpdateResult res;
+  if (hipGraphExecUpdate(exec, graph, &bad, &res) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+// A parked graph with this one's launches and arguments, or nullptr
+static hipGraphExec_t plan_graph_unpark(hipGraph_t graph, uint32_t n_nodes) {
+  int tries = 0;
+  for (size_t i = g_parked.size(); i-- > 0 && tries < PARKED_TRIES;) {
+    if (g_parked[i].n_nodes != n_nodes) continue;
+    tries++;
+    const hipGraphExec_t exec = g_parked[i].exec;
+    if (!graph_update(exec, graph)) continue;
+    g_parked.erase(g_parked.begin() + (long)i);
+    return exec;
+  }
+  return nullptr;
+}
+
 static bool plan_graphs_on() {
   const char* e = getenv("ADAMAH_PLAN_GRAPH");
   return !(e && e[0] == '0');
@@ -908,8 +947,7 @@ static void plan_graph_drop(PlanGraph& pg, bool for_good) {
   for (int i = 0; i < PLAN_EXECS; i++) {
     if (pg.launched[i] && pg.done[i]) hipEventSynchronize(pg.done[i]);
     pg.launched[i] = false;
-    if (pg.exec[i]) hipGraphExecDestroy(pg.exec[i]);
-    pg.exec[i] = nullptr;
+    plan_graph_park(pg, i);
   }
   pg.ready = false;
   if (for_good) pg.disabled = true;
@@ -951,24 +989,20 @@ static void plan_graph_record(uint32_t plan_id, uint32_t pos, uint32_t seq_len) 
     hipEventSynchronize(pg.done[slot]);
     pg.launched[slot] = false;
   }
-  if (pg.exec[slot]) {
-    hipGraphNode_t bad = nullptr;
-    hipGraphExecUpdateResult res;
-    if (hipGraphExecUpdate(pg.exec[slot], graph, &bad, &res) != hipSuccess) {   // another launch shape (e.g. one more slice)
+  if (pg.exec[slot] && !graph_update(pg.exec[slot], graph)) plan_graph_park(pg, slot);      // another launch shape (e.g. one more slice)
+  if (!pg.exec[slot]) pg.exec[slot] = plan_graph_unpark(graph, n_nodes);
+  if (pg.exec[slot]) pg.n_update++;
+  else {
+    pg.n_inst++;
+    if (g_parked.size() >= PARKED_MOST || hipGraphInstantiate(&pg.exec[slot], graph, nullptr, nullptr, 0) != hipSuccess) {
       (void)hipGetLastError();
-      hipGraphExecDestroy(pg.exec[slot]);
       pg.exec[slot] = nullptr;
-    } else pg.n_update++;
+      hipGraphDestroy(graph);
+      plan_graph_drop(pg, true);
+      return;
+    }
   }
-  const bool fresh = !pg.exec[slot];
-  if (fresh) pg.n_inst++;
-  if (!pg.exec[slot] && hipGraphInstantiate(&pg.exec[slot], graph, nullptr, nullptr, 0) != hipSuccess) {
-    (void)hipGetLastError();
-    pg.exec[slot] = nullptr;
-    hipGraphDestroy(graph);
-    plan_graph_drop(pg, true);
-    return;
-  }
+  pg.exec_nodes[slot] = n_nodes;
   hipGraphDestroy(graph);
   pg.cur = slot; pg.ready = true; pg.pos = pos; pg.seq = seq_len; pg.n_nodes = n_nodes; pg.gen = g.layout_gen;
 }

@@ -347,6 +347,50 @@ def test_a_plan_called_with_the_same_step_is_not_recorded():
     assert line and " 0 steps from graphs" in line[-1] and " 0 instantiations" in line[-1], p.stderr[-1000:]
 
 
+_GRAPH_KEPT_SNIPPET = """
+import sys, json
+sys.path.insert(0, {root!r})
+import numpy as np
+from adam_amd import adamah as A
+n, ok = 4096, []
+vals = np.random.default_rng(0).standard_normal(2 * n).astype(np.float32)
+run = lambda lo: np.arange(lo, lo + n, dtype=np.uint32)
+for context in range(3):
+    gpu = A.init()
+    gpu.set_dtype(A.DTYPE_F32)
+    gpu.map_create(0, 1, 5 * n)
+    gpu.scatter_contiguous(0, 0, vals)
+    h = [gpu.upload_dev(run(i * n))[0] for i in range(5)]
+    op = lambda code, a, b, c: A.DecodePlanOp(kind=A.DECODE_OP_OP2, map_id=0, op_code=code, h0=h[a], h1=h[b], h2=h[c], u0=n)
+    plans = [[op(A.OP_ADD, 0, 1, 2)], [op(A.OP_MUL, 1, 0, 3)], [op(A.OP_ADD, 0, 1, 2), op(A.OP_MUL, 2, 1, 3), op(A.OP_ADD, 3, 2, 4)], [op(A.OP_ADD, 1, 1, 4)]]
+    a, b = vals[:n], vals[n:]
+    want = [(2, a + b), (3, a * b), (4, (a + b) * b + (a + b)), (4, b + b)]
+    for ops, (to, y) in zip(plans, want):
+        gpu.register_decode_plan(3, ops)
+        for step in range(9):
+            gpu.scatter_contiguous(0, to * n, np.zeros(n, np.float32))
+            gpu.decode_step(3, step, step + 1)
+            ok.append(bool(np.array_equal(gpu.gather(0, run(to * n)).view(np.float32), y)))
+    gpu.shutdown()
+print(json.dumps(ok))
+"""
+
+
+def test_graphs_of_a_dropped_plan_serve_the_next_one():
+    """An executable graph is kept for as long as the process lives (memory that is allocated behind its end has held wrong values) and
+    updated for whatever plan comes next: other operands, other ops, another library context."""
+    import json, os, re, subprocess, sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    note("decode plan graphs: kept for the next plan")
+    env = dict(os.environ, ADAMAH_PLAN_GRAPH="1", ADAMAH_DEBUG="1")
+    p = subprocess.run([sys.executable, "-c", _GRAPH_KEPT_SNIPPET.format(root=root)], env=env, capture_output=True, text=True, timeout=110)
+    assert p.returncode == 0, p.stderr[-2000:]
+    assert json.loads(p.stdout.strip().split("\n")[-1]) == [True] * 108, p.stdout
+    made = [tuple(map(int, re.search(r": (\d+) steps from graphs, .* (\d+) instantiations", l).groups())) for l in p.stderr.split("\n") if "steps from graphs" in l]
+    assert len(made) == 12 and all(steps >= 5 for steps, _ in made), made
+    assert made[0][1] == 3 and all(new == 0 for _, new in made[4:]), made          # the later contexts instantiate nothing
+
+
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
 @pytest.mark.parametrize("chunk", [64, 45])
 def test_prompts_of_a_batch_go_through_the_weights_together(hip, arch, chunk):
