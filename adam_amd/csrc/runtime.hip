@@ -871,7 +871,10 @@ static int replay_plan(uint32_t plan_id, uint32_t pos, uint32_t seq_len) {
   return ret;
 }
 
-// Graph replay of a plan (on unless ADAMAH_PLAN_GRAPH=0).  A decode loop calls the plan with pos, pos + 1, ...: after
+// Graph replay of a plan (ADAMAH_PLAN_GRAPH=1; by default a plan is replayed launch by launch: no slower now that a launch's
+// host work is short and its gap hidden -- ms, graphs and without: Llama 8B shape a token 1.554 and 1.546, 9 + 8 tokens of a toy Llama 1.8 - 2.0
+// and 1.3, 21 + 16 tokens of the 4096-wide mixers 9.56 and 9.42, the Gemma 1B turn 15.3 and 15.1, 17.6 and 16.6 without lookahead, steps of the
+// expert design level -- and the runtime keeps memory for every step of a graph, below).  A decode loop calls the plan with pos, pos + 1, ...: after
 // serving step (pos, seq_len) the library records the launches of step (pos + 1, seq_len + 1) into a HIP graph
 // -- stream capture of the same entry points, nothing executes -- while the device is still busy with the
 // current step, and the next call launches that graph if it asks for exactly that step (anything else is
@@ -916,7 +919,19 @@ static void plan_graph_park(PlanGraph& pg, int slot) {       // (its last launch
   pg.exec[slot] = nullptr;
 }
 
-static bool graph_update(hipGraphExec_t exec, hipGraph_t graph) {
+// The runtime keeps the arguments of every update: 680 bytes a launch (2400 turns of the Gemma 1B shape, 36000 steps of 130 launches:
+// 3.1 GB more in use).  So the updates of a process are counted, by launches, and plans are replayed the ordinary way
+// after GRAPH_MOST of them (11 GB; ADAMAH_PLAN_GRAPH_MOST: another number).
+#define GRAPH_MOST (16ull << 20)
+static uint64_t g_graph_nodes = 0;
+
+static bool graphs_spent() {
+  const char* e = getenv("ADAMAH_PLAN_GRAPH_MOST");
+  return g_graph_nodes >= (e && e[0] ? strtoull(e, nullptr, 10) : GRAPH_MOST);
+}
+
+static bool graph_update(hipGraphExec_t exec, hipGraph_t graph, uint32_t n_nodes) {
+  g_graph_nodes += n_nodes;
   hipGraphNode_t bad = nullptr;
   hipGraphExecUpdateResult res;
   if (hipGraphExecUpdate(exec, graph, &bad, &res) == hipSuccess) return true;
@@ -931,7 +946,7 @@ static hipGraphExec_t plan_graph_unpark(hipGraph_t graph, uint32_t n_nodes) {
     if (g_parked[i].n_nodes != n_nodes) continue;
     tries++;
     const hipGraphExec_t exec = g_parked[i].exec;
-    if (!graph_update(exec, graph)) continue;
+    if (!graph_update(exec, graph, n_nodes)) continue;
     g_parked.erase(g_parked.begin() + (long)i);
     return exec;
   }
@@ -940,7 +955,7 @@ static hipGraphExec_t plan_graph_unpark(hipGraph_t graph, uint32_t n_nodes) {
 
 static bool plan_graphs_on() {
   const char* e = getenv("ADAMAH_PLAN_GRAPH");
-  return !(e && e[0] == '0');
+  return e && e[0] && e[0] != '0';
 }
 
 static void plan_graph_drop(PlanGraph& pg, bool for_good) {
@@ -967,6 +982,7 @@ static std::vector<PendOp> take_trailing_norms() {
 static void plan_graph_record(uint32_t plan_id, uint32_t pos, uint32_t seq_len) {
   PlanGraph& pg = g_pg[plan_id];
   pg.ready = false;
+  if (graphs_spent()) { plan_graph_drop(pg, true); return; }
   const uint64_t gen0 = g.mem_gen, lay0 = g.layout_gen;
   const Stats saved = g.stats;
   if (hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal) != hipSuccess) { (void)hipGetLastError(); plan_graph_drop(pg, true); return; }
@@ -989,11 +1005,12 @@ static void plan_graph_record(uint32_t plan_id, uint32_t pos, uint32_t seq_len) 
     hipEventSynchronize(pg.done[slot]);
     pg.launched[slot] = false;
   }
-  if (pg.exec[slot] && !graph_update(pg.exec[slot], graph)) plan_graph_park(pg, slot);      // another launch shape (e.g. one more slice)
+  if (pg.exec[slot] && !graph_update(pg.exec[slot], graph, n_nodes)) plan_graph_park(pg, slot);      // another launch shape (e.g. one more slice)
   if (!pg.exec[slot]) pg.exec[slot] = plan_graph_unpark(graph, n_nodes);
   if (pg.exec[slot]) pg.n_update++;
   else {
     pg.n_inst++;
+    g_graph_nodes += n_nodes;
     if (g_parked.size() >= PARKED_MOST || hipGraphInstantiate(&pg.exec[slot], graph, nullptr, nullptr, 0) != hipSuccess) {
       (void)hipGetLastError();
       pg.exec[slot] = nullptr;
@@ -1033,7 +1050,7 @@ int adamah_decode_step(uint32_t plan_id, uint32_t pos, uint32_t seq_len) {
   if (opened) batch_begin();
   int ret;
   PlanGraph& pg = g_pg[plan_id];
-  if (!plan_graphs_on() || pg.disabled) ret = replay_plan(plan_id, pos, seq_len);
+  if (!plan_graphs_on() || pg.disabled) { ret = replay_plan(plan_id, pos, seq_len); pg.eager_steps++; }
   else {
     flush_pending();                                 // what was queued before the plan runs ahead of it
     if (pg.ready && pg.gen != g.layout_gen) pg.ready = false;   // a map or scratch buffer moved since the recording

@@ -612,8 +612,8 @@ def main():
                                f"timed steps at context {m['end_pos'] - args.steps + 1}..{m['end_pos']}",
                    "baseline_config": 2 if gemma else 4,
                    "scheduler": args.scheduler, "launches_per_token": round(m["launches_per_token"], 1),
-                   "issue": "one native decode_step call per token (registered decode plan, launched from HIP graphs "
-                            "recorded one step ahead); every token id is read back, in order, but the step that consumes "
+                   "issue": "one native decode_step call per token (registered decode plan, replayed launch by "
+                            "launch); every token id is read back, in order, but the step that consumes "
                             "token n takes it from the device and is issued before the host has read it (one step of "
                             "lookahead; 'read_then_issue' is the same loop without it)"},
         "timed_runs": {"protocol": "prefill (cold) and the warm-up steps, then the timed region of exactly `steps` steps "

@@ -241,7 +241,7 @@ print(json.dumps({{"tokens": out, "hidden": [float(v) for v in hid[:64]]}}))
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])
 def test_decode_plan_from_recorded_graphs_gives_the_same_tokens(arch):
     """The plan's launches for the next position are recorded into a HIP graph while the current step runs and
-    replayed by the next call (ADAMAH_PLAN_GRAPH=0: never).  Two generations (80 graph replays with the token read
+    replayed by the next call (ADAMAH_PLAN_GRAPH=1; else never).  Two generations (80 graph replays with the token read
     and the embedding upload between them) give the tokens and the final hidden state, bit for bit, of the
     ordinary replay.  Each mode runs in a process of its own, so the library's exit report can be read."""
     import json, os, subprocess, sys
@@ -338,7 +338,7 @@ def test_a_plan_called_with_the_same_step_is_not_recorded():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     note("decode plan graphs: the same step again and again")
     env = dict(os.environ, ADAMAH_DEBUG="1")
-    env.pop("ADAMAH_PLAN_GRAPH", None)
+    env["ADAMAH_PLAN_GRAPH"] = "1"
     p = subprocess.run([sys.executable, "-c", _GRAPH_SAME_STEP_SNIPPET.format(root=root)], env=env, capture_output=True, text=True,
                        timeout=110)
     assert p.returncode == 0, p.stderr[-2000:]
@@ -376,6 +376,20 @@ print(json.dumps(ok))
 """
 
 
+def test_plans_record_no_graphs_unless_asked_to():
+    """The default: every step is replayed launch by launch, whatever the walk."""
+    import json, os, subprocess, sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    note("decode plans without graphs")
+    env = dict(os.environ, ADAMAH_DEBUG="1")
+    env.pop("ADAMAH_PLAN_GRAPH", None)
+    p = subprocess.run([sys.executable, "-c", _GRAPH_KEPT_SNIPPET.format(root=root)], env=env, capture_output=True, text=True, timeout=110)
+    assert p.returncode == 0, p.stderr[-2000:]
+    assert json.loads(p.stdout.strip().split("\n")[-1]) == [True] * 108, p.stdout
+    lines = [l for l in p.stderr.split("\n") if "steps from graphs" in l]
+    assert len(lines) == 12 and all(" 0 steps from graphs, 9 replayed, 0 updates, 0 instantiations" in l for l in lines), lines
+
+
 def test_graphs_of_a_dropped_plan_serve_the_next_one():
     """An executable graph is kept for as long as the process lives (memory that is allocated behind its end has held wrong values) and
     updated for whatever plan comes next: other operands, other ops, another library context."""
@@ -389,6 +403,13 @@ def test_graphs_of_a_dropped_plan_serve_the_next_one():
     made = [tuple(map(int, re.search(r": (\d+) steps from graphs, .* (\d+) instantiations", l).groups())) for l in p.stderr.split("\n") if "steps from graphs" in l]
     assert len(made) == 12 and all(steps >= 5 for steps, _ in made), made
     assert made[0][1] == 3 and all(new == 0 for _, new in made[4:]), made          # the later contexts instantiate nothing
+    # the runtime keeps the arguments of every update: they are counted, and behind the last one plans are replayed the ordinary way
+    env["ADAMAH_PLAN_GRAPH_MOST"] = "4"
+    p = subprocess.run([sys.executable, "-c", _GRAPH_KEPT_SNIPPET.format(root=root)], env=env, capture_output=True, text=True, timeout=110)
+    assert p.returncode == 0, p.stderr[-2000:]
+    assert json.loads(p.stdout.strip().split("\n")[-1]) == [True] * 108, p.stdout
+    lines = [l for l in p.stderr.split("\n") if "steps from graphs" in l]
+    assert " 4 steps from graphs" in lines[0] and all(" 0 steps from graphs" in l and "graphs given up" in l for l in lines[1:]), lines
 
 
 @pytest.mark.parametrize("arch", ["gemma3", "llama"])

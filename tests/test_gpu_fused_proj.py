@@ -200,10 +200,11 @@ def test_fused_projection_kinds_in_a_decode_plan(hip):
 
 
 @pytest.mark.parametrize("kind", ["q4", "q8"])
-def test_graph_of_a_fused_qkv_plan_is_dropped_when_its_seventh_handle_is_rewritten(hip, kind):
+def test_graph_of_a_fused_qkv_plan_is_dropped_when_its_seventh_handle_is_rewritten(hip, monkeypatch, kind):
     """The Q/K/V kinds keep the V result's handle in u0.  A graph recorded one step ahead holds that offset by
     value, so re-uploading the handle between two steps must send the next step through the ordinary replay:
     V lands at the new place from that step on, and the old place is no longer written."""
+    monkeypatch.setenv("ADAMAH_PLAN_GRAPH", "1")
     K, rows = 1152, (256, 64, 64)
     x = np.random.default_rng(5).standard_normal(K).astype(np.float32)
     qt, bases = stacked(kind, rows, K, 17)
