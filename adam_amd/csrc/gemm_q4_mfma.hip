@@ -378,10 +378,10 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
 // Eight waves of 64 weight rows each, side by side, over 32 MA activation rows: a wave has 2 x MA results of 32 x 32.  A step
 // is 64 columns (two blocks); its packed weights (16 KB), their scales (2 KB) and both planes of the activations (8 KB per 32
 // rows) go straight to LDS, a ring of four stages (MA = 2) or three (MA = 3, 4).  512 x 28672 x 4096: 317 -> 248 us = 485
-// TFLOP/s.  96 rows a workgroup give every CU one where 128 leave a third of them without (384 x 28672 x 4096, 168 workgroups and
-// 224: 216 us and 197, not in proportion: with all CUs at work the clock falls from 2.3 to 2.0 GHz, the products' power).  What bounds it is the vector work beside the matrix instructions (a
-// multiply-add per result and block, the unpacking): they share a wave's issue, so what counts is that no instruction of
-// either kind waits for another.  LDS reads without bank conflicts: 266 -> 246 us.
+// TFLOP/s.  96 rows a workgroup put 224 of the 256 CUs to work where 128 put 168 (384 x 28672 x 4096: 216 us and 197, not in
+// proportion: with more CUs at work the clock falls, the products' power: 2.56 GHz with 32 workgroups, 2.0 with 224, 1.86 with 256,
+// launches one by one).  What bounds it is the vector work beside the matrix instructions (a multiply-add per result and block, the
+// unpacking): they share a wave's issue, so what counts is that no instruction of either kind waits for another.  LDS reads without bank conflicts: 266 -> 246 us.
 // v_mfma_f32_32x32x16_f16: lane l supplies row l % 32, k = 8 (l / 32) .. + 7 of either operand and receives rows
 // 8 (r / 4) + 4 (l / 32) + r % 4 of column l % 32 -- here the columns are weight rows, so a block's scale is one number per
 // lane.  S16 (rows of whole runs of 256 columns that begin on 16 bytes of scales): the scales of four steps come in one 16-byte piece a row.
