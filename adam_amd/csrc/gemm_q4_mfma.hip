@@ -26,6 +26,7 @@
 // through LDS in a fixed order.  At most 64 rows are converted to operand tiles (ActForm), more to rows.
 #include "gemv_common.h"
 #include "lds_ring.h"
+#include "tile_store.h"
 #include <algorithm>
 
 namespace adamah {
@@ -267,37 +268,22 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
     __syncthreads();
   }
   // lane (r16, g) holds D[4g + i][r16]: activation rows m0 + 16 t + 4g + i, weight row n0 + 16 r + r16
+  const auto row = [&](int t, int i) { return m0 + t * 16u + 4u * g + i; };
+  if (ksplit <= 1u) {      // (raw sums of a share of K: scale and placement are k_gemm_splitk_sum's)
 #pragma unroll
-  for (int t = 0; t < MT; t++)
+    for (int t = 0; t < MT; t++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const uint32_t row = m0 + t * 16u + 4u * g + i;
-      if (row >= M) continue;
-      if (ksplit > 1u) {   // raw sums of this share of K; scale and placement are k_gemm_splitk_sum's
-        float* pr = part + ((uint64_t)kz * M + row) * N;
+      for (int i = 0; i < 4; i++) {
+        const float inv = scale[2 * ((uint64_t)op * M + min(row(t, i), M - 1u)) + 1];
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-          const uint32_t n = n0 + r * 16u + r16;
-          if (n < N) pr[n] = acc[r][t][i];
-        }
-        continue;
+        for (int r = 0; r < R; r++) acc[r][t][i] *= inv;
       }
-      const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
-      float* c = out + c_off + (uint64_t)row * N;
+  }
+  uint32_t n[R];
 #pragma unroll
-      for (int r = 0; r < R; r++) {
-        const uint32_t n = n0 + r * 16u + r16;
-        if (n >= N) continue;
-        if (segs.count) {   // stacked matrices: the row's own matrix and its result base
-          uint32_t sgi = 0;
-#pragma unroll
-          for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = acc[r][t][i] * inv;
-        } else c[n] = acc[r][t][i] * inv;
-      }
-    }
+  for (int r = 0; r < R; r++) n[r] = n0 + r * 16u + r16;
+  store_columns<MT, 4, R>([&](int t, int i, int r) { return acc[r][t][i]; }, row, n, M, N, kz, c_off, out, ksplit > 1u ? part : nullptr, segs);
 }
-
 #undef GEMM_FETCH
 
 // The shares of K of a split launch of the kernel above, summed in the order of the shares, scaled by the row's factor
@@ -341,11 +327,9 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
       return;
     }
     if (segs.count) {
-      uint32_t s0 = 0, s3 = 0;
-#pragma unroll
-      for (uint32_t q = 1; q < 4; q++) { s0 += q < segs.count && n >= segs.begin[q] ? 1u : 0u; s3 += q < segs.count && n + 3u >= segs.begin[q] ? 1u : 0u; }
-      const uint64_t to = segs.c[s0] + (uint64_t)row * segs.n[s0] + (n - segs.begin[s0]);
-      if (s0 == s3 && (to & 3u) == 0u) { *(f4q_t*)(out + to) = (f4q_t){a[0][0] * inv, a[0][1] * inv, a[0][2] * inv, a[0][3] * inv}; return; }
+      const ColumnPlace p = column_place(n, N, 0u, out, segs), p3 = column_place(n + 3u, N, 0u, out, segs);
+      float* const to = p.col + (uint64_t)row * p.step;
+      if (p3.col == p.col + 3 && p3.step == p.step && ((to - out) & 3) == 0) { *(f4q_t*)to = (f4q_t){a[0][0] * inv, a[0][1] * inv, a[0][2] * inv, a[0][3] * inv}; return; }
     }
     v[0] = a[0][0]; v[1] = a[0][1]; v[2] = a[0][2]; v[3] = a[0][3];
   } else {
@@ -362,15 +346,9 @@ k_gemm_splitk_sum(const float* __restrict__ part, uint32_t ksplit, uint32_t M, u
     if (i >= total) break;
     const uint32_t row = (uint32_t)(i / N), n = (uint32_t)(i % N);
     const float y = v[e] * scale[2 * (uint64_t)row + 1];
-    if (segs.count) {
-      uint32_t sgi = 0;
-#pragma unroll
-      for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-      out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y;
-    } else {
-      out[c_off + (uint64_t)row * N + n] = y;
-      if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;   // the add behind it
-    }
+    const ColumnPlace p = column_place(n, N, c_off, out, segs);
+    p.col[(uint64_t)row * p.step] = y;
+    if (!segs.count && segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;   // the add behind it
   }
 }
 
@@ -543,30 +521,18 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
   for (int i = 0; i < 16; i++) acc[1][MA - 1][i] = fmaf(blk[1][i], dlast, acc[1][MA - 1][i]);
   ring_wait<0>();
   const uint64_t c_off = (by_val & 2u) || part || segs.count ? (uint64_t)c_val : (uint64_t)lc[0];
+  const auto row = [&](int t, int i) { return m0 + t * 32u + 8u * (i >> 2) + 4u * h + (i & 3u); };
+  if (!part) {
 #pragma unroll
-  for (int t = 0; t < MA; t++)
+    for (int t = 0; t < MA; t++)
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const uint32_t row = m0 + t * 32u + 8u * (i >> 2) + 4u * h + (i & 3u);
-      if (row >= M) continue;
-      const float inv = part ? 1.f : scale[2 * (uint64_t)row + 1];
-#pragma unroll
-      for (int w = 0; w < 2; w++) {
-        const uint32_t n = n0 + wave * 64u + w * 32u + r32;
-        if (n >= N) continue;
-        if (part) { part[((uint64_t)kz * M + row) * N + n] = acc[w][t][i]; continue; }
-        const float y = acc[w][t][i] * inv;
-        if (segs.count) {
-          uint32_t sgi = 0;
-#pragma unroll
-          for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y;
-        } else {
-          out[c_off + (uint64_t)row * N + n] = y;
-          if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;
-        }
+      for (int i = 0; i < 16; i++) {
+        const float inv = scale[2 * (uint64_t)min(row(t, i), M - 1u) + 1];
+        acc[0][t][i] *= inv; acc[1][t][i] *= inv;
       }
-    }
+  }
+  const uint32_t n[2] = {n0 + wave * 64u + r32, n0 + wave * 64u + 32u + r32};
+  store_columns<MA, 16, 2>([&](int t, int i, int w) { return acc[w][t][i]; }, row, n, M, N, kz, c_off, out, part, segs);
 }
 
 // 2 .. 64 activation rows: the weights are read once, so what counts is how fast they stream, and what stands in its way is
@@ -721,7 +687,15 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
       const uint32_t row = idx >> 4, c = idx & 15u, lo = M + row;
       const auto place = [&](uint32_t v) { return (v >> 4) * 256u + (v & 3u) * 64u + ((v >> 2) & 3u) * 16u + c; };
       const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
-      float y[RC];
+      const bool add = !segs.count && segs.add;
+      float y[RC], old[RC];
+      ColumnPlace to[RC];
+#pragma unroll
+      for (int r = 0; r < RC; r++) {
+        const uint32_t n = min(first_row(r0 + r) + c, N - 1u);
+        to[r] = column_place(n, N, c_off, out, segs);
+        if (add) old[r] = out[segs.res + (uint64_t)row * N + n];
+      }
 #pragma unroll
       for (int r = 0; r < RC; r++) {
         float a = 0.f, b = 0.f;
@@ -737,15 +711,8 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
       for (int r = 0; r < RC; r++) {
         const uint32_t n = first_row(r0 + r) + c;
         if (n >= (glum && !(r & 1) ? N >> 1 : N)) continue;
-        if (segs.count) {   // stacked matrices: the row's own matrix and its result base
-          uint32_t sgi = 0;
-#pragma unroll
-          for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y[r];
-        } else {
-          out[c_off + (uint64_t)row * N + n] = y[r];
-          if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y[r];
-        }
+        to[r].col[(uint64_t)row * to[r].step] = y[r];
+        if (add) out[segs.dst + (uint64_t)row * N + n] = old[r] + y[r];
       }
       if (glum && first_row(r0) + c < (N >> 1))   // act(gate) * up, as the element-wise op computes it
         out[segs.dst + (uint64_t)row * (N >> 1) + first_row(r0) + c] = (segs.glu == 34u ? gelu_tanh(y[0]) : y[0] / (1.0f + expf(-y[0]))) * y[RC - 1];
@@ -894,30 +861,27 @@ k_gemm_q8_f16_ksplit(const uint8_t* __restrict__ W, const __half* __restrict__ d
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[r][t][i] += part[(((w * R + r) * MT + t) * 4u + i) * 64u + lane];
   // lane (r16, g) holds D[4g + i][r16]: activation rows 16 t + 4g + i, weight row r16 of tile r
+  const auto row_of = [&](int t, int i) { return t * 16u + 4u * g + i; };
 #pragma unroll
   for (int t = 0; t < MT; t++)
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint32_t row = t * 16u + 4u * g + i;
-      if (row >= M) continue;
-      const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
+      const float inv = scale[2 * ((uint64_t)op * M + min(row_of(t, i), M - 1u)) + 1];
 #pragma unroll
-      for (int r = 0; r < R; r++) {
-        const uint32_t n = trow0[r] + r16;
-        if (n >= N) continue;
-        const float y = acc[r][t][i] * inv;
-        if (segs.count) {   // stacked matrices: the row's own matrix and its result base
-          uint32_t sgi = 0;
+      for (int r = 0; r < R; r++) acc[r][t][i] *= inv;
+    }
+  uint32_t nn[R];
 #pragma unroll
-          for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-          out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y;
-        } else {
-          out[c_off + (uint64_t)row * N + n] = y;
-          if (segs.add) out[segs.dst + (uint64_t)row * N + n] = out[segs.res + (uint64_t)row * N + n] + y;
-        }
-      }
-      if (glum && trow0[0] + r16 < (N >> 1)) {   // act(gate) * up, as the element-wise op computes it
-        const float a = acc[0][t][i] * inv, b = acc[R - 1][t][i] * inv;
+  for (int r = 0; r < R; r++) nn[r] = trow0[r] + r16;
+  store_columns<MT, 4, R>([&](int t, int i, int r) { return acc[r][t][i]; }, row_of, nn, M, N, 0u, c_off, out, nullptr, segs);
+  if (glum && trow0[0] + r16 < (N >> 1))         // act(gate) * up, as the element-wise op computes it
+#pragma unroll
+  for (int t = 0; t < MT; t++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t row = row_of(t, i);
+      if (row < M) {
+        const float a = acc[0][t][i], b = acc[R - 1][t][i];
         out[segs.dst + (uint64_t)row * (N >> 1) + trow0[0] + r16] =
             segs.glu == 34u ? gelu_tanh(a) * b : (a / (1.0f + expf(-a))) * b;
       }
@@ -1082,16 +1046,12 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
   }
   if (glum) __syncthreads();
   const bool n_ok = glum ? tb + r16 < (N >> 1) : n < N;
+  const ColumnPlace to = column_place(n, N, c_off, out, segs);
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const uint32_t row = 4u * g + i;
     if (row >= M || !n_ok) continue;
-    if (segs.count) {
-      uint32_t sgi = 0;
-#pragma unroll
-      for (uint32_t q = 1; q < 4; q++) sgi += (q < segs.count && n >= segs.begin[q]) ? 1u : 0u;
-      out[segs.c[sgi] + (uint64_t)row * segs.n[sgi] + (n - segs.begin[sgi])] = y[i];
-    } else out[c_off + (uint64_t)row * N + n] = y[i];
+    to.col[(uint64_t)row * to.step] = y[i];
     if (glum && wave < NW / 2u) {
       const float a = y[i], b = ybuf[(wave * 4u + i) * 64u + lane];
       out[segs.dst + (uint64_t)row * (N >> 1) + n] = segs.glu == 34u ? gelu_tanh(a) * b : (a / (1.0f + expf(-a))) * b;
