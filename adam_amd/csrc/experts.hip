@@ -373,11 +373,11 @@ __device__ __forceinline__ void put_part(const XSpec& s, float* parts, uint32_t 
   for (int i = 0; i < 4; i++) if (n0 + i < s.width) d[i] = v[i];
 }
 
-template <int BM, int BN, int WM, int WN, int ST, bool IN>
+template <int BM, int BN, int WM, int WN, int ST, int STX, bool IN>
 __global__ void __launch_bounds__(64 * WM * WN)
 k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
                 const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n) {
-  __shared__ __attribute__((aligned(16))) bf16_t la[ST * BN * 64], lb[ST * BM * 64];
+  __shared__ __attribute__((aligned(16))) bf16_t la[ST * BN * 64], lb[STX * BM * 64];
   constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16;
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t c = lane & 15u, kg = lane >> 4, kp = IN ? s.k_stride : s.ff_stride, n = IN ? 2u * ((s.ff + 15u) & ~15u) : s.width;
@@ -387,11 +387,11 @@ k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ 
   const bf16_t* We = W + (IN ? s.gate_up + (uint64_t)t.e * s.gate_up_step : s.down + (uint64_t)t.e * s.down_step);
   const uint32_t* le = list + (uint64_t)t.e * rows;
   f4_t acc[NTN][NTM];
-  tile_product<BM, BN, WM, WN, ST>(acc, TileRows<BN, WM * WN>(wave, lane, [&](uint32_t r) { return We + (uint64_t)min(n0 + r, n - 1u) * kp; }),
+  tile_product<BM, BN, WM, WN, ST, 1, STX>(acc, TileRows<BN, WM * WN>(wave, lane, [&](uint32_t r) { return We + (uint64_t)min(n0 + r, n - 1u) * kp; }),
                                    TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) {
                                      const uint32_t i = min(m0 + r, t.count - 1u);
                                      return opnd + (IN ? s.opnd + (uint64_t)(le[i] / s.top) * kp : s.act_opnd + (uint64_t)(t.first + i) * kp);
-                                   }), kp, 0u, kp, la, lb, wave, lane);
+                                   }), kp, 0u, kp, la, lb, wave, lane, m0 + wm < t.count);
 #pragma unroll
   for (int j = 0; j < NTM; j++) {
     const uint32_t i = m0 + wm + 16u * j + c;
@@ -500,10 +500,16 @@ static void experts_product(Map* mo, Map* mw, const XSpec& s, float* parts, cons
   };
   if (mo->dtype == DTYPE_F32)
     k_experts_f32<IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (float*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
+  // 256 tokens a tile where an expert has that many on average: what bounds both is the way of the weights and tokens into LDS, of which
+  // there is a third less (2048 rows, 6 of 34, experts 1024 wide in 2048: both products 243 us in tiles of 128, 196 so; 208 without a third buffer
+  // for the weights, which come from memory and not from the L2; 952 rows, 168 an expert, 146 in tiles of 128, 179 so).
+  // A wave whose rows all lie past the expert's last only loads.
+  else if (entries >= (uint64_t)s.experts * 256u)
+    k_experts_tiled<256, 256, 2, 4, 3, 2, IN><<<grid(256, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256));
   else if (entries >= (uint64_t)s.experts * 96u)
-    k_experts_tiled<128, 256, 2, 4, 3, IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256));
+    k_experts_tiled<128, 256, 2, 4, 3, 3, IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256));
   else
-    k_experts_tiled<64, 64, 2, 2, 4, IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
+    k_experts_tiled<64, 64, 2, 2, 4, 4, IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
   count_launch();
 }
 

@@ -47,46 +47,54 @@ template <int R, int NW> struct TileRows {
   }
 };
 // BM tokens x BN matrix rows by WM x WN waves; acc[i][j]: matrix rows wn + 16 i, tokens wm + 16 j of a wave's part; la: ST
-// BN 64, lb: ST BM 64 elements.  A ring of ST buffers of 64 columns: a step's loads are asked for ST - 1 steps ahead.  A
+// BN 64, lb: STX BM 64 elements.  A ring of ST buffers of 64 columns (STX of the tokens'): a step's loads are asked for ST - 1 steps ahead.  A
 // step is two halves of 32 columns; a half's operands are read from LDS under the products of the half before, on both
-// sides of the step's one barrier.  What bounds it (256 x 256, two buffers): of the 1.7 us a step takes on all CUs the
+// sides of the step's one barrier.  on: this wave has tokens.  What bounds it (256 x 256, two buffers): of the 1.7 us a step takes on all CUs the
 // products need 1.0 (matrix pipe 55 .. 62 % busy over a launch of 2048 rows), its loads come out of the L2s at 8.8 TB/s, reads
 // of LDS run beside both; loads and reads in a run ahead of the products instead of among them: 1.95 us.  Columns k0 .. k1 of
 // the tokens; column k of them meets column k mod kp of the matrix (k1 at most PL kp).  PL = 3, tokens in pieces, the largest last: an infinite weight and a lower piece
 // of 0 make no number where the whole product is infinite, so the lower pieces' sum counts only where it is finite (the
 // highest one's is infinite, or no number, exactly where the whole one is).
-template <int BM, int BN, int WM, int WN, int ST, int PL = 1>
+template <int BM, int BN, int WM, int WN, int ST, int PL = 1, int STX = ST>
 __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM / 16], const TileRows<BN, WM * WN>& w, const TileRows<BM, WM * WN>& x,
-                                             uint32_t kp, uint32_t k0, uint32_t k1, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane) {
-  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16, LOADS = TileRows<BN, WM * WN>::N + TileRows<BM, WM * WN>::N;
+                                             uint32_t kp, uint32_t k0, uint32_t k1, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane, bool on = true) {
+  constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16, LW = TileRows<BN, WM * WN>::N, LX = TileRows<BM, WM * WN>::N, LOADS = LW + LX;
+  constexpr int LESS = STX < ST ? STX : ST, MORE = STX < ST ? ST : STX, LF = STX < ST ? LX : LW;       // stages; loads of the operand with fewer, which go first
+  static_assert(MORE - LESS <= 1, "what may be on its way at a wait");
+  constexpr int FLY = (LESS - 2) * LOADS + (MORE > LESS ? LOADS - LF : 0);                  // on their way when the next step's tiles must be there
   const uint32_t c = lane & 15u, kg = lane >> 4, wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
   const uint32_t ba = lds_byte(la), bb = lds_byte(lb);
 #pragma unroll
   for (int i = 0; i < NTN; i++)
 #pragma unroll
     for (int j = 0; j < NTM; j++) acc[i][j] = (f4_t){0, 0, 0, 0};
-  const auto load = [&](int i, uint32_t k, uint32_t into) {       // (steps past the end re-read the last: the count in flight stays)
+  // load i of a step that is t steps behind the one from column k on, whose buffers are bw and bx
+  const auto load_w = [&](int i, uint32_t k, uint32_t into) {     // (steps past the end re-read the last: the count in flight stays)
     const uint32_t kc = min(k, k1 - 64u), kw = PL == 1 ? kc : kc >= 2u * kp ? kc - 2u * kp : kc >= kp ? kc - kp : kc;
-    if (i < TileRows<BN, WM * WN>::N) w.load(i, kw, ba + into * (BN * 128u), wave);
-    else x.load(i - TileRows<BN, WM * WN>::N, kc, bb + into * (BM * 128u), wave);
+    w.load(i, kw, ba + into * (BN * 128u), wave);
+  };
+  const auto load_x = [&](int i, uint32_t k, uint32_t into) { x.load(i, min(k, k1 - 64u), bb + into * (BM * 128u), wave); };
+  const auto load = [&](int i, uint32_t k, uint32_t bw, uint32_t bx) {      // of what step k has made room for
+    if (STX < ST ? i < LX : i >= LW) load_x(STX < ST ? i : i - LW, k + STX * 64u, bx);
+    else load_w(STX < ST ? i - LX : i, k + ST * 64u, bw);
   };
   bf8_t a[2][NTN], b[2][NTM];
-  const auto read = [&](int i, uint32_t buf, int h) {
+  const auto read = [&](int i, uint32_t bw, uint32_t bx, int h) {
     const uint32_t at = ((4u * h + kg) ^ (c & 7u)) << 3;
-    if (i < NTM) b[h][i] = *(const bf8_t*)(lb + buf * (BM * 64) + (wm + 16u * i + c) * 64u + at);
-    else a[h][i - NTM] = *(const bf8_t*)(la + buf * (BN * 64) + (wn + 16u * (i - NTM) + c) * 64u + at);
+    if (i < NTM) b[h][i] = *(const bf8_t*)(lb + bx * (BM * 64) + (wm + 16u * i + c) * 64u + at);
+    else a[h][i - NTM] = *(const bf8_t*)(la + bw * (BN * 64) + (wn + 16u * (i - NTM) + c) * 64u + at);
   };
   // four products, then a few of the next half's reads and (second half) some of the loads, and so on: the matrix pipe is never
   // behind a run of either
   constexpr int NP = NTN * NTM / 4, READS = NP > 1 ? (NTN + NTM + NP - 2) / (NP - 1) : NTN + NTM, LOADS_EACH = (LOADS + NP - 1) / NP;
-  const auto half = [&](int h, uint32_t from, uint32_t k, uint32_t into) {
+  const auto half = [&](int h, uint32_t fw, uint32_t fx, uint32_t k, uint32_t bw, uint32_t bx) {
 #pragma unroll
     for (int q = 0; q < NP; q++) {
 #pragma unroll
-      for (int i = 0; i < READS; i++) if (q * READS + i < NTN + NTM) read(q * READS + i, from, 1 - h);
+      for (int i = 0; i < READS; i++) if (q * READS + i < NTN + NTM) read(q * READS + i, fw, fx, 1 - h);
       if (h == 1) {
 #pragma unroll
-        for (int i = 0; i < LOADS_EACH; i++) if (q * LOADS_EACH + i < LOADS) load(q * LOADS_EACH + i, k, into);
+        for (int i = 0; i < LOADS_EACH; i++) if (q * LOADS_EACH + i < LOADS) load(q * LOADS_EACH + i, k, bw, bx);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -98,20 +106,32 @@ __device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM /
     }
   };
 #pragma unroll
-  for (int t = 0; t < ST; t++)
+  for (int t = 0; t < MORE; t++) {
 #pragma unroll
-    for (int i = 0; i < LOADS; i++) load(i, k0 + (uint32_t)t * 64u, t);
-  ring_wait<LOADS * (ST - 1)>();
+    for (int i = 0; i < LW; i++) if (t < ST) load_w(i, k0 + (uint32_t)t * 64u, t);
 #pragma unroll
-  for (int i = 0; i < NTN + NTM; i++) read(i, 0, 0);
-  uint32_t buf = 0, k = k0;
+    for (int i = 0; i < LX; i++) if (t < STX) load_x(i, k0 + (uint32_t)t * 64u, t);
+  }
+  ring_wait<STX * LX + ST * LW - LOADS>();
+  uint32_t bw = 0, bx = 0, k = k0;
+  if (PL == 1 && !on) {                            // a wave without tokens: its share of the loads, and the barriers
+    for (; k < k1; k += 64u, bw = bw + 1 == ST ? 0 : bw + 1, bx = bx + 1 == STX ? 0 : bx + 1) {
+      ring_wait<FLY>();
+#pragma unroll
+      for (int i = 0; i < LOADS; i++) load(i, k, bw, bx);
+    }
+    ring_wait<0>();
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < NTN + NTM; i++) read(i, 0, 0, 0);
   const auto walk = [&](uint32_t end) {
     for (; k < end; k += 64u) {
-      const uint32_t next = buf + 1 == ST ? 0 : buf + 1;
-      half(0, buf, 0, 0);
-      ring_wait<LOADS * (ST - 2)>();               // the next step's tiles have arrived, this step's are no longer read
-      half(1, next, k + ST * 64u, buf);
-      buf = next;
+      const uint32_t nw = bw + 1 == ST ? 0 : bw + 1, nx = STX == ST ? nw : bx + 1 == STX ? 0 : bx + 1;
+      half(0, bw, bx, 0, 0, 0);
+      ring_wait<FLY>();                            // the next step's tiles have arrived, this step's are no longer read
+      half(1, nw, nx, k, bw, bx);
+      bw = nw; bx = nx;
     }
   };
   if (PL == 3) {                                   // (a walk of its own: a condition in the steps cost 2 of 10 us at 16 x 512 x 512)

@@ -14,7 +14,7 @@ from adam_amd.engine import GenerationConfig
 from adam_amd.mixer_engine import MixerEngine
 from adam_amd.models import zaparax_config
 from adam_amd.safetensors_file import f32_to_bf16
-from gpu_util import f32map, note, read, up
+from gpu_util import f32map, note, read, rel_l2, up
 from mixer_cases import floats, rel, write_model
 from mixer_pair import CA, OP, ST, WS, WT, Pair
 from oracle import zaparax_np as Z
@@ -608,3 +608,46 @@ def test_sums_of_aligned_rows_are_those_of_shifted_ones(hip, E, I, top, shared, 
         hip.experts_dev(WS, OP, WT, up(hip, spec.words()), sh, rows)
         got.append(read(hip, WS, at["out"], rows * xs).reshape(rows, xs)[:, :width])
     assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,width,ff", [(256, 60, 16), (257, 130, 40), (383, 64, 300), (384, 200, 130), (385, 1040, 72), (511, 300, 600), (513, 192, 100)])
+def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
+    """One expert that every row takes: tiles of 256 rows whose last has none, a few or more than 128 of them, one step of columns to
+    seventeen, ragged in both directions: the words of the same rows in portions, which tiles of 64 take, and the product in 64 bits
+    within what bfloat16 activations give."""
+    note(f"experts of many rows {rows} width {width} ff {ff}")
+    rng = np.random.default_rng(rows + width)
+    ks, F, F16 = r64(width), r64(ff), (ff + 15) // 16 * 16
+    up_rows = np.zeros((2, F16, ks), np.float32)
+    up_rows[:, :ff, :width] = rng.standard_normal((2, ff, width)) / np.sqrt(width)
+    down = np.zeros((width, F), np.float32)
+    down[:, :ff] = rng.standard_normal((width, ff)) / np.sqrt(ff)
+    h = rng.standard_normal((rows, width)).astype(np.float32)
+    gu, dn, hb = f32_to_bf16(up_rows.reshape(2, -1, 16, ks).transpose(1, 0, 2, 3)), f32_to_bf16(down), f32_to_bf16(np.pad(h, ((0, 0), (0, ks - width))))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, gu.size + dn.size + 8)
+    hip.scatter_contiguous(WT, 0, np.concatenate([gu.reshape(-1), dn.reshape(-1)]))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * (ks + F) + 8)
+    hip.scatter_contiguous(OP, 0, hb.reshape(-1))
+    log, x, out = 4, 4 + 2 * rows, 4 + 2 * rows + rows * width
+    f32map(hip, WS, out + rows * width + 8, np.zeros(out, np.float32))
+    hip.scatter_contiguous(WS, x, h.reshape(-1))
+
+    def go(first, n):
+        spec = A.ExpertsSpec(experts=1, identity=0, top=1, ff=ff, ff_stride=F, width=width, k_stride=ks, gate_up=0, gate_up_step=2 * F16 * ks, down=gu.size,
+                             down_step=width * F, logits=log, logits_stride=2, correction=0, x=x + first * width, x_stride=width, opnd=first * ks, act=0,
+                             act_opnd=rows * ks, out=out + first * width, out_stride=width)
+        hip.experts_dev(WS, OP, WT, up(hip, spec.words()), 0, n)
+
+    go(0, rows)
+    whole = read(hip, WS, out, rows * width + 8)
+    hip.scatter_contiguous(WS, out, np.zeros(rows * width, np.float32))
+    for first in range(0, rows, 60):
+        go(first, min(60, rows - first))
+    parts = read(hip, WS, out, rows * width + 8)
+    assert not whole[rows * width:].any() and np.array_equal(whole.view(np.uint32), parts.view(np.uint32))
+    wide = lambda v: (v.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    hw, g = wide(hb), wide(f32_to_bf16(up_rows))
+    a = hw @ g[0].T
+    want = (a / (1 + np.exp(-a)) * (hw @ g[1].T))[:, :ff] @ wide(dn)[:, :ff].T
+    # (each activation is off by 2^-9 of itself at most, in no common direction: the whole by no more of its norm)
+    assert rel_l2(whole[:rows * width].reshape(rows, width), want) < 2.0 ** -9
