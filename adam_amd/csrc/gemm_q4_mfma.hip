@@ -18,6 +18,7 @@
 //
 // Tiled form: workgroup = NW waves, each with R tiles of 16 weight rows = 16 NW R weight rows x 16 MT activation
 // rows; one step = 128 weights of K (four blocks).
+// Narrow form (more than 64 activation rows of fewer than 2048 columns): 32 activation rows x 128 weight rows a workgroup.
 // Ring form (more than 64 activation rows): eight waves of 64 weight rows over 64, 96 or 128 activation rows, on 32x32x16
 // instructions, weights, scales and activations straight to a ring of LDS stages.
 // Either over shares of K, which k_gemm_splitk_sum adds up; gemm_plan says which.
@@ -533,6 +534,132 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
   }
   const uint32_t n[2] = {n0 + wave * 64u + r32, n0 + wave * 64u + 32u + r32};
   store_columns<MA, 16, 2>([&](int t, int i, int w) { return acc[w][t][i]; }, row, n, M, N, kz, c_off, out, part, segs);
+}
+
+// More than 64 activation rows and few columns, or few weight rows: tiles of 32 activation rows by 128 weight rows, so that a narrow matrix
+// still gives most CUs a workgroup.  A wave has 32 x 64 results of every fourth block: two waves side by side, four sharing out
+// the four blocks of a step of 128 columns, whose sums meet in LDS in the order of the blocks' places.  A workgroup's step (16 KB of both planes
+// of the activations, 8 of weights, 1 of scales) goes straight to LDS, a ring of three stages (four to six: 0.1 to 0.7 us slower); a wave reads the next
+// step's operands, and adds up the products of the one before, under the products of this one (added up behind its own: a fifth slower over long rows).
+// What bounds it: a step takes 0.44 us with a few workgroups, 0.65 with one on every CU, of which the products need 0.21; the rest is the
+// vector work beside them (unpacking for 32 rows only, a multiply-add per result and block) and, with many workgroups, the activations' way out of the L2s.
+// Against the tiled kernel, whose step of 128 columns waits for its loads (1.3 us): 512 x 1536 x 1152 16.2 -> 10.9 us, 189 x 1536 x 1152 15.1 -> 9.8, 189 x 1152
+// x 1024 13.8 -> 9.4, 70 x 13824 x 1152 22.3 -> 18.9.
+// LDS: piece j of an activation row at j ^ (row & 15), block j of a weight row at j ^ (row / 4 & 3): no two rows that are read together meet in a bank.
+#define NARROW_X 16384u
+#define NARROW_W 8192u
+#define NARROW_STAGE (NARROW_X + NARROW_W + 1024u)
+__global__ void __launch_bounds__(512)
+k_gemm_q4_narrow(const uint8_t* __restrict__ W, const __half* __restrict__ d16, const u4q_t* __restrict__ xh, const u4q_t* __restrict__ xl,
+                 uint32_t K, uint32_t N, uint32_t M, uint32_t gbase, uint32_t c_val, uint32_t by_val, float* out, const uint32_t* __restrict__ lc,
+                 const float* __restrict__ scale, GemmSegs segs) {
+  constexpr int LOADS = 4;                                   // of a wave and stage: 2 of activations, 1 of weights, 1 of scales (which two waves ask for)
+  constexpr uint32_t ST = 3;
+  static_assert(ST * NARROW_STAGE >= 65536u, "the sums' way over LDS");
+  __shared__ __attribute__((aligned(16))) uint8_t ring[ST * NARROW_STAGE];
+  const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t r32 = lane & 31u, h = lane >> 5, side = wave & 1u, kb = wave >> 1;
+  // workgroups land on the eight dies in turn: a die takes a run of tiles, those of the same activation rows next to each other
+  const uint32_t tiles_n = (N + 127u) / 128u, id = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const uint32_t n0 = id % tiles_n * 128u, m0 = id / tiles_n * 32u;
+  if (m0 >= M) return;
+  const uint32_t nblk = K >> 5, steps = K >> 7;
+  const uint32_t base = lds_byte(ring);
+
+  // a load is a base for the wave and an offset for the lane
+  uint32_t xo[2];
+#pragma unroll
+  for (uint32_t u = 0; u < 2; u++) {                         // 4 rows of 256 bytes an instruction; LDS: [plane][row][16 pieces]
+    const uint32_t row = ((wave * 2u + u) & 7u) * 4u + (lane >> 4);
+    xo[u] = (min(m0 + row, M - 1u) * (K >> 3) + ((lane & 15u) ^ (row & 15u))) << 4;
+  }
+  const uint32_t wr = wave * 16u + (lane >> 2), sr = (wave & 3u) * 32u + (lane >> 1);
+  const uint32_t wo = (min(n0 + wr, N - 1u) * nblk + ((lane & 3u) ^ (wr >> 2 & 3u))) << 4;       // 16 rows of 64 bytes; LDS: [row][4 blocks]
+  const uint32_t so = (min(n0 + sr, N - 1u) * nblk + (lane & 1u) * 2u) * 2u;                     // 32 rows of 8 bytes; LDS: [row][4]
+  const u4q_t* const xp = wave >= 4u ? xl : xh;
+  const auto load = [&](int i, uint32_t s, uint32_t into) {  // (steps past the end re-read the last: the count in flight stays)
+    const uint64_t st = min(s, steps - 1u);
+    const uint32_t at = base + into * NARROW_STAGE;
+    if (i < 2) load_to_lds(xp + st * 16u, xo[i], at + (wave * 2u + i) * 1024u);
+    else if (i == 2) load_to_lds(W + (((uint64_t)gbase + st * 4u) << 4), wo, at + NARROW_X + wave * 1024u);
+    else load4_to_lds(d16 + gbase + st * 4u, so, at + NARROW_X + NARROW_W + (wave & 3u) * 256u);
+  };
+
+  f16q_t acc[2], blk[2][2], zero;                            // blk: a block's products, [step's parity][tile]
+#pragma unroll
+  for (int i = 0; i < 16; i++) { zero[i] = 0.f; acc[0][i] = 0.f; acc[1][i] = 0.f; blk[1][0][i] = 0.f; blk[1][1][i] = 0.f; }
+  DEQK_INIT(dk);
+  u4q_t x[2][4], raw[2][2];                                  // [step's parity][plane, half of the block], [..][tile]
+  _Float16 ds[2][2];
+  float d[2] = {0.f, 0.f};
+  const auto add = [&](int p, int i0, int i1) {              // results i0 .. i1 of both tiles, each block's sum by its scale
+#pragma unroll
+    for (int i = i0; i < i1; i++) acc[i >> 4][i & 15] = fmaf(blk[p][i >> 4][i & 15], d[i >> 4], acc[i >> 4][i & 15]);
+  };
+  const auto read = [&](int i, int p, uint32_t buf) {
+    const uint8_t* const st = ring + buf * NARROW_STAGE;
+    if (i < 4) x[p][i] = *(const u4q_t*)(st + (i >> 1) * 8192u + r32 * 256u + (((4u * kb + 2u * (i & 1) + h) ^ (r32 & 15u)) << 4));
+    else {
+      const uint32_t row = side * 64u + (i - 4) * 32u + r32;
+      raw[p][i - 4] = *(const u4q_t*)(st + NARROW_X + row * 64u + ((kb ^ (row >> 2 & 3u)) << 4));
+      ds[p][i - 4] = *(const _Float16*)(st + NARROW_X + NARROW_W + row * 8u + kb * 2u);
+    }
+  };
+#pragma unroll
+  for (uint32_t s = 0; s < ST; s++)
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) load(i, s, s);
+  ring_wait<LOADS * (ST - 1)>();
+#pragma unroll
+  for (int i = 0; i < 6; i++) read(i, 0, 0);
+  uint32_t buf = 0;
+  const auto step = [&](int p, uint32_t s) {
+    const uint32_t next = buf + 1u == ST ? 0u : buf + 1u;
+    ring_wait<LOADS * (ST - 2)>();                           // the next step is here, this one's operands are in registers
+    u4q_t wf[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      wf[t][0] = deq_word(h ? raw[p][t].y : raw[p][t].x, dk);
+      wf[t][1] = deq_word(h ? raw[p][t].w : raw[p][t].z, dk);
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+#pragma unroll
+      for (int t = 0; t < 2; t++) blk[p][t] = MFMA32_F16(x[p][m], wf[t][m & 1], m ? blk[p][t] : zero);
+      add(1 - p, 8 * m, 8 * m + 8);                          // (of the step before: its products are there)
+      if (m < 3) { read(2 * m, 1 - p, next); read(2 * m + 1, 1 - p, next); }
+      load(m, s + ST, buf);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    d[0] = (float)ds[p][0]; d[1] = (float)ds[p][1];
+    buf = next;
+  };
+  for (uint32_t s = 0; s < steps; s += 2u) {
+    step(0, s);
+    if (s + 1u < steps) step(1, s + 1u);
+  }
+  if (steps & 1u) add(0, 0, 32); else add(1, 0, 32);
+  ring_wait<0>();
+  // the waves' sums: eight results of each lane a wave, quads of them beside each other
+  f4q_t* const sums = (f4q_t*)ring;
+#pragma unroll
+  for (int q = 0; q < 8; q++)
+    sums[(wave * 8u + q) * 64u + lane] = (f4q_t){acc[q >> 2][4 * (q & 3)], acc[q >> 2][4 * (q & 3) + 1], acc[q >> 2][4 * (q & 3) + 2], acc[q >> 2][4 * (q & 3) + 3]};
+  __syncthreads();
+  f4q_t y[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    f4q_t v[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; k++) v[k] = sums[((k * 2u + side) * 8u + kb * 2u + q) * 64u + lane];
+    y[q] = ((v[0] + v[1]) + v[2]) + v[3];
+  }
+  const auto row = [&](int, int i) { return m0 + 16u * (kb & 1u) + 8u * (i >> 2) + 4u * h + (i & 3u); };
+#pragma unroll
+  for (int i = 0; i < 8; i++) y[i >> 2][i & 3] *= scale[2 * (uint64_t)min(row(0, i), M - 1u) + 1];
+  const uint64_t c_off = (by_val & 2u) || segs.count ? (uint64_t)c_val : (uint64_t)lc[0];
+  const uint32_t n[1] = {n0 + side * 64u + (kb >> 1) * 32u + r32};
+  store_columns<1, 8, 1>([&](int, int i, int) { return y[i >> 2][i & 3]; }, row, n, M, N, 0u, c_off, out, nullptr, segs);
 }
 
 // 2 .. 64 activation rows: the weights are read once, so what counts is how fast they stream, and what stands in its way is
@@ -1317,8 +1444,8 @@ bool launch_attn_merge_rows_f16(const Map* ma, const float* partial, uint32_t o0
 // survive into a later state with the same count).
 void gemm_act_forget() { g_xh_key.valid = false; }
 
-// How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 0
-// k_gemm_q4_ring<ma>, 0 the tiled kernel, over how many shares of K; -1 k_gemm_q4_rows.
+// How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 1
+// k_gemm_q4_ring<ma>, 1 k_gemm_q4_narrow, 0 the tiled kernel, over how many shares of K; -1 k_gemm_q4_rows.
 // 33 .. 64 rows: k_gemm_q4_rows where a CU has few tiles of 16 weight rows and K is not long, by its time for a round of tiles and
 // a 128-column step (48 rows: 4096 x 4096 12.3 us, tiled 21.7, 6144 x 4096 14.9 and 23.8; 4096 x 14336 38.0 and 34.1; 64 rows:
 // 28672 x 4096 71.9 and 67.7).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
@@ -1337,6 +1464,10 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // The ring reads the scales of two blocks as one word and keeps a lane's place in the rows in 32 bits (in the matrix too: a Q4
 // map here has fewer than 2^32 elements): matrices that begin at an odd block stay on the tiled kernel, a narrow one from 128
 // rows on over 2 .. 4 shares (256 x 128 tile; 512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four).
+// Rows of fewer than 2048 columns: also k_gemm_q4_narrow, in steps of 128 columns of 0.42 us with few workgroups, 0.67 with one on every CU, and 3
+// a round of workgroups beside them (512 x 1536 x 1152 estimated 11.5 us, measured 10.9, tiled 16.2; 189 x 13824 x 1152 30.1, 28.7, tiled 29.9;
+// 512 x 13824 x 1152 66, 62, ring 42).  Longer rows go to the ring over shares of K, which is the better one where there are many of them and
+// where the matrix is narrow: 512 x 4096 x 4096 50 us and here 55, 70 x 1152 x 6912 23 and 30 (between them not everywhere: 189 x 4096 x 4096 31 and 26).
 struct GemmPlan { int ma; uint32_t shares; };
 static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   const auto up = [](uint64_t x, uint64_t y) { return (x + y - 1) / y; };
@@ -1365,8 +1496,14 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
     while (sp > 1 && K / sp < 1024u) sp--;
     return {0, sp > 1 && w * sp * 4 >= 3 * cu ? (uint32_t)sp : 1u};
   }
+  if (ring == 3) return {1, 1};
   if (ring == 2) best = 1e30;
   GemmPlan p = {0, 1};
+  if (ring == 1 && K < 2048) {
+    const uint64_t tiles = wgs(128, 32);
+    const double full = std::min(1.0, (double)tiles / (double)cu), us = 3.0 + (double)up(tiles, cu) * ((0.42 + 0.25 * full) * (double)steps + 3.0);
+    if (us < best) { best = us; p = {1, 1}; }
+  }
   for (int ma = 2; ma <= 4; ma++) {
     const uint64_t tiles = wgs(512, 32 * (uint64_t)ma);
     for (uint64_t sp = 1; sp <= most && (sp == 1 || (sp * 4 <= pairs && tiles * sp <= cu)); sp++) {
@@ -1498,6 +1635,13 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
   if (plan.shares > 1 && !ensure_part_buf((size_t)plan.shares * M * N)) {
     if (sg.add) return ADAMAH_ERR_MEMORY;        // (the tiled kernel in one launch stores no add)
     plan = {0, 1};
+  }
+  if (plan.ma == 1) {
+    const uint32_t run = cdiv(cdiv(N, 128) * cdiv(M, 32), 8);
+    k_gemm_q4_narrow<<<run * 8, 512, 0, g.stream>>>(mw->buf, mw->d16, (const u4q_t*)xh, (const u4q_t*)xl, K, N, M, (uint32_t)(b_host >> 5), c_val, by_val, act, lc, g_scale_buf, sg);
+    count_launch();
+    keep();
+    return check_launch();
   }
   if (plan.ma) {
     const uint32_t pairs = K >> 6, per = cdiv(pairs, plan.shares), shares = cdiv(pairs, per);

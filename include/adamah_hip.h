@@ -438,7 +438,7 @@ int adamah_hip_debug_dequant(uint32_t map_id, uint64_t start, uint64_t count, fl
 /* 0 = affine qparams only, 1 = fp16-scale block plane in use for the whole map, <0 = error. */
 int adamah_hip_map_layout(uint32_t map_id);
 /* How a Q4 matmul of rows activation rows (more than 64) by weights [n, k] from element base on would run: *tile activation rows a
- * workgroup of the ring kernel, 0 the tiled kernel; *shares of k, added up by a launch of their own if more than one. */
+ * workgroup of the ring kernel, 32 the narrow kernel, 0 the tiled kernel; *shares of k, added up by a launch of their own if more than one. */
 int adamah_hip_matmul_plan(uint32_t rows, uint32_t k, uint32_t n, uint64_t base, uint32_t* tile, uint32_t* shares);
 
 #ifdef __cplusplus

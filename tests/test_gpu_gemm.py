@@ -557,7 +557,12 @@ def test_ring_stores_stacked_results_and_adds_in_one_share(hip, monkeypatch, M, 
     monkeypatch.setenv("ADAMAH_GEMM_RING", "2")
     monkeypatch.setenv("ADAMAH_GEMM_SPLITK", "0")
     assert hip.matmul_plan(M, K, sum(Ns)) == (tile, 1)
-    note(f"gemm q4 ring, one share M={M} K={K} Ns={Ns} add={add}")
+    check_stacked_and_adds(hip, M, K, Ns, add, "ring, one share")
+
+
+def check_stacked_and_adds(hip, M, K, Ns, add, what):
+    """Results of stacked matrices, or one and the add behind it, in two launches with the conversion."""
+    note(f"gemm q4 {what} M={M} K={K} Ns={Ns} add={add}")
     rng = np.random.default_rng(M + sum(Ns))
     W = load_from(hip, rng, sum(Ns), K, 0)
     x = rng.standard_normal((M, K), dtype=np.float32)
@@ -631,6 +636,23 @@ def test_ring_off_leaves_the_tiled_kernel_its_shares(hip, monkeypatch):
         hip.batch_end()
         assert hip.get_last_barrier_count() == launches, (ring, split)
         assert rel_l2(read(hip, 0, M * K, M * N).reshape(M, N), want) < TOL_Q4, (ring, split)
+
+
+@pytest.mark.parametrize("M,N,K,base", [(65, 129, 128, 0), (96, 127, 256, 64), (257, 1000, 384, 64), (189, 13823, 640, 0), (512, 1536, 1152, 128), (100, 33, 1920, 0),
+                                        (333, 1152, 4096, 64), (4099, 60, 256, 0)])
+def test_narrow_tiles_at_ragged_ends(hip, monkeypatch, M, N, K, base):
+    """The tiles of 32 activation rows by 128 weight rows, one step of columns to more than the ring has stages, an odd number of them and an
+    even one, rows past the last tile in both directions, fewer tiles than there are dies and more than there are CUs."""
+    monkeypatch.setenv("ADAMAH_GEMM_RING", "3")
+    assert hip.matmul_plan(M, K, N, base) == (32, 1)
+    test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
+
+
+@pytest.mark.parametrize("M,K,Ns,add", [(70, 384, (500, 36, 700), False), (189, 1152, (1024, 256, 256), False), (301, 1152, (1152,), True), (66, 256, (31,), True)])
+def test_narrow_tiles_store_stacked_results_and_adds(hip, M, K, Ns, add):
+    """What the rule sends there: borders of stacked matrices inside a workgroup's 128 weight rows, and the add behind a single one."""
+    assert hip.matmul_plan(M, K, sum(Ns)) == (32, 1)
+    check_stacked_and_adds(hip, M, K, Ns, add, "narrow tiles")
 
 
 @pytest.mark.parametrize("M,N,K", [(200, 31300, 128), (256, 32000, 256), (100, 31300, 1024), (130, 24100, 256), (1000, 4700, 128)])
