@@ -16,6 +16,9 @@
 // softmax per wave and query; values with every lane owning D/64 dims of all 16 outputs.  The waves
 // merge through LDS.  The raw scores of the chunk's last token are stored to the score rows: that
 // is what the rows hold after the run executed token by token, each token overwriting the one before.
+// Bound by latency (queries, first tile, LDS), so by how many waves a CU holds: the weights of all 16 cache rows used to be in registers at once
+// (256 of them, a wave a SIMD), the sums having been moved behind them, and a thread's queries were waited for one by one.  8 runs of 48 tokens
+// over 32 heads of 128: 32.2 us, 26.7 with the queries asked for together, 15.4 with 142 registers (three waves a SIMD) as well.
 #include "attn_common.h"
 #include <algorithm>
 
@@ -93,16 +96,24 @@ k_attn_prefill(const float* data, float* out, const __half* kv, uint64_t kv_shif
     float* qs = &obuf[0][0][0];
     if (tid < 16u) hmax[tid] = 0u;
     __syncthreads();
-    for (uint32_t i = tid; i < 16u * D; i += NT) {          // a wave's 64 elements belong to one query
-      const uint32_t r = i / D;
-      const float x = r < rows ? data[(uint64_t)bs.q[head] + (uint64_t)(t0 + r) * q_stride + i % D] : 0.f;
-      qs[i] = x;
-      float mx = fabsf(x);
-      mx = wave_max(mx);
-      if (lane == 0u) atomicMax(&hmax[r], __float_as_uint(mx));
+    // all of them are asked for, and the first tile behind them, before one is waited for
+    constexpr uint32_t QL = 16u * D / NT;
+    float x[QL];
+#pragma unroll
+    for (uint32_t u = 0; u < QL; u++) {                     // a wave's 64 elements belong to one query
+      const uint32_t i = tid + u * NT;
+      x[u] = data[(uint64_t)bs.q[head] + (uint64_t)(t0 + min(i / D, rows - 1u)) * q_stride + i % D];
     }
     if (rbase < nkeys) fetch(kA, vA, rbase);
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (uint32_t u = 0; u < QL; u++) {
+      const uint32_t i = tid + u * NT, r = i / D;
+      if (r >= rows) x[u] = 0.f;
+      qs[i] = x[u];
+      const float mx = wave_max(fabsf(x[u]));
+      if (lane == 0u) atomicMax(&hmax[r], __float_as_uint(mx));
+    }
     __syncthreads();
     const uint32_t e = (hmax[c] >> 23) & 0xFFu;
     float s = 1.f, inv = 1.f;
@@ -181,8 +192,17 @@ k_attn_prefill(const float* data, float* out, const __half* kv, uint64_t kv_shif
 #pragma unroll
       for (int j = 0; j < DPL; j++) acc[h][j] *= al;
     }
+    // the weights of one cache row ahead, no more: the compiler would fetch all 16 rows' (256 registers) at once
+    float4 pw[2][4];
+    const auto weights = [&](int u) {
+#pragma unroll
+      for (int h4 = 0; h4 < 4; h4++) pw[u & 1][h4] = *(const float4*)&pbuf[wave][u][4 * h4];
+    };
+    weights(0);
 #pragma unroll
     for (int u = 0; u < 16; u++) {
+      if (u < 15) weights(u + 1);
+      __builtin_amdgcn_sched_barrier(0);
       float f[DPL];
       if (DPL == 1) f[0] = __half2float(__ushort_as_half((unsigned short)vA[u][0]));
       else {
@@ -194,15 +214,19 @@ k_attn_prefill(const float* data, float* out, const __half* kv, uint64_t kv_shif
       }
 #pragma unroll
       for (int h4 = 0; h4 < 4; h4++) {
-        const float4 pw = *(const float4*)&pbuf[wave][u][4 * h4];
+        const float4 p4 = pw[u & 1][h4];
 #pragma unroll
         for (int j = 0; j < DPL; j++) {
-          acc[4 * h4 + 0][j] = fmaf(pw.x, f[j], acc[4 * h4 + 0][j]);
-          acc[4 * h4 + 1][j] = fmaf(pw.y, f[j], acc[4 * h4 + 1][j]);
-          acc[4 * h4 + 2][j] = fmaf(pw.z, f[j], acc[4 * h4 + 2][j]);
-          acc[4 * h4 + 3][j] = fmaf(pw.w, f[j], acc[4 * h4 + 3][j]);
+          acc[4 * h4 + 0][j] = fmaf(p4.x, f[j], acc[4 * h4 + 0][j]);
+          acc[4 * h4 + 1][j] = fmaf(p4.y, f[j], acc[4 * h4 + 1][j]);
+          acc[4 * h4 + 2][j] = fmaf(p4.z, f[j], acc[4 * h4 + 2][j]);
+          acc[4 * h4 + 3][j] = fmaf(p4.w, f[j], acc[4 * h4 + 3][j]);
         }
       }
+#pragma unroll
+      for (int h = 0; h < 16; h++)
+#pragma unroll
+        for (int j = 0; j < DPL; j++) asm volatile("" : "+v"(acc[h][j]));      // (here, not where the sums are next used, with all the weights kept for it)
     }
     __builtin_amdgcn_wave_barrier();
     if (rbase + NW * 16u < nkeys) fetch(kA, vA, rbase + NW * 16u);
