@@ -129,105 +129,166 @@ k_topk_merge(float* data, const float* __restrict__ part_v, const uint32_t* __re
 }
 
 
-// Top-k of 4096 < n <= 40960 candidates in one launch: radix selection instead of k rounds.  A candidate's place in
-// the strict order (value descending, index ascending) is the 48-bit key (orderable value bits, 0xFFFF - index); five
-// histogram passes over its digits (11, 11, 10 bits of the value, then 8, 8 of the index, top down) find the key of the k-th best -- each pass counts
+// Top-k of 4096 < n <= 40960 candidates in one launch of one workgroup of 1024 threads, the values in registers (at most 40 per
+// thread).  A candidate's place in the strict order (value descending, index ascending) is the 48-bit key (orderable value bits, 0xFFFF - index).
+// Sixteen threads' candidates are a group: the k-th largest of the 64 groups' largest values has at least k candidates at or above it,
+// and hardly more than a hundred, which are listed and put in order by counting.  Where more than TSEL_LIST are (many equal values),
+// radix selection: five histogram passes over its digits (11, 11, 10 bits of the value, then 8, 8 of the index, top down) find the key of the k-th best -- each pass counts
 // the candidates that agree with the digits fixed so far, a suffix scan over the bins finds the bin the k-th falls in --
-// and everything at or above that key is gathered and put in order by counting.  One workgroup of 1024 threads, the
-// values in registers (at most 40 per thread).  Same results as the rounds (tests/test_gpu_sampling.py); the partial
-// lists of the sampled LM head (40960 candidates, k = 40) take 145 us in rounds; here 59 with each load under a condition and one
+// and everything at or above that key is gathered and put in order by counting.  Same results as the rounds
+// (tests/test_gpu_sampling.py).  Bound by latency: the partial lists of the sampled LM head (40960 candidates, k = 40) take 17.4 us, 41 by
+// radix selection alone (in no order in the map 29 and 51; 10240 of them 14.7 and 27; all equal 69 and 60); that one took 59 with each load under a condition and one
 // count a bin, 41 with loads on every path, TSEL_ASK at a time, and four counts a bin (the values share few bins of the first
 // passes, and a wave's counts of one address go one behind the other).
 #define TSEL_THREADS 1024u
 #define TSEL_PER 40u
 #define TSEL_ASK 20u
+typedef uint32_t u4l_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f4l_t __attribute__((ext_vector_type(4), aligned(4)));
+#define TSEL_LIST 1024u
 __global__ void __launch_bounds__(1024)
 k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __restrict__ li, const uint32_t* __restrict__ lv,
               uint32_t n, uint32_t k, uint64_t n_elems) {
   __shared__ uint4 hist[2048];                  // a bin's counts of the lanes with the same two last bits
   __shared__ uint32_t wtot[16];
-  __shared__ uint32_t sel_bin, sel_rem, n_win;
+  __shared__ uint32_t sel_bin, sel_rem, n_win, n_list, largest[64], to_i[SMP_MAX], to_v[SMP_MAX];
   __shared__ float win_v[SMP_MAX];
   __shared__ uint32_t win_i[SMP_MAX];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-  const uint32_t per = (n + TSEL_THREADS - 1u) / TSEL_THREADS;
-  uint32_t vk[TSEL_PER];   // orderable value bits of candidate u * 1024 + tid
+  // Four neighbouring candidates a load: chunk c begins at 4 c, the last one at n - 4 (what of it belongs to the one before does not count)
+  const uint32_t per = (n + 4u * TSEL_THREADS - 1u) / (4u * TSEL_THREADS);      // chunks a thread
+  uint32_t at = 4u * tid;
+  const auto anew = [&] { asm volatile("" : "+v"(at)); };      // places are worked out once more, not kept in registers from loop to loop
+  const auto first = [&](uint32_t u) { return at + u * (4u * TSEL_THREADS); };
+  const auto place = [&](uint32_t u) { return min(first(u), n - 4u); };         // candidate u's e-th is place(u) + e, there if that is at least first(u)
+  if (tid < k) { to_i[tid] = li[tid]; to_v[tid] = lv[tid]; }
+  if (tid == 0) { n_win = 0u; n_list = 0u; }
+  uint32_t vk[TSEL_PER];   // orderable value bits of candidate place(j / 4) + j % 4
 #pragma unroll
-  for (uint32_t u0 = 0; u0 < TSEL_PER; u0 += TSEL_ASK) {
+  for (uint32_t u0 = 0; u0 < TSEL_PER / 4u; u0 += TSEL_ASK / 4u) {
     if (u0 < per) {
-      uint32_t l[TSEL_ASK];
-      float x[TSEL_ASK];
+      u4l_t l[TSEL_ASK / 4u];
+      f4l_t x[TSEL_ASK / 4u];
+      bool run = true;                          // the four lie beside each other in the map
 #pragma unroll
-      for (uint32_t j = 0; j < TSEL_ASK; j++) l[j] = ls[min((u0 + j) * TSEL_THREADS + tid, n - 1u)];
+      for (uint32_t j = 0; j < TSEL_ASK / 4u; j++) l[j] = *(const u4l_t*)(ls + place(u0 + j));
 #pragma unroll
-      for (uint32_t j = 0; j < TSEL_ASK; j++) x[j] = data[min((uint64_t)l[j], n_elems - 1u)];
+      for (uint32_t j = 0; j < TSEL_ASK / 4u; j++)
+        run = run && l[j][1] == l[j][0] + 1u && l[j][2] == l[j][0] + 2u && l[j][3] == l[j][0] + 3u && l[j][0] < l[j][3] && l[j][3] < n_elems;
+      if (__all(run)) {
+#pragma unroll
+        for (uint32_t j = 0; j < TSEL_ASK / 4u; j++) x[j] = *(const f4l_t*)(data + l[j][0]);
+      } else {
+#pragma unroll
+        for (uint32_t j = 0; j < TSEL_ASK; j++) x[j / 4u][j % 4u] = data[min((uint64_t)l[j / 4u][j % 4u], n_elems - 1u)];
+      }
 #pragma unroll
       for (uint32_t j = 0; j < TSEL_ASK; j++) {
-        const float y = l[j] < n_elems && x[j] == x[j] ? x[j] : SMP_NEG_INF;
+        const float v = x[j / 4u][j % 4u], y = l[j / 4u][j % 4u] < n_elems && v == v ? v : SMP_NEG_INF;
         const uint32_t b = __float_as_uint(y);
-        vk[u0 + j] = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+        vk[4u * u0 + j] = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
       }
     } else {
 #pragma unroll
-      for (uint32_t j = 0; j < TSEL_ASK; j++) vk[u0 + j] = 0u;
+      for (uint32_t j = 0; j < TSEL_ASK; j++) vk[4u * u0 + j] = 0u;
     }
     __builtin_amdgcn_sched_barrier(0);
   }
   const uint32_t kk = min(k, n);
-  const uint32_t inv0 = 0xFFFFu - tid;          // index digits of candidate u: inv0 - u * 1024 (lower index = larger)
-  uint32_t prefix = 0, mask = 0, iprefix = 0, imask = 0;
-  uint32_t remaining = kk;
-#pragma unroll 1
-  for (uint32_t pass = 0; pass < 5u; pass++) {
-    const bool on_idx = pass >= 3u;             // passes 0..2: value bits 31..21, 20..10, 9..0; 3, 4: index bits 15..8, 7..0
-    const uint32_t sh = pass == 0u ? 21u : pass == 1u ? 10u : pass == 3u ? 8u : 0u;
-    const uint32_t bm = pass < 2u ? 2047u : pass == 2u ? 1023u : 255u;
-    hist[2u * tid] = make_uint4(0u, 0u, 0u, 0u); hist[2u * tid + 1u] = make_uint4(0u, 0u, 0u, 0u);
-    __syncthreads();
-    uint32_t inv = inv0, idx = tid;
-    asm volatile("" : "+v"(inv), "+v"(idx));   // per pass, so that the 40 index digits are not all kept in registers
+  anew();
+  uint32_t top = 0u;                            // (below every value's bits)
 #pragma unroll
-    for (uint32_t u = 0; u < TSEL_PER; u++) {
-      if (u < per && idx + u * TSEL_THREADS < n) {
-        const uint32_t iv = inv - u * TSEL_THREADS;
-        const bool in = on_idx ? (vk[u] == prefix && (iv & imask) == iprefix) : ((vk[u] & mask) == prefix);
-        if (in) atomicAdd((uint32_t*)&hist[((on_idx ? iv : vk[u]) >> sh) & bm] + (tid & 3u), 1u);
+  for (uint32_t j = 0; j < TSEL_PER; j++) if (j / 4u < per && place(j / 4u) + j % 4u >= first(j / 4u)) top = max(top, vk[j]);
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+  if ((tid & 15u) == 0u) largest[tid >> 4] = top;
+  __syncthreads();
+  const uint32_t mine = largest[lane];          // every wave for itself: which lane holds the kk-th largest
+  uint32_t before = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < 64u; j++) {
+    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j);
+    before += other > mine || (other == mine && j < lane) ? 1u : 0u;
+  }
+  const uint32_t least = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)__builtin_ctzll(__ballot(before == kk - 1u)));
+  unsigned long long* const list = (unsigned long long*)hist;
+  anew();
+#pragma unroll
+  for (uint32_t j = 0; j < TSEL_PER; j++) {
+    const uint32_t i = place(j / 4u) + j % 4u;
+    if (j / 4u < per && i >= first(j / 4u) && vk[j] >= least) {
+      const uint32_t slot = atomicAdd(&n_list, 1u);
+      if (slot < TSEL_LIST) list[slot] = (unsigned long long)vk[j] << 32 | (0xFFFFFFFFu - i);
+    }
+  }
+  __syncthreads();
+  const uint32_t listed = n_list;
+  if (listed <= TSEL_LIST) {
+    if (tid < listed) {
+      const unsigned long long key = list[tid];
+      uint32_t rank = 0;
+#pragma unroll 8
+      for (uint32_t j = 0; j < listed; j++) rank += list[j] > key ? 1u : 0u;
+      if (rank < kk) {
+        const uint32_t bits = (uint32_t)(key >> 32);
+        win_v[rank] = __uint_as_float((bits & 0x80000000u) ? (bits & 0x7FFFFFFFu) : ~bits);
+        win_i[rank] = 0xFFFFFFFFu - (uint32_t)key;
       }
     }
-    __syncthreads();
-    // suffix sums over the bins (two per thread), top down: the bin in which the count reaches `remaining`
-    const uint4 c0 = hist[2u * tid], c1 = hist[2u * tid + 1u];
-    const uint32_t h0 = c0.x + c0.y + c0.z + c0.w, h1 = c1.x + c1.y + c1.z + c1.w, own = h0 + h1;
-    uint32_t suf = own;   // inclusive suffix sum within the wave
+    if (tid == 0) n_win = kk;
+  } else {
+    uint32_t prefix = 0, mask = 0, iprefix = 0, imask = 0;
+    uint32_t remaining = kk;
+#pragma unroll 1
+    for (uint32_t pass = 0; pass < 5u; pass++) {
+      const bool on_idx = pass >= 3u;             // passes 0..2: value bits 31..21, 20..10, 9..0; 3, 4: index bits 15..8, 7..0
+      const uint32_t sh = pass == 0u ? 21u : pass == 1u ? 10u : pass == 3u ? 8u : 0u;
+      const uint32_t bm = pass < 2u ? 2047u : pass == 2u ? 1023u : 255u;
+      hist[2u * tid] = make_uint4(0u, 0u, 0u, 0u); hist[2u * tid + 1u] = make_uint4(0u, 0u, 0u, 0u);
+      __syncthreads();
+      anew();
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t t = __shfl_down(suf, o, 64);
-      if (lane + (uint32_t)o < 64u) suf += t;
-    }
-    if (lane == 0u) wtot[wave] = suf;
-    __syncthreads();
-    for (uint32_t w = wave + 1u; w < 16u; w++) suf += wtot[w];
-    const uint32_t above = suf - own;
-    if (above < remaining && remaining <= suf) {
-      if (above + h1 >= remaining) { sel_bin = 2u * tid + 1u; sel_rem = remaining - above; }
-      else { sel_bin = 2u * tid; sel_rem = remaining - above - h1; }
-    }
-    __syncthreads();
-    if (on_idx) { iprefix |= sel_bin << sh; imask |= bm << sh; }
-    else { prefix |= sel_bin << sh; mask |= bm << sh; }
-    remaining = sel_rem;
-  }
-  // (prefix, iprefix) is now the key of the kk-th best: everything at or above it wins
-  if (tid == 0) n_win = 0u;
-  __syncthreads();
+      for (uint32_t j = 0; j < TSEL_PER; j++) {
+        const uint32_t i = place(j / 4u) + j % 4u, iv = 0xFFFFu - i;
+        if (j / 4u < per && i >= first(j / 4u)) {
+          const bool in = on_idx ? (vk[j] == prefix && (iv & imask) == iprefix) : ((vk[j] & mask) == prefix);
+          if (in) atomicAdd((uint32_t*)&hist[((on_idx ? iv : vk[j]) >> sh) & bm] + (tid & 3u), 1u);
+        }
+      }
+      __syncthreads();
+      // suffix sums over the bins (two per thread), top down: the bin in which the count reaches `remaining`
+      const uint4 c0 = hist[2u * tid], c1 = hist[2u * tid + 1u];
+      const uint32_t h0 = c0.x + c0.y + c0.z + c0.w, h1 = c1.x + c1.y + c1.z + c1.w, own = h0 + h1;
+      uint32_t suf = own;   // inclusive suffix sum within the wave
 #pragma unroll
-  for (uint32_t u = 0; u < TSEL_PER; u++) {
-    const uint32_t i = u * TSEL_THREADS + tid;
-    if (u < per && i < n && (vk[u] > prefix || (vk[u] == prefix && inv0 - u * TSEL_THREADS >= iprefix))) {
-      const uint32_t slot = atomicAdd(&n_win, 1u);
-      if (slot < SMP_MAX) {
-        const uint32_t b = (vk[u] & 0x80000000u) ? (vk[u] & 0x7FFFFFFFu) : ~vk[u];
-        win_v[slot] = __uint_as_float(b); win_i[slot] = i;
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = __shfl_down(suf, o, 64);
+        if (lane + (uint32_t)o < 64u) suf += t;
+      }
+      if (lane == 0u) wtot[wave] = suf;
+      __syncthreads();
+      for (uint32_t w = wave + 1u; w < 16u; w++) suf += wtot[w];
+      const uint32_t above = suf - own;
+      if (above < remaining && remaining <= suf) {
+        if (above + h1 >= remaining) { sel_bin = 2u * tid + 1u; sel_rem = remaining - above; }
+        else { sel_bin = 2u * tid; sel_rem = remaining - above - h1; }
+      }
+      __syncthreads();
+      if (on_idx) { iprefix |= sel_bin << sh; imask |= bm << sh; }
+      else { prefix |= sel_bin << sh; mask |= bm << sh; }
+      remaining = sel_rem;
+    }
+    anew();
+    // (prefix, iprefix) is now the key of the kk-th best: everything at or above it wins
+#pragma unroll
+    for (uint32_t j = 0; j < TSEL_PER; j++) {
+      const uint32_t i = place(j / 4u) + j % 4u;
+      if (j / 4u < per && i >= first(j / 4u) && (vk[j] > prefix || (vk[j] == prefix && 0xFFFFu - i >= iprefix))) {
+        const uint32_t slot = atomicAdd(&n_win, 1u);
+        if (slot < SMP_MAX) {
+          const uint32_t b = (vk[j] & 0x80000000u) ? (vk[j] & 0x7FFFFFFFu) : ~vk[j];
+          win_v[slot] = __uint_as_float(b); win_i[slot] = i;
+        }
       }
     }
   }
@@ -239,11 +300,11 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
       const uint32_t i = win_i[tid];
       uint32_t rank = 0;
       for (uint32_t j = 0; j < cnt; j++) rank += (win_v[j] > v || (win_v[j] == v && win_i[j] < i)) ? 1u : 0u;
-      if (li[rank] < n_elems) data[li[rank]] = (float)i;
-      if (lv[rank] < n_elems) data[lv[rank]] = v;
+      if (to_i[rank] < n_elems) data[to_i[rank]] = (float)i;
+      if (to_v[rank] < n_elems) data[to_v[rank]] = v;
     } else {   // fewer candidates than k: the rounds past the last one
-      if (li[tid] < n_elems) data[li[tid]] = 0.0f;
-      if (lv[tid] < n_elems) data[lv[tid]] = SMP_NEG_INF;
+      if (to_i[tid] < n_elems) data[to_i[tid]] = 0.0f;
+      if (to_v[tid] < n_elems) data[to_v[tid]] = SMP_NEG_INF;
     }
   }
 }

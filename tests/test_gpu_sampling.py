@@ -38,6 +38,42 @@ def test_topk(hip, n, k, seed):
     assert np.array_equal(outs[0][1].view(np.uint32), outs[1][1].view(np.uint32))
 
 
+@pytest.mark.parametrize("n,k,order", [(4097, 40, "random"), (40960, 40, "random"), (10240, 64, "lists"), (40960, 40, "lists"), (40960, 64, "up"), (9999, 64, "down"),
+                                       (5000, 1, "random"), (5000, 64, "infinite"), (20000, 40, 1024), (20000, 40, 1025), (20000, 64, 30), (4103, 40, "scattered"), (33001, 64, "scattered"), (33002, 40, 2000)])
+def test_topk_listed_or_by_radix(hip, n, k, order):
+    """Candidates beside each other in the map and all over it, some outside of it; in no order, in sorted lists of 40 as the LM head leaves them, rising and falling along the whole list, with infinities and zeros of
+    either sign, and as many equal largest ones as the kernel's list holds, one more, and fewer than k."""
+    rng = np.random.default_rng(n + k)
+    v = rng.standard_normal(n).astype(np.float32)
+    if order == "lists":
+        v = -np.sort(-v.reshape(-1, 40), axis=1).reshape(-1)
+    elif order in ("up", "down"):
+        v = np.sort(v) if order == "up" else -np.sort(v)
+    elif order == "infinite":
+        v[:] = -np.inf
+        v[rng.permutation(n)[:50]] = np.array([np.inf, 0.0, -0.0, np.nan, -1.0] * 10, np.float32)
+    elif order not in ("random", "scattered"):
+        v[rng.permutation(n)[:order]] = 9.0
+    note(f"topk listed n={n} k={k} {order}")
+    f32map(hip, 0, n + 256, np.concatenate([v, np.full(256, 7.0, np.float32)]))
+    at = np.arange(n)
+    if order == "scattered":
+        at = rng.permutation(n)
+        v = v[at]
+        at[rng.integers(0, n, 9)] = 0xFFFFFFF0
+        v = np.where(at < n, v, np.float32(np.nan))
+    hip.map_topk_dev(0, up(hip, at), up(hip, n + np.arange(k)), up(hip, n + 128 + np.arange(k)), n, k)
+    x = np.where(np.isnan(v), np.float32(-3.402823466e+38), v)
+    # (zeros of either sign are one value where results are put in order; the larger sign is taken first, and all 50 are taken here)
+    want = np.argsort(-x, kind="stable")[:k]
+    got = read(hip, 0, n, k)
+    if order == "infinite":
+        want = want[:30]                             # (behind the finite ones: lowest values and infinities below them)
+    assert np.array_equal(got[:len(want)].astype(np.int64), want)
+    assert np.array_equal(read(hip, 0, n + 128, k)[:len(want)].view(np.uint32), x[want].view(np.uint32))
+    assert (read(hip, 0, n + 128 + k, 1) == 7.0).all()
+
+
 @pytest.mark.parametrize("n,temp,top_p,seed", [(4, 1.0, 0.9, 0), (64, 0.7, 0.95, 1), (40, 1.5, 0.3, 2), (8, 1e-9, 0.5, 3),
                                                (16, 1.0, 1.0, 4), (10, 1.0, 0.0, 5)])
 def test_topp(hip, n, temp, top_p, seed):

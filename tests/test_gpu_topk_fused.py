@@ -79,6 +79,27 @@ def test_topk_against_oracle(hip, kind, N, K, k, rpg, n_pen):
     check(got, o, N, k, rpg)
 
 
+@pytest.mark.parametrize("N,k,rpg,distinct", [(5000, 40, 1024, 1), (3000, 64, 333, 2), (2050, 1, 1024, 3), (1025, 40, 1024, 70), (700, 64, 63, 1)])
+def test_topk_of_equal_rows(hip, N, k, rpg, distinct):
+    """Groups of few distinct logits, zeros of either sign among them: every row is listed, or many that tie; the lowest rows come first."""
+    K = 128
+    rng = np.random.default_rng(N)
+    w = rng.standard_normal((distinct, K), dtype=np.float32)
+    w[0] = 0.0
+    qt = quant.quantize_q4_0(w[np.arange(N) % distinct])
+    x = rng.standard_normal(K).astype(np.float32)
+    pen = np.array([0, distinct], np.uint32)                     # (a zero logit times -1: a negative zero)
+    note(f"matvec_topk equal rows {N} k={k} rpg={rpg}")
+    idx, val = run_topk(hip, qt, x, k, rpg, pen, -1.0)
+    o = oracle.init()
+    run_topk(o, qt, x, k, rpg, pen, -1.0)
+    for g in range(idx.shape[0]):
+        rows = np.arange(g * rpg, min(N, (g + 1) * rpg))
+        best = np.argsort(-np.round(o.last_logits[rows], 3), kind="stable")[:k]
+        assert np.array_equal(idx[g, :len(best)].astype(np.int64), rows[best])
+        assert np.all(np.abs(val[g, :len(best)] - o.last_logits[rows[best]]) <= 1e-3 * max(1.0, np.abs(o.last_logits).max()))
+
+
 def test_topk_default_group_and_penalty_effect(hip):
     """The form without rows_per_group uses 256; a penalised favourite drops out of its group's list."""
     rng = np.random.default_rng(3)
