@@ -326,33 +326,44 @@ k_experts_list(const uint32_t* __restrict__ ids, uint32_t* __restrict__ list, ui
 // neighbours share the matrix rows; workgroups land on the eight dies in turn, and every die gets a run of neighbours.
 // Every wave finds it for itself from the experts' counts.
 struct Tile { uint32_t e, count, first, m, n; };     // expert, its rows, its first activation row, tile of tokens / matrix rows
-__device__ __forceinline__ bool pick_tile(const uint32_t* __restrict__ cnt, uint32_t experts, uint32_t bm, uint32_t tiles_n, Tile& t) {
+// What stands ahead of a tile is its launch's time once more a round, so sums and running sums stay in the vector unit and counts are loaded once.
+__device__ __forceinline__ uint32_t running_sum(uint32_t v) {      // of this lane and those before it
+#define RUN_STEP(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
+  RUN_STEP(0x111, 0xF); RUN_STEP(0x112, 0xF); RUN_STEP(0x114, 0xF); RUN_STEP(0x118, 0xF);     // 1, 2, 4, 8 lanes back in a row of 16
+  RUN_STEP(0x142, 0xA); RUN_STEP(0x143, 0xC);                                                 // the row before's last lane, the lower half's
+#undef RUN_STEP
+  return v;
+}
+__device__ __forceinline__ uint32_t lane_of(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
+// counts of the first 64 experts, a lane each
+__device__ __forceinline__ uint32_t first_counts(const uint32_t* __restrict__ cnt, uint32_t experts) {
+  const uint32_t lane = threadIdx.x & 63u, c = cnt[min(lane, experts - 1u)];
+  return lane < experts ? c : 0u;
+}
+// tiles of bm rows over all experts
+__device__ __forceinline__ uint32_t count_tiles(const uint32_t* __restrict__ cnt, uint32_t experts, uint32_t c0, uint32_t bm) {
+  uint32_t n = (c0 + bm - 1u) / bm;
+  for (uint32_t e = 64u + (threadIdx.x & 63u); e < experts; e += 64u) n += (cnt[e] + bm - 1u) / bm;
+  return lane_of(running_sum(n), 63);
+}
+__device__ __forceinline__ bool pick_tile(const uint32_t* __restrict__ cnt, uint32_t experts, uint32_t c0, uint32_t bm, uint32_t total, uint32_t tiles_n, Tile& t) {
   const uint32_t lane = threadIdx.x & 63u;
-  uint32_t total = 0;
-  for (uint32_t b = 0; b < experts; b += 64u) total += b + lane < experts ? (cnt[b + lane] + bm - 1u) / bm : 0u;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) total += (uint32_t)__shfl_xor((int)total, o, 64);
   total *= tiles_n;
   const uint32_t per = (total + 7u) / 8u, id = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= per || id >= total) return false;
   uint32_t tiles = 0, rows = 0;                              // ahead of this run of 64 experts
   for (uint32_t b = 0; b < experts; b += 64u) {
-    const uint32_t c = b + lane < experts ? cnt[b + lane] : 0u, mine = (c + bm - 1u) / bm * tiles_n;
-    uint32_t ts = mine, rs = c;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t u = (uint32_t)__shfl_up((int)ts, o, 64), v = (uint32_t)__shfl_up((int)rs, o, 64);
-      if ((int)lane >= o) { ts += u; rs += v; }
-    }
+    const uint32_t c = b == 0u ? c0 : b + lane < experts ? cnt[b + lane] : 0u, mine = (c + bm - 1u) / bm * tiles_n;
+    const uint32_t ts = running_sum(mine), rs = running_sum(c);
     const uint64_t here = __ballot(tiles + ts > id);
     if (here) {
       const int l = __ffsll((unsigned long long)here) - 1;
-      const uint32_t tm = (uint32_t)__shfl((int)mine, l, 64) / tiles_n, at = id - (tiles + (uint32_t)__shfl((int)(ts - mine), l, 64));
-      t.e = b + (uint32_t)l; t.count = (uint32_t)__shfl((int)c, l, 64); t.first = rows + (uint32_t)__shfl((int)(rs - c), l, 64);
+      const uint32_t tm = lane_of(mine, l) / tiles_n, at = id - (tiles + lane_of(ts - mine, l));
+      t.e = b + (uint32_t)l; t.count = lane_of(c, l); t.first = rows + lane_of(rs - c, l);
       t.m = at % tm; t.n = at / tm;
       return true;
     }
-    tiles += (uint32_t)__shfl((int)ts, 63, 64); rows += (uint32_t)__shfl((int)rs, 63, 64);
+    tiles += lane_of(ts, 63); rows += lane_of(rs, 63);
   }
   return false;
 }
@@ -373,25 +384,24 @@ __device__ __forceinline__ void put_part(const XSpec& s, float* parts, uint32_t 
   for (int i = 0; i < 4; i++) if (n0 + i < s.width) d[i] = v[i];
 }
 
-template <int BM, int BN, int WM, int WN, int ST, int STX, bool IN>
-__global__ void __launch_bounds__(64 * WM * WN)
-k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
-                const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n) {
-  __shared__ __attribute__((aligned(16))) bf16_t la[ST * BN * 64], lb[STX * BM * 64];
+// la: ST BN 64 elements, lb: STX BM 64; ONCE: weights that hardly any other tile reads
+template <int BM, int BN, int WM, int WN, int ST, int STX, bool ONCE, bool IN>
+__device__ __forceinline__ void experts_tile(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec& s, const uint32_t* __restrict__ list,
+                                             const uint32_t* __restrict__ cnt, uint32_t c0, uint32_t total, uint32_t rows, uint32_t tiles_n, bf16_t* la, bf16_t* lb) {
   constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16;
   const uint32_t lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint32_t c = lane & 15u, kg = lane >> 4, kp = IN ? s.k_stride : s.ff_stride, n = IN ? 2u * ((s.ff + 15u) & ~15u) : s.width;
   Tile t;
-  if (!pick_tile(cnt, s.experts, BM, tiles_n, t)) return;
+  if (!pick_tile(cnt, s.experts, c0, BM, total, tiles_n, t)) return;
   const uint32_t m0 = t.m * BM, n0 = t.n * BN, wn = (wave % WN) * (BN / WN), wm = (wave / WN) * (BM / WM);
   const bf16_t* We = W + (IN ? s.gate_up + (uint64_t)t.e * s.gate_up_step : s.down + (uint64_t)t.e * s.down_step);
   const uint32_t* le = list + (uint64_t)t.e * rows;
   f4_t acc[NTN][NTM];
-  tile_product<BM, BN, WM, WN, ST, 1, STX>(acc, TileRows<BN, WM * WN>(wave, lane, [&](uint32_t r) { return We + (uint64_t)min(n0 + r, n - 1u) * kp; }),
-                                   TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) {
-                                     const uint32_t i = min(m0 + r, t.count - 1u);
-                                     return opnd + (IN ? s.opnd + (uint64_t)(le[i] / s.top) * kp : s.act_opnd + (uint64_t)(t.first + i) * kp);
-                                   }), kp, 0u, kp, la, lb, wave, lane, m0 + wm < t.count);
+  tile_product<BM, BN, WM, WN, ST, 1, STX, ONCE>(acc, TileRows<BN, WM * WN, ONCE>(wave, lane, [&](uint32_t r) { return We + (uint64_t)min(n0 + r, n - 1u) * kp; }),
+                                                 TileRows<BM, WM * WN>(wave, lane, [&](uint32_t r) {
+                                                   const uint32_t i = min(m0 + r, t.count - 1u);
+                                                   return opnd + (IN ? s.opnd + (uint64_t)(le[i] / s.top) * kp : s.act_opnd + (uint64_t)(t.first + i) * kp);
+                                                 }), kp, 0u, kp, la, lb, wave, lane, m0 + wm < t.count);
 #pragma unroll
   for (int j = 0; j < NTM; j++) {
     const uint32_t i = m0 + wm + 16u * j + c;
@@ -407,6 +417,42 @@ k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ 
   }
 }
 
+// few rows an expert
+template <bool IN>
+__global__ void __launch_bounds__(256)
+k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
+                const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n) {
+  __shared__ __attribute__((aligned(16))) bf16_t la[4 * 64 * 64], lb[4 * 64 * 64];
+  const uint32_t c0 = first_counts(cnt, s.experts);
+  experts_tile<64, 64, 2, 2, 4, 4, false, IN>(W, opnd, parts, s, list, cnt, c0, count_tiles(cnt, s.experts, c0, 64u), rows, tiles_n, la, lb);
+}
+// More: tiles of 128, 192 or 256 rows, a workgroup a CU.  A launch takes as many rounds of tiles as a CU gets, whatever the last one holds, and that
+// hangs on the experts' counts, which only the device knows: every workgroup finds by them the size that costs least (MANY_128 and so on: what a round
+// of each takes beside the others).  The results do not hang on it.  Weights that one tile alone reads, as in a single round, do not
+// stay in the L2, where the tokens are (300 rows, 256 a tile: 108 us, so 96).  Where an expert has 256 rows and more what bounds it is the way of
+// weights and tokens into LDS, of which larger tiles have less; a third buffer for the weights, which come from memory: 2048 rows 208 us with two, 196.
+// Both products, 6 of 34 experts 1024 wide in 2048, by their average (64 from 53 rows on, 128 from 96, 256 from 256) and so, us: 300 rows 112 and 94,
+// 450 129 and 101, 600 140 and 116, 800 143 and 143, 952 144 and 145, 1300 191 and 166, 2048 201 and 202 (weights alone 83 at a large copy's rate).
+#define MANY_128 65u
+#define MANY_192 80u
+#define MANY_256 100u
+template <bool IN>
+__global__ void __launch_bounds__(512)
+k_experts_many(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
+               const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n, uint32_t cus) {
+  __shared__ __attribute__((aligned(16))) bf16_t lds[(3 * 256 + 2 * 256) * 64];
+  const uint32_t c0 = first_counts(cnt, s.experts);
+  const uint32_t t1 = count_tiles(cnt, s.experts, c0, 128u), t2 = count_tiles(cnt, s.experts, c0, 192u), t3 = count_tiles(cnt, s.experts, c0, 256u);
+  const auto rounds = [&](uint32_t tiles) { return (tiles * tiles_n + cus - 1u) / cus; };
+  const uint32_t r1 = rounds(t1), r2 = rounds(t2), r3 = rounds(t3);
+  const uint32_t c1 = r1 > 1u ? r1 * MANY_128 : ~0u, c2 = r2 * MANY_192, c3 = r3 * MANY_256;      // (in one round 128 are no quicker than 192)
+  bf16_t* const lb = lds + 3 * 256 * 64;
+  if (c2 <= min(c1, c3)) experts_tile<192, 256, 2, 4, 3, 2, true, IN>(W, opnd, parts, s, list, cnt, c0, t2, rows, tiles_n, lds, lb);
+  else if (c1 <= c3) experts_tile<128, 256, 2, 4, 3, 3, false, IN>(W, opnd, parts, s, list, cnt, c0, t1, rows, tiles_n, lds, lb);
+  else if (r3 == 1u) experts_tile<256, 256, 2, 4, 3, 2, true, IN>(W, opnd, parts, s, list, cnt, c0, t3, rows, tiles_n, lds, lb);
+  else experts_tile<256, 256, 2, 4, 3, 2, false, IN>(W, opnd, parts, s, list, cnt, c0, t3, rows, tiles_n, lds, lb);
+}
+
 template <bool IN>
 __global__ void __launch_bounds__(256)
 k_experts_f32(const bf16_t* __restrict__ W, float* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
@@ -415,7 +461,8 @@ k_experts_f32(const bf16_t* __restrict__ W, float* opnd, float* __restrict__ par
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, c = lane & 15u, kg = lane >> 4;
   const uint32_t kp = IN ? s.k_stride : s.ff_stride, n = IN ? 2u * ((s.ff + 15u) & ~15u) : s.width;
   Tile t;
-  if (!pick_tile(cnt, s.experts, 64u, tiles_n, t)) return;
+  const uint32_t c0 = first_counts(cnt, s.experts);
+  if (!pick_tile(cnt, s.experts, c0, 64u, count_tiles(cnt, s.experts, c0, 64u), tiles_n, t)) return;
   const uint32_t m0 = t.m * 64u, n0 = t.n * 64u, wn = (wave & 1u) * 32u, wm = (wave >> 1) * 32u, lr = tid >> 2, lc = (tid & 3u) * 8u;
   const bf16_t* We = W + (IN ? s.gate_up + (uint64_t)t.e * s.gate_up_step : s.down + (uint64_t)t.e * s.down_step);
   const uint32_t* le = list + (uint64_t)t.e * rows;
@@ -500,16 +547,10 @@ static void experts_product(Map* mo, Map* mw, const XSpec& s, float* parts, cons
   };
   if (mo->dtype == DTYPE_F32)
     k_experts_f32<IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (float*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
-  // 256 tokens a tile where an expert has that many on average: what bounds both is the way of the weights and tokens into LDS, of which
-  // there is a third less (2048 rows, 6 of 34, experts 1024 wide in 2048: both products 243 us in tiles of 128, 196 so; 208 without a third buffer
-  // for the weights, which come from memory and not from the L2; 952 rows, 168 an expert, 146 in tiles of 128, 179 so).
-  // A wave whose rows all lie past the expert's last only loads.
-  else if (entries >= (uint64_t)s.experts * 256u)
-    k_experts_tiled<256, 256, 2, 4, 3, 2, IN><<<grid(256, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256));
-  else if (entries >= (uint64_t)s.experts * 96u)
-    k_experts_tiled<128, 256, 2, 4, 3, 3, IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256));
+  else if (entries >= (uint64_t)s.experts * 32u)
+    k_experts_many<IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256), (uint32_t)g.n_cu);
   else
-    k_experts_tiled<64, 64, 2, 2, 4, 4, IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
+    k_experts_tiled<IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
   count_launch();
 }
 

@@ -14,6 +14,10 @@ namespace adamah {
 __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
 }
+// the same of bytes that are read once: first to leave the L2 again
+__device__ __forceinline__ void load_to_lds_once(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(p) : "memory", "m0");
+}
 // the same from a base all lanes share and an offset of each; 4 bytes a lane
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t off, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory", "m0");

@@ -30,7 +30,7 @@ __device__ __forceinline__ float row16_sum(float v) {
 // of a row sits at slot j ^ (row & 7), which spreads the 16-byte reads of neighbouring rows over the banks (no conflict
 // counted; runs of 32 columns, whose rows are half a line, loaded 15 % slower).  Where a lane's rows start is settled once,
 // so they may lie anywhere.
-template <int R, int NW> struct TileRows {
+template <int R, int NW, bool ONCE = false> struct TileRows {
   static constexpr int N = R / (8 * NW);                     // loads a step and lane
   static_assert(N * 8 * NW == R, "whole loads");
   const bf16_t* p[N];
@@ -43,7 +43,8 @@ template <int R, int NW> struct TileRows {
     }
   }
   __device__ __forceinline__ void load(int i, uint32_t k, uint32_t lds, uint32_t wave) const {      // from column k on
-    load_to_lds(p[i] + k, lds + ((uint32_t)i * NW + wave) * 1024u);
+    if (ONCE) load_to_lds_once(p[i] + k, lds + ((uint32_t)i * NW + wave) * 1024u);
+    else load_to_lds(p[i] + k, lds + ((uint32_t)i * NW + wave) * 1024u);
   }
 };
 // BM tokens x BN matrix rows by WM x WN waves; acc[i][j]: matrix rows wn + 16 i, tokens wm + 16 j of a wave's part; la: ST
@@ -55,8 +56,8 @@ template <int R, int NW> struct TileRows {
 // the tokens; column k of them meets column k mod kp of the matrix (k1 at most PL kp).  PL = 3, tokens in pieces, the largest last: an infinite weight and a lower piece
 // of 0 make no number where the whole product is infinite, so the lower pieces' sum counts only where it is finite (the
 // highest one's is infinite, or no number, exactly where the whole one is).
-template <int BM, int BN, int WM, int WN, int ST, int PL = 1, int STX = ST>
-__device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM / 16], const TileRows<BN, WM * WN>& w, const TileRows<BM, WM * WN>& x,
+template <int BM, int BN, int WM, int WN, int ST, int PL = 1, int STX = ST, bool ONCE = false>
+__device__ __forceinline__ void tile_product(f4_t (&acc)[BN / WN / 16][BM / WM / 16], const TileRows<BN, WM * WN, ONCE>& w, const TileRows<BM, WM * WN>& x,
                                              uint32_t kp, uint32_t k0, uint32_t k1, bf16_t* la, bf16_t* lb, uint32_t wave, uint32_t lane, bool on = true) {
   constexpr int NTN = BN / WN / 16, NTM = BM / WM / 16, LW = TileRows<BN, WM * WN>::N, LX = TileRows<BM, WM * WN>::N, LOADS = LW + LX;
   constexpr int LESS = STX < ST ? STX : ST, MORE = STX < ST ? ST : STX, LF = STX < ST ? LX : LW;       // stages; loads of the operand with fewer, which go first

@@ -651,3 +651,57 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
     want = (a / (1 + np.exp(-a)) * (hw @ g[1].T))[:, :ff] @ wide(dn)[:, :ff].T
     # (each activation is off by 2^-9 of itself at most, in no common direction: the whole by no more of its norm)
     assert rel_l2(whole[:rows * width].reshape(rows, width), want) < 2.0 ** -9
+
+
+@pytest.mark.parametrize("E,counts,ff,width", [(16, (150, 192), 2040, 64), (17, (193, 256), 2048, 60), (16, (193, 256), 2030, 64), (32, (230, 256), 2048, 64),
+                                               (70, (0, 130), 130, 200), (66, (30, 300), 1000, 64), (3, (300, 700), 40, 130)])
+def test_tiles_of_every_size_give_the_same_words(hip, E, counts, ff, width):
+    """Experts with as many rows as make tiles of 192, 128, 256 in one round and 256 in more the cheapest, more than 64 of them, some without a
+    row: the words of the same rows in portions that tiles of 64 take, and the product in 64 bits within what bfloat16 activations give."""
+    note(f"experts, tiles of every size E={E} {counts} ff {ff} width {width}")
+    rng = np.random.default_rng(E + ff)
+    per = rng.integers(counts[0], counts[1] + 1, E)
+    to = rng.permutation(np.repeat(np.arange(E), per))
+    rows = len(to)
+    ks, F, F16 = r64(width), r64(ff), (ff + 15) // 16 * 16
+    g = np.zeros((E, 2, F16, ks), np.float32)
+    g[:, :, :ff, :width] = rng.standard_normal((E, 2, ff, width), dtype=np.float32) / np.float32(np.sqrt(width))
+    down = np.zeros((E, width, F), np.float32)
+    down[:, :, :ff] = rng.standard_normal((E, width, ff), dtype=np.float32) / np.float32(np.sqrt(ff))
+    h = rng.standard_normal((rows, width), dtype=np.float32)
+    gu, dn, hb = f32_to_bf16(g.reshape(E, 2, -1, 16, ks).transpose(0, 2, 1, 3, 4)), f32_to_bf16(down), f32_to_bf16(np.pad(h, ((0, 0), (0, ks - width))))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, gu.size + dn.size + 8)
+    hip.scatter_contiguous(WT, 0, np.concatenate([gu.reshape(-1), dn.reshape(-1)]))
+    hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * (ks + F) + 8)
+    hip.scatter_contiguous(OP, 0, hb.reshape(-1))
+    L = (E + 4) // 4 * 4
+    log, x = L, L + rows * L
+    out = x + rows * width
+    f32map(hip, WS, out + rows * width + 8, np.zeros(out, np.float32))
+    z = np.zeros((rows, L), np.float32)
+    z[np.arange(rows), to] = 200.0                             # (weight one for the chosen expert)
+    hip.scatter_contiguous(WS, log, z.reshape(-1))
+    hip.scatter_contiguous(WS, x, h.reshape(-1))
+
+    def go(first, n):
+        spec = A.ExpertsSpec(experts=E, identity=0, top=1, ff=ff, ff_stride=F, width=width, k_stride=ks, gate_up=0, gate_up_step=2 * F16 * ks, down=gu.size,
+                             down_step=width * F, logits=log + first * L, logits_stride=L, correction=0, x=x + first * width, x_stride=width, opnd=first * ks,
+                             act=0, act_opnd=rows * ks, out=out + first * width, out_stride=width)
+        hip.experts_dev(WS, OP, WT, up(hip, spec.words()), 0, n)
+
+    go(0, rows)
+    whole = read(hip, WS, out, rows * width + 8)
+    hip.scatter_contiguous(WS, out, np.zeros(rows * width, np.float32))
+    step = 32 * E - 1
+    for first in range(0, rows, step):
+        go(first, min(step, rows - first))
+    parts = read(hip, WS, out, rows * width + 8)
+    assert not whole[rows * width:].any() and np.array_equal(whole.view(np.uint32), parts.view(np.uint32))
+    wide = lambda v: (v.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    hw, gw, dw = wide(hb), wide(f32_to_bf16(g)), wide(dn).reshape(E, width, F)
+    want = np.zeros((rows, width))
+    for e in range(E):
+        r = to == e
+        a = hw[r] @ gw[e, 0].T
+        want[r] = (a / (1 + np.exp(-a)) * (hw[r] @ gw[e, 1].T))[:, :ff] @ dw[e, :, :ff].T
+    assert rel_l2(whole[:rows * width].reshape(rows, width), want) < 2.0 ** -9      # (as above)
