@@ -654,10 +654,10 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
 
 
 @pytest.mark.parametrize("E,counts,ff,width", [(16, (150, 192), 2040, 64), (17, (193, 256), 2048, 60), (16, (193, 256), 2030, 64), (32, (230, 256), 2048, 64),
-                                               (70, (0, 130), 130, 200), (66, (30, 300), 1000, 64), (3, (300, 700), 40, 130)])
+                                               (70, (0, 130), 130, 200), (66, (30, 300), 1000, 64), (3, (300, 700), 40, 130), (64, (257, 262), 16, 60)])
 def test_tiles_of_every_size_give_the_same_words(hip, E, counts, ff, width):
     """Experts with as many rows as make tiles of 192, 128, 256 in one round and 256 in more the cheapest, more than 64 of them, some without a
-    row: the words of the same rows in portions that tiles of 64 take, and the product in 64 bits within what bfloat16 activations give."""
+    row, more entries than a walk over them keeps: the words of the same rows in portions that tiles of 64 take, and the product in 64 bits within what bfloat16 activations give."""
     note(f"experts, tiles of every size E={E} {counts} ff {ff} width {width}")
     rng = np.random.default_rng(E + ff)
     per = rng.integers(counts[0], counts[1] + 1, E)
