@@ -613,7 +613,7 @@ def test_sums_of_aligned_rows_are_those_of_shifted_ones(hip, E, I, top, shared, 
 @pytest.mark.parametrize("rows,width,ff", [(256, 60, 16), (257, 130, 40), (383, 64, 300), (384, 200, 130), (385, 1040, 72), (511, 300, 600), (513, 192, 100)])
 def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
     """One expert that every row takes: tiles of 256 rows whose last has none, a few or more than 128 of them, one step of columns to
-    seventeen, ragged in both directions: the words of the same rows in portions, which tiles of 64 take, and the product in 64 bits
+    seventeen, ragged in both directions: the words of the same rows in portions, which other tiles take, and the product in 64 bits
     within what bfloat16 activations give."""
     note(f"experts of many rows {rows} width {width} ff {ff}")
     rng = np.random.default_rng(rows + width)
