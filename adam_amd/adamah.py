@@ -179,6 +179,7 @@ _SIGS = {
     "adamah_hip_timer_begin": (i32, []), "adamah_hip_timer_end": (f32c, []),
     "adamah_hip_debug_dequant": (i32, [_U, u64, u64, pf32]),
     "adamah_hip_map_layout": (i32, [_U]), "adamah_hip_matmul_plan": (i32, [_U, _U, _U, u64, pu32, pu32]),
+    "adamah_hip_experts_plan": (i32, [pu32, _U, _U, u64, _U, _U, pu32, pu32]),
     "adamah_hip_stream_probe": (f32c, [u64, u64, _U, _U, _U]),
 }
 
@@ -849,6 +850,15 @@ class Adamah:
         if ret != 0:
             raise RuntimeError(f"adamah_hip_matmul_plan failed with code {ret}")
         return tile.value, shares.value
+
+    def experts_plan(self, counts, identity, entries, k, n):
+        """(rows a tile, whether its weights are marked as read once) of a product over experts' matrices [n, k]; counts: rows of each expert."""
+        c = np.ascontiguousarray(counts, np.uint32)
+        tile, once = ctypes.c_uint32(), ctypes.c_uint32()
+        ret = self._lib.adamah_hip_experts_plan(c.ctypes.data_as(pu32), c.size, identity, entries, k, n, ctypes.byref(tile), ctypes.byref(once))
+        if ret != 0:
+            raise RuntimeError(f"adamah_hip_experts_plan failed with code {ret}")
+        return tile.value, once.value
 
     # ---- misc ------------------------------------------------------------------------
     def reset_metrics(self):

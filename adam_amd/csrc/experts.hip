@@ -8,7 +8,7 @@
 // give it back is added at the end.
 //
 // More rows: k_experts_choose (a wave per row), k_experts_list (a workgroup per expert: its rows in order), then the two
-// products over tiles of one expert's rows each, k_experts_tiled (bfloat16 operands) or k_experts_f32.  The rows of an
+// products over tiles of one expert's rows each: k_experts_tiled or k_experts_many (bfloat16 operands), k_experts_f32.  The rows of an
 // expert are picked up where they lie; activations and results are laid down so that k_experts_sum can add up a row's in a
 // fixed order: what a row gets does not depend on which other rows there are.
 #include "linear_common.h"
@@ -444,31 +444,48 @@ k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ 
   const uint32_t c0 = first_counts(cnt, s.experts);
   experts_tile<64, 64, 2, 2, 4, 4, false, IN>(W, opnd, parts, s, list, cnt, c0, count_tiles(cnt, s.experts, c0, 64u), rows, tiles_n, la, lb);
 }
-// More: tiles of 128, 192 or 256 rows, a workgroup a CU.  A launch takes as many rounds of tiles as a CU gets, whatever the last one holds, and that
-// hangs on the experts' counts, which only the device knows: every workgroup finds by them the size that costs least (MANY_128 and so on: what a round
-// of each takes beside the others).  The results do not hang on it.  Weights that one tile alone reads, as in a single round, do not
-// stay in the L2, where the tokens are (300 rows, 256 a tile: 108 us, so 96).  Where an expert has 256 rows and more what bounds it is the way of
-// weights and tokens into LDS, of which larger tiles have less; a third buffer for the weights, which come from memory: 2048 rows 208 us with two, 196.
-// Both products, 6 of 34 experts 1024 wide in 2048, by their average (64 from 53 rows on, 128 from 96, 256 from 256) and so, us: 300 rows 112 and 94,
-// 450 129 and 101, 600 140 and 116, 800 143 and 143, 952 144 and 145, 1300 191 and 166, 2048 201 and 202 (weights alone 83 at a large copy's rate).
-#define MANY_128 65u
-#define MANY_192 80u
-#define MANY_256 100u
+// More: tiles of 128, 192 or 256 rows by 256 matrix rows, a workgroup a CU.  A launch takes as many rounds of tiles as a CU gets, whatever the last one
+// holds, and that hangs on the experts' counts, which only the device knows: every workgroup finds by them the size that costs least.  The results do not
+// hang on it.  A round takes what stands around a tile's steps and those steps, which are longer the more CUs have a tile, and less than in proportion to the rows
+// (weights and tokens on their way into LDS bound them; a third buffer for the weights, which come from memory: 2048 rows, 6 of 34 experts 1024 wide in 2048, both
+// products 208 us with two, 196 so).  Over 16 shapes of 3 .. 128 experts, 1 .. 64 steps and 8 .. 600 rows an expert, weights from memory, both products take 0.7 %
+// longer than in the best sizes (64 rows among them) in the mean, 13 % at most (24 experts 768 wide in 1536, 64 rows: 58 us and 51).
+#define MANY_SIZES 3u
+struct Chip { uint32_t cus, magic; float inv; };                                  // tiles / cus = umulhi(tiles, magic)
+__host__ __device__ __forceinline__ float many_us(uint32_t size, uint32_t tiles, uint32_t steps, const Chip& c) {      // of `tiles` tiles of 128 + 64 size rows
+  const float around = 9.f + (float)size, alone = size == 0u ? 0.6f : size == 1u ? 0.75f : 0.85f, full = size == 0u ? 0.47f : size == 1u ? 0.7f : 1.f;
+  const uint32_t rounds = (uint32_t)((uint64_t)(tiles + c.cus - 1u) * c.magic >> 32);
+  return (float)rounds * (around + (float)steps * (alone + full * (rounds > 1u ? 1.f : (float)tiles * c.inv)));
+}
+// Weights that one tile alone reads do not stay in the L2, where the tokens are, if every CU has a tile (32 experts 1024 wide in 2048, 50 rows each: 67 us and
+// so 60 in tiles of 128, 69 and 61 in tiles of 256; 8 of them, 128 rows, a CU in four at work: 38 and 40; 64 of 4 steps, 95 rows: 16.5 and 18.2).
+struct Many { uint32_t size; bool once; };
+__host__ __device__ __forceinline__ Many many_pick(const uint32_t (&tiles_m)[MANY_SIZES], uint32_t experts_with_rows, uint32_t tiles_n, uint32_t steps, const Chip& c) {
+  const float u0 = many_us(0u, tiles_m[0] * tiles_n, steps, c), u1 = many_us(1u, tiles_m[1] * tiles_n, steps, c), u2 = many_us(2u, tiles_m[2] * tiles_n, steps, c);
+  const uint32_t i = u0 <= u1 && u0 <= u2 ? 0u : u1 <= u2 ? 1u : 2u, t = i == 0u ? tiles_m[0] : i == 1u ? tiles_m[1] : tiles_m[2];
+  return {i, t == experts_with_rows && t * tiles_n >= c.cus && steps >= 8u};
+}
 template <bool IN>
 __global__ void __launch_bounds__(512)
 k_experts_many(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ parts, const XSpec s, const uint32_t* __restrict__ list,
-               const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n, uint32_t cus) {
+               const uint32_t* __restrict__ cnt, uint32_t rows, uint32_t tiles_n, const Chip chip) {
   __shared__ __attribute__((aligned(16))) bf16_t lds[(3 * 256 + 2 * 256) * 64];
   const uint32_t c0 = first_counts(cnt, s.experts);
-  const uint32_t t1 = count_tiles(cnt, s.experts, c0, 128u), t2 = count_tiles(cnt, s.experts, c0, 192u), t3 = count_tiles(cnt, s.experts, c0, 256u);
-  const auto rounds = [&](uint32_t tiles) { return (tiles * tiles_n + cus - 1u) / cus; };
-  const uint32_t r1 = rounds(t1), r2 = rounds(t2), r3 = rounds(t3);
-  const uint32_t c1 = r1 > 1u ? r1 * MANY_128 : ~0u, c2 = r2 * MANY_192, c3 = r3 * MANY_256;      // (in one round 128 are no quicker than 192)
+  uint32_t t[MANY_SIZES] = {(c0 + 127u) / 128u, (c0 + 191u) / 192u, (c0 + 255u) / 256u}, some = __popcll(__ballot(c0 != 0u));
+  for (uint32_t b = 64u; b < s.experts; b += 64u) {
+    const uint32_t e = b + (threadIdx.x & 63u), c = e < s.experts ? cnt[e] : 0u;
+    t[0] += (c + 127u) / 128u; t[1] += (c + 191u) / 192u; t[2] += (c + 255u) / 256u;
+    some += __popcll(__ballot(c != 0u));
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < MANY_SIZES; i++) t[i] = lane_of(running_sum(t[i]), 63);
+  const Many m = many_pick(t, some, tiles_n, (IN ? s.k_stride : s.ff_stride) >> 6, chip);
   bf16_t* const lb = lds + 3 * 256 * 64;
-  if (c2 <= min(c1, c3)) experts_tile<192, 256, 2, 4, 3, 2, true, IN>(W, opnd, parts, s, list, cnt, c0, t2, rows, tiles_n, lds, lb);
-  else if (c1 <= c3) experts_tile<128, 256, 2, 4, 3, 3, false, IN>(W, opnd, parts, s, list, cnt, c0, t1, rows, tiles_n, lds, lb);
-  else if (r3 == 1u) experts_tile<256, 256, 2, 4, 3, 2, true, IN>(W, opnd, parts, s, list, cnt, c0, t3, rows, tiles_n, lds, lb);
-  else experts_tile<256, 256, 2, 4, 3, 2, false, IN>(W, opnd, parts, s, list, cnt, c0, t3, rows, tiles_n, lds, lb);
+#define MANY_TILE(BM, STX, ONCE) experts_tile<BM, 256, 2, 4, 3, STX, ONCE, IN>(W, opnd, parts, s, list, cnt, c0, t[BM / 64 - 2], rows, tiles_n, lds, lb)
+  if (m.size == 0u) { if (m.once) MANY_TILE(128, 3, true); else MANY_TILE(128, 3, false); }
+  else if (m.size == 1u) { if (m.once) MANY_TILE(192, 2, true); else MANY_TILE(192, 2, false); }
+  else { if (m.once) MANY_TILE(256, 2, true); else MANY_TILE(256, 2, false); }
+#undef MANY_TILE
 }
 
 template <bool IN>
@@ -555,6 +572,27 @@ k_experts_sum(const XSpec s, float* act, const float* __restrict__ parts, const 
 static Scratch g_experts;
 void experts_release() { scratch_free(g_experts); }
 
+static Chip chip() {
+  const uint32_t n = (uint32_t)g.n_cu;
+  return {n, (uint32_t)((0x100000000ull + n - 1u) / n), 1.f / (float)n};
+}
+// Whether k_experts_many is the quicker one over matrices of n rows of kp columns, by the experts' average (the device alone knows their counts).
+// k_experts_tiled has four tiles of 64 x 64 to one of 256 columns, so that few rows still fill the chip, but twice the bytes a product on their way into LDS.
+// Weights from memory, both products, us in tiles of 64 and in the best of the others: 8 experts 1024 wide in 2048, 50 rows each 40 and 52, 128 rows 55
+// and 61, 200 rows 66 and 58; 32 of them, 40 rows 91 and 89, 64 rows 113 and 93; 8 experts 256 wide in 512, 97 rows 12 and 23, 600 rows 27 and 29; 64 experts
+// 1408 wide in 2048, 33 rows 226 and 214, 64 rows 305 and 240; 128 experts 128 wide in 512, 50 rows 30 and 27.
+static bool many_rows_pay(uint32_t experts, uint32_t identity, uint64_t entries, uint32_t kp, uint32_t n) {
+  const float to = (float)std::min<uint64_t>(experts, entries), avg = (float)entries * (float)experts / (float)(experts + identity) / to;
+  const Chip c = chip();
+  const uint32_t steps = kp >> 6;
+  const auto tiles = [&](float bm) { return avg > 0.8f * bm ? to * (avg / bm + 0.5f) : to; };      // (half of an expert's last one is empty)
+  const float few = tiles(64.f) * (float)cdiv(n, 64) * c.inv;                // a CU's
+  float many = 1e30f;
+  for (uint32_t i = 0; i < MANY_SIZES; i++)
+    many = std::min(many, many_us(i, (uint32_t)std::min(1.6e7f, tiles(128.f + 64.f * (float)i) * (float)cdiv(n, 256)), steps, c));
+  return many < 4.f + 0.25f * (float)steps * std::max(1.f, few) + 1.6f * few;
+}
+
 template <bool IN>
 static void experts_product(Map* mo, Map* mw, const XSpec& s, float* parts, const uint32_t* list, const uint32_t* cnt, uint32_t rows) {
   const bf16_t* W = (const bf16_t*)mw->buf;
@@ -565,8 +603,8 @@ static void experts_product(Map* mo, Map* mw, const XSpec& s, float* parts, cons
   };
   if (mo->dtype == DTYPE_F32)
     k_experts_f32<IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (float*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
-  else if (entries >= (uint64_t)s.experts * 32u)
-    k_experts_many<IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256), (uint32_t)g.n_cu);
+  else if (many_rows_pay(s.experts, s.identity, entries, IN ? s.k_stride : s.ff_stride, n))
+    k_experts_many<IN><<<grid(128, cdiv(n, 256)), 512, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 256), chip());
   else
     k_experts_tiled<IN><<<grid(64, cdiv(n, 64)), 256, 0, g.stream>>>(W, (bf16_t*)mo->buf, parts, s, list, cnt, rows, cdiv(n, 64));
   count_launch();
@@ -575,6 +613,20 @@ static void experts_product(Map* mo, Map* mw, const XSpec& s, float* parts, cons
 }  // namespace adamah
 
 using namespace adamah;
+
+extern "C" int adamah_hip_experts_plan(const uint32_t* counts, uint32_t experts, uint32_t identity, uint64_t entries, uint32_t k, uint32_t n, uint32_t* tile, uint32_t* once) {
+  if (g.n_cu <= 0 || !counts || experts == 0u || entries == 0u || k == 0u || (k & 63u) || n == 0u || !tile || !once) return ADAMAH_ERR_INVALID;
+  *tile = 64u; *once = 0u;
+  if (!many_rows_pay(experts, identity, entries, k, n)) return ADAMAH_OK;
+  uint32_t t[MANY_SIZES] = {0, 0, 0}, some = 0;
+  for (uint32_t e = 0; e < experts; e++) {
+    for (uint32_t i = 0; i < MANY_SIZES; i++) t[i] += cdiv(counts[e], 128u + 64u * i);
+    some += counts[e] ? 1u : 0u;
+  }
+  const Many m = many_pick(t, some, cdiv(n, 256), k >> 6, chip());
+  *tile = 128u + 64u * m.size; *once = m.once ? 1u : 0u;
+  return ADAMAH_OK;
+}
 
 extern "C" int adamah_experts_dev(uint32_t map_act, uint32_t map_opnd, uint32_t map_wt, uint32_t h_spec, uint32_t h_shared, uint32_t rows) { ADAMAH_API();
   Map *ma = get_f32_map(map_act), *mo = get_map(map_opnd), *mw = get_map(map_wt);

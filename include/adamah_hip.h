@@ -440,6 +440,9 @@ int adamah_hip_map_layout(uint32_t map_id);
 /* How a Q4 matmul of rows activation rows (more than 64) by weights [n, k] from element base on would run: *tile activation rows a
  * workgroup of the ring kernel, 32 the narrow kernel, 0 the tiled kernel; *shares of k, added up by a launch of their own if more than one. */
 int adamah_hip_matmul_plan(uint32_t rows, uint32_t k, uint32_t n, uint64_t base, uint32_t* tile, uint32_t* shares);
+/* How the bfloat16 product of several rows over experts' matrices [n, k] would run where expert e has counts[e] of `entries` chosen places
+ * (some of them of the `identity` choices): *tile rows a workgroup, *once 1 where its weights do not stay in the L2. */
+int adamah_hip_experts_plan(const uint32_t* counts, uint32_t experts, uint32_t identity, uint64_t entries, uint32_t k, uint32_t n, uint32_t* tile, uint32_t* once);
 
 #ifdef __cplusplus
 }

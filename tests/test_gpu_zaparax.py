@@ -632,6 +632,8 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
     f32map(hip, WS, out + rows * width + 8, np.zeros(out, np.float32))
     hip.scatter_contiguous(WS, x, h.reshape(-1))
 
+    assert hip.experts_plan([rows], 0, rows, ks, 2 * F16) == (64, 0) == hip.experts_plan([rows], 0, rows, F, width)
+
     def go(first, n):
         spec = A.ExpertsSpec(experts=1, identity=0, top=1, ff=ff, ff_stride=F, width=width, k_stride=ks, gate_up=0, gate_up_step=2 * F16 * ks, down=gu.size,
                              down_step=width * F, logits=log, logits_stride=2, correction=0, x=x + first * width, x_stride=width, opnd=first * ks, act=0,
@@ -653,25 +655,35 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
     assert rel_l2(whole[:rows * width].reshape(rows, width), want) < 2.0 ** -9
 
 
-@pytest.mark.parametrize("E,counts,ff,width", [(16, (150, 192), 2040, 64), (17, (193, 256), 2048, 60), (16, (193, 256), 2030, 64), (32, (230, 256), 2048, 64),
-                                               (70, (0, 130), 130, 200), (66, (30, 300), 1000, 64), (3, (300, 700), 40, 130), (64, (257, 262), 16, 60)])
-def test_tiles_of_every_size_give_the_same_words(hip, E, counts, ff, width):
-    """Experts with as many rows as make tiles of 192, 128, 256 in one round and 256 in more the cheapest, more than 64 of them, some without a
-    row, more entries than a walk over them keeps: the words of the same rows in portions that tiles of 64 take, and the product in 64 bits within what bfloat16 activations give."""
-    note(f"experts, tiles of every size E={E} {counts} ff {ff} width {width}")
-    rng = np.random.default_rng(E + ff)
-    per = rng.integers(counts[0], counts[1] + 1, E)
+@pytest.mark.parametrize("counts,ff,width,first,second", [
+    ([(16, 150, 192)], 2040, 64, (192, 0), (64, 0)), ([(17, 193, 256)], 2048, 60, (256, 0), (64, 0)), ([(16, 193, 256)], 2030, 64, (256, 0), (64, 0)),
+    ([(32, 230, 256)], 2048, 64, (256, 0), (64, 0)), ([(70, 0, 130)], 130, 200, (64, 0), (64, 0)), ([(66, 30, 300)], 1000, 64, (192, 0), (64, 0)),
+    ([(3, 300, 700)], 40, 130, (64, 0), (64, 0)), ([(64, 257, 262)], 16, 60, (64, 0), (64, 0)),
+    ([(32, 90, 128)], 1000, 300, (128, 0), (64, 0)), ([(32, 150, 192)], 1024, 320, (192, 0), (64, 0)), ([(30, 200, 250), (10, 257, 380)], 1024, 320, (256, 0), (64, 0)),
+    ([(32, 90, 128)], 1024, 512, (128, 1), (64, 0)), ([(32, 150, 192)], 1024, 512, (192, 1), (64, 0)), ([(32, 200, 256)], 1024, 512, (256, 1), (128, 0)),
+    ([(32, 90, 128)], 300, 2000, (64, 0), (128, 0)), ([(32, 150, 192)], 320, 2048, (128, 0), (192, 0)), ([(30, 200, 250), (10, 257, 380)], 576, 2000, (256, 0), (256, 0)),
+    ([(32, 90, 128)], 512, 2048, (128, 0), (128, 1)), ([(32, 150, 192)], 512, 2040, (128, 0), (192, 1)), ([(32, 200, 256)], 512, 2048, (128, 0), (256, 1))])
+def test_tiles_of_every_size_give_the_same_words(hip, counts, ff, width, first, second):
+    """Experts with as many rows as make each size of tile the cheapest, in one round and in more, with weights that stay in the L2 and that do not, in either
+    product, over one step of columns to nine; tiles with rows for one half of their waves only, more than 64 experts, some without a
+    row, more entries than a walk over them keeps: the words of the same rows in portions that tiles of 64 take, and the product of a few experts in 64 bits within
+    what bfloat16 activations give."""
+    note(f"experts, tiles of every size {counts} ff {ff} width {width}")
+    rng = np.random.default_rng(ff + width)
+    per = np.concatenate([rng.integers(lo, hi + 1, n) for n, lo, hi in counts])
+    E = len(per)
     to = rng.permutation(np.repeat(np.arange(E), per))
     rows = len(to)
     ks, F, F16 = r64(width), r64(ff), (ff + 15) // 16 * 16
+    pool = rng.standard_normal(1000003, dtype=np.float32)      # (a prime: no two rows are alike)
     g = np.zeros((E, 2, F16, ks), np.float32)
-    g[:, :, :ff, :width] = rng.standard_normal((E, 2, ff, width), dtype=np.float32) / np.float32(np.sqrt(width))
+    g[:, :, :ff, :width] = np.resize(pool, (E, 2, ff, width)) / np.float32(np.sqrt(width))
     down = np.zeros((E, width, F), np.float32)
-    down[:, :, :ff] = rng.standard_normal((E, width, ff), dtype=np.float32) / np.float32(np.sqrt(ff))
+    down[:, :, :ff] = np.resize(pool[::-1], (E, width, ff)) / np.float32(np.sqrt(ff))
     h = rng.standard_normal((rows, width), dtype=np.float32)
-    gu, dn, hb = f32_to_bf16(g.reshape(E, 2, -1, 16, ks).transpose(0, 2, 1, 3, 4)), f32_to_bf16(down), f32_to_bf16(np.pad(h, ((0, 0), (0, ks - width))))
-    hip.map_create_typed(WT, A.DTYPE_BF16, 1, gu.size + dn.size + 8)
-    hip.scatter_contiguous(WT, 0, np.concatenate([gu.reshape(-1), dn.reshape(-1)]))
+    gb, dn, hb = f32_to_bf16(g), f32_to_bf16(down), f32_to_bf16(np.pad(h, ((0, 0), (0, ks - width))))
+    hip.map_create_typed(WT, A.DTYPE_BF16, 1, gb.size + dn.size + 8)
+    hip.scatter_contiguous(WT, 0, np.concatenate([gb.reshape(E, 2, -1, 16, ks).transpose(0, 2, 1, 3, 4).reshape(-1), dn.reshape(-1)]))
     hip.map_create_typed(OP, A.DTYPE_BF16, 1, rows * (ks + F) + 8)
     hip.scatter_contiguous(OP, 0, hb.reshape(-1))
     L = (E + 4) // 4 * 4
@@ -683,25 +695,50 @@ def test_tiles_of_every_size_give_the_same_words(hip, E, counts, ff, width):
     hip.scatter_contiguous(WS, log, z.reshape(-1))
     hip.scatter_contiguous(WS, x, h.reshape(-1))
 
-    def go(first, n):
-        spec = A.ExpertsSpec(experts=E, identity=0, top=1, ff=ff, ff_stride=F, width=width, k_stride=ks, gate_up=0, gate_up_step=2 * F16 * ks, down=gu.size,
-                             down_step=width * F, logits=log + first * L, logits_stride=L, correction=0, x=x + first * width, x_stride=width, opnd=first * ks,
-                             act=0, act_opnd=rows * ks, out=out + first * width, out_stride=width)
+    def plans(lo, n):
+        c = np.bincount(to[lo:lo + n], minlength=E)
+        return hip.experts_plan(c, 0, n, ks, 2 * F16), hip.experts_plan(c, 0, n, F, width)
+
+    def go(lo, n):
+        spec = A.ExpertsSpec(experts=E, identity=0, top=1, ff=ff, ff_stride=F, width=width, k_stride=ks, gate_up=0, gate_up_step=2 * F16 * ks, down=gb.size,
+                             down_step=width * F, logits=log + lo * L, logits_stride=L, correction=0, x=x + lo * width, x_stride=width, opnd=lo * ks,
+                             act=0, act_opnd=rows * ks, out=out + lo * width, out_stride=width)
         hip.experts_dev(WS, OP, WT, up(hip, spec.words()), 0, n)
 
+    assert plans(0, rows) == (first, second)
     go(0, rows)
     whole = read(hip, WS, out, rows * width + 8)
     hip.scatter_contiguous(WS, out, np.zeros(rows * width, np.float32))
-    step = 32 * E - 1
-    for first in range(0, rows, step):
-        go(first, min(step, rows - first))
+    few = ((64, 0), (64, 0))
+    step = next(n for n in (63, 31, 16, 8) if plans(0, n) == few)
+    for lo in range(0, rows, step):
+        n = min(step, rows - lo)
+        assert n == 1 or plans(lo, n) == few
+        go(lo, n)
     parts = read(hip, WS, out, rows * width + 8)
-    assert not whole[rows * width:].any() and np.array_equal(whole.view(np.uint32), parts.view(np.uint32))
+    assert not whole[rows * width:].any()
+    # (a last portion of one row has an order of its own)
+    same = rows * width if rows % step != 1 else (rows - 1) * width
+    assert np.array_equal(whole[:same].view(np.uint32), parts[:same].view(np.uint32))
     wide = lambda v: (v.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
-    hw, gw, dw = wide(hb), wide(f32_to_bf16(g)), wide(dn).reshape(E, width, F)
-    want = np.zeros((rows, width))
-    for e in range(E):
+    got = whole[:rows * width].reshape(rows, width)
+    for e in (0, E // 2, E - 1):
         r = to == e
-        a = hw[r] @ gw[e, 0].T
-        want[r] = (a / (1 + np.exp(-a)) * (hw[r] @ gw[e, 1].T))[:, :ff] @ dw[e, :, :ff].T
-    assert rel_l2(whole[:rows * width].reshape(rows, width), want) < 2.0 ** -9      # (as above)
+        hw, gw, dw = wide(hb[r]), wide(gb[e]), wide(dn[e])
+        a = hw @ gw[0].T
+        want = (a / (1 + np.exp(-a)) * (hw @ gw[1].T))[:, :ff] @ dw[:, :ff].T
+        # (each activation is off by 2^-9 of itself at most, in no common direction: the whole by no more of its norm)
+        assert not r.any() or rel_l2(got[r], want) < 2.0 ** -9
+
+
+# (rows an expert, of so many experts; first product's tiles, second one's): where tiles of 64 fill the chip and larger ones do not, and where larger ones do
+@pytest.mark.parametrize("E,top,rows,ff,width,first,second", [
+    (8, 2, 50, 1024, 2048, 64, 64), (8, 2, 128, 1024, 2048, 64, 64), (8, 2, 257, 1024, 2048, 128, 128), (4, 1, 97, 1024, 2048, 64, 64), (8, 1, 400, 64, 256, 64, 64),
+    (16, 2, 95, 512, 1024, 64, 64), (16, 2, 257, 512, 1024, 128, 128), (8, 2, 168, 256, 512, 64, 64), (32, 6, 64, 1024, 2048, 128, 128), (32, 6, 400, 1024, 2048, 256, 256),
+    (64, 6, 300, 1408, 2048, 192, 192), (64, 6, 33, 1408, 2048, 64, 64), (16, 4, 168, 1024, 2048, 128, 128)])
+def test_experts_rule_by_tiles_and_cus(hip, E, top, rows, ff, width, first, second):
+    """The rule at shapes whose forms were timed against each other (256 CUs): equal experts."""
+    F16, entries = (ff + 15) // 16 * 16, E * rows
+    counts = np.full(E, rows)
+    note(f"experts plan E={E} rows={rows} {ff} in {width}")
+    assert hip.experts_plan(counts, 0, entries, r64(width), 2 * F16)[0] == first and hip.experts_plan(counts, 0, entries, r64(ff), width)[0] == second
