@@ -301,16 +301,17 @@ k_experts_choose(const XSpec s, const float* __restrict__ act, uint32_t* __restr
 }
 
 // A workgroup per expert: the entries that chose it, in order, at list + e * rows; cnt[e]: how many.  A wave takes a run of entries, 64 neighbours a load,
-// and counts and places them by the lanes that hold the expert.  Bound by latency: 12288 entries 13.0 us with a run of neighbours a thread, 5.2 so, 3600 5.6 and 4.9.
-#define LIST_WAVES 16u
-__global__ void __launch_bounds__(64 * LIST_WAVES)
+// and counts and places them by the lanes that hold the expert; the first KEPT loads are asked for at once and kept for the second walk.  Bound by latency:
+// 12288 entries in 32 lists 5.1 us (13.1 with a run of neighbours a thread); as many loads and waves as the entries need and no more, 48 entries 1.8 us (3.8 with 16 of
+// either), 960 2.6 (4.3), 3584 3.0 (4.4).
+template <uint32_t WAVES, uint32_t KEPT>
+__global__ void __launch_bounds__(64 * WAVES)
 k_experts_list(const uint32_t* __restrict__ ids, uint32_t* __restrict__ list, uint32_t* __restrict__ cnt, uint32_t rows, uint32_t top) {
-  __shared__ uint32_t part[LIST_WAVES];
+  __shared__ uint32_t part[WAVES];
   const uint32_t e = blockIdx.x, lane = threadIdx.x & 63u, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), total = rows * top;
-  const uint32_t run = (total + LIST_WAVES * 64u - 1u) / (LIST_WAVES * 64u), lo = wave * run * 64u;      // (of 64 entries)
+  const uint32_t run = (total + WAVES * 64u - 1u) / (WAVES * 64u), lo = wave * run * 64u;      // (of 64 entries)
   const auto id_at = [&](uint32_t j) { return ids[min(lo + 64u * j + lane, total - 1u)]; };
   const auto mine = [&](uint32_t j, uint32_t id) { return (uint64_t)__ballot(id == e && lo + 64u * j + lane < total); };      // which lanes' entries chose it
-  constexpr uint32_t KEPT = 16;                              // of the first ones, for the second walk
   uint64_t kept[KEPT];
   {
     uint32_t id[KEPT];
@@ -328,7 +329,7 @@ k_experts_list(const uint32_t* __restrict__ ids, uint32_t* __restrict__ list, ui
   __syncthreads();
   uint32_t at = 0;
   for (uint32_t w = 0; w < wave; w++) at += part[w];
-  if (wave == LIST_WAVES - 1u && lane == 0u) cnt[e] = min(at + n, rows);             // (a row takes an expert once)
+  if (wave == WAVES - 1u && lane == 0u) cnt[e] = min(at + n, rows);             // (a row takes an expert once)
   const auto place = [&](uint32_t j, uint64_t m) {
     const uint32_t to = at + __popcll(m & ((1ull << lane) - 1ull));
     if ((m >> lane & 1ull) && to < rows) list[(uint64_t)e * rows + to] = lo + 64u * j + lane;
@@ -685,7 +686,9 @@ extern "C" int adamah_experts_dev(uint32_t map_act, uint32_t map_opnd, uint32_t 
 #undef CHOOSE
   count_launch();
   if (int r = check_launch()) return r;
-  k_experts_list<<<(uint32_t)E, 64 * LIST_WAVES, 0, g.stream>>>(ids, list, cnt, rows, s->top);
+#define LIST(W, K) k_experts_list<W, K><<<(uint32_t)E, 64 * W, 0, g.stream>>>(ids, list, cnt, rows, s->top)
+  if (entries <= 1024u) LIST(4, 4); else if (entries <= 4096u) LIST(16, 4); else LIST(16, 16);
+#undef LIST
   count_launch();
   if (int r = check_launch()) return r;
   experts_product<true>(mo, mw, *s, parts, list, cnt, rows);

@@ -659,6 +659,8 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
     ([(16, 150, 192)], 2040, 64, (192, 0), (64, 0)), ([(17, 193, 256)], 2048, 60, (256, 0), (64, 0)), ([(16, 193, 256)], 2030, 64, (256, 0), (64, 0)),
     ([(32, 230, 256)], 2048, 64, (256, 0), (64, 0)), ([(70, 0, 130)], 130, 200, (64, 0), (64, 0)), ([(66, 30, 300)], 1000, 64, (192, 0), (64, 0)),
     ([(3, 300, 700)], 40, 130, (64, 0), (64, 0)), ([(64, 257, 262)], 16, 60, (64, 0), (64, 0)),
+    ([(4, 205, 205), (1, 204, 204)], 16, 60, (64, 0), (64, 0)), ([(5, 205, 205)], 16, 60, (64, 0), (64, 0)), ([(4, 819, 819), (1, 820, 820)], 16, 60, (64, 0), (64, 0)),
+    ([(4, 819, 819), (1, 821, 821)], 16, 60, (64, 0), (64, 0)), ([(4, 3277, 3277), (1, 3276, 3276)], 16, 60, (64, 0), (64, 0)), ([(5, 3277, 3277)], 16, 60, (64, 0), (64, 0)),
     ([(32, 90, 128)], 1000, 300, (128, 0), (64, 0)), ([(32, 150, 192)], 1024, 320, (192, 0), (64, 0)), ([(30, 200, 250), (10, 257, 380)], 1024, 320, (256, 0), (64, 0)),
     ([(32, 90, 128)], 1024, 512, (128, 1), (64, 0)), ([(32, 150, 192)], 1024, 512, (192, 1), (64, 0)), ([(32, 200, 256)], 1024, 512, (256, 1), (128, 0)),
     ([(32, 90, 128)], 300, 2000, (64, 0), (128, 0)), ([(32, 150, 192)], 320, 2048, (128, 0), (192, 0)), ([(30, 200, 250), (10, 257, 380)], 576, 2000, (256, 0), (256, 0)),
@@ -666,7 +668,7 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
 def test_tiles_of_every_size_give_the_same_words(hip, counts, ff, width, first, second):
     """Experts with as many rows as make each size of tile the cheapest, in one round and in more, with weights that stay in the L2 and that do not, in either
     product, over one step of columns to nine; tiles with rows for one half of their waves only, more than 64 experts, some without a
-    row, more entries than a walk over them keeps: the words of the same rows in portions that tiles of 64 take, and the product of a few experts in 64 bits within
+    row, as many entries as each form of the lists' walk takes and one more: the words of the same rows in portions that tiles of 64 take, and the product of a few experts in 64 bits within
     what bfloat16 activations give."""
     note(f"experts, tiles of every size {counts} ff {ff} width {width}")
     rng = np.random.default_rng(ff + width)
