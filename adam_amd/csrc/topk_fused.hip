@@ -14,7 +14,7 @@
 // by smaller row index; slots a group cannot fill hold index 0 and the most negative float.  A NaN
 // logit ranks as the most negative float (the reference's insertion leaves a NaN wherever it was
 // first put, which no caller relies on).  Groups of up to 1024 rows are ranked by counting, for every
-// row, the rows that beat it; larger groups by k rounds of a workgroup-wide best-of.
+// row or those that can be among the k best, the rows that beat it; larger groups by k rounds of a workgroup-wide best-of.
 #include "gemv_common.h"
 #include <cstdio>
 #include <algorithm>
@@ -138,29 +138,32 @@ k_group_topk(float* act, float* logits, const uint32_t* __restrict__ pen, const 
   }
 }
 
-// Groups of at most 1024 rows: the group's (penalised) logits sit in LDS.  The k-th largest of the maxima that four threads have together (64 of
-// them) has at least k rows at or above it, and hardly more than a hundred: these are listed, every thread counts those that rank before its own
-// and stores the ones with fewer than k of them straight into their slot.  Bound by latency and LDS reads: 1024 groups of 256 rows, k = 40,
-// 13.0 us with each row compared with all of its group, 6.7 so.
+// Groups of at most 1024 rows: the group's (penalised) logits sit in LDS.  Up to RANK_ALL of them, every thread counts the rows that rank before
+// its own and stores those with fewer than k of them straight into their slot.  More: the k-th largest of the maxima that four threads have together (64 of
+// them) has at least k rows at or above it, and hardly more than a hundred: only these are listed and counted.  Where many rows are equal to it
+// (more than RANK_TIES listed), only the first k of those: 65536 rows in groups of 1024, all equal, k = 8, with the product 61 us with each of them counted, 19 so.
+// Bound by latency and LDS reads: 1024 groups of 256 rows, k = 40, 6.7 us, 13.0 with each row compared with all of its group; 8192 groups of 32 rows
+// with the product 49.5 by the bound, 34 by comparing all, 1002 of 128 rows 21.8 and 21.2.
 #define RANK_MAX 1024u
+#define RANK_ALL 128u
+#define RANK_TIES 192u
+template <bool ALL>
 __global__ void __launch_bounds__(256)
 k_group_topk_rank(float* act, const float* __restrict__ logits, const uint32_t* __restrict__ pen,
                   const uint32_t* __restrict__ lidx, const uint32_t* __restrict__ lval, uint32_t N, uint32_t k,
                   uint32_t n_pen, float rp, uint32_t rows_per_group, uint64_t act_elems) {
-  __shared__ float vs[RANK_MAX];
-  __shared__ __attribute__((aligned(16))) unsigned long long list[RANK_MAX + 1u];   // a value as bits in order, ~row of the group: larger is before
-  __shared__ float largest[64];
-  __shared__ uint32_t pen_s[TOPK_MAX], to_i[TOPK_MAX], to_v[TOPK_MAX];
-  __shared__ uint32_t n_list;
-  const uint32_t tid = threadIdx.x, grp = blockIdx.x, lane = tid & 63u;
+  constexpr uint32_t MAX = ALL ? RANK_ALL : RANK_MAX;
+  __shared__ __attribute__((aligned(16))) float vs[MAX];
+  __shared__ uint32_t pen_s[TOPK_MAX];
+  const uint32_t tid = threadIdx.x, grp = blockIdx.x;
   const uint32_t row0 = grp * rows_per_group, rows = min(N, row0 + rows_per_group) - row0;
-  if (tid < k) { to_i[tid] = lidx[(uint64_t)grp * k + tid]; to_v[tid] = lval[(uint64_t)grp * k + tid]; }
   for (uint32_t i = tid; i < rows; i += 256u) {
     const float v = logits[row0 + i];
     vs[i] = v != v ? NEG_FLT_MAX : v;
   }
+  // padding of the last quad: NaN compares false both ways, so it is never counted
+  if (ALL) for (uint32_t i = rows + tid; i < ((rows + 3u) & ~3u); i += 256u) vs[i] = __uint_as_float(0x7FC00000u);
   if (tid < n_pen) pen_s[tid] = pen[tid];
-  if (tid == 0) n_list = 0u;
   __syncthreads();
   if (tid < n_pen) {
     const uint32_t id = pen_s[tid];
@@ -168,42 +171,87 @@ k_group_topk_rank(float* act, const float* __restrict__ logits, const uint32_t* 
     for (uint32_t j = 0; j < tid; j++) first = first && pen_s[j] != id;
     if (first) vs[id - row0] = penalised(vs[id - row0], rp);
   }
-  __syncthreads();
-  float top = -INFINITY;                        // (also of threads without a row: every row is at or above it)
-  for (uint32_t i = tid; i < rows; i += 256u) top = fmaxf(top, vs[i]);
-  top = fmaxf(top, __shfl_xor(top, 1, 64)); top = fmaxf(top, __shfl_xor(top, 2, 64));
-  if ((tid & 3u) == 0u) largest[tid >> 2] = top;
-  __syncthreads();
-  const float mine = largest[lane];             // every wave for itself: which lane holds the k-th largest
-  uint32_t before = 0;
+  const auto put = [&](uint32_t i, uint64_t di, uint64_t dv) {
+    if (di < act_elems) act[di] = (float)(row0 + i);
+    if (dv < act_elems) act[dv] = vs[i];
+  };
+  if constexpr (ALL) {
+    __syncthreads();
+    if (tid < rows) {
+      const float v = vs[tid];
+      uint32_t cnt = 0;
+      for (uint32_t j = 0; j < rows; j += 4u) {   // branch-free: rows before this one win ties
+        const float4 w = *(const float4*)&vs[j];
+        cnt += (uint32_t)(w.x > v) | ((uint32_t)(w.x == v) & (uint32_t)(j < tid));
+        cnt += (uint32_t)(w.y > v) | ((uint32_t)(w.y == v) & (uint32_t)(j + 1u < tid));
+        cnt += (uint32_t)(w.z > v) | ((uint32_t)(w.z == v) & (uint32_t)(j + 2u < tid));
+        cnt += (uint32_t)(w.w > v) | ((uint32_t)(w.w == v) & (uint32_t)(j + 3u < tid));
+      }
+      if (cnt < k) put(tid, lidx[(uint64_t)grp * k + cnt], lval[(uint64_t)grp * k + cnt]);
+    }
+  } else {
+    __shared__ __attribute__((aligned(16))) unsigned long long list[RANK_MAX + 1u];   // a value as bits in order, ~row of the group: larger is before
+    __shared__ float largest[64];
+    __shared__ uint32_t to_i[TOPK_MAX], to_v[TOPK_MAX], ties[RANK_MAX / 64u], n_list[2];
+    const uint32_t lane = tid & 63u, wave = tid >> 6;
+    if (tid < k) { to_i[tid] = lidx[(uint64_t)grp * k + tid]; to_v[tid] = lval[(uint64_t)grp * k + tid]; }
+    if (tid < 2u) n_list[tid] = 0u;
+    __syncthreads();
+    float top = -INFINITY;                        // (also of threads without a row: every row is at or above it)
+    for (uint32_t i = tid; i < rows; i += 256u) top = fmaxf(top, vs[i]);
+    top = fmaxf(top, __shfl_xor(top, 1, 64)); top = fmaxf(top, __shfl_xor(top, 2, 64));
+    if ((tid & 3u) == 0u) largest[tid >> 2] = top;
+    __syncthreads();
+    const float mine = largest[lane];             // every wave for itself: which lane holds the k-th largest
+    uint32_t before = 0;
 #pragma unroll
-  for (uint32_t j = 0; j < 64u; j++) {
-    const float other = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(mine), (int)j));
-    before += other > mine || (other == mine && j < lane) ? 1u : 0u;
-  }
-  const float least = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(mine), (int)__builtin_ctzll(__ballot(before == k - 1u))));
-  for (uint32_t i = tid; i < rows; i += 256u)
-    if (vs[i] >= least) {
+    for (uint32_t j = 0; j < 64u; j++) {
+      const float other = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(mine), (int)j));
+      before += other > mine || (other == mine && j < lane) ? 1u : 0u;
+    }
+    const float least = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(mine), (int)__builtin_ctzll(__ballot(before == k - 1u))));
+    const auto note = [&](uint32_t i, uint32_t which) {
       const uint32_t b = __float_as_uint(vs[i] + 0.f);      // (zeros of either sign are one value)
-      list[atomicAdd(&n_list, 1u)] = (unsigned long long)((b & 0x80000000u) ? ~b : (b | 0x80000000u)) << 32 | (0xFFFFFFFFu - i);
+      list[atomicAdd(&n_list[which], 1u)] = (unsigned long long)((b & 0x80000000u) ? ~b : (b | 0x80000000u)) << 32 | (0xFFFFFFFFu - i);
+    };
+    uint64_t tie[RANK_MAX / 256u];                // which lanes' rows are equal to the bound: rows 256 j + 64 wave + lane
+#pragma unroll
+    for (uint32_t j = 0; j < RANK_MAX / 256u; j++) {
+      const uint32_t i = tid + 256u * j;
+      tie[j] = 0u;
+      if (256u * j < rows) {
+        const float v = i < rows ? vs[i] : -INFINITY;
+        tie[j] = __ballot(i < rows && v == least);
+        if (lane == 0u) ties[4u * j + wave] = __popcll(tie[j]);
+        if (i < rows && v >= least) note(i, 0u);
+      }
     }
-  __syncthreads();
-  const uint32_t listed = n_list;
-  if (tid == 0) list[listed] = 0u;              // (read in pairs)
-  __syncthreads();
-  for (uint32_t c = tid; c < listed; c += 256u) {
-    const unsigned long long key = list[c];
-    const uint32_t i = 0xFFFFFFFFu - (uint32_t)key;
-    uint32_t cnt = 0;
+    __syncthreads();
+    uint32_t listed = n_list[0];
+    if (listed > RANK_TIES) {                     // again, of the equal ones those that fewer than k others are ahead of
+      uint32_t ahead = 0, q = 0;
+#pragma unroll
+      for (uint32_t j = 0; j < RANK_MAX / 256u; j++) {
+        if (256u * j < rows) {
+          for (; q < 4u * j + wave; q++) ahead += ties[q];
+          const uint32_t i = tid + 256u * j;
+          if (i < rows && (vs[i] > least || ((tie[j] >> lane & 1u) && ahead + __popcll(tie[j] & ((1ull << lane) - 1ull)) < k))) note(i, 1u);
+        }
+      }
+      __syncthreads();
+      listed = n_list[1];
+    }
+    if (tid == 0) list[listed] = 0u;              // (read in pairs)
+    __syncthreads();
+    for (uint32_t c = tid; c < listed; c += 256u) {
+      const unsigned long long key = list[c];
+      uint32_t cnt = 0;
 #pragma unroll 8
-    for (uint32_t j = 0; j < listed; j += 2u) {
-      const ulonglong2 w = *(const ulonglong2*)(list + j);
-      cnt += (w.x > key ? 1u : 0u) + (w.y > key ? 1u : 0u);
-    }
-    if (cnt < k) {
-      const uint64_t di = to_i[cnt], dv = to_v[cnt];
-      if (di < act_elems) act[di] = (float)(row0 + i);
-      if (dv < act_elems) act[dv] = vs[i];
+      for (uint32_t j = 0; j < listed; j += 2u) {
+        const ulonglong2 w = *(const ulonglong2*)(list + j);
+        cnt += (w.x > key ? 1u : 0u) + (w.y > key ? 1u : 0u);
+      }
+      if (cnt < k) put(0xFFFFFFFFu - (uint32_t)key, to_i[cnt], to_v[cnt]);
     }
   }
   for (uint32_t t = rows + tid; t < k; t += 256u) {   // slots the group cannot fill
@@ -293,11 +341,13 @@ static int op_matvec_topk(uint32_t dtype, uint32_t map_act, uint32_t map_wt, uin
   }
   if (r) return r;
   // one choice from the listed rows or k rounds of a pick: 65536 rows in groups of 1024, k = 8 / 40 / 64, 14.5 / 15.5 / 23 us with the product and
-  // 25 / 80 / 121, in groups of 512, k = 2, 13.7 and 14.6; only where all rows are equal and k is small are the rounds quicker (k = 8: 58 and 26)
-  if (tuning("ADAMAH_TOPK_RANK", 1) != 0 && rows_per_group <= RANK_MAX)
-    k_group_topk_rank<<<n_groups, 256, 0, g.stream>>>(act, logits, pen, lidx, lval, N, k, n_pen, rp,
-                                                      rows_per_group, ma->n_elems);
-  else
+  // 25 / 80 / 121, in groups of 512, k = 2, 13.9 and 14.0, k = 1 13.4 and 12.6 (all rows equal, groups of 1024, k = 2: 19.2 and 18.3)
+  if (tuning("ADAMAH_TOPK_RANK", k > 1u || std::min(rows_per_group, N) <= 102u ? 1 : 0) != 0 && rows_per_group <= RANK_MAX) {
+    if (std::min(rows_per_group, N) <= RANK_ALL)
+      k_group_topk_rank<true><<<n_groups, 256, 0, g.stream>>>(act, logits, pen, lidx, lval, N, k, n_pen, rp, rows_per_group, ma->n_elems);
+    else
+      k_group_topk_rank<false><<<n_groups, 256, 0, g.stream>>>(act, logits, pen, lidx, lval, N, k, n_pen, rp, rows_per_group, ma->n_elems);
+  } else
     k_group_topk<<<n_groups, 256, 0, g.stream>>>(act, logits, pen, lidx, lval, N, k, n_pen, rp, rows_per_group,
                                                  ma->n_elems);
   count_launch();

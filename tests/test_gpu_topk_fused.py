@@ -79,9 +79,11 @@ def test_topk_against_oracle(hip, kind, N, K, k, rpg, n_pen):
     check(got, o, N, k, rpg)
 
 
-@pytest.mark.parametrize("N,k,rpg,distinct", [(5000, 40, 1024, 1), (3000, 64, 333, 2), (2050, 1, 1024, 3), (1025, 40, 1024, 70), (700, 64, 63, 1)])
+@pytest.mark.parametrize("N,k,rpg,distinct", [(5000, 40, 1024, 1), (3000, 64, 333, 2), (2050, 1, 1024, 3), (1025, 40, 1024, 70), (700, 64, 63, 1), (2050, 2, 1024, 1),
+                                            (1000, 64, 129, 1), (1000, 64, 128, 2), (300, 1, 102, 1), (309, 1, 103, 2), (4000, 64, 777, 3), (3000, 8, 1000, 2), (500, 64, 193, 1)])
 def test_topk_of_equal_rows(hip, N, k, rpg, distinct):
-    """Groups of few distinct logits, zeros of either sign among them: every row is listed, or many that tie; the lowest rows come first."""
+    """Groups of few distinct logits, zeros of either sign among them, on both sides of the lines between comparing all rows, listing those at the bound and
+    listing only the first of those that tie there, and between lists and rounds: the lowest rows come first."""
     K = 128
     rng = np.random.default_rng(N)
     w = rng.standard_normal((distinct, K), dtype=np.float32)
