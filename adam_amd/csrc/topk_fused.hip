@@ -169,7 +169,10 @@ k_group_topk_rank(float* act, const float* __restrict__ logits, const uint32_t* 
     const uint32_t id = pen_s[tid];
     bool first = id >= row0 && id - row0 < rows;
     for (uint32_t j = 0; j < tid; j++) first = first && pen_s[j] != id;
-    if (first) vs[id - row0] = penalised(vs[id - row0], rp);
+    if (first) {
+      const float v = penalised(vs[id - row0], rp);
+      vs[id - row0] = v != v ? NEG_FLT_MAX : v;
+    }
   }
   const auto put = [&](uint32_t i, uint64_t di, uint64_t dv) {
     if (di < act_elems) act[di] = (float)(row0 + i);

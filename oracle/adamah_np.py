@@ -1015,6 +1015,7 @@ class NumpyAdamah(MixerOps):
         for r in pen:
             if r < N:
                 y[r] = y[r] / rp if y[r] > 0 else y[r] * rp
+        y[np.isnan(y)] = NEG_MAX                       # (0 by an infinite penalty)
         for g in range(ng):
             rows = np.arange(g * rpg, min(N, (g + 1) * rpg))
             order = sorted(rows.tolist(), key=lambda r: (-float(y[r]), r))[:k]

@@ -102,6 +102,30 @@ def test_topk_of_equal_rows(hip, N, k, rpg, distinct):
         assert np.all(np.abs(val[g, :len(best)] - o.last_logits[rows[best]]) <= 1e-3 * max(1.0, np.abs(o.last_logits).max()))
 
 
+@pytest.mark.parametrize("N,k,rpg", [(70, 64, 32), (256, 40, 128), (520, 64, 129), (2060, 12, 1030)])
+def test_topk_of_logits_that_a_penalty_makes_no_number(hip, N, k, rpg):
+    """A zero logit times an infinite penalty ranks as the most negative float, as a NaN logit does, in groups of every kind: it takes no other's slot."""
+    K = 128
+    rng = np.random.default_rng(N)
+    w = rng.standard_normal((N, K), dtype=np.float32)
+    w[::7] = 0.0
+    qt = quant.quantize_q4_0(w)
+    x = rng.standard_normal(K).astype(np.float32)
+    pen = np.array([0, 7, 14, rpg // 7 * 7 + 7, 3], np.uint32)
+    note(f"matvec_topk no number {N} k={k} rpg={rpg}")
+    idx, val = run_topk(hip, qt, x, k, rpg, pen, np.inf)
+    o = oracle.init()
+    with np.errstate(invalid="ignore"):
+        run_topk(o, qt, x, k, rpg, pen, np.inf)
+    for g in range(idx.shape[0]):
+        rows = np.arange(g * rpg, min(N, (g + 1) * rpg))
+        y = o.last_logits[rows].astype(np.float64)
+        best = np.argsort(-np.round(y, 3), kind="stable")[:k]
+        best = best[np.isfinite(y[best])]                      # (row 3 may be a negative infinity)
+        assert np.array_equal(idx[g, :len(best)].astype(np.int64), rows[best])
+        assert np.all(np.abs(val[g, :len(best)] - o.last_logits[rows[best]]) <= 1e-3 * np.abs(y[np.abs(y) < 1e30]).max())
+
+
 def test_topk_default_group_and_penalty_effect(hip):
     """The form without rows_per_group uses 256; a penalised favourite drops out of its group's list."""
     rng = np.random.default_rng(3)
