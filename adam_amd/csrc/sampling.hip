@@ -131,15 +131,16 @@ k_topk_merge(float* data, const float* __restrict__ part_v, const uint32_t* __re
 
 // Top-k of 4096 < n <= 40960 candidates in one launch of one workgroup of 1024 threads, the values in registers (at most 40 per
 // thread).  A candidate's place in the strict order (value descending, index ascending) is the 48-bit key (orderable value bits, 0xFFFF - index).
-// Sixteen threads' candidates are a group: the k-th largest of the 64 groups' largest values has at least k candidates at or above it,
-// and hardly more than a hundred, which are listed and put in order by counting.  Where more than TSEL_LIST are (many equal values),
-// radix selection: five histogram passes over its digits (11, 11, 10 bits of the value, then 8, 8 of the index, top down) find the key of the k-th best -- each pass counts
+// Sixteen threads' candidates are a group, one a wave, another lane in each, so that the best of neither a sorted run nor sorted lists beside each other meet in
+// few groups: the k-th largest of the 64 groups' largest values has at least k candidates at or above it,
+// and hardly more than a hundred, which are listed and put in order by counting.  Where more than TSEL_LIST are, only the first k of those equal to the bound; where that
+// leaves more than TSEL_LIST still, radix selection: five histogram passes over its digits (11, 11, 10 bits of the value, then 8, 8 of the index, top down) find the key of the k-th best -- each pass counts
 // the candidates that agree with the digits fixed so far, a suffix scan over the bins finds the bin the k-th falls in --
 // and everything at or above that key is gathered and put in order by counting.  Same results as the rounds
-// (tests/test_gpu_sampling.py).  Bound by latency: the partial lists of the sampled LM head (40960 candidates, k = 40) take 17.4 us, 41 by
-// radix selection alone (in no order in the map 29 and 51; 10240 of them 14.7 and 27; all equal 69 and 60); that one took 59 with each load under a condition and one
-// count a bin, 41 with loads on every path, TSEL_ASK at a time, and four counts a bin (the values share few bins of the first
-// passes, and a wave's counts of one address go one behind the other).
+// (tests/test_gpu_sampling.py).  Bound by latency: the partial lists of the sampled LM head (40960 candidates, k = 40) take 17.3 us, by
+// radix selection alone 40 (in no order in the map 28.7 and 51, sorted 18 and 44, all equal 26.4 and 60; 10240 of them 13.8 and 27); where that is what it comes to
+// after all (large values in fewer than k of the groups) 51 and 43.  Radix selection: loads on every path, TSEL_ASK at a time, and four counts a bin (the values share
+// few bins of the first passes, and a wave's counts of one address go one behind the other); 59 us with each load under a condition and one count a bin.
 #define TSEL_THREADS 1024u
 #define TSEL_PER 40u
 #define TSEL_ASK 20u
@@ -151,7 +152,7 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
               uint32_t n, uint32_t k, uint64_t n_elems) {
   __shared__ uint4 hist[2048];                  // a bin's counts of the lanes with the same two last bits
   __shared__ uint32_t wtot[16];
-  __shared__ uint32_t sel_bin, sel_rem, n_win, n_list, largest[64], to_i[SMP_MAX], to_v[SMP_MAX];
+  __shared__ uint32_t sel_bin, sel_rem, n_win, n_list[2], largest[TSEL_THREADS], ties[16][TSEL_PER / 4u], to_i[SMP_MAX], to_v[SMP_MAX];
   __shared__ float win_v[SMP_MAX];
   __shared__ uint32_t win_i[SMP_MAX];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
@@ -162,7 +163,7 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
   const auto first = [&](uint32_t u) { return at + u * (4u * TSEL_THREADS); };
   const auto place = [&](uint32_t u) { return min(first(u), n - 4u); };         // candidate u's e-th is place(u) + e, there if that is at least first(u)
   if (tid < k) { to_i[tid] = li[tid]; to_v[tid] = lv[tid]; }
-  if (tid == 0) { n_win = 0u; n_list = 0u; }
+  if (tid == 0) { n_win = 0u; n_list[0] = 0u; n_list[1] = 0u; }
   uint32_t vk[TSEL_PER];   // orderable value bits of candidate place(j / 4) + j % 4
 #pragma unroll
   for (uint32_t u0 = 0; u0 < TSEL_PER / 4u; u0 += TSEL_ASK / 4u) {
@@ -199,11 +200,11 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
   uint32_t top = 0u;                            // (below every value's bits)
 #pragma unroll
   for (uint32_t j = 0; j < TSEL_PER; j++) if (j / 4u < per && place(j / 4u) + j % 4u >= first(j / 4u)) top = max(top, vk[j]);
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
-  if ((tid & 15u) == 0u) largest[tid >> 4] = top;
+  largest[64u * wave + ((lane + 7u * wave) & 63u)] = top;
   __syncthreads();
-  const uint32_t mine = largest[lane];          // every wave for itself: which lane holds the kk-th largest
+  uint32_t mine = 0u;                           // every wave for itself: which lane holds the kk-th largest
+#pragma unroll
+  for (uint32_t w = 0; w < 16u; w++) mine = max(mine, largest[64u * w + lane]);
   uint32_t before = 0;
 #pragma unroll
   for (uint32_t j = 0; j < 64u; j++) {
@@ -212,17 +213,73 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
   }
   const uint32_t least = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)__builtin_ctzll(__ballot(before == kk - 1u)));
   unsigned long long* const list = (unsigned long long*)hist;
+  const auto note = [&](uint32_t j, uint32_t i, uint32_t which) {
+    const uint32_t slot = atomicAdd(&n_list[which], 1u);
+    if (slot < TSEL_LIST) list[slot] = (unsigned long long)vk[j] << 32 | (0xFFFFFFFFu - i);
+    return slot < TSEL_LIST;
+  };
   anew();
+  bool room = true;
 #pragma unroll
   for (uint32_t j = 0; j < TSEL_PER; j++) {
     const uint32_t i = place(j / 4u) + j % 4u;
-    if (j / 4u < per && i >= first(j / 4u) && vk[j] >= least) {
-      const uint32_t slot = atomicAdd(&n_list, 1u);
-      if (slot < TSEL_LIST) list[slot] = (unsigned long long)vk[j] << 32 | (0xFFFFFFFFu - i);
+    if (j / 4u < per && room) {
+      bool noted = true;
+      if (i >= first(j / 4u) && vk[j] >= least) noted = note(j, i, 0u);
+      room = __all(noted);
     }
   }
   __syncthreads();
-  const uint32_t listed = n_list;
+  uint32_t listed = n_list[0];
+  if (listed > TSEL_LIST) {                     // many equal values: again, of those at the bound the first kk
+    anew();
+    uint32_t more = 0;                          // this wave's above the bound
+#pragma unroll
+    for (uint32_t u = 0; u < TSEL_PER / 4u; u++) {
+      uint32_t c = 0;
+      if (u < per) {
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) {
+          const bool in = place(u) + e >= first(u);
+          c += __popcll(__ballot(in && vk[4u * u + e] == least));
+          more += __popcll(__ballot(in && vk[4u * u + e] > least));
+        }
+      }
+      if (lane == 0u) ties[wave][u] = c;
+    }
+    if (lane == 0u) wtot[wave] = more;
+    __syncthreads();
+    more = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 16u; w++) more += wtot[w];
+    anew();
+    uint32_t ahead = 0;                         // (places in order: u, wave, lane, e)
+#pragma unroll
+    for (uint32_t u = 0; u < TSEL_PER / 4u; u++) {
+      if (u < per && more + kk <= TSEL_LIST) {
+        uint32_t mine_first = ahead;
+        for (uint32_t w = 0; w < 16u; w++) {
+          const uint32_t c = ties[w][u];
+          mine_first += w < wave ? c : 0u;
+          ahead += c;
+        }
+        bool tie[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) {
+          tie[e] = place(u) + e >= first(u) && vk[4u * u + e] == least;
+          mine_first += __popcll(__ballot(tie[e]) & ((1ull << lane) - 1ull));
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < 4u; e++) {
+          const uint32_t i = place(u) + e;
+          if (i >= first(u) && (vk[4u * u + e] > least || (tie[e] && mine_first < kk))) note(4u * u + e, i, 1u);
+          mine_first += tie[e] ? 1u : 0u;
+        }
+      }
+    }
+    __syncthreads();                            // (and wtot is free again)
+    listed = more + kk <= TSEL_LIST ? n_list[1] : TSEL_LIST + 1u;
+  }
   if (listed <= TSEL_LIST) {
     if (tid < listed) {
       const unsigned long long key = list[tid];

@@ -39,10 +39,12 @@ def test_topk(hip, n, k, seed):
 
 
 @pytest.mark.parametrize("n,k,order", [(4097, 40, "random"), (40960, 40, "random"), (10240, 64, "lists"), (40960, 40, "lists"), (40960, 64, "up"), (9999, 64, "down"),
-                                       (5000, 1, "random"), (5000, 64, "infinite"), (20000, 40, 1024), (20000, 40, 1025), (20000, 64, 30), (4103, 40, "scattered"), (33001, 64, "scattered"), (33002, 40, 2000)])
+                                       (5000, 1, "random"), (5000, 64, "infinite"), (20000, 40, 1024), (20000, 40, 1025), (20000, 64, 30), (4103, 40, "scattered"), (33001, 64, "scattered"), (33002, 40, 2000),
+                                       (40957, 64, 40957), (4097, 64, 4000), (40960, 40, "lanes"), (5001, 64, "lanes"), (12000, 64, "infinite"), (9000, 40, "steps")])
 def test_topk_listed_or_by_radix(hip, n, k, order):
     """Candidates beside each other in the map and all over it, some outside of it; in no order, in sorted lists of 40 as the LM head leaves them, rising and falling along the whole list, with infinities and zeros of
-    either sign, and as many equal largest ones as the kernel's list holds, one more, and fewer than k."""
+    either sign, as many equal largest ones as the kernel's list holds, one more, all, and fewer than k, many equal ones behind a few larger, and large ones that share few of the maxima that
+    the bound is taken from (radix selection)."""
     rng = np.random.default_rng(n + k)
     v = rng.standard_normal(n).astype(np.float32)
     if order == "lists":
@@ -52,6 +54,10 @@ def test_topk_listed_or_by_radix(hip, n, k, order):
     elif order == "infinite":
         v[:] = -np.inf
         v[rng.permutation(n)[:50]] = np.array([np.inf, 0.0, -0.0, np.nan, -1.0] * 10, np.float32)
+    elif order == "lanes":
+        v = np.where((np.arange(n) // 4 % 64 + np.arange(n) % 4096 // 256 * 7) % 64 < k - 1, np.abs(v) + np.float32(9), v)
+    elif order == "steps":
+        v = np.floor(v * 2).astype(np.float32)
     elif order not in ("random", "scattered"):
         v[rng.permutation(n)[:order]] = 9.0
     note(f"topk listed n={n} k={k} {order}")
@@ -64,13 +70,9 @@ def test_topk_listed_or_by_radix(hip, n, k, order):
         v = np.where(at < n, v, np.float32(np.nan))
     hip.map_topk_dev(0, up(hip, at), up(hip, n + np.arange(k)), up(hip, n + 128 + np.arange(k)), n, k)
     x = np.where(np.isnan(v), np.float32(-3.402823466e+38), v)
-    # (zeros of either sign are one value where results are put in order; the larger sign is taken first, and all 50 are taken here)
-    want = np.argsort(-x, kind="stable")[:k]
-    got = read(hip, 0, n, k)
-    if order == "infinite":
-        want = want[:30]                             # (behind the finite ones: lowest values and infinities below them)
-    assert np.array_equal(got[:len(want)].astype(np.int64), want)
-    assert np.array_equal(read(hip, 0, n + 128, k)[:len(want)].view(np.uint32), x[want].view(np.uint32))
+    want = np.argsort(-x, kind="stable")[:k]                   # (zeros of either sign are one value)
+    assert np.array_equal(read(hip, 0, n, k).astype(np.int64), want)
+    assert np.array_equal(read(hip, 0, n + 128, k).view(np.uint32), x[want].view(np.uint32))
     assert (read(hip, 0, n + 128 + k, 1) == 7.0).all()
 
 
