@@ -648,6 +648,14 @@ def test_narrow_tiles_at_ragged_ends(hip, monkeypatch, M, N, K, base):
     test_many_rows_on_every_tile_and_share_of_k(hip, M, N, K, base)
 
 
+@pytest.mark.parametrize("M,N,K,plan", [(512, 1152, 1536, (32, 1)), (189, 1024, 1152, (32, 1)), (65, 64, 1920, (32, 1)), (512, 6912, 1920, (64, 2)), (256, 13824, 1920, (64, 2)),
+                                        (512, 1152, 2048, (0, 1)), (512, 13824, 1152, (64, 1))])
+def test_narrow_tiles_where_they_are_the_quicker_ones(hip, M, N, K, plan):
+    """The rule at shapes whose forms were timed against each other (256 CUs)."""
+    note(f"gemm q4 plan M={M} N={N} K={K}")
+    assert hip.matmul_plan(M, K, N) == plan
+
+
 @pytest.mark.parametrize("M,K,Ns,add", [(70, 384, (500, 36, 700), False), (189, 1152, (1024, 256, 256), False), (301, 1152, (1152,), True), (66, 256, (31,), True)])
 def test_narrow_tiles_store_stacked_results_and_adds(hip, M, K, Ns, add):
     """What the rule sends there: borders of stacked matrices inside a workgroup's 128 weight rows, and the add behind a single one."""
