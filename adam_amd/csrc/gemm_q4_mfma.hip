@@ -809,41 +809,47 @@ k_gemm_q4_rows(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 #pragma unroll
         for (int k = 0; k < 4; k++) part[((wave * RC + r) * NA + t) * 256u + k * 64u + lane] = acc[r0 + r][t][k];
     __syncthreads();
-    for (uint32_t idx = tid; idx < M * 16u; idx += 64u * NWV) {
-      // activation row `row` of tile column c: operand rows `row` and M + row of every wave (PAIR: row `row` of the one sum)
-      const uint32_t row = idx >> 4, c = idx & 15u, lo = M + row;
-      const auto place = [&](uint32_t v) { return (v >> 4) * 256u + (v & 3u) * 64u + ((v >> 2) & 3u) * 16u + c; };
-      const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
-      const bool add = !segs.count && segs.add;
-      float y[RC], old[RC];
-      ColumnPlace to[RC];
+    // how: 0 one matrix, 1 and the add behind it, 2 stacked matrices (one by the stacked ones' places: 40 x 28672 x 1152 25.0 us, 23.2 so)
+    const auto rows = [&](auto how) {
+      for (uint32_t idx = tid; idx < M * 16u; idx += 64u * NWV) {
+        // activation row `row` of tile column c: operand rows `row` and M + row of every wave (PAIR: row `row` of the one sum)
+        const uint32_t row = idx >> 4, c = idx & 15u, lo = M + row;
+        const auto place = [&](uint32_t v) { return (v >> 4) * 256u + (v & 3u) * 64u + ((v >> 2) & 3u) * 16u + c; };
+        const float inv = scale[2 * ((uint64_t)op * M + row) + 1];
+        float y[RC], old[RC];
+        ColumnPlace to[RC];
 #pragma unroll
-      for (int r = 0; r < RC; r++) {
-        const uint32_t n = min(first_row(r0 + r) + c, N - 1u);
-        to[r] = column_place(n, N, c_off, out, segs);
-        if (add) old[r] = out[segs.res + (uint64_t)row * N + n];
-      }
-#pragma unroll
-      for (int r = 0; r < RC; r++) {
-        float a = 0.f, b = 0.f;
-#pragma unroll
-        for (uint32_t w = 0; w < NWV; w++) {
-          const float* p = part + (w * RC + r) * NA * 256u;
-          a += p[place(row)];
-          if (!PAIR) b += p[place(lo)];
+        for (int r = 0; r < RC; r++) {
+          const uint32_t n = min(first_row(r0 + r) + c, N - 1u);
+          if (how == 2) to[r] = column_place(n, N, c_off, out, segs);
+          if (how == 1) old[r] = out[segs.res + (uint64_t)row * N + n];
         }
-        y[r] = (a + b) * inv;
-      }
 #pragma unroll
-      for (int r = 0; r < RC; r++) {
-        const uint32_t n = first_row(r0 + r) + c;
-        if (n >= (glum && !(r & 1) ? N >> 1 : N)) continue;
-        to[r].col[(uint64_t)row * to[r].step] = y[r];
-        if (add) out[segs.dst + (uint64_t)row * N + n] = old[r] + y[r];
+        for (int r = 0; r < RC; r++) {
+          float a = 0.f, b = 0.f;
+#pragma unroll
+          for (uint32_t w = 0; w < NWV; w++) {
+            const float* p = part + (w * RC + r) * NA * 256u;
+            a += p[place(row)];
+            if (!PAIR) b += p[place(lo)];
+          }
+          y[r] = (a + b) * inv;
+        }
+#pragma unroll
+        for (int r = 0; r < RC; r++) {
+          const uint32_t n = first_row(r0 + r) + c;
+          if (n >= (glum && !(r & 1) ? N >> 1 : N)) continue;
+          if (how == 2) to[r].col[(uint64_t)row * to[r].step] = y[r];
+          else out[c_off + (uint64_t)row * N + n] = y[r];
+          if (how == 1) out[segs.dst + (uint64_t)row * N + n] = old[r] + y[r];
+        }
+        if (how == 2 && glum && first_row(r0) + c < (N >> 1))   // act(gate) * up, as the element-wise op computes it
+          out[segs.dst + (uint64_t)row * (N >> 1) + first_row(r0) + c] = (segs.glu == 34u ? gelu_tanh(y[0]) : y[0] / (1.0f + expf(-y[0]))) * y[RC - 1];
       }
-      if (glum && first_row(r0) + c < (N >> 1))   // act(gate) * up, as the element-wise op computes it
-        out[segs.dst + (uint64_t)row * (N >> 1) + first_row(r0) + c] = (segs.glu == 34u ? gelu_tanh(y[0]) : y[0] / (1.0f + expf(-y[0]))) * y[RC - 1];
-    }
+    };
+    if (segs.count) rows(std::integral_constant<int, 2>{});
+    else if (segs.add) rows(std::integral_constant<int, 1>{});
+    else rows(std::integral_constant<int, 0>{});
   }
 }
 
@@ -1173,6 +1179,12 @@ k_gemm_q4_f16_rows16(const uint8_t* __restrict__ W, const __half* __restrict__ d
   }
   if (glum) __syncthreads();
   const bool n_ok = glum ? tb + r16 < (N >> 1) : n < N;
+  if (!segs.count) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (4u * g + i < M && n_ok) out[c_off + (uint64_t)(4u * g + i) * N + n] = y[i];
+    return;
+  }
   const ColumnPlace to = column_place(n, N, c_off, out, segs);
 #pragma unroll
   for (int i = 0; i < 4; i++) {

@@ -1,10 +1,9 @@
 // Where a matmul's results in registers go: a lane holds single columns of one or many rows.
 //
 // What hangs on the column is worked out once a column, ahead of the stores, from arguments that scalar loads bring: which of the
-// stacked matrices it belongs to, its first element, its rows' distance.  Looked up by result, from the arguments in memory, each waited for
+// stacked matrices it belongs to, its first element, its rows' distance.  Looked up by result, from the arguments in memory, each would wait for
 // three loads and, since loads and stores are counted together, for the store before it: 512 x 28672 x 4096 into two matrices on the
-// ring 245 us, 217 so; 512 x 13824 x 1152 59 and 42; five shares
-// of 512 x 6144 x 4096, raw sums, 64 and 57 (a branch a result less).  1877 tokens through the Llama 8B shape 81.3 -> 75.2 ms.
+// ring 217 us, 245 with that; 512 x 13824 x 1152 42 and 59; five shares of 512 x 6144 x 4096, raw sums, 57 and 64.
 #pragma once
 #include "gemv_common.h"
 
@@ -27,10 +26,24 @@ __device__ __forceinline__ ColumnPlace column_place(uint32_t n, uint32_t N, uint
 template <int T, int I, int W, class V, class R>
 __device__ __forceinline__ void store_columns(const V& value, const R& row, const uint32_t (&n)[W], uint32_t M, uint32_t N, uint32_t kz, uint64_t c_off,
                                               float* out, float* part, const GemmSegs& segs) {
-  ColumnPlace to[W];
+  // (a branch for each: one matrix by way of the stacked ones' places, 2 x 13824 x 1152 of Q8 5.1 us, 4.9 so)
+  if (!part && segs.count) {
+    ColumnPlace to[W];
 #pragma unroll
-  for (int w = 0; w < W; w++) to[w] = part ? ColumnPlace{part + (uint64_t)kz * M * N + n[w], N} : column_place(n[w], N, c_off, out, segs);
-  if (!part && !segs.count && segs.add) {                    // the add behind it: a tile's rows are asked for at once
+    for (int w = 0; w < W; w++) to[w] = column_place(n[w], N, c_off, out, segs);
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+      for (int i = 0; i < I; i++) {
+        if (row(t, i) >= M) continue;
+#pragma unroll
+        for (int w = 0; w < W; w++)
+          if (n[w] < N) to[w].col[(uint64_t)row(t, i) * to[w].step] = value(t, i, w);
+      }
+    return;
+  }
+  float* const at = part ? part + (uint64_t)kz * M * N : out + c_off;
+  if (!part && segs.add) {                                   // the add behind it: a tile's rows are asked for at once
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
@@ -44,7 +57,7 @@ __device__ __forceinline__ void store_columns(const V& value, const R& row, cons
 #pragma unroll
         for (int i = 0; i < I; i++) {
           if (row(t, i) >= M) continue;
-          to[w].col[(uint64_t)row(t, i) * N] = value(t, i, w);
+          at[(uint64_t)row(t, i) * N + n[w]] = value(t, i, w);
           dst[(uint64_t)row(t, i) * N] = old[i] + value(t, i, w);
         }
       }
@@ -57,7 +70,7 @@ __device__ __forceinline__ void store_columns(const V& value, const R& row, cons
       if (row(t, i) >= M) continue;
 #pragma unroll
       for (int w = 0; w < W; w++)
-        if (n[w] < N) to[w].col[(uint64_t)row(t, i) * to[w].step] = value(t, i, w);
+        if (n[w] < N) at[(uint64_t)row(t, i) * N + n[w]] = value(t, i, w);
     }
 }
 
