@@ -283,7 +283,7 @@ k_gemm_q4_f16_tiled(const uint8_t* __restrict__ W, const __half* __restrict__ d1
   uint32_t n[R];
 #pragma unroll
   for (int r = 0; r < R; r++) n[r] = n0 + r * 16u + r16;
-  store_columns<MT, 4, R>([&](int t, int i, int r) { return acc[r][t][i]; }, row, n, M, N, kz, c_off, out, ksplit > 1u ? part : nullptr, segs);
+  store_columns<MT, 4, R, false>([&](int t, int i, int r) { return acc[r][t][i]; }, row, n, M, N, kz, c_off, out, ksplit > 1u ? part : nullptr, segs);
 }
 #undef GEMM_FETCH
 

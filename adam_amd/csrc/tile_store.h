@@ -22,8 +22,8 @@ __device__ __forceinline__ ColumnPlace column_place(uint32_t n, uint32_t N, uint
 }
 
 // value(t, i, w) is the result of row(t, i), i < I, and column n[w]; rows from M and columns from N on have no place.  part: raw sums of
-// share kz; else the places that `segs` names, or element c_off on.
-template <int T, int I, int W, class V, class R>
+// share kz; else the places that `segs` names, or element c_off on.  ADDS: such launches may also store the add behind a single matrix.
+template <int T, int I, int W, bool ADDS = true, class V, class R>
 __device__ __forceinline__ void store_columns(const V& value, const R& row, const uint32_t (&n)[W], uint32_t M, uint32_t N, uint32_t kz, uint64_t c_off,
                                               float* out, float* part, const GemmSegs& segs) {
   // (a branch for each: one matrix by way of the stacked ones' places, 2 x 13824 x 1152 of Q8 5.1 us, 4.9 so)
@@ -43,7 +43,7 @@ __device__ __forceinline__ void store_columns(const V& value, const R& row, cons
     return;
   }
   float* const at = part ? part + (uint64_t)kz * M * N : out + c_off;
-  if (!part && segs.add) {                                   // the add behind it: a tile's rows are asked for at once
+  if (ADDS && !part && segs.add) {                           // the add behind it: a tile's rows are asked for at once
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
