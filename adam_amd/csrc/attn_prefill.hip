@@ -16,9 +16,9 @@
 // softmax per wave and query; values with every lane owning D/64 dims of all 16 outputs.  The waves
 // merge through LDS.  The raw scores of the chunk's last token are stored to the score rows: that
 // is what the rows hold after the run executed token by token, each token overwriting the one before.
-// Bound by latency (queries, first tile, LDS), so by how many waves a CU holds: the weights of all 16 cache rows used to be in registers at once
-// (256 of them, a wave a SIMD), the sums having been moved behind them, and a thread's queries were waited for one by one.  8 runs of 48 tokens
-// over 32 heads of 128: 32.2 us, 26.7 with the queries asked for together, 15.4 with 142 registers (three waves a SIMD) as well.
+// Bound by latency (queries, first tile, LDS), so by how many waves a CU holds: heads of 128 three a SIMD at 142 registers.  Left to itself the compiler moves a tile's
+// sums behind the next tile and holds the weights of all 16 cache rows for them (256 registers, a wave a SIMD).  8 runs of 48 tokens over 32 heads of 128
+// 15.4 us; 26.7 so, 32.2 with a thread's queries waited for one by one as well.  One run of 48 tokens, 32 heads of 64 6.6 us (8.0 so), 4 heads of 256 20.4 (25.7).
 #include "attn_common.h"
 #include <algorithm>
 

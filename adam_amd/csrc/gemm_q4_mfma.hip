@@ -543,8 +543,8 @@ k_gemm_q4_ring(const uint8_t* __restrict__ W, const __half* __restrict__ d16, co
 // step's operands, and adds up the products of the one before, under the products of this one (added up behind its own: a fifth slower over long rows).
 // What bounds it: a step takes 0.44 us with a few workgroups, 0.65 with one on every CU, of which the products need 0.21; the rest is the
 // vector work beside them (unpacking for 32 rows only, a multiply-add per result and block) and, with many workgroups, the activations' way out of the L2s.
-// Against the tiled kernel, whose step of 128 columns waits for its loads (1.3 us): 512 x 1536 x 1152 16.2 -> 10.9 us, 189 x 1536 x 1152 15.1 -> 9.8, 189 x 1152
-// x 1024 13.8 -> 9.4, 70 x 13824 x 1152 22.3 -> 18.9.
+// The tiled kernel, whose step of 128 columns waits for its loads (1.3 us), and so: 512 x 1536 x 1152 16.2 and 10.9 us, 189 x 1536 x 1152 15.1 and 9.8, 189 x 1152
+// x 1024 13.8 and 9.4, 70 x 13824 x 1152 22.3 and 18.9.
 // LDS: piece j of an activation row at j ^ (row & 15), block j of a weight row at j ^ (row / 4 & 3): no two rows that are read together meet in a bank.
 #define NARROW_X 16384u
 #define NARROW_W 8192u
@@ -1458,29 +1458,30 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 
 // How a one-op Q4 matmul of more than 32 rows over a matrix [N, K] from element b on (b < 0: not known here) runs: ma > 1
 // k_gemm_q4_ring<ma>, 1 k_gemm_q4_narrow, 0 the tiled kernel, over how many shares of K; -1 k_gemm_q4_rows.
-// 33 .. 64 rows: k_gemm_q4_rows where a CU has few tiles of 16 weight rows and K is not long, by its time for a round of tiles and
-// a 128-column step (48 rows: 4096 x 4096 12.3 us, tiled 21.7, 6144 x 4096 14.9 and 23.8; 4096 x 14336 38.0 and 34.1; 64 rows:
-// 28672 x 4096 71.9 and 67.7).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
-// a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 136 -> 32 us over 16 shares, 48 x 2048 x
-// 2048: 23 -> 17 over four; 64 x 28672 x 2048 38 in one, 44 in four, 64 x 28672 x 4096 67 and 62).
-// More: the least of these estimates, in us.  Over 360 products of 65 .. 2049 rows by 512 .. 32000 x 128 .. 14336 the plan it picks takes
-// 0.9 % longer than the best one in the mean where N is a multiple of four (15 % at most, 357 rows of 10092 x 1536: 53 us tiled,
-// 46 over two shares), else 1.2 % (20 %, 134 rows of 3575 x 9344: 66 us over 12 shares, 55 over 9).  Tiled, by the tile it would take
+// (All us with the conversion of the rows.)  33 .. 64 rows: k_gemm_q4_rows where a CU has few tiles of 16 weight rows and K is not long, by its time for a round of
+// tiles and a 128-column step (48 rows: 4096 x 4096 16.0, tiled 21.5, 6144 x 4096 17.4 and 23.7; 4096 x 14336 38.1 and 32.7; 64 rows:
+// 28672 x 4096 66.5 and 57.6).  Otherwise tiled; its 64 x 256 tile over shares takes 3 us a 128-column step and 11 for the two launches while no CU has
+// a second one, 4.7 and 17.8 beyond, and a pass over the sums each (48 x 4096 x 14336: 142 in one, 33 over 16 shares; 64 x 28672 x 2048
+// 36.7 in one, 38.5 in four, 64 x 28672 x 4096 63.5 and 57.6).
+// More: the least of these estimates.  Over 850 products of 65 .. 2100 rows by 64 .. 33000 x 128 .. 14336 the plan it picks takes, against the best of tiled, narrow
+// and the ring's own plan, 2.8 % longer in the mean under 2048 columns (40 % at most, 551 rows of 6096 x 1792: 57 tiled, 41 over two shares of the ring,
+// whose estimates lie above what it takes), 11 % from there on (91 %, 65 rows of 4096 x 2048: 22.5 tiled, 11.7 narrow, which has no part there).  Tiled, by the
+// tile it would take
 // (below): 128-column steps of 1.27 us while no CU has a second 64 x 64 tile and 0.72 more for each further one, 4.0 and 2.7
 // more for every two rounds of 64 x 128, 4.6 a round of 256 x 128.  Ring: 64-column steps of 1.7 (ma = 2), 2.35 (3) or 3.0 us (4), up to a
 // quarter more as the CUs fill; shares cost their second launch and a pass over the sums each, where N is no multiple of four two and a
-// half (a result at a time, one share behind the other: 88 rows of 9007 x 5760 57 us over 7 shares of 64 rows a workgroup, 65 over
-// 13 of 96, of 9008 x 5760 50 and 48; 730 of 559 x 11904 69 over 10, 81 over 16, of 560 61 and 63).  (us, conversion included, without and
-// with 96 rows a workgroup: 28672 x 4096 under 96 rows 88 and 76, 150 129 and 114, 192 129 and 118, 288 231 and 184, 384 241 and 212;
-// 4096 x 14336 288 116 and 105, 384 139 and 128; 6144 x 4096 480 90 and 83.)
+// half (a result at a time, one share behind the other: 88 rows of 9007 x 5760 50 over 7 shares of 64 rows a workgroup, 57 over
+// 13 of 96, of 9008 x 5760 45 and 41; 730 of 559 x 11904 65 over 10, 74 over 16 of 96, of 560 56 and 55).  (Without and with 96 rows a
+// workgroup: 28672 x 4096 under 150 rows 106 and 98, 192 103 and 99, 288 174 and 139, 384 177 and 165;
+// 4096 x 14336 288 89 and 83, 384 104 and 101; 6144 x 4096 480 68 and 63.)
 // The ring reads the scales of two blocks as one word and keeps a lane's place in the rows in 32 bits (in the matrix too: a Q4
 // map here has fewer than 2^32 elements): matrices that begin at an odd block stay on the tiled kernel, a narrow one from 128
 // rows on over 2 .. 4 shares (256 x 128 tile; 512 x 4096 x 14336 from an odd block: 234 us in one, 160 in four).
 // Rows of fewer than 2048 columns: also k_gemm_q4_narrow, in steps of 128 columns of 0.42 us with few workgroups, 0.67 with one on every CU, and 3
-// a round of workgroups beside them (512 x 1536 x 1152 estimated 11.5 us, measured 10.9, tiled 16.2; 189 x 13824 x 1152 30.1, 28.7, tiled 29.9;
-// 512 x 13824 x 1152 66, 62, ring 42), where that is a tenth less than the ring's estimate, which is above what the ring takes by that and more (512 x 6912 x 1920
-// estimated 55 and 56 us, measured 51 and 42).  Longer rows go to the ring over shares of K, which is the better one where there are many of them and
-// where the matrix is narrow: 512 x 4096 x 4096 50 us and here 55, 70 x 1152 x 6912 23 and 30 (between them not everywhere: 189 x 4096 x 4096 31 and 26).
+// a round of workgroups beside them (512 x 1536 x 1152 estimated 11.5, measured 12.5, tiled 19.3; 189 x 13824 x 1152 30.1, 28.4, tiled 29.8;
+// 512 x 13824 x 1152 66, 62, ring 44), where that is a tenth less than the ring's estimate, which is above what the ring takes by that and more (512 x 6912 x 1920
+// estimated 55 and 56, measured 54.5 and 47).  Longer rows go to the ring over shares of K, which is the better one where there are many of them and
+// where the matrix is narrow: 512 x 4096 x 4096 51 and here 56, 70 x 1152 x 6912 26 and 36 (between them not everywhere: 189 x 4096 x 4096 32 and 28).
 struct GemmPlan { int ma; uint32_t shares; };
 static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   const auto up = [](uint64_t x, uint64_t y) { return (x + y - 1) / y; };
