@@ -137,9 +137,9 @@ k_topk_merge(float* data, const float* __restrict__ part_v, const uint32_t* __re
 // leaves more than TSEL_LIST still, radix selection: five histogram passes over its digits (11, 11, 10 bits of the value, then 8, 8 of the index, top down) find the key of the k-th best -- each pass counts
 // the candidates that agree with the digits fixed so far, a suffix scan over the bins finds the bin the k-th falls in --
 // and everything at or above that key is gathered and put in order by counting.  Same results as the rounds
-// (tests/test_gpu_sampling.py).  Bound by latency: the partial lists of the sampled LM head (40960 candidates, k = 40) take 17.3 us, by
-// radix selection alone 40 (in no order in the map 28.7 and 51, sorted 18 and 44, all equal 26.4 and 60; 10240 of them 13.8 and 27); where that is what it comes to
-// after all (large values in fewer than k of the groups) 51 and 43.  Radix selection: loads on every path, TSEL_ASK at a time, and four counts a bin (the values share
+// (tests/test_gpu_sampling.py).  Bound by latency: the partial lists of the sampled LM head (40960 candidates, k = 40) take 16.6 us, by
+// radix selection alone 40 (in no order in the map 28.4 and 51, sorted 17.9 and 45, all equal 31 and 60; 10240 of them 14.5 and 27); where that is what it comes to
+// after all (large values in fewer than k of the groups) 56 and 43.  Radix selection: loads on every path, TSEL_ASK at a time, and four counts a bin (the values share
 // few bins of the first passes, and a wave's counts of one address go one behind the other); 59 us with each load under a condition and one count a bin.
 #define TSEL_THREADS 1024u
 #define TSEL_PER 40u
@@ -216,18 +216,12 @@ k_topk_select(float* data, const uint32_t* __restrict__ ls, const uint32_t* __re
   const auto note = [&](uint32_t j, uint32_t i, uint32_t which) {
     const uint32_t slot = atomicAdd(&n_list[which], 1u);
     if (slot < TSEL_LIST) list[slot] = (unsigned long long)vk[j] << 32 | (0xFFFFFFFFu - i);
-    return slot < TSEL_LIST;
   };
   anew();
-  bool room = true;
 #pragma unroll
   for (uint32_t j = 0; j < TSEL_PER; j++) {
     const uint32_t i = place(j / 4u) + j % 4u;
-    if (j / 4u < per && room) {
-      bool noted = true;
-      if (i >= first(j / 4u) && vk[j] >= least) noted = note(j, i, 0u);
-      room = __all(noted);
-    }
+    if (j / 4u < per && i >= first(j / 4u) && vk[j] >= least) note(j, i, 0u);
   }
   __syncthreads();
   uint32_t listed = n_list[0];
