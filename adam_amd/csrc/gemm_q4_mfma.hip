@@ -1480,7 +1480,7 @@ void gemm_act_forget() { g_xh_key.valid = false; }
 // Rows of fewer than 2048 columns: also k_gemm_q4_narrow, in steps of 128 columns of 0.42 us with few workgroups, 0.67 with one on every CU, and 3
 // a round of workgroups beside them (512 x 1536 x 1152 estimated 11.5, measured 12.5, tiled 19.3; 189 x 13824 x 1152 30.1, 28.4, tiled 29.8;
 // 512 x 13824 x 1152 66, 62, ring 44), where that is a tenth less than the ring's estimate, which is above what the ring takes by that and more (512 x 6912 x 1920
-// estimated 55 and 56, measured 54.5 and 47).  Longer rows go to the ring over shares of K, which is the better one where there are many of them and
+// estimated 55 and 56, measured 54.5 and 47), else, where it is less than tiled, the ring (320 x 6912 x 1536 without the conversion 30.0, tiled 32.9, ring 28.7).  Longer rows go to the ring over shares of K, which is the better one where there are many of them and
 // where the matrix is narrow: 512 x 4096 x 4096 51 and here 56, 70 x 1152 x 6912 26 and 36 (between them not everywhere: 189 x 4096 x 4096 32 and 28).
 struct GemmPlan { int ma; uint32_t shares; };
 static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
@@ -1515,20 +1515,21 @@ static GemmPlan gemm_plan(uint64_t M, uint64_t K, uint64_t N, int64_t b) {
   GemmPlan p = {0, 1};
   const double tiled = best;
   double rings = 1e30;
+  GemmPlan of_rings = p;
   for (int ma = 2; ma <= 4; ma++) {
     const uint64_t tiles = wgs(512, 32 * (uint64_t)ma);
     for (uint64_t sp = 1; sp <= most && (sp == 1 || (sp * 4 <= pairs && tiles * sp <= cu)); sp++) {
       const double full = std::min(1.0, (double)(tiles * sp) / (double)cu), step = ma == 2 ? 1.7 + 0.35 * full : ma == 3 ? 2.35 + 0.6 * full : 3.0 + 0.8 * full;
       const double sums = sp == 1 ? 0.0 : N % 4 == 0 ? 9.0 + (double)(sp + 1) * pass : 7.0 + (2.5 * (double)sp - 3.0) * pass;
       const double us = (double)up(tiles * sp, cu) * ((double)up(pairs, sp) * step + 7.0) + sums;
-      rings = std::min(rings, us);
-      if (us < best) { best = us; p = {ma, (uint32_t)sp}; }
+      if (us < rings) { rings = us; of_rings = {ma, (uint32_t)sp}; }
+      if (us < best) { best = us; p = of_rings; }
     }
   }
   if (ring == 1 && K < 2048) {
     const uint64_t tiles = wgs(128, 32);
     const double full = std::min(1.0, (double)tiles / (double)cu), us = 3.0 + (double)up(tiles, cu) * ((0.42 + 0.25 * full) * (double)steps + 3.0);
-    if (us < tiled && us < 0.9 * rings) p = {1, 1};
+    if (us < tiled) p = us < 0.9 * rings ? GemmPlan{1, 1} : of_rings;
   }
   return p;
 }
