@@ -586,12 +586,12 @@ static bool many_rows_pay(uint32_t experts, uint32_t identity, uint64_t entries,
   const float to = (float)std::min<uint64_t>(experts, entries), avg = (float)entries * (float)experts / (float)(experts + identity) / to;
   const Chip c = chip();
   const uint32_t steps = kp >> 6;
-  const auto tiles = [&](float bm) { return avg > 0.8f * bm ? to * (avg / bm + 0.5f) : to; };      // (half of an expert's last one is empty)
+  const auto tiles = [&](float bm) { return avg > 0.7f * bm ? to * (avg / bm + 0.5f) : to; };      // (half of an expert's last one is empty)
   const float few = tiles(64.f) * (float)cdiv(n, 64) * c.inv;                // a CU's
   float many = 1e30f;
   for (uint32_t i = 0; i < MANY_SIZES; i++)
     many = std::min(many, many_us(i, (uint32_t)std::min(1.6e7f, tiles(128.f + 64.f * (float)i) * (float)cdiv(n, 256)), steps, c));
-  return many < 4.f + 0.25f * (float)steps * std::max(1.f, few) + 1.6f * few;
+  return many < 3.f + 0.25f * (float)steps * std::max(1.f, few) + 2.f * few;
 }
 
 template <bool IN>

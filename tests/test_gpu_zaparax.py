@@ -662,7 +662,7 @@ def test_experts_of_many_rows_are_those_of_few(hip, rows, width, ff):
     ([(4, 205, 205), (1, 204, 204)], 16, 60, (64, 0), (64, 0)), ([(5, 205, 205)], 16, 60, (64, 0), (64, 0)), ([(4, 819, 819), (1, 820, 820)], 16, 60, (64, 0), (64, 0)),
     ([(4, 819, 819), (1, 821, 821)], 16, 60, (64, 0), (64, 0)), ([(4, 3277, 3277), (1, 3276, 3276)], 16, 60, (64, 0), (64, 0)), ([(5, 3277, 3277)], 16, 60, (64, 0), (64, 0)),
     ([(32, 90, 128)], 1000, 300, (128, 0), (64, 0)), ([(32, 150, 192)], 1024, 320, (192, 0), (64, 0)), ([(30, 200, 250), (10, 257, 380)], 1024, 320, (256, 0), (64, 0)),
-    ([(32, 90, 128)], 1024, 512, (128, 1), (64, 0)), ([(32, 150, 192)], 1024, 512, (192, 1), (64, 0)), ([(32, 200, 256)], 1024, 512, (256, 1), (128, 0)),
+    ([(32, 90, 128)], 1024, 512, (128, 1), (64, 0)), ([(32, 150, 192)], 1024, 512, (192, 1), (128, 0)), ([(32, 200, 256)], 1024, 512, (256, 1), (128, 0)),
     ([(32, 90, 128)], 300, 2000, (64, 0), (128, 0)), ([(32, 150, 192)], 320, 2048, (128, 0), (192, 0)), ([(30, 200, 250), (10, 257, 380)], 576, 2000, (256, 0), (256, 0)),
     ([(32, 90, 128)], 512, 2048, (128, 0), (128, 1)), ([(32, 150, 192)], 512, 2040, (128, 0), (192, 1)), ([(32, 200, 256)], 512, 2048, (128, 0), (256, 1))])
 def test_tiles_of_every_size_give_the_same_words(hip, counts, ff, width, first, second):
