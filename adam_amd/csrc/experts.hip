@@ -449,8 +449,8 @@ k_experts_tiled(const bf16_t* __restrict__ W, bf16_t* opnd, float* __restrict__ 
 // holds, and that hangs on the experts' counts, which only the device knows: every workgroup finds by them the size that costs least.  The results do not
 // hang on it.  A round takes what stands around a tile's steps and those steps, which are longer the more CUs have a tile, and less than in proportion to the rows
 // (weights and tokens on their way into LDS bound them; a third buffer for the weights, which come from memory: 2048 rows, 6 of 34 experts 1024 wide in 2048, both
-// products 208 us with two, 196 so).  Over 16 shapes of 3 .. 128 experts, 1 .. 64 steps and 8 .. 600 rows an expert, weights from memory, both products take 0.7 %
-// longer than in the best sizes (64 rows among them) in the mean, 13 % at most (24 experts 768 wide in 1536, 64 rows: 58 us and 51).
+// products 208 us with two, 196 so).  Over 16 shapes of 3 .. 128 experts, 1 .. 64 steps and 8 .. 600 rows an expert, weights from memory, both products take 0.6 %
+// longer than in the best sizes (64 rows among them) in the mean, 12 % at most (16 experts 1024 wide in 2048, 64 rows: 70 us and 62).
 #define MANY_SIZES 3u
 struct Chip { uint32_t cus, magic; float inv; };                                  // tiles / cus = umulhi(tiles, magic)
 __host__ __device__ __forceinline__ float many_us(uint32_t size, uint32_t tiles, uint32_t steps, const Chip& c) {      // of `tiles` tiles of 128 + 64 size rows
