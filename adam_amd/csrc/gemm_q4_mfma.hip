@@ -1651,8 +1651,8 @@ int launch_gemm_q4_mfma(const Map* ma, const Map* mw, const uint32_t* la, const 
     count_launch();
   };
   if (plan.shares > 1 && !ensure_part_buf((size_t)plan.shares * M * N)) {
-    if (sg.add) return ADAMAH_ERR_MEMORY;        // (the tiled kernel in one launch stores no add)
-    plan = {0, 1};
+    if (sg.add && !plan.ma) return ADAMAH_ERR_MEMORY;        // (the tiled kernel in one launch stores no add; narrow tiles do, of what the ring takes)
+    plan = {sg.add ? 1 : 0, 1};
   }
   if (plan.ma == 1) {
     const uint32_t run = cdiv(cdiv(N, 128) * cdiv(M, 32), 8);
