@@ -649,6 +649,7 @@ def test_narrow_tiles_at_ragged_ends(hip, monkeypatch, M, N, K, base):
 
 
 @pytest.mark.parametrize("M,N,K,plan", [(512, 1152, 1536, (32, 1)), (189, 1024, 1152, (32, 1)), (65, 64, 1920, (32, 1)), (512, 6912, 1920, (64, 2)), (256, 13824, 1920, (64, 2)),
+                                        (320, 6912, 1536, (64, 3)), (130, 13824, 1536, (64, 3)),
                                         (512, 1152, 2048, (0, 1)), (512, 13824, 1152, (64, 1))])
 def test_narrow_tiles_where_they_are_the_quicker_ones(hip, M, N, K, plan):
     """The rule at shapes whose forms were timed against each other (256 CUs)."""
